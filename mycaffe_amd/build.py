@@ -5,12 +5,14 @@
 Outputs (next to this file, git-ignored):
     libmycaffe_hip.so          the CudaDnnDLL-compatible C ABI (include/mycaffe_hip_abi.h)
     libmycaffe_hip_llama2.so   the llama2 extension library loaded through CREATE_EXTENSION
+    _hostcall.so               CPython module that packs the arguments of the Python mirror's calls (plain g++)
 and, beside their sources, two C++ host programs built on include/mycaffe_hip_host.hpp (plain g++, they only
 dlopen the libraries): tests/cpp/host_parity (parity) and host_bench/csa_layer_bench (whole-layer wall clock).
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -82,9 +84,24 @@ def build(force=False, verbose=True):
         built.append(out)
         if verbose:
             print("built", out)
+    built.append(build_hostcall(force, verbose))
     built.append(build_host_program(force, verbose))
     built.append(build_host_program(force, verbose, os.path.join(HERE, "host_bench", "csa_layer_bench.cpp"), host_bench_path()))
     return built
+
+
+def hostcall_path():
+    return os.path.join(HERE, "_hostcall.so")
+
+
+def build_hostcall(force=False, verbose=True):
+    src, out = os.path.join(CSRC, "hostcall.cpp"), hostcall_path()
+    if force or _stale(out, [src]):
+        subprocess.check_call([os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-I", sysconfig.get_path("include"),
+                               "-o", out, src])
+    if verbose:
+        print("built", out)
+    return out
 
 
 def host_program_path():

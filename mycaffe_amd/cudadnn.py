@@ -194,6 +194,21 @@ def llama2_extension_path():
     return os.path.join(_HERE, "libmycaffe_hip_llama2.so")
 
 
+def _hostcall():
+    """The native module that packs the arguments of a call (csrc/hostcall.cpp), built first only when no built file exists."""
+    global _host
+    if _host is None:
+        if not os.path.exists(_build.hostcall_path()):
+            _build.build_hostcall(verbose=False)
+        from . import _hostcall as module
+        module.set_error_class(CudaDnnError)
+        _host = module
+    return _host
+
+
+_host = None
+
+
 def load_library(path=None):
     """dlopen the HIP library (building it first only when no built file exists)."""
     path = path or default_library_path()
@@ -202,6 +217,7 @@ def load_library(path=None):
     if not os.path.exists(path):
         raise FileNotFoundError("HIP library not built: %s" % path)
     lib = ctypes.CDLL(path)
+    _hostcall()
     lib.DLL_InvokeFloat.argtypes = [_c_long, _c_long, _c_float_p, _c_long, ctypes.POINTER(_c_float_p),
                                     ctypes.POINTER(_c_long), _c_tchar_p, _c_long]
     lib.DLL_InvokeFloat.restype = _c_long
@@ -262,6 +278,9 @@ class CudaDnn:
 
     def __init__(self, nDeviceID=0, flags=DEVINIT.CUBLAS | DEVINIT.CURAND, lSeed=None, strPath=None):
         self._lib = load_library(strPath)
+        self._call = _hostcall().invoke
+        self._addr = ctypes.cast(getattr(self._lib, self._INVOKE_EX2), ctypes.c_void_p).value
+        self._double = self.DTYPE is np.float64
         self.Path = strPath or default_library_path()
         self.m_hKernel = 0
         args = [nDeviceID, flags] + ([lSeed] if lSeed is not None else [])
@@ -361,8 +380,9 @@ class CudaDnn:
         self._check(err, errbuf)
         return [_from_utf16(out)]
 
-    def _ex2(self, fn, rgf, rgl, cap=None):
-        return self.RunFloatEx2(self.m_hKernel, fn, rgf, rgl, cap)
+    def _ex2(self, fn, rgf, rgl):
+        """One Ex2 call whose arguments are a few Python numbers and whose result, if any, is a handful of values."""
+        return self._call(self._addr, self._double, self.m_hKernel, fn, rgf, rgl)
 
     # ---- lifetime / device ------------------------------------------------------
     def Dispose(self):
@@ -402,7 +422,7 @@ class CudaDnn:
             raise ValueError("no data")
         head = [data.size] + ([hStream] if hStream > 0 else [])
         rgf = np.concatenate([np.array(head, self.DTYPE), data])
-        return int(self._ex2(fn, rgf, head)[0])
+        return int(self.RunFloatEx2(self.m_hKernel, fn, rgf, head)[0])
 
     def FreeMemory(self, hMem):
         """CudaDnn.cs:2763-2790."""
@@ -412,7 +432,7 @@ class CudaDnn:
         """CudaDnn.cs:2935-2970: ``l{h, count}``; the DLL swaps in its own buffer when
         the caller's is too small."""
         cap = max(int(lCount), 1) if lCount >= 0 else self.OUT_CAPACITY
-        return self._ex2(CUDAFN.GETMEM, None, [hMem, lCount], cap)
+        return self.RunFloatEx2(self.m_hKernel, CUDAFN.GETMEM, None, [hMem, lCount], cap)
 
     def SetMemory(self, hMem, src, hStream=0, nCount=-1):
         """CudaDnn.cs:3027-3095: ``f{h, count, [stream,] data}``, ``l{h, count}``."""
@@ -423,7 +443,7 @@ class CudaDnn:
             raise ValueError("There are no data items to set!")
         head = [hMem, nCount] + ([hStream] if hStream > 0 else [])
         rgf = np.concatenate([np.array(head, self.DTYPE), data[:nCount]])
-        self._ex2(CUDAFN.SETMEM, rgf, [hMem, nCount])
+        self.RunFloatEx2(self.m_hKernel, CUDAFN.SETMEM, rgf, [hMem, nCount])
 
     def CreateMemoryPointer(self, hData, lOffset, lCount):
         """CudaDnn.cs:3274-3287."""

@@ -29,7 +29,10 @@ class Blob:
 
     def Reshape(self, *shape):
         if len(shape) == 1 and isinstance(shape[0], (list, tuple)):
-            shape = tuple(shape[0])
+            shape = shape[0]
+        shape = list(shape)
+        if shape == self.shape_ and self.gpu_data:
+            return
         self.shape_ = [int(s) for s in shape]
         n = self.count()
         if n > self._capacity:
@@ -42,8 +45,7 @@ class Blob:
         self.Reshape(*other.shape_)
 
     def count(self, start=0, end=None):
-        s = self.shape_[start:end]
-        return int(np.prod(s)) if s else 1
+        return math.prod(self.shape_[start:end])
 
     def shape(self, i):
         return self.shape_[i]
@@ -197,46 +199,55 @@ class InnerProductLayer:
 class TransposeLayer:
     """MyCaffe.layers.beta/layers.beta/TransposeLayer.cs:127-232."""
 
+    MAX_SHAPES = 8
+
     def __init__(self, cuda, dim):
         self.cuda, self.dim = cuda, list(dim)
-        self._key = None
+        # The attention layers send two shapes through one transpose layer in turn, (B,T,H,hs) on the way in and (B,H,T,hs)
+        # on the way out, so the blobs of a few shapes are kept: uploading them again on every call cost five allocations
+        # and five frees, each waiting for the device (0.5 ms a call).
+        self._shapes = {}
+        self._buffer, self._buffer_count = 0, 0
         self._handles = []
 
     def _reshape(self, shape):
         """Reshape (TransposeLayer.cs:127-200): stride arrays of bottom and top, forward and backward axis maps."""
-        key = (tuple(shape), tuple(self.dim))
-        top_shape = [shape[d] for d in self.dim]
-        if key != self._key:
-            for h in self._handles:
-                self.cuda.FreeMemory(h)
+        key = tuple(shape)
+        known = self._shapes.get(key)
+        if known is None:
             n = len(shape)
-            bc = [int(np.prod(shape[i + 1:])) for i in range(n)]
-            tc = [int(np.prod(top_shape[i + 1:])) for i in range(n)]
+            top_shape = [shape[d] for d in self.dim]
+            bc = [math.prod(shape[i + 1:]) for i in range(n)]
+            tc = [math.prod(top_shape[i + 1:]) for i in range(n)]
             bmap = [0] * n
             for i, d in enumerate(self.dim):
                 bmap[d] = i
-            self.counts_b = self.cuda.AllocMemory(np.float32(bc))
-            self.counts_t = self.cuda.AllocMemory(np.float32(tc))
-            self.fmap = self.cuda.AllocMemory(np.float32(self.dim))
-            self.bmap = self.cuda.AllocMemory(np.float32(bmap))
-            self.buffer = self.cuda.AllocMemory(int(np.prod(shape)) * n)
-            self._handles = [self.counts_b, self.counts_t, self.fmap, self.bmap, self.buffer]
-            self._key = key
-        return top_shape
+            if len(self._shapes) >= self.MAX_SHAPES:
+                for h in self._shapes.pop(next(iter(self._shapes)))[1]:
+                    self.cuda.FreeMemory(h)
+            known = self._shapes[key] = (top_shape, [self.cuda.AllocMemory(np.float32(v)) for v in (bc, tc, self.dim, bmap)])
+            if math.prod(shape) * n > self._buffer_count:
+                if self._buffer:
+                    self.cuda.FreeMemory(self._buffer)
+                self._buffer_count = math.prod(shape) * n
+                self._buffer = self.cuda.AllocMemory(self._buffer_count)
+            self._handles = [h for _, hs in self._shapes.values() for h in hs] + [self._buffer]
+        self.counts_b, self.counts_t, self.fmap, self.bmap = known[1]
+        return known[0]
 
     def Forward(self, bottom, top):
         if bottom.gpu_data == top.gpu_data:
             raise ValueError("The Transpose layer does not support in-place computation.")
         top.Reshape(*self._reshape(bottom.shape_))
         self.cuda.transpose(bottom.count(), bottom.gpu_data, top.gpu_data, self.counts_b, self.counts_t, self.fmap,
-                            len(bottom.shape_), self.buffer)
+                            len(bottom.shape_), self._buffer)
 
     def Backward(self, top, bottom):
         """TransposeLayer.cs:223-232: reshape for this bottom, then the same kernel with the count arrays swapped and the
         inverse axis map."""
         self._reshape(bottom.shape_)
         self.cuda.transpose(bottom.count(), top.gpu_diff, bottom.gpu_diff, self.counts_t, self.counts_b, self.bmap,
-                            len(bottom.shape_), self.buffer)
+                            len(bottom.shape_), self._buffer)
 
 
 class SoftmaxLayer:
