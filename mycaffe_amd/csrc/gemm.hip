@@ -13,30 +13,9 @@
 
 #include <type_traits>
 
-#include "kernels.h"
+#include "gemm_common.h"
 
 namespace mch {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-typedef float floatx2v __attribute__((ext_vector_type(2)));
-
-__device__ inline uint32_t pack2_bf16(float a, float b)
-{
-    floatx2v f = {a, b};
-    bf16x2v r = __builtin_convertvector(f, bf16x2v);
-    return *reinterpret_cast<uint32_t*>(&r);
-}
-
-template <typename T> __device__ inline float ldf(const T* p, size_t i);
-template <> __device__ inline float ldf<float>(const float* p, size_t i) { return p[i]; }
-template <> __device__ inline float ldf<bf16_t>(const bf16_t* p, size_t i) { return bf16_to_f32(p[i]); }
-template <typename T> __device__ inline void stf(T* p, size_t i, float v);
-template <> __device__ inline void stf<float>(float* p, size_t i, float v) { p[i] = v; }
-template <> __device__ inline void stf<bf16_t>(bf16_t* p, size_t i, float v) { p[i] = f32_to_bf16(v); }
 
 // ---------------------------------------------------------------------------
 // generic strided GEMM: C(i,j) = alpha * sum_k A(i,k) B(k,j) + beta * C(i,j)
@@ -114,104 +93,9 @@ static hipError_t launch_generic(hipStream_t s, int M, int N, int K, float alpha
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------
-// fp32 MFMA, NT.  4 wavefronts in a 2x2 arrangement, each owning 64x64 of the
-// 128x128 tile as 2x2 MFMA 32x32 blocks.  One 128-bit LDS read feeds four
-// MFMA steps: lane group g (= lane/32) holds k = kk+4g .. kk+4g+3, and MFMA step
-// j contracts the two slots {kk+j, kk+4+j}; the slot-to-k assignment is free as
-// long as A and B use the same one.
-__global__ __launch_bounds__(256) void gemm_nt_f32_mfma_kernel(int M, int N, int K, float alpha,
-                                                               const float* __restrict__ A,
-                                                               const float* __restrict__ B, float beta,
-                                                               float* __restrict__ C)
-{
-    constexpr int BM = 128, BN = 128, BK = 16, LDK = BK + 4;
-    __shared__ __attribute__((aligned(16))) float As[2][BM * LDK];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BN * LDK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int lr = tid >> 2, lc = (tid & 3) * 4;  // 64 rows x 4 float4 per pass, 2 passes
-
-    floatx16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-
-    float4 ra[2], rb[2];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            int r = lr + p * 64;
-            ra[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-            rb[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m0 + r < M && k0 + lc < K) ra[p] = *(const float4*)(A + (size_t)(m0 + r) * K + k0 + lc);
-            if (n0 + r < N && k0 + lc < K) rb[p] = *(const float4*)(B + (size_t)(n0 + r) * K + k0 + lc);
-        }
-    };
-    auto sstore = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            int r = lr + p * 64;
-            *(float4*)(&As[buf][r * LDK + lc]) = ra[p];
-            *(float4*)(&Bs[buf][r * LDK + lc]) = rb[p];
-        }
-    };
-
-    const int nk = (K + BK - 1) / BK;
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    const int fr = lane & 31, fg = (lane >> 5) * 4;
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) gload((kt + 1) * BK);
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 8) {
-            float4 a[2], b[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                a[t] = *(const float4*)(&As[buf][(wm + t * 32 + fr) * LDK + kk + fg]);
-                b[t] = *(const float4*)(&Bs[buf][(wn + t * 32 + fr) * LDK + kk + fg]);
-            }
-            const float* af0 = (const float*)&a[0];
-            const float* af1 = (const float*)&a[1];
-            const float* bf0 = (const float*)&b[0];
-            const float* bf1 = (const float*)&b[1];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(af0[j], bf0[j], acc[0][0], 0, 0, 0);
-                acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(af0[j], bf1[j], acc[0][1], 0, 0, 0);
-                acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(af1[j], bf0[j], acc[1][0], 0, 0, 0);
-                acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(af1[j], bf1[j], acc[1][1], 0, 0, 0);
-            }
-        }
-        if (kt + 1 < nk) sstore(buf ^ 1);
-        __syncthreads();
-    }
-    // accumulator register v of a 32x32 block: row = 8*(v/4) + 4*(lane/32) + v%4, col = lane%32
-    const int col_l = lane & 31, row_l = (lane >> 5) * 4;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int c = n0 + wn + j * 32 + col_l;
-            if (c >= N) continue;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                int r = m0 + wm + i * 32 + (v >> 2) * 8 + row_l + (v & 3);
-                if (r < M) {
-                    size_t ci = (size_t)r * N + c;
-                    float o = alpha * acc[i][j][v];
-                    if (beta != 0.f) o += beta * C[ci];
-                    C[ci] = o;
-                }
-            }
-        }
-}
+// A handful of outputs and a short contraction: one workgroup of the scalar kernel is done before a matrix-core tile has its
+// first stage in LDS.
+static inline bool gemm_is_tiny(int m, int n, int k) { return (long long)m * n <= 1024 && k <= 64; }
 
 // ---------------------------------------------------------------------------
 // bf16 MFMA, NT, 128x128x32 tiles, 4 wavefronts each 64x64 (2x2 MFMA 32x32x16).
@@ -312,88 +196,6 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_mfma_kernel(int M, int N, in
 // a group of eight and step e contracts {e, 4 + e}; the slot assignment only has to agree between A and B).
 // Tiles are numbered so that each XCD (workgroup index mod 8) works on a contiguous band of tile rows and
 // re-uses its A rows out of its own L2.
-template <typename T> struct BigTraits;
-template <> struct BigTraits<bf16_t> {
-    static constexpr int E = 8;   // elements per 16-byte chunk
-    __device__ static inline floatx16 mma(u32x4 a, u32x4 b, floatx16 c)
-    {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<bf16x8*>(&a), *reinterpret_cast<bf16x8*>(&b), c, 0, 0, 0);
-    }
-    __device__ static inline float ld(const bf16_t* p) { return bf16_to_f32(*p); }
-    __device__ static inline void st(bf16_t* p, float v) { *p = f32_to_bf16(v); }
-    __device__ static inline void st4(bf16_t* p, float a, float b, float c, float d)
-    {
-        uint2 w;
-        w.x = pack2_bf16(a, b);
-        w.y = pack2_bf16(c, d);
-        *(uint2*)p = w;
-    }
-};
-template <> struct BigTraits<float> {
-    static constexpr int E = 4;
-    __device__ static inline floatx16 mma(u32x4 a, u32x4 b, floatx16 c)
-    {
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
-        return c;
-    }
-    __device__ static inline float ld(const float* p) { return *p; }
-    __device__ static inline void st(float* p, float v) { *p = v; }
-    __device__ static inline void st4(float* p, float a, float b, float c, float d) { *(float4*)p = make_float4(a, b, c, d); }
-};
-
-// Epilogue of the fused QKV projection (HEADS): row r = (b, t) of the M = B*T rows, column c = (which, h, d) of the
-// N = 3*H*hs columns goes, bias added, to element (b, h, t, d) of tensor `which` (q, k, v), i.e. the layout the
-// attention kernels read, instead of to C[r][c].  Replaces the bias GEMM, the three channel copies and the three head
-// transposes that follow the fused InnerProduct in CausalSelfAttentionLayer.forward (CausalSelfAttentionLayer.cs:526-557).
-// With fcos / fsin set (tables [seq][hs/2]) the q and k thirds are also rotated, after their rounding to the storage type:
-// adjacent pairs (2i, 2i+1) of row r by the angle of table row r % seq, column i - the rotary embedding that the layer
-// applies to q and k in (B,T,H,hs) layout before the head transposes (CausalSelfAttentionLayer.cs:538-545, rope.cu:785-825).
-struct HeadsEpilogue { const void* bias; void* dst[3]; int T, H, hs; const float* fcos; const float* fsin; int seq; };
-
-template <typename T>
-__device__ __forceinline__ T* heads_dst(const HeadsEpilogue& he, int row, int col)
-{
-    const int Cd = he.H * he.hs;
-    const int which = col / Cd, w = col - which * Cd, h = w / he.hs, d = w - h * he.hs;
-    const int b = row / he.T, t = row - b * he.T;
-    return (T*)he.dst[which] + (((size_t)b * he.H + h) * he.T + t) * he.hs + d;
-}
-
-// (re, im) of one pair of q or k, rotated; the expressions of rope_kernel (ew_kernels.hip)
-__device__ __forceinline__ void heads_rope_pair(float c, float sn, float& re, float& im)
-{
-    const float a = re * c - im * sn, b = re * sn + im * c;
-    re = a; im = b;
-}
-
-// the rotation applied to one 16-byte piece (columns col .. col + 16 / sizeof(T) - 1 of row `row`; whole pairs of one head)
-template <typename T>
-__device__ __forceinline__ u32x4 heads_rope_piece(const HeadsEpilogue& he, int row, int col, u32x4 v)
-{
-    if (!he.fcos || col >= 2 * he.H * he.hs) return v;
-    constexpr int NP = 8 / (int)sizeof(T);
-    const size_t ti = (size_t)(row % he.seq) * (he.hs >> 1) + ((col % he.hs) >> 1);
-    uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const float c = he.fcos[ti + i], sn = he.fsin[ti + i];
-        if constexpr (sizeof(T) == 4) {
-            float re = __uint_as_float(w[2 * i]), im = __uint_as_float(w[2 * i + 1]);
-            heads_rope_pair(c, sn, re, im);
-            w[2 * i] = __float_as_uint(re); w[2 * i + 1] = __float_as_uint(im);
-        } else {
-            float re = __uint_as_float(w[i] << 16), im = __uint_as_float(w[i] & 0xffff0000u);
-            heads_rope_pair(c, sn, re, im);
-            w[i] = (uint32_t)f32_to_bf16(re) | ((uint32_t)f32_to_bf16(im) << 16);
-        }
-    }
-    u32x4 o; o.x = w[0]; o.y = w[1]; o.z = w[2]; o.w = w[3];
-    return o;
-}
-
 // Epilogues of the prompt pass of the Llama engine (fp32 results of 16-bit operands; llama2_ext.hip), which save the
 // round trip of the product through memory and the kernel that would read it back:
 //   EPI 1, SwiGLU of the stacked W1 | W3 product.  Tile column c multiplies weight row (c & 1) hid + c / 2, so that a
@@ -976,15 +778,6 @@ static bool launch_small_if_few(hipError_t* e, hipStream_t s, int m, int n, int 
     return true;
 }
 
-// fp32 keeps the matrix cores busy with 128 x 128 tiles as well (512 of them fill the chip at two workgroups per CU) and
-// measures 3 % faster with them when their rounds are full or half full; the wide tile wins (8192 x 2304 x 768: 232 ->
-// 214 us) where the last round of 128 x 128 tiles would be mostly empty.
-static bool short_last_round(long long t128)
-{
-    const long long rem = t128 % 512;
-    return rem != 0 && rem * 10 < 512 * 4;
-}
-
 // one stage of K is 128 bytes of a row: 64 elements in 16-bit storage, 32 in fp32
 template <typename T, bool HEADS>
 static bool launch_wide_if_fits(hipError_t* e, hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, void* C,
@@ -999,20 +792,6 @@ static bool launch_wide_if_fits(hipError_t* e, hipStream_t s, int m, int n, int 
 
 // K = 1: the rank-1 update C[i,j] = alpha a[i] b[j] + beta C[i,j] that InnerProductLayer uses to add its bias
 // (ones (M,1) x bias (1,N), InnerProductLayer.cs:405-414): one streaming pass over C, four columns per thread
-template <typename T> struct Quad;
-template <> struct Quad<float> {
-    __device__ static inline void load(const float* p, float (&v)[4]) { const float4 a = *(const float4*)p; v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; }
-    __device__ static inline void store(float* p, const float (&v)[4]) { *(float4*)p = make_float4(v[0], v[1], v[2], v[3]); }
-};
-template <> struct Quad<bf16_t> {
-    __device__ static inline void load(const bf16_t* p, float (&v)[4])
-    {
-        const uint2 a = *(const uint2*)p;
-        v[0] = __uint_as_float(a.x << 16); v[1] = __uint_as_float(a.x & 0xffff0000u);
-        v[2] = __uint_as_float(a.y << 16); v[3] = __uint_as_float(a.y & 0xffff0000u);
-    }
-    __device__ static inline void store(bf16_t* p, const float (&v)[4]) { *(uint2*)p = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3])); }
-};
 template <typename T, bool VEC>
 __global__ void gemm_rank1_kernel(int m, int n, float alpha, const T* __restrict__ a, const T* __restrict__ b, float beta, T* C)
 {
@@ -1065,39 +844,45 @@ __global__ void qkv_split_heads_kernel(const T* __restrict__ tmp, size_t total, 
     }
 }
 
-// X (m x kk) W^T (n x kk) through the tile kernels' HEADS epilogue `he`, or through `tmp` (m x n) and the splitting pass
-// whether a product with these operands goes through the scratch matrix (shapes and addresses the tile kernels do not take)
-static bool gemm_heads_through_tmp(DType dt, int kk, int rowUnit, const void* X, const void* W, const void* d0, const void* d1, const void* d2)
+// X (m x kk) W^T (n x kk) through the tile kernels' HEADS epilogue `he`; in 16-bit storage, shapes and addresses the tile
+// kernels do not take go through a scratch matrix (m x n) and a splitting pass
+static bool gemm_heads_through_tmp(int kk, int rowUnit, const void* X, const void* W, const void* d0, const void* d1, const void* d2)
 {
-    const int vec = dt == F32 ? 4 : 8;
-    const bool aligned = (((uintptr_t)X | (uintptr_t)W | (uintptr_t)d0 | (uintptr_t)d1 | (uintptr_t)d2) % 16 == 0) && rowUnit % vec == 0;
-    return !(aligned && kk % (dt == F32 ? 32 : 64) == 0);
+    const bool aligned = (((uintptr_t)X | (uintptr_t)W | (uintptr_t)d0 | (uintptr_t)d1 | (uintptr_t)d2) % 16 == 0) && rowUnit % 8 == 0;
+    return !(aligned && kk % 64 == 0);
 }
-bool k_gemm_bias_needs_tmp(DType dt, int n, int k, const void* X, const void* W, const void* Y)
+static size_t gemm_heads_workspace_bytes(DType dt, int m, int n, int kk, int rowUnit, const void* X, const void* W, const void* d0, const void* d1, const void* d2)
 {
-    return gemm_heads_through_tmp(dt, k, n, X, W, Y, Y, Y);
+    if (dt == F32) return gemm_f32_workspace_bytes(m, n, kk, 1, false);
+    return gemm_heads_through_tmp(kk, rowUnit, X, W, d0, d1, d2) ? (size_t)m * n * sizeof(bf16_t) : 0;
 }
-bool k_gemm_qkv_heads_needs_tmp(DType dt, int H, int hs, const void* X, const void* W, const void* q, const void* k, const void* v)
+size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W, const void* Y)
 {
-    return gemm_heads_through_tmp(dt, H * hs, hs, X, W, q, k, v);
+    return gemm_heads_workspace_bytes(dt, m, n, k, n, X, W, Y, Y, Y);
+}
+size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* q, const void* k, const void* v)
+{
+    return gemm_heads_workspace_bytes(dt, B * T, 3 * H * hs, H * hs, hs, X, W, q, k, v);
 }
 
 // (tiles256: the 256 x 256 tiles may be chosen as k_gemm chooses them)
 static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int kk, const void* X, const void* W, const HeadsEpilogue& he,
-                                      int rowUnit, void* tmp, bool tiles256)
+                                      int rowUnit, void* ws, size_t wsBytes, bool tiles256)
 {
+    if (dt == F32) {
+        GemmF32 g = {};
+        g.m = m; g.n = n; g.k = kk;
+        g.A = (const float*)X; g.B = (const float*)W;
+        g.lda = g.ldb = kk; g.ldc = n;
+        g.aK = g.bK = true;
+        g.alpha = 1.f; g.batch = 1;
+        g.heads = &he;
+        return gemm_f32(s, g, ws, wsBytes);
+    }
     const long long t256 = (long long)((m + 255) / 256) * ((n + 255) / 256);
     const bool full256 = tiles256 && (double)t256 / (double)(((t256 + 255) / 256) * 256) >= 0.85;
-    const bool aligned = !gemm_heads_through_tmp(dt, kk, rowUnit, X, W, he.dst[0], he.dst[1], he.dst[2]);   // and K in whole stages
+    const bool aligned = !gemm_heads_through_tmp(kk, rowUnit, X, W, he.dst[0], he.dst[1], he.dst[2]);   // and K in whole stages
     const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-    if (aligned && dt == F32) {
-        hipError_t e;
-        if (full256 && kk >= 1024) return launch_big<float, 4, 4, 1, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
-        if (launch_small_if_few<float, true>(&e, s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he)) return e;
-        if (n % 192 == 0 && t128 <= 512) return launch_big<float, 2, 3, 2, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
-        if (short_last_round(t128) && launch_wide_if_fits<float, true>(&e, s, m, n, kk, 1.f, X, W, nullptr, &he)) return e;
-        return launch_big<float, 2, 2, 2, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
-    }
     if (aligned && dt == BF16) {
         hipError_t e;
         if (full256 && kk >= 2048) return launch_big<bf16_t, 4, 4, 1, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
@@ -1107,18 +892,17 @@ static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int
         return launch_big<bf16_t, 2, 2, 2, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
     }
     // any other shape: plain product into the caller's scratch matrix, then one splitting pass
-    if (!tmp) return hipErrorInvalidValue;
-    hipError_t e = k_gemm(s, dt, false, true, m, n, kk, 1.f, X, W, 0.f, tmp);
+    if (!ws || wsBytes < (size_t)m * n * sizeof(bf16_t)) return hipErrorInvalidValue;
+    hipError_t e = k_gemm(s, dt, false, true, m, n, kk, 1.f, X, W, 0.f, ws);
     if (e != hipSuccess) return e;
     const size_t total = (size_t)m * n;
     const int grid = (int)std::min<size_t>((total + 255) / 256, 8192);
-    if (dt == F32) hipLaunchKernelGGL(qkv_split_heads_kernel<float>, grid, 256, 0, s, (const float*)tmp, total, n, he);
-    else hipLaunchKernelGGL(qkv_split_heads_kernel<bf16_t>, grid, 256, 0, s, (const bf16_t*)tmp, total, n, he);
+    hipLaunchKernelGGL(qkv_split_heads_kernel<bf16_t>, grid, 256, 0, s, (const bf16_t*)ws, total, n, he);
     return hipGetLastError();
 }
 
 hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* bias,
-                            void* q, void* k, void* v, void* tmp, const float* fcos, const float* fsin, int ropeSeq)
+                            void* q, void* k, void* v, void* ws, size_t wsBytes, const float* fcos, const float* fsin, int ropeSeq)
 {
     if (fcos && (!fsin || ropeSeq < 1 || (hs & 1))) return hipErrorInvalidValue;
     const int m = B * T, C = H * hs, n = 3 * C, kk = C;
@@ -1126,19 +910,19 @@ hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs
     HeadsEpilogue he;
     he.bias = bias; he.dst[0] = q; he.dst[1] = k; he.dst[2] = v; he.T = T; he.H = H; he.hs = hs;
     he.fcos = fcos; he.fsin = fcos ? fsin : nullptr; he.seq = fcos ? ropeSeq : 1;
-    return gemm_heads_dispatch(s, dt, m, n, kk, X, W, he, hs, tmp, false);
+    return gemm_heads_dispatch(s, dt, m, n, kk, X, W, he, hs, ws, wsBytes, false);
 }
 
 // Y (m x n) = X (m x k) W^T (n x k) + bias (n): the inner product layer's forward in one launch (InnerProductLayer.cs:
 // 372-417 issues the product and a rank-1 update with a vector of ones).  The HEADS epilogue with one head of n values
 // over m positions is the plain row-major layout, so the same kernels serve.
-hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* tmp)
+hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes)
 {
     if (m <= 0 || n <= 0) return hipSuccess;
     HeadsEpilogue he;
     he.bias = bias; he.dst[0] = he.dst[1] = he.dst[2] = Y; he.T = m; he.H = 1; he.hs = n;
     he.fcos = nullptr; he.fsin = nullptr; he.seq = 1;
-    return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, n, tmp, true);
+    return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, n, ws, wsBytes, true);
 }
 
 // C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
@@ -1227,27 +1011,25 @@ __global__ __launch_bounds__(256) void transpose2d_kernel(const T* __restrict__ 
     }
 }
 
-static hipError_t transpose2d(hipStream_t s, DType dt, const void* x, void* y, int rows, int cols)
+static hipError_t transpose2d(hipStream_t s, const void* x, void* y, int rows, int cols)
 {
     dim3 grid((cols + 63) / 64, (rows + 63) / 64);
     if (grid.y > 65535) return hipErrorInvalidValue;
-    if (dt == F32) hipLaunchKernelGGL(transpose2d_kernel<float>, grid, 256, 0, s, (const float*)x, (float*)y, rows, cols);
-    else hipLaunchKernelGGL(transpose2d_kernel<bf16_t>, grid, 256, 0, s, (const bf16_t*)x, (bf16_t*)y, rows, cols);
+    hipLaunchKernelGGL(transpose2d_kernel<bf16_t>, grid, 256, 0, s, (const bf16_t*)x, (bf16_t*)y, rows, cols);
     return hipGetLastError();
 }
 
-// The transpose combinations other than A B^T (InnerProductLayer backward: data gradient dY W, weight gradient dY^T X,
-// InnerProductLayer.cs:429-494).  The tile kernels want both operands with the contracted index at unit stride; an
-// operand that lies the other way is turned once into scratch memory and the product then runs on them.  In 16-bit
-// storage that replaces the strided scalar kernel (8192 x 768 x 2304: 604 -> 36 us, the weight gradient 1778 -> 63 us),
-// in fp32 the strided MFMA kernel where the product is large enough to pay for the pass over the operand.
+// The transpose combinations other than A B^T in 16-bit storage (InnerProductLayer backward: data gradient dY W, weight
+// gradient dY^T X, InnerProductLayer.cs:429-494).  The tile kernels want both operands with the contracted index at unit
+// stride; an operand that lies the other way is turned once into scratch memory and the product then runs on them
+// (8192 x 768 x 2304: 604 -> 36 us, the weight gradient 1778 -> 63 us against the strided scalar kernel).
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // A long contraction with few tiles (weight gradients: K is the token count) is cut into 2 .. 16 equal parts, one row of
 // workgroups of 128 x 128 tiles each, until the launch has some 400 workgroups; every part stays 512 long at least.
-static int gemm_ksplits(DType dt, int m, int n, int k)
+static int gemm_ksplits(int m, int n, int k)
 {
-    const int bk = dt == F32 ? 32 : 64;
+    const int bk = 64;
     const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
     if (t128 >= 200 || k < 2048 || ((long long)m * n) % 4) return 1;
     int S = 1;
@@ -1274,54 +1056,54 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int S, size
         Quad<T>::store(C + 4 * e, v);
     }
 }
-static bool gemm_turns_operands(DType dt, bool tA, bool tB, int m, int n, int k)
+static bool gemm_turns_operands(bool tA, bool tB, int m, int n, int k)
 {
     if (!tA && tB) return false;
-    const int vec = dt == F32 ? 4 : 8;
-    if (k < 64 || k % vec || (tA && m % vec) || (!tB && n % vec)) return false;
-    const double turned = (tA ? (double)m * k : 0.0) + (!tB ? (double)n * k : 0.0);
-    if (dt == BF16) return (double)m * n >= 64.0 * 64.0;
-    // fp32: 136 against 88 TFLOP/s for the product, about 3 TB/s (read + write) for the pass over an operand
-    // Also where the strided kernel would split a long contraction over workgroups that add their parts with atomics
-    // (few tiles, K of 2048 and more): here the parts are summed in a fixed order, so a weight gradient comes out the
-    // same bits every run, at the same speed to within a few per cent.
-    if ((long long)((m + 127) / 128) * ((n + 127) / 128) < 256 && k >= 2048) return true;
-    return (double)m * n * k * 8.0e-15 > 1.5 * turned * 8.0 / 3.0e12;
+    if (k < 64 || k % 8 || (tA && m % 8) || (!tB && n % 8)) return false;
+    return (double)m * n >= 64.0 * 64.0;
 }
-static size_t gemm_turned_bytes(DType dt, bool tA, bool tB, int m, int n, int k)
+static size_t gemm_turned_bytes(bool tA, bool tB, int m, int n, int k)
 {
-    const size_t es = dt == F32 ? 4 : 2;
-    return (tA ? round256((size_t)m * k * es) : 0) + (!tB ? round256((size_t)n * k * es) : 0);
+    return (tA ? round256((size_t)m * k * sizeof(bf16_t)) : 0) + (!tB ? round256((size_t)n * k * sizeof(bf16_t)) : 0);
 }
 size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k)
 {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    if (m <= 0 || n <= 0 || k <= 1) return 0;
+    if (dt == F32) return gemm_is_tiny(m, n, k) ? 0 : gemm_f32_workspace_bytes(m, n, k, 1, false);
     const bool nt = !tA && tB;
-    if (!nt && !gemm_turns_operands(dt, tA, tB, m, n, k)) return 0;
-    const int S = k % (dt == F32 ? 4 : 8) == 0 ? gemm_ksplits(dt, m, n, k) : 1;
-    return (nt ? 0 : gemm_turned_bytes(dt, tA, tB, m, n, k)) + (S > 1 ? (size_t)S * m * n * sizeof(float) : 0);
+    if (!nt && !gemm_turns_operands(tA, tB, m, n, k)) return 0;
+    const int S = k % 8 == 0 ? gemm_ksplits(m, n, k) : 1;
+    return (nt ? 0 : gemm_turned_bytes(tA, tB, m, n, k)) + (S > 1 ? (size_t)S * m * n * sizeof(float) : 0);
 }
 
 hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k, float alpha, const void* A,
                   const void* B, float beta, void* C, void* ws, size_t wsBytes)
 {
     if (m <= 0 || n <= 0) return hipSuccess;
-    if (ws && k > 1 && (((uintptr_t)A | (uintptr_t)B | (uintptr_t)ws) % 16 == 0) && gemm_turns_operands(dt, tA, tB, m, n, k) &&
+    if (dt == F32 && k > 1 && !gemm_is_tiny(m, n, k)) {
+        GemmF32 g = {};
+        g.m = m; g.n = n; g.k = k;
+        g.A = (const float*)A; g.B = (const float*)B; g.C = (float*)C;
+        g.aK = !tA; g.bK = tB;
+        g.lda = tA ? m : k; g.ldb = tB ? k : n; g.ldc = n;
+        g.alpha = alpha; g.beta = beta; g.batch = 1;
+        return gemm_f32(s, g, ws, wsBytes);
+    }
+    if (dt == BF16 && ws && k > 1 && (((uintptr_t)A | (uintptr_t)B | (uintptr_t)ws) % 16 == 0) && gemm_turns_operands(tA, tB, m, n, k) &&
         wsBytes >= k_gemm_workspace_bytes(dt, tA, tB, m, n, k)) {
-        const size_t es = dt == F32 ? 4 : 2;
         const void *a2 = A, *b2 = B;
         char* w = (char*)ws;
         if (tA) {   // stored (k, m)
-            hipError_t e = transpose2d(s, dt, A, w, k, m);
+            hipError_t e = transpose2d(s, A, w, k, m);
             if (e != hipSuccess) return e;
             a2 = w;
-            w += round256((size_t)m * k * es);
+            w += round256((size_t)m * k * sizeof(bf16_t));
         }
         if (!tB) {  // stored (k, n)
-            hipError_t e = transpose2d(s, dt, B, w, k, n);
+            hipError_t e = transpose2d(s, B, w, k, n);
             if (e != hipSuccess) return e;
             b2 = w;
-            w += round256((size_t)n * k * es);
+            w += round256((size_t)n * k * sizeof(bf16_t));
         }
         return k_gemm(s, dt, false, true, m, n, k, alpha, a2, b2, beta, C, w, wsBytes - (size_t)(w - (char*)ws));
     }
@@ -1336,12 +1118,10 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
 #undef RANK1
         return hipGetLastError();
     }
-    if (m <= 0 || n <= 0) return hipSuccess;
     if (k <= 0) k = 0;
-    // MFMA fast path: A (m,k) and B (n,k) both k-contiguous, 16-byte aligned rows
-    const int vec = dt == F32 ? 4 : 8;
-    bool aligned = (k % vec == 0) && (((uintptr_t)A | (uintptr_t)B) % 16 == 0) && k >= vec;
-    if (!tA && tB && aligned) {
+    // MFMA path in 16-bit storage: A (m,k) and B (n,k) both k-contiguous, 16-byte aligned rows
+    const bool aligned = (k % 8 == 0) && (((uintptr_t)A | (uintptr_t)B) % 16 == 0) && k >= 8;
+    if (dt == BF16 && !tA && tB && aligned) {
         dim3 grid((n + 127) / 128, (m + 127) / 128);
         if (grid.y > 65535) return hipErrorInvalidValue;
         // Large-tile kernels need whole 128-byte stages along K.  256 x 256 tiles (one wavefront per SIMD, 128 x 128
@@ -1351,40 +1131,24 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
         const long long t256 = (long long)((m + 255) / 256) * ((n + 255) / 256);
         const double fill = (double)t256 / (double)(((t256 + 255) / 256) * 256);
         const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-        const int S = ws && (((uintptr_t)ws | (uintptr_t)C) % 16 == 0) ? gemm_ksplits(dt, m, n, k) : 1;
+        const int S = ws && (((uintptr_t)ws | (uintptr_t)C) % 16 == 0) ? gemm_ksplits(m, n, k) : 1;
         if (S > 1 && wsBytes >= (size_t)S * m * n * sizeof(float)) {
-            hipError_t e = dt == F32 ? launch_big<float, 2, 2, 2>(s, m, n, k, alpha, A, B, 0.f, ws, nullptr, nullptr, S)
-                                     : launch_big<bf16_t, 2, 2, 2, false, float>(s, m, n, k, alpha, A, B, 0.f, ws, nullptr, nullptr, S);
+            hipError_t e = launch_big<bf16_t, 2, 2, 2, false, float>(s, m, n, k, alpha, A, B, 0.f, ws, nullptr, nullptr, S);
             if (e != hipSuccess) return e;
             const size_t total4 = (size_t)m * n / 4;
             const int g = (int)std::min<size_t>((total4 + 255) / 256, 4096);
-            if (dt == F32) hipLaunchKernelGGL(splitk_reduce_kernel<float>, g, 256, 0, s, (const float*)ws, S, total4, beta, (float*)C);
-            else hipLaunchKernelGGL(splitk_reduce_kernel<bf16_t>, g, 256, 0, s, (const float*)ws, S, total4, beta, (bf16_t*)C);
+            hipLaunchKernelGGL(splitk_reduce_kernel<bf16_t>, g, 256, 0, s, (const float*)ws, S, total4, beta, (bf16_t*)C);
             return hipGetLastError();
         }
-        if (dt == F32) {
-            if (k % 32 == 0) {
-                if (k >= 1024 && fill >= 0.85) return launch_big<float, 4, 4, 1>(s, m, n, k, alpha, A, B, beta, C);
-                hipError_t e;
-                if (launch_small_if_few<float, false>(&e, s, m, n, k, alpha, A, B, beta, C)) return e;
-                if (n % 192 == 0 && t128 <= 512) return launch_big<float, 2, 3, 2>(s, m, n, k, alpha, A, B, beta, C);
-                if (beta == 0.f && short_last_round(t128) && launch_wide_if_fits<float, false>(&e, s, m, n, k, alpha, A, B, C)) return e;
-                return launch_big<float, 2, 2, 2>(s, m, n, k, alpha, A, B, beta, C);
-            }
-            hipLaunchKernelGGL(gemm_nt_f32_mfma_kernel, grid, 256, 0, s, m, n, k, alpha, (const float*)A, (const float*)B,
-                               beta, (float*)C);
-        } else {
-            if (k % 64 == 0) {
-                if (k >= 2048 && fill >= 0.85) return launch_big<bf16_t, 4, 4, 1>(s, m, n, k, alpha, A, B, beta, C);
-                hipError_t e;
-                if (beta == 0.f && launch_wide_if_fits<bf16_t, false>(&e, s, m, n, k, alpha, A, B, C)) return e;
-                if (launch_small_if_few<bf16_t, false>(&e, s, m, n, k, alpha, A, B, beta, C)) return e;
-                if (n % 192 == 0 && t128 <= 512) return launch_big<bf16_t, 2, 3, 2>(s, m, n, k, alpha, A, B, beta, C);
-                return launch_big<bf16_t, 2, 2, 2>(s, m, n, k, alpha, A, B, beta, C);
-            }
-            hipLaunchKernelGGL(gemm_nt_bf16_mfma_kernel, grid, 256, 0, s, m, n, k, alpha, (const bf16_t*)A,
-                               (const bf16_t*)B, beta, (bf16_t*)C);
+        if (k % 64 == 0) {
+            if (k >= 2048 && fill >= 0.85) return launch_big<bf16_t, 4, 4, 1>(s, m, n, k, alpha, A, B, beta, C);
+            hipError_t e;
+            if (beta == 0.f && launch_wide_if_fits<bf16_t, false>(&e, s, m, n, k, alpha, A, B, C)) return e;
+            if (launch_small_if_few<bf16_t, false>(&e, s, m, n, k, alpha, A, B, beta, C)) return e;
+            if (n % 192 == 0 && t128 <= 512) return launch_big<bf16_t, 2, 3, 2>(s, m, n, k, alpha, A, B, beta, C);
+            return launch_big<bf16_t, 2, 2, 2>(s, m, n, k, alpha, A, B, beta, C);
         }
+        hipLaunchKernelGGL(gemm_nt_bf16_mfma_kernel, grid, 256, 0, s, m, n, k, alpha, (const bf16_t*)A, (const bf16_t*)B, beta, (bf16_t*)C);
         return hipGetLastError();
     }
     GemmStrides st;
@@ -1392,192 +1156,12 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
     st.bk = tB ? 1 : n;  st.bj = tB ? k : 1;   // B stored (k,n) or (n,k)
     st.ci = n;           st.cj = 1;
     st.sA = st.sB = st.sC = 0;
-    if (dt == F32 && k > 0) {
-        // the other transpose combinations (InnerProductLayer backward: weight gradient dY^T X, data gradient dY W) run on
-        // the strided fp32 MFMA kernel: row-major C = op(A) op(B) is column-major C^T = op(B)^T op(A)^T
-        return k_gemm2(s, tB, tA, n, m, k, alpha, (const float*)B, (const float*)A, beta, (float*)C, tB ? k : n, tA ? m : k, n, 0, 0, 0, 1);
-    }
     if (dt == F32)
         return launch_generic<float>(s, m, n, k, alpha, (const float*)A, (const float*)B, beta, (float*)C, st, 1);
     return launch_generic<bf16_t>(s, m, n, k, alpha, (const bf16_t*)A, (const bf16_t*)B, beta, (bf16_t*)C, st, 1);
 }
 
 // ---------------------------------------------------------------------------
-// fp32 MFMA for the strided-batched gemm2 (the Blob.MatMul route of the explicit attention chain: Q K^T and P V per
-// (batch, head), math.cu:1750-1788).  Column-major operands with any leading dimension: A(i,k) has either i or k at unit
-// stride, B(k,j) either k or j, C(i,j) has i at unit stride.  An operand with k at unit stride is staged into LDS as
-// [row][k], so that one 128-bit LDS read feeds four v_mfma_f32_32x32x2_f32 steps (slot trick as in
-// gemm_nt_f32_mfma_kernel); one with the row index at unit stride is staged as it lies, [k][row], and a lane gathers its
-// four k with 32-bit reads (consecutive lanes, consecutive words: no bank conflicts on either side).  The MFMA row operand is B and the column
-// operand is A: the accumulator then has i in the lane and every store instruction of a wavefront writes two 128-byte
-// runs of C.  TI x TJ tile (i x j), four wavefronts 2 x 2.
-template <bool A_IFAST, bool B_KFAST, int TI, int TJ>
-__global__ __launch_bounds__(256) void gemm2_f32_mfma_kernel(int M, int N, int K, float alpha, const float* __restrict__ A,
-                                                             const float* __restrict__ B, float beta, float* __restrict__ C,
-                                                             GemmStrides st, int splits, int kChunk, const int* causalFlag, int epoch)
-{
-    // B(k,j) known to be zero for k > j (the probabilities of a causal softmax, unless the flag carries this launch's
-    // epoch): the contraction of this tile of columns stops at its last column
-    // Tiles of columns then differ in length.  Consecutive workgroups go to consecutive dies, and workgroup i shares its CU
-    // with i + 256, i + 512, ... (all are resident at once): the tile a workgroup takes is rotated by its batch index, so
-    // that no die is left with the long ones, and every other round of 256 takes them in reverse, so that a long tile
-    // meets a short one on its CU.
-    int jTile = blockIdx.y;
-    if (causalFlag) {
-        // (decided per batch index, so that the tiles of one batch entry are still each taken once)
-        const unsigned first = gridDim.x * gridDim.y * blockIdx.z;
-        jTile = (int)((blockIdx.y + blockIdx.z) % gridDim.y);
-        if ((first >> 8) & 1) jTile = (int)gridDim.y - 1 - jTile;
-    }
-    // (B given transposed, B(k,j) stored as [k][j]: the same tensor read the other way, zero for k < j - the product with the
-    // transposed probabilities in the backward pass - and the contraction begins at the tile's first column instead)
-    const bool causal = causalFlag && *causalFlag != epoch;
-    if (causal && B_KFAST) K = min(K, (jTile + 1) * TJ);
-    constexpr int BK = 16, LDK = BK + 4;
-    constexpr int LDI = TI + 4, LDJ = TJ + 4;        // row strides of the [k][row] layouts
-    constexpr int NI = TI / 64, NJ = TJ / 64;        // 32x32 blocks per wavefront along i and j
-    __shared__ __attribute__((aligned(16))) float Is[2][A_IFAST ? BK * LDI : TI * LDK];   // A: [k][i] or [i][k]
-    __shared__ __attribute__((aligned(16))) float Js[2][B_KFAST ? TJ * LDK : BK * LDJ];   // B: [j][k] or [k][j]
-    // blockIdx.z = batch * splits + split; with splits > 1 every workgroup covers kChunk of the contraction and adds its
-    // part to C with float atomics (C holds beta * C already)
-    const int batchIdx = blockIdx.z / splits, split = blockIdx.z % splits;
-    const int kBegin = (causal && !B_KFAST) ? min(K, jTile * TJ) : split * kChunk;
-    if (splits > 1) K = min(K, kBegin + kChunk);
-    A += (size_t)batchIdx * st.sA;
-    B += (size_t)batchIdx * st.sB;
-    C += (size_t)batchIdx * st.sC;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave & 1) * (TI / 2), wj = (wave >> 1) * (TJ / 2);
-    const int i0 = blockIdx.x * TI, j0 = jTile * TJ;
-    const long long lda = A_IFAST ? st.ak : st.ai, ldb = B_KFAST ? st.bj : st.bk;
-
-    floatx16 acc[NJ][NI];
-#pragma unroll
-    for (int a = 0; a < NJ; a++)
-#pragma unroll
-        for (int b = 0; b < NI; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[a][b][v] = 0.f;
-
-    // staging: TI*BK/4 float4 of A and TJ*BK/4 of B per stage, 256 threads
-    constexpr int PA = TI * BK / 4 / 256, PB = TJ * BK / 4 / 256;
-    float4 ra[PA], rb[PB];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int p = 0; p < PA; p++) {
-            const int e = tid + p * 256;
-            ra[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (A_IFAST) {   // four consecutive i at one k
-                const int ig = e % (TI / 4), k = e / (TI / 4);
-                if (i0 + 4 * ig < M && k0 + k < K) ra[p] = *(const float4*)(A + (size_t)(i0 + 4 * ig) + (size_t)(k0 + k) * lda);
-            } else {         // four consecutive k at one i
-                const int kg = e % (BK / 4), i = e / (BK / 4);
-                if (i0 + i < M && k0 + 4 * kg < K) ra[p] = *(const float4*)(A + (size_t)(i0 + i) * lda + (size_t)(k0 + 4 * kg));
-            }
-        }
-#pragma unroll
-        for (int p = 0; p < PB; p++) {
-            const int e = tid + p * 256;
-            rb[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (B_KFAST) {
-                const int kg = e % (BK / 4), j = e / (BK / 4);
-                if (j0 + j < N && k0 + 4 * kg < K) rb[p] = *(const float4*)(B + (size_t)(j0 + j) * ldb + (size_t)(k0 + 4 * kg));
-            } else {
-                const int jg = e % (TJ / 4), k = e / (TJ / 4);
-                if (j0 + 4 * jg < N && k0 + k < K) rb[p] = *(const float4*)(B + (size_t)(j0 + 4 * jg) + (size_t)(k0 + k) * ldb);
-            }
-        }
-    };
-    auto sstore = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < PA; p++) {
-            const int e = tid + p * 256;
-            if (A_IFAST) {
-                const int ig = e % (TI / 4), k = e / (TI / 4);
-                *(float4*)(&Is[buf][k * LDI + 4 * ig]) = ra[p];
-            } else {
-                const int kg = e % (BK / 4), i = e / (BK / 4);
-                *(float4*)(&Is[buf][i * LDK + 4 * kg]) = ra[p];
-            }
-        }
-#pragma unroll
-        for (int p = 0; p < PB; p++) {
-            const int e = tid + p * 256;
-            if (B_KFAST) {
-                const int kg = e % (BK / 4), j = e / (BK / 4);
-                *(float4*)(&Js[buf][j * LDK + 4 * kg]) = rb[p];
-            } else {
-                const int jg = e % (TJ / 4), k = e / (TJ / 4);
-                *(float4*)(&Js[buf][k * LDJ + 4 * jg]) = rb[p];
-            }
-        }
-    };
-
-    const int nk = (K - kBegin + BK - 1) / BK;
-    gload(kBegin);
-    sstore(0);
-    __syncthreads();
-    const int fr = lane & 31, fg = (lane >> 5) * 4;
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) gload(kBegin + (kt + 1) * BK);
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 8) {
-            float4 fj[NJ], fi[NI];
-#pragma unroll
-            for (int t = 0; t < NJ; t++) {
-                if (B_KFAST) {
-                    fj[t] = *(const float4*)(&Js[buf][(wj + t * 32 + fr) * LDK + kk + fg]);
-                } else {   // four k of one j: consecutive lanes read consecutive words
-                    const float* q = &Js[buf][(kk + fg) * LDJ + wj + t * 32 + fr];
-                    fj[t] = make_float4(q[0], q[LDJ], q[2 * LDJ], q[3 * LDJ]);
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < NI; t++) {
-                if (A_IFAST) {
-                    const float* q = &Is[buf][(kk + fg) * LDI + wi + t * 32 + fr];
-                    fi[t] = make_float4(q[0], q[LDI], q[2 * LDI], q[3 * LDI]);
-                } else {
-                    fi[t] = *(const float4*)(&Is[buf][(wi + t * 32 + fr) * LDK + kk + fg]);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int a = 0; a < NJ; a++)
-#pragma unroll
-                    for (int b = 0; b < NI; b++)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float*)&fj[a])[e], ((const float*)&fi[b])[e], acc[a][b], 0, 0, 0);
-        }
-        if (kt + 1 < nk) sstore(buf ^ 1);
-        __syncthreads();
-    }
-    // accumulator register v of a block: j = 8*(v/4) + 4*(lane/32) + v%4, i = lane%32
-    const int il = lane & 31, jl = (lane >> 5) * 4;
-#pragma unroll
-    for (int a = 0; a < NJ; a++)
-#pragma unroll
-        for (int b = 0; b < NI; b++) {
-            const int i = i0 + wi + b * 32 + il;
-            if (i >= M) continue;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int j = j0 + wj + a * 32 + (v >> 2) * 8 + jl + (v & 3);
-                if (j < N) {
-                    const size_t ci = (size_t)i + (size_t)j * st.cj;
-                    float o = alpha * acc[a][b][v];
-                    if (splits > 1) {
-                        unsafeAtomicAdd(&C[ci], o);
-                    } else {
-                        if (beta != 0.f) o += beta * C[ci];
-                        C[ci] = o;
-                    }
-                }
-            }
-        }
-}
-
 // The same product for a short contraction (K = KC of at most 128: Q K^T of the explicit attention chain, K = head size)
 // with A(i,k) i-fast and B(k,j) k-fast.  A tile of such a product is all prologue and epilogue for the kernel above: one
 // trip to memory for the operands, a few MFMAs, 64 KB of C to write.  Here a workgroup keeps its 128 rows of B (the j
@@ -1724,42 +1308,6 @@ static hipError_t launch_gemm2_panel(hipStream_t s, int M, int N, float alpha, c
     return hipGetLastError();
 }
 
-template <typename T> __global__ void gemm_prescale_kernel(T* c, size_t n, float beta)
-{
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)blockDim.x * gridDim.x)
-        c[i] = beta == 0.f ? 0.f : beta * c[i];
-}
-
-template <bool A_IFAST, bool B_KFAST>
-static hipError_t launch_gemm2_mfma(hipStream_t s, int M, int N, int K, float alpha, const float* A, const float* B, float beta,
-                                    float* C, const GemmStrides& st, int batch, const int* causalFlag = nullptr, int epoch = 0)
-{
-    const bool si = M <= 64, sj = N <= 64;
-    const int gi = (M + (si ? 63 : 127)) / (si ? 64 : 128), gj = (N + (sj ? 63 : 127)) / (sj ? 64 : 128);
-    // Split the contraction when one batch of few tiles has a long K (weight gradients: K = batch x sequence): enough
-    // workgroups for two per CU, at least 512 of K each.  Needs a dense C (ldc == M) for the beta pre-pass.
-    int splits = 1, kChunk = K;
-    const long long tiles = (long long)gi * gj;
-    if (batch == 1 && tiles < 256 && K >= 2048 && st.cj == M) {
-        splits = (int)std::min<long long>((512 + tiles - 1) / tiles, K / 512);
-        if (splits > 1) {
-            kChunk = (((K + splits - 1) / splits) + 15) / 16 * 16;
-            splits = (K + kChunk - 1) / kChunk;
-        }
-        if (splits > 1 && beta != 1.f) {
-            const size_t cn = (size_t)M * N;
-            hipLaunchKernelGGL(gemm_prescale_kernel<float>, (int)std::min<size_t>((cn + 255) / 256, 4096), 256, 0, s, C, cn, beta);
-        }
-    }
-    dim3 grid(gi, gj, batch * splits);
-    if (grid.y > 65535 || grid.z > 65535) return hipErrorInvalidValue;
-    if (si && sj) hipLaunchKernelGGL((gemm2_f32_mfma_kernel<A_IFAST, B_KFAST, 64, 64>), grid, 256, 0, s, M, N, K, alpha, A, B, beta, C, st, splits, kChunk, splits > 1 ? nullptr : causalFlag, epoch);
-    else if (si) hipLaunchKernelGGL((gemm2_f32_mfma_kernel<A_IFAST, B_KFAST, 64, 128>), grid, 256, 0, s, M, N, K, alpha, A, B, beta, C, st, splits, kChunk, splits > 1 ? nullptr : causalFlag, epoch);
-    else if (sj) hipLaunchKernelGGL((gemm2_f32_mfma_kernel<A_IFAST, B_KFAST, 128, 64>), grid, 256, 0, s, M, N, K, alpha, A, B, beta, C, st, splits, kChunk, splits > 1 ? nullptr : causalFlag, epoch);
-    else hipLaunchKernelGGL((gemm2_f32_mfma_kernel<A_IFAST, B_KFAST, 128, 128>), grid, 256, 0, s, M, N, K, alpha, A, B, beta, C, st, splits, kChunk, splits > 1 ? nullptr : causalFlag, epoch);
-    return hipGetLastError();
-}
-
 hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float alpha, const float* A, const float* B,
                    float beta, float* C, int lda, int ldb, int ldc, long long sA, long long sB, long long sC, int batch,
                    const int* causalFlag, int epoch, bool skipAboveDiagonal)
@@ -1773,23 +1321,23 @@ hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float a
     st.ci = 1;             st.cj = ldc;
     st.sA = sA; st.sB = sB; st.sC = sC;
     if (m <= 0 || n <= 0 || batch <= 0) return hipSuccess;
-    // MFMA path: every float4 the staging loads must be aligned and whole (the unit-stride extent a multiple of 4)
     const bool aligned = ((((uintptr_t)A | (uintptr_t)B) & 15) == 0) && lda % 4 == 0 && ldb % 4 == 0 && sA % 4 == 0 && sB % 4 == 0;
-    const bool aOk = tA ? (k % 4 == 0) : (m % 4 == 0);
-    const bool bOk = tB ? (n % 4 == 0) : (k % 4 == 0);
-    if (aligned && aOk && bOk && k > 0 && (long long)m * n >= 1024) {
-        if (!tA && !tB && m >= 256 && n >= 128 && (long long)m * n * batch >= (1ll << 22)) {
-            // a short contraction over large matrices (Q K^T of the attention chain): the j panel stays in registers
-            if (k == 32) return launch_gemm2_panel<32>(s, m, n, alpha, A, B, beta, C, st, batch, skipAboveDiagonal);
-            if (k == 64) return launch_gemm2_panel<64>(s, m, n, alpha, A, B, beta, C, st, batch, skipAboveDiagonal);
-            if (k == 128) return launch_gemm2_panel<128>(s, m, n, alpha, A, B, beta, C, st, batch, skipAboveDiagonal);
-        }
-        if (!tA && !tB) return launch_gemm2_mfma<true, true>(s, m, n, k, alpha, A, B, beta, C, st, batch, causalFlag, epoch);
-        if (!tA && tB) return launch_gemm2_mfma<true, false>(s, m, n, k, alpha, A, B, beta, C, st, batch, causalFlag, epoch);
-        if (tA && !tB) return launch_gemm2_mfma<false, true>(s, m, n, k, alpha, A, B, beta, C, st, batch);
-        return launch_gemm2_mfma<false, false>(s, m, n, k, alpha, A, B, beta, C, st, batch);
+    if (!tA && !tB && aligned && m % 4 == 0 && k % 4 == 0 && m >= 256 && n >= 128 && (long long)m * n * batch >= (1ll << 22)) {
+        // a short contraction over large matrices (Q K^T of the attention chain): the j panel stays in registers
+        if (k == 32) return launch_gemm2_panel<32>(s, m, n, alpha, A, B, beta, C, st, batch, skipAboveDiagonal);
+        if (k == 64) return launch_gemm2_panel<64>(s, m, n, alpha, A, B, beta, C, st, batch, skipAboveDiagonal);
+        if (k == 128) return launch_gemm2_panel<128>(s, m, n, alpha, A, B, beta, C, st, batch, skipAboveDiagonal);
     }
-    return launch_generic<float>(s, m, n, k, alpha, A, B, beta, C, st, batch);
+    if (k <= 0 || gemm_is_tiny(m, n, k)) return launch_generic<float>(s, m, n, k, alpha, A, B, beta, C, st, batch);
+    // column-major C = op(A) op(B) is row-major C^T = op(B)^T op(A)^T
+    GemmF32 g = {};
+    g.m = n; g.n = m; g.k = k;
+    g.A = B; g.B = A; g.C = C;
+    g.lda = ldb; g.ldb = lda; g.ldc = ldc; g.sA = sB; g.sB = sA; g.sC = sC;
+    g.aK = !tB; g.bK = tA;
+    g.alpha = alpha; g.beta = beta; g.batch = batch;
+    if (causalFlag) { g.causal = tB ? CAUSAL_UPPER : CAUSAL_LOWER; g.flag = causalFlag; g.epoch = epoch; }
+    return gemm_f32(s, g, nullptr, 0);
 }
 
 // ---------------------------------------------------------------------------

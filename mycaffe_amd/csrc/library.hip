@@ -329,7 +329,10 @@ long Kernel::flush_pending_product(bool causal)
     MemItem *A, *B, *C;
     if (m_mem.get(p.hA, &A) || m_mem.get(p.hB, &B) || m_mem.get(p.hC, &C)) return 0;   // an operand is gone
     if (p.kind == 1) {
-        HIPCHK(k_gemm(m_stream, F32, false, true, p.m, p.n, p.k, p.alpha, A->ptr, B->ptr, 0.f, C->ptr));
+        void* ws = nullptr;
+        const size_t wsb = k_gemm_workspace_bytes(F32, false, true, p.m, p.n, p.k);
+        if (wsb) ERRCHK(workspace(wsb, &ws));
+        HIPCHK(k_gemm(m_stream, F32, false, true, p.m, p.n, p.k, p.alpha, A->ptr, B->ptr, 0.f, C->ptr, ws, wsb));
         return 0;
     }
     HIPCHK(k_gemm2(m_stream, false, false, p.m, p.n, p.k, p.alpha, (const float*)A->ptr, (const float*)B->ptr, 0.f, (float*)C->ptr,
@@ -783,8 +786,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 if (!m_mem.get(p.hA, &X) && !m_mem.get(p.hB, &W) && !m_mem.get(p.hC, &C)) {
                     m_pendingProduct = PendingProduct();
                     void* ws = nullptr;
-                    if (k_gemm_bias_needs_tmp(F32, p.n, p.k, X->ptr, W->ptr, C->ptr)) ERRCHK(workspace((size_t)p.m * p.n * 4, &ws));
-                    HIPCHK(k_gemm_bias(s, F32, p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws));
+                    const size_t wsb = k_gemm_bias_workspace_bytes(F32, p.m, p.n, p.k, X->ptr, W->ptr, C->ptr);
+                    if (wsb) ERRCHK(workspace(wsb, &ws));
+                    HIPCHK(k_gemm_bias(s, F32, p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws, wsb));
                     m_mem.touch(hC);
                     return 0;
                 }
@@ -804,11 +808,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             RANGE(A, aOff, (long long)m * k);
             RANGE(B, bOff, (long long)k * n);
             if (m_pendingProduct.hC == hC) m_pendingProduct = PendingProduct();
-            // Y = X W^T of an inner product layer, large enough for the saved pass to matter and not one whose contraction
-            // the library would split over workgroups (that sum has another order than the fused launch's)
+            // Y = X W^T of an inner product layer, large enough for the saved pass to matter
             if (!timing && !tA && tB && !A->half && pf[0] == 1.f && aOff == 0 && bOff == 0 && m >= 256 && n >= 64 && k >= 32 &&
-                (long long)m * n >= (1ll << 20) && !A->view && !B->view && !A->exposed && !B->exposed && !C->exposed &&
-                k_gemm_workspace_bytes(F32, false, true, m, n, k) == 0) {
+                (long long)m * n >= (1ll << 20) && !A->view && !B->view && !A->exposed && !B->exposed && !C->exposed) {
                 if (m_pendingProduct.hC) ERRCHK(flush_pending_product());   // one at a time
                 PendingProduct& pp = m_pendingProduct;
                 pp.kind = 1; pp.hA = hA; pp.hB = hB; pp.hC = hC; pp.m = m; pp.n = n; pp.k = k; pp.alpha = 1.f;
@@ -2003,10 +2005,10 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             }
         }
         void* ws = nullptr;
-        if (k_gemm_qkv_heads_needs_tmp(X->dt(), (int)H, (int)hs, X->ptr, W->ptr, Q->ptr, K->ptr, V->ptr))
-            ERRCHK(workspace((size_t)(M * 3 * C) * X->esize(), &ws));
+        const size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Q->ptr, K->ptr, V->ptr);
+        if (wsb) ERRCHK(workspace(wsb, &ws));
         HIPCHK(k_gemm_qkv_heads(s, X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Q->ptr, K->ptr,
-                                V->ptr, ws, r ? (const float*)r->dcos.get() : nullptr, r ? (const float*)r->dsin.get() : nullptr,
+                                V->ptr, ws, wsb, r ? (const float*)r->dcos.get() : nullptr, r ? (const float*)r->dsin.get() : nullptr,
                                 r ? r->seq : 0));
         m_mem.touch((long)pl[7]);
         m_mem.touch((long)pl[8]);
@@ -2030,8 +2032,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
         void* ws = nullptr;
-        if (k_gemm_bias_needs_tmp(X->dt(), (int)N, (int)K, X->ptr, W->ptr, Y->ptr)) ERRCHK(workspace((size_t)(M * N) * X->esize(), &ws));
-        HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws));
+        const size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Y->ptr);
+        if (wsb) ERRCHK(workspace(wsb, &ws));
+        HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
         m_mem.touch((long)pl[6]);
         return 0;
     }
