@@ -94,30 +94,159 @@ __global__ void d_mask_kernel(size_t n, size_t md1, size_t dd1, const double* x,
     GRID_STRIDE(i, n) y[i] = mask[i % md1 + (i / dd1) * md1] == search ? replace : x[i];
 }
 
-// C(i,j) = alpha sum_k A(i,k) B(k,j) + beta C(i,j) for any element strides (row-major GEMM and column-major GEMM2 alike),
-// batched over blockIdx.z.  16 x 16 outputs per workgroup, K in slices of 16 through LDS.
-__global__ __launch_bounds__(256) void d_gemm_kernel(int m, int n, int k, double alpha, const double* A, long long ars, long long acs,
-                                                     const double* B, long long brs, long long bcs, double beta, double* C,
-                                                     long long crs, long long ccs, long long sA, long long sB, long long sC)
+// C(i,j) = alpha sum_k A(i,k) B(k,j) + beta C(i,j) with any element strides, on the double matrix cores
+// (v_mfma_f64_16x16x4_f64: lane l holds A(l % 16, l / 16) and B(l / 16, l % 16) of a step, register v of the result is row
+// 4 v + l / 16, column l % 16).  2 x 2 wavefronts of W x W MFMA tiles each, stages of 16 k double-buffered in LDS as
+// [row][k] with 18 doubles a row (conflict-free 64-bit reads), the next stage held in registers meanwhile.  An operand is
+// fetched along whichever index lies at unit stride.
+// The layers of this type are small: a product is some dozens of tiles and what bounds it is the latency of one stage after
+// the other.  G groups of four wavefronts of a workgroup therefore take every G-th stage each, with stages of their own, and
+// their sums are added in order through LDS at the end (256 x 256 x 1024: 27 us with one group, 9 us with four; one output
+// per thread took 45 us).
+// zdiv: matrix z of C lies at (z / zdiv) sC + (z % zdiv) sC2.
+typedef double d_vec4 __attribute__((ext_vector_type(4)));
+struct GemmD { int m, n, k; double alpha, beta; const double *A, *B; double* C; long long ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2; int zdiv; };
+template <int W, int G> __global__ __launch_bounds__(256 * G) void d_gemm_kernel(GemmD g)
 {
-    __shared__ double as[16][17], bs[16][17];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int i = blockIdx.y * 16 + ty, j = blockIdx.x * 16 + tx;
-    A += (size_t)blockIdx.z * sA;
-    B += (size_t)blockIdx.z * sB;
-    C += (size_t)blockIdx.z * sC;
-    double acc = 0.0;
-    for (int k0 = 0; k0 < k; k0 += 16) {
-        as[ty][tx] = (i < m && k0 + tx < k) ? A[(long long)i * ars + (long long)(k0 + tx) * acs] : 0.0;
-        bs[ty][tx] = (k0 + ty < k && j < n) ? B[(long long)(k0 + ty) * brs + (long long)j * bcs] : 0.0;
-        __syncthreads();
+    constexpr int BT = 32 * W, BK = 16, LD = BK + 2, NE = BT * BK / 256, STAGE = 2 * BT * LD;
+    extern __shared__ double d_smem[];
+    const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+    double* stages = d_smem + group * 2 * STAGE;   // two of this group
+    const int m0 = blockIdx.y * BT, n0 = blockIdx.x * BT, wm = (wave >> 1) * 16 * W, wn = (wave & 1) * 16 * W;
+    const double* A = g.A + (size_t)blockIdx.z * g.sA;
+    const double* B = g.B + (size_t)blockIdx.z * g.sB;
+    double* C = g.C + (size_t)(blockIdx.z / g.zdiv) * g.sC + (size_t)(blockIdx.z % g.zdiv) * g.sC2;
+    const bool ak = g.acs == 1, bk = g.brs == 1;
+    d_vec4 acc[W][W];
 #pragma unroll
-        for (int kk = 0; kk < 16; kk++) acc += as[ty][kk] * bs[kk][tx];
+    for (int i = 0; i < W; i++)
+#pragma unroll
+        for (int j = 0; j < W; j++) acc[i][j] = d_vec4{0.0, 0.0, 0.0, 0.0};
+    double ra[NE], rb[NE];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < NE; q++) {
+            const int e = tid + 256 * q;
+            const int ia = ak ? e / BK : e % BT, ka = ak ? e % BK : e / BT;
+            const int jb = bk ? e / BK : e % BT, kb = bk ? e % BK : e / BT;
+            ra[q] = (m0 + ia < g.m && k0 + ka < g.k) ? A[(long long)(m0 + ia) * g.ars + (long long)(k0 + ka) * g.acs] : 0.0;
+            rb[q] = (n0 + jb < g.n && k0 + kb < g.k) ? B[(long long)(k0 + kb) * g.brs + (long long)(n0 + jb) * g.bcs] : 0.0;
+        }
+    };
+    auto put = [&](int buf) {
+        double *as = stages + buf * STAGE, *bs = as + BT * LD;
+#pragma unroll
+        for (int q = 0; q < NE; q++) {
+            const int e = tid + 256 * q;
+            as[ak ? (e / BK) * LD + e % BK : (e % BT) * LD + e / BT] = ra[q];
+            bs[bk ? (e / BK) * LD + e % BK : (e % BT) * LD + e / BT] = rb[q];
+        }
+    };
+    // trips are the same for every group: stages past the end are zeros
+    const int trips = (g.k + BK * G - 1) / (BK * G), fr = lane & 15, fk = lane >> 4;
+    fetch(group * BK);
+    put(0);
+    __syncthreads();
+    for (int kt = 0; kt < trips; kt++) {
+        const double *as = stages + (kt & 1) * STAGE, *bs = as + BT * LD;
+        if (kt + 1 < trips) fetch(((kt + 1) * G + group) * BK);
+#pragma unroll
+        for (int kk = 0; kk < BK; kk += 4) {
+            double a[W], b[W];
+#pragma unroll
+            for (int t = 0; t < W; t++) {
+                a[t] = as[(wm + 16 * t + fr) * LD + kk + fk];
+                b[t] = bs[(wn + 16 * t + fr) * LD + kk + fk];
+            }
+#pragma unroll
+            for (int i = 0; i < W; i++)
+#pragma unroll
+                for (int j = 0; j < W; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if (kt + 1 < trips) put((kt & 1) ^ 1);
         __syncthreads();
     }
-    if (i < m && j < n) {
-        double* c = C + (long long)i * crs + (long long)j * ccs;
-        *c = beta == 0.0 ? alpha * acc : alpha * acc + beta * *c;
+    if (G > 1) {
+        // group q > 0 leaves its sums at [q - 1][register][thread]; group 0 adds them
+        constexpr int NR = W * W * 4;
+        if (group > 0) {
+#pragma unroll
+            for (int i = 0; i < W; i++)
+#pragma unroll
+                for (int j = 0; j < W; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) d_smem[((group - 1) * NR + (i * W + j) * 4 + v) * 256 + tid] = acc[i][j][v];
+        }
+        __syncthreads();
+        if (group > 0) return;
+        for (int q = 0; q < G - 1; q++)
+#pragma unroll
+            for (int i = 0; i < W; i++)
+#pragma unroll
+                for (int j = 0; j < W; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc[i][j][v] += d_smem[(q * NR + (i * W + j) * 4 + v) * 256 + tid];
+    }
+#pragma unroll
+    for (int i = 0; i < W; i++)
+#pragma unroll
+        for (int j = 0; j < W; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = m0 + wm + 16 * i + 4 * v + fk, c = n0 + wn + 16 * j + fr;
+                if (r >= g.m || c >= g.n) continue;
+                double* cp = C + (long long)r * g.crs + (long long)c * g.ccs;
+                const double t = g.alpha * acc[i][j][v];
+                *cp = g.beta == 0.0 ? t : t + g.beta * *cp;
+            }
+}
+// 64 x 64 tiles once they give every CU one, 32 x 32 below; four groups while the workgroups leave CUs to spare (two of
+// them fit a CU) and the contraction has stages for them
+static hipError_t d_gemm(hipStream_t s, int batch, int m, int n, int k, double alpha, const double* A, long long ars, long long acs, const double* B,
+                         long long brs, long long bcs, double beta, double* C, long long crs, long long ccs, long long sA, long long sB, long long sC,
+                         int zdiv = 1, long long sC2 = 0)
+{
+    GemmD g = {m, n, k, alpha, beta, A, B, C, ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2, zdiv};
+    const long long big = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch, small = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch;
+    const dim3 gridBig((n + 63) / 64, (m + 63) / 64, batch), gridSmall((n + 31) / 32, (m + 31) / 32, batch);
+    if (gridSmall.y > 65535) return hipErrorInvalidValue;
+    if (big >= 256) hipLaunchKernelGGL((d_gemm_kernel<2, 1>), gridBig, 256, 2 * 2 * 64 * 18 * 8, s, g);
+    else if (small <= 512 && k >= 128) {
+        constexpr int lds = 4 * 2 * 2 * 32 * 18 * 8;
+        static const hipError_t attr = hipFuncSetAttribute((const void*)d_gemm_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (attr != hipSuccess) return attr;
+        hipLaunchKernelGGL((d_gemm_kernel<1, 4>), gridSmall, 1024, lds, s, g);
+    } else hipLaunchKernelGGL((d_gemm_kernel<1, 1>), gridSmall, 256, 2 * 2 * 32 * 18 * 8, s, g);
+    return hipGetLastError();
+}
+// y (n) = alpha A^T x + beta y, A row-major (m, n): 16 columns by 64 rows a trip, sums of the 64 row lanes added in order
+__global__ __launch_bounds__(1024) void d_gemv_t_kernel(int m, int n, double alpha, const double* A, const double* x, double beta, double* y)
+{
+    __shared__ double red[64][17];
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4, j = blockIdx.x * 16 + c;
+    double acc = 0.0;
+    if (j < n)
+        for (int i = r; i < m; i += 64) acc += A[(size_t)i * n + j] * x[i];
+    red[r][c] = acc;
+    __syncthreads();
+    if (r == 0 && j < n) {
+        double t = 0.0;
+        for (int q = 0; q < 64; q++) t += red[q][c];
+        t *= alpha;
+        y[j] = beta == 0.0 ? t : t + beta * y[j];
+    }
+}
+// y (m) = alpha A x + beta y: one wavefront a row
+__global__ __launch_bounds__(256) void d_gemv_n_kernel(int m, int n, double alpha, const double* A, const double* x, double beta, double* y)
+{
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= m) return;
+    double acc = 0.0;
+    for (int j = lane; j < n; j += 64) acc += A[(size_t)row * n + j] * x[j];
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (lane == 0) {
+        acc *= alpha;
+        y[row] = beta == 0.0 ? acc : acc + beta * y[row];
     }
 }
 
@@ -192,24 +321,47 @@ __global__ void d_spread_kernel(int mode, size_t n, size_t spatial, size_t perio
     }
 }
 // y[row] = scale * sum of the row's `inner` values, one thread per row (channel_mean, channel_sum within a channel)
-__global__ void d_rowsum_kernel(size_t rows, int inner, const double* x, double* y, double scale)
+// one wavefront a row; with a: the sum of the products x a
+__global__ __launch_bounds__(256) void d_rowsum_kernel(size_t rows, int inner, const double* x, const double* a, double* y, double scale)
 {
-    GRID_STRIDE(r, rows)
-    {
-        double acc = 0.0;
-        for (int i = 0; i < inner; i++) acc += x[r * inner + i];
-        y[r] = acc * scale;
+    const size_t r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= rows) return;
+    const int lane = threadIdx.x & 63;
+    double acc = 0.0;
+    for (int i = lane; i < inner; i += 64) acc += a ? x[r * inner + i] * a[r * inner + i] : x[r * inner + i];
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (lane == 0) y[r] = acc * scale;
+}
+static void d_rowsum(hipStream_t s, size_t rows, int inner, const double* x, const double* a, double* y, double scale)
+{
+    hipLaunchKernelGGL(d_rowsum_kernel, (unsigned)((rows + 3) / 4), 256, 0, s, rows, inner, x, a, y, scale);
+}
+// y[n, s] = sum over c of x[n, c, s] (math.cu:6945-6980), or of x a (channel_dot, math.cu:7335-7351): 16 columns by 64
+// channels a trip, the sums of the 64 lanes added in order
+__global__ __launch_bounds__(1024) void d_colsum_kernel(int channels, int spatial, const double* x, const double* a, double* y)
+{
+    __shared__ double red[64][17];
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4, sp = blockIdx.x * 16 + c;
+    const size_t base = (size_t)blockIdx.y * channels * spatial + sp;
+    double acc = 0.0;
+    if (sp < spatial)
+        for (int ch = r; ch < channels; ch += 64) acc += a ? x[base + (size_t)ch * spatial] * a[base + (size_t)ch * spatial] : x[base + (size_t)ch * spatial];
+    red[r][c] = acc;
+    __syncthreads();
+    if (r == 0 && sp < spatial) {
+        double t = 0.0;
+        for (int q = 0; q < 64; q++) t += red[q][c];
+        y[(size_t)blockIdx.y * spatial + sp] = t;
     }
 }
-// y[n, s] = sum over c of x[n, c, s] (math.cu:6945-6980), or of x a (channel_dot, math.cu:7335-7351)
-__global__ void d_colsum_kernel(size_t rows, int channels, int spatial, const double* x, const double* a, double* y)
+// outer tensors; a last axis (spatial 1) is a sum of rows
+static void d_colsum(hipStream_t s, size_t outer, int channels, int spatial, const double* x, const double* a, double* y)
 {
-    GRID_STRIDE(i, rows)
-    {
-        const size_t n = i / spatial, sp = i % spatial, base = n * channels * (size_t)spatial + sp;
-        double acc = 0.0;
-        for (int c = 0; c < channels; c++) acc += a ? x[base + (size_t)c * spatial] * a[base + (size_t)c * spatial] : x[base + (size_t)c * spatial];
-        y[i] = acc;
+    if (spatial == 1) { d_rowsum(s, outer, channels, x, a, y, 1.0); return; }
+    for (size_t o = 0; o < outer; o += 65535) {
+        const size_t n = outer - o < 65535 ? outer - o : 65535, at = o * channels * (size_t)spatial;
+        hipLaunchKernelGGL(d_colsum_kernel, dim3((spatial + 15) / 16, (unsigned)n), 1024, 0, s, channels, spatial, x + at, a ? a + at : nullptr,
+                           y + o * spatial);
     }
 }
 // channel_max across channels or within one, value or first index (math.cu:6697-6810); starts from -DBL_MAX
@@ -333,24 +485,50 @@ __global__ __launch_bounds__(256) void d_rmsnorm_kernel(int dim, const double* x
     const double inv = 1.0 / sqrt(d_block_reduce(ss, red, false) / dim + eps);
     for (int i = threadIdx.x; i < dim; i += 256) yr[i] = w ? w[i] * (inv * xr[i]) : inv * xr[i];
 }
-// dS = P (dP - sum_k P dP) per row, in place in dp (the softmax gradient of attn.cu:608-661)
-__global__ __launch_bounds__(256) void d_attn_ds_kernel(const double* p, double* dp, int Tk)
+// dS = P (dP - sum_k P dP) per row, in place in dp (the softmax gradient of attn.cu:608-661); one wavefront a row
+__global__ __launch_bounds__(256) void d_attn_ds_kernel(size_t rows, const double* p, double* dp, int Tk)
 {
-    __shared__ double red[4];
-    const size_t base = (size_t)blockIdx.x * Tk;
+    const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const size_t base = row * Tk;
+    const int lane = threadIdx.x & 63;
     double sum = 0.0;
-    for (int j = threadIdx.x; j < Tk; j += 256) sum += p[base + j] * dp[base + j];
-    sum = d_block_reduce(sum, red, false);
-    for (int j = threadIdx.x; j < Tk; j += 256) dp[base + j] = p[base + j] * (dp[base + j] - sum);
+    for (int j = lane; j < Tk; j += 64) sum += p[base + j] * dp[base + j];
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    for (int j = lane; j < Tk; j += 64) dp[base + j] = p[base + j] * (dp[base + j] - sum);
+}
+// softmax over the keys of the scaled scores p (B, H, Tq, Tk), in place, masked ones -1e29 (kinds as below); one wavefront a row
+__global__ __launch_bounds__(256) void d_attn_softmax_kernel(size_t rows, double* p, int H, int Tq, int Tk, const double* mask, int kind)
+{
+    const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int lane = threadIdx.x & 63, t = (int)(row % Tq);
+    const size_t b = row / Tq / H;
+    const double* mrow = kind == 1 ? mask + (size_t)t * Tk : kind == 2 ? mask + b * Tk : kind == 3 ? mask + (b * Tq + t) * Tk : nullptr;
+    p += row * Tk;
+    double mx = -INFINITY;
+    for (int j = lane; j < Tk; j += 64) {
+        const double s = mrow && mrow[j] == 0.0 ? -1e29 : p[j];
+        p[j] = s;
+        mx = fmax(mx, s);
+    }
+    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+    double sum = 0.0;
+    for (int j = lane; j < Tk; j += 64) {
+        const double e = exp(p[j] - mx);
+        p[j] = e;
+        sum += e;
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    for (int j = lane; j < Tk; j += 64) p[j] /= sum;
 }
 
 // Attention forward as the reference's chain computes it (attn.cu:518-602): scores = scale q . k, masked ones -1e29,
 // softmax over the keys, y = p V.  One workgroup per (sequence, head, query row); the row of probabilities stays in LDS.
 // kind 0: no mask, 1: mask (Tq,Tk), 2: mask (B,Tk), 3: mask (B,Tq,Tk); merged: y written (B,Tq,H,hs)
-// probs != nullptr: the row's probabilities are written there as well (B, H, Tq, Tk) and y may be null (the backward pass)
+// Used where the probabilities of all rows are too many to keep.
 __global__ __launch_bounds__(256) void d_attn_row_kernel(const double* q, const double* k, const double* v, double* y, int H, int Tq,
-                                                         int Tk, int hs, double scale, const double* mask, int kind, bool merged,
-                                                         double* probs)
+                                                         int Tk, int hs, double scale, const double* mask, int kind, bool merged)
 {
     extern __shared__ double d_smem[];
     double* p = d_smem;        // Tk
@@ -387,9 +565,6 @@ __global__ __launch_bounds__(256) void d_attn_row_kernel(const double* q, const 
         sum += e;
     }
     sum = d_block_reduce(sum, red, false);
-    if (probs)
-        for (int j = threadIdx.x; j < Tk; j += 256) probs[row * Tk + j] = p[j] / sum;
-    if (!y) return;
     double* yr = merged ? y + ((b * Tq + t) * H + h) * (size_t)hs : y + row * hs;
     for (int d = threadIdx.x; d < hs; d += 256) {
         double acc = 0.0;
@@ -499,7 +674,11 @@ __global__ void d_qkv_split_kernel(size_t pairs, const double* tmp, const double
 __global__ void d_add_bias_rows_kernel(size_t n, int N, const double* bias, double* y) { GRID_STRIDE(i, n) y[i] += bias[i % N]; }
 
 // ---- the kernel object --------------------------------------------------------------------------------------------
-struct MemD { double* ptr = nullptr; size_t count = 0; bool used = false; long base = 0; };   // base != 0: a view into that handle's allocation
+struct MemD {
+    double* ptr = nullptr; size_t count = 0; bool used = false; long base = 0;   // base != 0: a view into that handle's allocation
+    // of an allocation: changes whenever a call could have written it, and never repeats; exposed: its address was handed out
+    uint64_t version = 0; bool exposed = false;
+};
 struct AttnD { bool set = false; int batch = 0, block = 0, heads = 0, hs = 0; double scale = 1.0;
                int lastTq = 0, lastTk = 0; long long lastBatchMask = 0; long lastMask = 0; };   // of the last forward call
 struct LayerNormD { bool set = false; int count = 0, outer = 0, channels = 0, inner = 0, backwards = 0; double eps = 1e-10; double* stdev = nullptr;
@@ -548,6 +727,7 @@ public:
     {
         MemD* it;
         ERRCHK(mem(h, &it));
+        m_mem[it->base ? it->base : h].exposed = true;
         *pp = it->ptr;
         return 0;
     }
@@ -559,6 +739,16 @@ private:
     {
         if (h <= 0 || (size_t)h >= m_mem.size() || !m_mem[h].used) return MCH_ERROR_MEMORY_NOT_FOUND;
         *it = &m_mem[h];
+        m_mem[(*it)->base ? (*it)->base : h].version = ++m_clock;
+        return 0;
+    }
+    // for reading only: (root, version) name the contents; version 0: they can change without a call
+    long mem_read(long h, MemD** it, long* root, uint64_t* version)
+    {
+        if (h <= 0 || (size_t)h >= m_mem.size() || !m_mem[h].used) return MCH_ERROR_MEMORY_NOT_FOUND;
+        *it = &m_mem[h];
+        *root = (*it)->base ? (*it)->base : h;
+        *version = m_mem[*root].exposed ? 0 : m_mem[*root].version;
         return 0;
     }
     long alloc(size_t count, long* h)
@@ -569,7 +759,7 @@ private:
         if (e != hipSuccess) { (void)hipFree(p); return (long)e; }
         const size_t slot = new_slot();
         m_mem[slot] = MemD();
-        m_mem[slot].ptr = p; m_mem[slot].count = count; m_mem[slot].used = true;
+        m_mem[slot].ptr = p; m_mem[slot].count = count; m_mem[slot].used = true; m_mem[slot].version = ++m_clock;
         *h = (long)slot;
         return 0;
     }
@@ -597,6 +787,10 @@ private:
     int m_device = 0;
     hipStream_t m_stream = nullptr;
     std::vector<MemD> m_mem{1};
+    uint64_t m_clock = 0;
+    // decoded TRANSPOSE arguments by the contents of their three blobs: reading them back waits for the device (25 us a call)
+    struct PermuteCacheD { uint64_t key[9]; PermuteD args; };
+    std::vector<PermuteCacheD> m_permuteCache;
     std::vector<double*> m_host;
     HandleTable<CudnnState> m_cudnn;
     HandleTable<TensorDesc> m_tdesc;
@@ -612,6 +806,16 @@ private:
             m_wsCount = count;
         }
         *p = m_ws;
+        return 0;
+    }
+    // P (B, H, T, Tk) = softmax(mask(scale Q K^T))
+    long attn_probs(const double* Q, const double* K, double* P, const AttnD* st, int T, int Tk, const MemD* M, int kind)
+    {
+        const long long bh = (long long)st->batch * st->heads, rows = bh * T, hs = st->hs;
+        HIPCHK(d_gemm(m_stream, (int)bh, T, Tk, (int)hs, st->scale, Q, hs, 1ll, K, 1ll, hs, 0.0, P, Tk, 1ll, T * hs, Tk * hs, (long long)T * Tk));
+        hipLaunchKernelGGL(d_attn_softmax_kernel, (unsigned)((rows + 3) / 4), 256, 0, m_stream, (size_t)rows, P, st->heads, T, Tk,
+                           M ? (const double*)M->ptr : nullptr, kind);
+        HIPCHK(hipGetLastError());
         return 0;
     }
     long attn_mask_kind(AttnD* st, MemD* M, long long batchMask, int T, int Tk, int* kind)
@@ -772,7 +976,8 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         if (dofs < 0) dofs = 0;
         RANGE(src, so, n);
         RANGE(dst, dofs, n);
-        if (n) HIPCHK(hipMemcpyAsync(dst->ptr + dofs, src->ptr + so, (size_t)n * 8, hipMemcpyDeviceToDevice, s));
+        if (n) hipLaunchKernelGGL(d_scale_kernel, grid_of((size_t)n), 256, 0, s, (size_t)n, 1.0, (const double*)src->ptr + so, dst->ptr + dofs);
+        LAUNCHED();
         return 0;
     }
 
@@ -800,10 +1005,8 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
             RANGE(B, bo, (long long)k * n);
             RANGE(C, co, (long long)m * n);
             if (m == 0 || n == 0) continue;
-            hipLaunchKernelGGL(d_gemm_kernel, dim3((n + 15) / 16, (m + 15) / 16, 1), 256, 0, s, m, n, k, pf[0], A->ptr + ao,
-                               tA ? 1ll : (long long)k, tA ? (long long)m : 1ll, B->ptr + bo, tB ? 1ll : (long long)n,
-                               tB ? (long long)k : 1ll, pf[1], C->ptr + co, (long long)n, 1ll, 0ll, 0ll, 0ll);
-            LAUNCHED();
+            HIPCHK(d_gemm(s, 1, m, n, k, pf[0], A->ptr + ao, tA ? 1ll : (long long)k, tA ? (long long)m : 1ll, B->ptr + bo, tB ? 1ll : (long long)n,
+                          tB ? (long long)k : 1ll, pf[1], C->ptr + co, (long long)n, 1ll, 0ll, 0ll, 0ll));
         }
         return 0;
     }
@@ -830,9 +1033,8 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(B, 0, (batch - 1) * sB + (bc - 1) * ldb + br);
         RANGE(C, 0, (batch - 1) * sC + (long long)(n - 1) * ldc + m);
         // column-major: element (i, kk) of op(A) is A[i + kk lda], or A[kk + i lda] when transposed
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((n + 15) / 16, (m + 15) / 16, batch), 256, 0, s, m, n, k, pf[0], A->ptr,
-                           tA ? lda : 1ll, tA ? 1ll : lda, B->ptr, tB ? ldb : 1ll, tB ? 1ll : ldb, pf[1], C->ptr, 1ll, ldc, sA, sB, sC);
-        LAUNCHED();
+        HIPCHK(d_gemm(s, batch, m, n, k, pf[0], A->ptr, tA ? lda : 1ll, tA ? 1ll : lda, B->ptr, tB ? ldb : 1ll, tB ? 1ll : ldb, pf[1], C->ptr, 1ll,
+                      ldc, sA, sB, sC));
         return 0;
     }
     case MCH_FN_GEMV: {
@@ -853,11 +1055,9 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(A, aOff, (long long)m * n);
         RANGE(X, xOff, tA ? m : n);
         RANGE(Y, yOff, tA ? n : m);
-        const int rows = tA ? n : m, inner = tA ? m : n;   // y (rows) = op(A) (rows x inner) x (inner)
-        if (rows == 0) return 0;
-        hipLaunchKernelGGL(d_gemm_kernel, dim3(1, (rows + 15) / 16, 1), 256, 0, s, rows, 1, inner, pf[0], A->ptr + aOff,
-                           tA ? 1ll : (long long)n, tA ? (long long)n : 1ll, X->ptr + xOff, 1ll, 1ll, pf[1], Y->ptr + yOff, 1ll, 1ll,
-                           0ll, 0ll, 0ll);
+        if (tA ? n == 0 : m == 0) return 0;
+        if (tA) hipLaunchKernelGGL(d_gemv_t_kernel, (n + 15) / 16, 1024, 0, s, m, n, pf[0], A->ptr + aOff, X->ptr + xOff, pf[1], Y->ptr + yOff);
+        else hipLaunchKernelGGL(d_gemv_n_kernel, (m + 3) / 4, 256, 0, s, m, n, pf[0], A->ptr + aOff, X->ptr + xOff, pf[1], Y->ptr + yOff);
         LAUNCHED();
         return 0;
     }
@@ -971,25 +1171,43 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         MemD *X, *Y, *XC, *YC, *MP;
         ERRCHK(mem((long)pl[1], &X));
         ERRCHK(mem((long)pl[2], &Y));
-        ERRCHK(mem((long)pl[3], &XC));
-        ERRCHK(mem((long)pl[4], &YC));
-        ERRCHK(mem((long)pl[5], &MP));
+        PermuteCacheD e = {};
+        MemD** blobs[3] = {&XC, &YC, &MP};
+        bool known = true;
+        for (int i = 0; i < 3; i++) {
+            long root;
+            ERRCHK(mem_read((long)pl[3 + i], blobs[i], &root, &e.key[3 * i + 1]));
+            e.key[3 * i] = (uint64_t)root;
+            e.key[3 * i + 2] = (uint64_t)((*blobs[i])->ptr - m_mem[root].ptr);
+            known = known && e.key[3 * i + 1] != 0;
+        }
         if (axes < 1 || axes > 8) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         RANGE(X, 0, n);
         RANGE(Y, 0, n);
         RANGE(XC, 0, axes);
         RANGE(YC, 0, axes);
         RANGE(MP, 0, axes);
-        double hx[8], hy[8], hm[8];
-        HIPCHK(hipMemcpyAsync(hx, XC->ptr, axes * 8, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(hy, YC->ptr, axes * 8, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(hm, MP->ptr, axes * 8, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
         PermuteD a;
-        a.axes = axes;
-        for (int i = 0; i < axes; i++) {
-            a.xs[i] = (long long)hx[i]; a.ys[i] = (long long)hy[i]; a.map[i] = (int)hm[i];
-            if (a.xs[i] < 1 || a.ys[i] < 1 || a.map[i] < 0 || a.map[i] >= axes) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        a.axes = 0;
+        if (known)
+            for (const PermuteCacheD& c : m_permuteCache)
+                if (c.args.axes == axes && memcmp(c.key, e.key, sizeof(e.key)) == 0) { a = c.args; break; }
+        if (!a.axes) {
+            double hx[8], hy[8], hm[8];
+            HIPCHK(hipMemcpyAsync(hx, XC->ptr, axes * 8, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipMemcpyAsync(hy, YC->ptr, axes * 8, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipMemcpyAsync(hm, MP->ptr, axes * 8, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            a.axes = axes;
+            for (int i = 0; i < axes; i++) {
+                a.xs[i] = (long long)hx[i]; a.ys[i] = (long long)hy[i]; a.map[i] = (int)hm[i];
+                if (a.xs[i] < 1 || a.ys[i] < 1 || a.map[i] < 0 || a.map[i] >= axes) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+            }
+            if (known) {
+                e.args = a;
+                if (m_permuteCache.size() >= 64) m_permuteCache.erase(m_permuteCache.begin());
+                m_permuteCache.push_back(e);
+            }
         }
         if (n) hipLaunchKernelGGL(d_permute_kernel, grid_of((size_t)n), 256, 0, s, (size_t)n, X->ptr, Y->ptr, a);
         LAUNCHED();
@@ -1398,8 +1616,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         ERRCHK(mem((long)pl[5], &Y));
         RANGE(X, xo, outer * ch * inner);
         RANGE(Y, 0, outer * ch);
-        if (outer * ch) hipLaunchKernelGGL(d_rowsum_kernel, grid_of((size_t)(outer * ch)), 256, 0, s, (size_t)(outer * ch), (int)inner,
-                                           (const double*)X->ptr + xo, Y->ptr, 1.0 / (double)inner);
+        if (outer * ch) d_rowsum(s, (size_t)(outer * ch), (int)inner, (const double*)X->ptr + xo, nullptr, Y->ptr, 1.0 / (double)inner);
         LAUNCHED();
         return 0;
     }
@@ -1459,8 +1676,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(X, 0, outer * ch * inner);
         RANGE(A, 0, outer * ch * inner);
         RANGE(Y, 0, outer * inner);
-        if (outer * inner) hipLaunchKernelGGL(d_colsum_kernel, grid_of((size_t)(outer * inner)), 256, 0, s, (size_t)(outer * inner), (int)ch, (int)inner,
-                                              (const double*)X->ptr, (const double*)A->ptr, Y->ptr);
+        if (outer * inner) d_colsum(s, (size_t)outer, (int)ch, (int)inner, (const double*)X->ptr, (const double*)A->ptr, Y->ptr);
         LAUNCHED();
         return 0;
     }
@@ -1488,9 +1704,8 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         if (dir == 0) {
             if (X->ptr == Y->ptr) return MCH_ERROR_PARAM_OUT_OF_RANGE;
             if (reduced == 0) return 0;
-            if (across) hipLaunchKernelGGL(d_colsum_kernel, grid_of((size_t)reduced), 256, 0, s, (size_t)reduced, (int)ch, (int)inner, (const double*)X->ptr,
-                                           (const double*)nullptr, Y->ptr);
-            else hipLaunchKernelGGL(d_rowsum_kernel, grid_of((size_t)reduced), 256, 0, s, (size_t)reduced, (int)inner, (const double*)X->ptr, Y->ptr, 1.0);
+            if (across) d_colsum(s, (size_t)(reduced / inner), (int)ch, (int)inner, X->ptr, nullptr, Y->ptr);
+            else d_rowsum(s, (size_t)reduced, (int)inner, X->ptr, nullptr, Y->ptr, 1.0);
             LAUNCHED();
             return 0;
         }
@@ -1584,13 +1799,24 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
             return MCH_ERROR_ATTN_INCOMPATIBLE_BLOB_SIZE;
         int kind = 0;
         ERRCHK(attn_mask_kind(st, M, batchMask, T, Tk, &kind));
-        const size_t lds = ((size_t)Tk + st->hs) * sizeof(double);
-        if (lds > 60000) { last_detail = "the double attention call keeps a row of scores in LDS: up to about 7000 keys"; return MCH_ERROR_NOT_IMPLEMENTED; }
-        const long long rows = (long long)st->batch * st->heads * T;
-        if (rows > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
-        hipLaunchKernelGGL(d_attn_row_kernel, (int)rows, 256, lds, s, (const double*)Q->ptr, (const double*)K->ptr, (const double*)V->ptr,
-                           Y->ptr, st->heads, T, Tk, st->hs, st->scale, M ? (const double*)M->ptr : nullptr, kind, merged, (double*)nullptr);
-        LAUNCHED();
+        const long long bh = (long long)st->batch * st->heads, rows = bh * T, pn = rows * Tk;
+        if (bh <= 65535 && rows <= INT_MAX && pn <= (1ll << 28)) {
+            // scores, softmax and product as three launches, the probabilities in scratch memory
+            double* P;
+            ERRCHK(workspace((size_t)pn, &P));
+            ERRCHK(attn_probs(Q->ptr, K->ptr, P, st, T, Tk, M, kind));
+            const long long sp = (long long)T * Tk, sk = (long long)Tk * st->hs, hs = st->hs;
+            if (merged) HIPCHK(d_gemm(s, (int)bh, T, (int)hs, Tk, 1.0, P, Tk, 1ll, V->ptr, hs, 1ll, 0.0, Y->ptr, st->heads * hs, 1ll, sp, sk,
+                                      T * st->heads * hs, st->heads, hs));
+            else HIPCHK(d_gemm(s, (int)bh, T, (int)hs, Tk, 1.0, P, Tk, 1ll, V->ptr, hs, 1ll, 0.0, Y->ptr, hs, 1ll, sp, sk, T * hs));
+        } else {
+            const size_t lds = ((size_t)Tk + st->hs) * sizeof(double);
+            if (lds > 60000) { last_detail = "the double attention call keeps a row of scores in LDS: up to about 7000 keys"; return MCH_ERROR_NOT_IMPLEMENTED; }
+            if (rows > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+            hipLaunchKernelGGL(d_attn_row_kernel, (int)rows, 256, lds, s, (const double*)Q->ptr, (const double*)K->ptr, (const double*)V->ptr,
+                               Y->ptr, st->heads, T, Tk, st->hs, st->scale, M ? (const double*)M->ptr : nullptr, kind, merged);
+            LAUNCHED();
+        }
         st->lastTq = T; st->lastTk = Tk; st->lastBatchMask = batchMask; st->lastMask = (long)pl[6];
         return 0;
     }
@@ -1620,31 +1846,24 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
             return MCH_ERROR_ATTN_INCOMPATIBLE_BLOB_SIZE;
         int kind = 0;
         ERRCHK(attn_mask_kind(st, M, batchMask, T, Tk, &kind));
-        const size_t lds = ((size_t)Tk + hs) * sizeof(double);
         const long long rows = bh * T, pn = rows * Tk;
-        if (lds > 60000 || rows > INT_MAX || bh > 65535 || pn > (1ll << 28)) {
-            last_detail = "the double attention gradient keeps the probabilities of all rows: up to 2^28 of them, about 7000 keys a row";
+        if (rows > INT_MAX || bh > 65535 || pn > (1ll << 28)) {
+            last_detail = "the double attention gradient keeps the probabilities of all rows: up to 2^28 of them";
             return MCH_ERROR_NOT_IMPLEMENTED;
         }
         double* P;
         ERRCHK(workspace((size_t)pn * 2, &P));
         double* dP = P + pn;
-        hipLaunchKernelGGL(d_attn_row_kernel, (int)rows, 256, lds, s, (const double*)Q->ptr, (const double*)K->ptr, (const double*)V->ptr,
-                           (double*)nullptr, H, T, Tk, hs, st->scale, M ? (const double*)M->ptr : nullptr, kind, false, P);
-        LAUNCHED();
+        ERRCHK(attn_probs(Q->ptr, K->ptr, P, st, T, Tk, M, kind));
         const long long sq = (long long)T * hs, sk = (long long)Tk * hs, sp = (long long)T * Tk;
         // dV (Tk x hs) = P^T dY
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((hs + 15) / 16, (Tk + 15) / 16, (int)bh), 256, 0, s, Tk, hs, T, 1.0, (const double*)P, 1ll, (long long)Tk,
-                           (const double*)dY->ptr, (long long)hs, 1ll, 0.0, dV->ptr, (long long)hs, 1ll, sp, sq, sk);
+        HIPCHK(d_gemm(s, (int)bh, Tk, hs, T, 1.0, (const double*)P, 1ll, (long long)Tk, (const double*)dY->ptr, (long long)hs, 1ll, 0.0, dV->ptr, (long long)hs, 1ll, sp, sq, sk));
         // dP (T x Tk) = dY V^T
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((Tk + 15) / 16, (T + 15) / 16, (int)bh), 256, 0, s, T, Tk, hs, 1.0, (const double*)dY->ptr, (long long)hs, 1ll,
-                           (const double*)V->ptr, 1ll, (long long)hs, 0.0, dP, (long long)Tk, 1ll, sq, sk, sp);
-        hipLaunchKernelGGL(d_attn_ds_kernel, (int)rows, 256, 0, s, (const double*)P, dP, Tk);
+        HIPCHK(d_gemm(s, (int)bh, T, Tk, hs, 1.0, (const double*)dY->ptr, (long long)hs, 1ll, (const double*)V->ptr, 1ll, (long long)hs, 0.0, dP, (long long)Tk, 1ll, sq, sk, sp));
+        hipLaunchKernelGGL(d_attn_ds_kernel, (unsigned)((rows + 3) / 4), 256, 0, s, (size_t)rows, (const double*)P, dP, Tk);
         // dQ (T x hs) = scale dS K;  dK (Tk x hs) = scale dS^T Q
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((hs + 15) / 16, (T + 15) / 16, (int)bh), 256, 0, s, T, hs, Tk, st->scale, (const double*)dP, (long long)Tk, 1ll,
-                           (const double*)K->ptr, (long long)hs, 1ll, 0.0, dQ->ptr, (long long)hs, 1ll, sp, sk, sq);
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((hs + 15) / 16, (Tk + 15) / 16, (int)bh), 256, 0, s, Tk, hs, T, st->scale, (const double*)dP, 1ll, (long long)Tk,
-                           (const double*)Q->ptr, (long long)hs, 1ll, 0.0, dK->ptr, (long long)hs, 1ll, sp, sq, sk);
+        HIPCHK(d_gemm(s, (int)bh, T, hs, Tk, st->scale, (const double*)dP, (long long)Tk, 1ll, (const double*)K->ptr, (long long)hs, 1ll, 0.0, dQ->ptr, (long long)hs, 1ll, sp, sk, sq));
+        HIPCHK(d_gemm(s, (int)bh, Tk, hs, T, st->scale, (const double*)dP, 1ll, (long long)Tk, (const double*)Q->ptr, (long long)hs, 1ll, 0.0, dK->ptr, (long long)hs, 1ll, sp, sq, sk));
         LAUNCHED();
         return 0;
     }
@@ -1747,8 +1966,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(W, 0, N * K);
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((unsigned)((N + 15) / 16), (unsigned)((M + 15) / 16), 1), 256, 0, s, (int)M, (int)N, (int)K, 1.0,
-                           (const double*)X->ptr, K, 1ll, (const double*)W->ptr, 1ll, K, 0.0, Y->ptr, N, 1ll, 0ll, 0ll, 0ll);
+        HIPCHK(d_gemm(s, 1, (int)M, (int)N, (int)K, 1.0, (const double*)X->ptr, K, 1ll, (const double*)W->ptr, 1ll, K, 0.0, Y->ptr, N, 1ll, 0ll, 0ll, 0ll));
         LAUNCHED();
         if (Bi) {
             hipLaunchKernelGGL(d_add_bias_rows_kernel, grid_of((size_t)(M * N)), 256, 0, s, (size_t)(M * N), (int)N, (const double*)Bi->ptr, Y->ptr);
@@ -1790,8 +2008,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         }
         double* tmp;
         ERRCHK(workspace((size_t)(M * 3 * C), &tmp));
-        hipLaunchKernelGGL(d_gemm_kernel, dim3((unsigned)((3 * C + 15) / 16), (unsigned)((M + 15) / 16), 1), 256, 0, s, (int)M, (int)(3 * C), (int)C,
-                           1.0, (const double*)X->ptr, C, 1ll, (const double*)W->ptr, 1ll, C, 0.0, tmp, 3 * C, 1ll, 0ll, 0ll, 0ll);
+        HIPCHK(d_gemm(s, 1, (int)M, (int)(3 * C), (int)C, 1.0, (const double*)X->ptr, C, 1ll, (const double*)W->ptr, 1ll, C, 0.0, tmp, 3 * C, 1ll, 0ll, 0ll, 0ll));
         LAUNCHED();
         const size_t pairs = (size_t)(M * 3 * C) / 2;
         hipLaunchKernelGGL(d_qkv_split_kernel, grid_of(pairs), 256, 0, s, pairs, (const double*)tmp, Bi ? (const double*)Bi->ptr : nullptr,

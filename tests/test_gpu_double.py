@@ -544,3 +544,30 @@ def test_double_ids_outside_the_built_set_say_so(devd):
     with pytest.raises(CudaDnnError) as e:
         devd.cuda.SetAttn(hc, ha, 0, True, 1, 8, 1, 8, 0.1)
     assert e.value.code == 90009
+
+
+@pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False)])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 33, 17), (64, 64, 128), (65, 40, 300), (520, 1030, 40), (100, 36, 1024)])
+def test_double_gemm_tile_edges(devd, m, n, k, tA, tB):
+    """Tiles of 32 and 64, contractions shared out over four groups of wavefronts, and their remainders."""
+    rng = np.random.default_rng(m + n + k)
+    a, b, c = rng.standard_normal((m, k)), rng.standard_normal((k, n)), rng.standard_normal((m, n))
+    ha, hb, hc = devd.put((a.T if tA else a).copy()), devd.put((b.T if tB else b).copy()), devd.put(c)
+    devd.cuda.gemm(tA, tB, m, n, k, 0.5, ha, hb, 1.0, hc)
+    ref = 0.5 * (a @ b) + c
+    assert np.abs(devd.get(hc, (m, n)) - ref).max() / np.abs(ref).max() < 1e-13
+
+
+def test_double_transpose_follows_its_blobs(devd):
+    """The decoded axis map is kept per contents of its blobs: writing one of them, or a part of it, is seen."""
+    x = np.arange(24.0).reshape(2, 3, 4)
+    hx, hy = devd.put(x), devd.zeros(24)
+    xc, yc, mp = devd.put([12, 4, 1]), devd.put([8, 4, 1]), devd.put([1, 0, 2])
+    for _ in range(2):
+        devd.cuda.transpose(24, hx, hy, xc, yc, mp, 3, 0)
+        assert np.array_equal(devd.get(hy, (3, 2, 4)), x.transpose(1, 0, 2))
+    devd.cuda.SetMemory(yc, [6, 3, 1])
+    view = devd.cuda.CreateMemoryPointer(mp, 0, 3)
+    devd.cuda.SetMemory(view, [2, 0, 1])
+    devd.cuda.transpose(24, hx, hy, xc, yc, mp, 3, 0)
+    assert np.array_equal(devd.get(hy, (4, 2, 3)), x.transpose(2, 0, 1))
