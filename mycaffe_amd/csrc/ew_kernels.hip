@@ -104,12 +104,34 @@ template <typename F> static hipError_t launch_map(hipStream_t s, DType dt, size
 }
 
 // ---------------------------------------------------------------------------
-template <typename T> __global__ void set_kernel(T* y, size_t n, float v) { GRID_STRIDE(i, n) st(y, i, v); }
+// Fills and copies in 16-byte pieces of raw bits (`pieces` of them, then `tail` elements of E bytes).  The runtime's own fill
+// and copy kernels take 4.6 and 5.8 us for what these do in 2 - 3 us at the sizes of a layer's gradients.
+template <typename E> __global__ void fill_kernel(E* y, size_t n, size_t pieces, E v)
+{
+    constexpr int W = 16 / sizeof(E);
+    uint32_t w = (uint32_t)v;
+    if (sizeof(E) == 2) w |= w << 16;
+    const size_t gid = (size_t)blockIdx.x * TPB + threadIdx.x, stride = (size_t)TPB * gridDim.x;
+    for (size_t i = gid; i < pieces; i += stride) ((uint4*)y)[i] = make_uint4(w, w, w, w);
+    for (size_t i = pieces * W + gid; i < n; i += stride) y[i] = v;
+}
+template <typename E> __global__ void copy_kernel(const E* x, E* y, size_t n, size_t pieces)
+{
+    constexpr int W = 16 / sizeof(E);
+    const size_t gid = (size_t)blockIdx.x * TPB + threadIdx.x, stride = (size_t)TPB * gridDim.x;
+    for (size_t i = gid; i < pieces; i += stride) ((uint4*)y)[i] = ((const uint4*)x)[i];
+    for (size_t i = pieces * W + gid; i < n; i += stride) y[i] = x[i];
+}
 
 hipError_t k_set(hipStream_t s, DType dt, void* y, size_t n, float v)
 {
     if (n == 0) return hipSuccess;
-    DISPATCH_DT(dt, hipLaunchKernelGGL(set_kernel<T>, grid_for(n), TPB, 0, s, (T*)y, n, v));
+    const size_t pieces = ((uintptr_t)y & 15) == 0 ? n / (dt == F32 ? 4 : 8) : 0;
+    const int g = grid_for(pieces ? pieces : n);
+    union { float f; uint32_t u; } c;
+    c.f = v;
+    if (dt == F32) hipLaunchKernelGGL(fill_kernel<uint32_t>, g, TPB, 0, s, (uint32_t*)y, n, pieces, c.u);
+    else hipLaunchKernelGGL(fill_kernel<uint16_t>, g, TPB, 0, s, (uint16_t*)y, n, pieces, f32_to_bf16(v));
     return hipGetLastError();
 }
 
@@ -122,10 +144,13 @@ hipError_t k_convert(hipStream_t s, DType sdt, const void* src, DType ddt, void*
 {
     if (n == 0) return hipSuccess;
     int g = grid_for(n);
-    if (sdt == F32 && ddt == F32)
-        return hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyDeviceToDevice, s);
-    if (sdt == BF16 && ddt == BF16)
-        return hipMemcpyAsync(dst, src, n * sizeof(bf16_t), hipMemcpyDeviceToDevice, s);
+    if (sdt == ddt) {
+        const size_t pieces = (((uintptr_t)src | (uintptr_t)dst) & 15) == 0 ? n / (sdt == F32 ? 4 : 8) : 0;
+        g = grid_for(pieces ? pieces : n);
+        if (sdt == F32) hipLaunchKernelGGL(copy_kernel<uint32_t>, g, TPB, 0, s, (const uint32_t*)src, (uint32_t*)dst, n, pieces);
+        else hipLaunchKernelGGL(copy_kernel<uint16_t>, g, TPB, 0, s, (const uint16_t*)src, (uint16_t*)dst, n, pieces);
+        return hipGetLastError();
+    }
     if (sdt == F32)
         hipLaunchKernelGGL((convert_kernel<float, bf16_t>), g, TPB, 0, s, (const float*)src, (bf16_t*)dst, n);
     else
@@ -442,52 +467,22 @@ template <int NW> __device__ inline float block_sum(float v, float* red)
     return r;
 }
 
-// one workgroup per row (inner == 1); the row is read once into registers when it
-// fits (len <= 256*8) and re-read from L2 otherwise
+// one workgroup per row (inner == 1) of more values than the kernels further down hold in registers: three passes, L2 behind
 template <typename T> __global__ void softmax_rows_kernel(const T* x, T* y, int len, bool logsm)
 {
     __shared__ float red[4];
     const T* xr = x + (size_t)blockIdx.x * len;
     T* yr = y + (size_t)blockIdx.x * len;
-    constexpr int R = 8;
-    float v[R];
-    bool cached = len <= TPB * R;
     float mx = -INFINITY;
-    if (cached) {
-        for (int j = 0; j < R; j++) {
-            int i = threadIdx.x + j * TPB;
-            v[j] = i < len ? ld(xr, i) : -INFINITY;
-            mx = fmaxf(mx, v[j]);
-        }
-    } else {
-        for (int i = threadIdx.x; i < len; i += TPB) mx = fmaxf(mx, ld(xr, i));
-    }
+    for (int i = threadIdx.x; i < len; i += TPB) mx = fmaxf(mx, ld(xr, i));
     mx = block_max<4>(mx, red);
     float sum = 0.f;
-    if (cached) {
-        for (int j = 0; j < R; j++) {
-            int i = threadIdx.x + j * TPB;
-            if (i < len) {
-                v[j] = expf(v[j] - mx);
-                sum += v[j];
-            }
-        }
-    } else {
-        for (int i = threadIdx.x; i < len; i += TPB) sum += expf(ld(xr, i) - mx);
-    }
+    for (int i = threadIdx.x; i < len; i += TPB) sum += expf(ld(xr, i) - mx);
     sum = block_sum<4>(sum, red);
-    if (logsm) {
-        float ls = logf(sum);
-        for (int i = threadIdx.x; i < len; i += TPB) st(yr, i, ld(xr, i) - mx - ls);
-        return;
-    }
-    if (cached) {
-        for (int j = 0; j < R; j++) {
-            int i = threadIdx.x + j * TPB;
-            if (i < len) st(yr, i, v[j] / sum);
-        }
-    } else {
-        for (int i = threadIdx.x; i < len; i += TPB) st(yr, i, expf(ld(xr, i) - mx) / sum);
+    const float ls = logf(sum);
+    for (int i = threadIdx.x; i < len; i += TPB) {
+        const float d = ld(xr, i) - mx;
+        st(yr, i, logsm ? d - ls : expf(d) / sum);
     }
 }
 
@@ -511,11 +506,13 @@ template <typename T> __global__ void softmax_strided_kernel(const T* x, T* y, s
 }
 
 static bool softmax_fwd_wave_launch(hipStream_t s, DType dt, const void* x, void* y, size_t rows, int len, bool logsm);
+static bool softmax_fwd_long_launch(hipStream_t s, DType dt, const void* x, void* y, size_t rows, int len, bool logsm);
 
 hipError_t k_softmax(hipStream_t s, DType dt, const void* x, void* y, size_t outer, int len, int inner, bool logsm)
 {
     if (outer == 0 || len <= 0 || inner <= 0) return hipSuccess;
-    if (inner == 1 && softmax_fwd_wave_launch(s, dt, x, y, outer, len, logsm)) return hipGetLastError();
+    if (inner == 1 && (softmax_fwd_wave_launch(s, dt, x, y, outer, len, logsm) || softmax_fwd_long_launch(s, dt, x, y, outer, len, logsm)))
+        return hipGetLastError();
     if (inner == 1) {
         if (outer > 0x7fffffffu) return hipErrorInvalidValue;
         DISPATCH_DT(dt, hipLaunchKernelGGL(softmax_rows_kernel<T>, (int)outer, TPB, 0, s, (const T*)x, (T*)y, len, logsm));
@@ -776,7 +773,7 @@ hipError_t k_layernorm_bwd(hipStream_t s, DType dt, int rows, int inner, const v
 // Softmax gradient (cudnnSoftmaxBackward as called from SoftmaxLayer.cs:359-367): per series of `len` values
 //   accurate / fast : dx = (dy - sum(dy * y)) * y
 //   log             : dx = dy - exp(y) * sum(dy)
-// inner == 1 and len % 4 == 0, len <= 2048: one wavefront per row, the row kept in registers between the two passes.
+// inner == 1 and len <= 2048: one wavefront per row, the row kept in registers between the two passes.
 // Forward pass of the same shape class: one wavefront per row, max, exp and sum on the registers that hold the row.
 // MASKED: the row is first put through a mask call that was held back for this purpose,
 //   x = mask[mi] == search ? replace : xscale * x,   mi = i % md1 + (i / dd1) * md1   (i = flat index; md1 and dd1 are
@@ -785,96 +782,117 @@ hipError_t k_layernorm_bwd(hipStream_t s, DType dt, int rows, int inner, const v
 // long, so it is not read, and neither are the chunks of x that lie wholly above the diagonal.
 struct SoftmaxMask { const void* mask; size_t md1, dd1; float search, replace, xscale; int causalT; int* zeroFlag; int epoch; };
 
-template <typename T, int R, bool MASKED>
+// VEC: rows of whole aligned quads, a lane holds quads lane + 64 r; otherwise it holds the elements lane + 64 j.
+template <typename T, int R, bool VEC> struct RowInLanes {
+    __device__ static inline int at(int lane, int r, int i) { return VEC ? 4 * (lane + r * 64) + i : lane + 64 * (4 * r + i); }
+    // v[r][i] = element at(lane, r, i) where that is below `end` (VEC: where its quad begins below it), else `fill`
+    __device__ static inline void load(const T* p, int lane, int end, float fill, float (&v)[R][4])
+    {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (VEC) {
+                if (at(lane, r, 0) < end) Vec4<T>::load(p + at(lane, r, 0), v[r]);
+                else v[r][0] = v[r][1] = v[r][2] = v[r][3] = fill;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[r][i] = at(lane, r, i) < end ? ld(p, at(lane, r, i)) : fill;
+            }
+        }
+    }
+    __device__ static inline void store(T* p, int lane, int len, const float (&v)[R][4])
+    {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (VEC) {
+                if (at(lane, r, 0) < len) Vec4<T>::store(p + at(lane, r, 0), v[r]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (at(lane, r, i) < len) st(p, at(lane, r, i), v[r][i]);
+            }
+        }
+    }
+};
+
+template <typename T, int R, bool MASKED, bool VEC>
 __global__ __launch_bounds__(256) void softmax_fwd_wave_kernel(size_t rows, int len, const T* x, T* y, bool logsm, SoftmaxMask mk)
 {
+    typedef RowInLanes<T, R, VEC> L;
     const int lane = threadIdx.x & 63;
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const int chunks = len >> 2;
     const T* xr = x + row * len;
-    T* yr = y + row * len;
-    const T* mr = nullptr;
-    int qrow = 0;
-    if (MASKED) {
-        if (mk.causalT) {
-            qrow = (int)(row % (size_t)mk.causalT);
-        } else {
-            const size_t i0 = row * (size_t)len;
-            mr = (const T*)mk.mask + i0 % mk.md1 + (i0 / mk.dd1) * mk.md1;
-        }
-    }
+    const int qrow = MASKED && mk.causalT ? (int)(row % (size_t)mk.causalT) : len - 1;   // last entry that is kept and read
     float v[R][4];
+    L::load(xr, lane, qrow + 1, 0.f, v);
+    if (MASKED && mk.causalT) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[r][i] = L::at(lane, r, i) > qrow ? mk.replace : mk.xscale * v[r][i];
+    } else if (MASKED) {
+        const size_t i0 = row * (size_t)len;
+        float mv[R][4];
+        L::load((const T*)mk.mask + i0 % mk.md1 + (i0 / mk.dd1) * mk.md1, lane, len, 0.f, mv);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[r][i] = mv[r][i] == mk.search ? mk.replace : mk.xscale * v[r][i];
+    }
     float mx = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int c = lane + r * 64;
-        if (c < chunks) {
-            if (MASKED && mk.causalT) {
-                if (4 * c > qrow) {
+    for (int r = 0; r < R; r++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) v[r][i] = mk.replace;
-                } else {
-                    Vec4<T>::load(xr + 4 * c, v[r]);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) v[r][i] = 4 * c + i > qrow ? mk.replace : mk.xscale * v[r][i];
-                }
-            } else {
-                Vec4<T>::load(xr + 4 * c, v[r]);
-            }
-            if (MASKED && !mk.causalT) {
-                float mv[4];
-                Vec4<T>::load(mr + 4 * c, mv);
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[r][i] = mv[i] == mk.search ? mk.replace : mk.xscale * v[r][i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) mx = fmaxf(mx, v[r][i]);
-        }
-    }
+        for (int i = 0; i < 4; i++)
+            if (L::at(lane, r, i) < len) mx = fmaxf(mx, v[r][i]);
     mx = wave_max(mx);
     // a later product over this row may skip the masked entries if every one of them comes out as an exact zero
     if (MASKED && mk.causalT && mk.zeroFlag && lane == 0 && qrow + 1 < len && (logsm || expf(mk.replace - mx) != 0.f))
         *mk.zeroFlag = mk.epoch;
     float sum = 0.f;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        if (lane + r * 64 < chunks) {
+    for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float d = v[r][i] - mx;
-                const float e = expf(d);
+        for (int i = 0; i < 4; i++)
+            if (L::at(lane, r, i) < len) {
+                const float d = v[r][i] - mx, e = expf(d);
                 sum += e;
                 v[r][i] = logsm ? d : e;
             }
-        }
-    }
     sum = wave_sum(sum);
     const float ls = logf(sum);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int c = lane + r * 64;
-        if (c < chunks) {
-            float o[4];
+    for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) o[i] = logsm ? v[r][i] - ls : v[r][i] / sum;
-            Vec4<T>::store(yr + 4 * c, o);
-        }
-    }
+        for (int i = 0; i < 4; i++) v[r][i] = logsm ? v[r][i] - ls : v[r][i] / sum;
+    L::store(y + row * len, lane, len, v);
+}
+
+// quads per lane (1, 2, 4, 8) of a row of up to 2048 values, and whether it can be read in whole aligned quads
+static inline int softmax_wave_quads(int len)
+{
+    const int r = (len + 255) / 256;
+    return r <= 1 ? 1 : (r <= 2 ? 2 : (r <= 4 ? 4 : 8));
+}
+static inline bool softmax_whole_quads(int len, const void* a, const void* b, const void* c, DType dt)
+{
+    return len % 4 == 0 && (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & (dt == F32 ? 15 : 7)) == 0;
 }
 
 template <bool MASKED>
 static bool softmax_fwd_wave_launch_t(hipStream_t s, DType dt, const void* x, void* y, size_t rows, int len, bool logsm, SoftmaxMask mk)
 {
-    const int R = layernorm_wave_chunks(len, x, y, MASKED ? mk.mask : y, dt == F32 ? 4 : 2);
-    if (R == 0 || (rows + 3) / 4 > 0x7fffffffu) return false;
-    const int g = (int)((rows + 3) / 4);
-#define SM_FWD(RR) DISPATCH_DT(dt, hipLaunchKernelGGL((softmax_fwd_wave_kernel<T, RR, MASKED>), g, 256, 0, s, rows, len, (const T*)x, (T*)y, logsm, mk))
+    if (len > 2048 || (rows + 3) / 4 > 0x7fffffffu) return false;
+    const int R = softmax_wave_quads(len), g = (int)((rows + 3) / 4);
+    const bool vec = softmax_whole_quads(len, x, y, MASKED ? mk.mask : y, dt);
+#define SM_FWD2(RR, VV) DISPATCH_DT(dt, hipLaunchKernelGGL((softmax_fwd_wave_kernel<T, RR, MASKED, VV>), g, 256, 0, s, rows, len, (const T*)x, (T*)y, logsm, mk))
+#define SM_FWD(RR) do { if (vec) SM_FWD2(RR, true); else SM_FWD2(RR, false); } while (0)
     if (R == 1) SM_FWD(1);
     else if (R == 2) SM_FWD(2);
     else if (R == 4) SM_FWD(4);
     else SM_FWD(8);
 #undef SM_FWD
+#undef SM_FWD2
     return true;
 }
 static bool softmax_fwd_wave_launch(hipStream_t s, DType dt, const void* x, void* y, size_t rows, int len, bool logsm)
@@ -896,39 +914,141 @@ hipError_t k_softmax_masked(hipStream_t s, DType dt, const void* x, void* y, siz
     return hipGetLastError();
 }
 
-template <typename T, int R>
-__global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(size_t rows, int len, const T* y, const T* dy, T* dx, bool logsm)
+// causalT != 0: y is the output of a softmax under the causal mask of causalT x causalT whose masked entries are exact zeros
+// unless *zeroFlag == epoch.  What lies above the diagonal is then neither read nor multiplied: its gradient is zero.
+template <typename T, int R, bool VEC>
+__global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(size_t rows, int len, const T* y, const T* dy, T* dx, bool logsm, int causalT,
+                                                               const int* zeroFlag, int epoch)
 {
+    typedef RowInLanes<T, R, VEC> L;
     const int lane = threadIdx.x & 63;
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const int chunks = len >> 2;
-    const T* yr = y + row * len;
-    const T* gr = dy + row * len;
-    T* xr = dx + row * len;
+    const int end = causalT && *zeroFlag != epoch ? (int)(row % (size_t)causalT) + 1 : len;
     float yv[R][4], gv[R][4];
+    L::load(y + row * len, lane, end, 0.f, yv);
+    L::load(dy + row * len, lane, end, 0.f, gv);
     float sum = 0.f;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int c = lane + r * 64;
-        if (c < chunks) {
-            Vec4<T>::load(yr + 4 * c, yv[r]);
-            Vec4<T>::load(gr + 4 * c, gv[r]);
+    for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) sum += logsm ? gv[r][i] : gv[r][i] * yv[r][i];
-        }
-    }
+        for (int i = 0; i < 4; i++)
+            if (L::at(lane, r, i) < end) sum += logsm ? gv[r][i] : gv[r][i] * yv[r][i];
     sum = wave_sum(sum);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int c = lane + r * 64;
-        if (c < chunks) {
-            float o[4];
+    for (int r = 0; r < R; r++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) o[i] = logsm ? gv[r][i] - __expf(yv[r][i]) * sum : (gv[r][i] - sum) * yv[r][i];
-            Vec4<T>::store(xr + 4 * c, o);
+        for (int i = 0; i < 4; i++)
+            gv[r][i] = L::at(lane, r, i) >= end ? 0.f : logsm ? gv[r][i] - __expf(yv[r][i]) * sum : (gv[r][i] - sum) * yv[r][i];
+    L::store(dx + row * len, lane, len, gv);
+}
+
+// Rows of 2049 to 32768 values (a vocabulary): one workgroup of sixteen wavefronts per row, the row in registers between its
+// passes, so that each tensor crosses memory once (1000 x 32000: forward 150 -> 62 us, gradient 180 -> 90 us).
+template <typename T, int R, bool VEC>
+__global__ __launch_bounds__(1024) void softmax_fwd_long_kernel(int len, const T* x, T* y, bool logsm)
+{
+    __shared__ float red[16];
+    const size_t base = (size_t)blockIdx.x * len;
+    float v[R][4];
+    auto at = [&](int r, int i) { return VEC ? 4 * ((int)threadIdx.x + 1024 * r) + i : (int)threadIdx.x + 1024 * (4 * r + i); };
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (VEC) {
+            if (at(r, 0) < len) Vec4<T>::load(x + base + at(r, 0), v[r]);
+            else v[r][0] = v[r][1] = v[r][2] = v[r][3] = -INFINITY;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[r][i] = at(r, i) < len ? ld(x, base + at(r, i)) : -INFINITY;
         }
     }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) mx = fmaxf(mx, v[r][i]);
+    mx = block_max<16>(mx, red);
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float d = v[r][i] - mx, e = expf(d);
+            if (at(r, i) < len) sum += e;
+            v[r][i] = logsm ? d : e;
+        }
+    sum = block_sum<16>(sum, red);
+    const float ls = logf(sum);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[r][i] = logsm ? v[r][i] - ls : v[r][i] / sum;
+        if (VEC) {
+            if (at(r, 0) < len) Vec4<T>::store(y + base + at(r, 0), v[r]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (at(r, i) < len) st(y, base + at(r, i), v[r][i]);
+        }
+    }
+}
+template <typename T, int R, bool VEC>
+__global__ __launch_bounds__(1024) void softmax_bwd_long_kernel(int len, const T* y, const T* dy, T* dx, bool logsm)
+{
+    __shared__ float red[16];
+    const size_t base = (size_t)blockIdx.x * len;
+    float yv[R][4], gv[R][4];
+    auto at = [&](int r, int i) { return VEC ? 4 * ((int)threadIdx.x + 1024 * r) + i : (int)threadIdx.x + 1024 * (4 * r + i); };
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (VEC) {
+            if (at(r, 0) < len) { Vec4<T>::load(y + base + at(r, 0), yv[r]); Vec4<T>::load(dy + base + at(r, 0), gv[r]); }
+            else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) yv[r][i] = gv[r][i] = 0.f;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                yv[r][i] = at(r, i) < len ? ld(y, base + at(r, i)) : 0.f;
+                gv[r][i] = at(r, i) < len ? ld(dy, base + at(r, i)) : 0.f;
+            }
+        }
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum += logsm ? gv[r][i] : gv[r][i] * yv[r][i];   // zeros past the end
+    sum = block_sum<16>(sum, red);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) gv[r][i] = logsm ? gv[r][i] - expf(yv[r][i]) * sum : (gv[r][i] - sum) * yv[r][i];
+        if (VEC) {
+            if (at(r, 0) < len) Vec4<T>::store(dx + base + at(r, 0), gv[r]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (at(r, i) < len) st(dx, base + at(r, i), gv[r][i]);
+        }
+    }
+}
+static inline int softmax_long_quads(int len) { return len <= 4096 ? 1 : len <= 8192 ? 2 : len <= 16384 ? 4 : len <= 32768 ? 8 : 0; }
+static bool softmax_fwd_long_launch(hipStream_t s, DType dt, const void* x, void* y, size_t rows, int len, bool logsm)
+{
+    const int R = softmax_long_quads(len);
+    if (!R || rows > 0x7fffffffu) return false;
+    const bool vec = softmax_whole_quads(len, x, y, y, dt);
+#define SM_LONG2(RR, VV) DISPATCH_DT(dt, hipLaunchKernelGGL((softmax_fwd_long_kernel<T, RR, VV>), (unsigned)rows, 1024, 0, s, len, (const T*)x, (T*)y, logsm))
+#define SM_LONG(RR) do { if (vec) SM_LONG2(RR, true); else SM_LONG2(RR, false); } while (0)
+    if (R == 1) SM_LONG(1);
+    else if (R == 2) SM_LONG(2);
+    else if (R == 4) SM_LONG(4);
+    else SM_LONG(8);
+#undef SM_LONG
+#undef SM_LONG2
+    return true;
 }
 
 // any (outer, len, inner): one workgroup per series, two passes over global memory
@@ -951,20 +1071,36 @@ __global__ void softmax_bwd_kernel(int len, int inner, const T* y, const T* dy, 
     }
 }
 
-hipError_t k_softmax_bwd(hipStream_t s, DType dt, const void* y, const void* dy, void* dx, size_t outer, int len, int inner, bool logsm)
+hipError_t k_softmax_bwd(hipStream_t s, DType dt, const void* y, const void* dy, void* dx, size_t outer, int len, int inner, bool logsm,
+                         int causalT, const int* zeroFlag, int epoch)
 {
     if (outer == 0 || len <= 0 || inner <= 0) return hipSuccess;
-    const int R = inner == 1 ? layernorm_wave_chunks(len, y, dy, dx, dt == F32 ? 4 : 2) : 0;
     const size_t series = outer * (size_t)inner;
     if (series > 0x7fffffffu) return hipErrorInvalidValue;
-    const int g = (int)((outer + 3) / 4);
-#define SM_BWD(RR) DISPATCH_DT(dt, hipLaunchKernelGGL((softmax_bwd_wave_kernel<T, RR>), g, 256, 0, s, outer, len, (const T*)y, (const T*)dy, (T*)dx, logsm))
-    if (R == 1) SM_BWD(1);
-    else if (R == 2) SM_BWD(2);
-    else if (R == 4) SM_BWD(4);
-    else if (R == 8) SM_BWD(8);
-    else DISPATCH_DT(dt, hipLaunchKernelGGL(softmax_bwd_kernel<T>, (int)series, TPB, 0, s, len, inner, (const T*)y, (const T*)dy, (T*)dx, logsm));
+    const bool vec = softmax_whole_quads(len, y, dy, dx, dt);
+    if (inner == 1 && len <= 2048) {
+        const int R = softmax_wave_quads(len), g = (int)((outer + 3) / 4);
+#define SM_BWD2(RR, VV) DISPATCH_DT(dt, hipLaunchKernelGGL((softmax_bwd_wave_kernel<T, RR, VV>), g, 256, 0, s, outer, len, (const T*)y, (const T*)dy, (T*)dx, logsm, causalT, zeroFlag, epoch))
+#define SM_BWD(RR) do { if (vec) SM_BWD2(RR, true); else SM_BWD2(RR, false); } while (0)
+        if (R == 1) SM_BWD(1);
+        else if (R == 2) SM_BWD(2);
+        else if (R == 4) SM_BWD(4);
+        else SM_BWD(8);
 #undef SM_BWD
+#undef SM_BWD2
+    } else if (inner == 1 && softmax_long_quads(len)) {
+        const int R = softmax_long_quads(len);
+#define SM_BWD2(RR, VV) DISPATCH_DT(dt, hipLaunchKernelGGL((softmax_bwd_long_kernel<T, RR, VV>), (unsigned)outer, 1024, 0, s, len, (const T*)y, (const T*)dy, (T*)dx, logsm))
+#define SM_BWD(RR) do { if (vec) SM_BWD2(RR, true); else SM_BWD2(RR, false); } while (0)
+        if (R == 1) SM_BWD(1);
+        else if (R == 2) SM_BWD(2);
+        else if (R == 4) SM_BWD(4);
+        else SM_BWD(8);
+#undef SM_BWD
+#undef SM_BWD2
+    } else {
+        DISPATCH_DT(dt, hipLaunchKernelGGL(softmax_bwd_kernel<T>, (int)series, TPB, 0, s, len, inner, (const T*)y, (const T*)dy, (T*)dx, logsm));
+    }
     return hipGetLastError();
 }
 

@@ -1310,9 +1310,9 @@ static hipError_t launch_gemm2_panel(hipStream_t s, int M, int N, float alpha, c
 
 hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float alpha, const float* A, const float* B,
                    float beta, float* C, int lda, int ldb, int ldc, long long sA, long long sB, long long sC, int batch,
-                   const int* causalFlag, int epoch, bool skipAboveDiagonal)
+                   const int* causalFlag, int epoch, bool skipAboveDiagonal, bool causalA)
 {
-    if (causalFlag && (tA || n != k)) return hipErrorInvalidValue;
+    if (causalFlag && (causalA ? m : n) != k) return hipErrorInvalidValue;
     if (skipAboveDiagonal && (tA || tB || m != n || beta != 0.f)) return hipErrorInvalidValue;
     // column-major: op(A)(i,kk) = tA ? A[kk + i*lda] : A[i + kk*lda]
     GemmStrides st;
@@ -1336,7 +1336,7 @@ hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float a
     g.lda = ldb; g.ldb = lda; g.ldc = ldc; g.sA = sB; g.sB = sA; g.sC = sC;
     g.aK = !tB; g.bK = tA;
     g.alpha = alpha; g.beta = beta; g.batch = batch;
-    if (causalFlag) { g.causal = tB ? CAUSAL_UPPER : CAUSAL_LOWER; g.flag = causalFlag; g.epoch = epoch; }
+    if (causalFlag) { g.causal = causalA ? (tA ? CAUSAL_B_UPPER : CAUSAL_B_LOWER) : (tB ? CAUSAL_A_UPPER : CAUSAL_A_LOWER); g.flag = causalFlag; g.epoch = epoch; }
     return gemm_f32(s, g, nullptr, 0);
 }
 

@@ -134,13 +134,13 @@ struct GemmF32 {
     bool aK, bK;
     float alpha, beta;
     int batch;
-    // CAUSAL_*: op(A) (m == k) is known to be exactly zero on one side of the diagonal unless *flag == epoch
+    // CAUSAL_*: op(A) (m == k) or op(B) (n == k) is known to be exactly zero on one side of the diagonal unless *flag == epoch
     int causal;
     const int* flag;
     int epoch;
     const HeadsEpilogue* heads;            // written through this epilogue instead of to C (alpha 1, beta 0, batch 1)
 };
-enum { CAUSAL_NO = 0, CAUSAL_LOWER = 1 /* zero for k > i */, CAUSAL_UPPER = 2 /* zero for k < i */ };
+enum { CAUSAL_NO = 0, CAUSAL_A_LOWER /* A(i,k) zero for k > i */, CAUSAL_A_UPPER /* k < i */, CAUSAL_B_LOWER /* B(k,j) zero for k < j */, CAUSAL_B_UPPER /* k > j */ };
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal);
 hipError_t gemm_f32(hipStream_t s, const GemmF32& g, void* ws, size_t wsBytes);
 

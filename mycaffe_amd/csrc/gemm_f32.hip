@@ -91,19 +91,26 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g)
     const int group = tile / (GROUP * g.tilesN), inGroup = tile - group * GROUP * g.tilesN;
     const int groupRows = min(GROUP, g.tilesM - group * GROUP);
     int tr = group * GROUP + inGroup % groupRows;
-    const int tc = inGroup / groupRows;
+    int tc = inGroup / groupRows;
     bool causal = false;
     if (g.causal) {
-        // rows of tiles differ in length: every other round of an XCD's 32 CUs takes them in reverse, so that a CU that had
-        // a long one gets a short one (decided per matrix, so that each of its tiles is still taken once)
-        if (((batch * tiles) >> 5) & 1) tr = g.tilesM - 1 - tr;
+        // tiles differ in length along one side: every other round of an XCD's 32 CUs takes them in reverse, so that a CU
+        // that had a long one gets a short one (decided per matrix, so that each of its tiles is still taken once)
+        if (((batch * tiles) >> 5) & 1) {
+            if (g.causal >= CAUSAL_B_LOWER) tc = g.tilesN - 1 - tc;
+            else tr = g.tilesM - 1 - tr;
+        }
         causal = *g.flag != g.epoch;
     }
     const int M = g.M, N = g.N;
     const int m0 = tr * BM, n0 = tc * BN;
     int kBegin = split ? part * g.kChunk : 0, kEnd = min(g.K, kBegin + g.kChunk);
-    if (causal && g.causal == CAUSAL_LOWER) kEnd = min(kEnd, m0 + BM);
-    if (causal && g.causal == CAUSAL_UPPER) kBegin = min(m0, kEnd - 1);
+    if (causal) {
+        if (g.causal == CAUSAL_A_LOWER) kEnd = min(kEnd, m0 + BM);
+        else if (g.causal == CAUSAL_A_UPPER) kBegin = m0;
+        else if (g.causal == CAUSAL_B_LOWER) kBegin = n0;
+        else kEnd = min(kEnd, n0 + BN);
+    }
     const float* __restrict__ A = g.A + (size_t)batch * g.sA;
     const float* __restrict__ B = g.B + (size_t)batch * g.sB;
     const int wm = (wave >> 1) * (32 * WM), wn = (wave & 1) * (32 * WN);
@@ -413,7 +420,7 @@ static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const Gem
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
 {
     if (q.m <= 0 || q.n <= 0 || q.batch <= 0) return hipSuccess;
-    if (q.k <= 0 || (q.causal && (q.m != q.k || !q.flag)) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || q.batch != 1 || !q.aK || !q.bK)))
+    if (q.k <= 0 || (q.causal && ((q.causal >= CAUSAL_B_LOWER ? q.n : q.m) != q.k || !q.flag)) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || q.batch != 1 || !q.aK || !q.bK)))
         return hipErrorInvalidValue;
     GemmF32Plan p = gemm_f32_plan(q.m, q.n, q.k, q.batch, q.causal != 0);
     if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }

@@ -62,7 +62,11 @@ hipError_t k_softmax_masked(hipStream_t s, DType dt, const void* x, void* y, siz
                             size_t md1, size_t dd1, float search, float replace, float xscale, bool causal = false,
                             int* zeroFlag = nullptr, int epoch = 0);
 // gradient with respect to the softmax input from the output y and its gradient dy (dx may alias dy)
-hipError_t k_softmax_bwd(hipStream_t s, DType dt, const void* y, const void* dy, void* dx, size_t outer, int len, int inner, bool logsm);
+// causalT: y is causal (rows of causalT over causalT queries, entries above the diagonal exact zeros unless *zeroFlag == epoch);
+// taken into account for inner == 1 and len <= 2048, where dx then has the same zeros (softmax_bwd_keeps_zeros)
+hipError_t k_softmax_bwd(hipStream_t s, DType dt, const void* y, const void* dy, void* dx, size_t outer, int len, int inner, bool logsm,
+                         int causalT = 0, const int* zeroFlag = nullptr, int epoch = 0);
+inline bool softmax_bwd_keeps_zeros(int len, int inner) { return inner == 1 && len <= 2048; }
 // adjacent-pair rotary embedding with the CudaDnnDLL index rule; x == y allowed
 hipError_t k_rope(hipStream_t s, DType dt, size_t n, const void* x, void* y, const float* fcos, const float* fsin,
                   int seqLen, int heads, int hs, int tableOff, bool grad = false);
@@ -124,11 +128,12 @@ hipError_t k_gemm_bf16_swiglu(hipStream_t s, int m, int hid, int k, const void* 
 hipError_t k_gemm_bf16_qkv_rope(hipStream_t s, int B, int P, int H, int kvH, int hs, int k, const void* A, bool split, const void* Wqkv,
                                 void* q, void* kh, void* vh, bool heads16, void* kc, void* vc, bool cache16, int seqLen,
                                 const float* fcos, const float* fsin);
-// causalFlag != nullptr (no transposes, n == k): B(k,j) is known to be exactly zero for k > j unless *causalFlag == epoch,
-// and the contraction of a tile of columns stops at its last column
+// causalFlag != nullptr: op(B) (causalA: op(A)) is square, and what lies on one side of its diagonal is known to be exactly
+// zero unless *causalFlag == epoch: B(k,j) for k > j, transposed for k < j; A(i,k) for k < i, transposed for k > i.  The
+// contraction of a tile of C then stops or begins at the diagonal.
 hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float alpha, const float* A, const float* B,
                    float beta, float* C, int lda, int ldb, int ldc, long long sA, long long sB, long long sC,
-                   int batch, const int* causalFlag = nullptr, int epoch = 0, bool skipAboveDiagonal = false);
+                   int batch, const int* causalFlag = nullptr, int epoch = 0, bool skipAboveDiagonal = false, bool causalA = false);
 // skipAboveDiagonal (no transposes, m == n, short contraction): entries C(i,j) of tiles that lie wholly at i > j need not
 // be computed (their memory is left as it is); other shapes ignore the request
 // A row-major (m,n) of type adt; x, y fp32.  y = alpha*A*x + beta*y, or with tA y = alpha*A^T*x + beta*y

@@ -218,7 +218,7 @@ Kernel::~Kernel()
     m_layernorm.clear();
     m_mem.free_all();
     if (m_ws) (void)hipFree(m_ws);
-    if (m_zeroFlag) (void)hipFree(m_zeroFlag);
+    if (m_zeroFlags) (void)hipFree(m_zeroFlags);
     if (m_tickets) (void)hipFree(m_tickets);
     if (m_stage) (void)hipHostFree(m_stage);
     for (float* p : m_hostAllocs) (void)hipHostFree(p);
@@ -330,9 +330,9 @@ long Kernel::flush_pending_product(bool causal)
     if (m_mem.get(p.hA, &A) || m_mem.get(p.hB, &B) || m_mem.get(p.hC, &C)) return 0;   // an operand is gone
     if (p.kind == 1) {
         void* ws = nullptr;
-        const size_t wsb = k_gemm_workspace_bytes(F32, false, true, p.m, p.n, p.k);
+        const size_t wsb = k_gemm_workspace_bytes(C->dt(), false, true, p.m, p.n, p.k);
         if (wsb) ERRCHK(workspace(wsb, &ws));
-        HIPCHK(k_gemm(m_stream, F32, false, true, p.m, p.n, p.k, p.alpha, A->ptr, B->ptr, 0.f, C->ptr, ws, wsb));
+        HIPCHK(k_gemm(m_stream, C->dt(), false, true, p.m, p.n, p.k, p.alpha, A->ptr, B->ptr, 0.f, C->ptr, ws, wsb));
         return 0;
     }
     HIPCHK(k_gemm2(m_stream, false, false, p.m, p.n, p.k, p.alpha, (const float*)A->ptr, (const float*)B->ptr, 0.f, (float*)C->ptr,
@@ -363,12 +363,12 @@ long Kernel::flush_pending_mask()
     return 0;
 }
 
-// Holds a mask call back when it masks a large whole allocation in place (the attention chain's score tensor), so that
+// Holds a mask call back when it masks a whole allocation in place (the attention chain's score tensor), so that
 // the softmax that follows can do both in one pass.  The folded-in scaling of X moves into the record.
 bool Kernel::defer_mask(long hX, long hM, long hY, MemItem* X, MemItem* M, long long n, int md, int batch, float search,
                         float replace, float xscale, bool timing)
 {
-    if (timing || hX != hY || hX == hM || X->view || X->views != 0 || X->exposed || M->view || M->exposed || (size_t)n != X->count || n < (1 << 20)) return false;
+    if (timing || hX != hY || hX == hM || X->view || X->views != 0 || X->exposed || M->view || M->exposed || (size_t)n != X->count) return false;
     m_pendingMask.hX = hX; m_pendingMask.hM = hM; m_pendingMask.n = n; m_pendingMask.md = md; m_pendingMask.batch = batch;
     m_pendingMask.search = search; m_pendingMask.replace = replace; m_pendingMask.xscale = xscale;
     X->pending = 1.f;
@@ -524,33 +524,49 @@ bool Kernel::tril_scan(MemItem* mask, int T, bool* causal)
     return true;
 }
 
-__global__ void check_ones_kernel(const float* v, int n, int* bad)
+__global__ void check_ones_kernel(const void* v, bool half, int n, int* bad)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += blockDim.x * gridDim.x)
-        if (v[i] != 1.f) *bad = 1;
+        if ((half ? bf16_to_f32(((const bf16_t*)v)[i]) : ((const float*)v)[i]) != 1.f) *bad = 1;
 }
 
 bool Kernel::vector_is_ones(long h, MemItem* v, int n)
 {
-    if (v->half || v->view || v->exposed || v->count < (size_t)n) return false;
+    if (v->view || v->exposed || v->count < (size_t)n) return false;
     const uint64_t ver = m_mem.version(h);
-    for (const OnesCacheEntry& e : m_onesCache)
-        if (e.handle == h && e.version == ver && e.n >= n && e.ones) return true;
-        else if (e.handle == h && e.version == ver && e.n <= n && !e.ones) return false;
+    const auto known = m_onesCache.find(h);
+    if (known != m_onesCache.end() && known->second.version == ver) {
+        if (known->second.n >= n && known->second.ones) return true;
+        if (known->second.n <= n && !known->second.ones) return false;
+    }
     void* ws;
     if (workspace(256, &ws)) return false;
     int* flag = (int*)ws;
     if (hipMemsetAsync(flag, 0, sizeof(int), m_stream) != hipSuccess) return false;
     int grid = (n + 255) / 256;
     if (grid > 1024) grid = 1024;
-    hipLaunchKernelGGL(check_ones_kernel, grid, 256, 0, m_stream, (const float*)v->ptr, n, flag);
+    hipLaunchKernelGGL(check_ones_kernel, grid, 256, 0, m_stream, v->ptr, v->half, n, flag);
     int bad = 1;
     if (hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, m_stream) != hipSuccess) return false;
     if (hipStreamSynchronize(m_stream) != hipSuccess) return false;
-    OnesCacheEntry& e = m_onesCache[m_onesNext];
-    m_onesNext = (m_onesNext + 1) % 16;
-    e.handle = h; e.version = ver; e.n = n; e.ones = (bad == 0);
-    return e.ones;
+    if (m_onesCache.size() > 4096) m_onesCache.clear();
+    m_onesCache[h] = OnesCacheEntry{ver, n, bad == 0};
+    return bad == 0;
+}
+
+const Kernel::ZeroTag* Kernel::zero_tag(long h)
+{
+    for (const ZeroTag& t : m_zeroTags)
+        if (t.handle == h && t.version == m_mem.version(h)) return &t;
+    return nullptr;
+}
+void Kernel::zero_tag_set(long h, int len, size_t rows, int slot, int epoch)
+{
+    const ZeroTag t = {h, m_mem.version(h), len, rows, slot, epoch};
+    for (ZeroTag& e : m_zeroTags)
+        if (e.handle == h) { e = t; return; }
+    if (m_zeroTags.size() >= 2 * ZERO_SLOTS) m_zeroTags.erase(m_zeroTags.begin());
+    m_zeroTags.push_back(t);
 }
 
 // the same question for the mask blob of a held-back mask call (no attention handle to keep the answer on): cached per
@@ -724,7 +740,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         ERRCHK(mem((long)pl[1], &it));
         m_mem.touch((long)pl[1]);
         if (pf[0] == 0.f && idx == -1 && off == 0) {
-            HIPCHK(hipMemsetAsync(it->ptr, 0, it->count * it->esize(), s));
+            HIPCHK(k_set(s, it->dt(), it->ptr, it->count, 0.f));
             return 0;
         }
         if (off < 0) off = 0;
@@ -779,16 +795,16 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             hB != m_pendingProduct.hB) {
             ERRCHK(mem(hA, &A));
             ERRCHK(mem(hB, &B));
-            if (m_pendingProduct.kind == 1 && m_pendingProduct.hC == hC && !A->half && !B->half && !B->view && B->count >= (size_t)n &&
+            if (m_pendingProduct.kind == 1 && m_pendingProduct.hC == hC && A->half == B->half && !B->view && B->count >= (size_t)n &&
                 vector_is_ones(hA, A, m)) {
                 const PendingProduct p = m_pendingProduct;
                 MemItem *X, *W;
-                if (!m_mem.get(p.hA, &X) && !m_mem.get(p.hB, &W) && !m_mem.get(p.hC, &C)) {
+                if (!m_mem.get(p.hA, &X) && !m_mem.get(p.hB, &W) && !m_mem.get(p.hC, &C) && C->half == A->half) {
                     m_pendingProduct = PendingProduct();
                     void* ws = nullptr;
-                    const size_t wsb = k_gemm_bias_workspace_bytes(F32, p.m, p.n, p.k, X->ptr, W->ptr, C->ptr);
+                    const size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, C->ptr);
                     if (wsb) ERRCHK(workspace(wsb, &ws));
-                    HIPCHK(k_gemm_bias(s, F32, p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws, wsb));
+                    HIPCHK(k_gemm_bias(s, C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws, wsb));
                     m_mem.touch(hC);
                     return 0;
                 }
@@ -808,9 +824,8 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             RANGE(A, aOff, (long long)m * k);
             RANGE(B, bOff, (long long)k * n);
             if (m_pendingProduct.hC == hC) m_pendingProduct = PendingProduct();
-            // Y = X W^T of an inner product layer, large enough for the saved pass to matter
-            if (!timing && !tA && tB && !A->half && pf[0] == 1.f && aOff == 0 && bOff == 0 && m >= 256 && n >= 64 && k >= 32 &&
-                (long long)m * n >= (1ll << 20) && !A->view && !B->view && !A->exposed && !B->exposed && !C->exposed) {
+            // Y = X W^T of an inner product layer
+            if (!timing && !tA && tB && pf[0] == 1.f && aOff == 0 && bOff == 0 && m > 0 && n > 0 && k > 1 && !A->view && !B->view && !A->exposed && !B->exposed && !C->exposed) {
                 if (m_pendingProduct.hC) ERRCHK(flush_pending_product());   // one at a time
                 PendingProduct& pp = m_pendingProduct;
                 pp.kind = 1; pp.hA = hA; pp.hB = hB; pp.hC = hC; pp.m = m; pp.n = n; pp.k = k; pp.alpha = 1.f;
@@ -891,17 +906,24 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 return 0;
             }
         }
-        // The second operand is the output of a softmax with a causal mask folded in (the P V product of the explicit
-        // attention chain): its entries above the diagonal are exact zeros - the softmax kernel raises a flag on the
-        // device if a row's are not - and the contraction stops at the diagonal.
-        const int* zeroFlag = nullptr;
-        // (given transposed - the product P^T dY of the backward pass - the same zeros let it begin at the diagonal)
-        if (m_zeroHandle && (long)pl[7] == m_zeroHandle && (long)pl[9] != m_zeroHandle && !tA && n == k && k == m_zeroLen &&
-            ldb == k && (batch == 1 || sB == (long long)k * n) && (unsigned long long)batch * n <= m_zeroRows &&
-            m_mem.version(m_zeroHandle) == m_zeroVersion && !B->view && !B->exposed)
-            zeroFlag = m_zeroFlag;
+        // An operand is the output of a softmax with a causal mask folded in, or its gradient (P V and P^T dY, dS K and Q^T dS
+        // of the explicit attention chain): on one side of the diagonal it holds exact zeros - the softmax kernel raises a
+        // flag on the device if it does not - and the contraction stops or begins at the diagonal.
+        const ZeroTag* tag = nullptr;
+        bool causalA = false;
+        if (!m_zeroTags.empty()) {
+            for (int op = 0; op < 2 && !tag; op++) {
+                const MemItem* it = op == 0 ? B : A;
+                const long h = (long)pl[op == 0 ? 7 : 6];
+                const int side = op == 0 ? n : m, ld = op == 0 ? ldb : lda;
+                const long long stride = op == 0 ? sB : sA;
+                if (h == (long)pl[9] || side != k || ld != k || (batch > 1 && stride != (long long)k * k) || it->view || it->exposed) continue;
+                const ZeroTag* t = zero_tag(h);
+                if (t && t->len == k && (unsigned long long)batch * k <= t->rows) { tag = t; causalA = op == 1; }
+            }
+        }
         HIPCHK(k_gemm2(s, tA, tB, m, n, k, alpha2, (const float*)A->ptr, (const float*)B->ptr, pf[1], (float*)C->ptr, lda,
-                       ldb, ldc, sA, sB, sC, batch, zeroFlag, m_zeroEpoch));
+                       ldb, ldc, sA, sB, sC, batch, tag ? m_zeroFlags + tag->slot : nullptr, tag ? tag->epoch : 0, false, causalA));
         m_mem.touch((long)pl[9]);
         return 0;
     }
@@ -982,11 +1004,14 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         }
         ERRCHK(mem((long)pl[2], &X));
         RANGE(X, xo, n);
-        if (!timing && !X->view && X->views == 0 && !X->exposed && xo == 0 && (size_t)n == X->count && n >= (1 << 20)) {
-            // a large whole tensor: the multiplication waits for the next call that touches the tensor; the mask calls
+        if (!timing && !X->view && X->views == 0 && !X->exposed && xo == 0 && (size_t)n == X->count) {
+            // a whole tensor: the multiplication waits for the next call that touches the tensor; the mask calls
             // of the attention chain (scale, then mask in place) do it in their own pass
             X->pending = pf[0];
+            const ZeroTag* t = std::isfinite(pf[0]) ? zero_tag((long)pl[2]) : nullptr;
+            const ZeroTag tag = t ? *t : ZeroTag();
             m_mem.touch((long)pl[2]);
+            if (tag.len) zero_tag_set((long)pl[2], tag.len, tag.rows, tag.slot, tag.epoch);   // a scaled zero is a zero
             return 0;
         }
         HIPCHK(k_scale(s, X->dt(), (size_t)n, pf[0], PTR(X, xo), PTR(X, xo)));
@@ -1733,17 +1758,23 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                     ERRCHK(flush_pending_product(causal && m_pendingProduct.kind == 0 && m_pendingProduct.m == len && (long long)m_pendingProduct.batch * len == (long long)outer));
                 // a causal pass over fp32 probabilities leaves word of whether every masked entry came out as an exact zero
                 const bool tag = causal && alg != 2 && !Y->view && !Y->exposed;
-                if (tag && !m_zeroFlag) {
-                    HIPCHK(hipMalloc((void**)&m_zeroFlag, sizeof(int)));
-                    HIPCHK(hipMemsetAsync(m_zeroFlag, 0, sizeof(int), s));
+                int slot = 0;
+                if (tag) {
+                    if (!m_zeroFlags) {
+                        HIPCHK(hipMalloc((void**)&m_zeroFlags, ZERO_SLOTS * sizeof(int)));
+                        HIPCHK(hipMemsetAsync(m_zeroFlags, 0, ZERO_SLOTS * sizeof(int), s));
+                    }
+                    slot = m_zeroNext;
+                    m_zeroNext = (m_zeroNext + 1) % ZERO_SLOTS;
+                    m_zeroEpoch = m_zeroEpoch == INT_MAX ? 1 : m_zeroEpoch + 1;
+                    for (size_t i = m_zeroTags.size(); i-- > 0;)   // what the slot said until now is forgotten
+                        if (m_zeroTags[i].slot == slot) m_zeroTags.erase(m_zeroTags.begin() + i);
                 }
-                m_zeroHandle = 0;
-                if (tag) m_zeroEpoch = m_zeroEpoch == INT_MAX ? 1 : m_zeroEpoch + 1;
                 hipError_t e = k_softmax_masked(s, X->dt(), X->ptr, Y->ptr, outer, len, alg == 2, M->ptr, md1, dd1, p.search, p.replace, p.xscale, causal,
-                                                tag ? m_zeroFlag : nullptr, m_zeroEpoch);
+                                                tag ? m_zeroFlags + slot : nullptr, m_zeroEpoch);
                 if (e == hipSuccess) {
                     m_mem.touch((long)pl[6]);
-                    if (tag) { m_zeroHandle = (long)pl[6]; m_zeroVersion = m_mem.version((long)pl[6]); m_zeroLen = len; m_zeroRows = outer; }
+                    if (tag) zero_tag_set((long)pl[6], len, outer, slot, m_zeroEpoch);
                     return 0;
                 }
                 if (e != hipErrorNotSupported) return (long)e;
@@ -1794,8 +1825,15 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         size_t outer = yd->n;
         int len = mode == 0 ? yd->c * yd->h * yd->w : yd->c;
         int inner = mode == 0 ? 1 : yd->h * yd->w;
-        HIPCHK(k_softmax_bwd(s, Y->dt(), Y->ptr, G->ptr, X->ptr, outer, len, inner, alg == 2));
+        // the gradient of a causal softmax has the zeros of its output
+        ZeroTag tag = {};
+        if (alg != 2 && !Y->half && !Y->view && !Y->exposed && !X->view && !X->exposed && softmax_bwd_keeps_zeros(len, inner)) {
+            const ZeroTag* t = zero_tag((long)pl[3]);
+            if (t && t->len == len && t->rows == outer) tag = *t;
+        }
+        HIPCHK(k_softmax_bwd(s, Y->dt(), Y->ptr, G->ptr, X->ptr, outer, len, inner, alg == 2, tag.len, tag.len ? m_zeroFlags + tag.slot : nullptr, tag.epoch));
         m_mem.touch((long)pl[8]);
+        if (tag.len) zero_tag_set((long)pl[8], len, outer, tag.slot, tag.epoch);
         return 0;
     }
 
@@ -1905,7 +1943,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                               M ? (const float*)M->ptr : nullptr, kind, lse, mergedY, drop ? &st->drop : nullptr));
         // the backward pass needs this output (dY . Y per row); the C# layer hands ATTN_BWD a Y buffer that holds the
         // head-merged layout by then (CausalSelfAttentionLayer.cs:668-672), so a copy stays with the handle
-        if (lse) HIPCHK(hipMemcpyAsync(st->ysave, Y->ptr, (size_t)qn * Y->esize(), hipMemcpyDeviceToDevice, s));
+        if (lse) HIPCHK(k_convert(s, Y->dt(), Y->ptr, Y->dt(), st->ysave, (size_t)qn));
         st->lseValid = lse != nullptr;
         st->lastTq = T; st->lastTk = Tk; st->lastBatchMask = batchMask; st->lastMask = hMask;
         m_mem.touch((long)pl[7]);

@@ -12,6 +12,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/mycaffe_hip_abi.h"
@@ -131,9 +132,10 @@ struct PendingMask {
 // computed (the softmax does not read them and the mask call, whenever it is applied, overwrites them).
 //
 // kind 1 is a GEMM call held back the same way: the product of an inner product layer, Y = X W^T written over the whole of
-// Y in fp32.  When the next call on Y is the rank-1 update that adds the bias to every row (ones (m) times bias (n), alpha =
-// beta = 1), both run as one launch with the bias added where the tile is stored - the sum is rounded once either way, so
-// no result changes.  lda/ldb/ldc, the strides and batch are unused then.
+// Y.  When the next call on Y is the rank-1 update that adds the bias to every row (ones (m) times bias (n), alpha =
+// beta = 1), both run as one launch with the bias added where the tile is stored: in fp32 the sum is rounded once either
+// way and no result changes, in 16-bit storage the product is no longer rounded before the bias is added.  lda/ldb/ldc, the
+// strides and batch are unused then.
 struct PendingProduct {
     int kind = 0;
     long hA = 0, hB = 0, hC = 0;
@@ -141,7 +143,7 @@ struct PendingProduct {
     long long sA = 0, sB = 0, sC = 0;
     float alpha = 1.f;
 };
-struct OnesCacheEntry { long handle = 0; uint64_t version = 0; int n = 0; bool ones = false; };
+struct OnesCacheEntry { uint64_t version = 0; int n = 0; bool ones = false; };
 struct PermuteCacheEntry { uint64_t key[6]; int axes; PermuteArgs args; };
 struct ExtensionState {
     void* lib = nullptr;
@@ -192,15 +194,20 @@ private:
     bool mask_is_causal(AttnState* st, long hMask, MemItem* mask, int T);
     bool tril_scan(MemItem* mask, int T, bool* causal);
     bool held_mask_is_causal(long hMask, MemItem* mask, int T);
-    // whether the first n entries of an fp32 blob are all 1.0 (the bias multiplier of an inner product layer): one scan and
-    // host read-back per (handle, content version), a few blobs remembered
+    // whether the first n entries of a blob are all 1.0 (the bias multiplier of an inner product layer): one scan and
+    // host read-back per content of a handle (a model has one such blob per inner product)
     bool vector_is_ones(long h, MemItem* v, int n);
-    OnesCacheEntry m_onesCache[16]; int m_onesNext = 0;
+    std::unordered_map<long, OnesCacheEntry> m_onesCache;
     long m_heldMaskHandle = 0; uint64_t m_heldMaskVersion = 0; int m_heldMaskT = 0; bool m_heldMaskCausal = false;
-    // the last output of a softmax with a causal mask folded in: (handle, content version) of the tensor, its row length
-    // and row count; m_zeroFlag (device) holds m_zeroEpoch if one of its rows has a masked entry that is not exactly zero
-    int* m_zeroFlag = nullptr; int m_zeroEpoch = 0;
-    long m_zeroHandle = 0; uint64_t m_zeroVersion = 0; int m_zeroLen = 0; size_t m_zeroRows = 0;
+    // Tensors whose entries above the diagonal of every (len, len) matrix are exact zeros: outputs of a softmax with a causal
+    // mask folded in, and their gradients.  m_zeroFlags[slot] (device) holds `epoch` if a masked entry was not exactly zero
+    // after all.  A slot belongs to one softmax output and what was derived from it.
+    struct ZeroTag { long handle; uint64_t version; int len; size_t rows; int slot, epoch; };
+    enum { ZERO_SLOTS = 64 };
+    std::vector<ZeroTag> m_zeroTags;
+    int* m_zeroFlags = nullptr; int m_zeroEpoch = 0, m_zeroNext = 0;
+    const ZeroTag* zero_tag(long h);                                            // null: nothing is known
+    void zero_tag_set(long h, int len, size_t rows, int slot, int epoch);
 
     int m_device = 0;
     hipStream_t m_stream = nullptr;

@@ -1,0 +1,54 @@
+"""Softmax rows of any length (quads or single elements in the lanes of one wavefront, one workgroup for a vocabulary), and the
+causal chain whose zeros shorten the products and the gradient pass, at lengths that are no multiple of anything."""
+import numpy as np
+import pytest
+
+from tests.conftest import bf16_round
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("length", [1, 3, 37, 255, 257, 1023, 2047, 2048, 2049, 4100, 8193, 20002, 32768, 32769])
+def test_softmax_forward_and_gradient(dev, length, log, half):
+    rng = np.random.default_rng(length)
+    rows = 5
+    x, g = (rng.standard_normal((rows, length)).astype(np.float32) * 2 for _ in range(2))
+    if half:
+        x, g = bf16_round(x), bf16_round(g)
+    hx, hg, hy, hd = dev.put(x, half), dev.put(g, half), dev.zeros(x.size, half), dev.zeros(x.size, half)
+    hc, d = dev.cuda.CreateCuDNN(), dev.cuda.CreateTensorDesc()
+    dev.cuda.SetTensorDesc(d, rows, length, 1, 1, half)
+    dev.cuda.SoftmaxForward(hc, 2 if log else 1, 0, 1.0, d, hx, 0.0, d, hy)
+    y = dev.get(hy, x.shape)
+    e = x.astype(np.float64) - x.max(1, keepdims=True)
+    ref = e - np.log(np.exp(e).sum(1, keepdims=True)) if log else np.exp(e) / np.exp(e).sum(1, keepdims=True)
+    tol = 1e-2 if half else 2e-6
+    assert np.abs(y - ref).max() <= tol * np.abs(ref).max() + 1e-30
+    dev.cuda.SoftmaxBackward(hc, 2 if log else 1, 0, 1.0, d, hy, d, hg, 0.0, d, hd)
+    y64, g64 = y.astype(np.float64), g.astype(np.float64)
+    want = g64 - np.exp(y64) * g64.sum(1, keepdims=True) if log else (g64 - (g64 * y64).sum(1, keepdims=True)) * y64
+    assert np.abs(dev.get(hd, x.shape) - want).max() <= (1e-2 if half else 1e-5) * max(np.abs(want).max(), 1e-30) + 1e-7
+
+
+@pytest.mark.parametrize("B,T,C,H", [(2, 37, 48, 3), (1, 130, 64, 4), (2, 300, 128, 2)])
+def test_explicit_chain_equals_the_attention_handle(dev, B, T, C, H):
+    from mycaffe_amd.layers import Blob, CausalSelfAttentionLayer
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((B, T, C)).astype(np.float32)
+    w = [rng.standard_normal(s).astype(np.float32) * 0.2 for s in ((3 * C, C), (3 * C,), (C, C), (C,))]
+    dy = rng.standard_normal((B, T, C)).astype(np.float32)
+    out = []
+    for sdpa in (False, True):
+        layer = CausalSelfAttentionLayer(dev.cuda, H, C, T, True, sdpa, training=True)
+        bx, top = Blob(dev.cuda, x.shape), Blob(dev.cuda, x.shape)
+        bx.mutable_cpu_data = x
+        layer.Setup(bx, *w)
+        for _ in range(2):   # the second pass finds the blobs of the first
+            layer.Forward(bx, top)
+            top.mutable_cpu_diff = dy
+            layer.Backward(top, bx)
+        out.append([top.mutable_cpu_data, bx.mutable_cpu_diff] + [b.mutable_cpu_diff for b in layer.c_attn.blobs + layer.c_proj.blobs])
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() <= 2e-5 * np.abs(b).max()
