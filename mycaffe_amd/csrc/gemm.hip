@@ -1,17 +1,12 @@
-// GEMM / GEMV kernels for gfx950.
+// GEMM / GEMV kernels for gfx950; the choice of a kernel for a product (k_gemm, k_gemm_bias, k_gemm_qkv_heads).
 //
-//  * gemm_nt_f32_mfma  : C = alpha*A[M,K]*B[N,K]^T + beta*C, fp32 in, fp32 MFMA
-//                        (v_mfma_f32_32x32x2_f32), 128x128x16 LDS-staged tiles.
-//                        This is the InnerProduct shape (weights stored [N,K]).
-//  * gemm_nt_bf16_mfma : same contraction on bf16 storage with
-//                        v_mfma_f32_32x32x16_bf16, fp32 accumulate, 128x128x32 tiles.
-//  * gemm_generic      : any transpose / stride combination (row-major gemm with
-//                        transposed operands, column-major strided-batched gemm2),
-//                        64x64x16 LDS tiles, fp32 FMA.
-//  * gemv              : HBM-bound y = A x, one wavefront per row, 128-bit loads.
+//  * gemm_f32.hip, gemm_bf16.hip : the tiled matrix-core kernels behind most products.
+//  * gemm_nt_wide_kernel  : 16-bit A B^T of sizes that 256 x 288 or 256 x 192 tiles divide, one workgroup per CU.
+//  * gemm_nt_f32out_kernel: fp32 A B^T of 16-bit operands (the Llama engine's prompt pass), with its epilogues.
+//  * gemm_generic         : any transpose / stride combination (column-major strided-batched gemm2, sizes the tiles do not
+//                           take), 64x64x16 LDS tiles, fp32 FMA.
+//  * gemv                 : HBM-bound y = A x, one wavefront per row, 128-bit loads.
 #include <algorithm>
-
-#include <type_traits>
 
 #include "gemm_common.h"
 
@@ -98,104 +93,11 @@ static hipError_t launch_generic(hipStream_t s, int M, int N, int K, float alpha
 static inline bool gemm_is_tiny(int m, int n, int k) { return (long long)m * n <= 1024 && k <= 64; }
 
 // ---------------------------------------------------------------------------
-// bf16 MFMA, NT, 128x128x32 tiles, 4 wavefronts each 64x64 (2x2 MFMA 32x32x16).
-// Lane l feeds row l%32 with the eight k values 8*(l/32) .. 8*(l/32)+7 of a
-// 16-wide MFMA step: one 128-bit LDS read per operand block and step.
-__global__ __launch_bounds__(256) void gemm_nt_bf16_mfma_kernel(int M, int N, int K, float alpha,
-                                                                const bf16_t* __restrict__ A,
-                                                                const bf16_t* __restrict__ B, float beta,
-                                                                bf16_t* __restrict__ C)
-{
-    constexpr int BM = 128, BN = 128, BK = 32, LDK = BK + 8;  // row stride 80 B
-    __shared__ __attribute__((aligned(16))) bf16_t As[2][BM * LDK];
-    __shared__ __attribute__((aligned(16))) bf16_t Bs[2][BN * LDK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int lr = tid >> 2, lc = (tid & 3) * 8;  // 64 rows x 4 x (8 bf16) per pass, 2 passes
-
-    floatx16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-
-    uint4 ra[2], rb[2];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            int r = lr + p * 64;
-            ra[p] = make_uint4(0, 0, 0, 0);
-            rb[p] = make_uint4(0, 0, 0, 0);
-            if (m0 + r < M && k0 + lc < K) ra[p] = *(const uint4*)(A + (size_t)(m0 + r) * K + k0 + lc);
-            if (n0 + r < N && k0 + lc < K) rb[p] = *(const uint4*)(B + (size_t)(n0 + r) * K + k0 + lc);
-        }
-    };
-    auto sstore = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            int r = lr + p * 64;
-            *(uint4*)(&As[buf][r * LDK + lc]) = ra[p];
-            *(uint4*)(&Bs[buf][r * LDK + lc]) = rb[p];
-        }
-    };
-
-    const int nk = (K + BK - 1) / BK;
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    const int fr = lane & 31, fg = (lane >> 5) * 8;
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) gload((kt + 1) * BK);
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 16) {
-            bf16x8 a[2], b[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                a[t] = *(const bf16x8*)(&As[buf][(wm + t * 32 + fr) * LDK + kk + fg]);
-                b[t] = *(const bf16x8*)(&Bs[buf][(wn + t * 32 + fr) * LDK + kk + fg]);
-            }
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], acc[1][1], 0, 0, 0);
-        }
-        if (kt + 1 < nk) sstore(buf ^ 1);
-        __syncthreads();
-    }
-    const int col_l = lane & 31, row_l = (lane >> 5) * 4;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int c = n0 + wn + j * 32 + col_l;
-            if (c >= N) continue;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                int r = m0 + wm + i * 32 + (v >> 2) * 8 + row_l + (v & 3);
-                if (r < M) {
-                    size_t ci = (size_t)r * N + c;
-                    float o = alpha * acc[i][j][v];
-                    if (beta != 0.f) o += beta * bf16_to_f32(C[ci]);
-                    C[ci] = f32_to_bf16(o);
-                }
-            }
-        }
-}
-
-// ---------------------------------------------------------------------------
-// MFMA, NT, large tiles, bf16 and fp32: 2 x 2 wavefronts, each owning WM x WN MFMA 32x32 tiles, so a workgroup
-// covers (64 WM) x (64 WN) of C.  A 128 x 128 wavefront tile (WM = WN = 4) reads 8 LDS fragments per 16 tile
-// products, a quarter of the LDS traffic per flop of the 64 x 64 wavefront tile, which is what keeps the matrix
-// cores fed; its 256 accumulators live in the accumulation registers.  K is walked in stages of 128 bytes per
-// row through a double-buffered LDS stage (one barrier per stage).  A k-step is one 16-byte fragment per lane
-// and operand: one v_mfma_f32_32x32x16_bf16, or four v_mfma_f32_32x32x2_f32 (lane half h holds k = 4h .. 4h+3 of
-// a group of eight and step e contracts {e, 4 + e}; the slot assignment only has to agree between A and B).
-// Tiles are numbered so that each XCD (workgroup index mod 8) works on a contiguous band of tile rows and
-// re-uses its A rows out of its own L2.
+// MFMA, NT, 16-bit operands with an fp32 result: 2 x 2 wavefronts, each owning WM x WN MFMA 32x32 tiles, so a workgroup
+// covers (64 WM) x (64 WN) of C.  K is walked in stages of 64 through a double-buffered LDS stage (one barrier per stage); a
+// k-step is one 16-byte fragment per lane and operand, one v_mfma_f32_32x32x16_bf16.
+// Tiles are numbered so that each XCD (workgroup index mod 8) works on a contiguous band of tile rows and re-uses its A rows
+// out of its own L2.
 // Epilogues of the prompt pass of the Llama engine (fp32 results of 16-bit operands; llama2_ext.hip), which save the
 // round trip of the product through memory and the kernel that would read it back:
 //   EPI 1, SwiGLU of the stacked W1 | W3 product.  Tile column c multiplies weight row (c & 1) hid + c / 2, so that a
@@ -265,23 +167,14 @@ __device__ __forceinline__ void prompt_epilogue_rope(const PromptEpilogue& pe, i
         pe_store4(which == 1 ? pe.k : pe.v, (((size_t)b * pe.H + h * kvMul + g) * pe.P + p) * pe.hs + d, pe.heads16, o);
 }
 
-// SPLIT (16-bit operands, fp32 C): a row of A is 2 K long, the upper halves of K fp32 values followed by what the upper
-// halves leave over (see k_gemm_bf16_split), and B is walked twice: C = alpha (A_hi + A_lo) B^T + beta C.
-template <typename T, int WM, int WN, int OCC, bool HEADS = false, typename TC = T, bool SPLIT = false, int EPI = 0>
-__global__ __launch_bounds__(256, OCC) void gemm_nt_big_kernel(int M, int N, int K, float alpha, const T* __restrict__ A,
-                                                               const T* __restrict__ B, float beta, TC* __restrict__ C, int tilesN,
-                                                               int tilesTotal, int bandRows, int colBlock, HeadsEpilogue he,
-                                                               PromptEpilogue pe, int ld)
+// SPLIT: a row of A is 2 K long, the upper halves of K fp32 values followed by what the upper halves leave over (see
+// k_gemm_bf16_split), and B is walked twice: C = alpha (A_hi + A_lo) B^T + beta C.
+template <int WM, int WN, int OCC, bool SPLIT, int EPI>
+__global__ __launch_bounds__(256, OCC) void gemm_nt_f32out_kernel(int M, int N, int K, float alpha, const bf16_t* __restrict__ A,
+                                                                  const bf16_t* __restrict__ B, float beta, float* __restrict__ C, int tilesN,
+                                                                  int tilesTotal, int bandRows, int colBlock, PromptEpilogue pe)
 {
-    // K: the contraction length of this launch's products, ld: the distance between rows of A and of B.  With a second
-    // grid dimension, workgroup row y multiplies columns y K .. y K + K - 1 of the operands into the y-th M x N matrix
-    // behind C (partial products of a long contraction, added up by splitk_reduce_kernel).
-    A += (size_t)blockIdx.y * K;
-    B += (size_t)blockIdx.y * K;
-    C += (size_t)blockIdx.y * M * N;
-    static_assert(EPI == 0 || !std::is_same<T, TC>::value, "the prompt epilogues take the fp32 results of 16-bit operands");
-    static_assert(std::is_same<T, TC>::value || (!HEADS && std::is_same<TC, float>::value), "C is of the operands' type, or fp32");
-    static_assert(!SPLIT || !std::is_same<T, TC>::value, "the split product writes fp32");
+    typedef bf16_t T;
     typedef BigTraits<T> TR;
     constexpr int E = TR::E;
     constexpr int BK = 8 * E;                                 // elements per stage and row (128 bytes)
@@ -329,11 +222,11 @@ __global__ __launch_bounds__(256, OCC) void gemm_nt_big_kernel(int M, int N, int
     const T* ga[PA];
     const T* gb[PB];
 #pragma unroll
-    for (int p = 0; p < PA; p++) ga[p] = A + (size_t)min(m0 + lr + p * RPP, M - 1) * (SPLIT ? 2 * K : ld) + lc;
+    for (int p = 0; p < PA; p++) ga[p] = A + (size_t)min(m0 + lr + p * RPP, M - 1) * (SPLIT ? 2 * K : K) + lc;
 #pragma unroll
     for (int p = 0; p < PB; p++) {
         const int c = min(n0 + lr + p * RPP, N - 1);
-        gb[p] = B + (size_t)(EPI == 1 ? (c & 1) * pe.hid + (c >> 1) : c) * ld + lc;
+        gb[p] = B + (size_t)(EPI == 1 ? (c & 1) * pe.hid + (c >> 1) : c) * K + lc;
     }
     T* sa = As + lr * LDK + lc;
     T* sb = Bs + lr * LDK + lc;
@@ -419,163 +312,73 @@ __global__ __launch_bounds__(256, OCC) void gemm_nt_big_kernel(int M, int N, int
     // row of C (lane%32) and register v is column 8*(v/4) + 4*(lane/32) + v%4: four consecutive columns per
     // register quad.
     const int row_l = lane & 31, col_l = (lane >> 5) * 4;
-    if constexpr (!std::is_same<T, TC>::value) {
-        // fp32 results of 16-bit operands.  A lane owns a row of the tile, so its own stores would be 16 bytes each in 32
-        // different rows; each wavefront passes its tile, 32 rows at a time, through its own slice of LDS (free after
-        // the last barrier) and the lanes then walk the rows: consecutive lanes take consecutive quads of columns, and
-        // whatever the epilogue stores is contiguous along the row.
-        constexpr int CW = 32 * WN, LDC = CW + 4;
-        constexpr int LPR = CW / 4, RPI = 64 / LPR;             // lanes per row, rows per pass
-        constexpr int NIT = (32 + RPI - 1) / RPI;
-        float* cs = reinterpret_cast<float*>(smem_raw) + wave * 32 * LDC;
-        const int rr = lane / LPR, cc = (lane % LPR) * 4;
-        const bool vec4 = (N & 3) == 0 && (((uintptr_t)C) & 15) == 0;
+    // fp32 results of 16-bit operands.  A lane owns a row of the tile, so its own stores would be 16 bytes each in 32
+    // different rows; each wavefront passes its tile, 32 rows at a time, through its own slice of LDS (free after
+    // the last barrier) and the lanes then walk the rows: consecutive lanes take consecutive quads of columns, and
+    // whatever the epilogue stores is contiguous along the row.
+    constexpr int CW = 32 * WN, LDC = CW + 4;
+    constexpr int LPR = CW / 4, RPI = 64 / LPR;             // lanes per row, rows per pass
+    constexpr int NIT = (32 + RPI - 1) / RPI;
+    float* cs = reinterpret_cast<float*>(smem_raw) + wave * 32 * LDC;
+    const int rr = lane / LPR, cc = (lane % LPR) * 4;
+    const bool vec4 = (N & 3) == 0 && (((uintptr_t)C) & 15) == 0;
 #pragma unroll
-        for (int i = 0; i < WM; i++) {
+    for (int i = 0; i < WM; i++) {
 #pragma unroll
-            for (int j = 0; j < WN; j++)
+        for (int j = 0; j < WN; j++)
 #pragma unroll
-                for (int g = 0; g < 4; g++)
-                    *(float4*)(cs + row_l * LDC + j * 32 + 8 * g + col_l) =
-                        make_float4(alpha * acc[i][j][4 * g], alpha * acc[i][j][4 * g + 1], alpha * acc[i][j][4 * g + 2], alpha * acc[i][j][4 * g + 3]);
-            // same wavefront wrote and reads: LDS operations of one wavefront complete in order
+            for (int g = 0; g < 4; g++)
+                *(float4*)(cs + row_l * LDC + j * 32 + 8 * g + col_l) =
+                    make_float4(alpha * acc[i][j][4 * g], alpha * acc[i][j][4 * g + 1], alpha * acc[i][j][4 * g + 2], alpha * acc[i][j][4 * g + 3]);
+        // same wavefront wrote and reads: LDS operations of one wavefront complete in order
 #pragma unroll 4
-            for (int it = 0; it < NIT; it++) {
-                const int row = it * RPI + rr, r = m0 + wm + i * 32 + row, c = n0 + wn + cc;
-                if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
-                const float4 v = *(const float4*)(cs + row * LDC + cc);
-                if (EPI != 0) {
-                    // N is a multiple of 4 here: a quad is inside the matrix or outside it
-                    const float a4[4] = {v.x, v.y, v.z, v.w};
-                    if (EPI == 1) prompt_epilogue_swiglu(pe, r, c, a4);
-                    else prompt_epilogue_rope(pe, r, c, a4);
-                    continue;
-                }
-                float* cp = C + (size_t)r * N + c;
-                if (vec4 && c + 3 < N) {
-                    float4 o = v;
-                    if (beta != 0.f) {
-                        const float4 old = *(const float4*)cp;
-                        o.x += beta * old.x; o.y += beta * old.y; o.z += beta * old.z; o.w += beta * old.w;
-                    }
-                    *(float4*)cp = o;
-                } else {
-                    const float a4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        if (c + q < N) cp[q] = a4[q] + (beta != 0.f ? beta * cp[q] : 0.f);
-                }
-            }
-        }
-        return;
-    } else
-    if (m0 + BM <= M && n0 + BN <= N && (HEADS || (beta == 0.f && (((uintptr_t)C) & 15) == 0)) && (N % E) == 0) {
-        // interior tile: each wavefront passes its tile, 32 rows at a time, through its own slice of LDS (free
-        // after the last barrier) and writes whole 16-byte pieces of rows, the lanes covering full cache lines
-        constexpr int CW = 32 * WN, LDC = CW + E;
-        constexpr int LPR = CW / E, RPI = 64 / LPR;            // lanes per row, rows per store instruction
-        constexpr int NIT = (32 + RPI - 1) / RPI;
-        T* cs = smem + wave * 32 * LDC;
-        const int rr = lane / LPR, cc = (lane % LPR) * E;
-#pragma unroll
-        for (int i = 0; i < WM; i++) {
-#pragma unroll
-            for (int j = 0; j < WN; j++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    float b0 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
-                    if (HEADS && he.bias) {
-                        const T* bp = (const T*)he.bias + n0 + wn + j * 32 + 8 * g + col_l;
-                        b0 = TR::ld(bp); b1 = TR::ld(bp + 1); b2 = TR::ld(bp + 2); b3 = TR::ld(bp + 3);
-                    }
-                    TR::st4(cs + row_l * LDC + j * 32 + 8 * g + col_l, alpha * acc[i][j][4 * g] + b0, alpha * acc[i][j][4 * g + 1] + b1,
-                            alpha * acc[i][j][4 * g + 2] + b2, alpha * acc[i][j][4 * g + 3] + b3);
-                }
-            // same wavefront wrote and reads: LDS operations of one wavefront complete in order
-            T* cg = C + (size_t)(m0 + wm + i * 32 + rr) * N + n0 + wn + cc;
-#pragma unroll
-            for (int it = 0; it < NIT; it++) {
-                // lanes past RPI * LPR (row widths that do not divide 64) and rows past the block stay idle
-                if (rr < RPI && it * RPI + rr < 32) {
-                    const u32x4 v = *(const u32x4*)(cs + (it * RPI + rr) * LDC + cc);
-                    if (HEADS) {
-                        const int hr = m0 + wm + i * 32 + it * RPI + rr, hc = n0 + wn + cc;
-                        *(u32x4*)heads_dst<T>(he, hr, hc) = heads_rope_piece<T>(he, hr, hc, v);
-                    }
-                    else *(u32x4*)(cg + (size_t)it * RPI * N) = v;
-                }
-            }
-        }
-        return;
-    }
-    // edge tiles, beta != 0: element-wise (unrolled, so the accumulators are never indexed dynamically)
-    if constexpr (std::is_same<T, TC>::value) {
-#pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-            const int r = m0 + wm + i * 32 + row_l;
-            if (r >= M) continue;
-            if constexpr (HEADS) {
-                // pairs of adjacent columns (N = 3 H hs with hs even: a pair is inside the matrix or outside it)
-#pragma unroll
-                for (int v = 0; v < 16; v += 2) {
-                    const int c = n0 + wn + j * 32 + (v >> 2) * 8 + col_l + (v & 3);
-                    if (c >= N) continue;
-                    float o0 = alpha * acc[i][j][v], o1 = alpha * acc[i][j][v + 1];
-                    if (he.bias) { o0 += TR::ld((const T*)he.bias + c); o1 += TR::ld((const T*)he.bias + c + 1); }
-                    T* dp = heads_dst<T>(he, r, c);
-                    if (he.fcos && c < 2 * he.H * he.hs) {
-                        TR::st(dp, o0); TR::st(dp + 1, o1);
-                        o0 = TR::ld(dp); o1 = TR::ld(dp + 1);      // the values as the storage type holds them
-                        const size_t ti = (size_t)(r % he.seq) * (he.hs >> 1) + ((c % he.hs) >> 1);
-                        heads_rope_pair(he.fcos[ti], he.fsin[ti], o0, o1);
-                    }
-                    TR::st(dp, o0); TR::st(dp + 1, o1);
-                }
+        for (int it = 0; it < NIT; it++) {
+            const int row = it * RPI + rr, r = m0 + wm + i * 32 + row, c = n0 + wn + cc;
+            if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
+            const float4 v = *(const float4*)(cs + row * LDC + cc);
+            if (EPI != 0) {
+                // N is a multiple of 4 here: a quad is inside the matrix or outside it
+                const float a4[4] = {v.x, v.y, v.z, v.w};
+                if (EPI == 1) prompt_epilogue_swiglu(pe, r, c, a4);
+                else prompt_epilogue_rope(pe, r, c, a4);
                 continue;
             }
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int c = n0 + wn + j * 32 + (v >> 2) * 8 + col_l + (v & 3);
-                if (c < N) {
-                    const size_t ci = (size_t)r * N + c;
-                    float o = alpha * acc[i][j][v];
-                    if (HEADS) {
-                        if (he.bias) o += TR::ld((const T*)he.bias + c);
-                        TR::st(heads_dst<T>(he, r, c), o);
-                    } else {
-                        if (beta != 0.f) o += beta * TR::ld(C + ci);
-                        TR::st(C + ci, o);
-                    }
+            float* cp = C + (size_t)r * N + c;
+            if (vec4 && c + 3 < N) {
+                float4 o = v;
+                if (beta != 0.f) {
+                    const float4 old = *(const float4*)cp;
+                    o.x += beta * old.x; o.y += beta * old.y; o.z += beta * old.z; o.w += beta * old.w;
                 }
+                *(float4*)cp = o;
+            } else {
+                const float a4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (c + q < N) cp[q] = a4[q] + (beta != 0.f ? beta * cp[q] : 0.f);
             }
         }
     }
 }
 
-template <typename T, int WM, int WN, int OCC, bool HEADS = false, typename TC = T, bool SPLIT = false, int EPI = 0>
-static hipError_t launch_big(hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, float beta, void* C,
-                             const HeadsEpilogue* heads = nullptr, const PromptEpilogue* prompt = nullptr, int ksplits = 1)
+template <int WM, int WN, int OCC, bool SPLIT, int EPI>
+static hipError_t launch_f32out(hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, float beta, float* C,
+                                const PromptEpilogue* prompt)
 {
-    // ksplits > 1: the contraction in ksplits equal parts, part y into the y-th m x n matrix behind C
-    const int ld = k;
-    k /= ksplits;
+    typedef bf16_t T;
     PromptEpilogue pe = {};
     if (prompt) pe = *prompt;
-    HeadsEpilogue he = {};
-    if (heads) he = *heads;
     constexpr int E = BigTraits<T>::E;
     const int tm = (m + 64 * WM - 1) / (64 * WM), tn = (n + 64 * WN - 1) / (64 * WN);
     const long long total = (long long)tm * tn;
     if (total > (1ll << 30)) return hipErrorInvalidValue;
     const int per = (int)((total + 7) / 8);
     size_t lds = (size_t)2 * (64 * WM + 64 * WN) * (9 * E) * sizeof(T);
-    const size_t ldsEpilogue = std::is_same<T, TC>::value ? (size_t)4 * 32 * (32 * WN + E) * sizeof(T) : (size_t)4 * 32 * (32 * WN + 4) * sizeof(float);
+    const size_t ldsEpilogue = (size_t)4 * 32 * (32 * WN + 4) * sizeof(float);
     if (ldsEpilogue > lds) lds = ldsEpilogue;
     static bool attr = false;   // per instantiation: allow more than the default 64 KB of dynamic LDS
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_nt_big_kernel<T, WM, WN, OCC, HEADS, TC, SPLIT, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_nt_f32out_kernel<WM, WN, OCC, SPLIT, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         attr = true;
     }
@@ -591,8 +394,8 @@ static hipError_t launch_big(hipStream_t s, int m, int n, int k, float alpha, co
             colBlock = (tn + nb - 1) / nb;   // equal-width blocks
         }
     }
-    hipLaunchKernelGGL((gemm_nt_big_kernel<T, WM, WN, OCC, HEADS, TC, SPLIT, EPI>), dim3(per * 8, ksplits), 256, lds, s, m, n, k, alpha, (const T*)A, (const T*)B, beta,
-                       (TC*)C, tn, (int)total, bandRows, colBlock, he, pe, ld);
+    hipLaunchKernelGGL((gemm_nt_f32out_kernel<WM, WN, OCC, SPLIT, EPI>), dim3(per * 8), 256, lds, s, m, n, k, alpha, (const T*)A, (const T*)B, beta,
+                       C, tn, (int)total, bandRows, colBlock, pe);
     return hipGetLastError();
 }
 
@@ -611,11 +414,12 @@ static hipError_t launch_big(hipStream_t s, int m, int n, int k, float alpha, co
 //   * A k-step is one A fragment and WN B fragments for WN tile products; only RB B fragments are held: fragment
 //     f + RB - 1 of the (k-step, column) sequence is read while fragment f is multiplied.
 // No edge handling: launched only where the tiles divide the matrix (wide_tile_fits).
-template <typename T, int WN, bool HEADS>
-__global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int K, float alpha, const T* __restrict__ A,
-                                                               const T* __restrict__ B, T* __restrict__ C, int tilesN,
+template <int WN, bool HEADS>
+__global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int K, float alpha, const bf16_t* __restrict__ A,
+                                                               const bf16_t* __restrict__ B, bf16_t* __restrict__ C, int tilesN,
                                                                int tilesTotal, HeadsEpilogue he)
 {
+    typedef bf16_t T;
     typedef BigTraits<T> TR;
     constexpr int E = TR::E, BK = 8 * E, BM = 256, BN = 32 * WN, KS = 4;   // a stage is 128 bytes of every row
     constexpr int ROWS = BM + BN;                 // rows of one stage: A's 256, then B's 32 WN
@@ -691,11 +495,10 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
         __syncthreads();
     }
 
-    // Epilogue as in gemm_nt_big_kernel: the products are the transposed 32x32 tiles, a lane owns row lane % 32 and
-    // register v is column 8 (v / 4) + 4 (lane / 32) + v % 4.  Each wavefront passes its 32 rows, CH tiles of columns at a
-    // time (all of them in 16-bit storage, three in fp32: eight slices have to fit the LDS), through its own slice of LDS
-    // (free after the last barrier) and stores 16-byte pieces, dealt to the lanes in row-major order.
-    constexpr int CH = sizeof(T) == 2 ? WN : 3;
+    // The products are the transposed 32x32 tiles, a lane owns row lane % 32 and
+    // register v is column 8 (v / 4) + 4 (lane / 32) + v % 4.  Each wavefront passes its 32 rows through its own slice
+    // of LDS (free after the last barrier) and stores 16-byte pieces, dealt to the lanes in row-major order.
+    constexpr int CH = WN;
     static_assert(WN % CH == 0, "whole column chunks");
     constexpr int CW = 32 * CH, LDC = CW + E, LPR = CW / E, NIT = (32 * LPR) / 64;
     static_assert((32 * LPR) % 64 == 0, "the pieces of a 32-row block fill whole store instructions");
@@ -709,7 +512,7 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
             for (int g = 0; g < 4; g++) {
                 const int j = c * CH + jj;
                 float b0 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
-                if (HEADS && he.bias) {
+                if (he.bias) {
                     const T* bp = (const T*)he.bias + n0 + j * 32 + 8 * g + col_l;
                     b0 = TR::ld(bp); b1 = TR::ld(bp + 1); b2 = TR::ld(bp + 2); b3 = TR::ld(bp + 3);
                 }
@@ -731,9 +534,9 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
 // The wide tiles have no edge handling and one workgroup per CU: they are used where they divide the matrix, fill whole
 // rounds of the 256 CUs to at least 85 % and K is long enough to pay for the larger prologue and epilogue.  Returns the
 // tile width in MFMA tiles (9: 256 x 288, 6: 256 x 192) or 0.
-static int wide_tile_fits(int m, int n, int k, int stageElems, const void* A, const void* B, const void* C)
+static int wide_tile_fits(int m, int n, int k, const void* A, const void* B, const void* C)
 {
-    if (m % 256 != 0 || k % stageElems != 0 || k < 8 * stageElems) return 0;
+    if (m % 256 != 0 || k % 64 != 0 || k < 512) return 0;
     if ((((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) != 0) return 0;
     for (int wn : {9, 6}) {
         if (n % (32 * wn) != 0) continue;
@@ -743,49 +546,35 @@ static int wide_tile_fits(int m, int n, int k, int stageElems, const void* A, co
     return 0;
 }
 
-template <typename T, int WN, bool HEADS>
+template <int WN, bool HEADS>
 static hipError_t launch_wide(hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, void* C,
                               const HeadsEpilogue* heads = nullptr)
 {
     HeadsEpilogue he = {};
     if (heads) he = *heads;
-    constexpr int BN = 32 * WN, E = BigTraits<T>::E, CH = sizeof(T) == 2 ? WN : 3;
+    typedef bf16_t T;
+    constexpr int BN = 32 * WN, E = BigTraits<T>::E, CH = WN;
     const int tm = m / 256, tn = n / BN, total = tm * tn, per = (total + 7) / 8;
     // two stages of (256 + BN) rows x 128 bytes, or the epilogue's eight slices of 32 x (32 CH + E) elements, whichever is larger
     const size_t lds = std::max((size_t)2 * (256 + BN) * 128, (size_t)8 * 32 * (32 * CH + E) * sizeof(T));
     static bool attr = false;   // per instantiation: allow more than the default 64 KB of dynamic LDS
     if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_nt_wide_kernel<T, WN, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_nt_wide_kernel<WN, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         attr = true;
     }
-    hipLaunchKernelGGL((gemm_nt_wide_kernel<T, WN, HEADS>), dim3(per * 8), 512, lds, s, m, n, k, alpha, (const T*)A, (const T*)B,
+    hipLaunchKernelGGL((gemm_nt_wide_kernel<WN, HEADS>), dim3(per * 8), 512, lds, s, m, n, k, alpha, (const T*)A, (const T*)B,
                        (T*)C, tn, total, he);
     return hipGetLastError();
 }
 
-// Fewer 128 x 128 tiles than CUs: 64 x 128 tiles if they give every CU one, 64 x 64 otherwise (three or four of these
-// small workgroups fit a CU, so more tiles than CUs is welcome).
-template <typename T, bool HEADS>
-static bool launch_small_if_few(hipError_t* e, hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, float beta, void* C,
-                                const HeadsEpilogue* heads = nullptr)
-{
-    const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-    if (t128 >= 200) return false;
-    const long long t64x128 = (long long)((m + 63) / 64) * ((n + 127) / 128);
-    if (t64x128 >= 200) *e = launch_big<T, 1, 2, 3, HEADS>(s, m, n, k, alpha, A, B, beta, C, heads);
-    else *e = launch_big<T, 1, 1, 3, HEADS>(s, m, n, k, alpha, A, B, beta, C, heads);
-    return true;
-}
-
-// one stage of K is 128 bytes of a row: 64 elements in 16-bit storage, 32 in fp32
-template <typename T, bool HEADS>
+template <bool HEADS>
 static bool launch_wide_if_fits(hipError_t* e, hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, void* C,
                                 const HeadsEpilogue* heads = nullptr)
 {
-    switch (wide_tile_fits(m, n, k, 8 * BigTraits<T>::E, A, B, C)) {
-    case 9: *e = launch_wide<T, 9, HEADS>(s, m, n, k, alpha, A, B, C, heads); return true;
-    case 6: *e = launch_wide<T, 6, HEADS>(s, m, n, k, alpha, A, B, C, heads); return true;
+    switch (wide_tile_fits(m, n, k, A, B, C)) {
+    case 9: *e = launch_wide<9, HEADS>(s, m, n, k, alpha, A, B, C, heads); return true;
+    case 6: *e = launch_wide<6, HEADS>(s, m, n, k, alpha, A, B, C, heads); return true;
     }
     return false;
 }
@@ -819,8 +608,7 @@ __global__ void gemm_rank1_kernel(int m, int n, float alpha, const T* __restrict
 
 // Fallback of the fused QKV projection: the plain product in `tmp` (M x 3C) is split, bias added, into the three
 // (B,H,T,hs) tensors in one pass.
-template <typename T>
-__global__ void qkv_split_heads_kernel(const T* __restrict__ tmp, size_t total, int N, HeadsEpilogue he)
+__global__ void qkv_split_heads_kernel(const bf16_t* __restrict__ tmp, size_t total, int N, HeadsEpilogue he)
 {
     // one pair of adjacent columns per step (hs is even when the rotation is asked for; otherwise N may be odd)
     const bool pairs = he.fcos != nullptr;
@@ -829,45 +617,44 @@ __global__ void qkv_split_heads_kernel(const T* __restrict__ tmp, size_t total, 
         const size_t i = pairs ? 2 * s : s;
         const int r = (int)(i / N), c = (int)(i - (size_t)r * N);
         float o = ldf(tmp, i);
-        if (he.bias) o += ldf((const T*)he.bias, c);
-        T* dp = heads_dst<T>(he, r, c);
+        if (he.bias) o += ldf((const bf16_t*)he.bias, c);
+        bf16_t* dp = heads_dst<bf16_t>(he, r, c);
         if (!pairs) { stf(dp, 0, o); continue; }
         float o1 = ldf(tmp, i + 1);
-        if (he.bias) o1 += ldf((const T*)he.bias, c + 1);
+        if (he.bias) o1 += ldf((const bf16_t*)he.bias, c + 1);
         if (c < 2 * he.H * he.hs) {
             stf(dp, 0, o); stf(dp, 1, o1);
             o = ldf(dp, 0); o1 = ldf(dp, 1);                       // the values as the storage type holds them
-            const size_t ti = (size_t)(r % he.seq) * (he.hs >> 1) + ((c % he.hs) >> 1);
+            const size_t ti = heads_rope_at(he, r, c);
             heads_rope_pair(he.fcos[ti], he.fsin[ti], o, o1);
         }
         stf(dp, 0, o); stf(dp, 1, o1);
     }
 }
 
-// X (m x kk) W^T (n x kk) through the tile kernels' HEADS epilogue `he`; in 16-bit storage, shapes and addresses the tile
-// kernels do not take go through a scratch matrix (m x n) and a splitting pass
-static bool gemm_heads_through_tmp(int kk, int rowUnit, const void* X, const void* W, const void* d0, const void* d1, const void* d2)
+static GemmB16 b16_product(bool tA, bool tB, int m, int n, int k, float alpha, const void* A, const void* B, float beta, void* C)
 {
-    const bool aligned = (((uintptr_t)X | (uintptr_t)W | (uintptr_t)d0 | (uintptr_t)d1 | (uintptr_t)d2) % 16 == 0) && rowUnit % 8 == 0;
-    return !(aligned && kk % 64 == 0);
+    return GemmB16{m, n, k, (const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, !tA, tB, alpha, beta, nullptr, nullptr};
 }
-static size_t gemm_heads_workspace_bytes(DType dt, int m, int n, int kk, int rowUnit, const void* X, const void* W, const void* d0, const void* d1, const void* d2)
+// X (m x kk) W^T (n x kk) through the tile kernels' HEADS epilogue `he`; in 16-bit storage, operands the tile kernels do not
+// take go through a scratch matrix (m x n) and a splitting pass
+static size_t gemm_heads_workspace_bytes(DType dt, int m, int n, int kk, const void* X, const void* W)
 {
     if (dt == F32) return gemm_f32_workspace_bytes(m, n, kk, 1, false);
-    return gemm_heads_through_tmp(kk, rowUnit, X, W, d0, d1, d2) ? (size_t)m * n * sizeof(bf16_t) : 0;
+    return gemm_b16_takes(b16_product(false, true, m, n, kk, 1.f, X, W, 0.f, nullptr)) ? gemm_b16_workspace_bytes(m, n, kk) : (size_t)m * n * sizeof(bf16_t);
 }
-size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W, const void* Y)
+size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W)
 {
-    return gemm_heads_workspace_bytes(dt, m, n, k, n, X, W, Y, Y, Y);
+    return gemm_heads_workspace_bytes(dt, m, n, k, X, W);
 }
-size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* q, const void* k, const void* v)
+size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W)
 {
-    return gemm_heads_workspace_bytes(dt, B * T, 3 * H * hs, H * hs, hs, X, W, q, k, v);
+    return gemm_heads_workspace_bytes(dt, B * T, 3 * H * hs, H * hs, X, W);
 }
 
-// (tiles256: the 256 x 256 tiles may be chosen as k_gemm chooses them)
-static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int kk, const void* X, const void* W, const HeadsEpilogue& he,
-                                      int rowUnit, void* ws, size_t wsBytes, bool tiles256)
+// Y: row-major result, only the bias of `he` is added; null: through `he`
+static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int kk, const void* X, const void* W, const HeadsEpilogue& he, void* Y,
+                                      void* ws, size_t wsBytes)
 {
     if (dt == F32) {
         GemmF32 g = {};
@@ -876,28 +663,26 @@ static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int
         g.lda = g.ldb = kk; g.ldc = n;
         g.aK = g.bK = true;
         g.alpha = 1.f; g.batch = 1;
-        g.heads = &he;
+        g.C = (float*)Y;
+        if (Y) g.bias = (const float*)he.bias;
+        else g.heads = &he;
         return gemm_f32(s, g, ws, wsBytes);
     }
-    const long long t256 = (long long)((m + 255) / 256) * ((n + 255) / 256);
-    const bool full256 = tiles256 && (double)t256 / (double)(((t256 + 255) / 256) * 256) >= 0.85;
-    const bool aligned = !gemm_heads_through_tmp(kk, rowUnit, X, W, he.dst[0], he.dst[1], he.dst[2]);   // and K in whole stages
-    const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-    if (aligned && dt == BF16) {
-        hipError_t e;
-        if (full256 && kk >= 2048) return launch_big<bf16_t, 4, 4, 1, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
-        if (launch_wide_if_fits<bf16_t, true>(&e, s, m, n, kk, 1.f, X, W, nullptr, &he)) return e;
-        if (launch_small_if_few<bf16_t, true>(&e, s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he)) return e;
-        if (n % 192 == 0 && t128 <= 512) return launch_big<bf16_t, 2, 3, 2, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
-        return launch_big<bf16_t, 2, 2, 2, true>(s, m, n, kk, 1.f, X, W, 0.f, nullptr, &he);
-    }
+    hipError_t fit;
+    if (Y ? launch_wide_if_fits<false>(&fit, s, m, n, kk, 1.f, X, W, Y, &he)
+          : he.hs % 8 == 0 && (((uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0 &&
+                launch_wide_if_fits<true>(&fit, s, m, n, kk, 1.f, X, W, he.dst[0], &he)) return fit;
+    GemmB16 g = b16_product(false, true, m, n, kk, 1.f, X, W, 0.f, Y);
+    if (Y) g.bias = (const bf16_t*)he.bias;
+    else g.heads = &he;
+    if (gemm_b16_takes(g)) return gemm_b16(s, g, ws, wsBytes);
     // any other shape: plain product into the caller's scratch matrix, then one splitting pass
     if (!ws || wsBytes < (size_t)m * n * sizeof(bf16_t)) return hipErrorInvalidValue;
     hipError_t e = k_gemm(s, dt, false, true, m, n, kk, 1.f, X, W, 0.f, ws);
     if (e != hipSuccess) return e;
     const size_t total = (size_t)m * n;
     const int grid = (int)std::min<size_t>((total + 255) / 256, 8192);
-    hipLaunchKernelGGL(qkv_split_heads_kernel<bf16_t>, grid, 256, 0, s, (const bf16_t*)ws, total, n, he);
+    hipLaunchKernelGGL(qkv_split_heads_kernel, grid, 256, 0, s, (const bf16_t*)ws, total, n, he);
     return hipGetLastError();
 }
 
@@ -907,22 +692,18 @@ hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs
     if (fcos && (!fsin || ropeSeq < 1 || (hs & 1))) return hipErrorInvalidValue;
     const int m = B * T, C = H * hs, n = 3 * C, kk = C;
     if (m <= 0 || C <= 0) return hipSuccess;
-    HeadsEpilogue he;
-    he.bias = bias; he.dst[0] = q; he.dst[1] = k; he.dst[2] = v; he.T = T; he.H = H; he.hs = hs;
-    he.fcos = fcos; he.fsin = fcos ? fsin : nullptr; he.seq = fcos ? ropeSeq : 1;
-    return gemm_heads_dispatch(s, dt, m, n, kk, X, W, he, hs, ws, wsBytes, false);
+    const HeadsEpilogue he = heads_epilogue(bias, q, k, v, T, H, hs, fcos, fcos ? fsin : nullptr, fcos ? ropeSeq : 1);
+    return gemm_heads_dispatch(s, dt, m, n, kk, X, W, he, nullptr, ws, wsBytes);
 }
 
 // Y (m x n) = X (m x k) W^T (n x k) + bias (n): the inner product layer's forward in one launch (InnerProductLayer.cs:
-// 372-417 issues the product and a rank-1 update with a vector of ones).  The HEADS epilogue with one head of n values
-// over m positions is the plain row-major layout, so the same kernels serve.
+// 372-417 issues the product and a rank-1 update with a vector of ones).  (One head of n values over m positions, for the
+// pass that splits a product the tile kernels do not take.)
 hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes)
 {
     if (m <= 0 || n <= 0) return hipSuccess;
-    HeadsEpilogue he;
-    he.bias = bias; he.dst[0] = he.dst[1] = he.dst[2] = Y; he.T = m; he.H = 1; he.hs = n;
-    he.fcos = nullptr; he.fsin = nullptr; he.seq = 1;
-    return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, n, ws, wsBytes, true);
+    const HeadsEpilogue he = heads_epilogue(bias, Y, Y, Y, m, 1, n, nullptr, nullptr, 1);
+    return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, Y, ws, wsBytes);
 }
 
 // C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
@@ -940,11 +721,11 @@ static hipError_t gemm_bf16_f32_tiles(hipStream_t s, int m, int n, int k, float 
     const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
     if (t128 < 200) {
         const long long t64x128 = (long long)((m + 63) / 64) * ((n + 127) / 128);
-        if (t64x128 >= 200) return launch_big<bf16_t, 1, 2, 3, false, float, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, nullptr, pe);
-        return launch_big<bf16_t, 1, 1, 3, false, float, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, nullptr, pe);
+        if (t64x128 >= 200) return launch_f32out<1, 2, 3, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
+        return launch_f32out<1, 1, 3, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
     }
-    if (n % 192 == 0 && t128 <= 512) return launch_big<bf16_t, 2, 3, 2, false, float, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, nullptr, pe);
-    return launch_big<bf16_t, 2, 2, 2, false, float, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, nullptr, pe);
+    if (n % 192 == 0 && t128 <= 512) return launch_f32out<2, 3, 2, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
+    return launch_f32out<2, 2, 2, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
 }
 static bool bf16_f32_operands_ok(int k, const void* A, const void* W) { return k > 0 && k % 64 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0; }
 hipError_t k_gemm_bf16_f32(hipStream_t s, int m, int n, int k, float alpha, const void* A, bool split, const void* W, float beta, float* C)
@@ -979,101 +760,11 @@ hipError_t k_gemm_bf16_qkv_rope(hipStream_t s, int B, int P, int H, int kvH, int
     return split ? gemm_bf16_f32_tiles<true, 2>(s, m, n, k, 1.f, A, Wqkv, 0.f, nullptr, &pe) : gemm_bf16_f32_tiles<false, 2>(s, m, n, k, 1.f, A, Wqkv, 0.f, nullptr, &pe);
 }
 
-// (rows, cols) -> (cols, rows), 64 x 64 elements per workgroup: 16-byte pieces in, a padded LDS tile, 16-byte pieces out
-// (rows and cols multiples of 16 bytes' worth of elements; edge tiles are clipped piece by piece)
-template <typename T>
-__global__ __launch_bounds__(256) void transpose2d_kernel(const T* __restrict__ x, T* __restrict__ y, int rows, int cols)
-{
-    constexpr int E = 16 / sizeof(T), PPR = 64 / E, NP = 64 * PPR / 256;   // elements per piece, pieces per tile row, pieces per thread
-    __shared__ T tile[64][64 + (sizeof(T) == 2 ? 2 : 1)];
-    const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const int p = threadIdx.x + 256 * i, r = p / PPR, c = (p % PPR) * E;
-        if (r0 + r < rows && c0 + c < cols) {
-            const u32x4 v = *(const u32x4*)(x + (size_t)(r0 + r) * cols + c0 + c);
-            const T* e = reinterpret_cast<const T*>(&v);
-#pragma unroll
-            for (int j = 0; j < E; j++) tile[r][c + j] = e[j];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const int p = threadIdx.x + 256 * i, c = p / PPR, r = (p % PPR) * E;   // output row c0 + c, columns r0 + r ..
-        if (c0 + c < cols && r0 + r < rows) {
-            u32x4 v;
-            T* e = reinterpret_cast<T*>(&v);
-#pragma unroll
-            for (int j = 0; j < E; j++) e[j] = tile[r + j][c];
-            *(u32x4*)(y + (size_t)(c0 + c) * rows + r0 + r) = v;
-        }
-    }
-}
-
-static hipError_t transpose2d(hipStream_t s, const void* x, void* y, int rows, int cols)
-{
-    dim3 grid((cols + 63) / 64, (rows + 63) / 64);
-    if (grid.y > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(transpose2d_kernel<bf16_t>, grid, 256, 0, s, (const bf16_t*)x, (bf16_t*)y, rows, cols);
-    return hipGetLastError();
-}
-
-// The transpose combinations other than A B^T in 16-bit storage (InnerProductLayer backward: data gradient dY W, weight
-// gradient dY^T X, InnerProductLayer.cs:429-494).  The tile kernels want both operands with the contracted index at unit
-// stride; an operand that lies the other way is turned once into scratch memory and the product then runs on them
-// (8192 x 768 x 2304: 604 -> 36 us, the weight gradient 1778 -> 63 us against the strided scalar kernel).
-static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
-
-// A long contraction with few tiles (weight gradients: K is the token count) is cut into 2 .. 16 equal parts, one row of
-// workgroups of 128 x 128 tiles each, until the launch has some 400 workgroups; every part stays 512 long at least.
-static int gemm_ksplits(int m, int n, int k)
-{
-    const int bk = 64;
-    const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-    if (t128 >= 200 || k < 2048 || ((long long)m * n) % 4) return 1;
-    int S = 1;
-    while (S < 16 && t128 * S < 400 && k % (2 * S * bk) == 0 && k / (2 * S) >= 512) S *= 2;
-    return S;
-}
-// C = sum of the S partial products (fp32, alpha already applied) + beta C
-template <typename T>
-__global__ void splitk_reduce_kernel(const float* __restrict__ part, int S, size_t total4, float beta, T* __restrict__ C)
-{
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total4; e += (size_t)blockDim.x * gridDim.x) {
-        float4 a = *(const float4*)(part + 4 * e);
-        for (int z = 1; z < S; z++) {
-            const float4 b = *(const float4*)(part + (size_t)z * total4 * 4 + 4 * e);
-            a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-        }
-        float v[4] = {a.x, a.y, a.z, a.w};
-        if (beta != 0.f) {
-            float c[4];
-            Quad<T>::load(C + 4 * e, c);
-#pragma unroll
-            for (int q = 0; q < 4; q++) v[q] += beta * c[q];
-        }
-        Quad<T>::store(C + 4 * e, v);
-    }
-}
-static bool gemm_turns_operands(bool tA, bool tB, int m, int n, int k)
-{
-    if (!tA && tB) return false;
-    if (k < 64 || k % 8 || (tA && m % 8) || (!tB && n % 8)) return false;
-    return (double)m * n >= 64.0 * 64.0;
-}
-static size_t gemm_turned_bytes(bool tA, bool tB, int m, int n, int k)
-{
-    return (tA ? round256((size_t)m * k * sizeof(bf16_t)) : 0) + (!tB ? round256((size_t)n * k * sizeof(bf16_t)) : 0);
-}
 size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k)
 {
     if (m <= 0 || n <= 0 || k <= 1) return 0;
     if (dt == F32) return gemm_is_tiny(m, n, k) ? 0 : gemm_f32_workspace_bytes(m, n, k, 1, false);
-    const bool nt = !tA && tB;
-    if (!nt && !gemm_turns_operands(tA, tB, m, n, k)) return 0;
-    const int S = k % 8 == 0 ? gemm_ksplits(m, n, k) : 1;
-    return (nt ? 0 : gemm_turned_bytes(tA, tB, m, n, k)) + (S > 1 ? (size_t)S * m * n * sizeof(float) : 0);
+    return gemm_b16_takes(b16_product(tA, tB, m, n, k, 1.f, nullptr, nullptr, 0.f, nullptr)) ? gemm_b16_workspace_bytes(m, n, k) : 0;
 }
 
 hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k, float alpha, const void* A,
@@ -1089,23 +780,11 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
         g.alpha = alpha; g.beta = beta; g.batch = 1;
         return gemm_f32(s, g, ws, wsBytes);
     }
-    if (dt == BF16 && ws && k > 1 && (((uintptr_t)A | (uintptr_t)B | (uintptr_t)ws) % 16 == 0) && gemm_turns_operands(tA, tB, m, n, k) &&
-        wsBytes >= k_gemm_workspace_bytes(dt, tA, tB, m, n, k)) {
-        const void *a2 = A, *b2 = B;
-        char* w = (char*)ws;
-        if (tA) {   // stored (k, m)
-            hipError_t e = transpose2d(s, A, w, k, m);
-            if (e != hipSuccess) return e;
-            a2 = w;
-            w += round256((size_t)m * k * sizeof(bf16_t));
-        }
-        if (!tB) {  // stored (k, n)
-            hipError_t e = transpose2d(s, B, w, k, n);
-            if (e != hipSuccess) return e;
-            b2 = w;
-            w += round256((size_t)n * k * sizeof(bf16_t));
-        }
-        return k_gemm(s, dt, false, true, m, n, k, alpha, a2, b2, beta, C, w, wsBytes - (size_t)(w - (char*)ws));
+    if (dt == BF16 && k > 1) {
+        hipError_t e;
+        if (!tA && tB && beta == 0.f && launch_wide_if_fits<false>(&e, s, m, n, k, alpha, A, B, C)) return e;
+        const GemmB16 g = b16_product(tA, tB, m, n, k, alpha, A, B, beta, C);
+        if (gemm_b16_takes(g)) return gemm_b16(s, g, ws, wsBytes);
     }
     if (k == 1) {
         const size_t es = dt == F32 ? 4 : 2;
@@ -1119,38 +798,6 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
         return hipGetLastError();
     }
     if (k <= 0) k = 0;
-    // MFMA path in 16-bit storage: A (m,k) and B (n,k) both k-contiguous, 16-byte aligned rows
-    const bool aligned = (k % 8 == 0) && (((uintptr_t)A | (uintptr_t)B) % 16 == 0) && k >= 8;
-    if (dt == BF16 && !tA && tB && aligned) {
-        dim3 grid((n + 127) / 128, (m + 127) / 128);
-        if (grid.y > 65535) return hipErrorInvalidValue;
-        // Large-tile kernels need whole 128-byte stages along K.  256 x 256 tiles (one wavefront per SIMD, 128 x 128
-        // per wavefront) win once K is long enough to amortise their prologue and the tile count fills the 256 CUs
-        // evenly; 128 x 128 tiles with two workgroups per CU otherwise, 128 x 192 when that gives at most one round
-        // of workgroups.
-        const long long t256 = (long long)((m + 255) / 256) * ((n + 255) / 256);
-        const double fill = (double)t256 / (double)(((t256 + 255) / 256) * 256);
-        const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-        const int S = ws && (((uintptr_t)ws | (uintptr_t)C) % 16 == 0) ? gemm_ksplits(m, n, k) : 1;
-        if (S > 1 && wsBytes >= (size_t)S * m * n * sizeof(float)) {
-            hipError_t e = launch_big<bf16_t, 2, 2, 2, false, float>(s, m, n, k, alpha, A, B, 0.f, ws, nullptr, nullptr, S);
-            if (e != hipSuccess) return e;
-            const size_t total4 = (size_t)m * n / 4;
-            const int g = (int)std::min<size_t>((total4 + 255) / 256, 4096);
-            hipLaunchKernelGGL(splitk_reduce_kernel<bf16_t>, g, 256, 0, s, (const float*)ws, S, total4, beta, (bf16_t*)C);
-            return hipGetLastError();
-        }
-        if (k % 64 == 0) {
-            if (k >= 2048 && fill >= 0.85) return launch_big<bf16_t, 4, 4, 1>(s, m, n, k, alpha, A, B, beta, C);
-            hipError_t e;
-            if (beta == 0.f && launch_wide_if_fits<bf16_t, false>(&e, s, m, n, k, alpha, A, B, C)) return e;
-            if (launch_small_if_few<bf16_t, false>(&e, s, m, n, k, alpha, A, B, beta, C)) return e;
-            if (n % 192 == 0 && t128 <= 512) return launch_big<bf16_t, 2, 3, 2>(s, m, n, k, alpha, A, B, beta, C);
-            return launch_big<bf16_t, 2, 2, 2>(s, m, n, k, alpha, A, B, beta, C);
-        }
-        hipLaunchKernelGGL(gemm_nt_bf16_mfma_kernel, grid, 256, 0, s, m, n, k, alpha, (const bf16_t*)A, (const bf16_t*)B, beta, (bf16_t*)C);
-        return hipGetLastError();
-    }
     GemmStrides st;
     st.ai = tA ? 1 : k;  st.ak = tA ? m : 1;   // A stored (m,k) or (k,m)
     st.bk = tB ? 1 : n;  st.bj = tB ? k : 1;   // B stored (k,n) or (n,k)

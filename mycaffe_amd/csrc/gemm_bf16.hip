@@ -1,0 +1,437 @@
+// 16-bit GEMM on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16), any operand layout, fp32 accumulation, gfx950.
+//
+// WVM x WVN wavefronts of WM x WN MFMA tiles each cover (32 WVM WM) x (32 WVN WN) of C and walk K in stages of 64 that go
+// from global memory straight into LDS (buffer loads to LDS: no staging registers, no writes to issue), double-buffered, one
+// barrier per stage.  At this matrix rate a tile is bound by what it moves: 128 x 128 needs 64 bytes per clock and CU from
+// L2, all that L2 has; 256 x 256 half of that.  Large products therefore take 256 x 256 or 256 x 192 with eight
+// wavefronts, one workgroup per CU, whichever leaves the shorter last round, small ones the tile that fills the chip.
+//
+//   * k at unit stride: LDS holds [row][64 k] without padding, the 16-byte piece c of row r at position c ^ ((r >> 1) & 7)
+//     (sixteen consecutive rows read by a 128-bit access then fall on sixteen bank groups).
+//   * row index at unit stride: LDS holds [k][row] as it is stored, the 32-row blocks of row k exchanged by a function of
+//     k & 3, and the fragments are read with the transposing 64-bit access (ds_read_b64_tr_b16: lane i of a group of
+//     sixteen receives column i of the 4 x 16 block whose rows four lanes each address).  Gradients need no operand turned
+//     in memory first (57 of 570 us of an MLP's training step).
+//   * The contraction may end anywhere a 16-byte chunk ends: chunks past the end get an offset outside the buffer, which
+//     reads as zeros.
+#include "gemm_common.h"
+
+namespace mch {
+
+struct GemmB16Args {
+    int M, N, K;
+    const bf16_t *A, *B;
+    bf16_t* C;
+    int lda, ldb;
+    float alpha, beta;
+    int tilesM, tilesN, parts, kChunk;
+    float* part;              // kChunk < K: partial products, [part][M][N]
+    bool vecC;
+    const bf16_t* bias;
+};
+
+#define LDS3(p) ((__attribute__((address_space(3))) void*)(p))
+
+// One operand fragment.  The transposing reads are written as instructions: as builtins the compiler makes each of them wait
+// for every fetch into LDS that is under way, the next stage's included (8000 x 768 x 3072 with one such operand: 109 us).
+// tr_read issues the two reads of k-step ks (ROWB bytes between k rows), tr_wait makes the values usable.
+struct TrFragment { union { u32x4 w; uint2 h[2]; }; };
+template <int ROWB> __device__ __forceinline__ void tr_read(uint32_t addr, int ks, TrFragment& o)
+{
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(o.h[0]) : "v"(addr), "n"(ks * 16 * ROWB) : "memory");
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(o.h[1]) : "v"(addr), "n"((ks * 16 + 4) * ROWB) : "memory");
+}
+__device__ __forceinline__ void tr_wait(TrFragment& o) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o.h[0]), "+v"(o.h[1]) : : "memory"); }
+
+// sixteen bytes per lane from the buffer to the wavefront's 1 KB of LDS at `lds` (wavefront-uniform)
+__device__ __forceinline__ void lds_fetch16(__amdgpu_buffer_rsrc_t rs, bf16_t* lds, uint32_t voffset, int soffset)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS3(lds), 16, voffset, soffset, 0, 0);
+}
+
+// exchange of 32-row blocks (64 bytes, four 16-byte chunks) in row k of a [k][row] stage: four consecutive k of one block of
+// rows have to lie on four different quarters of the 256 bytes of banks; rows are ROWB bytes apart
+template <int ROWB> __device__ __forceinline__ int block_swizzle(int k)
+{
+    return ROWB % 256 == 0 ? (k & 3) * 4 : ((k >> 1) & 1) * 4;   // in chunks; rows 128 bytes apart modulo 256 alternate already
+}
+
+// the bias of eight columns from c on (0 past the matrix)
+__device__ __forceinline__ void b16_bias8(const GemmB16Args& g, int c, float (&bias)[8])
+{
+#pragma unroll
+    for (int q = 0; q < 8; q++) bias[q] = g.bias && c + q < g.N ? bf16_to_f32(g.bias[c + q]) : 0.f;
+}
+
+// eight values of row r from column c on (inside the matrix up to N), alpha applied, and the bias, to C or through the heads
+// epilogue, whose column c of row 0 is at col
+template <bool HEADS>
+__device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<HEADS>& hp, int r, int c, const float (&bias)[8], bf16_t* col, float (&v)[8])
+{
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] += bias[q];
+    if (g.vecC) {
+        bf16_t* cp = g.C + (size_t)r * g.N + c;
+        if constexpr (HEADS) cp = col + heads_row(hp.he, r);
+        if (!HEADS && g.beta != 0.f) {
+            const u32x4 o = *(const u32x4*)cp;
+            const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                v[2 * q] += g.beta * __uint_as_float(w[q] << 16);
+                v[2 * q + 1] += g.beta * __uint_as_float(w[q] & 0xffff0000u);
+            }
+        }
+        u32x4 p;
+        p.x = pack2_bf16(v[0], v[1]); p.y = pack2_bf16(v[2], v[3]); p.z = pack2_bf16(v[4], v[5]); p.w = pack2_bf16(v[6], v[7]);
+        if constexpr (HEADS) p = heads_rope_piece<bf16_t>(hp.he, r, c, p);
+        *(u32x4*)cp = p;
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q += 2) {
+        if (c + q >= g.N) continue;
+        const bool two = c + q + 1 < g.N;
+        if constexpr (HEADS) {
+            float o0 = bf16_to_f32(f32_to_bf16(v[q])), o1 = bf16_to_f32(f32_to_bf16(v[q + 1]));   // as the storage type holds them
+            if (hp.he.fcos && c + q < 2 * hp.he.H * hp.he.hs) {
+                const size_t ti = heads_rope_at(hp.he, r, c + q);
+                heads_rope_pair(hp.he.fcos[ti], hp.he.fsin[ti], o0, o1);
+            }
+            *heads_dst<bf16_t>(hp.he, r, c + q) = f32_to_bf16(o0);
+            if (two) *heads_dst<bf16_t>(hp.he, r, c + q + 1) = f32_to_bf16(o1);
+        } else {
+            bf16_t* cp = g.C + (size_t)r * g.N + c + q;
+            cp[0] = f32_to_bf16(v[q] + (g.beta != 0.f ? g.beta * bf16_to_f32(cp[0]) : 0.f));
+            if (two) cp[1] = f32_to_bf16(v[q + 1] + (g.beta != 0.f ? g.beta * bf16_to_f32(cp[1]) : 0.f));
+        }
+    }
+}
+
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS>
+__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
+{
+    constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64, KS = 4;
+    constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;               // 16-byte chunks per thread and stage
+    constexpr int STAGE = (BM + BN) * BK;                           // elements of one stage: A's part, then B's
+    constexpr int NMF = WM * WN;
+    static_assert(PA * NT == BM * 8 && PB * NT == BN * 8, "whole chunks per thread");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    bf16_t* smem = reinterpret_cast<bf16_t*>(smem_raw);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = g.tilesM * g.tilesN, total = tiles * g.parts, per = (total + 7) / 8;
+    const int item = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);   // each XCD takes a contiguous run
+    if (item >= total) return;
+    const int part = item / tiles, tile = item - part * tiles;
+    constexpr int GROUP = 4;   // tile rows per group, walked down first: few rows of A and columns of B in flight per XCD
+    const int group = tile / (GROUP * g.tilesN), inGroup = tile - group * GROUP * g.tilesN;
+    const int groupRows = min(GROUP, g.tilesM - group * GROUP);
+    const int M = g.M, N = g.N;
+    const int m0 = (group * GROUP + inGroup % groupRows) * BM, n0 = (inGroup / groupRows) * BN;
+    const bool split = g.kChunk < g.K;
+    const int kBegin = split ? part * g.kChunk : 0, kEnd = min(g.K, kBegin + g.kChunk);
+    const int wm = (wave / WVN) * (32 * WM), wn = (wave % WVN) * (32 * WN);
+
+    // byte offsets of this thread's chunks (the operands are below 2 GB); rows past the edge are clamped and never stored
+    constexpr uint32_t OUTSIDE = 0x80000000u;
+    uint32_t va[PA], vb[PB];
+#pragma unroll
+    for (int p = 0; p < PA; p++) {
+        const int e = p * NT + tid;
+        if (AK) va[p] = (uint32_t)(min(m0 + e / 8, M - 1) * g.lda + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
+        else va[p] = (uint32_t)((e / (BM / 8)) * g.lda + min(m0 + ((e % (BM / 8)) ^ block_swizzle<BM * 2>(e / (BM / 8))) * 8, M - 8)) * 2;
+    }
+#pragma unroll
+    for (int p = 0; p < PB; p++) {
+        const int e = p * NT + tid;
+        if (BKC) vb[p] = (uint32_t)(min(n0 + e / 8, N - 1) * g.ldb + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
+        else vb[p] = (uint32_t)((e / (BN / 8)) * g.ldb + min(n0 + ((e % (BN / 8)) ^ block_swizzle<BN * 2>(e / (BN / 8))) * 8, N - 8)) * 2;
+    }
+    const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)g.A, 0, (int)(OUTSIDE - 16), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)g.B, 0, (int)(OUTSIDE - 16), 0x00020000);
+    // before the last stage is fetched, once: the chunks past the end of the contraction
+    auto lastStage = [&](int k0) {
+        asm volatile("" ::: "memory");   // a branch, not a select in every stage
+#pragma unroll
+        for (int p = 0; p < PA; p++) {
+            const int e = p * NT + tid;
+            if (k0 + (AK ? ((e & 7) ^ ((e >> 4) & 7)) * 8 : e / (BM / 8)) >= kEnd) va[p] = OUTSIDE;
+        }
+#pragma unroll
+        for (int p = 0; p < PB; p++) {
+            const int e = p * NT + tid;
+            if (k0 + (BKC ? ((e & 7) ^ ((e >> 4) & 7)) * 8 : e / (BN / 8)) >= kEnd) vb[p] = OUTSIDE;
+        }
+    };
+    // fetch p of a stage: this wavefront fills the 1 KB from chunk p NT + 64 wave on, lane i its i-th chunk
+    auto fetch = [&](int p, int k0, bf16_t* stage) {
+        if (p < PA) lds_fetch16(rsA, stage + (p * NT + wave * 64) * 8, va[p], (AK ? k0 : k0 * g.lda) * 2);
+        else lds_fetch16(rsB, stage + BM * BK + ((p - PA) * NT + wave * 64) * 8, vb[p - PA], (BKC ? k0 : k0 * g.ldb) * 2);
+    };
+
+    floatx16 acc[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+
+    // fragments: lane l holds row l % 32, k = 8 (l / 32) .. + 7 of a k-step of 16
+    const int fr = lane & 31, half = lane >> 5;
+    int koff[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) koff[ks] = ((2 * ks + half) ^ ((fr >> 1) & 7)) * 8;
+    // transposing reads: lane i of a group of sixteen addresses row k = 8 half + i / 4 (and + 4) of the k-step, columns
+    // 16 (group & 1) + 4 (i % 4) .. + 3; k % 4 is the same for both reads, so the exchange of the 32-row blocks is one
+    // constant per lane.  Byte offsets of this lane's first element of every block of rows:
+    const int tk = 8 * half + ((lane & 15) >> 2), tcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+    uint32_t ta[WM], tb[WN];
+#pragma unroll
+    for (int t = 0; t < WM; t++) ta[t] = (uint32_t)(tk * BM + ((wm + t * 32) ^ (block_swizzle<BM * 2>(tk) * 8)) + tcol) * 2;
+#pragma unroll
+    for (int t = 0; t < WN; t++) tb[t] = (uint32_t)(BM * BK + tk * BN + ((wn + t * 32) ^ (block_swizzle<BN * 2>(tk) * 8)) + tcol) * 2;
+    auto fragA = [&](const bf16_t* pa, uint32_t stageAddr, int t, int ks, TrFragment& o) {
+        if (AK) o.w = *(const u32x4*)(pa + (wm + t * 32 + fr) * BK + koff[ks]);
+        else tr_read<BM * 2>(stageAddr + ta[t], ks, o);
+    };
+    auto fragB = [&](const bf16_t* pb, uint32_t stageAddr, int t, int ks, TrFragment& o) {
+        if (BKC) o.w = *(const u32x4*)(pb + (wn + t * 32 + fr) * BK + koff[ks]);
+        else tr_read<BN * 2>(stageAddr + tb[t], ks, o);
+    };
+
+    const int nk = (kEnd - kBegin + BK - 1) / BK;
+    if (nk == 1) lastStage(kBegin);
+#pragma unroll
+    for (int p = 0; p < PA + PB; p++) fetch(p, kBegin, smem);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the fetches have landed in LDS
+    __syncthreads();
+    const uint32_t smemAddr = (uint32_t)(uintptr_t)LDS3(smem);
+    TrFragment a[2][WM], b[2][WN];
+    for (int kt = 0; kt < nk; kt++) {
+        const bf16_t* pa = smem + (kt & 1) * STAGE;
+        const bf16_t* pb = pa + BM * BK;
+        bf16_t* next = smem + ((kt & 1) ^ 1) * STAGE;   // read during stage kt - 1; free since the barrier that ended it
+        const int k1 = kBegin + min(kt + 1, nk - 1) * BK;   // past the end the last stage is fetched again, never read
+        if (kt + 2 == nk) lastStage(k1);
+        const uint32_t stageAddr = smemAddr + (kt & 1) * STAGE * 2;
+#pragma unroll
+        for (int t = 0; t < WM; t++) fragA(pa, stageAddr, t, 0, a[0][t]);
+#pragma unroll
+        for (int t = 0; t < WN; t++) fragB(pb, stageAddr, t, 0, b[0][t]);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int cur = ks & 1, nxt = cur ^ 1;
+            // what the transposing reads of this k-step's fragments brought, by now long issued
+#pragma unroll
+            for (int t = 0; t < WM; t++)
+                if (!AK) tr_wait(a[cur][t]);
+#pragma unroll
+            for (int t = 0; t < WN; t++)
+                if (!BKC) tr_wait(b[cur][t]);
+            // in issue order: a product, the fragments of the next k-step spread over the products, and from the first
+            // product on one fetch of the next stage each
+            constexpr int RF = (WM + WN + NMF - 1) / NMF * (AK && BKC ? 1 : 2);
+            constexpr int FE = (PA + PB + (KS - 1) * NMF - 1) / ((KS - 1) * NMF);   // fetches per product
+#pragma unroll
+            for (int q = 0; q < NMF; q++) {
+                const int i = q / WN, j = q % WN;
+                acc[i][j] = BigTraits<bf16_t>::mma(b[cur][j].w, a[cur][i].w, acc[i][j]);
+                if (ks + 1 < KS) {
+#pragma unroll
+                    for (int r = q * RF; r < (q + 1) * RF; r++) {
+                        if (r < WM) fragA(pa, stageAddr, r, ks + 1, a[nxt][r]);
+                        else if (r < WM + WN) fragB(pb, stageAddr, r - WM, ks + 1, b[nxt][r - WM]);
+                    }
+                }
+#pragma unroll
+                for (int f = (ks * NMF + q) * FE; f < (ks * NMF + q + 1) * FE; f++)
+                    if (f < PA + PB) fetch(f, k1, next);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+    }
+
+    // The products are the transposed tiles: a lane owns row lane % 32, register v is column 8 (v / 4) + 4 (lane / 32) + v % 4.
+    // Each wavefront passes 32 rows by CH tiles of columns at a time through its own slice of LDS (free after the last
+    // barrier; operations of one wavefront complete in order) and the lanes walk the rows eight columns each.
+    constexpr int CH = WN % 2 == 0 ? 2 : WN, CW = 32 * CH, LDC = CW + 4, LPR = CW / 8, RPI = 64 / LPR, NIT = (32 + RPI - 1) / RPI;
+    float* cs = reinterpret_cast<float*>(smem_raw) + wave * 32 * LDC;
+    const int rr = lane / LPR, cc = (lane % LPR) * 8, fg = half * 4;
+#pragma unroll
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+        for (int c0 = 0; c0 < WN; c0 += CH) {
+#pragma unroll
+            for (int j = 0; j < CH; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    *(float4*)(cs + fr * LDC + j * 32 + 8 * q + fg) = make_float4(g.alpha * acc[i][c0 + j][4 * q], g.alpha * acc[i][c0 + j][4 * q + 1],
+                                                                                 g.alpha * acc[i][c0 + j][4 * q + 2], g.alpha * acc[i][c0 + j][4 * q + 3]);
+            // a lane keeps its columns while it walks the rows
+            const int c = n0 + wn + c0 * 32 + cc;
+            float bias[8];
+            bf16_t* col = nullptr;
+            if (!split && c < N) {
+                b16_bias8(g, c, bias);
+                if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
+            }
+#pragma unroll 2
+            for (int it = 0; it < NIT; it++) {
+                const int row = it * RPI + rr, r = m0 + wm + i * 32 + row;
+                if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
+                const float4 t0 = *(const float4*)(cs + row * LDC + cc), t1 = *(const float4*)(cs + row * LDC + cc + 4);
+                float v[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
+                if (split) {
+                    float* cp = g.part + ((size_t)part * M + r) * N + c;
+                    if (g.vecC) {
+                        *(float4*)cp = t0;
+                        *(float4*)(cp + 4) = t1;
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 8; q++)
+                            if (c + q < N) cp[q] = v[q];
+                    }
+                } else {
+                    b16_store8<HEADS>(g, hp, r, c, bias, col, v);
+                }
+            }
+        }
+}
+
+// sum over the S partial products in their order, then as b16_store8
+template <bool HEADS>
+__global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<HEADS> hp, int S)
+{
+    const int oct = (g.N + 7) / 8;
+    const size_t mn = (size_t)g.M * g.N;
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < (size_t)g.M * oct; e += (size_t)256 * gridDim.x) {
+        const int r = (int)(e / oct), c = (int)(e % oct) * 8;
+        const float* p = g.part + (size_t)r * g.N + c;
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int z = 0; z < S; z++) {
+            if (g.vecC) {
+                const float4 a = *(const float4*)(p + z * mn), b = *(const float4*)(p + z * mn + 4);
+                v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w; v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 8; q++)
+                    if (c + q < g.N) v[q] += p[z * mn + q];
+            }
+        }
+        float bias[8];
+        b16_bias8(g, c, bias);
+        bf16_t* col = nullptr;
+        if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
+        b16_store8<HEADS>(g, hp, r, c, bias, col, v);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// How a product is cut: the tile and the number of parts of the contraction with the smallest estimated time.
+struct GemmB16Plan { int shape, splits, kChunk; };
+// microseconds of one tile per 768 k and for its ends (first fetches, and stores that all CUs issue at once), with two and
+// more workgroups on the CU and alone on it; fitted to 8000 x 3072 x 768, 8000 x 768 x 3072, 768 x 3072 x 8000,
+// 8192 x 512 x 512 and 8192 x 12288 x 4096
+struct GemmB16Shape { int bm, bn; double perK, ends, perKAlone, endsAlone; };
+static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 17.0, 5.0}, {256, 192, 10.0, 10.5, 10.0, 10.5}, {128, 192, 6.8, 4.4, 9.5, 6.0},
+                                           {128, 128, 4.2, 3.5, 6.0, 4.5}, {64, 128, 3.7, 1.0, 6.0, 1.5}, {64, 64, 2.5, 0.5, 4.1, 0.7}};
+
+static GemmB16Plan gemm_b16_plan(int m, int n, int k)
+{
+    GemmB16Plan best = {5, 1, k};
+    double bestT = 1e30;
+    for (int sh = 0; sh < 6; sh++) {
+        const GemmB16Shape& s = g_b16Shapes[sh];
+        const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn);
+        for (int S = 1; S <= 16; S++) {
+            if (S > 1 && k / S < 256) break;
+            const int chunk = ((k + S - 1) / S + 63) / 64 * 64;
+            if ((k + chunk - 1) / chunk != S) continue;
+            const double len = ((chunk + 63) / 64 * 64) / 768.0;
+            const long long perCu = ((tiles * S + 7) / 8 + 31) / 32;
+            double t = perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends);
+            if (S > 1) t += 4.0 + (double)(S + 1) * m * n * 4.0 / 4.0e6;
+            if (t < bestT) { bestT = t; best = {sh, S, S > 1 ? chunk : k}; }
+        }
+    }
+    return best;
+}
+
+bool gemm_b16_takes(const GemmB16& q)
+{
+    if (q.k < 8 || q.m < 1 || q.n < 1) return false;
+    if ((((uintptr_t)q.A | (uintptr_t)q.B) & 15) != 0) return false;
+    if (q.aK ? q.k % 8 != 0 : (q.m % 8 != 0 || q.m < 8)) return false;
+    if (q.bK ? q.k % 8 != 0 : (q.n % 8 != 0 || q.n < 8)) return false;
+    // 31-bit byte offsets
+    return ((long long)(q.aK ? q.m : q.k) + 64) * (q.aK ? q.k : q.m) < (1ll << 30) && ((long long)(q.bK ? q.n : q.k) + 64) * (q.bK ? q.k : q.n) < (1ll << 30);
+}
+size_t gemm_b16_workspace_bytes(int m, int n, int k)
+{
+    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    const GemmB16Plan p = gemm_b16_plan(m, n, k);
+    return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
+}
+
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS>
+static hipError_t launch_b16(hipStream_t s, const GemmB16Args& a, const HeadsEpilogue* he)
+{
+    constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN, CH = WN % 2 == 0 ? 2 : WN;
+    constexpr int stages = 2 * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    GemmB16Args g = a;
+    g.tilesM = (g.M + BM - 1) / BM;
+    g.tilesN = (g.N + BN - 1) / BN;
+    const long long total = (long long)g.tilesM * g.tilesN * g.parts;
+    if (total > (1ll << 27)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    return hipGetLastError();
+}
+template <bool AK, bool BKC, bool HEADS>
+static hipError_t launch_b16_shape(hipStream_t s, const GemmB16Args& a, int shape, const HeadsEpilogue* he = nullptr)
+{
+    switch (shape) {
+    case 0: return launch_b16<4, 2, 2, 4, 2, AK, BKC, HEADS>(s, a, he);
+    case 1: return launch_b16<4, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
+    case 2: return launch_b16<2, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
+    case 3: return launch_b16<2, 2, 2, 2, 2, AK, BKC, HEADS>(s, a, he);
+    case 4: return launch_b16<2, 2, 1, 2, 3, AK, BKC, HEADS>(s, a, he);
+    default: return launch_b16<2, 2, 1, 1, 4, AK, BKC, HEADS>(s, a, he);
+    }
+}
+
+hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
+{
+    if (!gemm_b16_takes(q) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || !q.aK || !q.bK))) return hipErrorInvalidValue;
+    GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
+    if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
+    GemmB16Args a = {};
+    a.M = q.m; a.N = q.n; a.K = q.k;
+    a.A = q.A; a.B = q.B; a.C = q.C;
+    a.lda = q.aK ? q.k : q.m; a.ldb = q.bK ? q.k : q.n;
+    a.alpha = q.alpha; a.beta = q.beta;
+    a.parts = p.splits; a.kChunk = p.kChunk;
+    a.part = (float*)ws;
+    a.bias = q.heads ? (const bf16_t*)q.heads->bias : q.bias;
+    if (q.heads) {
+        const HeadsEpilogue& he = *q.heads;
+        a.vecC = q.n % 8 == 0 && he.hs % 8 == 0 && (((uintptr_t)he.dst[0] | (uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0;
+    } else {
+        a.vecC = q.n % 8 == 0 && ((uintptr_t)q.C & 15) == 0;
+    }
+    hipError_t e;
+    if (q.heads) e = launch_b16_shape<true, true, true>(s, a, p.shape, q.heads);
+    else if (q.aK) e = q.bK ? launch_b16_shape<true, true, false>(s, a, p.shape) : launch_b16_shape<true, false, false>(s, a, p.shape);
+    else e = q.bK ? launch_b16_shape<false, true, false>(s, a, p.shape) : launch_b16_shape<false, false, false>(s, a, p.shape);
+    if (e != hipSuccess || p.splits == 1) return e;
+    const int grid = (int)std::min<size_t>(((size_t)q.m * ((q.n + 7) / 8) + 255) / 256, 4096);
+    if (q.heads) hipLaunchKernelGGL(gemm_b16_sum_kernel<true>, grid, 256, 0, s, a, heads_arg<true>(q.heads), p.splits);
+    else hipLaunchKernelGGL(gemm_b16_sum_kernel<false>, grid, 256, 0, s, a, HeadsArg<false>(), p.splits);
+    return hipGetLastError();
+}
+
+}  // namespace mch

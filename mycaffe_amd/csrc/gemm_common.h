@@ -1,4 +1,4 @@
-// Pieces shared by the GEMM kernels (gemm.hip, gemm_f32.hip): vector types, MFMA steps by operand type, and the epilogue
+// Pieces shared by the GEMM kernels (gemm.hip, gemm_f32.hip, gemm_bf16.hip): vector types, MFMA steps by operand type, and the epilogue
 // that adds a bias and writes head tensors.
 #pragma once
 #include <algorithm>
@@ -36,7 +36,6 @@ template <> struct BigTraits<bf16_t> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<bf16x8*>(&a), *reinterpret_cast<bf16x8*>(&b), c, 0, 0, 0);
     }
     __device__ static inline float ld(const bf16_t* p) { return bf16_to_f32(*p); }
-    __device__ static inline void st(bf16_t* p, float v) { *p = f32_to_bf16(v); }
     __device__ static inline void st4(bf16_t* p, float a, float b, float c, float d)
     {
         uint2 w;
@@ -55,9 +54,6 @@ template <> struct BigTraits<float> {
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
         return c;
     }
-    __device__ static inline float ld(const float* p) { return *p; }
-    __device__ static inline void st(float* p, float v) { *p = v; }
-    __device__ static inline void st4(float* p, float a, float b, float c, float d) { *(float4*)p = make_float4(a, b, c, d); }
 };
 
 // Epilogue of the fused QKV projection (HEADS): row r = (b, t) of the M = B*T rows, column c = (which, h, d) of the
@@ -67,15 +63,63 @@ template <> struct BigTraits<float> {
 // With fcos / fsin set (tables [seq][hs/2]) the q and k thirds are also rotated, after their rounding to the storage type:
 // adjacent pairs (2i, 2i+1) of row r by the angle of table row r % seq, column i - the rotary embedding that the layer
 // applies to q and k in (B,T,H,hs) layout before the head transposes (CausalSelfAttentionLayer.cs:538-545, rope.cu:785-825).
-struct HeadsEpilogue { const void* bias; void* dst[3]; int T, H, hs; const float* fcos; const float* fsin; int seq; };
-
-template <typename T>
-__device__ __forceinline__ T* heads_dst(const HeadsEpilogue& he, int row, int col)
+// Positions are found without divisions: with m = floor(2^32 / d), n m / 2^32 is at most one below n / d for every n < 2^32.
+// (Divided out per 16-byte piece they took 27 of the 74 us of 8000 x 3072 x 768 with its bias, 6 of the 14 us of 8192 x 512 x 512.)
+struct HeadsEpilogue {
+    const void* bias; void* dst[3]; int T, H, hs; const float* fcos; const float* fsin; int seq;
+    uint32_t mT, mC, mhs, mseq;   // floor(2^32 / T), / (H hs), / hs, / seq
+};
+static inline HeadsEpilogue heads_epilogue(const void* bias, void* q, void* k, void* v, int T, int H, int hs, const float* fcos, const float* fsin, int seq)
 {
-    const int Cd = he.H * he.hs;
-    const int which = col / Cd, w = col - which * Cd, h = w / he.hs, d = w - h * he.hs;
-    const int b = row / he.T, t = row - b * he.T;
-    return (T*)he.dst[which] + (((size_t)b * he.H + h) * he.T + t) * he.hs + d;
+    auto magic = [](int d) { const unsigned long long m = (1ull << 32) / (unsigned long long)d; return (uint32_t)(m > 0xffffffffull ? 0xffffffffull : m); };
+    HeadsEpilogue he;
+    he.bias = bias; he.dst[0] = q; he.dst[1] = k; he.dst[2] = v; he.T = T; he.H = H; he.hs = hs;
+    he.fcos = fcos; he.fsin = fsin; he.seq = seq;
+    he.mT = magic(T); he.mC = magic(H * hs); he.mhs = magic(hs); he.mseq = magic(seq);
+    return he;
+}
+// as a kernel argument: nothing where the kernel has no such epilogue (a launch with more than 200 bytes of arguments takes
+// the host a microsecond longer)
+template <bool HEADS> struct HeadsArg { HeadsEpilogue he; };
+template <> struct HeadsArg<false> {};
+template <bool HEADS> static inline HeadsArg<HEADS> heads_arg(const HeadsEpilogue* he)
+{
+    HeadsArg<HEADS> a;
+    if constexpr (HEADS) a.he = *he;
+    return a;
+}
+__device__ __forceinline__ int heads_div(int n, int d, uint32_t m, int& rem)
+{
+    int q = (int)__umulhi((uint32_t)n, m);
+    rem = n - q * d;
+    if (rem >= d) { rem -= d; q++; }
+    return q;
+}
+
+// address of column `col` in row 0, and what row `row` adds to it
+template <typename T>
+__device__ __forceinline__ T* heads_col(const HeadsEpilogue& he, int col)
+{
+    int w, d;
+    const int which = heads_div(col, he.H * he.hs, he.mC, w), h = heads_div(w, he.hs, he.mhs, d);
+    return (T*)(which == 0 ? he.dst[0] : which == 1 ? he.dst[1] : he.dst[2]) + (size_t)h * he.T * he.hs + d;
+}
+__device__ __forceinline__ size_t heads_row(const HeadsEpilogue& he, int row)
+{
+    int t;
+    const int b = heads_div(row, he.T, he.mT, t);
+    return ((size_t)b * he.H * he.T + t) * he.hs;
+}
+template <typename T>
+__device__ __forceinline__ T* heads_dst(const HeadsEpilogue& he, int row, int col) { return heads_col<T>(he, col) + heads_row(he, row); }
+
+// index into the rotation's tables for row `row`, column `col`
+__device__ __forceinline__ size_t heads_rope_at(const HeadsEpilogue& he, int row, int col)
+{
+    int p, d;
+    heads_div(row, he.seq, he.mseq, p);
+    heads_div(col, he.hs, he.mhs, d);
+    return (size_t)p * (he.hs >> 1) + (d >> 1);
 }
 
 // (re, im) of one pair of q or k, rotated; the expressions of rope_kernel (ew_kernels.hip)
@@ -91,7 +135,7 @@ __device__ __forceinline__ u32x4 heads_rope_piece(const HeadsEpilogue& he, int r
 {
     if (!he.fcos || col >= 2 * he.H * he.hs) return v;
     constexpr int NP = 8 / (int)sizeof(T);
-    const size_t ti = (size_t)(row % he.seq) * (he.hs >> 1) + ((col % he.hs) >> 1);
+    const size_t ti = heads_rope_at(he, row, col);
     uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < NP; i++) {
@@ -138,10 +182,25 @@ struct GemmF32 {
     int causal;
     const int* flag;
     int epoch;
-    const HeadsEpilogue* heads;            // written through this epilogue instead of to C (alpha 1, beta 0, batch 1)
+    const float* bias;                     // null, or n values added to every row of C (batch 1)
+    const HeadsEpilogue* heads;            // written through this epilogue instead of to C (alpha 1, beta 0, batch 1, bias null)
 };
 enum { CAUSAL_NO = 0, CAUSAL_A_LOWER /* A(i,k) zero for k > i */, CAUSAL_A_UPPER /* k < i */, CAUSAL_B_LOWER /* B(k,j) zero for k < j */, CAUSAL_B_UPPER /* k > j */ };
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal);
 hipError_t gemm_f32(hipStream_t s, const GemmF32& g, void* ws, size_t wsBytes);
+
+// The same in 16-bit storage, dense row-major operands (gemm_bf16.hip): op(A) stored (m, k) or (k, m), op(B) (n, k) or (k, n)
+struct GemmB16 {
+    int m, n, k;
+    const bf16_t *A, *B;
+    bf16_t* C;
+    bool aK, bK;
+    float alpha, beta;
+    const bf16_t* bias;   // as in GemmF32
+    const HeadsEpilogue* heads;
+};
+bool gemm_b16_takes(const GemmB16& g);   // 16-byte chunks of both operands aligned and whole
+size_t gemm_b16_workspace_bytes(int m, int n, int k);
+hipError_t gemm_b16(hipStream_t s, const GemmB16& g, void* ws, size_t wsBytes);
 
 }  // namespace mch

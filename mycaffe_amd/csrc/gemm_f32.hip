@@ -32,21 +32,25 @@ struct GemmF32Args {
     const int* flag;
     float* part;              // kChunk < K: partial products, [split][M][N]
     bool vecC;                // C rows can be read and written in 16-byte pieces
-    HeadsEpilogue he;
+    const float* bias;
 };
 
-// store of four consecutive values of row r from column c on, through the heads epilogue (c a multiple of 4)
-__device__ __forceinline__ void heads_store4(const HeadsEpilogue& he, int r, int c, int N, bool vec, float (&v)[4])
+// the bias of four columns from c on (0 past the matrix)
+__device__ __forceinline__ float4 f32_bias4(const float* bias, int c, int N)
 {
-    if (he.bias) {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (c + q < N) v[q] += ((const float*)he.bias)[c + q];
-    }
+    if (!bias) return make_float4(0.f, 0.f, 0.f, 0.f);
+    const float* b = bias + c;
+    return make_float4(b[0], c + 1 < N ? b[1] : 0.f, c + 2 < N ? b[2] : 0.f, c + 3 < N ? b[3] : 0.f);
+}
+
+// four consecutive values of row r from column c on (a multiple of 4), bias added, through the heads epilogue; column c of
+// row 0 is at col
+__device__ __forceinline__ void heads_store4(const HeadsEpilogue& he, int r, int c, int N, bool vec, float* col, float (&v)[4])
+{
     if (vec) {
         u32x4 p;
         p.x = __float_as_uint(v[0]); p.y = __float_as_uint(v[1]); p.z = __float_as_uint(v[2]); p.w = __float_as_uint(v[3]);
-        *(u32x4*)heads_dst<float>(he, r, c) = heads_rope_piece<float>(he, r, c, p);
+        *(u32x4*)(col + heads_row(he, r)) = heads_rope_piece<float>(he, r, c, p);
         return;
     }
 #pragma unroll
@@ -54,7 +58,7 @@ __device__ __forceinline__ void heads_store4(const HeadsEpilogue& he, int r, int
         // a rotation needs an even head size: a pair of columns is inside the matrix and one head, or outside
         if (c + q >= N) continue;
         if (he.fcos && c + q < 2 * he.H * he.hs) {
-            const size_t ti = (size_t)(r % he.seq) * (he.hs >> 1) + (((c + q) % he.hs) >> 1);
+            const size_t ti = heads_rope_at(he, r, c + q);
             heads_rope_pair(he.fcos[ti], he.fsin[ti], v[q], v[q + 1]);
         }
         *heads_dst<float>(he, r, c + q) = v[q];
@@ -64,7 +68,7 @@ __device__ __forceinline__ void heads_store4(const HeadsEpilogue& he, int r, int
 
 // VEC: every 16-byte chunk of an operand is aligned and lies inside it or outside as a whole
 template <int WM, int WN, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
-__global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g)
+__global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
 {
     constexpr int BK = 32, BM = 64 * WM, BN = 64 * WN, LDK = BK + 4;
     constexpr int LDA = AK ? LDK : BM, LDB = BKC ? LDK : BN;
@@ -276,6 +280,13 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g)
     const long long ldc = split ? N : g.ldc;
     const float beta = split ? 0.f : g.beta;
     const bool vec = split ? (N & 3) == 0 : g.vecC;
+    const int c = n0 + wn + cc;   // a lane keeps its columns while it walks the rows
+    float4 bias = make_float4(0.f, 0.f, 0.f, 0.f);
+    float* col = nullptr;
+    if (!split && c < N) {
+        bias = f32_bias4(g.bias, c, N);
+        if constexpr (HEADS) col = heads_col<float>(hp.he, c);
+    }
 #pragma unroll
     for (int i = 0; i < WM; i++) {
 #pragma unroll
@@ -286,13 +297,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g)
                     make_float4(g.alpha * acc[i][j][4 * q], g.alpha * acc[i][j][4 * q + 1], g.alpha * acc[i][j][4 * q + 2], g.alpha * acc[i][j][4 * q + 3]);
 #pragma unroll 4
         for (int it = 0; it < NIT; it++) {
-            const int row = it * RPI + rr, r = m0 + wm + i * 32 + row, c = n0 + wn + cc;
+            const int row = it * RPI + rr, r = m0 + wm + i * 32 + row;
             if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
             const float4 t = *(const float4*)(cs + row * LDC + cc);
-            float v[4] = {t.x, t.y, t.z, t.w};
-            if (HEADS && !split) {
-                heads_store4(g.he, r, c, N, vec, v);
-                continue;
+            float v[4] = {t.x + bias.x, t.y + bias.y, t.z + bias.z, t.w + bias.w};
+            if constexpr (HEADS) {
+                if (!split) {
+                    heads_store4(hp.he, r, c, N, vec, col, v);
+                    continue;
+                }
             }
             float* cp = C + (size_t)r * ldc + c;
             if (vec) {
@@ -313,7 +326,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g)
 // C = sum over the S partial products, in their order (alpha is in them already), + beta C; or through the heads epilogue
 template <bool HEADS>
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int S, int M, int N, long long ldc, float beta, bool vecC,
-                                                           float* __restrict__ C, HeadsEpilogue he)
+                                                           float* __restrict__ C, const float* __restrict__ bias, HeadsArg<HEADS> hp)
 {
     const int quads = (N + 3) / 4;
     const size_t mn = (size_t)M * N;
@@ -332,8 +345,10 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restri
                 for (int q = 0; q < 4; q++)
                     if (c + q < N) v[q] += p[z * mn + q];
         }
-        if (HEADS) {
-            heads_store4(he, r, c, N, vecC, v);
+        const float4 b = f32_bias4(bias, c, N);
+        v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
+        if constexpr (HEADS) {
+            heads_store4(hp.he, r, c, N, vecC, heads_col<float>(hp.he, c), v);
             continue;
         }
         float* cp = C + (size_t)r * ldc + c;
@@ -390,7 +405,7 @@ size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal)
 }
 
 template <int WM, int WN, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
-static hipError_t launch_f32(hipStream_t s, const GemmF32Args& a, int splits, int batch)
+static hipError_t launch_f32(hipStream_t s, const GemmF32Args& a, int splits, int batch, const HeadsEpilogue* he)
 {
     constexpr int BM = 64 * WM, BN = 64 * WN;
     constexpr int SA = AK ? BM * 36 : 32 * BM, SB = BKC ? BN * 36 : 32 * BN;
@@ -404,17 +419,17 @@ static hipError_t launch_f32(hipStream_t s, const GemmF32Args& a, int splits, in
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
     const int per = (int)((total + 7) / 8);
-    hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, OCC, AK, BKC, VEC, HEADS>), dim3(per * 8), 256, lds, s, g);
+    hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, OCC, AK, BKC, VEC, HEADS>), dim3(per * 8), 256, lds, s, g, heads_arg<HEADS>(he));
     return hipGetLastError();
 }
 
 template <bool AK, bool BKC, bool VEC, bool HEADS>
-static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const GemmF32Plan& p, int batch)
+static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
 {
-    if (p.wn == 3) return launch_f32<2, 3, 1, AK, BKC, VEC, HEADS>(s, a, p.splits, batch);
-    if (p.wm == 2) return launch_f32<2, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch);
-    if (p.wn == 2) return launch_f32<1, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch);
-    return launch_f32<1, 1, 3, AK, BKC, VEC, HEADS>(s, a, p.splits, batch);
+    if (p.wn == 3) return launch_f32<2, 3, 1, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+    if (p.wm == 2) return launch_f32<2, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+    if (p.wn == 2) return launch_f32<1, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+    return launch_f32<1, 1, 3, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
 }
 
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
@@ -432,9 +447,10 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     a.kChunk = p.kChunk;
     a.causal = q.causal; a.flag = q.flag; a.epoch = q.epoch;
     a.part = (float*)ws;
+    a.bias = q.heads ? (const float*)q.heads->bias : q.bias;
     if (q.heads) {
-        a.he = *q.heads;
-        a.vecC = q.n % 4 == 0 && a.he.hs % 4 == 0 && (((uintptr_t)a.he.dst[0] | (uintptr_t)a.he.dst[1] | (uintptr_t)a.he.dst[2]) & 15) == 0;
+        const HeadsEpilogue& he = *q.heads;
+        a.vecC = q.n % 4 == 0 && he.hs % 4 == 0 && (((uintptr_t)he.dst[0] | (uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0;
     } else {
         a.vecC = q.n % 4 == 0 && q.ldc % 4 == 0 && (q.batch == 1 || q.sC % 4 == 0) && ((uintptr_t)q.C & 15) == 0;
     }
@@ -442,7 +458,7 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
                      (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0) &&
                      ((q.aK ? q.m : q.k) + 64) * q.lda < (1ll << 29) && ((q.bK ? q.n : q.k) + 64) * q.ldb < (1ll << 29);   // 31-bit byte offsets
     hipError_t e;
-    if (q.heads) e = vec ? launch_f32_tile<true, true, true, true>(s, a, p, 1) : launch_f32_tile<true, true, false, true>(s, a, p, 1);
+    if (q.heads) e = vec ? launch_f32_tile<true, true, true, true>(s, a, p, 1, q.heads) : launch_f32_tile<true, true, false, true>(s, a, p, 1, q.heads);
 #define LAYOUT(AKV, BKV) (vec ? launch_f32_tile<AKV, BKV, true, false>(s, a, p, q.batch) : launch_f32_tile<AKV, BKV, false, false>(s, a, p, q.batch))
     else if (q.aK) e = q.bK ? LAYOUT(true, true) : LAYOUT(true, false);
     else e = q.bK ? LAYOUT(false, true) : LAYOUT(false, false);
@@ -450,8 +466,8 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     if (e != hipSuccess || p.splits == 1) return e;
     const size_t quads = (size_t)q.m * ((q.n + 3) / 4);
     const int grid = (int)std::min<size_t>((quads + 255) / 256, 4096);
-    if (q.heads) hipLaunchKernelGGL(gemm_f32_sum_kernel<true>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.he);
-    else hipLaunchKernelGGL(gemm_f32_sum_kernel<false>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.he);
+    if (q.heads) hipLaunchKernelGGL(gemm_f32_sum_kernel<true>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, heads_arg<true>(q.heads));
+    else hipLaunchKernelGGL(gemm_f32_sum_kernel<false>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, HeadsArg<false>());
     return hipGetLastError();
 }
 

@@ -103,8 +103,7 @@ hipError_t k_channel_dot(hipStream_t s, DType dt, size_t num, int channels, int 
 
 // ---- GEMM family (gemm.hip) ------------------------------------------------
 // row-major C[m,n] = alpha*op(A)*op(B) + beta*C; A, B, C all of storage type dt
-// ws: k_gemm_workspace_bytes(...) bytes of scratch for contractions cut into parts and, in 16-bit storage, for operands that
-// are turned first (without it neither is done)
+// ws: k_gemm_workspace_bytes(...) bytes of scratch for contractions cut into parts (without it they are not)
 hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k, float alpha, const void* A,
                   const void* B, float beta, void* C, void* ws = nullptr, size_t wsBytes = 0);
 size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k);
@@ -116,8 +115,8 @@ hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs
 // Y (m x n) = X (m x k) W^T + bias in one call; ws: k_gemm_bias_workspace_bytes(...) of scratch
 hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes);
 // scratch of k_gemm_bias / k_gemm_qkv_heads with these operands (0: none)
-size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W, const void* Y);
-size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* q, const void* k, const void* v);
+size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W);
+size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W);
 // column-major strided batched gemm with BLAS semantics (fp32)
 // C (fp32) = alpha X W^T + beta C on the bf16 matrix cores: W 16-bit (n x k), k % 64 == 0; A is X as bf16 (m x k) or,
 // split, every row of X as two bf16 rows (nearest bf16, then the bf16 nearest to the remainder; m x 2k)

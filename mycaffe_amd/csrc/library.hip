@@ -802,7 +802,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 if (!m_mem.get(p.hA, &X) && !m_mem.get(p.hB, &W) && !m_mem.get(p.hC, &C) && C->half == A->half) {
                     m_pendingProduct = PendingProduct();
                     void* ws = nullptr;
-                    const size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, C->ptr);
+                    const size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr);
                     if (wsb) ERRCHK(workspace(wsb, &ws));
                     HIPCHK(k_gemm_bias(s, C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws, wsb));
                     m_mem.touch(hC);
@@ -2043,7 +2043,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             }
         }
         void* ws = nullptr;
-        const size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Q->ptr, K->ptr, V->ptr);
+        const size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr);
         if (wsb) ERRCHK(workspace(wsb, &ws));
         HIPCHK(k_gemm_qkv_heads(s, X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Q->ptr, K->ptr,
                                 V->ptr, ws, wsb, r ? (const float*)r->dcos.get() : nullptr, r ? (const float*)r->dsin.get() : nullptr,
@@ -2070,7 +2070,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
         void* ws = nullptr;
-        const size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Y->ptr);
+        const size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr);
         if (wsb) ERRCHK(workspace(wsb, &ws));
         HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
         m_mem.touch((long)pl[6]);
