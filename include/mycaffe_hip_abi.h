@@ -187,14 +187,42 @@ enum {
      *
      * LINEAR_FWD replaces the two GEMM calls of InnerProductLayer.forward (InnerProductLayer.cs:372-417: the product
      * with the transposed weight, then the rank-1 update with the vector of ones) by one GEMM whose epilogue adds
-     * the bias:  l{M, N, K, hX (M x K), hWeight (N x K), hBias (N; 0 = none), hY (M x N)}.
+     * the bias:  l{M, N, K, hX (M x K), hWeight (N x K), hBias (N; 0 = none), hY (M x N) [, T, heads]}.
+     * With T and heads, Y is written head by head as (M/T, heads, T, N/heads): the projections of a multi-head attention layer
+     * without the transposes behind them (MultiheadAttentionLayer.cs:650-690).
      * With it the causal self attention layer's forward is three calls.
+     *
+     * LINEAR_BWD replaces the GEMM, GEMV and GEMM calls of InnerProductLayer.backward (InnerProductLayer.cs:429-494):
+     * dW += dY^T X, db += column sums of dY, dX = dY W (accumX: dX += dY W):
+     *   l{M, N, K, hX (M x K), hWeight (N x K), hdY (M x N), hdWeight, hdBias (0 = none), hdX (0 = none) [, accumX]}
+     *
+     * QKV_HEADS_GRAD is what lies between the attention's gradient and the projection's in
+     * CausalSelfAttentionLayer.backward (CausalSelfAttentionLayer.cs:700-740: three transposes, two ROPE_BWD calls, three
+     * channel copies): dX (batch*T, 3C) from dQ, dK, dV (batch, heads, T, hs):
+     *   l{batch, T, heads, hs, hdQ, hdK, hdV, hdX [, hRope]}
+     *
+     * RMSNORM_BWD replaces the chain of RMSNormLayer.backward (RMSNormLayer.cs:189-232); the weight gradient is overwritten
+     * with the sums of the first dwRows rows, which is what that chain's channel_sum leaves:
+     *   f{eps}  l{rows, dim, hX, hWeight (0 = none), hdY, hdX, hdWeight (0 = none), dwRows [, hAdd]}: dX (+ hAdd's values)
+     *
+     * SWIGLU_BWD: y = silu(a) b backward (TransformerBlockLayer.cs:924-1040):  l{n, hA, hB, hdY, hdA, hdB}
+     *
+     * NORM_ADD_FWD / NORM_ADD_BWD: a residual and the norm next to it in one pass.  Forward: total = x + add is stored, then
+     * normalised into y; hLayerNorm != 0 runs that handle, 0 the RMS norm of RMSNORM_FWD over rows of dim values:
+     *   f{eps}  l{hLayerNorm, rows, dim, hX, hAdd, hTotal, hWeight (0 = none), hY}
+     * Backward (layer norm handle): dX = the gradient of LAYERNORM_BWD plus hAdd's values:  l{hLayerNorm, hY, hdY, hdX, hAdd}
      */
     MCH_FN_ATTN_DECODE_FWD = 2001,
     MCH_FN_RMSNORM_FWD = 2002,
     MCH_FN_SWIGLU_FWD = 2003,
     MCH_FN_QKV_PROJ_HEADS = 2004,
-    MCH_FN_LINEAR_FWD = 2005
+    MCH_FN_LINEAR_FWD = 2005,
+    MCH_FN_LINEAR_BWD = 2006,
+    MCH_FN_QKV_HEADS_GRAD = 2007,
+    MCH_FN_RMSNORM_BWD = 2008,
+    MCH_FN_SWIGLU_BWD = 2009,
+    MCH_FN_NORM_ADD_FWD = 2010,
+    MCH_FN_NORM_ADD_BWD = 2011
 };
 
 /* DEVINIT flags (CudaDnnDLL/Cuda Files/device.h:18-22) */
@@ -226,10 +254,9 @@ MCH_LONG DLL_InvokeFloatEx(MCH_LONG lKernelIdx, MCH_LONG lFunctionIdx, float* pI
  * SUM2 / FILLFROM / COPYALL / DUP, EMBED_FWD, SILU / GELU / RELU forward and backward, SWIGLU_FWD, RMSNORM_FWD, CREATE /
  * FREE_LAYERNORM and LAYERNORM_FWD / BWD, CREATE / FREE_CUDNN, CREATE / FREE / SET_TENSORDESC, SOFTMAX_FWD / BWD,
  * ATTN_CREATE / FREE / SET / FWD / BWD (no dropout; the tenth and eleventh values of ATTN_FWD as on the float side),
- * CREATE_ROPE / FREE_ROPE / ROPE_FWD / BWD, and the fused ids ATTN_DECODE_FWD, QKV_PROJ_HEADS (even head sizes) and
- * LINEAR_FWD - same packing as the float ids above: what the attention, multi-head attention and transformer block layers
- * call, forward and backward.  These are one-element-per-thread kernels: the precision twin of the path, not a fast
- * one.  Any other id (blob loaders, extensions), and DLL_InvokeDoubleEx (extensions and blob loaders are float objects),
+ * CREATE_ROPE / FREE_ROPE / ROPE_FWD / BWD, and the fused ids ATTN_DECODE_FWD, QKV_PROJ_HEADS, QKV_HEADS_GRAD,
+ * LINEAR_FWD / BWD, RMSNORM_BWD, SWIGLU_BWD and NORM_ADD_FWD / BWD - same packing as the float ids above: what the attention, multi-head attention and transformer block layers
+ * call, forward and backward.  Products run on the double matrix cores, the rest in one-element-per-thread kernels.  Any other id (blob loaders, extensions), and DLL_InvokeDoubleEx (extensions and blob loaders are float objects),
  * returns MCH_ERROR_NOT_IMPLEMENTED with the id in the message. */
 MCH_LONG DLL_InvokeDouble(MCH_LONG lKernelIdx, MCH_LONG lFunctionIdx, double* pInput, MCH_LONG lInput,
                           double** ppOutput, MCH_LONG* plOutput, MCH_TCHAR* szErr, MCH_LONG lszErrMax);

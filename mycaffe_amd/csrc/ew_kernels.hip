@@ -555,43 +555,22 @@ hipError_t k_rope(hipStream_t s, DType dt, size_t n, const void* x, void* y, con
     return hipGetLastError();
 }
 
-// y = w * (x / sqrt(mean(x^2) + eps)); one workgroup per row
-template <typename T> __global__ void rmsnorm_kernel(int dim, const T* x, const T* w, T* y, float eps)
-{
-    __shared__ float red[4];
-    const T* xr = x + (size_t)blockIdx.x * dim;
-    T* yr = y + (size_t)blockIdx.x * dim;
-    float ss = 0.f;
-    for (int i = threadIdx.x; i < dim; i += TPB) {
-        float v = ld(xr, i);
-        ss += v * v;
-    }
-    ss = block_sum<4>(ss, red);
-    float inv = 1.0f / sqrtf(ss / dim + eps);
-    for (int i = threadIdx.x; i < dim; i += TPB) {
-        float v = inv * ld(xr, i);
-        st(yr, i, w ? ld(w, i) * v : v);
-    }
-}
-
-hipError_t k_rmsnorm(hipStream_t s, DType dt, int outer, int dim, const void* x, const void* w, void* y, float eps)
-{
-    if (outer <= 0 || dim <= 0) return hipSuccess;
-    DISPATCH_DT(dt, hipLaunchKernelGGL(rmsnorm_kernel<T>, outer, TPB, 0, s, dim, (const T*)x, (const T*)w, (T*)y, eps));
-    return hipGetLastError();
-}
-
-
 // ---------------------------------------------------------------------------
 // LayerNorm (no affine part; the reference chain of layernorm.cu:219-262 in one pass): per row of `inner` values
 // y = (x - mean) / sqrt(var + eps); the row's sqrt(var + eps) is kept for the backward pass.  One workgroup per
 // row; the row stays in L2 between the three sweeps, so HBM sees one read and one write.
-template <typename T> __global__ void layernorm_fwd_kernel(int inner, const T* x, T* y, float* stdev, float eps)
+// With `add`, x + add is stored in `total` first and normalised (a block's residual and its norm in one pass).
+template <typename T> __global__ void layernorm_fwd_kernel(int inner, const T* x, const T* add, T* total, T* y, float* stdev, float eps)
 {
     __shared__ float red[4];
     const T* xr = x + (size_t)blockIdx.x * inner;
     T* yr = y + (size_t)blockIdx.x * inner;
     float sum = 0.f;
+    if (add) {   // a thread reads back only what it wrote
+        T* tr = total + (size_t)blockIdx.x * inner;
+        for (int i = threadIdx.x; i < inner; i += TPB) st(tr, i, ld(xr, i) + ld(add + (size_t)blockIdx.x * inner, i));
+        xr = tr;
+    }
     for (int i = threadIdx.x; i < inner; i += TPB) sum += ld(xr, i);
     const float mean = block_sum<4>(sum, red) / inner;
     float sq = 0.f;
@@ -624,7 +603,19 @@ template <> struct Vec4<bf16_t> {
     }
 };
 
-template <typename T, int R> __global__ __launch_bounds__(256) void layernorm_fwd_wave_kernel(int rows, int inner, const T* x, T* y, float* stdev, float eps)
+// four values of x become those of x + add as `total` stores them
+template <typename T> __device__ inline void add_chunk(const T* add, T* total, size_t at, float (&v)[4])
+{
+    float a[4];
+    Vec4<T>::load(add + at, a);
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] += a[j];
+    Vec4<T>::store(total + at, v);
+    if (sizeof(T) == 2) Vec4<T>::load(total + at, v);
+}
+
+template <typename T, int R, bool ADD>
+__global__ __launch_bounds__(256) void layernorm_fwd_wave_kernel(int rows, int inner, const T* x, const T* add, T* total, T* y, float* stdev, float eps)
 {
     const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -638,6 +629,7 @@ template <typename T, int R> __global__ __launch_bounds__(256) void layernorm_fw
         const int c = lane + 64 * r;
         if (c < chunks) {
             Vec4<T>::load(xr + 4 * c, v[r]);
+            if (ADD) add_chunk(add, total, (size_t)row * inner + 4 * c, v[r]);
             sum += (v[r][0] + v[r][1]) + (v[r][2] + v[r][3]);
         }
     }
@@ -666,7 +658,7 @@ template <typename T, int R> __global__ __launch_bounds__(256) void layernorm_fw
 }
 
 template <typename T, int R>
-__global__ __launch_bounds__(256) void layernorm_bwd_wave_kernel(int rows, int inner, const T* y, const T* dy, T* dx, const float* stdev, float bump)
+__global__ __launch_bounds__(256) void layernorm_bwd_wave_kernel(int rows, int inner, const T* y, const T* dy, const T* add, T* dx, const float* stdev, float bump)
 {
     const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -699,31 +691,39 @@ __global__ __launch_bounds__(256) void layernorm_bwd_wave_kernel(int rows, int i
                 const float div = base + 4 * c + j < (size_t)rows ? sd + bump : sd;
                 o[j] = (vg[r][j] - (vy[r][j] * m1 + m2)) / div;
             }
+            if (add) {
+                float e[4];
+                Vec4<T>::load(add + base + 4 * c, e);
+#pragma unroll
+                for (int j = 0; j < 4; j++) o[j] += e[j];
+            }
             Vec4<T>::store(dx + base + 4 * c, o);
         }
     }
 }
 
 // register budget per lane: R chunks of four values
-static inline int layernorm_wave_chunks(int inner, const void* a, const void* b, const void* c, size_t esize)
+static inline int layernorm_wave_chunks(int inner, const void* a, const void* b, const void* c, size_t esize, const void* d = nullptr, const void* e = nullptr)
 {
     if (inner % 4 != 0 || inner > 2048) return 0;
-    if ((((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & (4 * esize - 1)) != 0) return 0;
+    if ((((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d | (uintptr_t)e) & (4 * esize - 1)) != 0) return 0;
     const int r = (inner / 4 + 63) / 64;
     return r <= 1 ? 1 : (r <= 2 ? 2 : (r <= 4 ? 4 : 8));
 }
 
-hipError_t k_layernorm_fwd(hipStream_t s, DType dt, int rows, int inner, const void* x, void* y, float* stdev, float eps)
+hipError_t k_layernorm_fwd(hipStream_t s, DType dt, int rows, int inner, const void* x, void* y, float* stdev, float eps, const void* add, void* total)
 {
     if (rows <= 0 || inner <= 0) return hipSuccess;
-    const int R = layernorm_wave_chunks(inner, x, y, y, dt == F32 ? 4 : 2);
+    const int R = layernorm_wave_chunks(inner, x, y, add, dt == F32 ? 4 : 2, total);
     const int g = (rows + 3) / 4;
-#define LN_FWD(RR) DISPATCH_DT(dt, hipLaunchKernelGGL((layernorm_fwd_wave_kernel<T, RR>), g, 256, 0, s, rows, inner, (const T*)x, (T*)y, stdev, eps))
-    if (R == 1) LN_FWD(1);
-    else if (R == 2) LN_FWD(2);
-    else if (R == 4) LN_FWD(4);
-    else if (R == 8) LN_FWD(8);
-    else DISPATCH_DT(dt, hipLaunchKernelGGL(layernorm_fwd_kernel<T>, rows, TPB, 0, s, inner, (const T*)x, (T*)y, stdev, eps));
+#define LN_FWD(RR, A) DISPATCH_DT(dt, hipLaunchKernelGGL((layernorm_fwd_wave_kernel<T, RR, A>), g, 256, 0, s, rows, inner, (const T*)x, (const T*)add, (T*)total, (T*)y, stdev, eps))
+#define LN_FWD2(RR) do { if (add) LN_FWD(RR, true); else LN_FWD(RR, false); } while (0)
+    if (R == 1) LN_FWD2(1);
+    else if (R == 2) LN_FWD2(2);
+    else if (R == 4) LN_FWD2(4);
+    else if (R == 8) LN_FWD2(8);
+    else DISPATCH_DT(dt, hipLaunchKernelGGL(layernorm_fwd_kernel<T>, rows, TPB, 0, s, inner, (const T*)x, (const T*)add, (T*)total, (T*)y, stdev, eps));
+#undef LN_FWD2
 #undef LN_FWD
     return hipGetLastError();
 }
@@ -732,7 +732,7 @@ hipError_t k_layernorm_fwd(hipStream_t s, DType dt, int rows, int inner, const v
 // reference adds eps to the first `rows` entries of its row-expanded stdev array on every backward call, which is
 // reproduced through `bump` = eps x (backward calls since the last forward), applied to flat indices < rows.
 template <typename T>
-__global__ void layernorm_bwd_kernel(int rows, int inner, const T* y, const T* dy, T* dx, const float* stdev, float bump)
+__global__ void layernorm_bwd_kernel(int rows, int inner, const T* y, const T* dy, const T* add, T* dx, const float* stdev, float bump)
 {
     __shared__ float red[4];
     const size_t base = (size_t)blockIdx.x * inner;
@@ -748,24 +748,253 @@ __global__ void layernorm_bwd_kernel(int rows, int inner, const T* y, const T* d
     for (int i = threadIdx.x; i < inner; i += TPB) {
         float w = ld(y, base + i) * m1 + m2;
         float div = base + i < (size_t)rows ? sd + bump : sd;
-        st(dx, base + i, (ld(dy, base + i) - w) / div);
+        const float g = (ld(dy, base + i) - w) / div;
+        st(dx, base + i, add ? g + ld(add, base + i) : g);
     }
 }
 
 hipError_t k_layernorm_bwd(hipStream_t s, DType dt, int rows, int inner, const void* y, const void* dy, void* dx,
-                           const float* stdev, float bump)
+                           const float* stdev, float bump, const void* add)
 {
     if (rows <= 0 || inner <= 0) return hipSuccess;
-    const int R = layernorm_wave_chunks(inner, y, dy, dx, dt == F32 ? 4 : 2);
+    const int R = layernorm_wave_chunks(inner, y, dy, dx, dt == F32 ? 4 : 2, add);
     const int g = (rows + 3) / 4;
-#define LN_BWD(RR) DISPATCH_DT(dt, hipLaunchKernelGGL((layernorm_bwd_wave_kernel<T, RR>), g, 256, 0, s, rows, inner, (const T*)y, (const T*)dy, (T*)dx, stdev, bump))
+#define LN_BWD(RR) DISPATCH_DT(dt, hipLaunchKernelGGL((layernorm_bwd_wave_kernel<T, RR>), g, 256, 0, s, rows, inner, (const T*)y, (const T*)dy, (const T*)add, (T*)dx, stdev, bump))
     if (R == 1) LN_BWD(1);
     else if (R == 2) LN_BWD(2);
     else if (R == 4) LN_BWD(4);
     else if (R == 8) LN_BWD(8);
-    else DISPATCH_DT(dt, hipLaunchKernelGGL(layernorm_bwd_kernel<T>, rows, TPB, 0, s, rows, inner, (const T*)y, (const T*)dy, (T*)dx,
+    else DISPATCH_DT(dt, hipLaunchKernelGGL(layernorm_bwd_kernel<T>, rows, TPB, 0, s, rows, inner, (const T*)y, (const T*)dy, (const T*)add, (T*)dx,
                                             stdev, bump));
 #undef LN_BWD
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// RMSNorm: y = w * (x / sqrt(mean(x^2) + eps)), with `add` of total = x + add.  Rows that fit a wavefront's registers
+// (layernorm_wave_chunks) take one wavefront each, the others one workgroup and a second sweep of the row out of L2.
+template <typename T, int R, bool ADD>
+__global__ __launch_bounds__(256) void rmsnorm_wave_kernel(int rows, int dim, const T* x, const T* add, T* total, const T* w, T* y, float eps)
+{
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int chunks = dim >> 2;
+    const size_t base = (size_t)row * dim;
+    float v[R][4], ss = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int c = lane + 64 * r;
+        if (c < chunks) {
+            Vec4<T>::load(x + base + 4 * c, v[r]);
+            if (ADD) add_chunk(add, total, base + 4 * c, v[r]);
+            ss += (v[r][0] * v[r][0] + v[r][1] * v[r][1]) + (v[r][2] * v[r][2] + v[r][3] * v[r][3]);
+        }
+    }
+    const float inv = 1.0f / sqrtf(wave_sum(ss) / dim + eps);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int c = lane + 64 * r;
+        if (c < chunks) {
+            float o[4] = {1.f, 1.f, 1.f, 1.f};
+            if (w) Vec4<T>::load(w + 4 * c, o);
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] *= inv * v[r][j];
+            Vec4<T>::store(y + base + 4 * c, o);
+        }
+    }
+}
+template <typename T> __global__ void rmsnorm_kernel(int dim, const T* x, const T* add, T* total, const T* w, T* y, float eps)
+{
+    __shared__ float red[4];
+    const size_t base = (size_t)blockIdx.x * dim;
+    const T* xr = x + base;
+    float ss = 0.f;
+    if (add) {   // a thread reads back only what it wrote
+        for (int i = threadIdx.x; i < dim; i += TPB) st(total, base + i, ld(xr, i) + ld(add, base + i));
+        xr = total + base;
+    }
+    for (int i = threadIdx.x; i < dim; i += TPB) {
+        float v = ld(xr, i);
+        ss += v * v;
+    }
+    ss = block_sum<4>(ss, red);
+    float inv = 1.0f / sqrtf(ss / dim + eps);
+    for (int i = threadIdx.x; i < dim; i += TPB) {
+        float v = inv * ld(xr, i);
+        st(y, base + i, w ? ld(w, i) * v : v);
+    }
+}
+
+hipError_t k_rmsnorm(hipStream_t s, DType dt, int outer, int dim, const void* x, const void* w, void* y, float eps, const void* add, void* total)
+{
+    if (outer <= 0 || dim <= 0) return hipSuccess;
+    const int R = layernorm_wave_chunks(dim, x, y, w, dt == F32 ? 4 : 2, add, total);
+    const int g = (outer + 3) / 4;
+#define RMS_FWD(RR, A) DISPATCH_DT(dt, hipLaunchKernelGGL((rmsnorm_wave_kernel<T, RR, A>), g, 256, 0, s, outer, dim, (const T*)x, (const T*)add, (T*)total, (const T*)w, (T*)y, eps))
+#define RMS_FWD2(RR) do { if (add) RMS_FWD(RR, true); else RMS_FWD(RR, false); } while (0)
+    if (R == 1) RMS_FWD2(1);
+    else if (R == 2) RMS_FWD2(2);
+    else if (R == 4) RMS_FWD2(4);
+    else if (R == 8) RMS_FWD2(8);
+    else DISPATCH_DT(dt, hipLaunchKernelGGL(rmsnorm_kernel<T>, outer, TPB, 0, s, dim, (const T*)x, (const T*)add, (T*)total, (const T*)w, (T*)y, eps));
+#undef RMS_FWD2
+#undef RMS_FWD
+    return hipGetLastError();
+}
+
+// Its gradient with g = dy w, r = 1 / sqrt(mean(x^2) + eps):  dx = g r - x r^3 sum(g x) / dim (+ add), and r kept per row for
+// the weight gradient (x and dy are at hand when the layer runs backward, so nothing of the forward pass is needed).
+template <typename T, int R>
+__global__ __launch_bounds__(256) void rmsnorm_bwd_wave_kernel(int rows, int dim, const T* x, const T* w, const T* dy, const T* add, T* dx, float* rinv, float eps)
+{
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int chunks = dim >> 2;
+    const size_t base = (size_t)row * dim;
+    float vx[R][4], vg[R][4], ss = 0.f, sg = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int c = lane + 64 * r;
+        if (c < chunks) {
+            Vec4<T>::load(x + base + 4 * c, vx[r]);
+            Vec4<T>::load(dy + base + 4 * c, vg[r]);
+            float vw[4] = {1.f, 1.f, 1.f, 1.f};
+            if (w) Vec4<T>::load(w + 4 * c, vw);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                vg[r][j] *= vw[j];
+                ss += vx[r][j] * vx[r][j];
+                sg += vg[r][j] * vx[r][j];
+            }
+        }
+    }
+    const float inv = 1.0f / sqrtf(wave_sum(ss) / dim + eps);
+    const float f = wave_sum(sg) * inv * inv * inv / dim;
+    if (rinv && lane == 0) rinv[row] = inv;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int c = lane + 64 * r;
+        if (c < chunks) {
+            float o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = vg[r][j] * inv - vx[r][j] * f;
+            if (add) {
+                float e[4];
+                Vec4<T>::load(add + base + 4 * c, e);
+#pragma unroll
+                for (int j = 0; j < 4; j++) o[j] += e[j];
+            }
+            Vec4<T>::store(dx + base + 4 * c, o);
+        }
+    }
+}
+template <typename T>
+__global__ void rmsnorm_bwd_kernel(int dim, const T* x, const T* w, const T* dy, const T* add, T* dx, float* rinv, float eps)
+{
+    __shared__ float red[4];
+    const size_t base = (size_t)blockIdx.x * dim;
+    float ss = 0.f, sg = 0.f;
+    for (int i = threadIdx.x; i < dim; i += TPB) {
+        const float v = ld(x, base + i), g = ld(dy, base + i) * (w ? ld(w, i) : 1.f);
+        ss += v * v;
+        sg += g * v;
+    }
+    const float inv = 1.0f / sqrtf(block_sum<4>(ss, red) / dim + eps);
+    const float f = block_sum<4>(sg, red) * inv * inv * inv / dim;
+    if (rinv && threadIdx.x == 0) rinv[blockIdx.x] = inv;
+    for (int i = threadIdx.x; i < dim; i += TPB) {
+        const float o = ld(dy, base + i) * (w ? ld(w, i) : 1.f) * inv - ld(x, base + i) * f;
+        st(dx, base + i, add ? o + ld(add, base + i) : o);
+    }
+}
+// dw[j] = sum over the rows of dy x r: 16 columns by 64 rows a trip, the sums of the 64 row lanes added in order
+template <typename T>
+__global__ __launch_bounds__(1024) void rmsnorm_dw_kernel(int rows, int dim, const T* x, const T* dy, const float* rinv, T* dw)
+{
+    __shared__ float red[64][17];
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4, j = blockIdx.x * 16 + c;
+    float acc = 0.f;
+    if (j < dim)
+#pragma unroll 4
+        for (int i = r; i < rows; i += 64) acc += ld(dy, (size_t)i * dim + j) * (ld(x, (size_t)i * dim + j) * rinv[i]);
+    red[r][c] = acc;
+    __syncthreads();
+    if (r == 0 && j < dim) {
+        float t = 0.f;
+        for (int q = 0; q < 64; q++) t += red[q][c];
+        st(dw, j, t);
+    }
+}
+
+hipError_t k_rmsnorm_bwd(hipStream_t s, DType dt, int rows, int dim, const void* x, const void* w, const void* dy, const void* add, void* dx, void* dw,
+                         int dwRows, float* rinv, float eps)
+{
+    if (rows <= 0 || dim <= 0) return hipSuccess;
+    const int R = layernorm_wave_chunks(dim, x, dy, dx, dt == F32 ? 4 : 2, w, add);
+    const int g = (rows + 3) / 4;
+#define RMS_BWD(RR) DISPATCH_DT(dt, hipLaunchKernelGGL((rmsnorm_bwd_wave_kernel<T, RR>), g, 256, 0, s, rows, dim, (const T*)x, (const T*)w, (const T*)dy, (const T*)add, (T*)dx, rinv, eps))
+    if (R == 1) RMS_BWD(1);
+    else if (R == 2) RMS_BWD(2);
+    else if (R == 4) RMS_BWD(4);
+    else if (R == 8) RMS_BWD(8);
+    else DISPATCH_DT(dt, hipLaunchKernelGGL(rmsnorm_bwd_kernel<T>, rows, TPB, 0, s, dim, (const T*)x, (const T*)w, (const T*)dy, (const T*)add, (T*)dx, rinv, eps));
+#undef RMS_BWD
+    if (dw) DISPATCH_DT(dt, hipLaunchKernelGGL(rmsnorm_dw_kernel<T>, (dim + 15) / 16, 1024, 0, s, dwRows, dim, (const T*)x, (const T*)dy, (const float*)rinv, (T*)dw));
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Gradient of the head layout: dq, dk, dv (B,H,T,hs) become the three thirds of a row of dx (B*T, 3C), dq and dk turned back
+// by the rotation of their position when the tables are given.  One pass where the chain has three transposes, two rotations
+// and three channel copies; V elements a thread (16 bytes where the head size and the addresses allow it).
+template <typename T, int V>
+__global__ void qkv_heads_grad_kernel(uint32_t pieces, const T* dq, const T* dk, const T* dv, T* dx, uint32_t Tn, uint32_t H, uint32_t hs,
+                                      const float* __restrict__ fcos, const float* __restrict__ fsin, uint32_t seq)
+{
+    const uint32_t C = H * hs, perRow = 3 * C / V;
+    for (uint32_t p = blockIdx.x * TPB + threadIdx.x; p < pieces; p += TPB * gridDim.x) {
+        const uint32_t row = p / perRow, col = (p - row * perRow) * V, which = col / C, w = col - which * C, h = w / hs, d = w - h * hs;
+        const uint32_t b = row / Tn, t = row - b * Tn;
+        const T* src = (which == 0 ? dq : which == 1 ? dk : dv) + ((size_t)(b * H + h) * Tn + t) * hs + d;
+        float v[V];
+        if constexpr (V == 4) Vec4<T>::load(src, v);
+        else
+#pragma unroll
+            for (int j = 0; j < V; j++) v[j] = ld(src, j);
+        if constexpr (V > 1) {
+            if (fcos && which < 2) {
+                const size_t ti = (size_t)(row % seq) * (hs >> 1) + (d >> 1);
+#pragma unroll
+                for (int j = 0; j < V; j += 2) {
+                    const float c = fcos[ti + j / 2], sn = -fsin[ti + j / 2], re = v[j], im = v[j + 1];
+                    v[j] = re * c - im * sn;
+                    v[j + 1] = re * sn + im * c;
+                }
+            }
+        }
+        T* dst = dx + (size_t)row * 3 * C + col;
+        if constexpr (V == 4) Vec4<T>::store(dst, v);
+        else
+#pragma unroll
+            for (int j = 0; j < V; j++) st(dst, j, v[j]);
+    }
+}
+
+hipError_t k_qkv_heads_grad(hipStream_t s, DType dt, int B, int Tn, int H, int hs, const void* dq, const void* dk, const void* dv, void* dx,
+                            const float* fcos, const float* fsin, int seq)
+{
+    const size_t n = (size_t)B * Tn * 3 * H * hs, es = dt == F32 ? 4 : 2;
+    if (n == 0) return hipSuccess;
+    if (n > 0xf0000000ull || (fcos && (hs & 1))) return hipErrorInvalidValue;
+    const bool aligned = (((uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv | (uintptr_t)dx) & (4 * es - 1)) == 0;
+    const int V = hs % 4 == 0 && aligned ? 4 : hs % 2 == 0 ? 2 : 1;
+    const uint32_t pieces = (uint32_t)(n / V);
+#define QKV_GRAD(VV) DISPATCH_DT(dt, hipLaunchKernelGGL((qkv_heads_grad_kernel<T, VV>), grid_for(pieces), TPB, 0, s, pieces, (const T*)dq, (const T*)dk, \
+                                                        (const T*)dv, (T*)dx, (uint32_t)Tn, (uint32_t)H, (uint32_t)hs, fcos, fsin, (uint32_t)(seq > 0 ? seq : 1)))
+    if (V == 4) QKV_GRAD(4);
+    else if (V == 2) QKV_GRAD(2);
+    else QKV_GRAD(1);
+#undef QKV_GRAD
     return hipGetLastError();
 }
 
@@ -1146,6 +1375,39 @@ struct SiluGradF {   // f(dy, x) = dy * s (1 + x (1 - s)) (math.cu:11740-11749)
         return dy * (sg * (1.0f + x * (1.0f - sg)));
     }
 };
+// y = silu(a) b: da = dy b silu'(a), db = dy silu(a), in one pass
+template <typename T> __global__ void swiglu_bwd_kernel(size_t n, size_t chunks, const T* a, const T* b, const T* dy, T* da, T* db)
+{
+    const size_t gid = (size_t)blockIdx.x * TPB + threadIdx.x, stride = (size_t)TPB * gridDim.x;
+    const SiluGradF grad;
+    for (size_t c = gid; c < chunks; c += stride) {
+        float va[8], vb[8], vd[8];
+        Vec8<T>::load(a + c * 8, va);
+        Vec8<T>::load(b + c * 8, vb);
+        Vec8<T>::load(dy + c * 8, vd);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            vb[j] = grad(vd[j] * vb[j], va[j]);
+            vd[j] *= silu_f(va[j]);
+        }
+        Vec8<T>::store(da + c * 8, vb);
+        Vec8<T>::store(db + c * 8, vd);
+    }
+    for (size_t i = chunks * 8 + gid; i < n; i += stride) {
+        const float va = ld(a, i), vb = ld(b, i), vd = ld(dy, i);
+        st(da, i, grad(vd * vb, va));
+        st(db, i, vd * silu_f(va));
+    }
+}
+hipError_t k_swiglu_bwd(hipStream_t s, DType dt, size_t n, const void* a, const void* b, const void* dy, void* da, void* db)
+{
+    if (n == 0) return hipSuccess;
+    const bool aligned = ((((uintptr_t)a | (uintptr_t)b | (uintptr_t)dy | (uintptr_t)da | (uintptr_t)db) & 15) == 0);
+    const size_t chunks = aligned ? n / 8 : 0;
+    DISPATCH_DT(dt, hipLaunchKernelGGL(swiglu_bwd_kernel<T>, grid_for(chunks ? chunks : n), TPB, 0, s, n, chunks, (const T*)a, (const T*)b, (const T*)dy,
+                                       (T*)da, (T*)db));
+    return hipGetLastError();
+}
 // ReLU with negative slope (math.cu:12038-12044) and its gradient, which looks at the TOP data (math.cu:12072-12078)
 struct ReluF { float slope; __device__ float operator()(float x, float) const { return x > 0.f ? x : x * slope; } };
 struct ReluGradF {   // f(dy, y)

@@ -706,6 +706,15 @@ hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void*
     return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, Y, ws, wsBytes);
 }
 
+// the same, Y written head by head: position t of sequence b and column h hs + d go to Y[b][h][t][d] (m = B T, n = H hs)
+hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, int k, const void* X, const void* W, const void* bias, void* Y,
+                             void* ws, size_t wsBytes)
+{
+    if (B <= 0 || T <= 0 || H <= 0 || hs <= 0) return hipSuccess;
+    const HeadsEpilogue he = heads_epilogue(bias, Y, Y, Y, T, H, hs, nullptr, nullptr, 1);
+    return gemm_heads_dispatch(s, dt, B * T, H * hs, k, X, W, he, nullptr, ws, wsBytes);
+}
+
 // C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
 // split = false: A is X rounded to bf16, m rows of k.  split = true keeps the activations' precision: A holds every row of
 // an fp32 X as two bf16 rows back to back, the bf16 nearest to each of its k values and then the bf16 nearest to what
@@ -1105,7 +1114,8 @@ __global__ __launch_bounds__(256) void gemv_t_part_kernel(int m, int n, int rows
     }
 }
 
-__global__ void gemv_t_sum_kernel(int n, int chunks, float alpha, const float* __restrict__ part, float beta, float* __restrict__ y)
+template <typename T>
+__global__ void gemv_t_sum_kernel(int n, int chunks, float alpha, const float* __restrict__ part, float beta, T* __restrict__ y)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
@@ -1113,8 +1123,43 @@ __global__ void gemv_t_sum_kernel(int n, int chunks, float alpha, const float* _
 #pragma unroll 8
     for (int c = 0; c < chunks; c++) acc += part[(size_t)c * n + j];
     float v = alpha * acc;
-    if (beta != 0.f) v += beta * y[j];
-    y[j] = v;
+    if (beta != 0.f) v += beta * ldf(y, j);
+    stf(y, j, v);
+}
+
+// y += column sums of A over at most a thousand rows, one launch: a workgroup takes 16 V columns, 64 rows a trip, and adds the
+// sums of its 64 row lanes in order.  (Above that the rows are dealt over workgroups.)
+template <typename T, int V>
+__global__ __launch_bounds__(1024) void colsum_add_kernel(int m, int n, const T* __restrict__ A, T* __restrict__ y)
+{
+    __shared__ float red[64][16 * V + 1];
+    const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4, j = (blockIdx.x * 16 + cl) * V;
+    float acc[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) acc[v] = 0.f;
+    if (j < n)
+#pragma unroll 4
+        for (int i = rl; i < m; i += 64) {
+            const T* a = A + (size_t)i * n + j;
+            if constexpr (V == 4 && sizeof(T) == 4) {
+                const float4 t = *(const float4*)a;
+                acc[0] += t.x; acc[1] += t.y; acc[2] += t.z; acc[3] += t.w;
+            } else if constexpr (V == 4) {
+                const uint2 t = *(const uint2*)a;
+                acc[0] += __uint_as_float(t.x << 16); acc[1] += __uint_as_float(t.x & 0xffff0000u);
+                acc[2] += __uint_as_float(t.y << 16); acc[3] += __uint_as_float(t.y & 0xffff0000u);
+            } else acc[0] += ldf(a, 0);
+        }
+#pragma unroll
+    for (int v = 0; v < V; v++) red[rl][cl * V + v] = acc[v];
+    __syncthreads();
+    const int jj = blockIdx.x * 16 * V + threadIdx.x;
+    if (threadIdx.x < 16 * V && jj < n) {
+        float t = 0.f;
+#pragma unroll 8
+        for (int q = 0; q < 64; q++) t += red[q][threadIdx.x];
+        stf(y, jj, ldf(y, jj) + t);
+    }
 }
 
 // how the rows of a transposed product are dealt: (columns per thread, rows per workgroup, workgroups along the rows)
@@ -1162,7 +1207,7 @@ hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, 
             if (V == 4) hipLaunchKernelGGL((gemv_t_part_kernel<bf16_t, 4>), grid, 256, 0, s, m, n, rowsPer, (const bf16_t*)A, x, part);
             else hipLaunchKernelGGL((gemv_t_part_kernel<bf16_t, 1>), grid, 256, 0, s, m, n, rowsPer, (const bf16_t*)A, x, part);
         }
-        hipLaunchKernelGGL(gemv_t_sum_kernel, (n + 63) / 64, 64, 0, s, n, chunks, alpha, part, beta, y);
+        hipLaunchKernelGGL(gemv_t_sum_kernel<float>, (n + 63) / 64, 64, 0, s, n, chunks, alpha, part, beta, y);
     } else {
         int grid = (n + 255) / 256;
         if (adt == F32)
@@ -1170,6 +1215,32 @@ hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, 
         else
             hipLaunchKernelGGL(gemv_t_kernel<bf16_t>, grid, 256, 0, s, m, n, alpha, (const bf16_t*)A, x, beta, y);
     }
+    return hipGetLastError();
+}
+
+// Bias gradient of an inner product: db (n) += column sums of dY (m x n), both in the storage type.  In 16-bit storage the
+// gemv call this replaces widened its vectors in launches of their own: six launches of some 5 us each at 8000 x 3072, two now.
+size_t k_bias_grad_workspace_bytes(int m, int n) { return m <= 1024 ? 0 : k_gemv_workspace_bytes(true, m, n); }
+template <typename T> static void bias_grad(hipStream_t s, DType dt, int m, int n, const T* dY, T* db, float* part)
+{
+    if (m <= 1024) {
+        if (n % 4 == 0 && ((uintptr_t)dY % (4 * sizeof(T))) == 0) hipLaunchKernelGGL((colsum_add_kernel<T, 4>), (n + 63) / 64, 1024, 0, s, m, n, dY, db);
+        else hipLaunchKernelGGL((colsum_add_kernel<T, 1>), (n + 15) / 16, 1024, 0, s, m, n, dY, db);
+        return;
+    }
+    int V, rowsPer, chunks;
+    gemv_t_split(dt, m, n, dY, &V, &rowsPer, &chunks);
+    const dim3 grid((n + 16 * V - 1) / (16 * V), chunks);
+    if (V == 4) hipLaunchKernelGGL((gemv_t_part_kernel<T, 4>), grid, 256, 0, s, m, n, rowsPer, dY, (const float*)nullptr, part);
+    else hipLaunchKernelGGL((gemv_t_part_kernel<T, 1>), grid, 256, 0, s, m, n, rowsPer, dY, (const float*)nullptr, part);
+    hipLaunchKernelGGL(gemv_t_sum_kernel<T>, (n + 63) / 64, 64, 0, s, n, chunks, 1.f, (const float*)part, 1.f, db);
+}
+hipError_t k_bias_grad(hipStream_t s, DType dt, int m, int n, const void* dY, void* db, void* ws, size_t wsBytes)
+{
+    if (m <= 0 || n <= 0) return hipSuccess;
+    if (wsBytes < k_bias_grad_workspace_bytes(m, n)) return hipErrorInvalidValue;
+    if (dt == F32) bias_grad<float>(s, dt, m, n, (const float*)dY, (float*)db, (float*)ws);
+    else bias_grad<bf16_t>(s, dt, m, n, (const bf16_t*)dY, (bf16_t*)db, (float*)ws);
     return hipGetLastError();
 }
 

@@ -70,10 +70,12 @@ inline bool softmax_bwd_keeps_zeros(int len, int inner) { return inner == 1 && l
 // adjacent-pair rotary embedding with the CudaDnnDLL index rule; x == y allowed
 hipError_t k_rope(hipStream_t s, DType dt, size_t n, const void* x, void* y, const float* fcos, const float* fsin,
                   int seqLen, int heads, int hs, int tableOff, bool grad = false);
-// LayerNorm without affine part over rows x inner; stdev[rows] keeps sqrt(var + eps) of every row for the gradient
-hipError_t k_layernorm_fwd(hipStream_t s, DType dt, int rows, int inner, const void* x, void* y, float* stdev, float eps);
+// LayerNorm without affine part over rows x inner; stdev[rows] keeps sqrt(var + eps) of every row for the gradient.
+// Norms with `add`: forward normalises total = x + add (stored), backward adds `add` to dx.
+hipError_t k_layernorm_fwd(hipStream_t s, DType dt, int rows, int inner, const void* x, void* y, float* stdev, float eps, const void* add = nullptr,
+                           void* total = nullptr);
 hipError_t k_layernorm_bwd(hipStream_t s, DType dt, int rows, int inner, const void* y, const void* dy, void* dx,
-                           const float* stdev, float bump);
+                           const float* stdev, float bump, const void* add = nullptr);
 hipError_t k_gelu_fwd(hipStream_t s, DType dt, size_t n, const void* x, void* y, bool bert);
 hipError_t k_gelu_bwd(hipStream_t s, DType dt, size_t n, const void* dy, const void* x, void* dx, bool bert);
 hipError_t k_relu_fwd(hipStream_t s, DType dt, size_t n, const void* x, void* y, float slope);
@@ -92,7 +94,15 @@ hipError_t k_channel_rowsum(hipStream_t s, DType dt, size_t rows, int inner, con
 hipError_t k_channel_colsum(hipStream_t s, DType dt, size_t outer, int channels, int spatial, const void* x, void* y);
 // mode 0 fillfrom forward, 1 fillfrom backward, 2 copyall, 3 duplicate (index rules in ew_kernels.hip)
 hipError_t k_channel_spread(hipStream_t s, DType dt, int mode, size_t n, size_t spatial, size_t period, size_t channels, void* x, void* y);
-hipError_t k_rmsnorm(hipStream_t s, DType dt, int outer, int dim, const void* x, const void* w, void* y, float eps);
+hipError_t k_rmsnorm(hipStream_t s, DType dt, int outer, int dim, const void* x, const void* w, void* y, float eps, const void* add = nullptr,
+                     void* total = nullptr);
+// dw (may be null) is overwritten with the sums of the first dwRows rows; rinv: scratch of `rows` floats, needed with dw
+hipError_t k_rmsnorm_bwd(hipStream_t s, DType dt, int rows, int dim, const void* x, const void* w, const void* dy, const void* add, void* dx, void* dw,
+                         int dwRows, float* rinv, float eps);
+// dx (B*T, 3 H hs) from the head gradients (B,H,T,hs), rotated back when the tables are given (row % seq is the position)
+hipError_t k_qkv_heads_grad(hipStream_t s, DType dt, int B, int Tn, int H, int hs, const void* dq, const void* dk, const void* dv, void* dx,
+                            const float* fcos, const float* fsin, int seq);
+hipError_t k_swiglu_bwd(hipStream_t s, DType dt, size_t n, const void* a, const void* b, const void* dy, void* da, void* db);
 // primitives of the CAFFE-engine softmax chain: x is (num, channels, spatial), reduced tensors (num, spatial)
 hipError_t k_exp(hipStream_t s, DType dt, size_t n, const void* a, void* y, float beta);
 hipError_t k_log(hipStream_t s, DType dt, size_t n, const void* a, void* y, float beta, float alpha);
@@ -115,6 +125,8 @@ hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs
 // Y (m x n) = X (m x k) W^T + bias in one call; ws: k_gemm_bias_workspace_bytes(...) of scratch
 hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes);
 // scratch of k_gemm_bias / k_gemm_qkv_heads with these operands (0: none)
+hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, int k, const void* X, const void* W, const void* bias, void* Y,
+                             void* ws, size_t wsBytes);   // Y as (B,H,T,hs); scratch as k_gemm_bias
 size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W);
 size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W);
 // column-major strided batched gemm with BLAS semantics (fp32)
@@ -139,6 +151,8 @@ hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float a
 size_t k_gemv_workspace_bytes(bool tA, int m, int n);   // scratch for the partial sums of a transposed product over many rows
 hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, const void* A, const float* x,
                   float beta, float* y, void* ws = nullptr, size_t wsBytes = 0);
+size_t k_bias_grad_workspace_bytes(int m, int n);
+hipError_t k_bias_grad(hipStream_t s, DType dt, int m, int n, const void* dY, void* db, void* ws, size_t wsBytes);   // db += column sums
 
 // ---- attention (attn_prefill.hip, attn_decode.hip) --------------------------
 enum MaskKind { MASK_NONE = 0, MASK_QK = 1, MASK_KEY = 2, MASK_BQK = 3, MASK_CAUSAL = 4 };

@@ -1686,6 +1686,111 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         return 0;
     }
 
+    case MCH_FN_SWIGLU_BWD: {
+        NEED_L(6, 6);
+        const long long n = pl[0];
+        MemItem *A, *B, *dY, *dA, *dB;
+        ERRCHK(mem((long)pl[1], &A));
+        ERRCHK(mem((long)pl[2], &B));
+        ERRCHK(mem((long)pl[3], &dY));
+        ERRCHK(mem((long)pl[4], &dA));
+        ERRCHK(mem((long)pl[5], &dB));
+        if (A->half != B->half || A->half != dY->half || A->half != dA->half || A->half != dB->half) return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+        RANGE(A, 0, n);
+        RANGE(B, 0, n);
+        RANGE(dY, 0, n);
+        RANGE(dA, 0, n);
+        RANGE(dB, 0, n);
+        HIPCHK(k_swiglu_bwd(s, A->dt(), (size_t)n, A->ptr, B->ptr, dY->ptr, dA->ptr, dB->ptr));
+        m_mem.touch((long)pl[4]);
+        m_mem.touch((long)pl[5]);
+        return 0;
+    }
+
+    case MCH_FN_RMSNORM_BWD: {
+        NEED_F(1, 1);
+        NEED_L(8, 9);
+        const long long rows = pl[0], dim = pl[1], dwRows = pl[7];
+        if (rows < 0 || dim < 1 || rows > INT_MAX || dim > INT_MAX || dwRows < 0 || dwRows > rows) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        MemItem *X, *W = nullptr, *dY, *dX, *dW = nullptr, *Add = nullptr;
+        ERRCHK(mem((long)pl[2], &X));
+        if (pl[3]) ERRCHK(mem((long)pl[3], &W));
+        ERRCHK(mem((long)pl[4], &dY));
+        ERRCHK(mem((long)pl[5], &dX));
+        if (pl[6]) ERRCHK(mem((long)pl[6], &dW));
+        if (ll > 8 && pl[8]) ERRCHK(mem((long)pl[8], &Add));
+        if (X->half != dY->half || X->half != dX->half || (W && W->half != X->half) || (dW && dW->half != X->half) || (Add && Add->half != X->half))
+            return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+        RANGE(X, 0, rows * dim);
+        RANGE(dY, 0, rows * dim);
+        RANGE(dX, 0, rows * dim);
+        if (W) RANGE(W, 0, dim);
+        if (dW) RANGE(dW, 0, dim);
+        if (Add) RANGE(Add, 0, rows * dim);
+        if (dW && (dX->ptr == X->ptr || dX->ptr == dY->ptr)) return MCH_ERROR_PARAM_OUT_OF_RANGE;   // the weight gradient reads both afterwards
+        void* ws = nullptr;
+        if (dW) ERRCHK(workspace((size_t)rows * sizeof(float), &ws));
+        HIPCHK(k_rmsnorm_bwd(s, X->dt(), (int)rows, (int)dim, X->ptr, W ? W->ptr : nullptr, dY->ptr, Add ? Add->ptr : nullptr, dX->ptr,
+                             dW ? dW->ptr : nullptr, (int)dwRows, (float*)ws, pf[0]));
+        m_mem.touch((long)pl[5]);
+        if (dW) m_mem.touch((long)pl[6]);
+        return 0;
+    }
+
+    case MCH_FN_NORM_ADD_FWD: {
+        NEED_F(1, 1);
+        NEED_L(8, 8);
+        LayerNormState* ln = nullptr;
+        long long rows = pl[1], dim = pl[2];
+        if (pl[0]) {
+            ln = m_layernorm.get((long)pl[0]);
+            if (!ln || !ln->set) return MCH_ERROR_LAYERNORM_NOT_INITIALIZED;
+            rows = (long long)ln->outer * ln->channels;
+            dim = ln->inner;
+        }
+        if (rows < 0 || dim < 1 || rows > INT_MAX || dim > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        MemItem *X, *Add, *Total, *W = nullptr, *Y;
+        ERRCHK(mem((long)pl[3], &X));
+        ERRCHK(mem((long)pl[4], &Add));
+        ERRCHK(mem((long)pl[5], &Total));
+        if (pl[6] && !ln) ERRCHK(mem((long)pl[6], &W));
+        ERRCHK(mem((long)pl[7], &Y));
+        if (X->half != Add->half || X->half != Total->half || X->half != Y->half || (W && W->half != X->half)) return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+        RANGE(X, 0, rows * dim);
+        RANGE(Add, 0, rows * dim);
+        RANGE(Total, 0, rows * dim);
+        RANGE(Y, 0, rows * dim);
+        if (W) RANGE(W, 0, dim);
+        if (Total->ptr == Y->ptr) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        if (ln) {
+            HIPCHK(k_layernorm_fwd(s, X->dt(), (int)rows, (int)dim, X->ptr, Y->ptr, ln->stdev, ln->eps, Add->ptr, Total->ptr));
+            ln->backwards = 0;
+        } else HIPCHK(k_rmsnorm(s, X->dt(), (int)rows, (int)dim, X->ptr, W ? W->ptr : nullptr, Y->ptr, pf[0], Add->ptr, Total->ptr));
+        m_mem.touch((long)pl[5]);
+        m_mem.touch((long)pl[7]);
+        return 0;
+    }
+    case MCH_FN_NORM_ADD_BWD: {
+        NEED_L(5, 5);
+        LayerNormState* ln = m_layernorm.get((long)pl[0]);
+        if (!ln || !ln->set) return MCH_ERROR_LAYERNORM_NOT_INITIALIZED;
+        MemItem *Y, *dY, *dX, *Add;
+        ERRCHK(mem((long)pl[1], &Y));
+        ERRCHK(mem((long)pl[2], &dY));
+        ERRCHK(mem((long)pl[3], &dX));
+        ERRCHK(mem((long)pl[4], &Add));
+        if (Y->half != dY->half || Y->half != dX->half || Y->half != Add->half) return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+        RANGE(Y, 0, ln->count);
+        RANGE(dY, 0, ln->count);
+        RANGE(dX, 0, ln->count);
+        RANGE(Add, 0, ln->count);
+        ln->backwards++;
+        HIPCHK(k_layernorm_bwd(s, Y->dt(), ln->outer * ln->channels, ln->inner, Y->ptr, dY->ptr, dX->ptr, ln->stdev,
+                               ln->eps * (float)ln->backwards, Add->ptr));
+        m_mem.touch((long)pl[3]);
+        return 0;
+    }
+
     // ---- cuDNN-shaped handles: opaque records here ---------------------------
     case MCH_FN_CREATE_CUDNN: {
         // f{[stream]} (device.h:1201-1221)
@@ -2055,10 +2160,13 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
     }
 
     case MCH_FN_LINEAR_FWD: {
-        // l{M, N, K, hX, hW, hBias(0 = none), hY}: Y (M x N) = X (M x K) W^T (N x K) + bias (N), one launch
-        NEED_L(7, 7);
+        // l{M, N, K, hX, hW, hBias(0 = none), hY[, T, heads]}: Y (M x N) = X (M x K) W^T (N x K) + bias (N), one launch; with
+        // T and heads written as (M/T, heads, T, N/heads)
+        NEED_L(7, 9);
         const long long M = pl[0], N = pl[1], K = pl[2];
         if (M < 1 || N < 1 || K < 1 || M > INT_MAX || N > INT_MAX || K > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        const long long T = ll > 7 ? pl[7] : 0, heads = ll > 8 ? pl[8] : 0;
+        if (ll > 7 && (ll != 9 || T < 1 || heads < 1 || M % T || N % heads)) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         MemItem *X, *W, *Bi = nullptr, *Y;
         ERRCHK(mem((long)pl[3], &X));
         ERRCHK(mem((long)pl[4], &W));
@@ -2072,8 +2180,75 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         void* ws = nullptr;
         const size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr);
         if (wsb) ERRCHK(workspace(wsb, &ws));
-        HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
+        if (heads)
+            HIPCHK(k_gemm_bias_heads(s, X->dt(), (int)(M / T), (int)T, (int)heads, (int)(N / heads), (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
+        else HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
         m_mem.touch((long)pl[6]);
+        return 0;
+    }
+
+    case MCH_FN_LINEAR_BWD: {
+        // l{M, N, K, hX, hW, hdY, hdW, hdBias(0 = none), hdX(0 = none)[, accumX]}
+        NEED_L(9, 10);
+        const long long M = pl[0], N = pl[1], K = pl[2];
+        const bool accum = ll > 9 && pl[9] != 0;
+        if (M < 1 || N < 1 || K < 1 || M > INT_MAX || N > INT_MAX || K > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        MemItem *X, *W, *dY, *dW, *dB = nullptr, *dX = nullptr;
+        ERRCHK(mem((long)pl[3], &X));
+        ERRCHK(mem((long)pl[4], &W));
+        ERRCHK(mem((long)pl[5], &dY));
+        ERRCHK(mem((long)pl[6], &dW));
+        if (pl[7]) ERRCHK(mem((long)pl[7], &dB));
+        if (pl[8]) ERRCHK(mem((long)pl[8], &dX));
+        if (X->half != W->half || X->half != dY->half || X->half != dW->half || (dB && dB->half != X->half) || (dX && dX->half != X->half))
+            return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+        RANGE(X, 0, M * K);
+        RANGE(W, 0, N * K);
+        RANGE(dY, 0, M * N);
+        RANGE(dW, 0, N * K);
+        if (dB) RANGE(dB, 0, N);
+        if (dX) RANGE(dX, 0, M * K);
+        const DType dt = X->dt();
+        const size_t wsW = k_gemm_workspace_bytes(dt, true, false, (int)N, (int)K, (int)M), wsB = dB ? k_bias_grad_workspace_bytes((int)M, (int)N) : 0;
+        const size_t wsX = dX ? k_gemm_workspace_bytes(dt, false, false, (int)M, (int)K, (int)N) : 0, most = std::max(wsW, std::max(wsB, wsX));
+        void* ws = nullptr;
+        if (most) ERRCHK(workspace(most, &ws));
+        HIPCHK(k_gemm(s, dt, true, false, (int)N, (int)K, (int)M, 1.f, dY->ptr, X->ptr, 1.f, dW->ptr, ws, wsW));
+        if (dB) HIPCHK(k_bias_grad(s, dt, (int)M, (int)N, dY->ptr, dB->ptr, ws, wsB));
+        if (dX) HIPCHK(k_gemm(s, dt, false, false, (int)M, (int)K, (int)N, 1.f, dY->ptr, W->ptr, accum ? 1.f : 0.f, dX->ptr, ws, wsX));
+        m_mem.touch((long)pl[6]);
+        if (dB) m_mem.touch((long)pl[7]);
+        if (dX) m_mem.touch((long)pl[8]);
+        return 0;
+    }
+    case MCH_FN_QKV_HEADS_GRAD: {
+        // l{batch, T, heads, hs, hdQ, hdK, hdV, hdX[, hRope]}
+        NEED_L(8, 9);
+        const long long B = pl[0], T = pl[1], H = pl[2], hs = pl[3];
+        if (B < 1 || T < 1 || H < 1 || hs < 1 || B * T > INT_MAX || 3 * H * hs > INT_MAX || B * T * 3 * H * hs > 0xf0000000ll) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        const long long n = B * T * H * hs;
+        MemItem *dQ, *dK, *dV, *dX;
+        ERRCHK(mem((long)pl[4], &dQ));
+        ERRCHK(mem((long)pl[5], &dK));
+        ERRCHK(mem((long)pl[6], &dV));
+        ERRCHK(mem((long)pl[7], &dX));
+        if (dX->half != dQ->half || dX->half != dK->half || dX->half != dV->half) return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+        RANGE(dQ, 0, n);
+        RANGE(dK, 0, n);
+        RANGE(dV, 0, n);
+        RANGE(dX, 0, 3 * n);
+        RopeState* r = nullptr;
+        if (ll > 8 && pl[8]) {
+            r = m_rope.get((long)pl[8]);
+            if (!r || !r->set) return MCH_ERROR_ROPE_NOT_INITIALIZED;
+            if (r->heads != H || r->hs != hs) {
+                last_detail = "the rope handle was created for other heads or another head size";
+                return MCH_ERROR_PARAM_OUT_OF_RANGE;
+            }
+        }
+        HIPCHK(k_qkv_heads_grad(s, dX->dt(), (int)B, (int)T, (int)H, (int)hs, dQ->ptr, dK->ptr, dV->ptr, dX->ptr,
+                                r ? (const float*)r->dcos.get() : nullptr, r ? (const float*)r->dsin.get() : nullptr, r ? r->seq : 1));
+        m_mem.touch((long)pl[7]);
         return 0;
     }
 
@@ -2490,7 +2665,7 @@ static const char* api_name(long fn)
 #define N(x) {MCH_FN_##x, "CUDA_FN_" #x}
     static const struct { long id; const char* name; } table[] = {
         {MCH_DLL_FREEMEM, "CUDA_DLL_FREEMEM"}, {MCH_DLL_INITIALIZE, "CUDA_DLL_INITIALIZE"}, {MCH_DLL_CLEANUP, "CUDA_DLL_CLEANUP"},
-        N(SETDEVICE), N(GETDEVICE), N(SYNCHRONIZEDEVICE), N(CREATE_MEMORYPOINTER), N(FREE_MEMORYPOINTER), N(ALLOCMEM_HALF), N(ALLOCMEM), N(FREEMEM), N(GETMEM), N(SETMEM), N(CREATE_CUDNN), N(FREE_CUDNN), N(CREATE_TENSORDESC), N(FREE_TENSORDESC), N(SET_TENSORDESC), N(CREATE_EXTENSION), N(FREE_EXTENSION), N(EXTENSION_RUN), N(SOFTMAX_FWD), N(SOFTMAX_BWD), N(ATTN_CREATE), N(ATTN_FREE), N(ATTN_SET), N(ATTN_FWD), N(ATTN_BWD), N(SET), N(COPY), N(GEMM2), N(GEMM), N(GEMV), N(AXPY), N(SCAL), N(SCALE), N(ADD_SCALAR), N(ADD), N(SUB), N(MUL), N(DIV), N(EXP), N(LOG), N(POWX), N(SQRT), N(TRANSPOSE), N(MASK), N(MASK_BATCH), N(TRANSPOSE_HW), N(INVERT), N(CHANNEL_MEAN), N(CHANNEL_MAX), N(CHANNEL_SUB), N(CHANNEL_SUM), N(CHANNEL_DIV), N(CHANNEL_DOT), N(CHANNEL_COPY), N(CHANNEL_FILLFROM), N(CHANNEL_COPYALL), N(CHANNEL_DUP), N(CHANNEL_SUM2), N(EMBED_FWD), N(RELU_FWD), N(RELU_BWD), N(GELU_FWD), N(GELU_BWD), N(SILU_FWD), N(SILU_BWD), N(CREATE_LAYERNORM), N(FREE_LAYERNORM), N(LAYERNORM_FWD), N(LAYERNORM_BWD), N(CREATE_ROPE), N(FREE_ROPE), N(ROPE_FWD), N(ROPE_BWD), N(CREATE_BLOBLOADER), N(FREE_BLOBLOADER), N(BLOBLOADER_LOAD), N(BLOBLOADER_RESETOFFSET), N(BLOBLOADER_ADDTOOFFSET), N(ATTN_DECODE_FWD), N(RMSNORM_FWD), N(SWIGLU_FWD), N(QKV_PROJ_HEADS), N(LINEAR_FWD)};
+        N(SETDEVICE), N(GETDEVICE), N(SYNCHRONIZEDEVICE), N(CREATE_MEMORYPOINTER), N(FREE_MEMORYPOINTER), N(ALLOCMEM_HALF), N(ALLOCMEM), N(FREEMEM), N(GETMEM), N(SETMEM), N(CREATE_CUDNN), N(FREE_CUDNN), N(CREATE_TENSORDESC), N(FREE_TENSORDESC), N(SET_TENSORDESC), N(CREATE_EXTENSION), N(FREE_EXTENSION), N(EXTENSION_RUN), N(SOFTMAX_FWD), N(SOFTMAX_BWD), N(ATTN_CREATE), N(ATTN_FREE), N(ATTN_SET), N(ATTN_FWD), N(ATTN_BWD), N(SET), N(COPY), N(GEMM2), N(GEMM), N(GEMV), N(AXPY), N(SCAL), N(SCALE), N(ADD_SCALAR), N(ADD), N(SUB), N(MUL), N(DIV), N(EXP), N(LOG), N(POWX), N(SQRT), N(TRANSPOSE), N(MASK), N(MASK_BATCH), N(TRANSPOSE_HW), N(INVERT), N(CHANNEL_MEAN), N(CHANNEL_MAX), N(CHANNEL_SUB), N(CHANNEL_SUM), N(CHANNEL_DIV), N(CHANNEL_DOT), N(CHANNEL_COPY), N(CHANNEL_FILLFROM), N(CHANNEL_COPYALL), N(CHANNEL_DUP), N(CHANNEL_SUM2), N(EMBED_FWD), N(RELU_FWD), N(RELU_BWD), N(GELU_FWD), N(GELU_BWD), N(SILU_FWD), N(SILU_BWD), N(CREATE_LAYERNORM), N(FREE_LAYERNORM), N(LAYERNORM_FWD), N(LAYERNORM_BWD), N(CREATE_ROPE), N(FREE_ROPE), N(ROPE_FWD), N(ROPE_BWD), N(CREATE_BLOBLOADER), N(FREE_BLOBLOADER), N(BLOBLOADER_LOAD), N(BLOBLOADER_RESETOFFSET), N(BLOBLOADER_ADDTOOFFSET), N(ATTN_DECODE_FWD), N(RMSNORM_FWD), N(SWIGLU_FWD), N(QKV_PROJ_HEADS), N(LINEAR_FWD), N(LINEAR_BWD), N(QKV_HEADS_GRAD), N(RMSNORM_BWD), N(SWIGLU_BWD), N(NORM_ADD_FWD), N(NORM_ADD_BWD)};
 #undef N
     for (const auto& t : table)
         if (t.id == fn) return t.name;

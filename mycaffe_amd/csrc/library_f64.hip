@@ -5,8 +5,8 @@
 // It covers the function ids of the attention path and of the layers around it - memory, GEMM / GEMM2 / GEMV and the
 // vector updates, mask, the transposes, channel copy and the channel reductions / broadcasts, softmax, the attention
 // handle, rotary embedding, layer norm handle, RMS norm, the activations, each forward and backward, embedding lookup -
-// with plain kernels: one output element per thread, reductions by one workgroup per row, nothing tiled for the matrix
-// cores.  This is the precision twin of the fp32 path, for hosts that instantiate their layers in
+// with plain kernels: one output element per thread, reductions by one workgroup per row; products run on the double
+// matrix cores.  This is the precision twin of the fp32 path, for hosts that instantiate their layers in
 // double; the fast kernels are the fp32 / bf16 ones.  Every other id returns MCH_ERROR_NOT_IMPLEMENTED with its number
 // in the message.  ALLOCMEM_HALF allocates doubles (no 16-bit storage under this base type).
 #include <hip/hip_runtime.h>
@@ -103,9 +103,9 @@ __global__ void d_mask_kernel(size_t n, size_t md1, size_t dd1, const double* x,
 // the other.  G groups of four wavefronts of a workgroup therefore take every G-th stage each, with stages of their own, and
 // their sums are added in order through LDS at the end (256 x 256 x 1024: 27 us with one group, 9 us with four; one output
 // per thread took 45 us).
-// zdiv: matrix z of C lies at (z / zdiv) sC + (z % zdiv) sC2.
+// zdiv: matrix z of C lies at (z / zdiv) sC + (z % zdiv) sC2.  bias (may be null): one value per column, added to every row.
 typedef double d_vec4 __attribute__((ext_vector_type(4)));
-struct GemmD { int m, n, k; double alpha, beta; const double *A, *B; double* C; long long ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2; int zdiv; };
+struct GemmD { int m, n, k; double alpha, beta; const double *A, *B; double* C; long long ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2; int zdiv; const double* bias; };
 template <int W, int G> __global__ __launch_bounds__(256 * G) void d_gemm_kernel(GemmD g)
 {
     constexpr int BT = 32 * W, BK = 16, LD = BK + 2, NE = BT * BK / 256, STAGE = 2 * BT * LD;
@@ -196,7 +196,8 @@ template <int W, int G> __global__ __launch_bounds__(256 * G) void d_gemm_kernel
                 const int r = m0 + wm + 16 * i + 4 * v + fk, c = n0 + wn + 16 * j + fr;
                 if (r >= g.m || c >= g.n) continue;
                 double* cp = C + (long long)r * g.crs + (long long)c * g.ccs;
-                const double t = g.alpha * acc[i][j][v];
+                double t = g.alpha * acc[i][j][v];
+                if (g.bias) t += g.bias[c];
                 *cp = g.beta == 0.0 ? t : t + g.beta * *cp;
             }
 }
@@ -204,9 +205,9 @@ template <int W, int G> __global__ __launch_bounds__(256 * G) void d_gemm_kernel
 // them fit a CU) and the contraction has stages for them
 static hipError_t d_gemm(hipStream_t s, int batch, int m, int n, int k, double alpha, const double* A, long long ars, long long acs, const double* B,
                          long long brs, long long bcs, double beta, double* C, long long crs, long long ccs, long long sA, long long sB, long long sC,
-                         int zdiv = 1, long long sC2 = 0)
+                         int zdiv = 1, long long sC2 = 0, const double* bias = nullptr)
 {
-    GemmD g = {m, n, k, alpha, beta, A, B, C, ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2, zdiv};
+    GemmD g = {m, n, k, alpha, beta, A, B, C, ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2, zdiv, bias};
     const long long big = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch, small = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch;
     const dim3 gridBig((n + 63) / 64, (m + 63) / 64, batch), gridSmall((n + 31) / 32, (m + 31) / 32, batch);
     if (gridSmall.y > 65535) return hipErrorInvalidValue;
@@ -443,10 +444,18 @@ __global__ __launch_bounds__(256) void d_softmax_bwd_kernel(const double* y, con
     }
 }
 // y = (x - mean) / sqrt(var + eps) per row, the row's sqrt(var + eps) kept (layernorm.cu:219-262)
-__global__ __launch_bounds__(256) void d_layernorm_fwd_kernel(int inner, const double* x, double* y, double* stdev, double eps)
+// with `add`: total = x + add is stored and normalised (a thread reads back only what it wrote)
+__device__ inline const double* d_add_row(int inner, const double* x, const double* add, double* total)
+{
+    const size_t base = (size_t)blockIdx.x * inner;
+    if (!add) return x + base;
+    for (int i = threadIdx.x; i < inner; i += 256) total[base + i] = x[base + i] + add[base + i];
+    return total + base;
+}
+__global__ __launch_bounds__(256) void d_layernorm_fwd_kernel(int inner, const double* x, const double* add, double* total, double* y, double* stdev, double eps)
 {
     __shared__ double red[4];
-    const double* xr = x + (size_t)blockIdx.x * inner;
+    const double* xr = d_add_row(inner, x, add, total);
     double* yr = y + (size_t)blockIdx.x * inner;
     double sum = 0.0;
     for (int i = threadIdx.x; i < inner; i += 256) sum += xr[i];
@@ -459,8 +468,8 @@ __global__ __launch_bounds__(256) void d_layernorm_fwd_kernel(int inner, const d
 }
 // dx = (dy - (y mean(y dy) + mean(dy))) / divisor (layernorm.cu:268-312); the reference adds eps to the first `rows`
 // entries of its row-expanded stdev array on every backward call: `bump` = eps x (backward calls since the forward)
-__global__ __launch_bounds__(256) void d_layernorm_bwd_kernel(int rows, int inner, const double* y, const double* dy, double* dx,
-                                                              const double* stdev, double bump)
+__global__ __launch_bounds__(256) void d_layernorm_bwd_kernel(int rows, int inner, const double* y, const double* dy, const double* add,
+                                                              double* dx, const double* stdev, double bump)
 {
     __shared__ double red[4];
     const size_t base = (size_t)blockIdx.x * inner;
@@ -471,19 +480,82 @@ __global__ __launch_bounds__(256) void d_layernorm_bwd_kernel(int rows, int inne
     const double sd = stdev[blockIdx.x];
     for (int i = threadIdx.x; i < inner; i += 256) {
         const double div = base + i < (size_t)rows ? sd + bump : sd;
-        dx[base + i] = (dy[base + i] - (y[base + i] * m1 + m2)) / div;
+        const double g = (dy[base + i] - (y[base + i] * m1 + m2)) / div;
+        dx[base + i] = add ? g + add[base + i] : g;
     }
 }
 // y = w (x / sqrt(mean(x^2) + eps)), one workgroup per row
-__global__ __launch_bounds__(256) void d_rmsnorm_kernel(int dim, const double* x, const double* w, double* y, double eps)
+__global__ __launch_bounds__(256) void d_rmsnorm_kernel(int dim, const double* x, const double* add, double* total, const double* w, double* y, double eps)
 {
     __shared__ double red[4];
-    const double* xr = x + (size_t)blockIdx.x * dim;
+    const double* xr = d_add_row(dim, x, add, total);
     double* yr = y + (size_t)blockIdx.x * dim;
     double ss = 0.0;
     for (int i = threadIdx.x; i < dim; i += 256) ss += xr[i] * xr[i];
     const double inv = 1.0 / sqrt(d_block_reduce(ss, red, false) / dim + eps);
     for (int i = threadIdx.x; i < dim; i += 256) yr[i] = w ? w[i] * (inv * xr[i]) : inv * xr[i];
+}
+// with g = dy w and r = 1 / sqrt(mean(x^2) + eps): dx = g r - x r^3 sum(g x) / dim (+ add); r kept per row for the weight gradient
+__global__ __launch_bounds__(256) void d_rmsnorm_bwd_kernel(int dim, const double* x, const double* w, const double* dy, const double* add, double* dx,
+                                                            double* rinv, double eps)
+{
+    __shared__ double red[4];
+    const size_t base = (size_t)blockIdx.x * dim;
+    double ss = 0.0, sg = 0.0;
+    for (int i = threadIdx.x; i < dim; i += 256) {
+        const double v = x[base + i];
+        ss += v * v;
+        sg += dy[base + i] * (w ? w[i] : 1.0) * v;
+    }
+    const double inv = 1.0 / sqrt(d_block_reduce(ss, red, false) / dim + eps);
+    const double f = d_block_reduce(sg, red, false) * inv * inv * inv / dim;
+    if (rinv && threadIdx.x == 0) rinv[blockIdx.x] = inv;
+    for (int i = threadIdx.x; i < dim; i += 256) {
+        const double g = dy[base + i] * (w ? w[i] : 1.0) * inv - x[base + i] * f;
+        dx[base + i] = add ? g + add[base + i] : g;
+    }
+}
+// the sums of the 64 row lanes [lane][column] of a workgroup of 1024 threads, added in order by its first sixteen
+__device__ inline double d_lane_sums(double acc, double (&red)[64][17])
+{
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+    red[r][c] = acc;
+    __syncthreads();
+    double t = 0.0;
+    if (r == 0)
+        for (int q = 0; q < 64; q++) t += red[q][c];
+    return t;
+}
+__global__ __launch_bounds__(1024) void d_rmsnorm_dw_kernel(int rows, int dim, const double* x, const double* dy, const double* rinv, double* dw)
+{
+    __shared__ double red[64][17];
+    const int r = threadIdx.x >> 4, j = blockIdx.x * 16 + (threadIdx.x & 15);
+    double acc = 0.0;
+    if (j < dim)
+        for (int i = r; i < rows; i += 64) acc += dy[(size_t)i * dim + j] * (x[(size_t)i * dim + j] * rinv[i]);
+    acc = d_lane_sums(acc, red);
+    if (r == 0 && j < dim) dw[j] = acc;
+}
+// y += column sums of A (m, n): the bias gradient of an inner product
+__global__ __launch_bounds__(1024) void d_colsum_add_kernel(int m, int n, const double* A, double* y)
+{
+    __shared__ double red[64][17];
+    const int r = threadIdx.x >> 4, j = blockIdx.x * 16 + (threadIdx.x & 15);
+    double acc = 0.0;
+    if (j < n)
+        for (int i = r; i < m; i += 64) acc += A[(size_t)i * n + j];
+    acc = d_lane_sums(acc, red);
+    if (r == 0 && j < n) y[j] += acc;
+}
+// y = silu(a) b: da = dy b silu'(a), db = dy silu(a)
+__global__ void d_swiglu_bwd_kernel(size_t n, const double* a, const double* b, const double* dy, double* da, double* db)
+{
+    GRID_STRIDE(i, n)
+    {
+        const double sg = 1.0 / (1.0 + exp(-a[i])), va = a[i], vb = b[i], vd = dy[i];
+        da[i] = vd * vb * (sg * (1.0 + va * (1.0 - sg)));
+        db[i] = vd * (va * sg);
+    }
 }
 // dS = P (dP - sum_k P dP) per row, in place in dp (the softmax gradient of attn.cu:608-661); one wavefront a row
 __global__ __launch_bounds__(256) void d_attn_ds_kernel(size_t rows, const double* p, double* dp, int Tk)
@@ -646,32 +718,44 @@ __global__ void d_rope_append_kernel(double* q, double* knew, const double* vnew
     }
 }
 
-// Epilogue of the fused QKV projection (id 2004): the plain product `tmp` (B*T, 3C) gets its bias and goes, head by head,
-// to q, k, v as (B,H,T,hs); q and k are rotated on the way when the tables are given (position = row % seq).
-__global__ void d_qkv_split_kernel(size_t pairs, const double* tmp, const double* bias, double* q, double* k, double* v, int T, int H,
-                                   int hs, const double* fcos, const double* fsin, int seq)
+// Between the rows of the fused QKV projection (B*T, 3C; a single projection: parts = 1) and q, k, v as (B,H,T,hs); q and k are rotated on the way when the
+// tables are given (position = row % seq; pairs of values, V = 2).  Forward (id 2004) the heads are written, backward (id 2007)
+// read, with the opposite rotation.
+template <int V>
+__global__ void d_qkv_split_kernel(size_t pieces, double* rows, double* q, double* k, double* v, int T, int H, int hs, const double* fcos,
+                                   const double* fsin, int seq, bool backward, int parts)
 {
-    const int C = H * hs;
-    GRID_STRIDE(pi, pairs)
+    const int C = H * hs, N = parts * C;
+    GRID_STRIDE(pi, pieces)
     {
-        const size_t i = 2 * pi;
-        const size_t r = i / (3 * C);
-        const int c = (int)(i - r * 3 * C);
-        double o0 = tmp[i], o1 = tmp[i + 1];
-        if (bias) { o0 += bias[c]; o1 += bias[c + 1]; }
+        const size_t i = V * pi;
+        const size_t r = i / N;
+        const int c = (int)(i - r * N);
         const int which = c / C, w = c - which * C, h = w / hs, d = w - h * hs;
-        if (fcos && which < 2) {
+        double* head = (which == 0 ? q : which == 1 ? k : v) + (((r / T) * H + h) * T + r % T) * hs + d;
+        const double* src = backward ? head : rows + i;
+        double* dst = backward ? rows + i : head;
+        double o[2] = {src[0], V > 1 ? src[V - 1] : 0.0};
+        if (V > 1 && fcos && which < 2) {
             const size_t ti = (size_t)(r % seq) * (hs >> 1) + (d >> 1);
-            const double cs = fcos[ti], sn = fsin[ti], re = o0, im = o1;
-            o0 = re * cs - im * sn;
-            o1 = re * sn + im * cs;
+            const double cs = fcos[ti], sn = backward ? -fsin[ti] : fsin[ti], re = o[0], im = o[1];
+            o[0] = re * cs - im * sn;
+            o[1] = re * sn + im * cs;
         }
-        double* dst = (which == 0 ? q : which == 1 ? k : v) + (((r / T) * H + h) * T + r % T) * hs + d;
-        dst[0] = o0;
-        dst[1] = o1;
+        dst[0] = o[0];
+        if (V > 1) dst[V - 1] = o[1];
     }
 }
-__global__ void d_add_bias_rows_kernel(size_t n, int N, const double* bias, double* y) { GRID_STRIDE(i, n) y[i] += bias[i % N]; }
+static hipError_t d_qkv_split(hipStream_t s, long long M, int T, int H, int hs, double* rows, double* q, double* k, double* v, const double* fcos,
+                              const double* fsin, int seq, bool backward, int parts = 3)
+{
+    const size_t n = (size_t)M * parts * H * hs;
+    if (hs & 1) {
+        if (fcos) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(d_qkv_split_kernel<1>, grid_of(n), 256, 0, s, n, rows, q, k, v, T, H, hs, fcos, fsin, seq, backward, parts);
+    } else hipLaunchKernelGGL(d_qkv_split_kernel<2>, grid_of(n / 2), 256, 0, s, n / 2, rows, q, k, v, T, H, hs, fcos, fsin, seq, backward, parts);
+    return hipGetLastError();
+}
 
 // ---- the kernel object --------------------------------------------------------------------------------------------
 struct MemD {
@@ -1458,7 +1542,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         ERRCHK(mem((long)pl[2], &Y));
         RANGE(X, 0, ln->count);
         RANGE(Y, 0, ln->count);
-        hipLaunchKernelGGL(d_layernorm_fwd_kernel, ln->outer * ln->channels, 256, 0, s, ln->inner, (const double*)X->ptr, Y->ptr, ln->stdev, ln->eps);
+        hipLaunchKernelGGL(d_layernorm_fwd_kernel, ln->outer * ln->channels, 256, 0, s, ln->inner, (const double*)X->ptr, (const double*)nullptr, (double*)nullptr, Y->ptr, ln->stdev, ln->eps);
         LAUNCHED();
         ln->backwards = 0;
         return 0;
@@ -1477,8 +1561,114 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(dX, 0, ln->count);
         ln->backwards++;
         const int rows = ln->outer * ln->channels;
-        hipLaunchKernelGGL(d_layernorm_bwd_kernel, rows, 256, 0, s, rows, ln->inner, (const double*)Y->ptr, (const double*)dY->ptr, dX->ptr,
+        hipLaunchKernelGGL(d_layernorm_bwd_kernel, rows, 256, 0, s, rows, ln->inner, (const double*)Y->ptr, (const double*)dY->ptr, (const double*)nullptr, dX->ptr,
                            (const double*)ln->stdev, ln->eps * (double)ln->backwards);
+        LAUNCHED();
+        return 0;
+    }
+    case MCH_FN_NORM_ADD_FWD: {
+        // f{eps}, l{hLayerNorm (0 = RMS norm), rows, dim, hX, hAdd, hTotal, hWeight (0 = none), hY}
+        NEED_F(1, 1);
+        NEED_L(8, 8);
+        LayerNormD* ln = nullptr;
+        long long rows = pl[1], dim = pl[2];
+        if (pl[0]) {
+            ln = m_layernorm.get((long)pl[0]);
+            if (!ln || !ln->set) return MCH_ERROR_LAYERNORM_NOT_INITIALIZED;
+            rows = (long long)ln->outer * ln->channels;
+            dim = ln->inner;
+        }
+        if (rows < 0 || dim < 1 || rows > INT_MAX || dim > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        MemD *X, *Add, *Total, *W = nullptr, *Y;
+        ERRCHK(mem((long)pl[3], &X));
+        ERRCHK(mem((long)pl[4], &Add));
+        ERRCHK(mem((long)pl[5], &Total));
+        if (pl[6] && !ln) ERRCHK(mem((long)pl[6], &W));
+        ERRCHK(mem((long)pl[7], &Y));
+        RANGE(X, 0, rows * dim);
+        RANGE(Add, 0, rows * dim);
+        RANGE(Total, 0, rows * dim);
+        RANGE(Y, 0, rows * dim);
+        if (W) RANGE(W, 0, dim);
+        if (Total->ptr == Y->ptr) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        if (ln) {
+            hipLaunchKernelGGL(d_layernorm_fwd_kernel, (int)rows, 256, 0, s, (int)dim, (const double*)X->ptr, (const double*)Add->ptr, Total->ptr, Y->ptr, ln->stdev, ln->eps);
+            ln->backwards = 0;
+        } else if (rows)
+            hipLaunchKernelGGL(d_rmsnorm_kernel, (int)rows, 256, 0, s, (int)dim, (const double*)X->ptr, (const double*)Add->ptr, Total->ptr,
+                               W ? (const double*)W->ptr : nullptr, Y->ptr, pf[0]);
+        LAUNCHED();
+        return 0;
+    }
+    case MCH_FN_NORM_ADD_BWD: {
+        // l{hLayerNorm, hY, hdY, hdX, hAdd}
+        NEED_L(5, 5);
+        LayerNormD* ln = m_layernorm.get((long)pl[0]);
+        if (!ln || !ln->set) return MCH_ERROR_LAYERNORM_NOT_INITIALIZED;
+        MemD *Y, *dY, *dX, *Add;
+        ERRCHK(mem((long)pl[1], &Y));
+        ERRCHK(mem((long)pl[2], &dY));
+        ERRCHK(mem((long)pl[3], &dX));
+        ERRCHK(mem((long)pl[4], &Add));
+        RANGE(Y, 0, ln->count);
+        RANGE(dY, 0, ln->count);
+        RANGE(dX, 0, ln->count);
+        RANGE(Add, 0, ln->count);
+        ln->backwards++;
+        const int rows = ln->outer * ln->channels;
+        hipLaunchKernelGGL(d_layernorm_bwd_kernel, rows, 256, 0, s, rows, ln->inner, (const double*)Y->ptr, (const double*)dY->ptr, (const double*)Add->ptr,
+                           dX->ptr, (const double*)ln->stdev, ln->eps * (double)ln->backwards);
+        LAUNCHED();
+        return 0;
+    }
+    case MCH_FN_RMSNORM_BWD: {
+        // f{eps}, l{rows, dim, hX, hWeight (0 = none), hdY, hdX, hdWeight (0 = none), dwRows[, hAdd]}
+        NEED_F(1, 1);
+        NEED_L(8, 9);
+        const long long rows = pl[0], dim = pl[1], dwRows = pl[7];
+        if (rows < 0 || dim < 1 || rows > INT_MAX || dim > INT_MAX || dwRows < 0 || dwRows > rows) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        MemD *X, *W = nullptr, *dY, *dX, *dW = nullptr, *Add = nullptr;
+        ERRCHK(mem((long)pl[2], &X));
+        if (pl[3]) ERRCHK(mem((long)pl[3], &W));
+        ERRCHK(mem((long)pl[4], &dY));
+        ERRCHK(mem((long)pl[5], &dX));
+        if (pl[6]) ERRCHK(mem((long)pl[6], &dW));
+        if (ll > 8 && pl[8]) ERRCHK(mem((long)pl[8], &Add));
+        RANGE(X, 0, rows * dim);
+        RANGE(dY, 0, rows * dim);
+        RANGE(dX, 0, rows * dim);
+        if (W) RANGE(W, 0, dim);
+        if (dW) RANGE(dW, 0, dim);
+        if (Add) RANGE(Add, 0, rows * dim);
+        if (dW && (dX->ptr == X->ptr || dX->ptr == dY->ptr)) return MCH_ERROR_PARAM_OUT_OF_RANGE;   // the weight gradient reads both afterwards
+        if (rows == 0) return 0;
+        double* rinv = nullptr;
+        if (dW) ERRCHK(workspace((size_t)rows, &rinv));
+        hipLaunchKernelGGL(d_rmsnorm_bwd_kernel, (int)rows, 256, 0, s, (int)dim, (const double*)X->ptr, W ? (const double*)W->ptr : nullptr,
+                           (const double*)dY->ptr, Add ? (const double*)Add->ptr : nullptr, dX->ptr, rinv, pf[0]);
+        LAUNCHED();
+        if (dW) hipLaunchKernelGGL(d_rmsnorm_dw_kernel, (int)((dim + 15) / 16), 1024, 0, s, (int)dwRows, (int)dim, (const double*)X->ptr,
+                                   (const double*)dY->ptr, (const double*)rinv, dW->ptr);
+        LAUNCHED();
+        return 0;
+    }
+    case MCH_FN_SWIGLU_BWD: {
+        // l{n, hA, hB, hdY, hdA, hdB}
+        NEED_L(6, 6);
+        const long long n = pl[0];
+        MemD *A, *B, *dY, *dA, *dB;
+        ERRCHK(mem((long)pl[1], &A));
+        ERRCHK(mem((long)pl[2], &B));
+        ERRCHK(mem((long)pl[3], &dY));
+        ERRCHK(mem((long)pl[4], &dA));
+        ERRCHK(mem((long)pl[5], &dB));
+        RANGE(A, 0, n);
+        RANGE(B, 0, n);
+        RANGE(dY, 0, n);
+        RANGE(dA, 0, n);
+        RANGE(dB, 0, n);
+        if (n) hipLaunchKernelGGL(d_swiglu_bwd_kernel, grid_of((size_t)n), 256, 0, s, (size_t)n, (const double*)A->ptr, (const double*)B->ptr,
+                                  (const double*)dY->ptr, dA->ptr, dB->ptr);
         LAUNCHED();
         return 0;
     }
@@ -1495,7 +1685,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(X, 0, outer * dim);
         RANGE(Y, 0, outer * dim);
         if (W) RANGE(W, 0, dim);
-        if (outer) hipLaunchKernelGGL(d_rmsnorm_kernel, (int)outer, 256, 0, s, (int)dim, (const double*)X->ptr, W ? (const double*)W->ptr : nullptr, Y->ptr, pf[0]);
+        if (outer) hipLaunchKernelGGL(d_rmsnorm_kernel, (int)outer, 256, 0, s, (int)dim, (const double*)X->ptr, (const double*)nullptr, (double*)nullptr, W ? (const double*)W->ptr : nullptr, Y->ptr, pf[0]);
         LAUNCHED();
         return 0;
     }
@@ -1953,10 +2143,12 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         return 0;
     }
     case MCH_FN_LINEAR_FWD: {
-        // l{M, N, K, hX, hW, hBias(0 = none), hY}: Y = X W^T + bias
-        NEED_L(7, 7);
+        // l{M, N, K, hX, hW, hBias(0 = none), hY[, T, heads]}: Y = X W^T + bias, with T and heads as (M/T, heads, T, N/heads)
+        NEED_L(7, 9);
         const long long M = pl[0], N = pl[1], K = pl[2];
         if (M < 1 || N < 1 || K < 1 || M > INT_MAX || N > INT_MAX || K > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        const long long T = ll > 7 ? pl[7] : 0, heads = ll > 8 ? pl[8] : 0;
+        if (ll > 7 && (ll != 9 || T < 1 || heads < 1 || M % T || N % heads)) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         MemD *X, *W, *Bi = nullptr, *Y;
         ERRCHK(mem((long)pl[3], &X));
         ERRCHK(mem((long)pl[4], &W));
@@ -1966,12 +2158,37 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(W, 0, N * K);
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
-        HIPCHK(d_gemm(s, 1, (int)M, (int)N, (int)K, 1.0, (const double*)X->ptr, K, 1ll, (const double*)W->ptr, 1ll, K, 0.0, Y->ptr, N, 1ll, 0ll, 0ll, 0ll));
+        double* out = Y->ptr;
+        if (heads) ERRCHK(workspace((size_t)(M * N), &out));
+        HIPCHK(d_gemm(s, 1, (int)M, (int)N, (int)K, 1.0, (const double*)X->ptr, K, 1ll, (const double*)W->ptr, 1ll, K, 0.0, out, N, 1ll, 0ll, 0ll, 0ll,
+                      1, 0, Bi ? (const double*)Bi->ptr : nullptr));
+        if (heads) HIPCHK(d_qkv_split(s, M, (int)T, (int)heads, (int)(N / heads), out, Y->ptr, Y->ptr, Y->ptr, nullptr, nullptr, 1, false, 1));
+        return 0;
+    }
+    case MCH_FN_LINEAR_BWD: {
+        // l{M, N, K, hX, hW, hdY, hdW, hdBias(0 = none), hdX(0 = none)[, accumX]}
+        NEED_L(9, 10);
+        const long long M = pl[0], N = pl[1], K = pl[2];
+        const bool accum = ll > 9 && pl[9] != 0;
+        if (M < 1 || N < 1 || K < 1 || M > INT_MAX || N > INT_MAX || K > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        MemD *X, *W, *dY, *dW, *dB = nullptr, *dX = nullptr;
+        ERRCHK(mem((long)pl[3], &X));
+        ERRCHK(mem((long)pl[4], &W));
+        ERRCHK(mem((long)pl[5], &dY));
+        ERRCHK(mem((long)pl[6], &dW));
+        if (pl[7]) ERRCHK(mem((long)pl[7], &dB));
+        if (pl[8]) ERRCHK(mem((long)pl[8], &dX));
+        RANGE(X, 0, M * K);
+        RANGE(W, 0, N * K);
+        RANGE(dY, 0, M * N);
+        RANGE(dW, 0, N * K);
+        if (dB) RANGE(dB, 0, N);
+        if (dX) RANGE(dX, 0, M * K);
+        HIPCHK(d_gemm(s, 1, (int)N, (int)K, (int)M, 1.0, (const double*)dY->ptr, 1ll, N, (const double*)X->ptr, K, 1ll, 1.0, dW->ptr, K, 1ll, 0ll, 0ll, 0ll));
+        if (dB) hipLaunchKernelGGL(d_colsum_add_kernel, (int)((N + 15) / 16), 1024, 0, s, (int)M, (int)N, (const double*)dY->ptr, dB->ptr);
         LAUNCHED();
-        if (Bi) {
-            hipLaunchKernelGGL(d_add_bias_rows_kernel, grid_of((size_t)(M * N)), 256, 0, s, (size_t)(M * N), (int)N, (const double*)Bi->ptr, Y->ptr);
-            LAUNCHED();
-        }
+        if (dX) HIPCHK(d_gemm(s, 1, (int)M, (int)K, (int)N, 1.0, (const double*)dY->ptr, N, 1ll, (const double*)W->ptr, K, 1ll, accum ? 1.0 : 0.0, dX->ptr, K, 1ll,
+                              0ll, 0ll, 0ll));
         return 0;
     }
     case MCH_FN_QKV_PROJ_HEADS: {
@@ -2002,19 +2219,40 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
                 return MCH_ERROR_PARAM_OUT_OF_RANGE;
             }
         }
-        if (hs & 1) {
-            last_detail = "the double form of the fused QKV projection takes even head sizes";
-            return MCH_ERROR_PARAM_OUT_OF_RANGE;
-        }
         double* tmp;
         ERRCHK(workspace((size_t)(M * 3 * C), &tmp));
-        HIPCHK(d_gemm(s, 1, (int)M, (int)(3 * C), (int)C, 1.0, (const double*)X->ptr, C, 1ll, (const double*)W->ptr, 1ll, C, 0.0, tmp, 3 * C, 1ll, 0ll, 0ll, 0ll));
-        LAUNCHED();
-        const size_t pairs = (size_t)(M * 3 * C) / 2;
-        hipLaunchKernelGGL(d_qkv_split_kernel, grid_of(pairs), 256, 0, s, pairs, (const double*)tmp, Bi ? (const double*)Bi->ptr : nullptr,
-                           Q->ptr, K->ptr, V->ptr, (int)T, (int)H, (int)hs, r ? (const double*)r->dcos : nullptr,
-                           r ? (const double*)r->dsin : nullptr, r ? r->seq : 1);
-        LAUNCHED();
+        HIPCHK(d_gemm(s, 1, (int)M, (int)(3 * C), (int)C, 1.0, (const double*)X->ptr, C, 1ll, (const double*)W->ptr, 1ll, C, 0.0, tmp, 3 * C, 1ll, 0ll, 0ll, 0ll,
+                      1, 0, Bi ? (const double*)Bi->ptr : nullptr));
+        HIPCHK(d_qkv_split(s, M, (int)T, (int)H, (int)hs, tmp, Q->ptr, K->ptr, V->ptr, r ? (const double*)r->dcos : nullptr,
+                           r ? (const double*)r->dsin : nullptr, r ? r->seq : 1, false));
+        return 0;
+    }
+    case MCH_FN_QKV_HEADS_GRAD: {
+        // l{batch, T, heads, hs, hdQ, hdK, hdV, hdX[, hRope]}
+        NEED_L(8, 9);
+        const long long B = pl[0], T = pl[1], H = pl[2], hs = pl[3];
+        if (B < 1 || T < 1 || H < 1 || hs < 1 || B * T > INT_MAX || 3 * H * hs > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        const long long n = B * T * H * hs;
+        MemD *Q, *K, *V, *X;
+        ERRCHK(mem((long)pl[4], &Q));
+        ERRCHK(mem((long)pl[5], &K));
+        ERRCHK(mem((long)pl[6], &V));
+        ERRCHK(mem((long)pl[7], &X));
+        RANGE(Q, 0, n);
+        RANGE(K, 0, n);
+        RANGE(V, 0, n);
+        RANGE(X, 0, 3 * n);
+        RopeD* r = nullptr;
+        if (ll > 8 && pl[8]) {
+            r = m_rope.get((long)pl[8]);
+            if (!r || !r->set) return MCH_ERROR_ROPE_NOT_INITIALIZED;
+            if (r->heads != H || r->hs != hs) {
+                last_detail = "the rope handle was created for other heads or another head size";
+                return MCH_ERROR_PARAM_OUT_OF_RANGE;
+            }
+        }
+        HIPCHK(d_qkv_split(s, B * T, (int)T, (int)H, (int)hs, X->ptr, Q->ptr, K->ptr, V->ptr, r ? (const double*)r->dcos : nullptr,
+                           r ? (const double*)r->dsin : nullptr, r ? r->seq : 1, true));
         return 0;
     }
     case MCH_FN_ATTN_DECODE_FWD: {

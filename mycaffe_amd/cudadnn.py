@@ -116,6 +116,12 @@ class CUDAFN:
     SWIGLU_FWD = 2003
     QKV_PROJ_HEADS = 2004
     LINEAR_FWD = 2005
+    LINEAR_BWD = 2006
+    QKV_HEADS_GRAD = 2007
+    RMSNORM_BWD = 2008
+    SWIGLU_BWD = 2009
+    NORM_ADD_FWD = 2010
+    NORM_ADD_BWD = 2011
 
 
 class CUDAQRY:
@@ -722,10 +728,24 @@ class CudaDnn:
             rgl.append(hRope)
         self._ex2(CUDAFN.QKV_PROJ_HEADS, None, rgl)
 
-    def LinearForward(self, nM, nN, nK, hX, hWeight, hBias, hY):
+    def LinearForward(self, nM, nN, nK, hX, hWeight, hBias, hY, nT=0, nHeads=0):
         """y (M,N) = x (M,K) W^T (N,K) + bias in one GEMM (no counterpart in the reference: replaces the product and
-        the rank-1 bias update of InnerProductLayer.cs:372-417).  hBias 0: no bias."""
-        self._ex2(CUDAFN.LINEAR_FWD, None, [nM, nN, nK, hX, hWeight, hBias, hY])
+        the rank-1 bias update of InnerProductLayer.cs:372-417).  hBias 0: no bias.  With nT and nHeads y is written as
+        (M/T, heads, T, N/heads), which replaces the head transpose behind an attention layer's projection."""
+        rgl = [nM, nN, nK, hX, hWeight, hBias, hY]
+        if nHeads:
+            rgl += [nT, nHeads]
+        self._ex2(CUDAFN.LINEAR_FWD, None, rgl)
+
+    def LinearBackward(self, nM, nN, nK, hX, hWeight, hdY, hdWeight, hdBias, hdX, bAccumulate=False):
+        """dW += dy^T x, dbias += column sums of dy, dx = (+=) dy W (replaces the three calls of InnerProductLayer.cs:429-494).
+        hdBias, hdX 0: not computed."""
+        self._ex2(CUDAFN.LINEAR_BWD, None, [nM, nN, nK, hX, hWeight, hdY, hdWeight, hdBias, hdX, 1 if bAccumulate else 0])
+
+    def QkvHeadsGrad(self, nBatch, nT, nHeads, nSize, hdQ, hdK, hdV, hdX, hRope=0):
+        """Gradient of the fused projection's output, (B*T, 3C), from those of q, k, v as (B,H,T,hs) (replaces the transposes,
+        rotations and channel copies of CausalSelfAttentionLayer.cs:700-740)."""
+        self._ex2(CUDAFN.QKV_HEADS_GRAD, None, [nBatch, nT, nHeads, nSize, hdQ, hdK, hdV, hdX, hRope])
 
     def AttnScaledDotProductBackward(self, hCuDnn, hAttn, hQdata, hQdiff, hKdata, hKdiff, hVdata, hVdiff, hMaskdata, hYData, hYdiff):
         """CudaDnn.cs:5695-5701."""
@@ -759,9 +779,26 @@ class CudaDnn:
         """Fused RMSNorm (replaces the chain of RMSNormLayer.cs:156-180)."""
         self._ex2(CUDAFN.RMSNORM_FWD, [fEps], [nOuter, nDim, hX, hWeight, hY])
 
+    def RmsNormBackward(self, nRows, nDim, hX, hWeight, hdY, hdX, hdWeight, nWeightRows, fEps=1e-5, hAdd=0):
+        """Gradient of RMSNorm in one call (replaces the chain of RMSNormLayer.cs:189-232); dx gets hAdd's values added, dweight
+        the sums of the first nWeightRows rows."""
+        self._ex2(CUDAFN.RMSNORM_BWD, [fEps], [nRows, nDim, hX, hWeight, hdY, hdX, hdWeight, nWeightRows, hAdd])
+
+    def NormAddForward(self, hLayerNorm, nRows, nDim, hX, hAdd, hTotal, hWeight, hY, fEps=1e-5):
+        """total = x + add, y = norm(total): the layer norm handle's, or with hLayerNorm 0 RMSNorm over rows of nDim values."""
+        self._ex2(CUDAFN.NORM_ADD_FWD, [fEps], [hLayerNorm, nRows, nDim, hX, hAdd, hTotal, hWeight, hY])
+
+    def NormAddBackward(self, hLayerNorm, hYdata, hYdiff, hXdiff, hAdd):
+        """LayerNormBackward with hAdd's values added to the gradient."""
+        self._ex2(CUDAFN.NORM_ADD_BWD, None, [hLayerNorm, hYdata, hYdiff, hXdiff, hAdd])
+
     def SwigluForward(self, n, hA, hB, hY):
         """y = silu(a) * b in one pass."""
         self._ex2(CUDAFN.SWIGLU_FWD, None, [n, hA, hB, hY])
+
+    def SwigluBackward(self, n, hA, hB, hdY, hdA, hdB):
+        """Gradients of y = silu(a) * b in one pass."""
+        self._ex2(CUDAFN.SWIGLU_BWD, None, [n, hA, hB, hdY, hdA, hdB])
 
     # ---- RoPE ---------------------------------------------------------------------------------
     def CreateRope(self, nSharedIndex, nGpuID, nCount, nBatch, nSeqLen, nHeads, nDim, fTheta=10000.0):

@@ -1,9 +1,9 @@
 """Host-side mirrors of the MyCaffe layers that call the attention hot path.
 
-These follow the C# ``forward`` methods call for call (cited per class), so that a
-forward pass here issues the same sequence of ``CudaDnn`` calls, with the same
-argument packing, as the unchanged C# host would issue against the native library.
-Dropout layers are the identity (inference, or training with ratio 0).  ``Backward`` is mirrored for the GPT block
+These follow the C# ``forward`` and ``backward`` methods (cited per class).  Where this library has one call for several of
+the reference's - inner product with its bias, projection into heads, gradients of both, a norm with the residual next to it -
+the layers make the one call; the reference's own sequences run against the library from the C++ host program and the tests of
+the single ids.  Dropout layers are the identity (inference, or training with ratio 0).  ``Backward`` is mirrored for the GPT block
 (InnerProduct, Transpose, LayerNorm, activations, CausalSelfAttention with the fused attention handle, TransformerBlock).
 """
 import math
@@ -144,10 +144,9 @@ class InnerProductLayer:
 
     def __init__(self, cuda, num_output, bias_term=True, axis=2, half=False, fused_bias=False):
         self.cuda, self.N, self.bias_term, self.axis, self.half = cuda, num_output, bias_term, axis, half
-        # product and bias in one call (an id with no counterpart in the reference) instead of the two GEMM calls
+        # a single row goes through gemv and axpy (:385-392) unless fused_bias asks for the one call there too
         self.fused_bias = fused_bias
         self.blobs = []
-        self.bias_multiplier = None
 
     def Setup(self, bottom, weight=None, bias=None):
         self.K = bottom.count(self.axis)
@@ -165,35 +164,25 @@ class InnerProductLayer:
         M = bottom.count(0, self.axis)
         top.Reshape(*(bottom.shape_[:self.axis] + [self.N]))
         hW = self.blobs[0].gpu_data
-        if self.fused_bias:
-            self.cuda.LinearForward(M, self.N, self.K, bottom.gpu_data, hW, self.blobs[1].gpu_data if self.bias_term else 0,
-                                    top.gpu_data)
-        elif M == 1 and not self.half:
+        if M == 1 and not self.half and not self.fused_bias:
             self.cuda.gemv(False, self.N, self.K, 1.0, hW, bottom.gpu_data, 0.0, top.gpu_data)
             if self.bias_term:
                 self.cuda.axpy(self.N, 1.0, self.blobs[1].gpu_data, top.gpu_data)
         else:
-            self.cuda.gemm(False, True, M, self.N, self.K, 1.0, bottom.gpu_data, hW, 0.0, top.gpu_data)
-            if self.bias_term:
-                if self.bias_multiplier is None or self.bias_multiplier.count() < M:
-                    self.bias_multiplier = Blob(self.cuda, (M,), self.half)
-                    self.bias_multiplier.SetData(1.0)
-                self.cuda.gemm(False, False, M, self.N, 1, 1.0, self.bias_multiplier.gpu_data, self.blobs[1].gpu_data, 1.0,
-                               top.gpu_data)
+            self.cuda.LinearForward(M, self.N, self.K, bottom.gpu_data, hW, self.blobs[1].gpu_data if self.bias_term else 0, top.gpu_data)
 
+    def ForwardHeads(self, bottom, top, heads):
+        """Forward with the result written head by head, (B,T,K) -> (B, heads, T, N/heads)."""
+        B, T = bottom.shape_[:2]
+        top.Reshape(B, heads, T, self.N // heads)
+        self.cuda.LinearForward(B * T, self.N, self.K, bottom.gpu_data, self.blobs[0].gpu_data, self.blobs[1].gpu_data if self.bias_term else 0,
+                                top.gpu_data, T, heads)
 
-    def Backward(self, top, bottom):
-        """InnerProductLayer.cs:429-494: weight gradient accumulates into the weight diff, bias gradient through gemv with
-        the ones vector, data gradient = top diff x W."""
-        M = bottom.count(0, self.axis)
-        hTopDiff, hW = top.gpu_diff, self.blobs[0].gpu_data
-        self.cuda.gemm(True, False, self.N, self.K, M, 1.0, hTopDiff, bottom.gpu_data, 1.0, self.blobs[0].gpu_diff)
-        if self.bias_term:
-            if self.bias_multiplier is None or self.bias_multiplier.count() < M:
-                self.bias_multiplier = Blob(self.cuda, (M,), self.half)
-                self.bias_multiplier.SetData(1.0)
-            self.cuda.gemv(True, M, self.N, 1.0, hTopDiff, self.bias_multiplier.gpu_data, 1.0, self.blobs[1].gpu_diff)
-        self.cuda.gemm(False, False, M, self.K, self.N, 1.0, hTopDiff, hW, 0.0, bottom.gpu_diff)
+    def Backward(self, top, bottom, accumulate=False):
+        """InnerProductLayer.cs:429-494: weight and bias gradients accumulate into their diffs, data gradient = top diff x W
+        (``accumulate``: added to what the bottom's diff holds)."""
+        self.cuda.LinearBackward(bottom.count(0, self.axis), self.N, self.K, bottom.gpu_data, self.blobs[0].gpu_data, top.gpu_diff,
+                                 self.blobs[0].gpu_diff, self.blobs[1].gpu_diff if self.bias_term else 0, bottom.gpu_diff, accumulate)
 
 
 class TransposeLayer:
@@ -330,10 +319,7 @@ class CausalSelfAttentionLayer:
                  enable_rotary_positional_embedding=False, rope_theta=10000.0, half=False, training=False,
                  fused_qkv_heads=False):
         self.training = training
-        # three calls per forward instead of seventeen (ids with no counterpart in the reference): the fused QKV
-        # projection writes q, k, v as (B,H,T,hs), rotated where the layer has a rotary embedding, the attention
-        # handle writes its output head-merged and the output projection adds its bias in the GEMM's epilogue.
-        # Inference, fused attention handle.
+        # inference with the fused attention handle as three calls: the handle writes its output head-merged
         self.fused_qkv_heads = fused_qkv_heads
         self.cuda, self.nHeads, self.nEmbed, self.nBlockSize = cuda, heads, embed, block_size
         self.nSize = embed // heads
@@ -346,7 +332,7 @@ class CausalSelfAttentionLayer:
         self.transpose = TransposeLayer(cuda, (0, 2, 1, 3))
         self.transposeQ = TransposeLayer(cuda, (0, 1, 3, 2))
         self.softmax = SoftmaxLayer(cuda, -1)
-        names = "IpAttn Q K V Qt Kt Vt Kt1 AttA AttB Work Y".split()
+        names = "IpAttn Qt Kt Vt Kt1 AttA AttB Work Y".split()
         self.b = {n: Blob(cuda, half=half) for n in names}
         self.blobMask = Blob(cuda, (1, 1, block_size, block_size))
         mask = np.tril(np.ones((block_size, block_size), np.float32))  # fillMask :276-291
@@ -384,44 +370,22 @@ class CausalSelfAttentionLayer:
             raise ValueError("sequence longer than block_size")
         self._reshape(B, T)
         b, cuda, H, hs = self.b, self.cuda, self.nHeads, self.nSize
-        if self.fused_qkv_heads:
-            if not self.enable_sdpa or self.training:
-                raise ValueError("fused_qkv_heads needs the fused attention handle, inference mode")
-            for name in ("Qt", "Kt", "Vt"):
-                b[name].Reshape(B, H, T, hs)
-            ip = self.c_attn
-            cuda.QkvProjHeads(B, T, H, hs, blobX.gpu_data, ip.blobs[0].gpu_data, ip.blobs[1].gpu_data if ip.bias_term else 0,
-                              b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data, self.hRope)
-            mask = self.blobMask
-            if T != self.nBlockSize:
-                if getattr(self, "_sdpa_mask_T", None) != T:
-                    self.blobMaskSdpa = Blob(cuda, (1, 1, T, T))
-                    self.blobMaskSdpa.mutable_cpu_data = np.tril(np.ones((T, T), np.float32))
-                    self._sdpa_mask_T = T
-                mask = self.blobMaskSdpa
-            b["Y"].Reshape(B, T, C)
-            cuda.AttnScaledDotProductForward(self.hCudnn, self.hAttn, T, b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data,
-                                             mask.gpu_data, b["Y"].gpu_data, False, T, True)
-            self.c_proj.Forward(b["Y"], top)
-            return
-        # q, k, v = self.c_attn(x).split(self.n_embd, dim=2)
-        self.c_attn.Forward(blobX, b["IpAttn"])
-        for name in "QKV":
-            b[name].Reshape(B, T, H, hs)
-        nCount = b["Q"].count()
-        ip = b["IpAttn"]
-        cuda.channel_copy(nCount, ip.num, ip.channels, 3, self.nEmbed, 0, ip.gpu_data, b["Q"].gpu_data, DIR.FWD)
-        cuda.channel_copy(nCount, ip.num, ip.channels, 3, self.nEmbed, 1, ip.gpu_data, b["K"].gpu_data, DIR.FWD)
-        cuda.channel_copy(nCount, ip.num, ip.channels, 3, self.nEmbed, 2, ip.gpu_data, b["V"].gpu_data, DIR.FWD)
-        if self.hRope:
-            cuda.RopeForward(self.hRope, b["Q"].count(), b["Q"].gpu_data, b["Q"].gpu_data)
-            cuda.RopeForward(self.hRope, b["K"].count(), b["K"].gpu_data, b["K"].gpu_data)
-        # (B, T, nh, hs) -> (B, nh, T, hs)
-        self.transpose.Forward(b["Q"], b["Qt"])
-        self.transpose.Forward(b["K"], b["Kt"])
-        self.transpose.Forward(b["V"], b["Vt"])
+        if self.fused_qkv_heads and (not self.enable_sdpa or self.training):
+            raise ValueError("fused_qkv_heads needs the fused attention handle, inference mode")
+        # q, k, v = self.c_attn(x).split(self.n_embd, dim=2), rotated, (B, T, nh, hs) -> (B, nh, T, hs): one call for the
+        # projection, its bias, three channel copies, two rotations and three transposes (:526-557)
+        for name in ("Qt", "Kt", "Vt"):
+            b[name].Reshape(B, H, T, hs)
+        w = self.c_attn.blobs
+        cuda.QkvProjHeads(B, T, H, hs, blobX.gpu_data, w[0].gpu_data, w[1].gpu_data if self.bias_term else 0, b["Qt"].gpu_data, b["Kt"].gpu_data,
+                          b["Vt"].gpu_data, self.hRope)
         if self.enable_sdpa:
-            b["Work"].ReshapeLike(b["Vt"])
+            out = b["Work"]
+            if self.fused_qkv_heads:
+                out = b["Y"]
+                out.Reshape(B, T, C)
+            else:
+                out.ReshapeLike(b["Vt"])
             mask = self.blobMask
             if T != self.nBlockSize:
                 # the handle reads a (1,1,T,T) mask for the block size it is run with
@@ -430,8 +394,13 @@ class CausalSelfAttentionLayer:
                     self.blobMaskSdpa.mutable_cpu_data = np.tril(np.ones((T, T), np.float32))
                     self._sdpa_mask_T = T
                 mask = self.blobMaskSdpa
+            if self.fused_qkv_heads:
+                cuda.AttnScaledDotProductForward(self.hCudnn, self.hAttn, T, b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data,
+                                                 mask.gpu_data, out.gpu_data, False, T, True)
+                self.c_proj.Forward(out, top)
+                return
             cuda.AttnScaledDotProductForward(self.hCudnn, self.hAttn, T, b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data,
-                                             mask.gpu_data, b["Work"].gpu_data, False)
+                                             mask.gpu_data, out.gpu_data, False)
         else:
             self.transposeQ.Forward(b["Kt"], b["Kt1"])
             dfScale = 1.0 / math.sqrt(hs)
@@ -443,7 +412,6 @@ class CausalSelfAttentionLayer:
             b["Work"].MatMul(b["AttB"], b["Vt"], bReshape=True)
         # y.transpose(1, 2).contiguous().view(B, T, C)
         self.transpose.Forward(b["Work"], b["Y"])
-        self._y_shape = list(b["Y"].shape_)
         b["Y"].Reshape(B, T, C)
         self.c_proj.Forward(b["Y"], top)
 
@@ -453,31 +421,24 @@ class CausalSelfAttentionLayer:
         two MatMulGrad calls around the softmax gradient (no dropout)."""
         b, cuda = self.b, self.cuda
         B, T, C = blobX.shape_[:3]
+        H, hs = self.nHeads, self.nSize
         self.c_proj.Backward(top, b["Y"])
-        b["Y"].Reshape(*self._y_shape)
+        b["Y"].Reshape(B, T, H, hs)
         self.transpose.Backward(b["Y"], b["Work"])
-        b["Y"].CopyFrom(b["Work"], True, True)
+        b["Y"].Reshape(B, T, C)
         if self.enable_sdpa:
             cuda.AttnScaledDotProductBackward(self.hCudnn, self.hAttn, b["Qt"].gpu_data, b["Qt"].gpu_diff, b["Kt"].gpu_data,
-                                              b["Kt"].gpu_diff, b["Vt"].gpu_data, b["Vt"].gpu_diff, 0, b["Y"].gpu_data, b["Y"].gpu_diff)
+                                              b["Kt"].gpu_diff, b["Vt"].gpu_data, b["Vt"].gpu_diff, 0, b["Work"].gpu_data, b["Work"].gpu_diff)
         else:
             # att' = y' @ v^T, vt' = att^T @ y'; softmax gradient; qt' = att' @ kt, kt1' = qt^T @ att' (scaled)
-            b["Y"].MatMulGrad(b["AttB"], b["Vt"])
+            b["Work"].MatMulGrad(b["AttB"], b["Vt"])
             self.softmax.Backward(b["AttB"], b["AttA"])
-            b["AttA"].MatMulGrad(b["Qt"], b["Kt1"], 1.0 / math.sqrt(self.nSize))
+            b["AttA"].MatMulGrad(b["Qt"], b["Kt1"], 1.0 / math.sqrt(hs))
             self.transposeQ.Backward(b["Kt1"], b["Kt"])
-        self.transpose.Backward(b["Kt"], b["K"])
-        self.transpose.Backward(b["Qt"], b["Q"])
-        self.transpose.Backward(b["Vt"], b["V"])
-        if self.hRope:
-            cuda.RopeBackward(self.hRope, b["Q"].count(), b["Q"].gpu_data, b["Q"].gpu_diff, b["Q"].gpu_diff)
-            cuda.RopeBackward(self.hRope, b["K"].count(), b["K"].gpu_data, b["K"].gpu_diff, b["K"].gpu_diff)
-        nCount = b["Q"].count()
+        # three transposes, two rotations and three channel copies (:700-740)
         ip = b["IpAttn"]
-        cuda.channel_copy(nCount, ip.num, ip.channels, 3, self.nEmbed, 0, ip.gpu_diff, b["Q"].gpu_diff, DIR.BWD)
-        cuda.channel_copy(nCount, ip.num, ip.channels, 3, self.nEmbed, 1, ip.gpu_diff, b["K"].gpu_diff, DIR.BWD)
-        cuda.channel_copy(nCount, ip.num, ip.channels, 3, self.nEmbed, 2, ip.gpu_diff, b["V"].gpu_diff, DIR.BWD)
-        b["Y"].Reshape(B, T, C)
+        ip.Reshape(B, T, 3 * C)
+        cuda.QkvHeadsGrad(B, T, H, hs, b["Qt"].gpu_diff, b["Kt"].gpu_diff, b["Vt"].gpu_diff, ip.gpu_diff, self.hRope)
         self.c_attn.Backward(ip, blobX)
 
 
@@ -511,7 +472,7 @@ class MultiheadAttentionLayer:
         self.transposeK = TransposeLayer(cuda, (0, 2, 1, 3))
         self.transposeQ = TransposeLayer(cuda, (0, 1, 3, 2))
         self.softmax = SoftmaxLayer(cuda, -1)
-        self.b = {n: Blob(cuda, half=half) for n in "Q K V Qt Kt Vt Kt1 AttA AttB Work Y KeyCache ValCache Work2 Work3".split()}
+        self.b = {n: Blob(cuda, half=half) for n in "Q K Qt Kt Vt Kt1 AttA AttB Work Y KeyCache ValCache Work2 Work3".split()}
         self.hCudnn = self.hAttn = self.hRope = 0
         self._set_for = None
         self.options = {}
@@ -531,21 +492,24 @@ class MultiheadAttentionLayer:
         B, Tq, C = q.shape_[:3]
         Tk = k.shape_[1]
         nPos = int(self.options.get("position", -1))
-        self.c_attnQ.Forward(q, b["Q"])
-        self.c_attnK.Forward(k, b["K"])
-        self.c_attnV.Forward(v, b["V"])
-        b["Q"].Reshape(B, Tq, H, hs)
-        b["K"].Reshape(B, Tk, H, hs)
-        b["V"].Reshape(B, Tk, H, hs)
         if self.enable_rope:
+            self.c_attnQ.Forward(q, b["Q"])
+            self.c_attnK.Forward(k, b["K"])
+            self.c_attnV.ForwardHeads(v, b["Vt"], H)
+            b["Q"].Reshape(B, Tq, H, hs)
+            b["K"].Reshape(B, Tk, H, hs)
             if not self.hRope:
                 self.hRope = cuda.CreateRope(0, 0, B * self.nBlockSize * C, B, self.nBlockSize, H, hs, self.rope_theta)
             nFreqOffset = nPos * hs // 2 if nPos > 0 else -1
             cuda.RopeForward(self.hRope, b["Q"].count(), b["Q"].gpu_data, b["Q"].gpu_data, nFreqOffset)
             cuda.RopeForward(self.hRope, b["K"].count(), b["K"].gpu_data, b["K"].gpu_data, nFreqOffset)
-        self.transpose.Forward(b["Q"], b["Qt"])
-        self.transposeK.Forward(b["K"], b["Kt"])
-        self.transposeK.Forward(b["V"], b["Vt"])
+            self.transpose.Forward(b["Q"], b["Qt"])
+            self.transposeK.Forward(b["K"], b["Kt"])
+        else:
+            # projections written head by head: no transposes behind them
+            self.c_attnQ.ForwardHeads(q, b["Qt"], H)
+            self.c_attnK.ForwardHeads(k, b["Kt"], H)
+            self.c_attnV.ForwardHeads(v, b["Vt"], H)
         is_qk_mask = (blobMask is not None and blobMask.num_axes == 4 and blobMask.num == 1 and blobMask.channels == 1
                       and blobMask.height == Tq and blobMask.width == Tk)
         full_mask = blobMask is not None and not is_qk_mask and blobMask.count() == B * Tq * Tk and Tq > 1
@@ -556,10 +520,12 @@ class MultiheadAttentionLayer:
                     self.hAttn = cuda.CreateAttn()
                 cuda.SetAttn(self.hCudnn, self.hAttn, 0, False, B, self.nBlockSize, H, hs, 0.0)
                 self._set_for = B
-            b["Work"].ReshapeLike(b["Qt"])
+            b["Y"].Reshape(B, Tq, C)
             cuda.AttnScaledDotProductForward(self.hCudnn, self.hAttn, Tq, b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data,
-                                             blobMask.gpu_data if blobMask is not None else 0, b["Work"].gpu_data,
-                                             2 if full_mask else (not is_qk_mask), Tk if Tk != Tq else None)
+                                             blobMask.gpu_data if blobMask is not None else 0, b["Y"].gpu_data,
+                                             2 if full_mask else (not is_qk_mask), Tk, True)
+            self.c_proj.Forward(b["Y"], top)
+            return
         else:
             # the fused handle only understands (1,1,T,T) or (B,T) masks (attn.cu:544-556); a
             # (B,T_q,T_k) mask goes through the explicit chain (MultiheadAttentionLayer.cs:733-742)
@@ -660,6 +626,23 @@ class LayerNormLayer:
         cuda.channel_fillfrom(n, o, c, i, b["Stdev"].gpu_data, b["StdevFull"].gpu_data, DIR.FWD)
         cuda.div(n, b["Xmu"].gpu_data, b["StdevFull"].gpu_data, top.gpu_data)
 
+    def ForwardAdd(self, x, add, total, top):
+        """total = x + add, top = norm(total)."""
+        total.ReshapeLike(x)
+        if not self.enable_cuda_impl:
+            self.cuda.add(x.count(), x.gpu_data, add.gpu_data, total.gpu_data)
+            return self.Forward(total, top)
+        self._reshape(x)
+        top.ReshapeLike(x)
+        self.cuda.NormAddForward(self.hLayerNorm, 0, 0, x.gpu_data, add.gpu_data, total.gpu_data, 0, top.gpu_data)
+
+    def BackwardAdd(self, top, bottom, hAdd):
+        """Backward with the values behind hAdd added to the bottom's diff."""
+        if not self.enable_cuda_impl:
+            self.Backward(top, bottom)
+            return self.cuda.add(bottom.count(), hAdd, bottom.gpu_diff, bottom.gpu_diff)
+        self.cuda.NormAddBackward(self.hLayerNorm, top.gpu_data, top.gpu_diff, bottom.gpu_diff, hAdd)
+
     def Backward(self, top, bottom):
         if self.enable_cuda_impl:
             self.cuda.LayerNormBackward(self.hLayerNorm, top.gpu_data, top.gpu_diff, bottom.gpu_diff)
@@ -682,8 +665,8 @@ class LayerNormLayer:
 
 class RMSNormLayer:
     """MyCaffe.layers.gpt/layers.gpt/RMSNormLayer.cs:96-180, the layer's own chain: powx(2), channel_mean, sqrt(+eps),
-    invert, channel_duplicate, mul, and with weights channel_copyall + mul.  ``fused`` replaces the chain by the
-    single call RMSNORM_FWD (id 2002), which has no counterpart in the reference."""
+    invert, channel_duplicate, mul, and with weights channel_copyall + mul.  ``fused`` replaces the chains by the
+    single calls RMSNORM_FWD and RMSNORM_BWD (ids 2002, 2008), which have no counterpart in the reference."""
 
     def __init__(self, cuda, epsilon=1e-5, enable_weights=True, fused=False):
         self.cuda, self.epsilon, self.enable_weights, self.fused = cuda, epsilon, enable_weights, fused
@@ -724,13 +707,35 @@ class RMSNormLayer:
             top.CopyFrom(b["Out"])
         self._dims = (n, outer, channels, inner)
 
-    def Backward(self, top, bottom, freeze_learning=False):
+    def ForwardAdd(self, x, add, total, top):
+        """total = x + add, top = norm(total)."""
+        total.ReshapeLike(x)
+        if not self.fused:
+            self.cuda.add(x.count(), x.gpu_data, add.gpu_data, total.gpu_data)
+            return self.Forward(total, top)
+        nAxis = len(x.shape_) - 1
+        top.ReshapeLike(x)
+        self.cuda.NormAddForward(0, x.count(0, nAxis), x.count(nAxis), x.gpu_data, add.gpu_data, total.gpu_data,
+                                 self.blobs[0].gpu_data if self.enable_weights else 0, top.gpu_data, self.epsilon)
+
+    def BackwardAdd(self, top, bottom, hAdd):
+        """Backward with the values behind hAdd added to the bottom's diff."""
+        if self.fused:
+            return self.Backward(top, bottom, hAdd=hAdd)
+        self.Backward(top, bottom)
+        self.cuda.add(bottom.count(), hAdd, bottom.gpu_diff, bottom.gpu_diff)
+
+    def Backward(self, top, bottom, freeze_learning=False, hAdd=0):
         """RMSNormLayer.cs:189-232, the layer's own chain (after a Forward through the chain): top.diff -> bottom.diff and,
         with weights, the weight gradient through channel_sum (which, as there, keeps the sums of the first batch
         entry: the call passes outer = batch and a gradient blob of `inner` values)."""
-        if self.fused:
-            raise NotImplementedError("the fused forward call keeps none of the chain's intermediates")
         cuda, b = self.cuda, self.b
+        if self.fused:
+            nAxis = len(bottom.shape_) - 1
+            hW, hdW = (self.blobs[0].gpu_data, 0 if freeze_learning else self.blobs[0].gpu_diff) if self.enable_weights else (0, 0)
+            cuda.RmsNormBackward(bottom.count(0, nAxis), bottom.count(nAxis), bottom.gpu_data, hW, top.gpu_diff, bottom.gpu_diff, hdW,
+                                 bottom.shape_[nAxis - 1], self.epsilon, hAdd)
+            return
         n, outer, channels, inner = self._dims
         if self.enable_weights:
             if not freeze_learning:
@@ -813,8 +818,9 @@ class TransformerBlockLayer:
         self.llama = enable_llama_style_head
         if self.llama:
             # RMSNorm, rotary attention without bias, SiLU-gated MLP (TransformerBlockLayer.cs:86-98, 239-247, 860-875)
-            self.norm1 = RMSNormLayer(cuda, epsilon, True, fused_rmsnorm)
-            self.norm2 = RMSNormLayer(cuda, epsilon, True, fused_rmsnorm)
+            # (the norms of a block are always the single calls; the argument stays for its callers)
+            self.norm1 = RMSNormLayer(cuda, epsilon, True, True)
+            self.norm2 = RMSNormLayer(cuda, epsilon, True, True)
             if hidden_dim == 0:
                 hidden_dim = 2 * (4 * embed) // 3
                 hidden_dim = multiple_of * ((hidden_dim + multiple_of - 1) // multiple_of)
@@ -833,7 +839,7 @@ class TransformerBlockLayer:
         self.fc2 = InnerProductLayer(cuda, hidden_dim, bias_term, 2) if self.llama else None
         self.proj = InnerProductLayer(cuda, embed, bias_term, 2)
         self.act = ActivationLayer(cuda, activation)
-        self.b = {n: Blob(cuda) for n in "Norm1 Attn1 X Norm2 NormA Mlp1 Mlp2 Mlp3 MlpOut".split()}
+        self.b = {n: Blob(cuda) for n in "Norm1 Attn1 X Norm2 Mlp1 Mlp2 Mlp3 MlpOut".split()}
 
     def Setup(self, bottom, p):
         """``p``: attn_weight, attn_bias, attn_proj_weight, attn_proj_bias (ENCODER type: wq, bq, wk, bk, wv, bv, wo, bo),
@@ -864,47 +870,47 @@ class TransformerBlockLayer:
             self.attn1.Forward(b["Norm1"], b["Norm1"], b["Norm1"], blobXMask, b["Attn1"])
         else:
             self.attn1.Forward(b["Norm1"], b["Attn1"])
-        b["X"].ReshapeLike(blobX)
-        cuda.add(nCount, blobX.gpu_data, b["Attn1"].gpu_data, b["X"].gpu_data)
-        self.norm2.Forward(b["X"], b["Norm2"])
-        self.fc1.Forward(b["Norm2"], b["Mlp1"])
-        self.act.Forward(b["Mlp1"], b["Mlp1"])
+        self.norm2.ForwardAdd(blobX, b["Attn1"], b["X"], b["Norm2"])
+        # the activation runs in place; those that need their input again get it in a blob of their own instead of a copy of it
+        blobPre = b["Mlp1"] if self.act.kind == "relu" else self.act.blobX
+        self.fc1.Forward(b["Norm2"], blobPre)
         blobMlp = b["Mlp1"]
         if self.llama:
-            self.fc2.Forward(b["Norm2"], b["Mlp2"])
-            b["Mlp3"].ReshapeLike(b["Mlp1"])
-            cuda.mul(b["Mlp1"].count(), b["Mlp1"].gpu_data, b["Mlp2"].gpu_data, b["Mlp3"].gpu_data)
             blobMlp = b["Mlp3"]
+            self.fc2.Forward(b["Norm2"], b["Mlp2"])
+            b["Mlp1"].ReshapeLike(blobPre)
+            blobMlp.ReshapeLike(blobPre)
+            if self.act.kind == "silu":
+                cuda.SwigluForward(blobPre.count(), blobPre.gpu_data, b["Mlp2"].gpu_data, blobMlp.gpu_data)
+            else:
+                self.act.Forward(blobPre, b["Mlp1"])
+                cuda.mul(blobMlp.count(), b["Mlp1"].gpu_data, b["Mlp2"].gpu_data, blobMlp.gpu_data)
+        else:
+            self.act.Forward(blobPre, blobMlp)
         self.proj.Forward(blobMlp, b["MlpOut"])
         top.ReshapeLike(blobX)
         cuda.add(nCount, b["X"].gpu_data, b["MlpOut"].gpu_data, top.gpu_data)
 
     def Backward(self, top, blobX):
-        """TransformerBlockLayer.cs:924-1040, CAUSAL_SELF_ATTENTION block: top.gpu_diff -> blobX.gpu_diff."""
+        """TransformerBlockLayer.cs:924-1040, CAUSAL_SELF_ATTENTION block: top.gpu_diff -> blobX.gpu_diff.  The gradients of the
+        two residuals are read where they are and added by the norms' calls."""
         if self.block_type != "causal_self_attention":
             raise NotImplementedError("backward is mirrored for the CAUSAL_SELF_ATTENTION block type")
         b, cuda = self.b, self.cuda
-        nCount = blobX.count()
-        cuda.copy(nCount, top.gpu_diff, b["MlpOut"].gpu_diff)
-        cuda.copy(nCount, top.gpu_diff, b["X"].gpu_diff)
-        self.proj.Backward(b["MlpOut"], b["Mlp3"] if self.llama else b["Mlp1"])
+        self.proj.Backward(top, b["Mlp3"] if self.llama else b["Mlp1"])
         if self.llama:
-            # gate: Mlp3 = silu(fc1) * fc2; the gradient through fc2 waits in NormA's data until fc1's has arrived
+            # gate: Mlp3 = act(fc1) * fc2
             n1 = b["Mlp1"].count()
-            cuda.mul(n1, b["Mlp3"].gpu_diff, b["Mlp2"].gpu_data, b["Mlp1"].gpu_diff)
-            cuda.mul(n1, b["Mlp3"].gpu_diff, b["Mlp1"].gpu_data, b["Mlp2"].gpu_diff)
+            if self.act.kind == "silu":
+                cuda.SwigluBackward(n1, self.act.blobX.gpu_data, b["Mlp2"].gpu_data, b["Mlp3"].gpu_diff, b["Mlp1"].gpu_diff, b["Mlp2"].gpu_diff)
+            else:
+                cuda.mul(n1, b["Mlp3"].gpu_diff, b["Mlp2"].gpu_data, b["Mlp1"].gpu_diff)
+                cuda.mul(n1, b["Mlp3"].gpu_diff, b["Mlp1"].gpu_data, b["Mlp2"].gpu_diff)
+                self.act.Backward(b["Mlp1"], b["Mlp1"])
             self.fc2.Backward(b["Mlp2"], b["Norm2"])
-            b["NormA"].ReshapeLike(b["Norm2"])
-            cuda.copy(b["Norm2"].count(), b["Norm2"].gpu_diff, b["NormA"].gpu_data)
-        self.act.Backward(b["Mlp1"], b["Mlp1"])
-        self.fc1.Backward(b["Mlp1"], b["Norm2"])
-        if self.llama:
-            cuda.add(b["Norm2"].count(), b["NormA"].gpu_data, b["Norm2"].gpu_diff, b["Norm2"].gpu_diff)
-        # x_2 = ln_2(xB): keep xB's own gradient aside, add the one that comes through the norm
-        b["Attn1"].CopyFrom(b["X"], True)
-        self.norm2.Backward(b["Norm2"], b["X"])
-        cuda.add(nCount, b["Attn1"].gpu_diff, b["X"].gpu_diff, b["X"].gpu_diff)
-        b["Attn1"].CopyFrom(b["X"], True)
-        self.attn1.Backward(b["Attn1"], b["Norm1"])
-        self.norm1.Backward(b["Norm1"], blobX)
-        cuda.add(nCount, b["X"].gpu_diff, blobX.gpu_diff, blobX.gpu_diff)
+        else:
+            self.act.Backward(b["Mlp1"], b["Mlp1"])
+        self.fc1.Backward(b["Mlp1"], b["Norm2"], self.llama)
+        self.norm2.BackwardAdd(b["Norm2"], b["X"], top.gpu_diff)
+        self.attn1.Backward(b["X"], b["Norm1"])
+        self.norm1.BackwardAdd(b["Norm1"], blobX, b["X"].gpu_diff)
