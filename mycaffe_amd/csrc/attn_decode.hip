@@ -9,6 +9,9 @@
 // so one wavefront load instruction fetches 64/LPR consecutive rows, and four
 // such loads per operand are kept in flight.  Each lane group keeps its own
 // running max / sum / output slice; groups are merged through LDS at the end.
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.h"
 #include "lane_ops.h"
 
@@ -198,28 +201,51 @@ __device__ __forceinline__ void decode_stream(const T* __restrict__ kc, const T*
 __device__ __forceinline__ void part_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float part_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Merges the 4 * (64/LPR) lane groups of a workgroup through LDS and writes {M, L, acc[hs]} to `out`, or, when
+// maximum or sum over the lane groups of LPR lanes of a wavefront, in every lane
+template <int LPR, bool MAX> __device__ __forceinline__ float across_groups(float v)
+{
+    auto step = [&](auto o) { v = MAX ? max_lane_xor<decltype(o)::value>(v) : add_lane_xor<decltype(o)::value>(v); };
+    if constexpr (LPR <= 1) step(std::integral_constant<int, 1>{});
+    if constexpr (LPR <= 2) step(std::integral_constant<int, 2>{});
+    if constexpr (LPR <= 4) step(std::integral_constant<int, 4>{});
+    if constexpr (LPR <= 8) step(std::integral_constant<int, 8>{});
+    if constexpr (LPR <= 16) step(std::integral_constant<int, 16>{});
+    if constexpr (LPR <= 32) step(std::integral_constant<int, 32>{});
+    return v;
+}
+
+// Merges the NW * (64/LPR) lane groups of a workgroup through LDS and writes {M, L, acc[hs]} to `out`, or, when
 // this workgroup saw every cached row (yfinal set), the normalised result straight to yfinal.  With plainAcc set the
 // partial is meant for the NEXT kernel of the stream, which merges the splits itself: {M, L} go to `out` and acc[hs] to
 // plainAcc with ordinary stores (the kernel boundary makes them visible).
-template <typename T, int LPR, typename TY = T>
-__device__ __forceinline__ void decode_reduce_wg(float m, float l, const float (&acc)[Vec16<T>::W], int wave, int grp, int gl,
+// More than four wavefronts (NW): each first adds up its own lane groups, so that one partial per wavefront meets in LDS.
+template <typename T, int LPR, typename TY = T, int NW = 4>
+__device__ __forceinline__ void decode_reduce_wg(float m, float l, float (&acc)[Vec16<T>::W], int wave, int grp, int gl,
                                                  int d0, bool active, int hs, float* __restrict__ out, TY* __restrict__ yfinal = nullptr,
                                                  float* __restrict__ plainAcc = nullptr)
 {
     constexpr int W = Vec16<T>::W;
-    constexpr int RPW = 64 / LPR, NW = 4;
-    __shared__ float sm[NW * RPW];
-    __shared__ float sl[NW * RPW];
-    __shared__ float sacc[NW * RPW][LPR * W + 1];
-    const int g = wave * RPW + grp;
-    if (gl == 0) { sm[g] = m; sl[g] = l; }
-    if (active) {
+    constexpr int RPW = NW > 4 ? 1 : 64 / LPR;
+    constexpr int NG = NW * RPW;
+    __shared__ float sm[NG];
+    __shared__ float sl[NG];
+    __shared__ float sacc[NG][LPR * W + 1];
+    if constexpr (NW > 4) {
+        const float M = across_groups<LPR, true>(m), c = m > -INFINITY ? __expf(m - M) : 0.f;
+        m = M;
+        l = across_groups<LPR, false>(l * c);
 #pragma unroll
-        for (int i = 0; i < W; i++) sacc[g][d0 + i] = acc[i];
+        for (int i = 0; i < W; i++) acc[i] = across_groups<LPR, false>(acc[i] * c);
+    }
+    const int g = NW > 4 ? wave : wave * RPW + grp;
+    if (NW == 4 || grp == 0) {
+        if (gl == 0) { sm[g] = m; sl[g] = l; }
+        if (active) {
+#pragma unroll
+            for (int i = 0; i < W; i++) sacc[g][d0 + i] = acc[i];
+        }
     }
     __syncthreads();
-    constexpr int NG = NW * RPW;
     if constexpr (NG <= 32) {
         // Every LDS read is unconditional and the group weights are computed once, side by side: with the reads under
         // `if (sm[i] > -inf)` the compiler emits one branch and one LDS round trip after the other.  An empty group has
@@ -237,7 +263,7 @@ __device__ __forceinline__ void decode_reduce_wg(float m, float l, const float (
             if (plainAcc) { out[0] = M; out[1] = L; }
             else { part_store(out, M); part_store(out + 1, L); }
         }
-        for (int d = threadIdx.x; d < hs; d += 256) {
+        for (int d = threadIdx.x; d < hs; d += NW * 64) {
             float v = 0.f;
 #pragma unroll
             for (int i = 0; i < NG; i++) v += sacc[i][d] * w[i];
@@ -248,13 +274,13 @@ __device__ __forceinline__ void decode_reduce_wg(float m, float l, const float (
         return;
     }
     float M = -INFINITY;
-    for (int i = 0; i < NW * RPW; i++) M = fmaxf(M, sm[i]);
+    for (int i = 0; i < NG; i++) M = fmaxf(M, sm[i]);
     if (yfinal) {
         float L = 0.f;
-        for (int i = 0; i < NW * RPW; i++) L += (sm[i] > -INFINITY) ? sl[i] * __expf(sm[i] - M) : 0.f;
-        for (int d = threadIdx.x; d < hs; d += 256) {
+        for (int i = 0; i < NG; i++) L += (sm[i] > -INFINITY) ? sl[i] * __expf(sm[i] - M) : 0.f;
+        for (int d = threadIdx.x; d < hs; d += NW * 64) {
             float v = 0.f;
-            for (int i = 0; i < NW * RPW; i++)
+            for (int i = 0; i < NG; i++)
                 if (sm[i] > -INFINITY) v += sacc[i][d] * __expf(sm[i] - M);
             st1(yfinal + d, v / L);
         }
@@ -262,13 +288,13 @@ __device__ __forceinline__ void decode_reduce_wg(float m, float l, const float (
     }
     if (threadIdx.x == 0) {
         float L = 0.f;
-        for (int i = 0; i < NW * RPW; i++) L += (sm[i] > -INFINITY) ? sl[i] * __expf(sm[i] - M) : 0.f;
+        for (int i = 0; i < NG; i++) L += (sm[i] > -INFINITY) ? sl[i] * __expf(sm[i] - M) : 0.f;
         if (plainAcc) { out[0] = M; out[1] = L; }
         else { part_store(out, M); part_store(out + 1, L); }
     }
-    for (int d = threadIdx.x; d < hs; d += 256) {
+    for (int d = threadIdx.x; d < hs; d += NW * 64) {
         float v = 0.f;
-        for (int i = 0; i < NW * RPW; i++)
+        for (int i = 0; i < NG; i++)
             if (sm[i] > -INFINITY) v += sacc[i][d] * __expf(sm[i] - M);
         if (plainAcc) plainAcc[d] = v;
         else part_store(out + 2 + d, v);
@@ -463,7 +489,8 @@ struct FusedDecodeArgs {
     const float* fcos; const float* fsin; const int* dlen;
     int B, H, kvMul, hs, dim, kvd, seqLen, splits, rowsPerIter;
     float scale;
-    bool oneIter;   // seqLen <= splits * rowsPerIter: a split never holds more than one iteration of rows
+    int reach;      // rows the caches may come to hold (<= seqLen)
+    bool oneIter;   // reach <= splits * rowsPerIter: a split never holds more than one iteration of rows
     // B == 1 and oneIter only: leave the merge of the splits to the next kernel.  Split s of head h writes its
     // accumulator to part[s * dim + h * hs ..] and {m, l} to part[splits * dim + (s * H + h) * 2 ..]; y is not written.
     bool deferMerge;
@@ -563,10 +590,11 @@ __global__ __launch_bounds__(256) void attn_decode_fused_kernel(FusedDecodeArgs 
     decode_merge<float>(a.part + bh * a.splits * (a.hs + 2), a.counters + bh, nAct, a.hs, yout);
 }
 
-// The engine form when the whole cache fits one iteration per split (seqLen <= splits * rowsPerIter): a kernel of its
-// own so that the order of its memory requests is the one written here.
-template <int LPR, typename TC>
-__global__ __launch_bounds__(256) void attn_decode_fused_step_kernel(FusedDecodeArgs a)
+// The engine form when the whole cache fits one iteration per split (reach <= splits * rowsPerIter): a kernel of its
+// own so that the order of its memory requests is the one written here.  NW wavefronts: four where several splits share a
+// cache, up to sixteen where one workgroup takes all of it (fused_waves).
+template <int LPR, typename TC, int NW>
+__global__ __launch_bounds__(NW * 64) void attn_decode_fused_step_kernel(FusedDecodeArgs a)
 {
     constexpr int W = Vec16<TC>::W;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
@@ -609,7 +637,7 @@ __global__ __launch_bounds__(256) void attn_decode_fused_step_kernel(FusedDecode
     // outstanding load at the first use of any.  The rotation factors follow as soon as the length is known, and
     // the row at `pos` (which the cache does not hold yet) is patched in registers instead of being stored and
     // read back.  Arithmetic and its order are those of attn_decode_fused_kernel.
-    constexpr int RPW = 64 / LPR, U = 4, STEP = 4 * RPW * U;
+    constexpr int RPW = 64 / LPR, U = 4, STEP = NW * RPW * U;
     const int t0 = split * STEP;
     const int tb = t0 + wave * RPW * U;
     const int dc = active ? d0 : 0;
@@ -619,9 +647,9 @@ __global__ __launch_bounds__(256) void attn_decode_fused_step_kernel(FusedDecode
     load_row(row + a.dim + a.kvd + (size_t)kvh * a.hs + dc, vr);
     DecodeStage<U> A;
 #pragma unroll
-    for (int u = 0; u < U; u++) A.k[u] = *(const u32x4*)(kc + (size_t)min(tb + u * RPW + grp, a.seqLen - 1) * a.kvd + dc);
+    for (int u = 0; u < U; u++) A.k[u] = *(const u32x4*)(kc + (size_t)min(tb + u * RPW + grp, a.reach - 1) * a.kvd + dc);
 #pragma unroll
-    for (int u = 0; u < U; u++) A.v[u] = *(const u32x4*)(vc + (size_t)min(tb + u * RPW + grp, a.seqLen - 1) * a.kvd + dc);
+    for (int u = 0; u < U; u++) A.v[u] = *(const u32x4*)(vc + (size_t)min(tb + u * RPW + grp, a.reach - 1) * a.kvd + dc);
     __builtin_amdgcn_sched_barrier(0);   // the requests above are issued before the length is asked for
     const int len = *a.dlen, pos = len - 1;
     const int nAct = (len + STEP - 1) / STEP;
@@ -662,6 +690,10 @@ __global__ __launch_bounds__(256) void attn_decode_fused_step_kernel(FusedDecode
 #pragma unroll
     for (int i = 0; i < W; i++) acc[i] = 0.f;
     decode_consume<TC, LPR, U>(A, tb, t1, grp, qv, m, l, acc);
+    if constexpr (NW > 4) {   // one workgroup per cache
+        decode_reduce_wg<TC, LPR, float, NW>(m, l, acc, wave, grp, gl, d0, active, a.hs, (float*)nullptr, a.y + (size_t)b * a.dim + (size_t)h * a.hs);
+        return;
+    }
     if (a.deferMerge) {
         decode_reduce_wg<TC, LPR, float>(m, l, acc, wave, grp, gl, d0, active, a.hs,
                                          a.part + (size_t)a.splits * a.dim + ((size_t)split * a.H + h) * 2, (float*)nullptr,
@@ -758,6 +790,16 @@ constexpr int kDecodeTargetWgs = 256;
 // split per pair needs no merge at all, and at 16 sequences x 12 heads that is worth more than a second split's
 // bandwidth (27.5k -> 27.9k tokens/s).  Fewer pairs keep the usual target.
 static int fused_target(int B, int H) { return (long long)B * H >= 128 ? 128 : kDecodeTargetWgs; }
+// Wavefronts of the one workgroup per (sequence, head) that takes a cache of up to `reach` rows in a single iteration, every
+// row requested before the length is known; 0 where that is not the form to use: caches longer than sixteen wavefronts hold
+// (256 fp32 rows of 64 values) or that four already hold, and fewer pairs than fill half the chip, whose caches are split over
+// more CUs instead (16 sequences x 12 heads, 160 rows: 7.8 -> 6.5 us; batch 1, 192 rows of the 110M model: 3.9 us in three splits, 6.0 us in one workgroup of twelve wavefronts).
+static int fused_waves(int B, int H, int lprp, int reach)
+{
+    if ((long long)B * H < 128 || lprp < 8 || lprp > 32) return 0;
+    const int w = (reach + 256 / lprp - 1) / (256 / lprp);   // four row groups of 64 / lprp rows a wavefront
+    return w <= 4 || w > 16 ? 0 : (w + 1) / 2 * 2;
+}
 static void pick_splits(int B, int H, int len, int rows_per_iter, int* splits, int* chunk, int target = kDecodeTargetWgs)
 {
     // never less than one full iteration per split
@@ -840,7 +882,7 @@ hipError_t k_attn_decode(hipStream_t s, DType dt, const void* q, const void* kc,
 
 // The splits of a launch that leaves the merge to the next kernel (batch 1, the whole cache in one iteration per split), and
 // the rows each of them covers; 0 when the launch cannot be of that kind.
-int attn_decode_fused_deferred_splits(int B, int H, int hs, int seqLen, DType cacheType, int* rowsPerSplit)
+int attn_decode_fused_deferred_splits(int B, int H, int hs, int seqLen, int reach, DType cacheType, int* rowsPerSplit)
 {
     const int W = cacheType == F32 ? 4 : 8;
     if (B != 1 || H <= 0 || hs <= 0 || hs % W != 0 || seqLen <= 0) return 0;
@@ -848,15 +890,17 @@ int attn_decode_fused_deferred_splits(int B, int H, int hs, int seqLen, DType ca
     while (lprp < lpr) lprp <<= 1;
     if (lprp > 64) return 0;
     const int rpi = 4 * (64 / lprp) * 4;
+    reach = std::min(reach, seqLen);
+    if (fused_waves(B, H, lprp, reach)) return 0;
     int splits, chunk;
-    pick_splits(B, H, seqLen, rpi, &splits, &chunk, fused_target(B, H));
-    if (seqLen > splits * rpi) return 0;
+    pick_splits(B, H, reach, rpi, &splits, &chunk, fused_target(B, H));
+    if (reach > splits * rpi) return 0;
     if (rowsPerSplit) *rowsPerSplit = rpi;
     return splits;
 }
 
 hipError_t k_attn_decode_fused(hipStream_t s, const float* qkv, void* kc, void* vc, DType cacheType, float* y, int B, int H, int kvH,
-                               int hs, int seqLen, float scale, const float* fcos, const float* fsin, const int* dlen, void* workspace,
+                               int hs, int seqLen, int reach, float scale, const float* fcos, const float* fsin, const int* dlen, void* workspace,
                                size_t workspaceBytes, int* counters, bool deferMerge)
 {
     if (B <= 0 || H <= 0 || hs <= 0 || seqLen <= 0) return hipSuccess;
@@ -866,29 +910,42 @@ hipError_t k_attn_decode_fused(hipStream_t s, const float* qkv, void* kc, void* 
     while (lprp < lpr) lprp <<= 1;
     if (lprp > 64) return hipErrorInvalidValue;
     if (workspaceBytes < attn_decode_workspace_bytes(B, H, hs, seqLen)) return hipErrorInvalidValue;
+    if (reach < 1 || reach > seqLen) return hipErrorInvalidValue;
     FusedDecodeArgs a;
     a.qkv = qkv; a.kc = kc; a.vc = vc; a.y = y; a.part = (float*)workspace; a.counters = counters;
     a.fcos = fcos; a.fsin = fsin; a.dlen = dlen;
     a.B = B; a.H = H; a.kvMul = H / kvH; a.hs = hs; a.dim = H * hs; a.kvd = kvH * hs; a.seqLen = seqLen;
     a.rowsPerIter = 4 * (64 / lprp) * 4;
     int chunk;
-    pick_splits(B, H, seqLen, a.rowsPerIter, &a.splits, &chunk, fused_target(B, H));
+    a.reach = reach;
+    pick_splits(B, H, reach, a.rowsPerIter, &a.splits, &chunk, fused_target(B, H));
+    const int waves = fused_waves(B, H, lprp, reach);
+    if (waves) a.splits = 1;
     a.scale = scale;
-    a.oneIter = seqLen <= a.splits * a.rowsPerIter;
+    a.oneIter = waves || reach <= a.splits * a.rowsPerIter;
     a.deferMerge = deferMerge;
     if (deferMerge && (B != 1 || !a.oneIter)) return hipErrorInvalidValue;
     dim3 grid(a.splits, H, B);
+#define FUSED_STEP(L, NW)                                                                                                  \
+    do {                                                                                                                   \
+        if (cacheType == F32) hipLaunchKernelGGL((attn_decode_fused_step_kernel<L, float, NW>), grid, NW * 64, 0, s, a);   \
+        else hipLaunchKernelGGL((attn_decode_fused_step_kernel<L, bf16_t, NW>), grid, NW * 64, 0, s, a);                   \
+    } while (0)
     switch (lprp) {
 #define CASE(L)                                                                                                            \
     case L:                                                                                                                \
         if (a.oneIter) {                                                                                                   \
-            if (cacheType == F32) hipLaunchKernelGGL((attn_decode_fused_step_kernel<L, float>), grid, 256, 0, s, a);       \
-            else hipLaunchKernelGGL((attn_decode_fused_step_kernel<L, bf16_t>), grid, 256, 0, s, a);                       \
+            if constexpr (L >= 8 && L <= 32) {                                                                             \
+                if (waves > 14) FUSED_STEP(L, 16); else if (waves > 12) FUSED_STEP(L, 14);                                  \
+                else if (waves > 10) FUSED_STEP(L, 12); else if (waves > 8) FUSED_STEP(L, 10);                              \
+                else if (waves > 6) FUSED_STEP(L, 8); else if (waves > 4) FUSED_STEP(L, 6); else FUSED_STEP(L, 4);          \
+            } else FUSED_STEP(L, 4);                                                                                       \
         } else if (cacheType == F32) hipLaunchKernelGGL((attn_decode_fused_kernel<L, float>), grid, 256, 0, s, a);         \
         else hipLaunchKernelGGL((attn_decode_fused_kernel<L, bf16_t>), grid, 256, 0, s, a);                                \
         break;
         CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32) CASE(64)
 #undef CASE
+#undef FUSED_STEP
     }
     return hipGetLastError();
 }

@@ -578,6 +578,171 @@ __global__ __launch_bounds__(NS * 64) void matvec_mfma_kernel(const T* __restric
     }
 }
 
+// The same product for a decode step on tile-packed weights.  A step's kernels are a few microseconds long and what bounds them
+// is how few workgroups 16-row tiles make (48 for the 768 rows of wo and w2) and what each of them has to pull out of L2 and
+// put through its matrix cores: at 16 sequences and 2048 columns 131 KB of activations and 1.9 us of fp32 MFMAs on 48 of 256
+// CUs.  So
+//  * a workgroup takes `seq` of the sequences, 16 or 4 of them, so that small matrices spread over the chip (the rule is in
+//    launch_matvec_step); lanes of absent columns read past the end of their buffer resource and get zeros without a fetch;
+//  * 16-bit weights are multiplied on v_mfma_f32_16x16x32_bf16 with every fp32 activation as three bf16 numbers - nearest,
+//    nearest to the remainder, and what is left: 24 bits, the value itself - whose products with a bf16 weight are exact and
+//    accumulate in fp32 as before; per slab 3 instructions of 16 cycles where the fp32 form has 8 of 32;
+//  * all slabs of a wavefront (up to U) are requested at once without a branch, the partial tiles are read back side by side
+//    and a quad of results is one 16-byte store.
+// NT tiles per workgroup share the activations: the two matrices of MODE 2, or two neighbouring row tiles.
+// 110M model, 16 sequences, bf16 weights, us per launch before -> after: see launch_matvec_step.
+typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
+template <typename T> struct StepSlab;
+template <> struct StepSlab<float> {
+    static constexpr int PIECES = 2, XLANE = 16, XPIECE = 64;   // columns 16 half + 4 kk .. + 3 per piece
+    typedef float X[8];
+    __device__ static inline void split(const float (&v)[8], X& x)
+    {
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = v[e];
+    }
+    __device__ static inline floatx4v mul(const uint4 (&w)[2], const X& x, floatx4v acc)
+    {
+        const uint32_t u[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(u[e]), x[e], acc, 0, 0, 0);
+        return acc;
+    }
+};
+template <> struct StepSlab<bf16_t> {
+    static constexpr int PIECES = 1, XLANE = 32, XPIECE = 16;   // columns 8 kk .. + 7
+    struct X { bf16x8v p[3]; };
+    __device__ static inline void split(const float (&v)[8], X& x)
+    {
+        float r[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) r[e] = v[e];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                x.p[q][e] = (__bf16)r[e];
+                if (q < 2) r[e] -= (float)x.p[q][e];
+            }
+    }
+    __device__ static inline floatx4v mul(const uint4 (&w)[1], const X& x, floatx4v acc)
+    {
+        const bf16x8v a = __builtin_bit_cast(bf16x8v, w[0]);
+#pragma unroll
+        for (int q = 0; q < 3; q++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, x.p[q], acc, 0, 0, 0);
+        return acc;
+    }
+};
+struct StepArgs { const void* W; const float* x; const float* g; float* y; int rows, n, B, ldy, seq, nGroups; };
+
+template <typename T, int MODE, bool NORM, int NT, int U, int NS>
+__global__ __launch_bounds__(NS * 64) void matvec_step_kernel(StepArgs a)
+{
+    typedef StepSlab<T> S;
+    constexpr int SLAB = 512 * sizeof(T);
+    __shared__ __attribute__((aligned(16))) float part[NS][NT * 256];
+    __shared__ float sspart[NS][16];
+    const int die = blockIdx.x & 7, slot = blockIdx.x >> 3;   // workgroups of the same rows on the same die, as above
+    const int nit = a.n >> 5, tiles = (a.rows + 15) >> 4;
+    const int unit = (slot / a.nGroups) * 8 + die, b0 = (slot % a.nGroups) * a.seq;
+    const int tile0 = MODE == 2 ? unit : unit * NT;
+    if (tile0 >= tiles) return;   // the grid is padded to a multiple of 8
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, kk = lane >> 4;
+    const int cnt = min(a.seq, a.B - b0);
+    const size_t tileBytes = (size_t)nit * SLAB;
+    __amdgpu_buffer_rsrc_t rw[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+        rw[t] = __builtin_amdgcn_make_buffer_rsrc((char*)a.W + (size_t)min(tile0 + (MODE == 2 ? t * tiles : t), MODE == 2 ? 2 * tiles - 1 : tiles - 1) * tileBytes, 0,
+                                                  (int)tileBytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((char*)(a.x + (size_t)b0 * a.n), 0, cnt * a.n * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((char*)(NORM ? a.g : a.x), 0, a.n * 4, 0x00020000);
+    const int xo = i < cnt ? i * a.n * 4 + kk * S::XLANE : 0x40000000;   // past the end for a column that does not exist
+    // the wavefront that finishes a tile requests the residual's old values with the first weights
+    const int ft = MODE == 2 ? 0 : min(wave, NT - 1), row = (tile0 + ft) * 16 + 4 * kk;
+    float* out = a.y + (size_t)(b0 + min(i, cnt - 1)) * a.ldy + min(row, a.rows - 4);
+    float4 prev = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (MODE == 1) prev = *(const float4*)out;
+    floatx4v acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[t] = floatx4v{0.f, 0.f, 0.f, 0.f};
+    float ss = 0.f;
+    for (int base = wave; base < nit; base += NS * U) {
+        uint4 w[U][NT][S::PIECES];
+        float xv[U][8], gv[NORM ? U : 1][8];
+        auto load8 = [&](const __amdgpu_buffer_rsrc_t r, int at, int slab, float (&o)[8]) {
+            const auto p0 = __builtin_amdgcn_raw_buffer_load_b128(r, at, slab * 128, 0), p1 = __builtin_amdgcn_raw_buffer_load_b128(r, at + S::XPIECE, slab * 128, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) { o[e] = __uint_as_float(p0[e]); o[4 + e] = __uint_as_float(p1[e]); }
+        };
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int sl = min(base + u * NS, nit - 1);   // past the end: the last slab once more, not used
+            load8(rx, xo, sl, xv[u]);
+            if (NORM) load8(rg, kk * S::XLANE, sl, gv[NORM ? u : 0]);
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int q = 0; q < S::PIECES; q++) {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw[t], lane * 16 + q * 1024, sl * SLAB, 0);
+                    w[u][t][q] = make_uint4(v[0], v[1], v[2], v[3]);
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (base + u * NS >= nit) break;
+            if (NORM) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    ss += xv[u][e] * xv[u][e];
+                    xv[u][e] *= gv[NORM ? u : 0][e];
+                }
+            }
+            typename S::X x;
+            S::split(xv[u], x);
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[t] = S::mul(w[u][t], x, acc[t]);
+        }
+    }
+    if (NORM) {
+        ss = add_lane_xor<16>(ss);
+        ss = add_lane_xor<32>(ss);
+        if (kk == 0) sspart[wave][i] = ss;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) *(floatx4v*)&part[wave][t * 256 + lane * 4] = acc[t];
+    __syncthreads();
+    if (wave >= (MODE == 2 ? 1 : NT)) return;
+    // accumulator register v of lane l is row 4 * (l / 16) + v, column l % 16
+    floatx4v p[NS], p2[MODE == 2 ? NS : 1];
+    float sp[NORM ? NS : 1];
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        p[q] = *(const floatx4v*)&part[q][ft * 256 + lane * 4];
+        if (MODE == 2) p2[MODE == 2 ? q : 0] = *(const floatx4v*)&part[q][(NT - 1) * 256 + lane * 4];
+        if (NORM) sp[NORM ? q : 0] = sspart[q][i];
+    }
+    floatx4v d = p[0], d2 = p2[0];
+    float sq = sp[0];
+#pragma unroll
+    for (int q = 1; q < NS; q++) {
+        d += p[q];
+        if (MODE == 2) d2 += p2[MODE == 2 ? q : 0];
+        if (NORM) sq += sp[NORM ? q : 0];
+    }
+    const float inv = NORM ? 1.0f / sqrtf(sq / a.n + 1e-5f) : 1.f;
+    float o[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const float a0 = d[v] * inv;
+        if (MODE == 0) o[v] = a0;
+        else if (MODE == 1) o[v] = (v == 0 ? prev.x : v == 1 ? prev.y : v == 2 ? prev.z : prev.w) + a0;
+        else o[v] = a0 * (1.0f / (1.0f + expf(-a0))) * (d2[v] * inv);
+    }
+    if (i < cnt && row < a.rows && tile0 + ft < tiles) *(float4*)out = make_float4(o[0], o[1], o[2], o[3]);
+}
+
 // End of a decode step, one workgroup per sequence: first-max argmax over the logits
 // (sample_argmax, llama2_sampler.cpp:25-36: strict '>' so the lowest index wins ties), record
 // the id, embed the token of the next position (forced prompt id while pos + 1 < n_prompt,
@@ -1387,6 +1552,7 @@ private:
     template <typename T> long step(hipStream_t s, int B, int nSteps, float* allLogits, StepProfile* prof = nullptr, int tail = 1);
     template <typename T> long advance_given(hipStream_t s, int B);
     long ensure_state(int B, int nSteps);
+    int step_reach(int nSteps) const;
     long ensure_prefill(size_t rows);
     template <typename T> long prefill(hipStream_t s, int B, int P, int nSteps, float* allLogits, int tail = 1);
     hipError_t embed_first(hipStream_t s, int B);
@@ -1406,6 +1572,8 @@ private:
     // where a matrix cannot be packed (columns not a multiple of 32) or the memory was not to be had
     std::vector<LayerW<void>> packed;
     void* wclsP = nullptr;
+    char* packArena = nullptr;
+    size_t packWanted = 0, packUsed = 0;
     template <typename T> void* pack_matrix(const void* W, size_t rows, size_t n, size_t second = 0);
     template <typename T> void pack_all();
     std::vector<LayerW<void>> layers;
@@ -1420,7 +1588,7 @@ private:
     int *dprompt = nullptr, *dnext = nullptr, *dcur = nullptr, *dout = nullptr;
     int *dcount = nullptr, *dticket = nullptr;   // attention merge tickets (B * heads) and the step ticket; zero between launches
     hipGraphExec_t graphExec = nullptr;
-    int graphB = 0;
+    int graphB = 0, graphReach = 0;
     int graphTail = 1;                           // the tail the captured step ends with (see step), and the sampler
     float graphTemperature = 0.f, graphTopp = 0.f;   // parameters captured with tail 2
     float sampleTemperature = 1.f, sampleTopp = 0.9f;
@@ -1530,8 +1698,10 @@ template <typename T> void* Engine::pack_matrix(const void* W, size_t rows, size
 {
     if (n % 32 != 0 || rows == 0) return nullptr;
     const size_t tiles = (rows + 15) / 16, per = tiles * 16 * n;
-    void* P = dalloc((second ? 2 : 1) * per * sizeof(T));
-    if (!P) { (void)hipGetLastError(); return nullptr; }
+    const size_t bytes = ((second ? 2 : 1) * per * sizeof(T) + 255) / 256 * 256;
+    if (!packArena) { packWanted += bytes; return nullptr; }   // first round: sizes only
+    void* P = packArena + packUsed;
+    packUsed += bytes;
     for (int m = 0; m < (second ? 2 : 1); m++) {
         const size_t pieces = per * sizeof(T) / 16;
         const int grid = (int)std::min<size_t>((pieces + 255) / 256, 65535);
@@ -1544,13 +1714,22 @@ template <typename T> void Engine::pack_all()
 {
     const size_t dim = cfg.dim, hid = cfg.hidden_dim, hs = dim / cfg.n_heads, kvd = hs * cfg.n_kv_heads;
     packed.assign(layers.size(), LayerW<void>{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr});
-    for (size_t l = 0; l < layers.size(); l++) {
-        packed[l].wqkv = pack_matrix<T>(layers[l].wqkv, dim + 2 * kvd, dim);
-        packed[l].wo = pack_matrix<T>(layers[l].wo, dim, dim);
-        packed[l].w13 = pack_matrix<T>(layers[l].w13, hid, dim, hid);
-        packed[l].w2 = pack_matrix<T>(layers[l].w2, dim, hid);
+    // all copies in one allocation: dozens of small ones are mapped in small pages
+    packArena = nullptr;
+    packWanted = packUsed = 0;
+    for (int round = 0; round < 2; round++) {
+        if (round) {
+            packArena = packWanted ? (char*)dalloc(packWanted) : nullptr;
+            if (!packArena) { (void)hipGetLastError(); break; }
+        }
+        for (size_t l = 0; l < layers.size(); l++) {
+            packed[l].wqkv = pack_matrix<T>(layers[l].wqkv, dim + 2 * kvd, dim);
+            packed[l].wo = pack_matrix<T>(layers[l].wo, dim, dim);
+            packed[l].w13 = pack_matrix<T>(layers[l].w13, hid, dim, hid);
+            packed[l].w2 = pack_matrix<T>(layers[l].w2, dim, hid);
+        }
+        wclsP = pack_matrix<T>(wcls, cfg.vocab_size, dim);
     }
-    wclsP = pack_matrix<T>(wcls, cfg.vocab_size, dim);
     (void)hipStreamSynchronize(stream);
 }
 
@@ -1637,10 +1816,22 @@ long Engine::ensure_state(int B, int nSteps)
     stateAllocs.clear();
     stateB = 0;
     const size_t dim = cfg.dim, hid = cfg.hidden_dim, hs = dim / cfg.n_heads, kvd = hs * cfg.n_kv_heads;
-    auto sa = [&](size_t bytes) -> void* {
+    char* slab = nullptr;
+    size_t slabLeft = 0;
+    auto sa = [&](size_t bytes) -> void* {   // the small buffers share allocations of 8 MB
+        constexpr size_t SLAB = 8u << 20;
+        bytes = (bytes + 255) / 256 * 256;
         void* p = nullptr;
-        if (hipMalloc(&p, bytes ? bytes : 4) != hipSuccess) return nullptr;
+        const bool small = bytes && bytes <= SLAB / 4;
+        if (small && bytes <= slabLeft) {
+            p = slab;
+            slab += bytes;
+            slabLeft -= bytes;
+            return p;
+        }
+        if (hipMalloc(&p, small ? SLAB : bytes ? bytes : 4) != hipSuccess) return nullptr;
         stateAllocs.push_back(p);
+        if (small) { slab = (char*)p + bytes; slabLeft = SLAB - bytes; }
         return p;
     };
     const size_t cacheN = (size_t)cfg.n_layers * B * cfg.seq_len * kvd;
@@ -1849,20 +2040,39 @@ template <typename T> long Engine::prefill(hipStream_t s, int B, int P, int nSte
     return 0;
 }
 
+// Sequences and row tiles per workgroup of a decode step's product (see matvec_step_kernel).  Under 100 row tiles a workgroup
+// takes four sequences, which is what it costs to give most CUs one (48 tiles, 16 sequences: 192 workgroups); from there on the
+// rows do that and every activation is fetched once for 16.  Matrices of four times as many tiles as CUs take two tiles per
+// workgroup, which halves the activations read.  More than 32 slabs of columns: eight slabs of a wavefront in flight, not four.
+// 110M model, 16 sequences, bf16 weights, us per launch before -> after: wqkv 6.3 -> 5.6, wo and w2 7.1 -> 4.8 and 5.6,
+// w1 and w3 7.5 -> 6.2, classifier 24.7 -> 15.5.
+template <int MODE, bool NORM, typename T>
+static hipError_t launch_matvec_step(hipStream_t s, const void* Wp, const float* x, const float* g, float* y, int rows, int n, int B, int ldy)
+{
+    const int tiles = (rows + 15) / 16, seq = tiles >= 100 ? 16 : 4;
+    const StepArgs a = {Wp, x, g, y, rows, n, B, ldy, seq, (B + seq - 1) / seq};
+    const bool two = MODE != 2 && tiles >= 1024, deep = (n >> 5) > 32;
+    const int units = two ? (tiles + 1) / 2 : tiles, grid = (units + 7) / 8 * 8 * a.nGroups;
+    constexpr int NT = MODE == 2 ? 2 : 1;
+    if (two) hipLaunchKernelGGL((matvec_step_kernel<T, MODE, NORM, 2, 4, 8>), grid, 512, 0, s, a);
+    else if (deep) hipLaunchKernelGGL((matvec_step_kernel<T, MODE, NORM, NT, NT == 2 ? 4 : 8, 8>), grid, 512, 0, s, a);
+    else hipLaunchKernelGGL((matvec_step_kernel<T, MODE, NORM, NT, 4, 8>), grid, 512, 0, s, a);
+    return hipGetLastError();
+}
+
 template <int MODE, bool NORM, typename T>
 static hipError_t launch_matvec(hipStream_t s, const void* W, const float* x, const float* g, float* y, int rows, int n, int B,
                                 int ldy, int rowsPerWave, const void* Wp = nullptr)
 {
     if (B >= 2 && n % 32 == 0) {
+        // Wp: the tile-packed copy of W, when the engine holds one
+        if (Wp && rows % 4 == 0 && ldy % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)g) & 15) == 0 && (long long)16 * n * 4 < 0x20000000)
+            return launch_matvec_step<MODE, NORM, T>(s, Wp, x, g, y, rows, n, B, ldy);
         // batched: matrix-core kernel, 16 sequences per pass over the weights
         const int ns = rows >= 8192 ? 4 : 8;   // fewer, longer wavefronts once the rows alone fill the chip
         // every group of 16 sequences walks the weights in the same launch
         const int nGroups = (B + 15) / 16, tiles8 = ((rows + 15) / 16 + 7) / 8;
-        // Wp: the tile-packed copy of W, when the engine holds one
-        if (Wp) {
-            if (ns == 4) hipLaunchKernelGGL((matvec_mfma_kernel<T, MODE, NORM, 1, 4, true>), tiles8 * 8 * nGroups, 256, 0, s, (const T*)Wp, x, g, y, rows, n, B, ldy, nGroups);
-            else hipLaunchKernelGGL((matvec_mfma_kernel<T, MODE, NORM, 1, 8, true>), tiles8 * 8 * nGroups, 512, 0, s, (const T*)Wp, x, g, y, rows, n, B, ldy, nGroups);
-        } else if (ns == 4) hipLaunchKernelGGL((matvec_mfma_kernel<T, MODE, NORM, 1, 4>), tiles8 * 8 * nGroups, 256, 0, s, (const T*)W, x, g, y, rows, n, B, ldy, nGroups);
+        if (ns == 4) hipLaunchKernelGGL((matvec_mfma_kernel<T, MODE, NORM, 1, 4>), tiles8 * 8 * nGroups, 256, 0, s, (const T*)W, x, g, y, rows, n, B, ldy, nGroups);
         else hipLaunchKernelGGL((matvec_mfma_kernel<T, MODE, NORM, 1, 8>), tiles8 * 8 * nGroups, 512, 0, s, (const T*)W, x, g, y, rows, n, B, ldy, nGroups);
         return hipGetLastError();
     }
@@ -1910,7 +2120,12 @@ static hipError_t launch_matvec_merge(hipStream_t s, const void* W, const float*
     const int grid = (rows + 3) / 4;
     const bool wide = sizeof(T) == 2 && n % 8 == 0 && (((uintptr_t)W) & 15) == 0;
     const int ch = wide ? 2 * ((n / 8 + 63) / 64) : (n / 4 + 63) / 64;
-#define MVM(C, WIDE_) hipLaunchKernelGGL((matvec_merge_kernel<T, C, WIDE_, kMergeSplits>), grid, 256, 0, s, (const T*)W, part, partML, dlen, splits, rowsPerSplit, H, hs, y, rows, n)
+    // short caches (up to four splits): four partials per thread in flight instead of sixteen mostly idle ones
+#define MVM(C, WIDE_)                                                                                                      \
+    do {                                                                                                                   \
+        if (splits <= 4) hipLaunchKernelGGL((matvec_merge_kernel<T, C, WIDE_, 4>), grid, 256, 0, s, (const T*)W, part, partML, dlen, splits, rowsPerSplit, H, hs, y, rows, n); \
+        else hipLaunchKernelGGL((matvec_merge_kernel<T, C, WIDE_, kMergeSplits>), grid, 256, 0, s, (const T*)W, part, partML, dlen, splits, rowsPerSplit, H, hs, y, rows, n); \
+    } while (0)
     if constexpr (sizeof(T) == 2) {
         if (wide) {
             if (ch <= 2) MVM(2, true); else MVM(4, true);
@@ -1950,6 +2165,15 @@ hipError_t Engine::embed_first(hipStream_t s, int B)
     return hipGetLastError();
 }
 
+// Rows of the caches a step is laid out for: steps of 32 up to 256 (where the attention kernel's workgroups differ), powers of
+// two above, so that generations of different lengths share a captured step.
+int Engine::step_reach(int nSteps) const
+{
+    int r = nSteps <= 256 ? (nSteps + 31) / 32 * 32 : 512;
+    while (r < nSteps) r *= 2;
+    return std::min(r, cfg.seq_len);
+}
+
 // enqueue one decode step for B sequences at the device-side position
 template <typename T> long Engine::step(hipStream_t s, int B, int nSteps, float* allLogits, StepProfile* prof, int tail)
 {
@@ -1958,9 +2182,10 @@ template <typename T> long Engine::step(hipStream_t s, int B, int nSteps, float*
 #define SPAN_BEGIN(cls) do { if (prof) HIPCHK(prof->begin(cls, s)); } while (0)
 #define SPAN_END() do { if (prof) HIPCHK(prof->end(s)); } while (0)
     const float scale = 1.0f / sqrtf((float)hs);
+    const int reach = step_reach(nSteps);
     // batch 1 with the cache in one iteration of rows per split: the attention leaves its splits to the output projection
     int deferRows = 0;
-    int deferSplits = defer_merge ? attn_decode_fused_deferred_splits(B, cfg.n_heads, hs, cfg.seq_len, state_kv_bf16 ? BF16 : F32, &deferRows) : 0;
+    int deferSplits = defer_merge ? attn_decode_fused_deferred_splits(B, cfg.n_heads, hs, cfg.seq_len, reach, state_kv_bf16 ? BF16 : F32, &deferRows) : 0;
     if (!matvec_merge_usable(dim, hs, deferSplits)) deferSplits = 0;
     for (int l = 0; l < cfg.n_layers; l++) {
         const LayerW<void>& w = layers[l];
@@ -1974,7 +2199,7 @@ template <typename T> long Engine::step(hipStream_t s, int B, int nSteps, float*
         SPAN_END();
         // xb = attention(rope(q), cache[0..pos] with rope(k), v appended)
         SPAN_BEGIN(SC_ATTN_DECODE);
-        HIPCHK(k_attn_decode_fused(s, qkv, kcl, vcl, state_kv_bf16 ? BF16 : F32, xb, B, cfg.n_heads, cfg.n_kv_heads, hs, cfg.seq_len, scale, fcos, fsin,
+        HIPCHK(k_attn_decode_fused(s, qkv, kcl, vcl, state_kv_bf16 ? BF16 : F32, xb, B, cfg.n_heads, cfg.n_kv_heads, hs, cfg.seq_len, reach, scale, fcos, fsin,
                                    &dstate->len, ws, wsBytes, dcount, deferSplits > 0));
         SPAN_END();
         // x += Wo xb (with the merge of the attention's splits in front when it was left to this kernel)
@@ -2214,7 +2439,7 @@ long Engine::generate(const int* prompts, int B, int nPrompt, int nSteps, bool w
     const hipEvent_t evA = sc.evA, evB = sc.evB;
     const int t0 = timedFrom < 0 ? nPrompt : timedFrom;
     bool graph = use_graph && !wantLogits;
-    if (graph && (!graphExec || graphB != B || graphTail != tail || (tail == 2 && (graphTemperature != sampleTemperature || graphTopp != sampleTopp)))) {
+    if (graph && (!graphExec || graphB != B || graphReach != step_reach(nSteps) || graphTail != tail || (tail == 2 && (graphTemperature != sampleTemperature || graphTopp != sampleTopp)))) {
         // one decode step, captured once; position / tokens are device-side so the graph is replayed as is
         if (graphExec) { (void)hipGraphExecDestroy(graphExec); graphExec = nullptr; }
         hipGraph_t g = nullptr;
@@ -2227,6 +2452,7 @@ long Engine::generate(const int* prompts, int B, int nPrompt, int nSteps, bool w
         }
         if (e || he != hipSuccess || !graphExec) { graphExec = nullptr; graph = false; e = 0; }
         graphB = B;
+        graphReach = step_reach(nSteps);
         graphTail = tail;
         graphTemperature = sampleTemperature;
         graphTopp = sampleTopp;

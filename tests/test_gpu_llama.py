@@ -600,3 +600,26 @@ def test_batched_prompt_pass_batch_of_sequences(llm, tmp_path):
         ref_ids, ref_logits = cpu.generate_greedy(prompts[b], n, want_logits=True)
         assert_close(logits[b], ref_logits, FP32_RTOL, "sequence %d" % b)
         assert np.array_equal(ids[b], ref_ids)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n", [70, 97, 128, 160, 180, 224, 256, 300])
+def test_batched_step_over_every_reach_of_the_attention_workgroup(llm, tmp_path, n, half):
+    """33 sequences x 4 heads: one attention workgroup per pair, of 6 to 16 wavefronts by the length of the generation (and
+    the split form beyond 256 rows); products of 16-sequence groups with a remainder of one, of 4-sequence groups, and a
+    classifier of 1025 row tiles, two per workgroup.  Weights are bf16 values, so both storages must give the fp32 result."""
+    cfg = dict(dim=256, hidden_dim=1056, n_layers=1, n_heads=4, n_kv_heads=2, vocab_size=16392, seq_len=320)
+    blob, _ = O.random_weights(cfg, seed=21, shared_classifier=False, std=0.08)
+    blob = bf16_round(blob)
+    path = str(tmp_path / "reach.bin")
+    O.write_checkpoint_v1(path, cfg, blob, False)
+    llm.SetOption(1, 1 if half else 0)
+    try:
+        llm.Load(path)
+        prompts = np.random.default_rng(n).integers(3, cfg["vocab_size"], (33, 5))
+        out = llm.GenerateBatch(prompts, n)
+    finally:
+        llm.SetOption(1, 0)
+    for b in (0, 32):
+        ref_ids, ref_logits = O.Llama(cfg, blob).generate_greedy(prompts[b], n, want_logits=True)
+        _check_ids(out[b], ref_ids, ref_logits, "batch row %d" % b)
