@@ -56,11 +56,19 @@ template <int ROWB> __device__ __forceinline__ int block_swizzle(int k)
     return ROWB % 256 == 0 ? (k & 3) * 4 : ((k >> 1) & 1) * 4;   // in chunks; rows 128 bytes apart modulo 256 alternate already
 }
 
-// the bias of eight columns from c on (0 past the matrix)
+// the bias of eight columns from c on (past the matrix the last one, never stored); all eight loads are under way at once
 __device__ __forceinline__ void b16_bias8(const GemmB16Args& g, int c, float (&bias)[8])
 {
+    if (!g.bias) {
 #pragma unroll
-    for (int q = 0; q < 8; q++) bias[q] = g.bias && c + q < g.N ? bf16_to_f32(g.bias[c + q]) : 0.f;
+        for (int q = 0; q < 8; q++) bias[q] = 0.f;
+        return;
+    }
+    bf16_t b[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) b[q] = g.bias[min(c + q, g.N - 1)];
+#pragma unroll
+    for (int q = 0; q < 8; q++) bias[q] = bf16_to_f32(b[q]);
 }
 
 // eight values of row r from column c on (inside the matrix up to N), alpha applied, and the bias, to C or through the heads
@@ -333,11 +341,15 @@ __global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsA
 // How a product is cut: the tile and the number of parts of the contraction with the smallest estimated time.
 struct GemmB16Plan { int shape, splits, kChunk; };
 // microseconds of one tile per 768 k and for its ends (first fetches, and stores that all CUs issue at once), with two and
-// more workgroups on the CU and alone on it; fitted to 8000 x 3072 x 768, 8000 x 768 x 3072, 768 x 3072 x 8000,
-// 8192 x 512 x 512 and 8192 x 12288 x 4096
+// more workgroups on the CU and alone on it.  Fitted to all six shapes, in 1 to 8 parts, at 32 sizes (M 512 .. 8192, N 384 ..
+// 3072, K 512 .. 8192, the three layouts): over those the shape taken is 0.5 % slower than the fastest on average and 12 % at
+// worst.  A 128 x 192 tile alone on its CU is dealt to eight wavefronts, two per SIMD, because with four nothing covers the wait
+// at the end of a stage (8192 x 768 x 768, 256 tiles: 14.8 us against 15.7 with four and 16.4 in 64 x 128 tiles); with two
+// such tiles on a CU four wavefronts each are better (8192 x 2304 x 768: 36.3 us against 42.9).
 struct GemmB16Shape { int bm, bn; double perK, ends, perKAlone, endsAlone; };
-static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 17.0, 5.0}, {256, 192, 10.0, 10.5, 10.0, 10.5}, {128, 192, 6.8, 4.4, 9.5, 6.0},
-                                           {128, 128, 4.2, 3.5, 6.0, 4.5}, {64, 128, 3.7, 1.0, 6.0, 1.5}, {64, 64, 2.5, 0.5, 4.1, 0.7}};
+static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 15.0, 7.5}, {256, 192, 10.0, 10.5, 10.0, 10.5}, {128, 192, 6.8, 4.4, 10.3, 4.5},
+                                           {128, 128, 4.2, 3.5, 7.0, 4.2}, {64, 128, 3.7, 1.3, 6.0, 1.5}, {64, 64, 2.5, 0.9, 4.1, 0.9}};
+enum { B16_128X192 = 2, B16_128X192_ALONE = 6 };
 
 static GemmB16Plan gemm_b16_plan(int m, int n, int k)
 {
@@ -354,7 +366,7 @@ static GemmB16Plan gemm_b16_plan(int m, int n, int k)
             const long long perCu = ((tiles * S + 7) / 8 + 31) / 32;
             double t = perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends);
             if (S > 1) t += 4.0 + (double)(S + 1) * m * n * 4.0 / 4.0e6;
-            if (t < bestT) { bestT = t; best = {sh, S, S > 1 ? chunk : k}; }
+            if (t < bestT) { bestT = t; best = {sh == B16_128X192 && perCu == 1 ? B16_128X192_ALONE : sh, S, S > 1 ? chunk : k}; }
         }
     }
     return best;
@@ -397,7 +409,8 @@ static hipError_t launch_b16_shape(hipStream_t s, const GemmB16Args& a, int shap
     switch (shape) {
     case 0: return launch_b16<4, 2, 2, 4, 2, AK, BKC, HEADS>(s, a, he);
     case 1: return launch_b16<4, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
-    case 2: return launch_b16<2, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
+    case B16_128X192: return launch_b16<2, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
+    case B16_128X192_ALONE: return launch_b16<4, 2, 1, 3, 2, AK, BKC, HEADS>(s, a, he);
     case 3: return launch_b16<2, 2, 2, 2, 2, AK, BKC, HEADS>(s, a, he);
     case 4: return launch_b16<2, 2, 1, 2, 3, AK, BKC, HEADS>(s, a, he);
     default: return launch_b16<2, 2, 1, 1, 4, AK, BKC, HEADS>(s, a, he);

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 # smallest, one past and one short of a tile, K of one chunk up to many stages, few tiles over a long K (parts), and sizes large
 # enough for each of the wider tiles; multiples of 8 (what the kernel takes in every layout), the last two not in N or M
 SHAPES = [(8, 8, 8), (64, 64, 64), (72, 56, 72), (128, 136, 200), (136, 264, 40), (200, 72, 2504), (768, 776, 8000), (2056, 1032, 264),
-          (3080, 2312, 136), (8000, 776, 136), (8192, 1544, 72), (8008, 3080, 64), (5128, 4104, 72), (100, 1001, 96), (1003, 136, 104)]
+          (3080, 2312, 136), (8000, 776, 136), (8192, 1544, 72), (8008, 3080, 64), (5128, 4104, 72), (8136, 760, 776), (4104, 1144, 520), (100, 1001, 96), (1003, 136, 104)]
 
 
 @pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False), (True, True)])
@@ -29,7 +29,7 @@ def test_gemm_edges(dev, m, n, k, tA, tB):
 
 
 @pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("m,n,k", [(70, 66, 40), (5, 50, 704), (64, 64, 4096), (8000, 776, 136), (8008, 3080, 64), (300, 7, 72)])
+@pytest.mark.parametrize("m,n,k", [(70, 66, 40), (5, 50, 704), (64, 64, 4096), (8000, 776, 136), (8008, 3080, 64), (300, 7, 72), (8136, 764, 776)])
 def test_linear_forward_edges(dev, m, n, k, bias):
     rng = np.random.default_rng(n)
     x, w, b = (bf16_round(rng.standard_normal(s).astype(np.float32)) for s in ((m, k), (n, k), (n,)))
