@@ -54,6 +54,8 @@ template <> struct BigTraits<float> {
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
         return c;
     }
+    __device__ static inline float ld(const float* p) { return *p; }
+    __device__ static inline void st4(float* p, float a, float b, float c, float d) { *(float4*)p = make_float4(a, b, c, d); }
 };
 
 // Epilogue of the fused QKV projection (HEADS): row r = (b, t) of the M = B*T rows, column c = (which, h, d) of the

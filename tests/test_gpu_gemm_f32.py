@@ -45,3 +45,36 @@ def test_linear_forward_edges(dev, m, n, k):
     dev.cuda.LinearForward(m, n, k, dev.put(x), dev.put(w), dev.put(b), hy)
     ref = x.astype(np.float64) @ w.T.astype(np.float64) + b
     assert np.abs(dev.get(hy, (m, n)) - ref).max() / np.abs(ref).max() < 4e-6
+
+
+# sizes that 256 x 288 tiles divide, fill one round of the chip, and 128 x 128 tiles would not: the smallest contraction taken,
+# one that ends an odd number of stages later, and the two ways the sizes can be met
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("m,n,k", [(8192, 2304, 256), (14592, 1152, 288), (8192, 2304, 252)])
+def test_one_round_of_wide_tiles(dev, m, n, k, bias):
+    rng = np.random.default_rng(k)
+    x, w, b = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (n, k), (n,)))
+    hx, hw, hb, hy = dev.put(x), dev.put(w), dev.put(b), dev.zeros(m * n)
+    ref = x.astype(np.float64) @ w.T.astype(np.float64)
+    dev.cuda.gemm(False, True, m, n, k, -0.5, hx, hw, 0.0, hy)
+    assert np.abs(dev.get(hy, (m, n)) + 0.5 * ref).max() / np.abs(ref).max() < 2e-6
+    dev.cuda.LinearForward(m, n, k, hx, hw, hb if bias else 0, hy)
+    assert np.abs(dev.get(hy, (m, n)) - ref - (b if bias else 0)).max() / np.abs(ref).max() < 2e-6
+
+
+@pytest.mark.parametrize("rope", [False, True])
+def test_one_round_of_wide_tiles_into_heads(dev, rope):
+    from oracle import attention_ref as R
+    B, T, H, hs = 16, 512, 12, 64
+    C = H * hs
+    rng = np.random.default_rng(5)
+    x, w, b = (rng.standard_normal(s).astype(np.float32) for s in ((B * T, C), (3 * C, C), (3 * C,)))
+    hq = [dev.zeros(B * T * C) for _ in range(3)]
+    hr = dev.cuda.CreateRope(0, 0, B * T * C, B, T, H, hs, 10000.0) if rope else 0
+    dev.cuda.QkvProjHeads(B, T, H, hs, dev.put(x), dev.put(w), dev.put(b), *hq, hr)
+    ref = (x.astype(np.float64) @ w.T.astype(np.float64) + b).reshape(B, T, 3, H, hs)
+    for i, h in enumerate(hq):
+        want = R.rope_forward(ref[:, :, i], T, H, hs, dtype=np.float64).reshape(B, T, H, hs) if rope and i < 2 else ref[:, :, i]
+        assert np.abs(dev.get(h, (B, H, T, hs)).transpose(0, 2, 1, 3) - want).max() <= (1e-4 if rope else 4e-6) * np.abs(ref).max()
+    if hr:
+        dev.cuda.FreeRope(hr)
