@@ -140,26 +140,39 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
     const int kBegin = split ? part * g.kChunk : 0, kEnd = min(g.K, kBegin + g.kChunk);
     const int wm = (wave / WVN) * (32 * WM), wn = (wave % WVN) * (32 * WN);
 
-    // byte offsets of this thread's chunks (the operands are below 2 GB); rows past the edge are clamped and never stored
+    // The buffer resource of an operand begins at the tile, and where the row index is at unit stride at the stage, so that
+    // operands of any size are reached with 32-bit byte offsets (gemm_b16_takes).  Offsets of this thread's chunks from there;
+    // rows past the edge are clamped and never stored.
     constexpr uint32_t OUTSIDE = 0x80000000u;
+    const bf16_t* baseA = g.A + (AK ? (size_t)m0 * g.lda : (size_t)m0);
+    const bf16_t* baseB = g.B + (BKC ? (size_t)n0 * g.ldb : (size_t)n0);
     uint32_t va[PA], vb[PB];
 #pragma unroll
     for (int p = 0; p < PA; p++) {
         const int e = p * NT + tid;
-        if (AK) va[p] = (uint32_t)(min(m0 + e / 8, M - 1) * g.lda + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
-        else va[p] = (uint32_t)((e / (BM / 8)) * g.lda + min(m0 + ((e % (BM / 8)) ^ block_swizzle<BM * 2>(e / (BM / 8))) * 8, M - 8)) * 2;
+        if (AK) va[p] = ((uint32_t)min(e / 8, M - 1 - m0) * (uint32_t)g.lda + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
+        else va[p] = ((uint32_t)(e / (BM / 8)) * (uint32_t)g.lda + min(((e % (BM / 8)) ^ block_swizzle<BM * 2>(e / (BM / 8))) * 8, M - 8 - m0)) * 2;
     }
 #pragma unroll
     for (int p = 0; p < PB; p++) {
         const int e = p * NT + tid;
-        if (BKC) vb[p] = (uint32_t)(min(n0 + e / 8, N - 1) * g.ldb + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
-        else vb[p] = (uint32_t)((e / (BN / 8)) * g.ldb + min(n0 + ((e % (BN / 8)) ^ block_swizzle<BN * 2>(e / (BN / 8))) * 8, N - 8)) * 2;
+        if (BKC) vb[p] = ((uint32_t)min(e / 8, N - 1 - n0) * (uint32_t)g.ldb + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
+        else vb[p] = ((uint32_t)(e / (BN / 8)) * (uint32_t)g.ldb + min(((e % (BN / 8)) ^ block_swizzle<BN * 2>(e / (BN / 8))) * 8, N - 8 - n0)) * 2;
     }
-    const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)g.A, 0, (int)(OUTSIDE - 16), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)g.B, 0, (int)(OUTSIDE - 16), 0x00020000);
+    auto resource = [](const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(OUTSIDE - 16), 0x00020000); };
+    const __amdgpu_buffer_rsrc_t rsA = resource(baseA), rsB = resource(baseB);
+    // where resources begin at stages: the stage that is fetched next, and the way to the one after it (0 from the last on).
+    // Added up and not multiplied out: the scalar instructions of a stage show (gradients at 1000 x 32000 x 768: 0.5 %).
+    const char *stageA = (const char*)(baseA + (size_t)kBegin * g.lda), *stageB = (const char*)(baseB + (size_t)kBegin * g.ldb);
+    long long stepA = (long long)(BK * sizeof(bf16_t)) * g.lda, stepB = (long long)(BK * sizeof(bf16_t)) * g.ldb;
+    auto advance = [&]() {
+        if (!AK) stageA += stepA;
+        if (!BKC) stageB += stepB;
+    };
     // before the last stage is fetched, once: the chunks past the end of the contraction
     auto lastStage = [&](int k0) {
         asm volatile("" ::: "memory");   // a branch, not a select in every stage
+        stepA = stepB = 0;
 #pragma unroll
         for (int p = 0; p < PA; p++) {
             const int e = p * NT + tid;
@@ -173,8 +186,15 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
     };
     // fetch p of a stage: this wavefront fills the 1 KB from chunk p NT + 64 wave on, lane i its i-th chunk
     auto fetch = [&](int p, int k0, bf16_t* stage) {
-        if (p < PA) lds_fetch16(rsA, stage + (p * NT + wave * 64) * 8, va[p], (AK ? k0 : k0 * g.lda) * 2);
-        else lds_fetch16(rsB, stage + BM * BK + ((p - PA) * NT + wave * 64) * 8, vb[p - PA], (BKC ? k0 : k0 * g.ldb) * 2);
+        if (p < PA) {
+            bf16_t* to = stage + (p * NT + wave * 64) * 8;
+            if (AK) lds_fetch16(rsA, to, va[p], k0 * 2);
+            else lds_fetch16(resource(stageA), to, va[p], 0);
+        } else {
+            bf16_t* to = stage + BM * BK + ((p - PA) * NT + wave * 64) * 8;
+            if (BKC) lds_fetch16(rsB, to, vb[p - PA], k0 * 2);
+            else lds_fetch16(resource(stageB), to, vb[p - PA], 0);
+        }
     };
 
     floatx16 acc[WM][WN];
@@ -221,6 +241,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
         const bf16_t* pb = pa + BM * BK;
         bf16_t* next = smem + ((kt & 1) ^ 1) * STAGE;   // read during stage kt - 1; free since the barrier that ended it
         const int k1 = kBegin + min(kt + 1, nk - 1) * BK;   // past the end the last stage is fetched again, never read
+        advance();
         if (kt + 2 == nk) lastStage(k1);
         const uint32_t stageAddr = smemAddr + (kt & 1) * STAGE * 2;
 #pragma unroll
@@ -378,8 +399,11 @@ bool gemm_b16_takes(const GemmB16& q)
     if ((((uintptr_t)q.A | (uintptr_t)q.B) & 15) != 0) return false;
     if (q.aK ? q.k % 8 != 0 : (q.m % 8 != 0 || q.m < 8)) return false;
     if (q.bK ? q.k % 8 != 0 : (q.n % 8 != 0 || q.n < 8)) return false;
-    // 31-bit byte offsets
-    return ((long long)(q.aK ? q.m : q.k) + 64) * (q.aK ? q.k : q.m) < (1ll << 30) && ((long long)(q.bK ? q.n : q.k) + 64) * (q.bK ? q.k : q.n) < (1ll << 30);
+    // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage
+    auto near = [&](bool kFast, int rows) {
+        return kFast ? ((long long)std::min(rows, 256) + 1) * q.k < (1ll << 30) : (long long)std::min(q.k, 64) * rows + 256 < (1ll << 30);
+    };
+    return near(q.aK, q.m) && near(q.bK, q.n);
 }
 size_t gemm_b16_workspace_bytes(int m, int n, int k)
 {
