@@ -1168,7 +1168,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(size_t rows, int 
     for (int r = 0; r < R; r++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            gv[r][i] = L::at(lane, r, i) >= end ? 0.f : logsm ? gv[r][i] - __expf(yv[r][i]) * sum : (gv[r][i] - sum) * yv[r][i];
+            gv[r][i] = L::at(lane, r, i) >= end ? 0.f : logsm ? gv[r][i] - expf(yv[r][i]) * sum : (gv[r][i] - sum) * yv[r][i];
     L::store(dx + row * len, lane, len, gv);
 }
 

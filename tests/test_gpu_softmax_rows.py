@@ -52,3 +52,17 @@ def test_explicit_chain_equals_the_attention_handle(dev, B, T, C, H):
         out.append([top.mutable_cpu_data, bx.mutable_cpu_diff] + [b.mutable_cpu_diff for b in layer.c_attn.blobs + layer.c_proj.blobs])
     for a, b in zip(*out):
         assert np.abs(a - b).max() <= 2e-5 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("length", [1, 37, 64, 255, 1024, 2047, 2048, 2049, 4100, 32769])
+def test_log_softmax_gradient_keeps_single_precision(dev, length):
+    """dx = g - exp(y) sum(g) with a gradient of one value per row, the last: everywhere else dx = -exp(y), off by no more than
+    the exponential (1 ulp) and its product with the sum, which is exactly 1 (2^-24 each way)."""
+    rng = np.random.default_rng(length)
+    y, g = -rng.uniform(0, 40, (3, length)).astype(np.float32), np.zeros((3, length), np.float32)
+    g[:, -1] = 1.0
+    hd, hc, d = dev.zeros(y.size), dev.cuda.CreateCuDNN(), dev.cuda.CreateTensorDesc()
+    dev.cuda.SetTensorDesc(d, 3, length, 1, 1, False)
+    dev.cuda.SoftmaxBackward(hc, 2, 0, 1.0, d, dev.put(y), d, dev.put(g), 0.0, d, hd)
+    want = -np.exp(y[:, :-1].astype(np.float64))
+    assert (np.abs(dev.get(hd, y.shape)[:, :-1] - want) <= 4 * 2.0 ** -24 * np.abs(want)).all()
