@@ -1144,10 +1144,12 @@ hipError_t k_softmax_masked(hipStream_t s, DType dt, const void* x, void* y, siz
 }
 
 // causalT != 0: y is the output of a softmax under the causal mask of causalT x causalT whose masked entries are exact zeros
-// unless *zeroFlag == epoch.  What lies above the diagonal is then neither read nor multiplied: its gradient is zero.
+// unless *zeroFlag == epoch.  What lies above the diagonal is then not read from y; dy is read whole, since an infinity or a
+// NaN in it reaches the row's sum through 0 x inf all the same (2 of 12 bytes an entry are saved, not 4).  Such a row's
+// gradient is NaN above the diagonal as well, and the flag is raised so that no later product takes it for zeros.
 template <typename T, int R, bool VEC>
 __global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(size_t rows, int len, const T* y, const T* dy, T* dx, bool logsm, int causalT,
-                                                               const int* zeroFlag, int epoch)
+                                                               int* zeroFlag, int epoch)
 {
     typedef RowInLanes<T, R, VEC> L;
     const int lane = threadIdx.x & 63;
@@ -1156,20 +1158,40 @@ __global__ __launch_bounds__(256) void softmax_bwd_wave_kernel(size_t rows, int 
     const int end = causalT && *zeroFlag != epoch ? (int)(row % (size_t)causalT) + 1 : len;
     float yv[R][4], gv[R][4];
     L::load(y + row * len, lane, end, 0.f, yv);
-    L::load(dy + row * len, lane, end, 0.f, gv);
+    L::load(dy + row * len, lane, len, 0.f, gv);
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (L::at(lane, r, i) < end) sum += logsm ? gv[r][i] : gv[r][i] * yv[r][i];
+        for (int i = 0; i < 4; i++) sum += logsm ? gv[r][i] : gv[r][i] * (L::at(lane, r, i) < end ? yv[r][i] : 0.f);   // zeros past the row
     sum = wave_sum(sum);
+    if (end < len && lane == 0 && !(fabsf(sum) < INFINITY)) *zeroFlag = epoch;
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            gv[r][i] = L::at(lane, r, i) >= end ? 0.f : logsm ? gv[r][i] - expf(yv[r][i]) * sum : (gv[r][i] - sum) * yv[r][i];
+            gv[r][i] = logsm ? gv[r][i] - expf(yv[r][i]) * sum : (gv[r][i] - sum) * (L::at(lane, r, i) < end ? yv[r][i] : 0.f);
     L::store(dx + row * len, lane, len, gv);
+}
+
+// raises the flag (*flag = epoch) if one of n values, 16-byte aligned, is infinite or no number
+__global__ __launch_bounds__(256) void flag_nonfinite_kernel(const float* __restrict__ x, size_t n, int* flag, int epoch)
+{
+    auto bad = [](float v) { return (int)((__float_as_uint(v) & 0x7f800000u) == 0x7f800000u); };
+    int any = 0;
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)256 * gridDim.x;
+    for (size_t i = t; i < n / 4; i += step) {
+        const float4 v = ((const float4*)x)[i];
+        any |= bad(v.x) | bad(v.y) | bad(v.z) | bad(v.w);
+    }
+    if (t < (n & 3)) any |= bad(x[(n & ~(size_t)3) + t]);
+    if (any) *flag = epoch;
+}
+hipError_t k_flag_nonfinite(hipStream_t s, const float* x, size_t n, int* flag, int epoch)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(flag_nonfinite_kernel, (int)std::min<size_t>((n / 4 + 1023) / 1024 + 1, 2048), 256, 0, s, x, n, flag, epoch);
+    return hipGetLastError();
 }
 
 // Rows of 2049 to 32768 values (a vocabulary): one workgroup of sixteen wavefronts per row, the row in registers between its
@@ -1301,7 +1323,7 @@ __global__ void softmax_bwd_kernel(int len, int inner, const T* y, const T* dy, 
 }
 
 hipError_t k_softmax_bwd(hipStream_t s, DType dt, const void* y, const void* dy, void* dx, size_t outer, int len, int inner, bool logsm,
-                         int causalT, const int* zeroFlag, int epoch)
+                         int causalT, int* zeroFlag, int epoch)
 {
     if (outer == 0 || len <= 0 || inner <= 0) return hipSuccess;
     const size_t series = outer * (size_t)inner;

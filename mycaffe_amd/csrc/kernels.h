@@ -63,9 +63,12 @@ hipError_t k_softmax_masked(hipStream_t s, DType dt, const void* x, void* y, siz
                             int* zeroFlag = nullptr, int epoch = 0);
 // gradient with respect to the softmax input from the output y and its gradient dy (dx may alias dy)
 // causalT: y is causal (rows of causalT over causalT queries, entries above the diagonal exact zeros unless *zeroFlag == epoch);
-// taken into account for inner == 1 and len <= 2048, where dx then has the same zeros (softmax_bwd_keeps_zeros)
+// taken into account for inner == 1 and len <= 2048, where dx then has the same zeros, or the flag is raised
+// (softmax_bwd_keeps_zeros)
 hipError_t k_softmax_bwd(hipStream_t s, DType dt, const void* y, const void* dy, void* dx, size_t outer, int len, int inner, bool logsm,
-                         int causalT = 0, const int* zeroFlag = nullptr, int epoch = 0);
+                         int causalT = 0, int* zeroFlag = nullptr, int epoch = 0);
+// *flag = epoch if one of n values at a 16-byte aligned address is infinite or no number
+hipError_t k_flag_nonfinite(hipStream_t s, const float* x, size_t n, int* flag, int epoch);
 inline bool softmax_bwd_keeps_zeros(int len, int inner) { return inner == 1 && len <= 2048; }
 // adjacent-pair rotary embedding with the CudaDnnDLL index rule; x == y allowed
 hipError_t k_rope(hipStream_t s, DType dt, size_t n, const void* x, void* y, const float* fcos, const float* fsin,

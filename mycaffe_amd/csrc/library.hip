@@ -908,7 +908,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         }
         // An operand is the output of a softmax with a causal mask folded in, or its gradient (P V and P^T dY, dS K and Q^T dS
         // of the explicit attention chain): on one side of the diagonal it holds exact zeros - the softmax kernel raises a
-        // flag on the device if it does not - and the contraction stops or begins at the diagonal.
+        // flag on the device if it does not - and the contraction stops or begins at the diagonal.  What is left out are products
+        // with zero: they are only zero if the other operand is finite, so that is looked at first and raises the same flag.
+        // The look takes a launch and a pass over the smaller operand, the contraction saves a third: from 2^28 flops on.
         const ZeroTag* tag = nullptr;
         bool causalA = false;
         if (!m_zeroTags.empty()) {
@@ -921,6 +923,11 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 const ZeroTag* t = zero_tag(h);
                 if (t && t->len == k && (unsigned long long)batch * k <= t->rows) { tag = t; causalA = op == 1; }
             }
+            const MemItem* other = causalA ? B : A;
+            const long long per = causalA ? bc * br : ac * ar;
+            const bool dense = causalA ? ldb == br && (batch == 1 || sB == per) : lda == ar && (batch == 1 || sA == per);
+            if (tag && (!dense || ((uintptr_t)other->ptr & 15) || 2ll * m * n * k * batch < (1ll << 28))) tag = nullptr;
+            if (tag) HIPCHK(k_flag_nonfinite(s, (const float*)other->ptr, (size_t)(per * batch), m_zeroFlags + tag->slot, tag->epoch));
         }
         HIPCHK(k_gemm2(s, tA, tB, m, n, k, alpha2, (const float*)A->ptr, (const float*)B->ptr, pf[1], (float*)C->ptr, lda,
                        ldb, ldc, sA, sB, sC, batch, tag ? m_zeroFlags + tag->slot : nullptr, tag ? tag->epoch : 0, false, causalA));

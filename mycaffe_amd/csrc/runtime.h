@@ -201,7 +201,7 @@ private:
     long m_heldMaskHandle = 0; uint64_t m_heldMaskVersion = 0; int m_heldMaskT = 0; bool m_heldMaskCausal = false;
     // Tensors whose entries above the diagonal of every (len, len) matrix are exact zeros: outputs of a softmax with a causal
     // mask folded in, and their gradients.  m_zeroFlags[slot] (device) holds `epoch` if a masked entry was not exactly zero
-    // after all.  A slot belongs to one softmax output and what was derived from it.
+    // after all, or what a product would multiply it by not finite.  A slot belongs to one softmax output and what was derived from it.
     struct ZeroTag { long handle; uint64_t version; int len; size_t rows; int slot, epoch; };
     enum { ZERO_SLOTS = 64 };
     std::vector<ZeroTag> m_zeroTags;

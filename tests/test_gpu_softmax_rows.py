@@ -66,3 +66,49 @@ def test_log_softmax_gradient_keeps_single_precision(dev, length):
     dev.cuda.SoftmaxBackward(hc, 2, 0, 1.0, d, dev.put(y), d, dev.put(g), 0.0, d, hd)
     want = -np.exp(y[:, :-1].astype(np.float64))
     assert (np.abs(dev.get(hd, y.shape)[:, :-1] - want) <= 4 * 2.0 ** -24 * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("where", ["none", "dy above the diagonal", "dy on the diagonal", "v", "k", "q", "weights"])
+def test_infinities_and_nan_spread_through_the_causal_zeros(dev, where):
+    """0 x inf: a masked weight or its gradient is an exact zero, and still carries an infinity or a NaN of what it is multiplied by
+    (sizes at which the products stop at the diagonal while everything is finite)."""
+    cuda, rng = dev.cuda, np.random.default_rng(3)
+    outer, T, hs = 32, 512, 64
+    sc, dy = (rng.standard_normal((outer, T, T)).astype(np.float32) for _ in range(2))
+    q, k, v = (rng.standard_normal((outer, T, hs)).astype(np.float32) for _ in range(3))
+    if where == "dy above the diagonal":
+        dy[3, 100, 400] = np.inf
+    elif where == "dy on the diagonal":
+        dy[3, 100, 100] = np.nan
+    elif where in "qkv":
+        {"q": q, "k": k, "v": v}[where][5, 17 if where == "q" else 500, 9] = -np.inf
+    hp, hs_, hm, hd = dev.zeros(sc.size), dev.put(sc), dev.put(np.tril(np.ones((T, T), np.float32))), dev.zeros(sc.size)
+    hc, d = cuda.CreateCuDNN(), cuda.CreateTensorDesc()
+    cuda.SetTensorDesc(d, outer * T, T, 1, 1, False)
+    cuda.scal(sc.size, 0.125, hs_)
+    cuda.mask(sc.size, T * T, 0.0, -1e9, hs_, hm, hs_)
+    cuda.SoftmaxForward(hc, 1, 0, 1.0, d, hs_, 0.0, d, hp)
+    if where == "weights":
+        cuda.set(1, hp, np.inf, 2 * T * T + 50 * T + 300)
+    hout = dev.zeros(q.size)
+    got, want = [], []
+    with np.errstate(all="ignore"):
+        masked = np.where(np.tril(np.ones((T, T))) == 0, -np.inf, sc.astype(np.float64) * 0.125)
+        p = np.exp(masked - masked.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        if where == "weights":
+            p[2, 50, 300] = np.inf
+        ds = (dy.astype(np.float64) - (dy * p).sum(-1, keepdims=True)) * p
+        for h, m, o, tA in ((hp, p, v, False), (hp, p, v, True), (hd, ds, k, False), (hd, ds, q, True)):
+            if h == hd and len(got) == 2:
+                cuda.SoftmaxBackward(hc, 1, 0, 1.0, d, hp, d, dev.put(dy), 0.0, d, hd)
+                got.append(dev.get(hd, sc.shape))
+                want.append(ds)
+            cuda.matmul(outer, T, hs, T, h, dev.put(o), hout, 1.0, tA, False)
+            got.append(dev.get(hout, o.shape))
+            want.append((m.transpose(0, 2, 1) if tA else m) @ o.astype(np.float64))
+    for i, (a, b) in enumerate(zip(got, want)):
+        finite = np.isfinite(b)
+        assert np.array_equal(np.isfinite(a), finite), (i, where)
+        assert np.array_equal(np.isnan(a), np.isnan(b)), (i, where)
+        assert np.abs(a[finite] - b[finite]).max() <= 2e-5 * np.abs(b[finite]).max(), (i, where)
