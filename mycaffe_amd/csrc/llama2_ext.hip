@@ -594,6 +594,7 @@ __global__ __launch_bounds__(NS * 64) void matvec_mfma_kernel(const T* __restric
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 template <typename T> struct StepSlab;
 template <> struct StepSlab<float> {
+    static constexpr bool SPLITS = false;
     static constexpr int PIECES = 2, XLANE = 16, XPIECE = 64;   // columns 16 half + 4 kk .. + 3 per piece
     typedef float X[8];
     __device__ static inline void split(const float (&v)[8], X& x)
@@ -611,6 +612,7 @@ template <> struct StepSlab<float> {
 };
 template <> struct StepSlab<bf16_t> {
     static constexpr int PIECES = 1, XLANE = 32, XPIECE = 16;   // columns 8 kk .. + 7
+    static constexpr bool SPLITS = true;
     struct X { bf16x8v p[3]; };
     __device__ static inline void split(const float (&v)[8], X& x)
     {
@@ -624,6 +626,21 @@ template <> struct StepSlab<bf16_t> {
                 x.p[q][e] = (__bf16)r[e];
                 if (q < 2) r[e] -= (float)x.p[q][e];
             }
+    }
+    // From 0x1.ffp127 on the nearest bf16 number is infinite and leaves infinity or NaN over, so that every result it enters is
+    // NaN.  Cut off instead, with nothing left over of an infinity, the three numbers are the value's own; of a NaN the
+    // remainders are NaN.
+    __device__ static inline void split_far(const float (&v)[8], X& x)
+    {
+        float r[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float h = __uint_as_float(__float_as_uint(v[e]) & 0xffff0000u);
+            x.p[0][e] = (__bf16)h;
+            r[e] = fabsf(v[e]) == INFINITY ? 0.f : v[e] - h;
+            x.p[1][e] = (__bf16)r[e];
+            x.p[2][e] = (__bf16)(r[e] - (float)x.p[1][e]);
+        }
     }
     __device__ static inline floatx4v mul(const uint4 (&w)[1], const X& x, floatx4v acc)
     {
@@ -667,14 +684,14 @@ __global__ __launch_bounds__(NS * 64) void matvec_step_kernel(StepArgs a)
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t] = floatx4v{0.f, 0.f, 0.f, 0.f};
     float ss = 0.f;
+    auto load8 = [&](const __amdgpu_buffer_rsrc_t r, int at, int slab, float (&o)[8]) {
+        const auto p0 = __builtin_amdgcn_raw_buffer_load_b128(r, at, slab * 128, 0), p1 = __builtin_amdgcn_raw_buffer_load_b128(r, at + S::XPIECE, slab * 128, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) { o[e] = __uint_as_float(p0[e]); o[4 + e] = __uint_as_float(p1[e]); }
+    };
     for (int base = wave; base < nit; base += NS * U) {
         uint4 w[U][NT][S::PIECES];
         float xv[U][8], gv[NORM ? U : 1][8];
-        auto load8 = [&](const __amdgpu_buffer_rsrc_t r, int at, int slab, float (&o)[8]) {
-            const auto p0 = __builtin_amdgcn_raw_buffer_load_b128(r, at, slab * 128, 0), p1 = __builtin_amdgcn_raw_buffer_load_b128(r, at + S::XPIECE, slab * 128, 0);
-#pragma unroll
-            for (int e = 0; e < 4; e++) { o[e] = __uint_as_float(p0[e]); o[4 + e] = __uint_as_float(p1[e]); }
-        };
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int sl = min(base + u * NS, nit - 1);   // past the end: the last slab once more, not used
@@ -703,6 +720,35 @@ __global__ __launch_bounds__(NS * 64) void matvec_step_kernel(StepArgs a)
             S::split(xv[u], x);
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[t] = S::mul(w[u][t], x, acc[t]);
+        }
+    }
+    if constexpr (S::SPLITS) {
+        // a NaN among the results: an activation too large for the split, or a NaN or infinities of its own.  Once more, slab by
+        // slab, with the split that takes those (one look at the end; at every slab it took 2 % of a generation).
+        float all = 0.f;   // NaN if one of them is (or if infinities of both signs are: then it is for nothing)
+#pragma unroll
+        for (int t = 0; t < NT; t++) all += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(all != all) != 0, 0)) {
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[t] = floatx4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int sl = wave; sl < nit; sl += NS) {
+                float xv[8], gv[8];
+                load8(rx, xo, sl, xv);
+                if (NORM) {
+                    load8(rg, kk * S::XLANE, sl, gv);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) xv[e] *= gv[e];
+                }
+                typename S::X x;
+                S::split_far(xv, x);
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rw[t], lane * 16, sl * SLAB, 0);
+                    const uint4 w[1] = {make_uint4(v[0], v[1], v[2], v[3])};
+                    acc[t] = S::mul(w, x, acc[t]);
+                }
+            }
         }
     }
     if (NORM) {

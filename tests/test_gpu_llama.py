@@ -623,3 +623,67 @@ def test_batched_step_over_every_reach_of_the_attention_workgroup(llm, tmp_path,
     for b in (0, 32):
         ref_ids, ref_logits = O.Llama(cfg, blob).generate_greedy(prompts[b], n, want_logits=True)
         _check_ids(out[b], ref_ids, ref_logits, "batch row %d" % b)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("B", [2, 5, 17])
+def test_logits_of_a_batched_step(llm, tmp_path, B, half):
+    """Logits of every decode step of a batch against the checker on the weights as they are stored, at fp32 tolerance: products
+    with 16-bit weights lose nothing of their fp32 activations."""
+    cfg = dict(dim=96, hidden_dim=1056, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=500, seq_len=64)
+    blob, views = O.random_weights(cfg, seed=31, shared_classifier=False, std=0.15)
+    views["rms_ffn"][...] = 1 + 0.3 * np.random.default_rng(4).standard_normal(views["rms_ffn"].shape).astype(np.float32)
+    path = str(tmp_path / "logits.bin")
+    O.write_checkpoint_v1(path, cfg, blob, False)
+    prompts, n = np.random.default_rng(B).integers(3, cfg["vocab_size"], (B, 3)), 20
+    llm.SetOption(1, 1 if half else 0)
+    llm.SetOption(7, 0)   # one step per position from the first on
+    try:
+        llm.Load(path)
+        ids, logits = llm.GenerateBatch(prompts, n, want_logits=True)
+    finally:
+        llm.SetOption(1, 0)
+        llm.SetOption(7, 1)
+    checker = O.Llama(cfg, _stored(blob, cfg) if half else blob)
+    for b in range(B):
+        ref_ids, ref_logits = checker.generate_greedy(prompts[b], n, want_logits=True)
+        _check_ids(ids[b], ref_ids, ref_logits, "batch row %d" % b)
+        assert_close(logits[b], ref_logits, FP32_RTOL, "batch row %d" % b)
+
+
+def _stored(blob, cfg):
+    """The weights as 16-bit storage holds them: matrices rounded, norm weights kept."""
+    out, off = bf16_round(blob), 0
+    for name, shape in O.tensor_shapes(cfg, False):
+        size = int(np.prod(shape))
+        if name.startswith("rms"):
+            out[off:off + size] = blob[off:off + size]
+        off += size
+    return out
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_batched_step_with_an_activation_past_the_largest_bf16(llm, tmp_path, half):
+    """One hidden unit is 1.9963 x 2^127: a finite fp32 number whose nearest bf16 number is infinite.  w2 takes it by 2^-126."""
+    cfg = dict(dim=64, hidden_dim=64, n_layers=1, n_heads=4, n_kv_heads=4, vocab_size=64, seq_len=32)
+    blob, v = O.random_weights(cfg, seed=5, shared_classifier=False, std=0.1)
+    v["tok_emb"][...] = 1.0
+    v["tok_emb"][:, 32:] = -1.0
+    for name in ("wo", "w1", "w2", "w3"):
+        v[name][...] = 0.0
+    v["w1"][0, 7, 3], v["w3"][0, 7, 3], v["w2"][0, 11, 7] = 1.15625 * 2.0 ** 64, 1.7265625 * 2.0 ** 63, 2.0 ** -126
+    blob = bf16_round(blob)
+    path = str(tmp_path / "far.bin")
+    O.write_checkpoint_v1(path, cfg, blob, False)
+    prompts, n = np.arange(12).reshape(4, 3) + 3, 6
+    ref_ids, ref_logits = O.Llama(cfg, blob).generate_greedy(prompts[0], n, want_logits=True)
+    assert np.isfinite(ref_logits).all()
+    llm.SetOption(1, 1 if half else 0)
+    llm.SetOption(7, 0)
+    try:
+        llm.Load(path)
+        ids, logits = llm.GenerateBatch(prompts, n, want_logits=True)
+    finally:
+        llm.SetOption(1, 0)
+        llm.SetOption(7, 1)
+    assert_close(logits[0], ref_logits, FP32_RTOL, "logits")
