@@ -340,7 +340,7 @@ enum {
      *                 -> f{batch x nSteps next ids [, logits with option 6]}
      *   QUERY_TIMING  f{hLlm} -> f{ms of the timed span (HIP events), steps in it, 1 if the steps were
      *                 replays of the captured graph / 0 if they were launched eagerly, ms of the batched
-     *                 prompt pass (0 if none ran), sequences x prompt positions it covered}
+     *                 prompt pass (0 if none ran), sequences x prompt positions it covered, steps captured so far}
      *   PROFILE_STEP  f{hLlm, pos, reps[, batch]} -> per kernel class of one decode step
      *                 f{ms per step, launches per step, algorithmic bytes per step}, classes in
      *                 the order qkv mat-vec, rope+cache store, decode attention, wo, w1|w3,

@@ -1564,6 +1564,7 @@ public:
     bool stored_bf16 = false;    // storage of the weights that are on the device now: every launch dispatches on this
     bool use_graph = true;
     bool lastUsedGraph = false;  // whether the last generate replayed a captured graph (false: eager launches)
+    int captures = 0;            // steps captured so far
     bool use_prefill = true;     // prompt positions as one batched pass (false: one decode step per position)
     bool prefill_act16 = false;  // 16-bit weights, many prompt rows: activations of the pass rounded to bf16 (false: kept to sixteen bits)
     bool device_sampling = true; // temperature / top-p on the device (false: logits to the host every step)
@@ -1633,10 +1634,18 @@ private:
     GenState* dstate = nullptr;
     int *dprompt = nullptr, *dnext = nullptr, *dcur = nullptr, *dout = nullptr;
     int *dcount = nullptr, *dticket = nullptr;   // attention merge tickets (B * heads) and the step ticket; zero between launches
-    hipGraphExec_t graphExec = nullptr;
-    int graphB = 0, graphReach = 0;
-    int graphTail = 1;                           // the tail the captured step ends with (see step), and the sampler
-    float graphTemperature = 0.f, graphTopp = 0.f;   // parameters captured with tail 2
+    // captured steps over the current state, one per reach of the attention, tail (see step) and, with tail 2, sampler
+    // parameters: generations whose lengths differ find theirs again (capturing and instantiating one takes 0.3 ms,
+    // as much as a step)
+    struct StepGraph { hipGraphExec_t exec; int reach, tail; float temperature, topp; };
+    enum { MAX_GRAPHS = 16 };
+    std::vector<StepGraph> graphs;
+    int graphB = 0;                              // sequences of the captured steps (-1: they are out of date)
+    void drop_graphs()
+    {
+        for (StepGraph& g : graphs) (void)hipGraphExecDestroy(g.exec);
+        graphs.clear();
+    }
     float sampleTemperature = 1.f, sampleTopp = 0.9f;
     unsigned long long* drng = nullptr;          // state of the device sampler's random stream
     int* dgiven = nullptr;                       // ids chosen by the host sampler (one per sequence)
@@ -1653,7 +1662,7 @@ private:
 void Engine::release()
 {
     if (stream) (void)hipStreamSynchronize(stream);
-    if (graphExec) { (void)hipGraphExecDestroy(graphExec); graphExec = nullptr; }
+    drop_graphs();
     if (hLogits) { (void)hipHostFree(hLogits); hLogits = nullptr; hLogitsCount = 0; }
     if (hGiven) { (void)hipHostFree(hGiven); hGiven = nullptr; }
     for (void* p : stateAllocs) (void)hipFree(p);
@@ -1855,7 +1864,7 @@ long Engine::ensure_state(int B, int nSteps)
 {
     if (B == stateB && nSteps <= stateSteps) return 0;
     HIPCHK(hipStreamSynchronize(stream));
-    if (graphExec) { (void)hipGraphExecDestroy(graphExec); graphExec = nullptr; }
+    drop_graphs();
     if (hLogits) { (void)hipHostFree(hLogits); hLogits = nullptr; hLogitsCount = 0; }
     if (hGiven) { (void)hipHostFree(hGiven); hGiven = nullptr; }
     for (void* p : stateAllocs) (void)hipFree(p);
@@ -2485,23 +2494,33 @@ long Engine::generate(const int* prompts, int B, int nPrompt, int nSteps, bool w
     const hipEvent_t evA = sc.evA, evB = sc.evB;
     const int t0 = timedFrom < 0 ? nPrompt : timedFrom;
     bool graph = use_graph && !wantLogits;
-    if (graph && (!graphExec || graphB != B || graphReach != step_reach(nSteps) || graphTail != tail || (tail == 2 && (graphTemperature != sampleTemperature || graphTopp != sampleTopp)))) {
-        // one decode step, captured once; position / tokens are device-side so the graph is replayed as is
-        if (graphExec) { (void)hipGraphExecDestroy(graphExec); graphExec = nullptr; }
-        hipGraph_t g = nullptr;
-        hipError_t he = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-        if (he == hipSuccess) {
-            e = enqueue();
-            he = hipStreamEndCapture(s, &g);
-            if (e == 0 && he == hipSuccess) he = hipGraphInstantiate(&graphExec, g, nullptr, nullptr, 0);
-            if (g) (void)hipGraphDestroy(g);
-        }
-        if (e || he != hipSuccess || !graphExec) { graphExec = nullptr; graph = false; e = 0; }
+    hipGraphExec_t graphExec = nullptr;
+    if (graph) {
+        if (graphB != B) drop_graphs();
         graphB = B;
-        graphReach = step_reach(nSteps);
-        graphTail = tail;
-        graphTemperature = sampleTemperature;
-        graphTopp = sampleTopp;
+        const int reach = step_reach(nSteps);
+        for (const StepGraph& c : graphs)
+            if (c.reach == reach && c.tail == tail && (tail != 2 || (c.temperature == sampleTemperature && c.topp == sampleTopp))) graphExec = c.exec;
+        if (!graphExec) {
+            // one decode step, captured once; position / tokens are device-side so the graph is replayed as is
+            hipGraph_t g = nullptr;
+            hipError_t he = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+            if (he == hipSuccess) {
+                e = enqueue();
+                he = hipStreamEndCapture(s, &g);
+                if (e == 0 && he == hipSuccess) he = hipGraphInstantiate(&graphExec, g, nullptr, nullptr, 0);
+                if (g) (void)hipGraphDestroy(g);
+            }
+            if (e || he != hipSuccess || !graphExec) { graphExec = nullptr; graph = false; e = 0; }
+            else {
+                if (graphs.size() >= MAX_GRAPHS) {
+                    (void)hipGraphExecDestroy(graphs.front().exec);
+                    graphs.erase(graphs.begin());
+                }
+                graphs.push_back(StepGraph{graphExec, reach, tail, sampleTemperature, sampleTopp});
+                captures++;
+            }
+        }
     }
     lastUsedGraph = graph;
     // The forced prompt positions in one batched pass.  The reference flips a coin at every position, forced ones
@@ -2797,7 +2816,7 @@ MCH_LONG DLL_InvokeFloatCustomExtension(MCH_LONG fn, float* pIn, MCH_LONG lIn, f
         std::shared_ptr<Llm> m = find_llm((long)pIn[0]);
         if (!m) return MCH_ERROR_PARAM;
         return (MCH_LONG)give({m->engine.lastTimedMs, (float)m->engine.lastTimedSteps, m->engine.lastUsedGraph ? 1.f : 0.f,
-                                m->engine.lastPrefillMs, (float)m->engine.lastPrefillRows}, ppOut, plOut);
+                                m->engine.lastPrefillMs, (float)m->engine.lastPrefillRows, (float)m->engine.captures}, ppOut, plOut);
     }
     case MCH_LLM_PROFILE_STEP: {
         if (lIn < 3) return MCH_ERROR_PARAM_OUT_OF_RANGE;

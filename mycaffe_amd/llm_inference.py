@@ -136,6 +136,11 @@ class LlmInference:
         rg = self.m_cuda.RunExtension(self.m_hExtension, CUDAFN_EXTENSION_LLM.QUERY_TIMING, self.m_rgLlm)
         return bool(rg[2] != 0)
 
+    def GraphCaptures(self):
+        """Decode steps captured into graphs since the model was created: one per reach of the attention, sampler setting and
+        number of sequences, kept while the number of sequences stays."""
+        return int(self.m_cuda.RunExtension(self.m_hExtension, CUDAFN_EXTENSION_LLM.QUERY_TIMING, self.m_rgLlm)[5])
+
     def LastPrefill(self):
         """(milliseconds, rows) of the batched prompt pass of the last generation: HIP-event time on the engine's stream
         and sequences x prompt positions covered; (0, 0) when the prompt went one decode step per position."""

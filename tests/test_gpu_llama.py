@@ -687,3 +687,51 @@ def test_batched_step_with_an_activation_past_the_largest_bf16(llm, tmp_path, ha
         llm.SetOption(1, 0)
         llm.SetOption(7, 1)
     assert_close(logits[0], ref_logits, FP32_RTOL, "logits")
+
+
+def test_generations_of_different_lengths_keep_their_graphs(llm, tmp_path):
+    """One captured step per reach of the attention, found again by later generations; captured anew for another number of
+    sequences or after an option that changes the step; never more than a bounded number kept."""
+    cfg = dict(dim=64, hidden_dim=128, n_layers=2, n_heads=4, n_kv_heads=4, vocab_size=512, seq_len=600)
+    blob, _ = O.random_weights(cfg, seed=3, std=0.2)
+    path = str(tmp_path / "lengths.bin")
+    O.write_checkpoint_v1(path, cfg, blob, False)
+    llm.Load(path)
+    prompts = np.random.default_rng(1).integers(3, cfg["vocab_size"], (3, 5))
+    ref, ref_logits = O.Llama(cfg, blob).generate_greedy(prompts[0], 600, want_logits=True)
+    before = llm.GraphCaptures()
+    for n in (20, 60, 20, 32, 64, 33, 300, 60, 600, 300, 20):
+        _check_ids(llm.GenerateIds(prompts[0], n), ref[:n], ref_logits[:n], "%d positions" % n)
+        assert llm.LastRunUsedGraph()
+    assert llm.GraphCaptures() - before == 4          # up to 32, 64, 512 and 600 positions
+    llm.SetOption(4, 1)
+    _check_ids(llm.GenerateIds(prompts[0], 20), ref[:20], ref_logits[:20], "after an option")
+    assert llm.GraphCaptures() - before == 5
+    for _ in range(2):
+        for n in (20, 60):
+            out = llm.GenerateBatch(prompts, n)
+            _check_ids(out[0], ref[:n], ref_logits[:n], "of a batch")
+    assert llm.GraphCaptures() - before == 7
+    _check_ids(llm.GenerateIds(prompts[0], 60), ref[:60], ref_logits[:60], "alone again")
+    assert llm.GraphCaptures() - before == 8
+
+
+def test_every_reach_keeps_a_graph(tmp_path):
+    """All ten reaches of a context of 640, taken twice in turn with eager generations in between."""
+    blob, _ = O.random_weights(TINY, seed=4, shared_classifier=False, std=0.25)
+    ckpt = str(tmp_path / "m.bin")
+    O.write_checkpoint_v1(ckpt, dict(TINY, seq_len=640), blob, False)
+    cuda = CudaDnn(0)
+    inf = LlmInference(cuda)
+    inf.Initialize(fTemperature=0.0)
+    inf.Load(ckpt)
+    lengths = [32 * i for i in range(1, 9)] + [300, 600]
+    ref = O.Llama(dict(TINY, seq_len=640), blob).generate_greedy([1, 17, 300], 600)
+    for _ in range(2):
+        for n in lengths:
+            for graph in (1, 0):
+                inf.SetOption(3, graph)
+                assert np.array_equal(inf.GenerateIds([1, 17, 300], n), ref[:n]), (n, graph)
+    assert inf.GraphCaptures() == len(lengths)
+    inf.CleanUp()
+    cuda.Dispose()
