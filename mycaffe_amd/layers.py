@@ -185,6 +185,23 @@ class InnerProductLayer:
                                  self.blobs[0].gpu_diff, self.blobs[1].gpu_diff if self.bias_term else 0, bottom.gpu_diff, accumulate)
 
 
+class _Kept(dict):
+    """What a layer builds for a shape and needs again when the shape comes back: the last few, the oldest given back."""
+
+    MAX = 8
+
+    def __init__(self, free):
+        super().__init__()
+        self._free = free
+
+    def get_or(self, key, make):
+        if key not in self:
+            while len(self) >= self.MAX:
+                self._free(self.pop(next(iter(self))))
+            self[key] = make()
+        return self[key]
+
+
 class TransposeLayer:
     """MyCaffe.layers.beta/layers.beta/TransposeLayer.cs:127-232."""
 
@@ -337,6 +354,7 @@ class CausalSelfAttentionLayer:
         self.blobMask = Blob(cuda, (1, 1, block_size, block_size))
         mask = np.tril(np.ones((block_size, block_size), np.float32))  # fillMask :276-291
         self.blobMask.mutable_cpu_data = mask
+        self._masks, self._ropes = _Kept(Blob.Dispose), _Kept(cuda.FreeRope)
         self.hCudnn = self.hAttn = self.hRope = 0
         self._set_for = None
 
@@ -355,14 +373,19 @@ class CausalSelfAttentionLayer:
                 self.hAttn = self.cuda.CreateAttn()
             self.cuda.SetAttn(self.hCudnn, self.hAttn, 0, self.training, B, self.nBlockSize, self.nHeads, self.nSize, 0.0)
         if self.enable_rope:
-            if self.hRope:
-                self.cuda.FreeRope(self.hRope)
-            self.hRope = self.cuda.CreateRope(0, 0, B * T * self.nEmbed, B, T, self.nHeads, self.nSize, self.rope_theta)
-        if T != self.nBlockSize and not self.enable_sdpa:
+            self.hRope = self._ropes.get_or((B, T), lambda: self.cuda.CreateRope(0, 0, B * T * self.nEmbed, B, T, self.nHeads, self.nSize, self.rope_theta))
+        self._set_for = (B, T)
+
+    def _mask(self, T):
+        """The causal mask of T positions: the layer's own, or one of the last few of shorter sequences."""
+        if T == self.nBlockSize:
+            return self.blobMask
+
+        def make():
             m = Blob(self.cuda, (1, 1, T, T))
             m.mutable_cpu_data = np.tril(np.ones((T, T), np.float32))
-            self.blobMaskT = m
-        self._set_for = (B, T)
+            return m
+        return self._masks.get_or(T, make)
 
     def Forward(self, blobX, top):
         B, T, C = blobX.shape_[:3]
@@ -386,14 +409,7 @@ class CausalSelfAttentionLayer:
                 out.Reshape(B, T, C)
             else:
                 out.ReshapeLike(b["Vt"])
-            mask = self.blobMask
-            if T != self.nBlockSize:
-                # the handle reads a (1,1,T,T) mask for the block size it is run with
-                if getattr(self, "_sdpa_mask_T", None) != T:
-                    self.blobMaskSdpa = Blob(cuda, (1, 1, T, T))
-                    self.blobMaskSdpa.mutable_cpu_data = np.tril(np.ones((T, T), np.float32))
-                    self._sdpa_mask_T = T
-                mask = self.blobMaskSdpa
+            mask = self._mask(T)   # the handle reads a (1,1,T,T) mask for the block size it is run with
             if self.fused_qkv_heads:
                 cuda.AttnScaledDotProductForward(self.hCudnn, self.hAttn, T, b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data,
                                                  mask.gpu_data, out.gpu_data, False, T, True)
@@ -406,7 +422,7 @@ class CausalSelfAttentionLayer:
             dfScale = 1.0 / math.sqrt(hs)
             b["AttA"].MatMul(b["Qt"], b["Kt1"], bReshape=True)
             b["AttA"].scale_data(dfScale)
-            mask = self.blobMask if T == self.nBlockSize else self.blobMaskT
+            mask = self._mask(T)
             cuda.mask(b["AttA"].count(), mask.count(), 0.0, self.dfIgnoreVal, b["AttA"].gpu_data, mask.gpu_data, b["AttA"].gpu_data)
             self.softmax.Forward(b["AttA"], b["AttB"])
             b["Work"].MatMul(b["AttB"], b["Vt"], bReshape=True)
@@ -588,6 +604,7 @@ class LayerNormLayer:
     def __init__(self, cuda, epsilon=1e-10, enable_cuda_impl=True):
         self.cuda, self.epsilon, self.enable_cuda_impl = cuda, epsilon, enable_cuda_impl
         self.hLayerNorm = 0
+        self._kept = _Kept(cuda.FreeLayerNorm)
         self._shape = None
         self.b = {n: Blob(cuda) for n in "Mu Xmu XmuSq Var Stdev StdevFull Work".split()}
 
@@ -598,9 +615,8 @@ class LayerNormLayer:
         if self._shape == bottom.shape_:
             return
         if self.enable_cuda_impl:
-            if self.hLayerNorm:
-                self.cuda.FreeLayerNorm(self.hLayerNorm)
-            self.hLayerNorm = self.cuda.CreateLayerNorm(0, self.nCount, self.nOuterNum, self.nChannels, self.nInnerNum, self.epsilon)
+            self.hLayerNorm = self._kept.get_or(tuple(bottom.shape_), lambda: self.cuda.CreateLayerNorm(
+                0, self.nCount, self.nOuterNum, self.nChannels, self.nInnerNum, self.epsilon))
         else:
             for n in ("Xmu", "XmuSq", "StdevFull"):
                 self.b[n].ReshapeLike(bottom)
