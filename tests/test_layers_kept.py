@@ -2,14 +2,14 @@
 is allocated and given back."""
 import numpy as np
 
-from mycaffe_amd.layers import Blob, CausalSelfAttentionLayer, LayerNormLayer, TransposeLayer, _Kept
+from mycaffe_amd.layers import Blob, CausalSelfAttentionLayer, InnerProductLayer, LayerNormLayer, TransposeLayer, _Kept
 
 
 class Context:
     DTYPE = np.float32
 
     def __init__(self):
-        self.live, self.made, self.next = {}, 0, 1
+        self.live, self.made, self.next, self.calls = {}, 0, 1, []
 
     def _make(self, kind):
         self.made += 1
@@ -32,7 +32,7 @@ class Context:
     FreeMemory = FreeLayerNorm = FreeRope = _free
 
     def __getattr__(self, name):
-        return lambda *a, **k: 0   # every other call does nothing
+        return lambda *a, **k: self.calls.append(name) or 0   # every other call is only noted
 
 
 def test_kept_things_are_bounded_and_given_back():
@@ -78,3 +78,14 @@ def test_transposes_of_many_shapes_are_bounded():
         x.Reshape(2, T, 2, 8)
         layer.Forward(x, y)
     assert len(cuda.live) <= 2 + 4 * TransposeLayer.MAX_SHAPES + 1
+
+
+def test_a_single_fp32_row_goes_through_gemv_whatever_its_layout():
+    for half, M, want in ((False, 1, ["gemv", "axpy"]), (False, 2, ["LinearForward"]), (True, 1, ["LinearForward"])):
+        cuda = Context()
+        layer, x, y = InnerProductLayer(cuda, 16, half=half), Blob(cuda, (1, M, 8), half), Blob(cuda, half=half)
+        layer.Setup(x)
+        for forward in (lambda: layer.Forward(x, y), lambda: layer.ForwardHeads(x, y, 4)):
+            cuda.calls.clear()
+            forward()
+            assert cuda.calls == want, (half, M, cuda.calls)
