@@ -948,14 +948,14 @@ hipError_t k_rmsnorm_bwd(hipStream_t s, DType dt, int rows, int dim, const void*
 // by the rotation of their position when the tables are given.  One pass where the chain has three transposes, two rotations
 // and three channel copies; V elements a thread (16 bytes where the head size and the addresses allow it).
 template <typename T, int V>
-__global__ void qkv_heads_grad_kernel(uint32_t pieces, const T* dq, const T* dk, const T* dv, T* dx, uint32_t Tn, uint32_t H, uint32_t hs,
+__global__ void qkv_heads_grad_kernel(uint32_t row0, uint32_t pieces, const T* dq, const T* dk, const T* dv, T* dx, uint32_t Tn, uint32_t H, uint32_t hs,
                                       const float* __restrict__ fcos, const float* __restrict__ fsin, uint32_t seq)
 {
     const uint32_t C = H * hs, perRow = 3 * C / V;
     for (uint32_t p = blockIdx.x * TPB + threadIdx.x; p < pieces; p += TPB * gridDim.x) {
-        const uint32_t row = p / perRow, col = (p - row * perRow) * V, which = col / C, w = col - which * C, h = w / hs, d = w - h * hs;
-        const uint32_t b = row / Tn, t = row - b * Tn;
-        const T* src = (which == 0 ? dq : which == 1 ? dk : dv) + ((size_t)(b * H + h) * Tn + t) * hs + d;
+        const uint32_t r = p / perRow, col = (p - r * perRow) * V, which = col / C, w = col - which * C, h = w / hs, d = w - h * hs;
+        const uint32_t row = row0 + r, b = row / Tn, t = row - b * Tn;
+        const T* src = (which == 0 ? dq : which == 1 ? dk : dv) + (((size_t)b * H + h) * Tn + t) * hs + d;
         float v[V];
         if constexpr (V == 4) Vec4<T>::load(src, v);
         else
@@ -983,19 +983,25 @@ __global__ void qkv_heads_grad_kernel(uint32_t pieces, const T* dq, const T* dk,
 hipError_t k_qkv_heads_grad(hipStream_t s, DType dt, int B, int Tn, int H, int hs, const void* dq, const void* dk, const void* dv, void* dx,
                             const float* fcos, const float* fsin, int seq)
 {
-    const size_t n = (size_t)B * Tn * 3 * H * hs, es = dt == F32 ? 4 : 2;
-    if (n == 0) return hipSuccess;
-    if (n > 0xf0000000ull || (fcos && (hs & 1))) return hipErrorInvalidValue;
+    const size_t rows = (size_t)B * Tn, perRow = (size_t)3 * H * hs, es = dt == F32 ? 4 : 2;
+    if (rows == 0 || perRow == 0) return hipSuccess;
+    if (rows > 0x7fffffffu || perRow > 0x7fffffffu || (fcos && (hs & 1))) return hipErrorInvalidValue;
     const bool aligned = (((uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv | (uintptr_t)dx) & (4 * es - 1)) == 0;
     const int V = hs % 4 == 0 && aligned ? 4 : hs % 2 == 0 ? 2 : 1;
-    const uint32_t pieces = (uint32_t)(n / V);
-#define QKV_GRAD(VV) DISPATCH_DT(dt, hipLaunchKernelGGL((qkv_heads_grad_kernel<T, VV>), grid_for(pieces), TPB, 0, s, pieces, (const T*)dq, (const T*)dk, \
-                                                        (const T*)dv, (T*)dx, (uint32_t)Tn, (uint32_t)H, (uint32_t)hs, fcos, fsin, (uint32_t)(seq > 0 ? seq : 1)))
-    if (V == 4) QKV_GRAD(4);
-    else if (V == 2) QKV_GRAD(2);
-    else QKV_GRAD(1);
+    // a launch numbers its pieces in 32 bits: as many rows as that allows at a time
+    const size_t most = std::max<size_t>(1, 0xe0000000ull / (perRow / V));
+    for (size_t r0 = 0; r0 < rows; r0 += most) {
+        const uint32_t pieces = (uint32_t)(std::min(most, rows - r0) * (perRow / V));
+#define QKV_GRAD(VV) DISPATCH_DT(dt, hipLaunchKernelGGL((qkv_heads_grad_kernel<T, VV>), grid_for(pieces), TPB, 0, s, (uint32_t)r0, pieces, (const T*)dq, \
+                                                        (const T*)dk, (const T*)dv, (T*)dx, (uint32_t)Tn, (uint32_t)H, (uint32_t)hs, fcos, fsin, (uint32_t)(seq > 0 ? seq : 1)))
+        if (V == 4) QKV_GRAD(4);
+        else if (V == 2) QKV_GRAD(2);
+        else QKV_GRAD(1);
 #undef QKV_GRAD
-    return hipGetLastError();
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // ---------------------------------------------------------------------------

@@ -2232,7 +2232,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         // l{batch, T, heads, hs, hdQ, hdK, hdV, hdX[, hRope]}
         NEED_L(8, 9);
         const long long B = pl[0], T = pl[1], H = pl[2], hs = pl[3];
-        if (B < 1 || T < 1 || H < 1 || hs < 1 || B * T > INT_MAX || 3 * H * hs > INT_MAX || B * T * 3 * H * hs > 0xf0000000ll) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        if (B < 1 || T < 1 || H < 1 || hs < 1 || B * T > INT_MAX || 3 * H * hs > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         const long long n = B * T * H * hs;
         MemItem *dQ, *dK, *dV, *dX;
         ERRCHK(mem((long)pl[4], &dQ));
