@@ -654,6 +654,10 @@ static size_t gemm_heads_workspace_bytes(DType dt, int m, int n, int kk, const v
     if (dt == F32) return gemm_f32_workspace_bytes(m, n, kk, 1, false);
     return gemm_b16_takes(b16_product(false, true, m, n, kk, 1.f, X, W, 0.f, nullptr)) ? gemm_b16_workspace_bytes(m, n, kk) : (size_t)m * n * sizeof(bf16_t);
 }
+bool k_gemm_bias_needs_workspace(DType dt, int m, int n, int k, const void* X, const void* W)
+{
+    return dt != F32 && !gemm_b16_takes(b16_product(false, true, m, n, k, 1.f, X, W, 0.f, nullptr));
+}
 size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W)
 {
     return gemm_heads_workspace_bytes(dt, m, n, k, X, W);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <stdlib.h>
 
 namespace mch {
 
@@ -28,6 +29,14 @@ __host__ __device__ inline bf16_t f32_to_bf16(float f)
         return (bf16_t)((c.u >> 16) | 0x40);
     uint32_t r = 0x7fffu + ((c.u >> 16) & 1u);
     return (bf16_t)((c.u + r) >> 16);
+}
+
+// the largest scratch allocation a kernel object makes, in bytes: no limit, or MYCAFFE_HIP_SCRATCH_LIMIT of the environment at
+// its creation
+inline size_t scratch_limit()
+{
+    const char* v = getenv("MYCAFFE_HIP_SCRATCH_LIMIT");
+    return v && *v ? (size_t)strtoull(v, nullptr, 10) : SIZE_MAX;
 }
 
 // ---- elementwise and layout kernels (ew_kernels.hip) ----------------------
@@ -131,6 +140,8 @@ hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void*
 hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, int k, const void* X, const void* W, const void* bias, void* Y,
                              void* ws, size_t wsBytes);   // Y as (B,H,T,hs); scratch as k_gemm_bias
 size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W);
+// whether the call fails without that scratch (otherwise its contraction stays in one part)
+bool k_gemm_bias_needs_workspace(DType dt, int m, int n, int k, const void* X, const void* W);
 size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W);
 // column-major strided batched gemm with BLAS semantics (fp32)
 // C (fp32) = alpha X W^T + beta C on the bf16 matrix cores: W 16-bit (n x k), k % 64 == 0; A is X as bf16 (m x k) or,

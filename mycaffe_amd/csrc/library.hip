@@ -255,6 +255,7 @@ std::string Kernel::device_name()
 long Kernel::workspace(size_t bytes, void** p)
 {
     if (bytes > m_wsBytes) {
+        if (bytes > m_wsLimit) return MCH_ERROR_MEMORY_OUT;
         if (m_ws) { HIPCHK(hipStreamSynchronize(m_stream)); HIPCHK(hipFree(m_ws)); m_ws = nullptr; m_wsBytes = 0; }
         size_t want = bytes < (size_t)(8u << 20) ? (size_t)(8u << 20) : bytes + bytes / 4;
         HIPCHK(hipMalloc(&m_ws, want));
@@ -262,6 +263,15 @@ long Kernel::workspace(size_t bytes, void** p)
     }
     *p = m_ws;
     return 0;
+}
+// scratch for a product that does without if there is none (its contraction then stays in one part): *bytes becomes what there is
+void Kernel::workspace_or_none(size_t* bytes, void** p)
+{
+    *p = nullptr;
+    if (!*bytes || !workspace(*bytes, p)) return;
+    (void)hipGetLastError();
+    *p = nullptr;
+    *bytes = 0;
 }
 
 long Kernel::tickets(size_t count, int** p)
@@ -330,8 +340,8 @@ long Kernel::flush_pending_product(bool causal)
     if (m_mem.get(p.hA, &A) || m_mem.get(p.hB, &B) || m_mem.get(p.hC, &C)) return 0;   // an operand is gone
     if (p.kind == 1) {
         void* ws = nullptr;
-        const size_t wsb = k_gemm_workspace_bytes(C->dt(), false, true, p.m, p.n, p.k);
-        if (wsb) ERRCHK(workspace(wsb, &ws));
+        size_t wsb = k_gemm_workspace_bytes(C->dt(), false, true, p.m, p.n, p.k);
+        workspace_or_none(&wsb, &ws);
         HIPCHK(k_gemm(m_stream, C->dt(), false, true, p.m, p.n, p.k, p.alpha, A->ptr, B->ptr, 0.f, C->ptr, ws, wsb));
         return 0;
     }
@@ -802,8 +812,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 if (!m_mem.get(p.hA, &X) && !m_mem.get(p.hB, &W) && !m_mem.get(p.hC, &C) && C->half == A->half) {
                     m_pendingProduct = PendingProduct();
                     void* ws = nullptr;
-                    const size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr);
-                    if (wsb) ERRCHK(workspace(wsb, &ws));
+                    size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr);
+                    if (k_gemm_bias_needs_workspace(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
+                    else workspace_or_none(&wsb, &ws);
                     HIPCHK(k_gemm_bias(s, C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws, wsb));
                     m_mem.touch(hC);
                     return 0;
@@ -840,8 +851,8 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             RANGE(C, co, (long long)m * n);
             // the transpose combinations of the layers' backward passes turn an operand in scratch memory
             void* ws = nullptr;
-            const size_t wsb = k_gemm_workspace_bytes(A->dt(), tA, tB, m, n, k);
-            if (wsb) ERRCHK(workspace(wsb, &ws));
+            size_t wsb = k_gemm_workspace_bytes(A->dt(), tA, tB, m, n, k);
+            workspace_or_none(&wsb, &ws);
             HIPCHK(k_gemm(s, A->dt(), tA, tB, m, n, k, pf[0], PTR(A, ao), PTR(B, bo), pf[1], PTR(C, co), ws, wsb));
         }
         m_mem.touch((long)pl[9]);
@@ -2155,8 +2166,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             }
         }
         void* ws = nullptr;
-        const size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr);
-        if (wsb) ERRCHK(workspace(wsb, &ws));
+        size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr);
+        if (k_gemm_bias_needs_workspace(X->dt(), (int)M, (int)(3 * C), (int)C, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
+        else workspace_or_none(&wsb, &ws);
         HIPCHK(k_gemm_qkv_heads(s, X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Q->ptr, K->ptr,
                                 V->ptr, ws, wsb, r ? (const float*)r->dcos.get() : nullptr, r ? (const float*)r->dsin.get() : nullptr,
                                 r ? r->seq : 0));
@@ -2185,8 +2197,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
         void* ws = nullptr;
-        const size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr);
-        if (wsb) ERRCHK(workspace(wsb, &ws));
+        size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr);
+        if (k_gemm_bias_needs_workspace(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
+        else workspace_or_none(&wsb, &ws);
         if (heads)
             HIPCHK(k_gemm_bias_heads(s, X->dt(), (int)(M / T), (int)T, (int)heads, (int)(N / heads), (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
         else HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
@@ -2219,10 +2232,12 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         const size_t wsW = k_gemm_workspace_bytes(dt, true, false, (int)N, (int)K, (int)M), wsB = dB ? k_bias_grad_workspace_bytes((int)M, (int)N) : 0;
         const size_t wsX = dX ? k_gemm_workspace_bytes(dt, false, false, (int)M, (int)K, (int)N) : 0, most = std::max(wsW, std::max(wsB, wsX));
         void* ws = nullptr;
-        if (most) ERRCHK(workspace(most, &ws));
-        HIPCHK(k_gemm(s, dt, true, false, (int)N, (int)K, (int)M, 1.f, dY->ptr, X->ptr, 1.f, dW->ptr, ws, wsW));
-        if (dB) HIPCHK(k_bias_grad(s, dt, (int)M, (int)N, dY->ptr, dB->ptr, ws, wsB));
-        if (dX) HIPCHK(k_gemm(s, dt, false, false, (int)M, (int)K, (int)N, 1.f, dY->ptr, W->ptr, accum ? 1.f : 0.f, dX->ptr, ws, wsX));
+        size_t have = most;
+        workspace_or_none(&have, &ws);
+        if (have < wsB) { have = wsB; ERRCHK(workspace(wsB, &ws)); }   // the products do without, the column sums do not
+        HIPCHK(k_gemm(s, dt, true, false, (int)N, (int)K, (int)M, 1.f, dY->ptr, X->ptr, 1.f, dW->ptr, ws, have));
+        if (dB) HIPCHK(k_bias_grad(s, dt, (int)M, (int)N, dY->ptr, dB->ptr, ws, have));
+        if (dX) HIPCHK(k_gemm(s, dt, false, false, (int)M, (int)K, (int)N, 1.f, dY->ptr, W->ptr, accum ? 1.f : 0.f, dX->ptr, ws, have));
         m_mem.touch((long)pl[6]);
         if (dB) m_mem.touch((long)pl[7]);
         if (dX) m_mem.touch((long)pl[8]);

@@ -882,9 +882,11 @@ private:
     HandleTable<RopeD> m_rope;
     HandleTable<LayerNormD> m_layernorm;
     double* m_ws = nullptr; size_t m_wsCount = 0;   // scratch of the attention backward call
+    const size_t m_wsLimit = scratch_limit();
     long workspace(size_t count, double** p)
     {
         if (count > m_wsCount) {
+            if (count * sizeof(double) > m_wsLimit) return MCH_ERROR_MEMORY_OUT;
             if (m_ws) { HIPCHK(hipStreamSynchronize(m_stream)); HIPCHK(hipFree(m_ws)); m_ws = nullptr; m_wsCount = 0; }
             HIPCHK(hipMalloc((void**)&m_ws, count * sizeof(double)));
             m_wsCount = count;
@@ -1990,10 +1992,13 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         int kind = 0;
         ERRCHK(attn_mask_kind(st, M, batchMask, T, Tk, &kind));
         const long long bh = (long long)st->batch * st->heads, rows = bh * T, pn = rows * Tk;
-        if (bh <= 65535 && rows <= INT_MAX && pn <= (1ll << 28)) {
+        double* P = nullptr;
+        if (bh <= 65535 && rows <= INT_MAX && pn <= (1ll << 28) && workspace((size_t)pn, &P)) {
+            (void)hipGetLastError();
+            P = nullptr;
+        }
+        if (P) {
             // scores, softmax and product as three launches, the probabilities in scratch memory
-            double* P;
-            ERRCHK(workspace((size_t)pn, &P));
             ERRCHK(attn_probs(Q->ptr, K->ptr, P, st, T, Tk, M, kind));
             const long long sp = (long long)T * Tk, sk = (long long)Tk * st->hs, hs = st->hs;
             if (merged) HIPCHK(d_gemm(s, (int)bh, T, (int)hs, Tk, 1.0, P, Tk, 1ll, V->ptr, hs, 1ll, 0.0, Y->ptr, st->heads * hs, 1ll, sp, sk,

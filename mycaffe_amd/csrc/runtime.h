@@ -175,6 +175,7 @@ public:
 private:
     long attn_decode_fwd(float* pf, long lf, MCH_LONGLONG* pl, long ll, bool staticScratch);
     long workspace(size_t bytes, void** p);
+    void workspace_or_none(size_t* bytes, void** p);
     long staging(size_t bytes, void** p);
     long tickets(size_t count, int** p);
     long mem(long h, MemItem** it);                                            // with any deferred scaling applied
@@ -221,6 +222,7 @@ private:
     HandleTable<BlobLoaderState> m_blobLoader;
     std::map<int, std::weak_ptr<void>> m_ropeSharedCos, m_ropeSharedSin;
     void* m_ws = nullptr; size_t m_wsBytes = 0;          // device scratch (split-K partials, conversions)
+    size_t m_wsLimit = scratch_limit();
     int* m_tickets = nullptr; size_t m_ticketCount = 0;  // split-K merge tickets; zero whenever no kernel is running
     void* m_stage = nullptr; size_t m_stageBytes = 0;    // pinned host staging
     std::mutex m_stageLock;
