@@ -1621,6 +1621,7 @@ private:
     void* wclsP = nullptr;
     char* packArena = nullptr;
     size_t packWanted = 0, packUsed = 0;
+    bool packEach = false;
     template <typename T> void* pack_matrix(const void* W, size_t rows, size_t n, size_t second = 0);
     template <typename T> void pack_all();
     std::vector<LayerW<void>> layers;
@@ -1754,9 +1755,14 @@ template <typename T> void* Engine::pack_matrix(const void* W, size_t rows, size
     if (n % 32 != 0 || rows == 0) return nullptr;
     const size_t tiles = (rows + 15) / 16, per = tiles * 16 * n;
     const size_t bytes = ((second ? 2 : 1) * per * sizeof(T) + 255) / 256 * 256;
-    if (!packArena) { packWanted += bytes; return nullptr; }   // first round: sizes only
-    void* P = packArena + packUsed;
-    packUsed += bytes;
+    void* P;
+    if (packEach) {
+        if (!(P = dalloc(bytes))) { (void)hipGetLastError(); return nullptr; }
+    } else {
+        if (!packArena) { packWanted += bytes; return nullptr; }   // first round: sizes only
+        P = packArena + packUsed;
+        packUsed += bytes;
+    }
     for (int m = 0; m < (second ? 2 : 1); m++) {
         const size_t pieces = per * sizeof(T) / 16;
         const int grid = (int)std::min<size_t>((pieces + 255) / 256, 65535);
@@ -1769,13 +1775,16 @@ template <typename T> void Engine::pack_all()
 {
     const size_t dim = cfg.dim, hid = cfg.hidden_dim, hs = dim / cfg.n_heads, kvd = hs * cfg.n_kv_heads;
     packed.assign(layers.size(), LayerW<void>{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr});
-    // all copies in one allocation: dozens of small ones are mapped in small pages
+    // all copies in one allocation: dozens of small ones are mapped in small pages.  Where that much is not to be had in one
+    // piece, each copy for itself as far as the memory goes.
     packArena = nullptr;
+    packEach = false;
     packWanted = packUsed = 0;
     for (int round = 0; round < 2; round++) {
         if (round) {
-            packArena = packWanted ? (char*)dalloc(packWanted) : nullptr;
-            if (!packArena) { (void)hipGetLastError(); break; }
+            if (!packWanted) break;
+            packArena = packWanted <= scratch_limit() ? (char*)dalloc(packWanted) : nullptr;
+            if (!packArena) { (void)hipGetLastError(); packEach = true; }
         }
         for (size_t l = 0; l < layers.size(); l++) {
             packed[l].wqkv = pack_matrix<T>(layers[l].wqkv, dim + 2 * kvd, dim);

@@ -735,3 +735,22 @@ def test_every_reach_keeps_a_graph(tmp_path):
     assert inf.GraphCaptures() == len(lengths)
     inf.CleanUp()
     cuda.Dispose()
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_packed_weights_one_by_one(llm, tmp_path, monkeypatch, half):
+    """The packed copies of the matrices in one allocation and, where that is not to be had, each for itself: the same kernels, so
+    the same logits to the bit."""
+    blob, _ = O.random_weights(C1, seed=13, std=0.05)
+    path = str(tmp_path / "pack.bin")
+    O.write_checkpoint_v1(path, C1, blob, False)
+    prompts, out = np.random.default_rng(2).integers(3, C1["vocab_size"], (3, 4)), []
+    llm.SetOption(1, 1 if half else 0)
+    try:
+        for limit in ("", "1000000"):
+            monkeypatch.setenv("MYCAFFE_HIP_SCRATCH_LIMIT", limit)
+            llm.Load(path)
+            out.append(llm.GenerateBatch(prompts, 20, want_logits=True))
+    finally:
+        llm.SetOption(1, 0)
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
