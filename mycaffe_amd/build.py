@@ -5,7 +5,7 @@
 Outputs (next to this file, git-ignored):
     libmycaffe_hip.so          the CudaDnnDLL-compatible C ABI (include/mycaffe_hip_abi.h)
     libmycaffe_hip_llama2.so   the llama2 extension library loaded through CREATE_EXTENSION
-    _hostcall.so               CPython module that packs the arguments of the Python mirror's calls (plain g++)
+    _hostcall.<tag>.so         CPython module that packs the arguments of the Python mirror's calls (plain g++)
 and, beside their sources, two C++ host programs built on include/mycaffe_hip_host.hpp (plain g++, they only
 dlopen the libraries): tests/cpp/host_parity (parity) and host_bench/csa_layer_bench (whole-layer wall clock).
 """
@@ -91,7 +91,8 @@ def build(force=False, verbose=True):
 
 
 def hostcall_path():
-    return os.path.join(HERE, "_hostcall.so")
+    """With this interpreter's tag: a file built under another Python is another file."""
+    return os.path.join(HERE, "_hostcall" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def build_hostcall(force=False, verbose=True):

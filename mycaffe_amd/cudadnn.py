@@ -12,7 +12,10 @@ There is no CPU fallback: constructing :class:`CudaDnn` loads the HIP library an
 fails loudly when it is missing.
 """
 import ctypes
+import importlib.util
 import os
+import subprocess
+import warnings
 
 import numpy as np
 
@@ -201,15 +204,23 @@ def llama2_extension_path():
 
 
 def _hostcall():
-    """The native module that packs the arguments of a call (csrc/hostcall.cpp), built first only when no built file exists."""
+    """The native module that packs the arguments of a call (csrc/hostcall.cpp), built first only when no built file exists; None
+    where it cannot be built or loaded: calls then go through ctypes, which takes the host several times as long (a block of the smallest size 1.8 ms against 0.34)."""
     global _host
     if _host is None:
-        if not os.path.exists(_build.hostcall_path()):
-            _build.build_hostcall(verbose=False)
-        from . import _hostcall as module
-        module.set_error_class(CudaDnnError)
-        _host = module
-    return _host
+        path = _build.hostcall_path()
+        try:
+            if not os.path.exists(path):
+                _build.build_hostcall(verbose=False)
+            spec = importlib.util.spec_from_file_location("mycaffe_amd._hostcall", path)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            module.set_error_class(CudaDnnError)
+            _host = module
+        except (ImportError, OSError, subprocess.CalledProcessError) as e:
+            warnings.warn("host calls go through ctypes: %s" % e)
+            _host = False
+    return _host or None
 
 
 _host = None
@@ -223,7 +234,6 @@ def load_library(path=None):
     if not os.path.exists(path):
         raise FileNotFoundError("HIP library not built: %s" % path)
     lib = ctypes.CDLL(path)
-    _hostcall()
     lib.DLL_InvokeFloat.argtypes = [_c_long, _c_long, _c_float_p, _c_long, ctypes.POINTER(_c_float_p),
                                     ctypes.POINTER(_c_long), _c_tchar_p, _c_long]
     lib.DLL_InvokeFloat.restype = _c_long
@@ -284,7 +294,8 @@ class CudaDnn:
 
     def __init__(self, nDeviceID=0, flags=DEVINIT.CUBLAS | DEVINIT.CURAND, lSeed=None, strPath=None):
         self._lib = load_library(strPath)
-        self._call = _hostcall().invoke
+        host = _hostcall()
+        self._call = host.invoke if host else None
         self._addr = ctypes.cast(getattr(self._lib, self._INVOKE_EX2), ctypes.c_void_p).value
         self._double = self.DTYPE is np.float64
         self.Path = strPath or default_library_path()
@@ -388,6 +399,8 @@ class CudaDnn:
 
     def _ex2(self, fn, rgf, rgl):
         """One Ex2 call whose arguments are a few Python numbers and whose result, if any, is a handful of values."""
+        if self._call is None:
+            return tuple(self.RunFloatEx2(self.m_hKernel, fn, rgf, rgl))
         return self._call(self._addr, self._double, self.m_hKernel, fn, rgf, rgl)
 
     # ---- lifetime / device ------------------------------------------------------

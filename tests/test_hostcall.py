@@ -52,3 +52,36 @@ def test_errors_are_raised():
     with pytest.raises(ValueError):
         call(addr, False, 1, 2, None, list(range(65)))
     del keep
+
+
+def test_the_built_file_carries_the_interpreters_tag():
+    import sysconfig
+
+    from mycaffe_amd import build
+    assert build.hostcall_path().endswith("_hostcall" + sysconfig.get_config_var("EXT_SUFFIX"))
+    assert cudadnn._hostcall().__file__ == build.hostcall_path()
+
+
+@pytest.mark.parametrize("how", ["no compiler", "no module"])
+def test_without_the_module_calls_go_through_ctypes(monkeypatch, tmp_path, how):
+    import subprocess
+
+    from mycaffe_amd import build
+    path = tmp_path / "_hostcall.so"
+    if how == "no module":
+        path.write_bytes(b"built for something else")
+
+    def fails(verbose=True):
+        raise subprocess.CalledProcessError(1, "g++")
+    monkeypatch.setattr(cudadnn, "_host", None)
+    monkeypatch.setattr(build, "hostcall_path", lambda: str(path))
+    monkeypatch.setattr(build, "build_hostcall", fails)
+    with pytest.warns(UserWarning, match="ctypes"):
+        assert cudadnn._hostcall() is None
+    seen = []
+    keep, _ = _entry(ctypes.c_float, seen, outs=(7.0, 2.5))
+    cuda = object.__new__(cudadnn.CudaDnn)
+    cuda._call, cuda.m_hKernel, cuda._lib = None, 3, type("Lib", (), {"DLL_InvokeFloatEx2": staticmethod(keep)})
+    assert cuda._ex2(220, [0.5], [1, 2]) == (7.0, 2.5)
+    assert seen == [(3, 220, [0.5], [1, 2])]
+    cuda.m_hKernel = 0   # nothing to clean up
