@@ -34,7 +34,10 @@ struct GemmB16Args {
 
 // One operand fragment.  The transposing reads are written as instructions: as builtins the compiler makes each of them wait
 // for every fetch into LDS that is under way, the next stage's included (8000 x 768 x 3072 with one such operand: 109 us).
-// tr_read issues the two reads of k-step ks (ROWB bytes between k rows), tr_wait makes the values usable.
+// tr_read issues the two reads of k-step ks (ROWB bytes between k rows), tr_wait makes the values usable.  In between the
+// compiler takes the registers for written: should it copy, spill or reuse one before the wait, the old contents would go on.
+// It has no reason to (every fragment is read once, by the product after its wait), and what it makes of this file is checked:
+// tests/test_asm_pending_reads.py finds no instruction that names a pending register, in any of the kernels.
 struct TrFragment { union { u32x4 w; uint2 h[2]; }; };
 template <int ROWB> __device__ __forceinline__ void tr_read(uint32_t addr, int ks, TrFragment& o)
 {
