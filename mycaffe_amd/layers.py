@@ -832,7 +832,7 @@ class TransformerBlockLayer:
 
     def __init__(self, cuda, heads, embed, block_size, activation="relu", bias_term=True, epsilon=1e-10,
                  enable_cuda_scaled_dot_product_attention=True, training=False, enable_llama_style_head=False, hidden_dim=0,
-                 multiple_of=64, enable_layernorm_cuda_impl=True, fused_rmsnorm=False, block_type="causal_self_attention",
+                 multiple_of=64, enable_layernorm_cuda_impl=True, fused_rmsnorm=None, block_type="causal_self_attention",
                  enable_key_value_cache=False):
         if block_type not in ("causal_self_attention", "encoder"):
             raise ValueError(block_type)
@@ -841,9 +841,9 @@ class TransformerBlockLayer:
         self.llama = enable_llama_style_head
         if self.llama:
             # RMSNorm, rotary attention without bias, SiLU-gated MLP (TransformerBlockLayer.cs:86-98, 239-247, 860-875)
-            # (the norms of a block are always the single calls; the argument stays for its callers)
-            self.norm1 = RMSNormLayer(cuda, epsilon, True, True)
-            self.norm2 = RMSNormLayer(cuda, epsilon, True, True)
+            # (the norms as single calls, unless fused_rmsnorm is False: then the layer's own chain)
+            self.norm1 = RMSNormLayer(cuda, epsilon, True, fused_rmsnorm is not False)
+            self.norm2 = RMSNormLayer(cuda, epsilon, True, fused_rmsnorm is not False)
             if hidden_dim == 0:
                 hidden_dim = 2 * (4 * embed) // 3
                 hidden_dim = multiple_of * ((hidden_dim + multiple_of - 1) // multiple_of)

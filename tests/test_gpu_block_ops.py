@@ -572,3 +572,32 @@ def test_explicit_chain_with_held_back_calls_matches_the_fused_handle_at_a_large
             att = layer.b["AttA"].mutable_cpu_data.reshape(B, H, T, T)
             assert np.all(att[:, :, 0, 1:] == np.float32(-1e29))
     assert_close(grads[False], grads[True], 5e-5, "input gradient, explicit chain against fused handle")
+
+
+@pytest.mark.parametrize("sdpa", [True, False])
+def test_llama_style_block_with_the_norms_as_chain_and_as_single_calls(dev, sdpa):
+    """fused_rmsnorm=False runs the layer's own chain of primitives inside the block, forward and backward: the same result."""
+    rng = np.random.default_rng(86)
+    B, T, C, H = 3, 10, 32, 2
+    x, dy = (rng.standard_normal((B, T, C)).astype(np.float32) for _ in range(2))
+    out, p = [], None
+    for fused in (False, True, None):
+        layer = TransformerBlockLayer(dev.cuda, H, C, T, "silu", False, 1e-5, sdpa, training=True, enable_llama_style_head=True, multiple_of=8,
+                                      fused_rmsnorm=fused)
+        assert layer.norm1.fused == layer.norm2.fused == (fused is not False)
+        hid = layer.fc1.N
+        if p is None:
+            p = {n: (rng.standard_normal(s) * 0.2 + (n[:3] == "rms")).astype(np.float32)
+                 for n, s in dict(rms1_weight=C, rms2_weight=C, attn_weight=(3 * C, C), attn_proj_weight=(C, C), fc_weight=(hid, C),
+                                  fc2_weight=(hid, C), proj_weight=(C, hid)).items()}
+        bx, top = Blob(dev.cuda, x.shape), Blob(dev.cuda, x.shape)
+        bx.mutable_cpu_data, top.mutable_cpu_diff = x, dy
+        layer.Setup(bx, p)
+        layer.Forward(bx, top)
+        layer.Backward(top, bx)
+        blobs = layer.attn1.c_attn.blobs + layer.attn1.c_proj.blobs + layer.fc1.blobs + layer.fc2.blobs + layer.proj.blobs + layer.norm1.blobs + layer.norm2.blobs
+        out.append([top.mutable_cpu_data, bx.mutable_cpu_diff] + [b.mutable_cpu_diff for b in blobs])
+    for a, b, c in zip(*out):
+        assert np.abs(b).max() > 0
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+        assert np.array_equal(b, c)
