@@ -171,10 +171,10 @@ def test_gemm_bf16_large_tile_paths(dev, m, n, k, alpha, beta):
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("tA,tB", [(False, False), (True, False), (True, True)])
 @pytest.mark.parametrize("m,n,k,beta", [
-    (1024, 768, 512, 0.0),      # data gradient shape: large enough in fp32 for the operand to be turned in scratch memory
+    (1024, 768, 512, 0.0),      # data gradient shape
     (768, 512, 2048, 1.0),      # weight gradient shape, accumulated into the result (beta = 1)
     (264, 200, 136, 0.5),       # ragged tiles, multiples of eight
-    (260, 132, 72, 0.0),        # multiples of four only: 16-bit storage keeps the strided kernel
+    (260, 132, 72, 0.0),        # multiples of four only: 16-bit storage takes the generic kernel
 ])
 def test_gemm_backward_transpose_combinations(dev, half, tA, tB, m, n, k, beta):
     """The transpose combinations of InnerProductLayer.backward (InnerProductLayer.cs:429-494) at sizes where an operand
