@@ -68,20 +68,20 @@ def test_log_softmax_gradient_keeps_single_precision(dev, length):
     assert (np.abs(dev.get(hd, y.shape)[:, :-1] - want) <= 4 * 2.0 ** -24 * np.abs(want)).all()
 
 
+@pytest.mark.parametrize("outer,T,hs,at", [(32, 512, 64, (5, 500, 9)), (3, 1023, 63, (-1, -1, -1))])   # the second: no whole quads, last value
 @pytest.mark.parametrize("where", ["none", "dy above the diagonal", "dy on the diagonal", "v", "k", "q", "weights"])
-def test_infinities_and_nan_spread_through_the_causal_zeros(dev, where):
+def test_infinities_and_nan_spread_through_the_causal_zeros(dev, where, outer, T, hs, at):
     """0 x inf: a masked weight or its gradient is an exact zero, and still carries an infinity or a NaN of what it is multiplied by
     (sizes at which the products stop at the diagonal while everything is finite)."""
     cuda, rng = dev.cuda, np.random.default_rng(3)
-    outer, T, hs = 32, 512, 64
     sc, dy = (rng.standard_normal((outer, T, T)).astype(np.float32) for _ in range(2))
     q, k, v = (rng.standard_normal((outer, T, hs)).astype(np.float32) for _ in range(3))
     if where == "dy above the diagonal":
-        dy[3, 100, 400] = np.inf
+        dy[2, 100, 400] = np.inf
     elif where == "dy on the diagonal":
-        dy[3, 100, 100] = np.nan
+        dy[2, 100, 100] = np.nan
     elif where in "qkv":
-        {"q": q, "k": k, "v": v}[where][5, 17 if where == "q" else 500, 9] = -np.inf
+        {"q": q, "k": k, "v": v}[where][(at[0], 17, at[2]) if where == "q" else at] = -np.inf
     hp, hs_, hm, hd = dev.zeros(sc.size), dev.put(sc), dev.put(np.tril(np.ones((T, T), np.float32))), dev.zeros(sc.size)
     hc, d = cuda.CreateCuDNN(), cuda.CreateTensorDesc()
     cuda.SetTensorDesc(d, outer * T, T, 1, 1, False)
