@@ -179,7 +179,7 @@ enum {
      * QKV_PROJ_HEADS replaces the head of CausalSelfAttentionLayer.forward (CausalSelfAttentionLayer.cs:526-557):
      * the fused InnerProduct, its bias GEMM, the three channel copies and the three head transposes become one
      * GEMM whose epilogue adds the bias and writes q, k, v as (batch, heads, T, hs):
-     *   l{batch, T, heads, hs, hX, hWeight (3C x C), hBias (0 = none), hQ, hK, hV [, hRope]}
+     *   l{batch, T, heads, hs, hX, hWeight (3C x C), hBias (0 = none), hQ, hK, hV [, hRope [, fp32Sums]]}
      * With hRope (a CREATE_ROPE handle of the same heads and hs) the epilogue also rotates q and k, which replaces the
      * two ROPE_FWD calls the layer makes between the channel copies and the transposes (:538-545).
      * Together with the 11th value of ATTN_FWD (Y written head-merged) the layer forward is four calls:
@@ -187,10 +187,12 @@ enum {
      *
      * LINEAR_FWD replaces the two GEMM calls of InnerProductLayer.forward (InnerProductLayer.cs:372-417: the product
      * with the transposed weight, then the rank-1 update with the vector of ones) by one GEMM whose epilogue adds
-     * the bias:  l{M, N, K, hX (M x K), hWeight (N x K), hBias (N; 0 = none), hY (M x N) [, T, heads]}.
+     * the bias:  l{M, N, K, hX (M x K), hWeight (N x K), hBias (N; 0 = none), hY (M x N) [, T, heads [, fp32Sums]]}.
      * With T and heads, Y is written head by head as (M/T, heads, T, N/heads): the projections of a multi-head attention layer
      * without the transposes behind them (MultiheadAttentionLayer.cs:650-690).
      * With it the causal self attention layer's forward is three calls.
+     * fp32Sums (T and heads may then be 0): in float storage the sums are those of the fp32 matrix cores at every size, not those of
+     * three bf16 parts per value, whose error is smaller and whose last bits are others.  No effect on other storage.
      *
      * LINEAR_BWD replaces the GEMM, GEMV and GEMM calls of InnerProductLayer.backward (InnerProductLayer.cs:429-494):
      * dW += dY^T X, db += column sums of dY, dX = dY W (accumX: dX += dY W):

@@ -577,7 +577,7 @@ static bool launch_wide_if_fits(hipError_t* e, hipStream_t s, int m, int n, int 
     }
     return false;
 }
-// fp32: one round of 256 x 288 tiles where 128 x 128 tiles, two to a CU, would leave their last round mostly empty (8192 x
+// fp32 sums (GemmF32): one round of 256 x 288 tiles where 128 x 128 tiles, two to a CU, would leave their last round mostly empty (8192 x
 // 2304 x 768: 213 us, 214 us with the bias, against 226 us as three rounds of 128 x 192 and 232 us as 128 x 128); elsewhere
 // the tiles of gemm_f32.hip cover the chip as well and hide their ends under a second workgroup.
 template <bool HEADS>
@@ -669,13 +669,13 @@ size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, c
 
 // Y: row-major result, only the bias of `he` is added; null: through `he`
 static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int kk, const void* X, const void* W, const HeadsEpilogue& he, void* Y,
-                                      void* ws, size_t wsBytes)
+                                      void* ws, size_t wsBytes, bool fp32Sums)
 {
     if (dt == F32) {
         hipError_t fit;
-        if (Y ? launch_wide_f32_if_fits<false>(&fit, s, m, n, kk, 1.f, X, W, Y, &he)
-              : he.hs % 4 == 0 && (((uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0 &&
-                    launch_wide_f32_if_fits<true>(&fit, s, m, n, kk, 1.f, X, W, he.dst[0], &he)) return fit;
+        if (fp32Sums && (Y ? launch_wide_f32_if_fits<false>(&fit, s, m, n, kk, 1.f, X, W, Y, &he)
+                           : he.hs % 4 == 0 && (((uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0 &&
+                                 launch_wide_f32_if_fits<true>(&fit, s, m, n, kk, 1.f, X, W, he.dst[0], &he))) return fit;
         GemmF32 g = {};
         g.m = m; g.n = n; g.k = kk;
         g.A = (const float*)X; g.B = (const float*)W;
@@ -685,6 +685,7 @@ static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int
         g.C = (float*)Y;
         if (Y) g.bias = (const float*)he.bias;
         else g.heads = &he;
+        g.fp32Sums = fp32Sums;
         return gemm_f32(s, g, ws, wsBytes);
     }
     hipError_t fit;
@@ -706,32 +707,33 @@ static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int
 }
 
 hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* bias,
-                            void* q, void* k, void* v, void* ws, size_t wsBytes, const float* fcos, const float* fsin, int ropeSeq)
+                            void* q, void* k, void* v, void* ws, size_t wsBytes, const float* fcos, const float* fsin, int ropeSeq, bool fp32Sums)
 {
     if (fcos && (!fsin || ropeSeq < 1 || (hs & 1))) return hipErrorInvalidValue;
     const int m = B * T, C = H * hs, n = 3 * C, kk = C;
     if (m <= 0 || C <= 0) return hipSuccess;
     const HeadsEpilogue he = heads_epilogue(bias, q, k, v, T, H, hs, fcos, fcos ? fsin : nullptr, fcos ? ropeSeq : 1);
-    return gemm_heads_dispatch(s, dt, m, n, kk, X, W, he, nullptr, ws, wsBytes);
+    return gemm_heads_dispatch(s, dt, m, n, kk, X, W, he, nullptr, ws, wsBytes, fp32Sums);
 }
 
 // Y (m x n) = X (m x k) W^T (n x k) + bias (n): the inner product layer's forward in one launch (InnerProductLayer.cs:
 // 372-417 issues the product and a rank-1 update with a vector of ones).  (One head of n values over m positions, for the
 // pass that splits a product the tile kernels do not take.)
-hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes)
+hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes,
+                       bool fp32Sums)
 {
     if (m <= 0 || n <= 0) return hipSuccess;
     const HeadsEpilogue he = heads_epilogue(bias, Y, Y, Y, m, 1, n, nullptr, nullptr, 1);
-    return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, Y, ws, wsBytes);
+    return gemm_heads_dispatch(s, dt, m, n, k, X, W, he, Y, ws, wsBytes, fp32Sums);
 }
 
 // the same, Y written head by head: position t of sequence b and column h hs + d go to Y[b][h][t][d] (m = B T, n = H hs)
 hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, int k, const void* X, const void* W, const void* bias, void* Y,
-                             void* ws, size_t wsBytes)
+                             void* ws, size_t wsBytes, bool fp32Sums)
 {
     if (B <= 0 || T <= 0 || H <= 0 || hs <= 0) return hipSuccess;
     const HeadsEpilogue he = heads_epilogue(bias, Y, Y, Y, T, H, hs, nullptr, nullptr, 1);
-    return gemm_heads_dispatch(s, dt, B * T, H * hs, k, X, W, he, nullptr, ws, wsBytes);
+    return gemm_heads_dispatch(s, dt, B * T, H * hs, k, X, W, he, nullptr, ws, wsBytes, fp32Sums);
 }
 
 // C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
@@ -800,8 +802,6 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
 {
     if (m <= 0 || n <= 0) return hipSuccess;
     if (dt == F32 && k > 1 && !gemm_is_tiny(m, n, k)) {
-        hipError_t e;
-        if (!tA && tB && beta == 0.f && launch_wide_f32_if_fits<false>(&e, s, m, n, k, alpha, A, B, C)) return e;
         GemmF32 g = {};
         g.m = m; g.n = n; g.k = k;
         g.A = (const float*)A; g.B = (const float*)B; g.C = (float*)C;
@@ -1013,6 +1013,7 @@ hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float a
     g.lda = ldb; g.ldb = lda; g.ldc = ldc; g.sA = sB; g.sB = sA; g.sC = sC;
     g.aK = !tB; g.bK = tA;
     g.alpha = alpha; g.beta = beta; g.batch = batch;
+    g.fp32Sums = !tA && !tB;   // MatMul; the products of its gradient have a transposed operand
     if (causalFlag) { g.causal = causalA ? (tA ? CAUSAL_B_UPPER : CAUSAL_B_LOWER) : (tB ? CAUSAL_A_UPPER : CAUSAL_A_LOWER); g.flag = causalFlag; g.epoch = epoch; }
     return gemm_f32(s, g, nullptr, 0);
 }

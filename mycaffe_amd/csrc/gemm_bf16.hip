@@ -30,33 +30,10 @@ struct GemmB16Args {
     const bf16_t* bias;
 };
 
-#define LDS3(p) ((__attribute__((address_space(3))) void*)(p))
-
-// One operand fragment.  The transposing reads are written as instructions: as builtins the compiler makes each of them wait
-// for every fetch into LDS that is under way, the next stage's included (8000 x 768 x 3072 with one such operand: 109 us).
-// tr_read issues the two reads of k-step ks (ROWB bytes between k rows), tr_wait makes the values usable.  In between the
-// compiler takes the registers for written: should it copy, spill or reuse one before the wait, the old contents would go on.
-// It has no reason to (every fragment is read once, by the product after its wait), and what it makes of this file is checked:
-// tests/test_asm_pending_reads.py finds no instruction that names a pending register, in any of the kernels.
-struct TrFragment { union { u32x4 w; uint2 h[2]; }; };
-template <int ROWB> __device__ __forceinline__ void tr_read(uint32_t addr, int ks, TrFragment& o)
-{
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(o.h[0]) : "v"(addr), "n"(ks * 16 * ROWB) : "memory");
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(o.h[1]) : "v"(addr), "n"((ks * 16 + 4) * ROWB) : "memory");
-}
-__device__ __forceinline__ void tr_wait(TrFragment& o) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o.h[0]), "+v"(o.h[1]) : : "memory"); }
-
 // sixteen bytes per lane from the buffer to the wavefront's 1 KB of LDS at `lds` (wavefront-uniform)
 __device__ __forceinline__ void lds_fetch16(__amdgpu_buffer_rsrc_t rs, bf16_t* lds, uint32_t voffset, int soffset)
 {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS3(lds), 16, voffset, soffset, 0, 0);
-}
-
-// exchange of 32-row blocks (64 bytes, four 16-byte chunks) in row k of a [k][row] stage: four consecutive k of one block of
-// rows have to lie on four different quarters of the 256 bytes of banks; rows are ROWB bytes apart
-template <int ROWB> __device__ __forceinline__ int block_swizzle(int k)
-{
-    return ROWB % 256 == 0 ? (k & 3) * 4 : ((k >> 1) & 1) * 4;   // in chunks; rows 128 bytes apart modulo 256 alternate already
 }
 
 // the bias of eight columns from c on (past the matrix the last one, never stored); all eight loads are under way at once
@@ -224,11 +201,11 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
     for (int t = 0; t < WN; t++) tb[t] = (uint32_t)(BM * BK + tk * BN + ((wn + t * 32) ^ (block_swizzle<BN * 2>(tk) * 8)) + tcol) * 2;
     auto fragA = [&](const bf16_t* pa, uint32_t stageAddr, int t, int ks, TrFragment& o) {
         if (AK) o.w = *(const u32x4*)(pa + (wm + t * 32 + fr) * BK + koff[ks]);
-        else tr_read<BM * 2>(stageAddr + ta[t], ks, o);
+        else tr_read<BM * 2>(stageAddr + ta[t], ks * 16 * (BM * 2), o);
     };
     auto fragB = [&](const bf16_t* pb, uint32_t stageAddr, int t, int ks, TrFragment& o) {
         if (BKC) o.w = *(const u32x4*)(pb + (wn + t * 32 + fr) * BK + koff[ks]);
-        else tr_read<BN * 2>(stageAddr + tb[t], ks, o);
+        else tr_read<BN * 2>(stageAddr + tb[t], ks * 16 * (BN * 2), o);
     };
 
     const int nk = (kEnd - kBegin + BK - 1) / BK;

@@ -22,6 +22,30 @@ __device__ inline uint32_t pack2_bf16(float a, float b)
     return *reinterpret_cast<uint32_t*>(&r);
 }
 
+#define LDS3(p) ((__attribute__((address_space(3))) void*)(p))
+
+// One operand fragment of a bf16 MFMA.  The transposing reads are written as instructions: as builtins the compiler makes each of
+// them wait for every fetch into LDS that is under way, the next stage's included (16-bit product of 8000 x 768 x 3072 with one such
+// operand: 109 us).  tr_read issues the two reads of a k-step whose first element is OFF bytes from addr (ROWB bytes between k rows),
+// tr_wait makes the values usable.  In between the compiler takes the registers for written: should it copy, spill or reuse one
+// before the wait, the old contents would go on.  It has no reason to (every fragment is read once, or only after its wait), and
+// what it makes of the files that use them is checked: tests/test_asm_pending_reads.py finds no instruction that names a pending
+// register, in any of the kernels.
+struct TrFragment { union { u32x4 w; uint2 h[2]; }; };
+template <int ROWB> __device__ __forceinline__ void tr_read(uint32_t addr, int off, TrFragment& o)
+{
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(o.h[0]) : "v"(addr), "n"(off) : "memory");
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(o.h[1]) : "v"(addr), "n"(off + 4 * ROWB) : "memory");
+}
+__device__ __forceinline__ void tr_wait(TrFragment& o) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o.h[0]), "+v"(o.h[1]) : : "memory"); }
+
+// exchange of 32-row blocks (64 bytes, four 16-byte chunks) in row k of a [k][row] stage: four consecutive k of one block of
+// rows have to lie on four different quarters of the 256 bytes of banks; rows are ROWB bytes apart
+template <int ROWB> __device__ __forceinline__ int block_swizzle(int k)
+{
+    return ROWB % 256 == 0 ? (k & 3) * 4 : ((k >> 1) & 1) * 4;   // in chunks; rows 128 bytes apart modulo 256 alternate already
+}
+
 template <typename T> __device__ inline float ldf(const T* p, size_t i);
 template <> __device__ inline float ldf<float>(const float* p, size_t i) { return p[i]; }
 template <> __device__ inline float ldf<bf16_t>(const bf16_t* p, size_t i) { return bf16_to_f32(p[i]); }
@@ -186,6 +210,7 @@ struct GemmF32 {
     int epoch;
     const float* bias;                     // null, or n values added to every row of C (batch 1)
     const HeadsEpilogue* heads;            // written through this epilogue instead of to C (alpha 1, beta 0, batch 1, bias null)
+    bool fp32Sums;                         // on the fp32 matrix cores, one value of k after the other, whatever the size
 };
 enum { CAUSAL_NO = 0, CAUSAL_A_LOWER /* A(i,k) zero for k > i */, CAUSAL_A_UPPER /* k < i */, CAUSAL_B_LOWER /* B(k,j) zero for k < j */, CAUSAL_B_UPPER /* k > j */ };
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal);

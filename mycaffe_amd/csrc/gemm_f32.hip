@@ -1,6 +1,7 @@
-// fp32 GEMM on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), any operand layout, gfx950.
+// fp32 GEMM, any operand layout, gfx950: on the bf16 matrix cores with every value as three bf16 numbers (gemm_f32_split_kernel,
+// below), and on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) where that is not taken.
 //
-// One kernel serves the inner products (A B^T), their gradients (A B and A^T B) and the batched products of the explicit
+// gemm_f32_kernel serves the inner products (A B^T), their gradients (A B and A^T B) and the batched products of the explicit
 // attention chain.  2 x 2 wavefronts, each owning WM x WN MFMA tiles of 32 x 32, so a workgroup covers (64 WM) x (64 WN) of
 // C and walks K in stages of 32 through a double-buffered LDS stage, one barrier per stage.  What bounds it is the matrix
 // core: a 32x32x2 step is 64 cycles, so a stage of a 128 x 128 tile is 4096 cycles of MFMA per wavefront against some 40
@@ -66,6 +67,109 @@ __device__ __forceinline__ void heads_store4(const HeadsEpilogue& he, int r, int
     }
 }
 
+// Which tile of which part of the contraction, or of which matrix of the batch, a workgroup has, and its range of k.
+struct F32Item { int part, batch, m0, n0, kBegin, kEnd; };
+// Work items are the tiles of every part of the contraction, or of every matrix of the batch; each XCD (workgroup index mod 8)
+// takes a contiguous run of them, so all dies get the same share whatever the tile count of one part.  False: none left.
+template <int BM, int BN>
+__device__ __forceinline__ bool f32_item(const GemmF32Args& g, F32Item& o)
+{
+    const int tiles = g.tilesM * g.tilesN, total = tiles * g.parts, per = (total + 7) / 8;
+    const int item = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (item >= total) return false;
+    o.part = item / tiles;
+    const int tile = item - o.part * tiles;
+    const bool split = g.kChunk < g.K;
+    o.batch = split ? 0 : o.part;
+    // tiles are numbered in groups of GROUP tile rows, down a group's rows first: the tiles an XCD has in flight then share
+    // few enough rows of A and columns of B for its 4 MB of L2
+    constexpr int GROUP = 8;
+    const int group = tile / (GROUP * g.tilesN), inGroup = tile - group * GROUP * g.tilesN;
+    const int groupRows = min(GROUP, g.tilesM - group * GROUP);
+    int tr = group * GROUP + inGroup % groupRows;
+    int tc = inGroup / groupRows;
+    bool causal = false;
+    if (g.causal) {
+        // tiles differ in length along one side: every other round of an XCD's 32 CUs takes them in reverse, so that a CU
+        // that had a long one gets a short one (decided per matrix, so that each of its tiles is still taken once)
+        if (((o.batch * tiles) >> 5) & 1) {
+            if (g.causal >= CAUSAL_B_LOWER) tc = g.tilesN - 1 - tc;
+            else tr = g.tilesM - 1 - tr;
+        }
+        causal = *g.flag != g.epoch;
+    }
+    o.m0 = tr * BM; o.n0 = tc * BN;
+    o.kBegin = split ? o.part * g.kChunk : 0;
+    o.kEnd = min(g.K, o.kBegin + g.kChunk);
+    if (causal) {
+        if (g.causal == CAUSAL_A_LOWER) o.kEnd = min(o.kEnd, o.m0 + BM);
+        else if (g.causal == CAUSAL_A_UPPER) o.kBegin = o.m0;
+        else if (g.causal == CAUSAL_B_LOWER) o.kBegin = o.n0;
+        else o.kEnd = min(o.kEnd, o.n0 + BN);
+    }
+    return true;
+}
+
+// The accumulators of a wavefront (the transposed tiles: register v is column 8 (v / 4) + 4 (lane / 32) + v % 4 of row lane % 32) to
+// C, to the part's partial product or through the heads epilogue.  Each wavefront passes its tile, 32 rows at a time, through its
+// own slice of LDS (free after the last barrier; operations of one wavefront complete in order) and the lanes then walk the rows,
+// so that a store instruction covers whole lines.  (m, n): the wavefront's first row and column.
+template <int WM, int WN, bool HEADS>
+__device__ __forceinline__ void f32_store(const GemmF32Args& g, const HeadsArg<HEADS>& hp, floatx16 (&acc)[WM][WN], float* slice, int lane, int m, int n,
+                                          int part, int batch)
+{
+    constexpr int CW = 32 * WN, LDC = CW + 4, LPR = CW / 4, RPI = 64 / LPR, NIT = (32 + RPI - 1) / RPI;
+    const int M = g.M, N = g.N;
+    const bool split = g.kChunk < g.K;
+    const int fr = lane & 31, fg = (lane >> 5) * 4;
+    const int rr = lane / LPR, cc = (lane % LPR) * 4;
+    float* C = split ? g.part + (size_t)part * M * N : g.C + (size_t)batch * g.sC;
+    const long long ldc = split ? N : g.ldc;
+    const float beta = split ? 0.f : g.beta;
+    const bool vec = split ? (N & 3) == 0 : g.vecC;
+    const int c = n + cc;   // a lane keeps its columns while it walks the rows
+    float4 bias = make_float4(0.f, 0.f, 0.f, 0.f);
+    float* col = nullptr;
+    if (!split && c < N) {
+        bias = f32_bias4(g.bias, c, N);
+        if constexpr (HEADS) col = heads_col<float>(hp.he, c);
+    }
+#pragma unroll
+    for (int i = 0; i < WM; i++) {
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *(float4*)(slice + fr * LDC + j * 32 + 8 * q + fg) =
+                    make_float4(g.alpha * acc[i][j][4 * q], g.alpha * acc[i][j][4 * q + 1], g.alpha * acc[i][j][4 * q + 2], g.alpha * acc[i][j][4 * q + 3]);
+#pragma unroll 4
+        for (int it = 0; it < NIT; it++) {
+            const int row = it * RPI + rr, r = m + i * 32 + row;
+            if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
+            const float4 t = *(const float4*)(slice + row * LDC + cc);
+            float v[4] = {t.x + bias.x, t.y + bias.y, t.z + bias.z, t.w + bias.w};
+            if constexpr (HEADS) {
+                if (!split) {
+                    heads_store4(hp.he, r, c, N, vec, col, v);
+                    continue;
+                }
+            }
+            float* cp = C + (size_t)r * ldc + c;
+            if (vec) {
+                if (beta != 0.f) {
+                    const float4 o = *(const float4*)cp;
+                    v[0] += beta * o.x; v[1] += beta * o.y; v[2] += beta * o.z; v[3] += beta * o.w;
+                }
+                *(float4*)cp = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (c + q < N) cp[q] = v[q] + (beta != 0.f ? beta * cp[q] : 0.f);
+            }
+        }
+    }
+}
+
 // VEC: every 16-byte chunk of an operand is aligned and lies inside it or outside as a whole
 template <int WM, int WN, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
 __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
@@ -81,40 +185,9 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, Heads
     float* As = reinterpret_cast<float*>(smem_raw);
     float* Bs = As + 2 * SA;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // Work items are the tiles of every part of the contraction, or of every matrix of the batch; each XCD (workgroup index
-    // mod 8) takes a contiguous run of them, so all dies get the same share whatever the tile count of one part.
-    const int tiles = g.tilesM * g.tilesN, total = tiles * g.parts, per = (total + 7) / 8;
-    const int item = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-    if (item >= total) return;
-    const int part = item / tiles, tile = item - part * tiles;
-    const bool split = g.kChunk < g.K;
-    const int batch = split ? 0 : part;
-    // tiles are numbered in groups of GROUP tile rows, down a group's rows first: the tiles an XCD has in flight then share
-    // few enough rows of A and columns of B for its 4 MB of L2
-    constexpr int GROUP = 8;
-    const int group = tile / (GROUP * g.tilesN), inGroup = tile - group * GROUP * g.tilesN;
-    const int groupRows = min(GROUP, g.tilesM - group * GROUP);
-    int tr = group * GROUP + inGroup % groupRows;
-    int tc = inGroup / groupRows;
-    bool causal = false;
-    if (g.causal) {
-        // tiles differ in length along one side: every other round of an XCD's 32 CUs takes them in reverse, so that a CU
-        // that had a long one gets a short one (decided per matrix, so that each of its tiles is still taken once)
-        if (((batch * tiles) >> 5) & 1) {
-            if (g.causal >= CAUSAL_B_LOWER) tc = g.tilesN - 1 - tc;
-            else tr = g.tilesM - 1 - tr;
-        }
-        causal = *g.flag != g.epoch;
-    }
-    const int M = g.M, N = g.N;
-    const int m0 = tr * BM, n0 = tc * BN;
-    int kBegin = split ? part * g.kChunk : 0, kEnd = min(g.K, kBegin + g.kChunk);
-    if (causal) {
-        if (g.causal == CAUSAL_A_LOWER) kEnd = min(kEnd, m0 + BM);
-        else if (g.causal == CAUSAL_A_UPPER) kBegin = m0;
-        else if (g.causal == CAUSAL_B_LOWER) kBegin = n0;
-        else kEnd = min(kEnd, n0 + BN);
-    }
+    F32Item it;
+    if (!f32_item<BM, BN>(g, it)) return;
+    const int M = g.M, N = g.N, m0 = it.m0, n0 = it.n0, kBegin = it.kBegin, kEnd = it.kEnd, part = it.part, batch = it.batch;
     const float* __restrict__ A = g.A + (size_t)batch * g.sA;
     const float* __restrict__ B = g.B + (size_t)batch * g.sB;
     const int wm = (wave >> 1) * (32 * WM), wn = (wave & 1) * (32 * WN);
@@ -287,59 +360,333 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, Heads
         }
         __syncthreads();
     }
-    // Register v of a tile is column 8 (v / 4) + 4 (lane / 32) + v % 4 of row lane % 32.  Each wavefront passes its tile, 32
-    // rows at a time, through its own slice of LDS (free after the last barrier; operations of one wavefront complete in
-    // order) and the lanes then walk the rows, so that a store instruction covers whole lines.
-    constexpr int CW = 32 * WN, LDC = CW + 4, LPR = CW / 4, RPI = 64 / LPR, NIT = (32 + RPI - 1) / RPI;
-    float* cs = reinterpret_cast<float*>(smem_raw) + wave * 32 * LDC;
-    const int rr = lane / LPR, cc = (lane % LPR) * 4;
-    float* C = split ? g.part + (size_t)part * M * N : g.C + (size_t)batch * g.sC;
-    const long long ldc = split ? N : g.ldc;
-    const float beta = split ? 0.f : g.beta;
-    const bool vec = split ? (N & 3) == 0 : g.vecC;
-    const int c = n0 + wn + cc;   // a lane keeps its columns while it walks the rows
-    float4 bias = make_float4(0.f, 0.f, 0.f, 0.f);
-    float* col = nullptr;
-    if (!split && c < N) {
-        bias = f32_bias4(g.bias, c, N);
-        if constexpr (HEADS) col = heads_col<float>(hp.he, c);
+    f32_store<WM, WN, HEADS>(g, hp, acc, reinterpret_cast<float*>(smem_raw) + wave * 32 * (32 * WN + 4), lane, m0 + wm, n0 + wn, part, batch);
+}
+
+// ---------------------------------------------------------------------------
+// The same products on the bf16 matrix cores, sixteen times the rate of the fp32 ones: every operand value is the sum of three
+// bf16 numbers, x = h + m + l exactly (24 bits of significand are three times eight; each part is the bf16 nearest to what the
+// parts before it leave), and of the nine products of parts the six down to 2^-18 of the first are added up in fp32:
+// hh + (hm + mh + mm) + (hl + lh).  What is left out is 2^-25 of a product at most.  An MFMA adds sixteen products at a time
+// where the fp32 one adds two, so the sums are rounded less often, and the error against 64 bits is below that of the fp32
+// matrix cores from 64 k on (N(0, 1), 2-norm of the error over that of the result: 1.35e-7 against 1.45e-7 at 64 k, 4.3e-7 against
+// 5.0e-7 at 768, 7.0e-7 against 8.0e-7 at 2048; the other way round at 16: 8.2e-8 against 7.4e-8); shorter contractions stay
+// there (SPLIT_MIN_K).
+//
+// Exact results where parts do not hold a value: an infinity or a value above the largest bf16 number leaves a NaN or an
+// infinity among the parts and so in the result, and below 2^-109 the last part loses bits (bf16 ends at 2^-133), 2^-134 of the
+// other factor at most.  A wavefront whose sums hold a NaN, an infinity or anything nonzero below 2^-90 therefore does its tile
+// again on the fp32 matrix cores, straight from memory.
+//
+// What bounds it is power: at 8192 x 3072 x 768 operands of zeros take 136 us in 128 x 192 tiles, random ones 197 (same instructions), so what
+// helps is fewer instructions and bytes per product.  Values are split once, on their way from registers to LDS (splitting whole
+// operands in a pass of their own costs more than the repeats), the larger tiles split a value less often, and one LDS read of a
+// fragment serves up to three products times WM or WN tiles.
+//
+// Measured, before (fp32 matrix cores) and now, us: 8192 x 3072 x 768 279 -> 188, 8192 x 768 x 3072 274 -> 190, 768 x 3072 x 8192
+// (A^T B) 303 -> 191, 1000 x 32000 x 768 370 -> 231, 4096 x 4096 x 4096 935 -> 564 (244 TFLOP/s), 2800 x 768 x 768 40 -> 31.
+//
+//   * Global loads of a stage (16 KS k) are one stage ahead in registers; between the products of a stage they are split and
+//     written to the other LDS buffer, and the stage after that is requested.
+//   * LDS holds three planes (h, m, l) per operand.  k at unit stride: eight k of a row are 16 bytes, rows next to each other,
+//     groups of eight k padded apart so that what a wavefront writes falls on different banks.  Row index at unit stride: [k][row],
+//     the layout and the transposing reads of the 16-bit kernel (gemm_bf16.hip).
+//   * One barrier a stage, placed before the last third of its products: by then every fragment of the stage has been read, and
+//     the first fragments of the next stage arrive behind the remaining products.
+__device__ __forceinline__ uint2 split_part(float (&v)[4], bool last)
+{
+    uint2 p;
+    p.x = pack2_bf16(v[0], v[1]);
+    p.y = pack2_bf16(v[2], v[3]);
+    if (!last) {
+        v[0] -= __uint_as_float(p.x << 16); v[1] -= __uint_as_float(p.x & 0xffff0000u);
+        v[2] -= __uint_as_float(p.y << 16); v[3] -= __uint_as_float(p.y & 0xffff0000u);
     }
+    return p;
+}
+
+// whether the parts may have lost something of these sums (the same for the whole wavefront)
+template <int WM, int WN> __device__ __forceinline__ bool split_lost(const floatx16 (&acc)[WM][WN])
+{
+    constexpr uint32_t TINY = (127u - 90u) << 24;   // 2^-90 without its sign
+    uint32_t low = 0xffffffffu;
+    float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < WM; i++) {
+    for (int i = 0; i < WM; i++)
 #pragma unroll
         for (int j = 0; j < WN; j++)
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                *(float4*)(cs + fr * LDC + j * 32 + 8 * q + fg) =
-                    make_float4(g.alpha * acc[i][j][4 * q], g.alpha * acc[i][j][4 * q + 1], g.alpha * acc[i][j][4 * q + 2], g.alpha * acc[i][j][4 * q + 3]);
-#pragma unroll 4
-        for (int it = 0; it < NIT; it++) {
-            const int row = it * RPI + rr, r = m0 + wm + i * 32 + row;
-            if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
-            const float4 t = *(const float4*)(cs + row * LDC + cc);
-            float v[4] = {t.x + bias.x, t.y + bias.y, t.z + bias.z, t.w + bias.w};
-            if constexpr (HEADS) {
-                if (!split) {
-                    heads_store4(hp.he, r, c, N, vec, col, v);
-                    continue;
-                }
+            for (int v = 0; v < 16; v++) {
+                low = min(low, (__float_as_uint(acc[i][j][v]) << 1) - 1u);   // zeros wrap to the top
+                sum += fabsf(acc[i][j][v]);
             }
-            float* cp = C + (size_t)r * ldc + c;
-            if (vec) {
-                if (beta != 0.f) {
-                    const float4 o = *(const float4*)cp;
-                    v[0] += beta * o.x; v[1] += beta * o.y; v[2] += beta * o.z; v[3] += beta * o.w;
-                }
-                *(float4*)cp = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
+    return __any(low < TINY - 1u || !(sum < __builtin_inff()));
+}
+
+// a wavefront's sums by the fp32 matrix cores, operands read from memory value by value
+template <int WM, int WN, bool AK, bool BKC>
+__device__ __forceinline__ void f32_sums(const GemmF32Args& g, const float* A, const float* B, int m, int n, int kBegin, int kEnd, int lane, floatx16 (&acc)[WM][WN])
+{
+    const int fr = lane & 31, half = lane >> 5;
+    const float* a[WM];
+    const float* b[WN];
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (c + q < N) cp[q] = v[q] + (beta != 0.f ? beta * cp[q] : 0.f);
-            }
+    for (int t = 0; t < WM; t++) a[t] = A + (size_t)min(m + t * 32 + fr, g.M - 1) * (AK ? g.lda : 1);
+#pragma unroll
+    for (int t = 0; t < WN; t++) b[t] = B + (size_t)min(n + t * 32 + fr, g.N - 1) * (BKC ? g.ldb : 1);
+#pragma unroll
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    for (int k0 = kBegin; k0 < kEnd; k0 += 8) {
+        float x[4][WM], y[4][WN];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int k = min(k0 + 2 * u + half, kEnd - 1);
+#pragma unroll
+            for (int t = 0; t < WM; t++) x[u][t] = a[t][(size_t)k * (AK ? 1 : g.lda)];
+#pragma unroll
+            for (int t = 0; t < WN; t++) y[u][t] = b[t][(size_t)k * (BKC ? 1 : g.ldb)];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const bool in = k0 + 2 * u + half < kEnd;
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? y[u][j] : 0.f, in ? x[u][i] : 0.f, acc[i][j], 0, 0, 0);
         }
     }
 }
 
+// bytes of one plane of R rows by 16 KS k
+template <int R, int KS, bool KFAST> constexpr int split_plane() { return KFAST ? 2 * KS * (R * 16 + 128 / KS) : 16 * KS * R * 2; }
+
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool HEADS>
+__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
+{
+    constexpr int NT = 64 * WVM * WVN, BK = 16 * KS, BM = 32 * WVM * WM, BN = 32 * WVN * WN;
+    constexpr int PA = (BM * BK / 4 + NT - 1) / NT, PB = (BN * BK / 4 + NT - 1) / NT, P = PA + PB;   // chunks of four values per thread and stage
+    constexpr int KGA = BM * 16 + 128 / KS, KGB = BN * 16 + 128 / KS;                                  // bytes between groups of eight k
+    constexpr int PLA = split_plane<BM, KS, AK>(), PLB = split_plane<BN, KS, BKC>(), STAGE = 3 * (PLA + PLB);
+    constexpr int NMF = WM * WN;
+    static_assert(PA * NT == BM * BK / 4 && (KS == 1 || KS % 2 == 0), "whole chunks of A; fragments change registers from k-step to k-step");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    F32Item it;
+    if (!f32_item<BM, BN>(g, it)) return;
+    const int M = g.M, N = g.N, m0 = it.m0, n0 = it.n0, kBegin = it.kBegin, kEnd = it.kEnd;
+    const float* __restrict__ A = g.A + (size_t)it.batch * g.sA;
+    const float* __restrict__ B = g.B + (size_t)it.batch * g.sB;
+    const int wm = (wave / WVN) * (32 * WM), wn = (wave % WVN) * (32 * WN);
+
+    floatx16 acc[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+
+    // Chunk e of a stage, k at unit stride: row e / (BK / 4), k = 4 (e % (BK / 4)); row index at unit stride: k = e / (rows / 4),
+    // rows 4 (e % (rows / 4)) .. + 3.  Where B's chunks do not divide by the threads, the last threads repeat earlier chunks.
+    // Byte offsets from a buffer resource that begins at the tile, and where the row index is at unit stride at the stage, so that
+    // operands of any size are reached with 32 bits; rows past the edge are clamped (valid memory) and never stored.
+    constexpr uint32_t OUTSIDE = 0x80000000u;
+    constexpr int CK = BK / 4;
+    const float* baseA = A + (AK ? (size_t)m0 * g.lda : (size_t)m0);
+    const float* baseB = B + (BKC ? (size_t)n0 * g.ldb : (size_t)n0);
+    uint32_t va[PA], vb[PB], wa[PA], wb[PB];   // where chunks come from, and where their h goes in a stage
+    auto chunkB = [&](int p) { return (tid + NT * p) % (BN * CK); };
+#pragma unroll
+    for (int p = 0; p < PA; p++) {
+        const int e = tid + NT * p;
+        if (AK) {
+            va[p] = 4 * ((uint32_t)min(e / CK, M - 1 - m0) * (uint32_t)g.lda + 4 * (e % CK));
+            wa[p] = (e % CK / 2) * KGA + (e / CK) * 16 + (e & 1) * 8;
+        } else {
+            const int k = e / (BM / 4), row = 4 * (e % (BM / 4));
+            va[p] = 4 * ((uint32_t)k * (uint32_t)g.lda + min(row, M - 4 - m0));
+            wa[p] = (k * BM + (row ^ (block_swizzle<BM * 2>(k) * 8))) * 2;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < PB; p++) {
+        const int e = chunkB(p);
+        if (BKC) {
+            vb[p] = 4 * ((uint32_t)min(e / CK, N - 1 - n0) * (uint32_t)g.ldb + 4 * (e % CK));
+            wb[p] = 3 * PLA + (e % CK / 2) * KGB + (e / CK) * 16 + (e & 1) * 8;
+        } else {
+            const int k = e / (BN / 4), row = 4 * (e % (BN / 4));
+            vb[p] = 4 * ((uint32_t)k * (uint32_t)g.ldb + min(row, N - 4 - n0));
+            wb[p] = 3 * PLA + (k * BN + (row ^ (block_swizzle<BN * 2>(k) * 8))) * 2;
+        }
+    }
+    auto resource = [](const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(OUTSIDE - 16), 0x00020000); };
+    const __amdgpu_buffer_rsrc_t rsA = resource(baseA), rsB = resource(baseB);
+    // as in gemm_f32_kernel: the stage that is fetched next and the way to the one after it, where resources begin at stages
+    const char *stageA = (const char*)(baseA + (size_t)kBegin * g.lda), *stageB = (const char*)(baseB + (size_t)kBegin * g.ldb);
+    long long stepA = (long long)(BK * sizeof(float)) * g.lda, stepB = (long long)(BK * sizeof(float)) * g.ldb;
+    auto advance = [&]() {
+        if (!AK) stageA += stepA;
+        if (!BKC) stageB += stepB;
+    };
+    // before the last stage is fetched, once: the chunks past the end of the contraction
+    auto lastStage = [&](int k0) {
+        asm volatile("" ::: "memory");   // a branch, not a select in every stage
+        stepA = stepB = 0;
+#pragma unroll
+        for (int p = 0; p < PA; p++) {
+            const int e = tid + NT * p;
+            if (k0 + (AK ? 4 * (e % CK) : e / (BM / 4)) >= kEnd) va[p] = OUTSIDE;
+        }
+#pragma unroll
+        for (int p = 0; p < PB; p++) {
+            const int e = chunkB(p);
+            if (k0 + (BKC ? 4 * (e % CK) : e / (BN / 4)) >= kEnd) vb[p] = OUTSIDE;
+        }
+    };
+    const int nk = (kEnd - kBegin + BK - 1) / BK;
+    int fetched = 0, kFetch = kBegin;   // the stage that is fetched and its first k
+    auto nextStage = [&]() {
+        if (fetched + 1 < nk) {         // past the end the last stage is fetched again, its products never made
+            kFetch += BK;
+            fetched++;
+        }
+        advance();
+        if (fetched + 1 == nk) lastStage(kFetch);
+    };
+    u32x4 raw[P];
+    auto fetch = [&](int c) {
+        if (c < PA) {
+            if (AK) raw[c] = __builtin_amdgcn_raw_buffer_load_b128(rsA, va[c], kFetch * 4, 0);
+            else raw[c] = __builtin_amdgcn_raw_buffer_load_b128(resource(stageA), va[c], 0, 0);
+        } else {
+            if (BKC) raw[c] = __builtin_amdgcn_raw_buffer_load_b128(rsB, vb[c - PA], kFetch * 4, 0);
+            else raw[c] = __builtin_amdgcn_raw_buffer_load_b128(resource(stageB), vb[c - PA], 0, 0);
+        }
+    };
+    // part s of chunk c to its plane of a stage
+    auto put = [&](int c, int s, unsigned char* stage) {
+        float v[4] = {__uint_as_float(raw[c].x), __uint_as_float(raw[c].y), __uint_as_float(raw[c].z), __uint_as_float(raw[c].w)};
+        const uint2 p = split_part(v, s == 2);
+        raw[c].x = __float_as_uint(v[0]); raw[c].y = __float_as_uint(v[1]); raw[c].z = __float_as_uint(v[2]); raw[c].w = __float_as_uint(v[3]);
+        *(uint2*)(stage + (c < PA ? wa[c] + s * PLA : wb[c - PA] + s * PLB)) = p;
+    };
+
+    // fragments: lane l holds row l % 32, k = 8 (l / 32) .. + 7 of a k-step of 16; transposing reads as in gemm_b16_kernel
+    const int fr = lane & 31, half = lane >> 5;
+    const int tk = 8 * half + ((lane & 15) >> 2), tcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+    uint32_t ta[WM], tb[WN];
+#pragma unroll
+    for (int t = 0; t < WM; t++)
+        ta[t] = AK ? half * KGA + (wm + t * 32 + fr) * 16 : (tk * BM + ((wm + t * 32) ^ (block_swizzle<BM * 2>(tk) * 8)) + tcol) * 2;
+#pragma unroll
+    for (int t = 0; t < WN; t++)
+        tb[t] = 3 * PLA + (BKC ? half * KGB + (wn + t * 32 + fr) * 16 : (tk * BN + ((wn + t * 32) ^ (block_swizzle<BN * 2>(tk) * 8)) + tcol) * 2);
+    const uint32_t smemAddr = (uint32_t)(uintptr_t)LDS3(smem_raw);
+    // part s of k-step ks of the stage at `at`
+    auto readA = [&](TrFragment (&f)[WM], int at, int ks, int s) {
+#pragma unroll
+        for (int t = 0; t < WM; t++) {
+            if (AK) f[t].w = *(const u32x4*)(smem_raw + at + ta[t] + s * PLA + ks * 2 * KGA);
+            else tr_read<BM * 2>(smemAddr + at + ta[t], s * PLA + ks * 16 * (BM * 2), f[t]);
+        }
+    };
+    auto readB = [&](TrFragment (&f)[WN], int at, int ks, int s) {
+#pragma unroll
+        for (int t = 0; t < WN; t++) {
+            if (BKC) f[t].w = *(const u32x4*)(smem_raw + at + tb[t] + s * PLB + ks * 2 * KGB);
+            else tr_read<BN * 2>(smemAddr + at + tb[t], s * PLB + ks * 16 * (BN * 2), f[t]);
+        }
+    };
+    auto arrived = [&](TrFragment (&a)[WM], TrFragment (&b)[WN]) {
+#pragma unroll
+        for (int t = 0; t < WM; t++)
+            if (!AK) tr_wait(a[t]);
+#pragma unroll
+        for (int t = 0; t < WN; t++)
+            if (!BKC) tr_wait(b[t]);
+    };
+
+    if (nk == 1) lastStage(kBegin);
+#pragma unroll
+    for (int c = 0; c < P; c++) fetch(c);
+    nextStage();
+#pragma unroll
+    for (int c = 0; c < P; c++) {
+#pragma unroll
+        for (int s = 0; s < 3; s++) put(c, s, smem_raw);
+        fetch(c);
+    }
+    __syncthreads();
+    TrFragment ah[2][WM], bh[2][WN], am[WM], bm[WN], al[WM], bl[WN];
+    readA(ah[0], 0, 0, 0);
+    readB(bh[0], 0, 0, 0);
+    arrived(ah[0], bh[0]);
+    // stage u of two: in buffer u, its first h fragments in ah[KS u & 1], bh[KS u & 1]
+    auto stage = [&](int u) {
+        const int at = u * STAGE;
+        unsigned char* next = smem_raw + STAGE - at;
+        nextStage();
+        // what goes between the products: chunks of the next stage part by part to the other buffer, each then fetched anew
+        constexpr int SLOTS = (6 * KS - 2) * NMF, STEPS = 3 * P;
+        auto slot = [&](int q) {
+#pragma unroll
+            for (int st = STEPS * q / SLOTS; st < STEPS * (q + 1) / SLOTS; st++) {
+                put(st / 3, st % 3, next);
+                if (st % 3 == 2) fetch(st / 3);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int cur = (KS * u + ks) & 1, nxt = cur ^ 1;
+            int q = ks * 6 * NMF;
+            auto products = [&](TrFragment (&a)[WM], TrFragment (&b)[WN], bool fill) {
+#pragma unroll
+                for (int t = 0; t < NMF; t++) {
+                    // the transposed tile (B as the row operand): a lane owns a row of C
+                    acc[t / WN][t % WN] = BigTraits<bf16_t>::mma(b[t % WN].w, a[t / WN].w, acc[t / WN][t % WN]);
+                    if (fill) slot(q + t);
+                }
+                q += NMF;
+            };
+            readA(am, at, ks, 1);
+            readB(bm, at, ks, 1);
+            products(ah[cur], bh[cur], true);
+            arrived(am, bm);
+            readA(al, at, ks, 2);
+            readB(bl, at, ks, 2);
+            products(ah[cur], bm, true);
+            products(am, bh[cur], true);
+            products(am, bm, true);
+            arrived(al, bl);
+            if (ks + 1 < KS) {
+                readA(ah[nxt], at, ks + 1, 0);
+                readB(bh[nxt], at, ks + 1, 0);
+            } else {
+                __syncthreads();
+                readA(ah[nxt], STAGE - at, 0, 0);
+                readB(bh[nxt], STAGE - at, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            products(ah[cur], bl, ks + 1 < KS);
+            products(al, bh[cur], ks + 1 < KS);
+            arrived(ah[nxt], bh[nxt]);
+        }
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+        stage(0);
+        if (kt + 1 < nk) stage(1);
+    }
+    __syncthreads();
+    if (split_lost(acc)) f32_sums<WM, WN, AK, BKC>(g, A, B, m0 + wm, n0 + wn, kBegin, kEnd, lane, acc);
+    f32_store<WM, WN, HEADS>(g, hp, acc, reinterpret_cast<float*>(smem_raw) + wave * 32 * (32 * WN + 4), lane, m0 + wm, n0 + wn, it.part, it.batch);
+}
 // C = sum over the S partial products, in their order (alpha is in them already), + beta C; or through the heads epilogue
 template <bool HEADS>
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int S, int M, int N, long long ldc, float beta, bool vecC,
@@ -383,42 +730,74 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restri
 }
 
 // ---------------------------------------------------------------------------
-// How a product is cut: the tile and the number of parts of the contraction with the smallest estimated time.
-struct GemmF32Plan { int wm, wn, splits, kChunk; };
+// How a product is cut: the tile and the number of parts of the contraction with the smallest estimated time.  A split contraction
+// pays for a second launch and for the partial products' way through memory (of at most wsBytes).
+struct GemmF32Plan { int shape, splits, kChunk; };
 
-static GemmF32Plan gemm_f32_plan(int m, int n, int k, int batch, bool causal)
+template <typename TIME>
+static GemmF32Plan best_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes, int shapes, const int (*tile)[2], TIME time)
 {
-    // Cycles of a tile: its products at 256 flops per cycle and CU over the efficiency of a CU's two or more workgroups, and
-    // its first fetches and its stores; a workgroup alone on its CU shows every stage's latency.  Fitted to tiles of 768 and
-    // 2304 k: 128 x 192 (one workgroup per CU: nothing covers its ends) 176k / 500k cycles, 128 x 128 111k / 332k, 64 x 128
-    // 59k / 169k, 64 x 64 31k / 88k.  A split contraction pays for a second
-    // launch and for the partial products' way through memory.
-    static const struct { int wm, wn; double eff, ends, alone; } shapes[] = {{2, 3, 0.909, 14000, 1.10}, {2, 2, 0.89, 600, 1.30}, {1, 2, 0.895, 4000, 1.45}, {1, 1, 0.863, 2200, 1.60}};
-    GemmF32Plan best = {1, 1, 1, k};
+    GemmF32Plan best = {shapes - 1, 1, k};
     double bestT = 1e30;
-    for (const auto& sh : shapes) {
-        const int bm = 64 * sh.wm, bn = 64 * sh.wn;
-        const long long tiles = (long long)((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch;
+    for (int sh = 0; sh < shapes; sh++) {
+        const long long tiles = (long long)((m + tile[sh][0] - 1) / tile[sh][0]) * ((n + tile[sh][1] - 1) / tile[sh][1]) * batch;
         for (int S = 1; S <= 32; S++) {
-            if (S > 1 && (batch > 1 || causal || k / S < 128)) break;
-            const int chunk = ((k + S - 1) / S + 31) / 32 * 32;
+            if (S > 1 && (batch > 1 || causal || k / S < 128 || (size_t)S * m * n * sizeof(float) > wsBytes)) break;
+            const int chunk = S > 1 ? ((k + S - 1) / S + 31) / 32 * 32 : k;
             if ((k + chunk - 1) / chunk != S) continue;
-            const double body = 2.0 * bm * bn * ((chunk + 31) / 32 * 32) / 256.0;
-            const long long perCu = ((tiles * S + 7) / 8 + 31) / 32;
-            const double cycles = perCu == 1 ? body * sh.alone + sh.ends : perCu * (body / sh.eff + sh.ends);
-            double t = cycles / 2.4e9;
-            if (S > 1) t += 4.5e-6 + (double)(S + 1) * m * n * 4.0 / 4.0e12;
-            if (t < bestT) { bestT = t; best = {sh.wm, sh.wn, S, S > 1 ? chunk : k}; }
+            double t = time(sh, tiles * S, ((tiles * S + 7) / 8 + 31) / 32, chunk);
+            if (S > 1) t += 4.5 + (double)(S + 1) * m * n * 4.0 / 4.0e6;
+            if (t < bestT) { bestT = t; best = {sh, S, chunk}; }
         }
     }
     return best;
 }
 
+// gemm_f32_kernel.  Cycles of a tile: its products at 256 flops per cycle and CU over the efficiency of a CU's two or more
+// workgroups, and its first fetches and its stores; a workgroup alone on its CU shows every stage's latency.  Fitted to tiles of
+// 768 and 2304 k: 128 x 192 (one workgroup per CU: nothing covers its ends) 176k / 500k cycles, 128 x 128 111k / 332k, 64 x 128
+// 59k / 169k, 64 x 64 31k / 88k.
+static GemmF32Plan gemm_f32_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes)
+{
+    static const int tile[4][2] = {{128, 192}, {128, 128}, {64, 128}, {64, 64}};
+    static const struct { double eff, ends, alone; } fit[4] = {{0.909, 14000, 1.10}, {0.89, 600, 1.30}, {0.895, 4000, 1.45}, {0.863, 2200, 1.60}};
+    return best_plan(m, n, k, batch, causal, wsBytes, 4, tile, [](int sh, long long, long long perCu, int chunk) {
+        const double body = 2.0 * tile[sh][0] * tile[sh][1] * ((chunk + 31) / 32 * 32) / 256.0;
+        return (perCu == 1 ? body * fit[sh].alone + fit[sh].ends : perCu * (body / fit[sh].eff + fit[sh].ends)) / 2400.0;
+    });
+}
+
+// gemm_f32_split_kernel.  Microseconds: what the workgroups of the busiest CU take for their stages and ends, and, because the
+// clock follows the load, a share that grows with the workgroups in all.  Fitted by least squares to 700 measurements of 40 sizes
+// in three layouts and up to 16 parts; the tile chosen is within 1 % of the best one on average, 8 % at most.
+static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes)
+{
+    static const int tile[6][2] = {{256, 256}, {256, 192}, {128, 192}, {128, 128}, {64, 128}, {64, 64}};
+    struct Fit { double stage, ends, loadStage, loadEnds, once; };
+    static const struct { int k; Fit alone, shared; } fit[6] = {
+        {16, {1.475, 9.5, 0.34, 0, 0}, {1.56, 4.9, 0.64, 0, 0}},      {16, {1.125, 9.55, 0.36, 0, 0}, {1.153, 5.7, 0.55, 0, 0}},
+        {16, {0.817, 8.9, 0.156, 0.7, 0}, {0.546, 3.1, 0.39, 0, 0}},  {16, {0.669, 3.64, 0, 5.0, 0}, {0.383, 0.25, 0.286, 0, 2.4}},
+        {32, {0.89, 1.3, 0.066, 2.1, 1.1}, {0.457, 0, 0.332, 0, 5.4}}, {32, {0.637, 1.1, 0.056, 1.07, 0}, {0.307, 0, 0.133, 0.38, 3.0}}};
+    return best_plan(m, n, k, batch, causal, wsBytes, 6, tile, [](int sh, long long items, long long perCu, int chunk) {
+        const Fit& f = perCu == 1 ? fit[sh].alone : fit[sh].shared;
+        const double nk = (chunk + fit[sh].k - 1) / fit[sh].k, load = items / 256.0;
+        return perCu * (nk * f.stage + f.ends) + load * (nk * f.loadStage + f.loadEnds) + f.once;
+    });
+}
+
+// Which products go to the bf16 matrix cores: from 64 k on (below, the split's error is larger than that of the fp32 matrix cores)
+// and from 2^29 multiplications on (2048 x 1536 x 512: 24 against 30 us; below neither fills the chip, 1024 x 768 x 288 with A as
+// stored and B turned: 10.5 against 9.1 us).
+constexpr int SPLIT_MIN_K = 64;
+static bool gemm_f32_splits(int m, int n, int k, int batch) { return k >= SPLIT_MIN_K && (double)m * n * k * batch >= 536870912.0; }
+
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal)
 {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
-    const GemmF32Plan p = gemm_f32_plan(m, n, k, batch, causal);
-    return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
+    // which kernel takes it depends on the operands' alignment too: enough for either
+    int splits = gemm_f32_plan(m, n, k, batch, causal, SIZE_MAX).splits;
+    if (gemm_f32_splits(m, n, k, batch)) splits = std::max(splits, gemm_f32_split_plan(m, n, k, batch, causal, SIZE_MAX).splits);
+    return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
 }
 
 template <int WM, int WN, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
@@ -443,10 +822,44 @@ static hipError_t launch_f32(hipStream_t s, const GemmF32Args& a, int splits, in
 template <bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
 {
-    if (p.wn == 3) return launch_f32<2, 3, 1, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
-    if (p.wm == 2) return launch_f32<2, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
-    if (p.wn == 2) return launch_f32<1, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+    if (p.shape == 0) return launch_f32<2, 3, 1, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+    if (p.shape == 1) return launch_f32<2, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+    if (p.shape == 2) return launch_f32<1, 2, 2, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
     return launch_f32<1, 1, 3, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+}
+
+// the shapes of gemm_f32_split_kernel, in the order of gemm_f32_split_plan: wavefronts, tiles of a wavefront, k-steps of a stage,
+// wavefronts of a SIMD that the registers are to hold
+#define SPLIT_SHAPES(X) X(0, 2, 4, 4, 2, 1, 2) X(1, 4, 2, 2, 3, 1, 2) X(2, 2, 2, 2, 3, 1, 2) X(3, 2, 2, 2, 2, 1, 2) X(4, 2, 2, 1, 2, 2, 2) X(5, 2, 2, 1, 1, 2, 2)
+
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool HEADS>
+static hipError_t launch_split(hipStream_t s, const GemmF32Args& a, int splits, int batch, const HeadsEpilogue* he)
+{
+    constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN;
+    constexpr int stages = 2 * 3 * (split_plane<BM, KS, AK>() + split_plane<BN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
+    constexpr int lds = stages > store ? stages : store;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    GemmF32Args g = a;
+    g.tilesM = (g.M + BM - 1) / BM;
+    g.tilesN = (g.N + BN - 1) / BN;
+    g.parts = splits > 1 ? splits : batch;
+    const long long total = (long long)g.tilesM * g.tilesN * g.parts;
+    if (total > (1ll << 27)) return hipErrorInvalidValue;
+    const int per = (int)((total + 7) / 8);
+    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, HEADS>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    return hipGetLastError();
+}
+
+template <bool AK, bool BKC, bool HEADS>
+static hipError_t launch_split_shape(hipStream_t s, const GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
+{
+    switch (p.shape) {
+#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, HEADS>(s, a, p.splits, batch, he);
+        SPLIT_SHAPES(X)
+#undef X
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
@@ -454,14 +867,11 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     if (q.m <= 0 || q.n <= 0 || q.batch <= 0) return hipSuccess;
     if (q.k <= 0 || (q.causal && ((q.causal >= CAUSAL_B_LOWER ? q.n : q.m) != q.k || !q.flag)) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || q.batch != 1 || !q.aK || !q.bK)))
         return hipErrorInvalidValue;
-    GemmF32Plan p = gemm_f32_plan(q.m, q.n, q.k, q.batch, q.causal != 0);
-    if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
     GemmF32Args a = {};
     a.M = q.m; a.N = q.n; a.K = q.k;
     a.A = q.A; a.B = q.B; a.C = q.C;
     a.lda = q.lda; a.ldb = q.ldb; a.ldc = q.ldc; a.sA = q.sA; a.sB = q.sB; a.sC = q.sC;
     a.alpha = q.alpha; a.beta = q.beta;
-    a.kChunk = p.kChunk;
     a.causal = q.causal; a.flag = q.flag; a.epoch = q.epoch;
     a.part = (float*)ws;
     a.bias = q.heads ? (const float*)q.heads->bias : q.bias;
@@ -471,14 +881,18 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     } else {
         a.vecC = q.n % 4 == 0 && q.ldc % 4 == 0 && (q.batch == 1 || q.sC % 4 == 0) && ((uintptr_t)q.C & 15) == 0;
     }
-    // 31-bit byte offsets within a tile's rows of k (128 at most), or within the k rows of a stage
-    auto near = [&](bool kFast, int rows, long long ld) { return (kFast ? (std::min(rows, 128) + 1) * ld : std::min(q.k, 32) * ld + 256) < (1ll << 29); };
+    // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage
+    auto near = [&](bool kFast, int rows, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(q.k, 32) * ld + 256) < (1ll << 29); };
     const bool vec = (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
                      (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0) &&
                      near(q.aK, q.m, q.lda) && near(q.bK, q.n, q.ldb);
+    if (!ws || ((uintptr_t)ws & 15)) wsBytes = 0;
+    const bool split = vec && !q.fp32Sums && gemm_f32_splits(q.m, q.n, q.k, q.batch);
+    const GemmF32Plan p = split ? gemm_f32_split_plan(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes) : gemm_f32_plan(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes);
+    a.kChunk = p.kChunk;
     hipError_t e;
-    if (q.heads) e = vec ? launch_f32_tile<true, true, true, true>(s, a, p, 1, q.heads) : launch_f32_tile<true, true, false, true>(s, a, p, 1, q.heads);
-#define LAYOUT(AKV, BKV) (vec ? launch_f32_tile<AKV, BKV, true, false>(s, a, p, q.batch) : launch_f32_tile<AKV, BKV, false, false>(s, a, p, q.batch))
+    if (q.heads) e = split ? launch_split_shape<true, true, true>(s, a, p, 1, q.heads) : vec ? launch_f32_tile<true, true, true, true>(s, a, p, 1, q.heads) : launch_f32_tile<true, true, false, true>(s, a, p, 1, q.heads);
+#define LAYOUT(AKV, BKV) (split ? launch_split_shape<AKV, BKV, false>(s, a, p, q.batch) : vec ? launch_f32_tile<AKV, BKV, true, false>(s, a, p, q.batch) : launch_f32_tile<AKV, BKV, false, false>(s, a, p, q.batch))
     else if (q.aK) e = q.bK ? LAYOUT(true, true) : LAYOUT(true, false);
     else e = q.bK ? LAYOUT(false, true) : LAYOUT(false, false);
 #undef LAYOUT

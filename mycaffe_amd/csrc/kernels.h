@@ -133,12 +133,13 @@ size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k);
 // straight into three (B,H,T,hs) tensors.  ws: k_gemm_qkv_heads_workspace_bytes(...) of scratch.
 hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* bias,
                             void* q, void* k, void* v, void* ws, size_t wsBytes, const float* fcos = nullptr, const float* fsin = nullptr,
-                            int ropeSeq = 0);
+                            int ropeSeq = 0, bool fp32Sums = false);
 // Y (m x n) = X (m x k) W^T + bias in one call; ws: k_gemm_bias_workspace_bytes(...) of scratch
-hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes);
+hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* W, const void* bias, void* Y, void* ws, size_t wsBytes,
+                       bool fp32Sums = false);   // fp32Sums: GemmF32
 // scratch of k_gemm_bias / k_gemm_qkv_heads with these operands (0: none)
 hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, int k, const void* X, const void* W, const void* bias, void* Y,
-                             void* ws, size_t wsBytes);   // Y as (B,H,T,hs); scratch as k_gemm_bias
+                             void* ws, size_t wsBytes, bool fp32Sums = false);   // Y as (B,H,T,hs); scratch as k_gemm_bias
 size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W);
 // whether the call fails without that scratch (otherwise its contraction stays in one part)
 bool k_gemm_bias_needs_workspace(DType dt, int m, int n, int k, const void* X, const void* W);

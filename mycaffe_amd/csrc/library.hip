@@ -2136,8 +2136,8 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
     case MCH_FN_QKV_PROJ_HEADS: {
         // l{batch, T, heads, hs, hX, hW, hBias(0 = none), hQ, hK, hV}: [q|k|v] = X W^T + bias, X (batch*T, C), W (3C, C),
         // C = heads*hs, each third written as (batch, heads, T, hs).  An eleventh value, hRope != 0, also applies that
-        // handle's rotation to q and k, as ROPE_FWD without an offset does to their (batch, T, heads, hs) form.
-        NEED_L(10, 11);
+        // handle's rotation to q and k, as ROPE_FWD without an offset does to their (batch, T, heads, hs) form; a twelfth, fp32Sums.
+        NEED_L(10, 12);
         const long long B = pl[0], T = pl[1], H = pl[2], hs = pl[3];
         if (B < 1 || T < 1 || H < 1 || hs < 1 || B * T > INT_MAX || 3 * H * hs > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         const long long C = H * hs, M = B * T;
@@ -2171,7 +2171,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         else workspace_or_none(&wsb, &ws);
         HIPCHK(k_gemm_qkv_heads(s, X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Q->ptr, K->ptr,
                                 V->ptr, ws, wsb, r ? (const float*)r->dcos.get() : nullptr, r ? (const float*)r->dsin.get() : nullptr,
-                                r ? r->seq : 0));
+                                r ? r->seq : 0, ll > 11 && pl[11] != 0));
         m_mem.touch((long)pl[7]);
         m_mem.touch((long)pl[8]);
         m_mem.touch((long)pl[9]);
@@ -2179,13 +2179,14 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
     }
 
     case MCH_FN_LINEAR_FWD: {
-        // l{M, N, K, hX, hW, hBias(0 = none), hY[, T, heads]}: Y (M x N) = X (M x K) W^T (N x K) + bias (N), one launch; with
-        // T and heads written as (M/T, heads, T, N/heads)
-        NEED_L(7, 9);
+        // l{M, N, K, hX, hW, hBias(0 = none), hY[, T, heads[, fp32Sums]]}: Y (M x N) = X (M x K) W^T (N x K) + bias (N), one
+        // launch; with T and heads written as (M/T, heads, T, N/heads); before fp32Sums both may be 0
+        NEED_L(7, 10);
         const long long M = pl[0], N = pl[1], K = pl[2];
         if (M < 1 || N < 1 || K < 1 || M > INT_MAX || N > INT_MAX || K > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         const long long T = ll > 7 ? pl[7] : 0, heads = ll > 8 ? pl[8] : 0;
-        if (ll > 7 && (ll != 9 || T < 1 || heads < 1 || M % T || N % heads)) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        const bool fp32Sums = ll > 9 && pl[9] != 0;
+        if (ll > 7 && !(ll == 10 && T == 0 && heads == 0) && (ll < 9 || T < 1 || heads < 1 || M % T || N % heads)) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         MemItem *X, *W, *Bi = nullptr, *Y;
         ERRCHK(mem((long)pl[3], &X));
         ERRCHK(mem((long)pl[4], &W));
@@ -2201,8 +2202,8 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (k_gemm_bias_needs_workspace(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
         else workspace_or_none(&wsb, &ws);
         if (heads)
-            HIPCHK(k_gemm_bias_heads(s, X->dt(), (int)(M / T), (int)T, (int)heads, (int)(N / heads), (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
-        else HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb));
+            HIPCHK(k_gemm_bias_heads(s, X->dt(), (int)(M / T), (int)T, (int)heads, (int)(N / heads), (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb, fp32Sums));
+        else HIPCHK(k_gemm_bias(s, X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr, ws, wsb, fp32Sums));
         m_mem.touch((long)pl[6]);
         return 0;
     }

@@ -2148,12 +2148,13 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         return 0;
     }
     case MCH_FN_LINEAR_FWD: {
-        // l{M, N, K, hX, hW, hBias(0 = none), hY[, T, heads]}: Y = X W^T + bias, with T and heads as (M/T, heads, T, N/heads)
-        NEED_L(7, 9);
+        // l{M, N, K, hX, hW, hBias(0 = none), hY[, T, heads[, fp32Sums: no meaning here]]}: Y = X W^T + bias, with T and heads as
+        // (M/T, heads, T, N/heads)
+        NEED_L(7, 10);
         const long long M = pl[0], N = pl[1], K = pl[2];
         if (M < 1 || N < 1 || K < 1 || M > INT_MAX || N > INT_MAX || K > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         const long long T = ll > 7 ? pl[7] : 0, heads = ll > 8 ? pl[8] : 0;
-        if (ll > 7 && (ll != 9 || T < 1 || heads < 1 || M % T || N % heads)) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        if (ll > 7 && !(ll == 10 && T == 0 && heads == 0) && (ll < 9 || T < 1 || heads < 1 || M % T || N % heads)) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         MemD *X, *W, *Bi = nullptr, *Y;
         ERRCHK(mem((long)pl[3], &X));
         ERRCHK(mem((long)pl[4], &W));
@@ -2197,8 +2198,8 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         return 0;
     }
     case MCH_FN_QKV_PROJ_HEADS: {
-        // l{batch, T, heads, hs, hX, hW, hBias(0 = none), hQ, hK, hV [, hRope]}
-        NEED_L(10, 11);
+        // l{batch, T, heads, hs, hX, hW, hBias(0 = none), hQ, hK, hV [, hRope [, fp32Sums: no meaning here]]}
+        NEED_L(10, 12);
         const long long B = pl[0], T = pl[1], H = pl[2], hs = pl[3];
         if (B < 1 || T < 1 || H < 1 || hs < 1 || B * T > INT_MAX || 3 * H * hs > INT_MAX) return MCH_ERROR_PARAM_OUT_OF_RANGE;
         const long long C = H * hs, M = B * T;

@@ -732,22 +732,27 @@ class CudaDnn:
             rgl.append(1)
         self._ex2(CUDAFN.CUDA_ATTN_FWD, None, rgl)
 
-    def QkvProjHeads(self, nBatch, nT, nHeads, nSize, hX, hWeight, hBias, hQ, hK, hV, hRope=0):
+    def QkvProjHeads(self, nBatch, nT, nHeads, nSize, hX, hWeight, hBias, hQ, hK, hV, hRope=0, bFp32Sums=False):
         """Fused QKV projection (no counterpart in the reference: replaces the InnerProduct, bias GEMM, three
         channel copies and three head transposes of CausalSelfAttentionLayer.cs:526-557): q, k, v written as
         (B,H,T,hs).  With hRope the two RopeForward calls on q and k (:538-545) are part of it as well."""
         rgl = [nBatch, nT, nHeads, nSize, hX, hWeight, hBias, hQ, hK, hV]
-        if hRope:
+        if hRope or bFp32Sums:
             rgl.append(hRope)
+        if bFp32Sums:
+            rgl.append(1)
         self._ex2(CUDAFN.QKV_PROJ_HEADS, None, rgl)
 
-    def LinearForward(self, nM, nN, nK, hX, hWeight, hBias, hY, nT=0, nHeads=0):
+    def LinearForward(self, nM, nN, nK, hX, hWeight, hBias, hY, nT=0, nHeads=0, bFp32Sums=False):
         """y (M,N) = x (M,K) W^T (N,K) + bias in one GEMM (no counterpart in the reference: replaces the product and
         the rank-1 bias update of InnerProductLayer.cs:372-417).  hBias 0: no bias.  With nT and nHeads y is written as
-        (M/T, heads, T, N/heads), which replaces the head transpose behind an attention layer's projection."""
+        (M/T, heads, T, N/heads), which replaces the head transpose behind an attention layer's projection.
+        bFp32Sums: the sums of the fp32 matrix cores at every size."""
         rgl = [nM, nN, nK, hX, hWeight, hBias, hY]
-        if nHeads:
+        if nHeads or bFp32Sums:
             rgl += [nT, nHeads]
+        if bFp32Sums:
+            rgl.append(1)
         self._ex2(CUDAFN.LINEAR_FWD, None, rgl)
 
     def LinearBackward(self, nM, nN, nK, hX, hWeight, hdY, hdWeight, hdBias, hdX, bAccumulate=False):

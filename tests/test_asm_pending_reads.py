@@ -1,5 +1,5 @@
-"""The transposing LDS reads of the 16-bit GEMM are written as instructions whose results arrive some instructions later
-(csrc/gemm_bf16.hip, tr_read / tr_wait): nothing but the compiler's own choice keeps it from copying, spilling or reusing such a
+"""The transposing LDS reads of the GEMMs are written as instructions whose results arrive some instructions later
+(csrc/gemm_common.h, tr_read / tr_wait): nothing but the compiler's own choice keeps it from copying, spilling or reusing such a
 register before the wait.  So the assembly it makes of the file is read: from each read to the next wait for all LDS reads no
 other instruction may name its registers, and no branch may come between."""
 import os
@@ -83,5 +83,19 @@ def test_no_instruction_touches_a_pending_read(tmp_path):
         found = [(name,) + check(body) for name, body in functions(f.read())]
     with_reads = [f for f in found if f[1]]
     assert len(with_reads) >= 21          # three layouts of seven tiles
+    for name, reads, bad in with_reads:
+        assert not bad, (name, bad[:5])
+
+
+def test_no_instruction_touches_a_pending_read_of_the_split_fp32_kernel(tmp_path):
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no compiler")
+    out = str(tmp_path / "gemm_f32.s")
+    subprocess.run([build.HIPCC] + build.FLAGS + ["-w", "--cuda-device-only", "-S", os.path.join(build.CSRC, "gemm_f32.hip"), "-o", out], check=True,
+                   stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    with open(out) as f:
+        found = [(name,) + check(body) for name, body in functions(f.read())]
+    with_reads = [f for f in found if f[1]]
+    assert len(with_reads) >= 18          # three layouts of six tiles
     for name, reads, bad in with_reads:
         assert not bad, (name, bad[:5])
