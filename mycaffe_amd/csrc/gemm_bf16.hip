@@ -30,12 +30,6 @@ struct GemmB16Args {
     const bf16_t* bias;
 };
 
-// sixteen bytes per lane from the buffer to the wavefront's 1 KB of LDS at `lds` (wavefront-uniform)
-__device__ __forceinline__ void lds_fetch16(__amdgpu_buffer_rsrc_t rs, bf16_t* lds, uint32_t voffset, int soffset)
-{
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS3(lds), 16, voffset, soffset, 0, 0);
-}
-
 // the bias of eight columns from c on (past the matrix the last one, never stored); all eight loads are under way at once
 __device__ __forceinline__ void b16_bias8(const GemmB16Args& g, int c, float (&bias)[8])
 {

@@ -1,5 +1,6 @@
 // fp32 GEMM, any operand layout, gfx950: on the bf16 matrix cores with every value as three bf16 numbers (gemm_f32_split_kernel,
-// below), and on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) where that is not taken.
+// below), and on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) where that is not taken: gemm_f32_small_kernel for products that do not
+// fill the chip, gemm_f32_kernel.
 //
 // gemm_f32_kernel serves the inner products (A B^T), their gradients (A B and A^T B) and the batched products of the explicit
 // attention chain.  2 x 2 wavefronts, each owning WM x WN MFMA tiles of 32 x 32, so a workgroup covers (64 WM) x (64 WN) of
@@ -687,6 +688,147 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     if (split_lost(acc)) f32_sums<WM, WN, AK, BKC>(g, A, B, m0 + wm, n0 + wn, kBegin, kEnd, lane, acc);
     f32_store<WM, WN, HEADS>(g, hp, acc, reinterpret_cast<float*>(smem_raw) + wave * 32 * (32 * WN + 4), lane, m0 + wm, n0 + wn, it.part, it.batch);
 }
+// ---------------------------------------------------------------------------
+// Products that do not fill the chip with the tiles above: 32 x 32 of C to a workgroup, every stage of the contraction dealt to its
+// NW wavefronts, whose sums are added up through LDS at the end.
+// With tiles of 64 x 64 such a product is a chain of short stages on a few CUs (1024 x 288 x 288: 80 workgroups, nine stages of 32 k,
+// each longer than its 1024 cycles of MFMA by a trip through LDS and a barrier), and cutting the contraction over workgroups costs a
+// second launch of 4 us.  Here there are four times the workgroups, a stage is 128 k that go from memory straight into LDS (16 bytes
+// per lane, two stages under way), and a wavefront's share of it is 32 k.  What bounds it is the fp32 matrix core of a CU, 0.43 us
+// for a tile's stage, and the latency of the first fetch and of the end, some 2.5 us.  Fragments fetched from memory straight into
+// registers, without LDS, take 1.5 - 2 times as long (1024 x 288 x 288: 8.5 us): 32 rows of 32 bytes to an instruction.
+// Stages of 256 k on eight wavefronts: 8.5 us there, the same at 1024 k.
+// Measured, before and now, us: 1024 x 288 x 288 8.7 -> 5.5, 1024 x 288 x 768 12.6 -> 9.1, 768 x 288 x 1024 (A^T B, beta 1) 13.3 -> 8.9,
+// 512 x 512 x 512 10.9 -> 7.0, 24 times 256 x 48 x 256 8.0 -> 5.7 (causal 8.1 -> 4.8), 96 x 192 x 48 4.5 -> 3.0.
+//
+// LDS holds [row][k] for an operand with k at unit stride, the 16-byte piece c of row r at c ^ (r & 15), and [k][row] for the other,
+// k and k + 4 of every eight next to each other: the two halves of a wavefront, four k apart, then read from the two halves of the banks.
+template <int NW, int BK, bool AK, bool BKC, bool HEADS>
+__global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
+{
+    constexpr int NT = 64 * NW, P = 8 * BK / NT, STAGE = 2 * 32 * BK;   // 16-byte chunks per thread, operand and stage; floats of a stage
+    constexpr int LDC = 36;                                              // floats between rows of a wavefront's sums in LDS
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    float* smem = reinterpret_cast<float*>(smem_raw);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    F32Item it;
+    if (!f32_item<32, 32>(g, it)) return;
+    const int kBegin = it.kBegin, kEnd = it.kEnd;
+    constexpr uint32_t OUTSIDE = 0x80000000u;
+    auto resource = [](const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(OUTSIDE - 16), 0x00020000); };
+    const float* baseA = g.A + (size_t)it.batch * g.sA + (AK ? (size_t)it.m0 * g.lda : (size_t)it.m0);
+    const float* baseB = g.B + (size_t)it.batch * g.sB + (BKC ? (size_t)it.n0 * g.ldb : (size_t)it.n0);
+    const __amdgpu_buffer_rsrc_t rsA = resource(baseA), rsB = resource(baseB);
+    const char *stageA = (const char*)(baseA + (size_t)kBegin * g.lda), *stageB = (const char*)(baseB + (size_t)kBegin * g.ldb);
+    // chunk e of a stage, k at unit stride: piece e % (BK / 4) of row e / (BK / 4) holds k = 4 (piece ^ (row & 15)) .. + 3; row index
+    // at unit stride: rows 4 (e % 8) .. + 3 of the k at place e / 8, where k and k + 4 of every eight are next to each other
+    auto chunkK = [&](bool kFast, int e) { return kFast ? 4 * (e % (BK / 4) ^ (e / (BK / 4) & 15)) : ((e / 8) & ~7) | ((e / 8 & 1) << 2) | (e / 16 & 3); };
+    uint32_t va[P], vb[P];
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        const int e = tid + NT * p;
+        va[p] = 4 * (AK ? (uint32_t)min(e / (BK / 4), g.M - 1 - it.m0) * (uint32_t)g.lda + chunkK(true, e)
+                        : (uint32_t)chunkK(false, e) * (uint32_t)g.lda + min(4 * (e % 8), g.M - 4 - it.m0));
+        vb[p] = 4 * (BKC ? (uint32_t)min(e / (BK / 4), g.N - 1 - it.n0) * (uint32_t)g.ldb + chunkK(true, e)
+                         : (uint32_t)chunkK(false, e) * (uint32_t)g.ldb + min(4 * (e % 8), g.N - 4 - it.n0));
+    }
+    const int nk = (kEnd - kBegin + BK - 1) / BK;
+    int fetched = 0;
+    auto fetch = [&](float* stage) {
+        const int k0 = kBegin + fetched * BK;
+        if (fetched + 1 == nk) {   // the chunks past the end of the contraction
+#pragma unroll
+            for (int p = 0; p < P; p++) {
+                const int e = tid + NT * p;
+                if (k0 + chunkK(AK, e) >= kEnd) va[p] = OUTSIDE;
+                if (k0 + chunkK(BKC, e) >= kEnd) vb[p] = OUTSIDE;
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            float* to = stage + (p * NT + wave * 64) * 4;
+            if (AK) lds_fetch16(rsA, to, va[p], k0 * 4);
+            else lds_fetch16(resource(stageA), to, va[p], 0);
+        }
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            float* to = stage + 32 * BK + (p * NT + wave * 64) * 4;
+            if (BKC) lds_fetch16(rsB, to, vb[p], k0 * 4);
+            else lds_fetch16(resource(stageB), to, vb[p], 0);
+        }
+        stageA += (size_t)(BK * sizeof(float)) * g.lda;
+        stageB += (size_t)(BK * sizeof(float)) * g.ldb;
+        fetched++;
+    };
+    const int fr = lane & 31, half = lane >> 5;
+    // unit of eight k: a lane's four k
+    auto fragment = [&](bool kFast, const float* stage, int unit) {
+        u32x4 v;
+        if (kFast) return *(const u32x4*)(stage + fr * BK + 4 * ((2 * unit + half) ^ (fr & 15)));
+        const uint32_t* q = (const uint32_t*)(stage + (8 * unit + half) * 32 + fr);
+        v.x = q[0]; v.y = q[64]; v.z = q[128]; v.w = q[192];
+        return v;
+    };
+    floatx16 acc;
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    fetch(smem);
+    if (nk > 1) fetch(smem + STAGE);
+    for (int kt = 0; kt < nk; kt++) {
+        // the stage has landed, of this wavefront and then of all, while the next one is still on its way (__syncthreads would wait
+        // for that too)
+        if (kt + 1 < nk) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(2 * P) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
+        float* stage = smem + (kt & 1) * STAGE;
+        const int units = (min(BK, kEnd - kBegin - kt * BK) + 7) / 8;
+        constexpr int J = BK / 8 / NW;
+        u32x4 a[J], b[J];
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            a[j] = fragment(AK, stage, wave + NW * j);
+            b[j] = fragment(BKC, stage + 32 * BK, wave + NW * j);
+        }
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            if (NW * j < units) acc = BigTraits<float>::mma(b[j], a[j], acc);   // the transposed tile (B as the row operand): a lane owns a row of C
+        if (kt + 2 < nk) {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");   // every wavefront has its fragments
+            fetch(stage);
+        }
+    }
+    __syncthreads();
+    float* slice = smem + wave * 32 * LDC;
+#pragma unroll
+    for (int q = 0; q < 4; q++) *(float4*)(slice + fr * LDC + 8 * q + 4 * half) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+    __syncthreads();
+    const int r = it.m0 + (tid >> 3), c = it.n0 + (tid & 7) * 4;   // four columns of a row each
+    if (tid >= 256 || r >= g.M || c >= g.N) return;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float4 t = *(const float4*)(smem + (w * 32 + (tid >> 3)) * LDC + (tid & 7) * 4);
+        v[0] += t.x; v[1] += t.y; v[2] += t.z; v[3] += t.w;
+    }
+    const float4 bias = f32_bias4(g.bias, c, g.N);
+    v[0] = g.alpha * v[0] + bias.x; v[1] = g.alpha * v[1] + bias.y; v[2] = g.alpha * v[2] + bias.z; v[3] = g.alpha * v[3] + bias.w;
+    if constexpr (HEADS) {
+        heads_store4(hp.he, r, c, g.N, g.vecC, heads_col<float>(hp.he, c), v);
+        return;
+    }
+    float* cp = g.C + (size_t)it.batch * g.sC + (size_t)r * g.ldc + c;
+    if (g.vecC) {
+        if (g.beta != 0.f) {
+            const float4 o = *(const float4*)cp;
+            v[0] += g.beta * o.x; v[1] += g.beta * o.y; v[2] += g.beta * o.z; v[3] += g.beta * o.w;
+        }
+        *(float4*)cp = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (c + q < g.N) cp[q] = v[q] + (g.beta != 0.f ? g.beta * cp[q] : 0.f);
+    }
+}
+
 // C = sum over the S partial products, in their order (alpha is in them already), + beta C; or through the heads epilogue
 template <bool HEADS>
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int S, int M, int N, long long ldc, float beta, bool vecC,
@@ -731,11 +873,11 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restri
 
 // ---------------------------------------------------------------------------
 // How a product is cut: the tile and the number of parts of the contraction with the smallest estimated time.  A split contraction
-// pays for a second launch and for the partial products' way through memory (of at most wsBytes).
+// pays for a second launch and for the partial products' way through memory (of at most wsBytes).  Estimates in microseconds.
 struct GemmF32Plan { int shape, splits, kChunk; };
 
 template <typename TIME>
-static GemmF32Plan best_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes, int shapes, const int (*tile)[2], TIME time)
+static GemmF32Plan best_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes, int shapes, const int (*tile)[2], double* estimate, TIME time)
 {
     GemmF32Plan best = {shapes - 1, 1, k};
     double bestT = 1e30;
@@ -750,6 +892,7 @@ static GemmF32Plan best_plan(int m, int n, int k, int batch, bool causal, size_t
             if (t < bestT) { bestT = t; best = {sh, S, chunk}; }
         }
     }
+    *estimate = bestT;
     return best;
 }
 
@@ -757,11 +900,11 @@ static GemmF32Plan best_plan(int m, int n, int k, int batch, bool causal, size_t
 // workgroups, and its first fetches and its stores; a workgroup alone on its CU shows every stage's latency.  Fitted to tiles of
 // 768 and 2304 k: 128 x 192 (one workgroup per CU: nothing covers its ends) 176k / 500k cycles, 128 x 128 111k / 332k, 64 x 128
 // 59k / 169k, 64 x 64 31k / 88k.
-static GemmF32Plan gemm_f32_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes)
+static GemmF32Plan gemm_f32_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes, double* estimate)
 {
     static const int tile[4][2] = {{128, 192}, {128, 128}, {64, 128}, {64, 64}};
     static const struct { double eff, ends, alone; } fit[4] = {{0.909, 14000, 1.10}, {0.89, 600, 1.30}, {0.895, 4000, 1.45}, {0.863, 2200, 1.60}};
-    return best_plan(m, n, k, batch, causal, wsBytes, 4, tile, [](int sh, long long, long long perCu, int chunk) {
+    return best_plan(m, n, k, batch, causal, wsBytes, 4, tile, estimate, [](int sh, long long, long long perCu, int chunk) {
         const double body = 2.0 * tile[sh][0] * tile[sh][1] * ((chunk + 31) / 32 * 32) / 256.0;
         return (perCu == 1 ? body * fit[sh].alone + fit[sh].ends : perCu * (body / fit[sh].eff + fit[sh].ends)) / 2400.0;
     });
@@ -770,7 +913,7 @@ static GemmF32Plan gemm_f32_plan(int m, int n, int k, int batch, bool causal, si
 // gemm_f32_split_kernel.  Microseconds: what the workgroups of the busiest CU take for their stages and ends, and, because the
 // clock follows the load, a share that grows with the workgroups in all.  Fitted by least squares to 700 measurements of 40 sizes
 // in three layouts and up to 16 parts; the tile chosen is within 1 % of the best one on average, 8 % at most.
-static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes)
+static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes, double* estimate)
 {
     static const int tile[6][2] = {{256, 256}, {256, 192}, {128, 192}, {128, 128}, {64, 128}, {64, 64}};
     struct Fit { double stage, ends, loadStage, loadEnds, once; };
@@ -778,25 +921,45 @@ static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool caus
         {16, {1.475, 9.5, 0.34, 0, 0}, {1.56, 4.9, 0.64, 0, 0}},      {16, {1.125, 9.55, 0.36, 0, 0}, {1.153, 5.7, 0.55, 0, 0}},
         {16, {0.817, 8.9, 0.156, 0.7, 0}, {0.546, 3.1, 0.39, 0, 0}},  {16, {0.669, 3.64, 0, 5.0, 0}, {0.383, 0.25, 0.286, 0, 2.4}},
         {32, {0.89, 1.3, 0.066, 2.1, 1.1}, {0.457, 0, 0.332, 0, 5.4}}, {32, {0.637, 1.1, 0.056, 1.07, 0}, {0.307, 0, 0.133, 0.38, 3.0}}};
-    return best_plan(m, n, k, batch, causal, wsBytes, 6, tile, [](int sh, long long items, long long perCu, int chunk) {
+    return best_plan(m, n, k, batch, causal, wsBytes, 6, tile, estimate, [](int sh, long long items, long long perCu, int chunk) {
         const Fit& f = perCu == 1 ? fit[sh].alone : fit[sh].shared;
         const double nk = (chunk + fit[sh].k - 1) / fit[sh].k, load = items / 256.0;
         return perCu * (nk * f.stage + f.ends) + load * (nk * f.loadStage + f.loadEnds) + f.once;
     });
 }
 
-// Which products go to the bf16 matrix cores: from 64 k on (below, the split's error is larger than that of the fp32 matrix cores)
-// and from 2^29 multiplications on (2048 x 1536 x 512: 24 against 30 us; below neither fills the chip, 1024 x 768 x 288 with A as
-// stored and B turned: 10.5 against 9.1 us).
-constexpr int SPLIT_MIN_K = 64;
-static bool gemm_f32_splits(int m, int n, int k, int batch) { return k >= SPLIT_MIN_K && (double)m * n * k * batch >= 536870912.0; }
+// gemm_f32_small_kernel, microseconds: the products of the busiest CU's workgroups, and what each two of them that run at once (by LDS)
+// take for their first fetch, their stages' latencies and their end.  Within 15 % of 34 sizes.
+static double gemm_f32_small_time(int m, int n, int k, int batch)
+{
+    const long long tiles = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, perCu = ((tiles + 7) / 8 + 31) / 32;
+    return 0.9 + (double)((perCu + 1) / 2) * (1.7 + 0.38 * k / 128) + (double)perCu * 0.4 * k / 128;
+}
+
+// Which kernel takes a product, and its plan.  The bf16 matrix cores from 64 k on (below, the split's error is larger than that of the
+// fp32 matrix cores) and from 2^28 multiplications on (2048 x 512 x 384: 10.2 against 11.0 us; below, the chip is not full, and 16 x 288 x
+// 32000 takes 51 against 44 us); 32 x 32 tiles where their estimate is the smallest, which is a tenth of a round of the larger ones.
+enum { F32_TILES, F32_SPLIT, F32_SMALL };
+struct GemmF32Choice { int kernel; GemmF32Plan plan; };
+static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool vec, bool fp32Sums)
+{
+    double t, tiles;
+    GemmF32Choice c = {F32_TILES, gemm_f32_plan(m, n, k, batch, causal, wsBytes, &tiles)};
+    if (!vec || fp32Sums) return c;
+    if (k >= 64 && (double)m * n * k * batch >= 268435456.0) {
+        c = {F32_SPLIT, gemm_f32_split_plan(m, n, k, batch, causal, wsBytes, &t)};
+        tiles = t;   // faster than the fp32 matrix cores at every size from there on
+    }
+    // a launch is in this estimate and not in the others
+    if (gemm_f32_small_time(m, n, k, batch) < tiles + 1.8) c = {F32_SMALL, {0, 1, k}};
+    return c;
+}
 
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal)
 {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
-    // which kernel takes it depends on the operands' alignment too: enough for either
-    int splits = gemm_f32_plan(m, n, k, batch, causal, SIZE_MAX).splits;
-    if (gemm_f32_splits(m, n, k, batch)) splits = std::max(splits, gemm_f32_split_plan(m, n, k, batch, causal, SIZE_MAX).splits);
+    // which kernel takes it depends on the operands' alignment and on the caller too: enough for any
+    const int splits = std::max(gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, true, false).plan.splits, gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, false, false).plan.splits);
     return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
 }
 
@@ -862,6 +1025,33 @@ static hipError_t launch_split_shape(hipStream_t s, const GemmF32Args& a, const 
     return hipErrorInvalidValue;
 }
 
+template <int NW, int BK, bool AK, bool BKC, bool HEADS>
+static hipError_t launch_small(hipStream_t s, const GemmF32Args& a, int batch, const HeadsEpilogue* he)
+{
+    constexpr int stages = 2 * 2 * 32 * BK * (int)sizeof(float), sums = NW * 32 * 36 * (int)sizeof(float), lds = stages > sums ? stages : sums;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_small_kernel<NW, BK, AK, BKC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    GemmF32Args g = a;
+    g.tilesM = (g.M + 31) / 32;
+    g.tilesN = (g.N + 31) / 32;
+    g.parts = batch;
+    g.kChunk = g.K;
+    const long long total = (long long)g.tilesM * g.tilesN * batch;
+    if (total > (1ll << 27)) return hipErrorInvalidValue;
+    const int per = (int)((total + 7) / 8);
+    hipLaunchKernelGGL((gemm_f32_small_kernel<NW, BK, AK, BKC, HEADS>), dim3(per * 8), 64 * NW, lds, s, g, heads_arg<HEADS>(he));
+    return hipGetLastError();
+}
+
+// operands in whole aligned 16-byte chunks
+template <bool AK, bool BKC, bool HEADS>
+static hipError_t launch_layout(hipStream_t s, const GemmF32Args& a, const GemmF32Choice& c, int batch, const HeadsEpilogue* he)
+{
+    if (c.kernel == F32_SMALL) return launch_small<4, 128, AK, BKC, HEADS>(s, a, batch, he);
+    if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, HEADS>(s, a, c.plan, batch, he);
+    return launch_f32_tile<AK, BKC, true, HEADS>(s, a, c.plan, batch, he);
+}
+
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
 {
     if (q.m <= 0 || q.n <= 0 || q.batch <= 0) return hipSuccess;
@@ -881,18 +1071,18 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     } else {
         a.vecC = q.n % 4 == 0 && q.ldc % 4 == 0 && (q.batch == 1 || q.sC % 4 == 0) && ((uintptr_t)q.C & 15) == 0;
     }
-    // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage
-    auto near = [&](bool kFast, int rows, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(q.k, 32) * ld + 256) < (1ll << 29); };
+    // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
+    auto near = [&](bool kFast, int rows, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(q.k, 128) * ld + 256) < (1ll << 29); };
     const bool vec = (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
                      (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0) &&
                      near(q.aK, q.m, q.lda) && near(q.bK, q.n, q.ldb);
     if (!ws || ((uintptr_t)ws & 15)) wsBytes = 0;
-    const bool split = vec && !q.fp32Sums && gemm_f32_splits(q.m, q.n, q.k, q.batch);
-    const GemmF32Plan p = split ? gemm_f32_split_plan(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes) : gemm_f32_plan(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes);
+    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, vec, q.fp32Sums);
+    const GemmF32Plan& p = choice.plan;
     a.kChunk = p.kChunk;
     hipError_t e;
-    if (q.heads) e = split ? launch_split_shape<true, true, true>(s, a, p, 1, q.heads) : vec ? launch_f32_tile<true, true, true, true>(s, a, p, 1, q.heads) : launch_f32_tile<true, true, false, true>(s, a, p, 1, q.heads);
-#define LAYOUT(AKV, BKV) (split ? launch_split_shape<AKV, BKV, false>(s, a, p, q.batch) : vec ? launch_f32_tile<AKV, BKV, true, false>(s, a, p, q.batch) : launch_f32_tile<AKV, BKV, false, false>(s, a, p, q.batch))
+    if (q.heads) e = vec ? launch_layout<true, true, true>(s, a, choice, 1, q.heads) : launch_f32_tile<true, true, false, true>(s, a, p, 1, q.heads);
+#define LAYOUT(AKV, BKV) (vec ? launch_layout<AKV, BKV, false>(s, a, choice, q.batch, nullptr) : launch_f32_tile<AKV, BKV, false, false>(s, a, p, q.batch))
     else if (q.aK) e = q.bK ? LAYOUT(true, true) : LAYOUT(true, false);
     else e = q.bK ? LAYOUT(false, true) : LAYOUT(false, false);
 #undef LAYOUT
