@@ -162,12 +162,12 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
     auto fetch = [&](int p, int k0, bf16_t* stage) {
         if (p < PA) {
             bf16_t* to = stage + (p * NT + wave * 64) * 8;
-            if (AK) lds_fetch16(rsA, to, va[p], k0 * 2);
-            else lds_fetch16(resource(stageA), to, va[p], 0);
+            if (AK) lds_fetch<16>(rsA, to, va[p], k0 * 2);
+            else lds_fetch<16>(resource(stageA), to, va[p], 0);
         } else {
             bf16_t* to = stage + BM * BK + ((p - PA) * NT + wave * 64) * 8;
-            if (BKC) lds_fetch16(rsB, to, vb[p - PA], k0 * 2);
-            else lds_fetch16(resource(stageB), to, vb[p - PA], 0);
+            if (BKC) lds_fetch<16>(rsB, to, vb[p - PA], k0 * 2);
+            else lds_fetch<16>(resource(stageB), to, vb[p - PA], 0);
         }
     };
 

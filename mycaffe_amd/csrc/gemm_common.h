@@ -39,10 +39,12 @@ template <int ROWB> __device__ __forceinline__ void tr_read(uint32_t addr, int o
 }
 __device__ __forceinline__ void tr_wait(TrFragment& o) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o.h[0]), "+v"(o.h[1]) : : "memory"); }
 
-// sixteen bytes per lane from the buffer to the wavefront's 1 KB of LDS at `lds` (wavefront-uniform)
-__device__ __forceinline__ void lds_fetch16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voffset, int soffset)
+// BYTES (16 or 4) per lane from the buffer to LDS from `lds` on (wavefront-uniform), lane after lane
+template <int BYTES> __device__ __forceinline__ void lds_fetch(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voffset, int soffset)
 {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS3(lds), 16, voffset, soffset, 0, 0);
+    static_assert(BYTES == 16 || BYTES == 4, "");
+    if constexpr (BYTES == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS3(lds), 16, voffset, soffset, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS3(lds), 4, voffset, soffset, 0, 0);
 }
 
 // exchange of 32-row blocks (64 bytes, four 16-byte chunks) in row k of a [k][row] stage: four consecutive k of one block of

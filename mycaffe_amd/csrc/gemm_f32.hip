@@ -71,13 +71,12 @@ __device__ __forceinline__ void heads_store4(const HeadsEpilogue& he, int r, int
 // Which tile of which part of the contraction, or of which matrix of the batch, a workgroup has, and its range of k.
 struct F32Item { int part, batch, m0, n0, kBegin, kEnd; };
 // Work items are the tiles of every part of the contraction, or of every matrix of the batch; each XCD (workgroup index mod 8)
-// takes a contiguous run of them, so all dies get the same share whatever the tile count of one part.  False: none left.
+// takes a contiguous run of them, so all dies get the same share whatever the tile count of one part.
+__device__ __forceinline__ int xcd_item(int total) { return (int)(blockIdx.x % 8) * ((total + 7) / 8) + (int)(blockIdx.x / 8); }
 template <int BM, int BN>
-__device__ __forceinline__ bool f32_item(const GemmF32Args& g, F32Item& o)
+__device__ __forceinline__ void f32_item(const GemmF32Args& g, int item, F32Item& o)
 {
-    const int tiles = g.tilesM * g.tilesN, total = tiles * g.parts, per = (total + 7) / 8;
-    const int item = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-    if (item >= total) return false;
+    const int tiles = g.tilesM * g.tilesN;
     o.part = item / tiles;
     const int tile = item - o.part * tiles;
     const bool split = g.kChunk < g.K;
@@ -108,7 +107,6 @@ __device__ __forceinline__ bool f32_item(const GemmF32Args& g, F32Item& o)
         else if (g.causal == CAUSAL_B_LOWER) o.kBegin = o.n0;
         else o.kEnd = min(o.kEnd, o.n0 + BN);
     }
-    return true;
 }
 
 // The accumulators of a wavefront (the transposed tiles: register v is column 8 (v / 4) + 4 (lane / 32) + v % 4 of row lane % 32) to
@@ -186,8 +184,10 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, Heads
     float* As = reinterpret_cast<float*>(smem_raw);
     float* Bs = As + 2 * SA;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int total = g.tilesM * g.tilesN * g.parts, item = xcd_item(total);
+    if (item >= total) return;
     F32Item it;
-    if (!f32_item<BM, BN>(g, it)) return;
+    f32_item<BM, BN>(g, item, it);
     const int M = g.M, N = g.N, m0 = it.m0, n0 = it.n0, kBegin = it.kBegin, kEnd = it.kEnd, part = it.part, batch = it.batch;
     const float* __restrict__ A = g.A + (size_t)batch * g.sA;
     const float* __restrict__ B = g.B + (size_t)batch * g.sB;
@@ -477,8 +477,10 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     static_assert(PA * NT == BM * BK / 4 && (KS == 1 || KS % 2 == 0), "whole chunks of A; fragments change registers from k-step to k-step");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int total = g.tilesM * g.tilesN * g.parts, item = xcd_item(total);
+    if (item >= total) return;
     F32Item it;
-    if (!f32_item<BM, BN>(g, it)) return;
+    f32_item<BM, BN>(g, item, it);
     const int M = g.M, N = g.N, m0 = it.m0, n0 = it.n0, kBegin = it.kBegin, kEnd = it.kEnd;
     const float* __restrict__ A = g.A + (size_t)it.batch * g.sA;
     const float* __restrict__ B = g.B + (size_t)it.batch * g.sB;
@@ -693,26 +695,27 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
 // NW wavefronts, whose sums are added up through LDS at the end.
 // With tiles of 64 x 64 such a product is a chain of short stages on a few CUs (1024 x 288 x 288: 80 workgroups, nine stages of 32 k,
 // each longer than its 1024 cycles of MFMA by a trip through LDS and a barrier), and cutting the contraction over workgroups costs a
-// second launch of 4 us.  Here there are four times the workgroups, a stage is 128 k that go from memory straight into LDS (16 bytes
-// per lane, two stages under way), and a wavefront's share of it is 32 k.  What bounds it is the fp32 matrix core of a CU, 0.43 us
-// for a tile's stage, and the latency of the first fetch and of the end, some 2.5 us.  Fragments fetched from memory straight into
-// registers, without LDS, take 1.5 - 2 times as long (1024 x 288 x 288: 8.5 us): 32 rows of 32 bytes to an instruction.
-// Stages of 256 k on eight wavefronts: 8.5 us there, the same at 1024 k.
-// Measured, before and now, us: 1024 x 288 x 288 8.7 -> 5.5, 1024 x 288 x 768 12.6 -> 9.1, 768 x 288 x 1024 (A^T B, beta 1) 13.3 -> 8.9,
-// 512 x 512 x 512 10.9 -> 7.0, 24 times 256 x 48 x 256 8.0 -> 5.7 (causal 8.1 -> 4.8), 96 x 192 x 48 4.5 -> 3.0.
+// second launch of 4 us.  Here there are four times the workgroups, a stage is 64 k that go from memory straight into LDS, two of
+// them under way and three workgroups to a CU, and a wavefront's share of it is 16 k.  What bounds it is the fp32 matrix core of a
+// CU, 0.21 us for a tile's stage of 0.36, and the latency of the first fetch and of the end, some 2.5 us.
+// Fragments fetched from memory straight into registers take 1.5 - 2 times as long (1024 x 288 x 288: 8.5 us): 32 rows of 32 bytes to
+// an instruction.  Stages of 128 k, two workgroups to a CU: 768 x 768 x 700 15.5 instead of 12.5 us, the same where every CU has
+// one; eight wavefronts, five stages, fragments read a stage ahead: no better.
+// Measured, before and now, us: 1024 x 288 x 288 8.7 -> 5.8, 1024 x 288 x 768 12.6 -> 9.9, 768 x 288 x 1024 (A^T B, beta 1) 13.3 -> 8.7,
+// 768 x 768 x 700 (A^T B) 17.1 -> 12.6, 24 times 256 x 48 x 256 8.0 -> 5.5 (causal 8.1 -> 4.9), 96 x 192 x 48 4.4 -> 2.9.
 //
 // LDS holds [row][k] for an operand with k at unit stride, the 16-byte piece c of row r at c ^ (r & 15), and [k][row] for the other,
 // k and k + 4 of every eight next to each other: the two halves of a wavefront, four k apart, then read from the two halves of the banks.
-template <int NW, int BK, bool AK, bool BKC, bool HEADS>
-__global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
+//
+// VEC: as above; otherwise 4 bytes per lane go into LDS, to the same places.
+// rowSums: null, or a value for every row of C to which the sum of the row of A is added (by the tiles of the first columns).
+constexpr int SMALL_STAGES = 3;
+template <int NW, int BK, bool AK, bool BKC, bool VEC, bool HEADS>
+__device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const HeadsArg<HEADS>& hp, const F32Item& it, float* rowSums, float* smem)
 {
-    constexpr int NT = 64 * NW, P = 8 * BK / NT, STAGE = 2 * 32 * BK;   // 16-byte chunks per thread, operand and stage; floats of a stage
-    constexpr int LDC = 36;                                              // floats between rows of a wavefront's sums in LDS
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    float* smem = reinterpret_cast<float*>(smem_raw);
+    constexpr int NT = 64 * NW, W = VEC ? 4 : 1, P = 32 * BK / W / NT, STAGE = 2 * 32 * BK, S = SMALL_STAGES;   // values per lane and fetch; fetches per thread, operand and stage
+    constexpr int LDC = 36;                                                                     // floats between rows of a wavefront's sums in LDS
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    F32Item it;
-    if (!f32_item<32, 32>(g, it)) return;
     const int kBegin = it.kBegin, kEnd = it.kEnd;
     constexpr uint32_t OUTSIDE = 0x80000000u;
     auto resource = [](const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(OUTSIDE - 16), 0x00020000); };
@@ -720,41 +723,40 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, 
     const float* baseB = g.B + (size_t)it.batch * g.sB + (BKC ? (size_t)it.n0 * g.ldb : (size_t)it.n0);
     const __amdgpu_buffer_rsrc_t rsA = resource(baseA), rsB = resource(baseB);
     const char *stageA = (const char*)(baseA + (size_t)kBegin * g.lda), *stageB = (const char*)(baseB + (size_t)kBegin * g.ldb);
-    // chunk e of a stage, k at unit stride: piece e % (BK / 4) of row e / (BK / 4) holds k = 4 (piece ^ (row & 15)) .. + 3; row index
-    // at unit stride: rows 4 (e % 8) .. + 3 of the k at place e / 8, where k and k + 4 of every eight are next to each other
-    auto chunkK = [&](bool kFast, int e) { return kFast ? 4 * (e % (BK / 4) ^ (e / (BK / 4) & 15)) : ((e / 8) & ~7) | ((e / 8 & 1) << 2) | (e / 16 & 3); };
+    // value e of a stage, k at unit stride: piece e % BK / 4 of row e / BK holds k = 4 (piece ^ (row & 15)) .. + 3; row index at unit
+    // stride: row e % 32 of the k at place e / 32, where k and k + 4 of every eight are next to each other
+    auto valueK = [&](bool kFast, int e) { return kFast ? (4 * (e % BK / 4 ^ (e / BK & 15)) | (e & 3)) : ((e / 32) & ~7) | ((e / 32 & 1) << 2) | (e / 64 & 3); };
+    auto valueRow = [&](bool kFast, int e, int left) { return min(kFast ? e / BK : e % 32, kFast || !VEC ? left - 1 : left - 4); };
     uint32_t va[P], vb[P];
 #pragma unroll
     for (int p = 0; p < P; p++) {
-        const int e = tid + NT * p;
-        va[p] = 4 * (AK ? (uint32_t)min(e / (BK / 4), g.M - 1 - it.m0) * (uint32_t)g.lda + chunkK(true, e)
-                        : (uint32_t)chunkK(false, e) * (uint32_t)g.lda + min(4 * (e % 8), g.M - 4 - it.m0));
-        vb[p] = 4 * (BKC ? (uint32_t)min(e / (BK / 4), g.N - 1 - it.n0) * (uint32_t)g.ldb + chunkK(true, e)
-                         : (uint32_t)chunkK(false, e) * (uint32_t)g.ldb + min(4 * (e % 8), g.N - 4 - it.n0));
+        const int e = W * (tid + NT * p), ka = valueK(AK, e), kb = valueK(BKC, e), ra = valueRow(AK, e, g.M - it.m0), rb = valueRow(BKC, e, g.N - it.n0);
+        va[p] = 4 * (AK ? (uint32_t)ra * (uint32_t)g.lda + ka : (uint32_t)ka * (uint32_t)g.lda + ra);
+        vb[p] = 4 * (BKC ? (uint32_t)rb * (uint32_t)g.ldb + kb : (uint32_t)kb * (uint32_t)g.ldb + rb);
     }
     const int nk = (kEnd - kBegin + BK - 1) / BK;
     int fetched = 0;
     auto fetch = [&](float* stage) {
         const int k0 = kBegin + fetched * BK;
-        if (fetched + 1 == nk) {   // the chunks past the end of the contraction
+        if (fetched + 1 == nk) {   // what lies past the end of the contraction
 #pragma unroll
             for (int p = 0; p < P; p++) {
-                const int e = tid + NT * p;
-                if (k0 + chunkK(AK, e) >= kEnd) va[p] = OUTSIDE;
-                if (k0 + chunkK(BKC, e) >= kEnd) vb[p] = OUTSIDE;
+                const int e = W * (tid + NT * p);
+                if (k0 + valueK(AK, e) >= kEnd) va[p] = OUTSIDE;
+                if (k0 + valueK(BKC, e) >= kEnd) vb[p] = OUTSIDE;
             }
         }
 #pragma unroll
         for (int p = 0; p < P; p++) {
-            float* to = stage + (p * NT + wave * 64) * 4;
-            if (AK) lds_fetch16(rsA, to, va[p], k0 * 4);
-            else lds_fetch16(resource(stageA), to, va[p], 0);
+            float* to = stage + (p * NT + wave * 64) * W;
+            if (AK) lds_fetch<4 * W>(rsA, to, va[p], k0 * 4);
+            else lds_fetch<4 * W>(resource(stageA), to, va[p], 0);
         }
 #pragma unroll
         for (int p = 0; p < P; p++) {
-            float* to = stage + 32 * BK + (p * NT + wave * 64) * 4;
-            if (BKC) lds_fetch16(rsB, to, vb[p], k0 * 4);
-            else lds_fetch16(resource(stageB), to, vb[p], 0);
+            float* to = stage + 32 * BK + (p * NT + wave * 64) * W;
+            if (BKC) lds_fetch<4 * W>(rsB, to, vb[p], k0 * 4);
+            else lds_fetch<4 * W>(resource(stageB), to, vb[p], 0);
         }
         stageA += (size_t)(BK * sizeof(float)) * g.lda;
         stageB += (size_t)(BK * sizeof(float)) * g.ldb;
@@ -772,14 +774,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, 
     floatx16 acc;
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[v] = 0.f;
-    fetch(smem);
-    if (nk > 1) fetch(smem + STAGE);
+    const bool sumRows = rowSums && it.n0 == 0;
+    float rowSum = 0.f;
+#pragma unroll
+    for (int i = 0; i < S - 1; i++)
+        if (i < nk) fetch(smem + i * STAGE);
+    int buf = 0, free = S - 1;
     for (int kt = 0; kt < nk; kt++) {
-        // the stage has landed, of this wavefront and then of all, while the next one is still on its way (__syncthreads would wait
-        // for that too)
-        if (kt + 1 < nk) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(2 * P) : "memory");
+        // the stage has landed, of this wavefront and then of all, while the stages after it are still on their way (__syncthreads
+        // would wait for those too)
+        if (kt + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(2 * P * (S - 2)) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
-        float* stage = smem + (kt & 1) * STAGE;
+        const float* stage = smem + buf * STAGE;
+        buf = buf == S - 1 ? 0 : buf + 1;
         const int units = (min(BK, kEnd - kBegin - kt * BK) + 7) / 8;
         constexpr int J = BK / 8 / NW;
         u32x4 a[J], b[J];
@@ -788,19 +795,30 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, 
             a[j] = fragment(AK, stage, wave + NW * j);
             b[j] = fragment(BKC, stage + 32 * BK, wave + NW * j);
         }
+        if (kt + S - 1 < nk) {   // into the buffer of stage kt - 1, whose fragments every wavefront has had since the barrier
+            fetch(smem + free * STAGE);
+            free = free == S - 1 ? 0 : free + 1;
+        }
 #pragma unroll
         for (int j = 0; j < J; j++)
             if (NW * j < units) acc = BigTraits<float>::mma(b[j], a[j], acc);   // the transposed tile (B as the row operand): a lane owns a row of C
-        if (kt + 2 < nk) {
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");   // every wavefront has its fragments
-            fetch(stage);
-        }
+        if (sumRows)
+#pragma unroll
+            for (int j = 0; j < J; j++)   // zeros past the end
+                rowSum += (__uint_as_float(a[j].x) + __uint_as_float(a[j].y)) + (__uint_as_float(a[j].z) + __uint_as_float(a[j].w));
     }
     __syncthreads();
     float* slice = smem + wave * 32 * LDC;
 #pragma unroll
     for (int q = 0; q < 4; q++) *(float4*)(slice + fr * LDC + 8 * q + 4 * half) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+    if (sumRows) smem[NW * 32 * LDC + tid] = rowSum;
     __syncthreads();
+    if (sumRows && tid < 32 && it.m0 + tid < g.M) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < 2 * NW; w++) t += smem[NW * 32 * LDC + 32 * w + tid];
+        rowSums[it.m0 + tid] += t;
+    }
     const int r = it.m0 + (tid >> 3), c = it.n0 + (tid & 7) * 4;   // four columns of a row each
     if (tid >= 256 || r >= g.M || c >= g.N) return;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -826,6 +844,40 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, 
 #pragma unroll
         for (int q = 0; q < 4; q++)
             if (c + q < g.N) cp[q] = v[q] + (g.beta != 0.f ? g.beta * cp[q] : 0.f);
+    }
+}
+
+template <int NW, int BK, bool AK, bool BKC, bool VEC, bool HEADS>
+__global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int total = g.tilesM * g.tilesN * g.parts, item = xcd_item(total);
+    if (item >= total) return;
+    F32Item it;
+    f32_item<32, 32>(g, item, it);
+    f32_small_tile<NW, BK, AK, BKC, VEC, HEADS>(g, hp, it, nullptr, reinterpret_cast<float*>(smem_raw));
+}
+
+// The gradients of an inner product whose products do not fill the chip, as one launch: w is dW += dY^T X, its tiles of the first
+// columns add the column sums of dY to db, and x is dX = dY W.  Apart they are three or four launches, each with its own first
+// fetch and end, on half the CUs.  (The ones with the longer contraction come
+// first.)  Kernel trace, us: 1024 rows, 288 to 768 11.5 + 4.0 + 10.9 + 3.9 -> 14.0, 1024 rows, 288 to 864 12.0 + 4.2 + 11.1 + 4.0 -> 19.1, 12
+// rows, 12 to 3 with the column sums 4.1 + 1.9 + 3.2 -> 3.9 (and two launches of the host's 3.6 us each fewer).
+template <int NW, int BK, bool VEC>
+__global__ __launch_bounds__(64 * NW) void linear_bwd_f32_small_kernel(GemmF32Args w, GemmF32Args x, float* db)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    float* smem = reinterpret_cast<float*>(smem_raw);
+    const int tilesW = w.tilesM * w.tilesN, tilesX = x.tilesM * x.tilesN, total = tilesW + tilesX, at = xcd_item(total);
+    if (at >= total) return;
+    const int item = w.K >= x.K ? at : at < tilesX ? tilesW + at : at - tilesX;
+    F32Item it;
+    if (item < tilesW) {
+        f32_item<32, 32>(w, item, it);
+        f32_small_tile<NW, BK, false, false, VEC, false>(w, HeadsArg<false>(), it, db, smem);
+    } else {
+        f32_item<32, 32>(x, item - tilesW, it);
+        f32_small_tile<NW, BK, true, false, VEC, false>(x, HeadsArg<false>(), it, nullptr, smem);
     }
 }
 
@@ -928,30 +980,34 @@ static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool caus
     });
 }
 
-// gemm_f32_small_kernel, microseconds: the products of the busiest CU's workgroups, and what each two of them that run at once (by LDS)
-// take for their first fetch, their stages' latencies and their end.  Within 15 % of 34 sizes.
-static double gemm_f32_small_time(int m, int n, int k, int batch)
+// gemm_f32_small_kernel, microseconds: what the workgroups of the busiest CU take for their products, and what each three of them that
+// run at once (by LDS) take for their stages' latencies.  Within 10 % of 34 sizes.
+static double gemm_f32_small_time(long long tiles, int k)
 {
-    const long long tiles = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, perCu = ((tiles + 7) / 8 + 31) / 32;
-    return 0.9 + (double)((perCu + 1) / 2) * (1.7 + 0.38 * k / 128) + (double)perCu * 0.4 * k / 128;
+    const long long perCu = ((tiles + 7) / 8 + 31) / 32;
+    return 1.7 + (double)((perCu + 2) / 3) * (0.8 + 0.28 * k / 128) + (double)perCu * (0.3 + 0.46 * k / 128);
 }
 
 // Which kernel takes a product, and its plan.  The bf16 matrix cores from 64 k on (below, the split's error is larger than that of the
 // fp32 matrix cores) and from 2^28 multiplications on (2048 x 512 x 384: 10.2 against 11.0 us; below, the chip is not full, and 16 x 288 x
 // 32000 takes 51 against 44 us); 32 x 32 tiles where their estimate is the smallest, which is a tenth of a round of the larger ones.
 enum { F32_TILES, F32_SPLIT, F32_SMALL };
-struct GemmF32Choice { int kernel; GemmF32Plan plan; };
-static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool vec, bool fp32Sums)
+struct GemmF32Choice { int kernel; GemmF32Plan plan; double time; };
+static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool vec, bool fp32Sums, bool heads = false)
 {
-    double t, tiles;
-    GemmF32Choice c = {F32_TILES, gemm_f32_plan(m, n, k, batch, causal, wsBytes, &tiles)};
-    if (!vec || fp32Sums) return c;
-    if (k >= 64 && (double)m * n * k * batch >= 268435456.0) {
-        c = {F32_SPLIT, gemm_f32_split_plan(m, n, k, batch, causal, wsBytes, &t)};
-        tiles = t;   // faster than the fp32 matrix cores at every size from there on
+    GemmF32Choice c;
+    c.kernel = F32_TILES;
+    c.plan = gemm_f32_plan(m, n, k, batch, causal, wsBytes, &c.time);
+    if (fp32Sums) return c;
+    if (vec && k >= 64 && (double)m * n * k * batch >= 268435456.0) {   // faster than the fp32 matrix cores at every size from there on
+        c.kernel = F32_SPLIT;
+        c.plan = gemm_f32_split_plan(m, n, k, batch, causal, wsBytes, &c.time);
     }
-    // a launch is in this estimate and not in the others
-    if (gemm_f32_small_time(m, n, k, batch) < tiles + 1.8) c = {F32_SMALL, {0, 1, k}};
+    c.time += 1.8;   // a launch, which the next estimate holds
+    // the heads epilogue of 16 rows and more a lane, one after the other (1024 x 864 x 288: 13.3 us, 9.3 without it)
+    if (heads) c.time += 3;
+    const double t = gemm_f32_small_time((long long)((m + 31) / 32) * ((n + 31) / 32) * batch, k);
+    if (t < c.time) c = {F32_SMALL, {0, 1, k}, t};
     return c;
 }
 
@@ -1025,11 +1081,14 @@ static hipError_t launch_split_shape(hipStream_t s, const GemmF32Args& a, const 
     return hipErrorInvalidValue;
 }
 
-template <int NW, int BK, bool AK, bool BKC, bool HEADS>
+// LDS of gemm_f32_small_kernel: the stages, in which the sums find room at the end
+template <int NW, int BK> constexpr int small_lds() { static_assert(SMALL_STAGES * 2 * 32 * BK >= NW * (32 * 36 + 64), ""); return SMALL_STAGES * 2 * 32 * BK * (int)sizeof(float); }
+
+template <int NW, int BK, bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_small(hipStream_t s, const GemmF32Args& a, int batch, const HeadsEpilogue* he)
 {
-    constexpr int stages = 2 * 2 * 32 * BK * (int)sizeof(float), sums = NW * 32 * 36 * (int)sizeof(float), lds = stages > sums ? stages : sums;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_small_kernel<NW, BK, AK, BKC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    constexpr int lds = small_lds<NW, BK>();
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_small_kernel<NW, BK, AK, BKC, VEC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     GemmF32Args g = a;
     g.tilesM = (g.M + 31) / 32;
@@ -1039,18 +1098,22 @@ static hipError_t launch_small(hipStream_t s, const GemmF32Args& a, int batch, c
     const long long total = (long long)g.tilesM * g.tilesN * batch;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
     const int per = (int)((total + 7) / 8);
-    hipLaunchKernelGGL((gemm_f32_small_kernel<NW, BK, AK, BKC, HEADS>), dim3(per * 8), 64 * NW, lds, s, g, heads_arg<HEADS>(he));
+    hipLaunchKernelGGL((gemm_f32_small_kernel<NW, BK, AK, BKC, VEC, HEADS>), dim3(per * 8), 64 * NW, lds, s, g, heads_arg<HEADS>(he));
     return hipGetLastError();
 }
 
-// operands in whole aligned 16-byte chunks
-template <bool AK, bool BKC, bool HEADS>
+// VEC: operands in whole aligned 16-byte chunks
+template <bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_layout(hipStream_t s, const GemmF32Args& a, const GemmF32Choice& c, int batch, const HeadsEpilogue* he)
 {
-    if (c.kernel == F32_SMALL) return launch_small<4, 128, AK, BKC, HEADS>(s, a, batch, he);
-    if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, HEADS>(s, a, c.plan, batch, he);
-    return launch_f32_tile<AK, BKC, true, HEADS>(s, a, c.plan, batch, he);
+    if (c.kernel == F32_SMALL) return launch_small<4, 64, AK, BKC, VEC, HEADS>(s, a, batch, he);
+    if constexpr (VEC)
+        if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, HEADS>(s, a, c.plan, batch, he);
+    return launch_f32_tile<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
 }
+
+// 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
+static bool f32_near(bool kFast, int rows, int k, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(k, 128) * ld + 256) < (1ll << 29); }
 
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
 {
@@ -1071,18 +1134,16 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     } else {
         a.vecC = q.n % 4 == 0 && q.ldc % 4 == 0 && (q.batch == 1 || q.sC % 4 == 0) && ((uintptr_t)q.C & 15) == 0;
     }
-    // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
-    auto near = [&](bool kFast, int rows, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(q.k, 128) * ld + 256) < (1ll << 29); };
-    const bool vec = (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
-                     (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0) &&
-                     near(q.aK, q.m, q.lda) && near(q.bK, q.n, q.ldb);
+    const bool near = f32_near(q.aK, q.m, q.k, q.lda) && f32_near(q.bK, q.n, q.k, q.ldb);
+    const bool vec = near && (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
+                     (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0);
     if (!ws || ((uintptr_t)ws & 15)) wsBytes = 0;
-    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, vec, q.fp32Sums);
+    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, vec, q.fp32Sums || !near, q.heads != nullptr);
     const GemmF32Plan& p = choice.plan;
     a.kChunk = p.kChunk;
     hipError_t e;
-    if (q.heads) e = vec ? launch_layout<true, true, true>(s, a, choice, 1, q.heads) : launch_f32_tile<true, true, false, true>(s, a, p, 1, q.heads);
-#define LAYOUT(AKV, BKV) (vec ? launch_layout<AKV, BKV, false>(s, a, choice, q.batch, nullptr) : launch_f32_tile<AKV, BKV, false, false>(s, a, p, q.batch))
+    if (q.heads) e = vec ? launch_layout<true, true, true, true>(s, a, choice, 1, q.heads) : launch_layout<true, true, false, true>(s, a, choice, 1, q.heads);
+#define LAYOUT(AKV, BKV) (vec ? launch_layout<AKV, BKV, true, false>(s, a, choice, q.batch, nullptr) : launch_layout<AKV, BKV, false, false>(s, a, choice, q.batch, nullptr))
     else if (q.aK) e = q.bK ? LAYOUT(true, true) : LAYOUT(true, false);
     else e = q.bK ? LAYOUT(false, true) : LAYOUT(false, false);
 #undef LAYOUT
@@ -1091,6 +1152,53 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     const int grid = (int)std::min<size_t>((quads + 255) / 256, 4096);
     if (q.heads) hipLaunchKernelGGL(gemm_f32_sum_kernel<true>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, heads_arg<true>(q.heads));
     else hipLaunchKernelGGL(gemm_f32_sum_kernel<false>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, HeadsArg<false>());
+    return hipGetLastError();
+}
+
+// The gradients of an inner product as one launch, if that is what the sizes call for (*done): dW (n x k) += dY^T (n x m) X (m x k),
+// db (n, or null) += column sums of dY, dX (m x k) = dY W (n x k) + beta dX.
+hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float* X, const float* W, const float* dY, float* dW, float* db, float* dX, float beta,
+                                bool* done)
+{
+    *done = false;
+    // what is written lies apart from everything else: the three calls, one after the other, may share memory
+    const struct { const float* p; size_t n; bool out; } mem[] = {{dW, (size_t)n * k, true}, {dX, (size_t)m * k, true}, {db, db ? (size_t)n : 0, true},
+                                                                 {X, (size_t)m * k, false}, {W, (size_t)n * k, false}, {dY, (size_t)m * n, false}};
+    for (int i = 0; i < 3; i++)
+        for (int j = i + 1; j < 6; j++)
+            if (mem[i].n && mem[j].n && mem[i].p < mem[j].p + mem[j].n && mem[j].p < mem[i].p + mem[i].n) return hipSuccess;
+    if (!f32_near(false, n, m, n) || !f32_near(false, k, m, k) || !f32_near(true, m, n, n) || !f32_near(false, k, n, k)) return hipSuccess;
+    const bool vec = ((((uintptr_t)X | (uintptr_t)W | (uintptr_t)dY) & 15) == 0) && n % 4 == 0 && k % 4 == 0;
+    const long long tilesK = (k + 31) / 32, tilesW = (n + 31) / 32 * tilesK, tilesX = (m + 31) / 32 * tilesK;
+    if (tilesW + tilesX > (1ll << 20)) return hipSuccess;
+    // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
+    // time that one launch waits for the last one's stores
+    const double apart = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, vec, false).time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, vec, false).time + 2.5 +
+                         (db ? m <= 1024 ? 4.5 : 9.0 : 0.0);
+    if (gemm_f32_small_time(tilesW + tilesX, std::max(m, n)) >= apart) return hipSuccess;
+    GemmF32Args w = {}, x = {};
+    w.M = n; w.N = k; w.K = w.kChunk = m;
+    w.A = dY; w.B = X; w.C = dW;
+    w.lda = n; w.ldb = k; w.ldc = k;
+    w.alpha = 1.f; w.beta = 1.f; w.parts = 1;
+    w.vecC = k % 4 == 0 && ((uintptr_t)dW & 15) == 0;
+    w.tilesM = (n + 31) / 32; w.tilesN = (int)tilesK;
+    x.M = m; x.N = k; x.K = x.kChunk = n;
+    x.A = dY; x.B = W; x.C = dX;
+    x.lda = n; x.ldb = k; x.ldc = k;
+    x.alpha = 1.f; x.beta = beta; x.parts = 1;
+    x.vecC = k % 4 == 0 && ((uintptr_t)dX & 15) == 0;
+    x.tilesM = (m + 31) / 32; x.tilesN = (int)tilesK;
+    constexpr int lds = small_lds<4, 64>();
+    static const hipError_t attr = [] {
+        const hipError_t e = hipFuncSetAttribute((const void*)linear_bwd_f32_small_kernel<4, 64, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        return e != hipSuccess ? e : hipFuncSetAttribute((const void*)linear_bwd_f32_small_kernel<4, 64, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    }();
+    if (attr != hipSuccess) return attr;
+    const int grid = (int)((tilesW + tilesX + 7) / 8) * 8;
+    *done = true;
+    if (vec) hipLaunchKernelGGL((linear_bwd_f32_small_kernel<4, 64, true>), grid, 256, lds, s, w, x, db);
+    else hipLaunchKernelGGL((linear_bwd_f32_small_kernel<4, 64, false>), grid, 256, lds, s, w, x, db);
     return hipGetLastError();
 }
 

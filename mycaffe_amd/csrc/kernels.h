@@ -166,6 +166,8 @@ hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float a
 size_t k_gemv_workspace_bytes(bool tA, int m, int n);   // scratch for the partial sums of a transposed product over many rows
 hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, const void* A, const float* x,
                   float beta, float* y, void* ws = nullptr, size_t wsBytes = 0);
+hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float* X, const float* W, const float* dY, float* dW, float* db, float* dX, float beta,
+                                bool* done);   // the gradients of an inner product as one launch, where sizes and memory allow (*done)
 size_t k_bias_grad_workspace_bytes(int m, int n);
 hipError_t k_bias_grad(hipStream_t s, DType dt, int m, int n, const void* dY, void* db, void* ws, size_t wsBytes);   // db += column sums
 

@@ -2230,6 +2230,17 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (dB) RANGE(dB, 0, N);
         if (dX) RANGE(dX, 0, M * K);
         const DType dt = X->dt();
+        if (dt == F32 && dX) {
+            bool done;
+            HIPCHK(linear_bwd_f32_small(s, (int)M, (int)N, (int)K, (const float*)X->ptr, (const float*)W->ptr, (const float*)dY->ptr, (float*)dW->ptr,
+                                        dB ? (float*)dB->ptr : nullptr, (float*)dX->ptr, accum ? 1.f : 0.f, &done));
+            if (done) {
+                m_mem.touch((long)pl[6]);
+                if (dB) m_mem.touch((long)pl[7]);
+                m_mem.touch((long)pl[8]);
+                return 0;
+            }
+        }
         const size_t wsW = k_gemm_workspace_bytes(dt, true, false, (int)N, (int)K, (int)M), wsB = dB ? k_bias_grad_workspace_bytes((int)M, (int)N) : 0;
         const size_t wsX = dX ? k_gemm_workspace_bytes(dt, false, false, (int)M, (int)K, (int)N) : 0, most = std::max(wsW, std::max(wsB, wsX));
         void* ws = nullptr;

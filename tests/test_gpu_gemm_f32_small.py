@@ -71,3 +71,46 @@ def test_infinities_and_nan(dev):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[[5, 95]], want[[5, 95]].astype(np.float32))
     rest = np.setdiff1d(np.arange(m), [5, 40, 95])
     assert np.isfinite(got[rest]).all()
+
+
+# odd sizes and operands that begin anywhere: 4 bytes a lane
+@pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(33, 31, 3), (12, 3, 12), (65, 130, 127), (129, 34, 129), (31, 97, 257), (1, 5, 1023)])
+def test_odd_sizes(dev, m, n, k, tA, tB):
+    rng = np.random.default_rng(m + n + k)
+    a, b, c = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n), (m, n)))
+    ha, hb, hc = dev.put((a.T if tA else a).copy()), dev.put((b.T if tB else b).copy()), dev.put(c)
+    want, scale = a.astype(np.float64) @ b.astype(np.float64), np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64))
+    dev.cuda.gemm(tA, tB, m, n, k, 2.0, ha, hb, 1.0, hc)
+    assert (np.abs(dev.get(hc, (m, n)) - (c + 2 * want)) <= BOUND(k) * (2 * scale + np.abs(c))).all()
+
+
+# the gradients of an inner product as one launch: the longer contraction in either, edges of tiles and stages, with and without bias,
+# data gradients that are added up; and memory that the three results or the operands share, which takes the calls one by one
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("m,n,k", [(12, 3, 3), (12, 12, 3), (64, 64, 64), (1024, 288, 288), (256, 768, 96), (33, 131, 65), (1, 40, 36), (1030, 100, 32), (7, 500, 12)])
+def test_gradients_of_an_inner_product(dev, m, n, k, bias):
+    rng = np.random.default_rng(m + n + k)
+    x, w, dy, dw, db, dx = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (n, k), (m, n), (n, k), (n,), (m, k)))
+    x64, w64, dy64 = (v.astype(np.float64) for v in (x, w, dy))
+    for accumulate in (False, True):
+        hdw, hdb, hdx = dev.put(dw), dev.put(db), dev.put(dx)
+        dev.cuda.LinearBackward(m, n, k, dev.put(x), dev.put(w), dev.put(dy), hdw, hdb if bias else 0, hdx, accumulate)
+        scale = np.abs(dy64).T @ np.abs(x64) + np.abs(dw)
+        assert (np.abs(dev.get(hdw, (n, k)) - (dw + dy64.T @ x64)) <= BOUND(m) * scale).all()
+        scale = np.abs(dy64) @ np.abs(w64) + np.abs(dx)
+        assert (np.abs(dev.get(hdx, (m, k)) - (accumulate * dx + dy64 @ w64)) <= BOUND(n) * scale).all()
+        want = db + dy64.sum(0) if bias else db
+        assert (np.abs(dev.get(hdb, (n,)) - want) <= BOUND(m) * (np.abs(dy64).sum(0) + np.abs(db))).all()
+
+
+def test_gradients_of_an_inner_product_in_shared_memory(dev):
+    # the data gradient over the input, which the calls one after the other allow: the weight gradient has been made by then
+    rng = np.random.default_rng(1)
+    m = n = k = 64
+    x, w, dy = (rng.standard_normal((64, 64), dtype=np.float32) for _ in range(3))
+    hx, hdw, hdb = dev.put(x), dev.zeros(n * k), dev.zeros(n)
+    dev.cuda.LinearBackward(m, n, k, hx, dev.put(w), dev.put(dy), hdw, hdb, hx)
+    x, w, dy = (v.astype(np.float64) for v in (x, w, dy))
+    for h, want in ((hx, dy @ w), (hdw, dy.T @ x), (hdb, dy.sum(0))):
+        assert np.abs(dev.get(h, want.shape) - want).max() <= 1e-5 * np.abs(want).max()
