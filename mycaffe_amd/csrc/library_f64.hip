@@ -19,6 +19,7 @@
 #include <string>
 #include <vector>
 
+#include "gemm_f64.h"
 #include "runtime.h"
 
 namespace mch {
@@ -94,132 +95,6 @@ __global__ void d_mask_kernel(size_t n, size_t md1, size_t dd1, const double* x,
     GRID_STRIDE(i, n) y[i] = mask[i % md1 + (i / dd1) * md1] == search ? replace : x[i];
 }
 
-// C(i,j) = alpha sum_k A(i,k) B(k,j) + beta C(i,j) with any element strides, on the double matrix cores
-// (v_mfma_f64_16x16x4_f64: lane l holds A(l % 16, l / 16) and B(l / 16, l % 16) of a step, register v of the result is row
-// 4 v + l / 16, column l % 16).  2 x 2 wavefronts of W x W MFMA tiles each, stages of 16 k double-buffered in LDS as
-// [row][k] with 18 doubles a row (conflict-free 64-bit reads), the next stage held in registers meanwhile.  An operand is
-// fetched along whichever index lies at unit stride.
-// The layers of this type are small: a product is some dozens of tiles and what bounds it is the latency of one stage after
-// the other.  G groups of four wavefronts of a workgroup therefore take every G-th stage each, with stages of their own, and
-// their sums are added in order through LDS at the end (256 x 256 x 1024: 27 us with one group, 9 us with four; one output
-// per thread took 45 us).
-// zdiv: matrix z of C lies at (z / zdiv) sC + (z % zdiv) sC2.  bias (may be null): one value per column, added to every row.
-typedef double d_vec4 __attribute__((ext_vector_type(4)));
-struct GemmD { int m, n, k; double alpha, beta; const double *A, *B; double* C; long long ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2; int zdiv; const double* bias; };
-template <int W, int G> __global__ __launch_bounds__(256 * G) void d_gemm_kernel(GemmD g)
-{
-    constexpr int BT = 32 * W, BK = 16, LD = BK + 2, NE = BT * BK / 256, STAGE = 2 * BT * LD;
-    extern __shared__ double d_smem[];
-    const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-    double* stages = d_smem + group * 2 * STAGE;   // two of this group
-    const int m0 = blockIdx.y * BT, n0 = blockIdx.x * BT, wm = (wave >> 1) * 16 * W, wn = (wave & 1) * 16 * W;
-    const double* A = g.A + (size_t)blockIdx.z * g.sA;
-    const double* B = g.B + (size_t)blockIdx.z * g.sB;
-    double* C = g.C + (size_t)(blockIdx.z / g.zdiv) * g.sC + (size_t)(blockIdx.z % g.zdiv) * g.sC2;
-    const bool ak = g.acs == 1, bk = g.brs == 1;
-    d_vec4 acc[W][W];
-#pragma unroll
-    for (int i = 0; i < W; i++)
-#pragma unroll
-        for (int j = 0; j < W; j++) acc[i][j] = d_vec4{0.0, 0.0, 0.0, 0.0};
-    double ra[NE], rb[NE];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int q = 0; q < NE; q++) {
-            const int e = tid + 256 * q;
-            const int ia = ak ? e / BK : e % BT, ka = ak ? e % BK : e / BT;
-            const int jb = bk ? e / BK : e % BT, kb = bk ? e % BK : e / BT;
-            ra[q] = (m0 + ia < g.m && k0 + ka < g.k) ? A[(long long)(m0 + ia) * g.ars + (long long)(k0 + ka) * g.acs] : 0.0;
-            rb[q] = (n0 + jb < g.n && k0 + kb < g.k) ? B[(long long)(k0 + kb) * g.brs + (long long)(n0 + jb) * g.bcs] : 0.0;
-        }
-    };
-    auto put = [&](int buf) {
-        double *as = stages + buf * STAGE, *bs = as + BT * LD;
-#pragma unroll
-        for (int q = 0; q < NE; q++) {
-            const int e = tid + 256 * q;
-            as[ak ? (e / BK) * LD + e % BK : (e % BT) * LD + e / BT] = ra[q];
-            bs[bk ? (e / BK) * LD + e % BK : (e % BT) * LD + e / BT] = rb[q];
-        }
-    };
-    // trips are the same for every group: stages past the end are zeros
-    const int trips = (g.k + BK * G - 1) / (BK * G), fr = lane & 15, fk = lane >> 4;
-    fetch(group * BK);
-    put(0);
-    __syncthreads();
-    for (int kt = 0; kt < trips; kt++) {
-        const double *as = stages + (kt & 1) * STAGE, *bs = as + BT * LD;
-        if (kt + 1 < trips) fetch(((kt + 1) * G + group) * BK);
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 4) {
-            double a[W], b[W];
-#pragma unroll
-            for (int t = 0; t < W; t++) {
-                a[t] = as[(wm + 16 * t + fr) * LD + kk + fk];
-                b[t] = bs[(wn + 16 * t + fr) * LD + kk + fk];
-            }
-#pragma unroll
-            for (int i = 0; i < W; i++)
-#pragma unroll
-                for (int j = 0; j < W; j++) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (kt + 1 < trips) put((kt & 1) ^ 1);
-        __syncthreads();
-    }
-    if (G > 1) {
-        // group q > 0 leaves its sums at [q - 1][register][thread]; group 0 adds them
-        constexpr int NR = W * W * 4;
-        if (group > 0) {
-#pragma unroll
-            for (int i = 0; i < W; i++)
-#pragma unroll
-                for (int j = 0; j < W; j++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) d_smem[((group - 1) * NR + (i * W + j) * 4 + v) * 256 + tid] = acc[i][j][v];
-        }
-        __syncthreads();
-        if (group > 0) return;
-        for (int q = 0; q < G - 1; q++)
-#pragma unroll
-            for (int i = 0; i < W; i++)
-#pragma unroll
-                for (int j = 0; j < W; j++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) acc[i][j][v] += d_smem[(q * NR + (i * W + j) * 4 + v) * 256 + tid];
-    }
-#pragma unroll
-    for (int i = 0; i < W; i++)
-#pragma unroll
-        for (int j = 0; j < W; j++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = m0 + wm + 16 * i + 4 * v + fk, c = n0 + wn + 16 * j + fr;
-                if (r >= g.m || c >= g.n) continue;
-                double* cp = C + (long long)r * g.crs + (long long)c * g.ccs;
-                double t = g.alpha * acc[i][j][v];
-                if (g.bias) t += g.bias[c];
-                *cp = g.beta == 0.0 ? t : t + g.beta * *cp;
-            }
-}
-// 64 x 64 tiles once they give every CU one, 32 x 32 below; four groups while the workgroups leave CUs to spare (two of
-// them fit a CU) and the contraction has stages for them
-static hipError_t d_gemm(hipStream_t s, int batch, int m, int n, int k, double alpha, const double* A, long long ars, long long acs, const double* B,
-                         long long brs, long long bcs, double beta, double* C, long long crs, long long ccs, long long sA, long long sB, long long sC,
-                         int zdiv = 1, long long sC2 = 0, const double* bias = nullptr)
-{
-    GemmD g = {m, n, k, alpha, beta, A, B, C, ars, acs, brs, bcs, crs, ccs, sA, sB, sC, sC2, zdiv, bias};
-    const long long big = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch, small = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch;
-    const dim3 gridBig((n + 63) / 64, (m + 63) / 64, batch), gridSmall((n + 31) / 32, (m + 31) / 32, batch);
-    if (gridSmall.y > 65535) return hipErrorInvalidValue;
-    if (big >= 256) hipLaunchKernelGGL((d_gemm_kernel<2, 1>), gridBig, 256, 2 * 2 * 64 * 18 * 8, s, g);
-    else if (small <= 512 && k >= 128) {
-        constexpr int lds = 4 * 2 * 2 * 32 * 18 * 8;
-        static const hipError_t attr = hipFuncSetAttribute((const void*)d_gemm_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (attr != hipSuccess) return attr;
-        hipLaunchKernelGGL((d_gemm_kernel<1, 4>), gridSmall, 1024, lds, s, g);
-    } else hipLaunchKernelGGL((d_gemm_kernel<1, 1>), gridSmall, 256, 2 * 2 * 32 * 18 * 8, s, g);
-    return hipGetLastError();
-}
 // y (n) = alpha A^T x + beta y, A row-major (m, n): 16 columns by 64 rows a trip, sums of the 64 row lanes added in order
 __global__ __launch_bounds__(1024) void d_gemv_t_kernel(int m, int n, double alpha, const double* A, const double* x, double beta, double* y)
 {
@@ -2164,6 +2039,12 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(W, 0, N * K);
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
+        if (heads) {
+            const HeadsD he = {{Y->ptr, Y->ptr, Y->ptr}, (int)T, (int)heads, (int)(N / heads), nullptr, nullptr, 1};
+            bool done;
+            HIPCHK(d_gemm_heads(s, (int)M, (int)N, (int)K, (const double*)X->ptr, (const double*)W->ptr, Bi ? (const double*)Bi->ptr : nullptr, he, &done));
+            if (done) return 0;
+        }
         double* out = Y->ptr;
         if (heads) ERRCHK(workspace((size_t)(M * N), &out));
         HIPCHK(d_gemm(s, 1, (int)M, (int)N, (int)K, 1.0, (const double*)X->ptr, K, 1ll, (const double*)W->ptr, 1ll, K, 0.0, out, N, 1ll, 0ll, 0ll, 0ll,
@@ -2190,6 +2071,12 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         RANGE(dW, 0, N * K);
         if (dB) RANGE(dB, 0, N);
         if (dX) RANGE(dX, 0, M * K);
+        if (dX) {
+            bool done;
+            HIPCHK(d_linear_bwd_small(s, (int)M, (int)N, (int)K, (const double*)X->ptr, (const double*)W->ptr, (const double*)dY->ptr, dW->ptr, dB ? dB->ptr : nullptr,
+                                      dX->ptr, accum ? 1.0 : 0.0, &done));
+            if (done) return 0;
+        }
         HIPCHK(d_gemm(s, 1, (int)N, (int)K, (int)M, 1.0, (const double*)dY->ptr, 1ll, N, (const double*)X->ptr, K, 1ll, 1.0, dW->ptr, K, 1ll, 0ll, 0ll, 0ll));
         if (dB) hipLaunchKernelGGL(d_colsum_add_kernel, (int)((N + 15) / 16), 1024, 0, s, (int)M, (int)N, (const double*)dY->ptr, dB->ptr);
         LAUNCHED();
@@ -2224,6 +2111,12 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
                 last_detail = "the rope handle was created for other heads or another head size";
                 return MCH_ERROR_PARAM_OUT_OF_RANGE;
             }
+        }
+        const HeadsD he = {{Q->ptr, K->ptr, V->ptr}, (int)T, (int)H, (int)hs, r ? (const double*)r->dcos : nullptr, r ? (const double*)r->dsin : nullptr, r ? r->seq : 1};
+        if (!(hs & 1) || !r) {
+            bool done;
+            HIPCHK(d_gemm_heads(s, (int)M, (int)(3 * C), (int)C, (const double*)X->ptr, (const double*)W->ptr, Bi ? (const double*)Bi->ptr : nullptr, he, &done));
+            if (done) return 0;
         }
         double* tmp;
         ERRCHK(workspace((size_t)(M * 3 * C), &tmp));
