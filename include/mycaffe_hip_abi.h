@@ -213,6 +213,9 @@ enum {
      * normalised into y; hLayerNorm != 0 runs that handle, 0 the RMS norm of RMSNORM_FWD over rows of dim values:
      *   f{eps}  l{hLayerNorm, rows, dim, hX, hAdd, hTotal, hWeight (0 = none), hY}
      * Backward (layer norm handle): dX = the gradient of LAYERNORM_BWD plus hAdd's values:  l{hLayerNorm, hY, hdY, hdX, hAdd}
+     *
+     * LINEAR_HEADS_GROUP: the projections of a multi-head attention layer as one call, each as LINEAR_FWD with T and heads:
+     *   l{count (2 or 3), N, K, heads, then M, T, hX, hWeight, hBias (0 = none), hY of each}
      */
     MCH_FN_ATTN_DECODE_FWD = 2001,
     MCH_FN_RMSNORM_FWD = 2002,
@@ -224,7 +227,8 @@ enum {
     MCH_FN_RMSNORM_BWD = 2008,
     MCH_FN_SWIGLU_BWD = 2009,
     MCH_FN_NORM_ADD_FWD = 2010,
-    MCH_FN_NORM_ADD_BWD = 2011
+    MCH_FN_NORM_ADD_BWD = 2011,
+    MCH_FN_LINEAR_HEADS_GROUP = 2012
 };
 
 /* DEVINIT flags (CudaDnnDLL/Cuda Files/device.h:18-22) */

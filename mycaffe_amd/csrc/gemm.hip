@@ -736,6 +736,30 @@ hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int h
     return gemm_heads_dispatch(s, dt, B * T, H * hs, k, X, W, he, nullptr, ws, wsBytes, fp32Sums);
 }
 
+hipError_t k_gemm_bias_heads_group(hipStream_t s, int count, int n, int k, int H, const HeadsProjection* p, bool* done)
+{
+    *done = false;
+    if (count < 2 || count > 3) return hipSuccess;
+    HeadsEpilogue he[3];
+    GemmB16 q[3];
+    for (int i = 0; i < count; i++) {
+        he[i] = heads_epilogue(p[i].bias, p[i].Y, p[i].Y, p[i].Y, p[i].T, H, n / H, nullptr, nullptr, 1);
+        q[i] = b16_product(false, true, p[i].m, n, k, 1.f, p[i].X, p[i].W, 0.f, nullptr);
+        q[i].heads = &he[i];
+    }
+    // a result over another product's operand or result: one after the other
+    auto apart = [](const void* a, size_t na, const void* b, size_t nb) { return !a || !b || (const bf16_t*)a + na <= (const bf16_t*)b || (const bf16_t*)b + nb <= (const bf16_t*)a; };
+    for (int i = 0; i < count; i++)
+        for (int j = 0; j < count; j++) {
+            const size_t out = (size_t)p[i].m * n;
+            if (!apart(p[i].Y, out, p[j].X, (size_t)p[j].m * k) || !apart(p[i].Y, out, p[j].W, (size_t)n * k) || !apart(p[i].Y, out, p[j].bias, n) ||
+                (i != j && !apart(p[i].Y, out, p[j].Y, (size_t)p[j].m * n))) return hipSuccess;
+        }
+    hipError_t e = hipSuccess;
+    *done = gemm_b16_group(s, q, count, &e);
+    return e;
+}
+
 // C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
 // split = false: A is X rounded to bf16, m rows of k.  split = true keeps the activations' precision: A holds every row of
 // an fp32 X as two bf16 rows back to back, the bf16 nearest to each of its k values and then the bf16 nearest to what

@@ -90,8 +90,9 @@ __device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<
     }
 }
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS>
-__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
+// tile `item` of a product
+template <int WVM, int WVN, int WM, int WN, bool AK, bool BKC, bool HEADS>
+__device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HEADS>& hp, int item)
 {
     constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64, KS = 4;
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;               // 16-byte chunks per thread and stage
@@ -101,9 +102,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     bf16_t* smem = reinterpret_cast<bf16_t*>(smem_raw);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tiles = g.tilesM * g.tilesN, total = tiles * g.parts, per = (total + 7) / 8;
-    const int item = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);   // each XCD takes a contiguous run
-    if (item >= total) return;
+    const int tiles = g.tilesM * g.tilesN;
     const int part = item / tiles, tile = item - part * tiles;
     constexpr int GROUP = 4;   // tile rows per group, walked down first: few rows of A and columns of B in flight per XCD
     const int group = tile / (GROUP * g.tilesN), inGroup = tile - group * GROUP * g.tilesN;
@@ -304,6 +303,28 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
         }
 }
 
+// each XCD (workgroup index mod 8) takes a contiguous run of the tiles
+__device__ __forceinline__ int b16_xcd_item(int total) { return (int)(blockIdx.x % 8) * ((total + 7) / 8) + (int)(blockIdx.x / 8); }
+
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS>
+__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
+{
+    const int total = g.tilesM * g.tilesN * g.parts, item = b16_xcd_item(total);
+    if (item < total) b16_tile<WVM, WVN, WM, WN, AK, BKC, HEADS>(g, hp, item);
+}
+
+// Up to three products with heads epilogues as one launch: the projections of a multi-head attention layer.  One by one each is less
+// than two rounds of the chip with its own first fetches and last stores (4096 and twice 8192 rows, 512 to 512: @GROUPDOC@).
+struct GemmB16Group { GemmB16Args g[3]; HeadsArg<true> h[3]; int first[4]; };   // first: of the tiles of all, of each; then their number
+template <int WVM, int WVN, int WM, int WN, int OCC>
+__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_group_kernel(GemmB16Group grp)
+{
+    const int item = b16_xcd_item(grp.first[3]);
+    if (item >= grp.first[3]) return;
+    const int p = item >= grp.first[2] ? 2 : item >= grp.first[1] ? 1 : 0;
+    b16_tile<WVM, WVN, WM, WN, true, true, true>(grp.g[p], grp.h[p], item - grp.first[p]);
+}
+
 // sum over the S partial products in their order, then as b16_store8
 template <bool HEADS>
 __global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<HEADS> hp, int S)
@@ -346,6 +367,13 @@ static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 15.0, 7.5}, {25
                                            {128, 128, 4.2, 3.5, 7.0, 4.2}, {64, 128, 3.7, 1.3, 6.0, 1.5}, {64, 64, 2.5, 0.9, 4.1, 0.9}};
 enum { B16_128X192 = 2, B16_128X192_ALONE = 6 };
 
+static double b16_time(const GemmB16Shape& s, long long tiles, int k)
+{
+    const double len = ((k + 63) / 64 * 64) / 768.0;
+    const long long perCu = ((tiles + 7) / 8 + 31) / 32;
+    return perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends);
+}
+
 static GemmB16Plan gemm_b16_plan(int m, int n, int k)
 {
     GemmB16Plan best = {5, 1, k};
@@ -357,9 +385,8 @@ static GemmB16Plan gemm_b16_plan(int m, int n, int k)
             if (S > 1 && k / S < 256) break;
             const int chunk = ((k + S - 1) / S + 63) / 64 * 64;
             if ((k + chunk - 1) / chunk != S) continue;
-            const double len = ((chunk + 63) / 64 * 64) / 768.0;
             const long long perCu = ((tiles * S + 7) / 8 + 31) / 32;
-            double t = perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends);
+            double t = b16_time(s, tiles * S, chunk);
             if (S > 1) t += 4.0 + (double)(S + 1) * m * n * 4.0 / 4.0e6;
             if (t < bestT) { bestT = t; best = {sh == B16_128X192 && perCu == 1 ? B16_128X192_ALONE : sh, S, S > 1 ? chunk : k}; }
         }
@@ -415,18 +442,14 @@ static hipError_t launch_b16_shape(hipStream_t s, const GemmB16Args& a, int shap
     }
 }
 
-hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
+static GemmB16Args b16_args(const GemmB16& q)
 {
-    if (!gemm_b16_takes(q) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || !q.aK || !q.bK))) return hipErrorInvalidValue;
-    GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
-    if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
     GemmB16Args a = {};
-    a.M = q.m; a.N = q.n; a.K = q.k;
+    a.M = q.m; a.N = q.n; a.K = a.kChunk = q.k;
     a.A = q.A; a.B = q.B; a.C = q.C;
     a.lda = q.aK ? q.k : q.m; a.ldb = q.bK ? q.k : q.n;
     a.alpha = q.alpha; a.beta = q.beta;
-    a.parts = p.splits; a.kChunk = p.kChunk;
-    a.part = (float*)ws;
+    a.parts = 1;
     a.bias = q.heads ? (const bf16_t*)q.heads->bias : q.bias;
     if (q.heads) {
         const HeadsEpilogue& he = *q.heads;
@@ -434,6 +457,17 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
     } else {
         a.vecC = q.n % 8 == 0 && ((uintptr_t)q.C & 15) == 0;
     }
+    return a;
+}
+
+hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
+{
+    if (!gemm_b16_takes(q) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || !q.aK || !q.bK))) return hipErrorInvalidValue;
+    GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
+    if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
+    GemmB16Args a = b16_args(q);
+    a.parts = p.splits; a.kChunk = p.kChunk;
+    a.part = (float*)ws;
     hipError_t e;
     if (q.heads) e = launch_b16_shape<true, true, true>(s, a, p.shape, q.heads);
     else if (q.aK) e = q.bK ? launch_b16_shape<true, true, false>(s, a, p.shape) : launch_b16_shape<true, false, false>(s, a, p.shape);
@@ -443,6 +477,63 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
     if (q.heads) hipLaunchKernelGGL(gemm_b16_sum_kernel<true>, grid, 256, 0, s, a, heads_arg<true>(q.heads), p.splits);
     else hipLaunchKernelGGL(gemm_b16_sum_kernel<false>, grid, 256, 0, s, a, HeadsArg<false>(), p.splits);
     return hipGetLastError();
+}
+
+template <int WVM, int WVN, int WM, int WN, int OCC>
+static hipError_t launch_b16_group(hipStream_t s, GemmB16Group& grp, int count)
+{
+    constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN, CH = WN % 2 == 0 ? 2 : WN;
+    constexpr int stages = 2 * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_group_kernel<WVM, WVN, WM, WN, OCC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    long long total = 0;
+    for (int p = 0; p < 3; p++) {
+        GemmB16Args& g = grp.g[p];
+        grp.first[p] = (int)total;
+        if (p >= count) continue;
+        g.tilesM = (g.M + BM - 1) / BM;
+        g.tilesN = (g.N + BN - 1) / BN;
+        total += (long long)g.tilesM * g.tilesN;
+        if (total > (1ll << 27)) return hipErrorInvalidValue;
+    }
+    grp.first[3] = (int)total;
+    for (int p = count; p < 3; p++) grp.first[p] = (int)total;
+    hipLaunchKernelGGL((gemm_b16_group_kernel<WVM, WVN, WM, WN, OCC>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, grp);
+    return hipGetLastError();
+}
+
+// `count` (2 or 3) products A B^T through their heads epilogues, all of one n and k, as one launch.  False: a product is none that
+// gemm_b16 takes, or they are too few rows to fill a CU each (gemm_b16 may cut those in parts).
+bool gemm_b16_group(hipStream_t s, const GemmB16* q, int count, hipError_t* e)
+{
+    GemmB16Group grp = {};
+    for (int p = 0; p < count; p++) {
+        if (!gemm_b16_takes(q[p]) || !q[p].heads || !q[p].aK || !q[p].bK || q[p].n != q[0].n || q[p].k != q[0].k) return false;
+        grp.g[p] = b16_args(q[p]);
+        grp.h[p].he = *q[p].heads;
+    }
+    int best = 0;
+    double bestT = 1e30;
+    long long small = 0;
+    for (int sh = 0; sh < 6; sh++) {
+        const GemmB16Shape& c = g_b16Shapes[sh];
+        long long tiles = 0;
+        for (int p = 0; p < count; p++) tiles += (long long)((q[p].m + c.bm - 1) / c.bm) * ((q[p].n + c.bn - 1) / c.bn);
+        const double t = b16_time(c, tiles, q[0].k);
+        if (t < bestT) { bestT = t; best = sh == B16_128X192 && tiles <= 256 ? B16_128X192_ALONE : sh; }
+        small = tiles;
+    }
+    if (small < 256) return false;
+    switch (best) {
+    case 0: *e = launch_b16_group<4, 2, 2, 4, 2>(s, grp, count); break;
+    case 1: *e = launch_b16_group<4, 2, 2, 3, 2>(s, grp, count); break;
+    case B16_128X192: *e = launch_b16_group<2, 2, 2, 3, 2>(s, grp, count); break;
+    case B16_128X192_ALONE: *e = launch_b16_group<4, 2, 1, 3, 2>(s, grp, count); break;
+    case 3: *e = launch_b16_group<2, 2, 2, 2, 2>(s, grp, count); break;
+    case 4: *e = launch_b16_group<2, 2, 1, 2, 3>(s, grp, count); break;
+    default: *e = launch_b16_group<2, 2, 1, 1, 4>(s, grp, count); break;
+    }
+    return true;
 }
 
 }  // namespace mch

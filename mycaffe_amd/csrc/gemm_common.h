@@ -237,5 +237,6 @@ struct GemmB16 {
 bool gemm_b16_takes(const GemmB16& g);   // 16-byte chunks of both operands aligned and whole
 size_t gemm_b16_workspace_bytes(int m, int n, int k);
 hipError_t gemm_b16(hipStream_t s, const GemmB16& g, void* ws, size_t wsBytes);
+bool gemm_b16_group(hipStream_t s, const GemmB16* q, int count, hipError_t* e);   // several with heads, of one n and k, as one launch
 
 }  // namespace mch

@@ -140,6 +140,9 @@ hipError_t k_gemm_bias(hipStream_t s, DType dt, int m, int n, int k, const void*
 // scratch of k_gemm_bias / k_gemm_qkv_heads with these operands (0: none)
 hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, int k, const void* X, const void* W, const void* bias, void* Y,
                              void* ws, size_t wsBytes, bool fp32Sums = false);   // Y as (B,H,T,hs); scratch as k_gemm_bias
+// several of those in 16-bit storage, of one width and contraction, as one launch, if that takes them (*done)
+struct HeadsProjection { int m, T; const void *X, *W, *bias; void* Y; };
+hipError_t k_gemm_bias_heads_group(hipStream_t s, int count, int n, int k, int H, const HeadsProjection* p, bool* done);
 size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W);
 // whether the call fails without that scratch (otherwise its contraction stays in one part)
 bool k_gemm_bias_needs_workspace(DType dt, int m, int n, int k, const void* X, const void* W);

@@ -2208,6 +2208,41 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         return 0;
     }
 
+    case MCH_FN_LINEAR_HEADS_GROUP: {
+        // l{count, N, K, heads, {M, T, hX, hW, hBias(0 = none), hY} of each}: LINEAR_FWD with T and heads of each
+        NEED_L(16, 22);
+        const long long count = pl[0], N = pl[1], K = pl[2], heads = pl[3];
+        if (count < 2 || count > 3 || ll != 4 + 6 * count || N < 1 || K < 1 || heads < 1 || N > INT_MAX || K > INT_MAX || N % heads) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+        HeadsProjection hp[3];
+        bool half = true;
+        for (int i = 0; i < count; i++) {
+            const MCH_LONGLONG* a = pl + 4 + 6 * i;
+            const long long M = a[0], T = a[1];
+            if (M < 1 || M > INT_MAX || T < 1 || M % T) return MCH_ERROR_PARAM_OUT_OF_RANGE;
+            MemItem *X, *W, *Bi = nullptr, *Y;
+            ERRCHK(mem((long)a[2], &X));
+            ERRCHK(mem((long)a[3], &W));
+            if (a[4]) ERRCHK(mem((long)a[4], &Bi));
+            ERRCHK(mem((long)a[5], &Y));
+            if (X->half != W->half || X->half != Y->half || (Bi && Bi->half != X->half)) return MCH_ERROR_MEMORY_MIXED_HALF_TYPES;
+            RANGE(X, 0, M * K);
+            RANGE(W, 0, N * K);
+            if (Bi) RANGE(Bi, 0, N);
+            RANGE(Y, 0, M * N);
+            half = half && X->half;
+            hp[i] = HeadsProjection{(int)M, (int)T, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Y->ptr};
+        }
+        bool done = false;
+        if (half) HIPCHK(k_gemm_bias_heads_group(s, (int)count, (int)N, (int)K, (int)heads, hp, &done));
+        for (int i = 0; i < count; i++) {
+            const MCH_LONGLONG* a = pl + 4 + 6 * i;
+            MCH_LONGLONG one[9] = {a[0], N, K, a[2], a[3], a[4], a[5], a[1], heads};
+            if (done) m_mem.touch((long)a[5]);
+            else ERRCHK(run(MCH_FN_LINEAR_FWD, nullptr, 0, one, 9, ppOut, plOut, timing));
+        }
+        return 0;
+    }
+
     case MCH_FN_LINEAR_BWD: {
         // l{M, N, K, hX, hW, hdY, hdW, hdBias(0 = none), hdX(0 = none)[, accumX]}
         NEED_L(9, 10);
@@ -2699,7 +2734,7 @@ static const char* api_name(long fn)
 #define N(x) {MCH_FN_##x, "CUDA_FN_" #x}
     static const struct { long id; const char* name; } table[] = {
         {MCH_DLL_FREEMEM, "CUDA_DLL_FREEMEM"}, {MCH_DLL_INITIALIZE, "CUDA_DLL_INITIALIZE"}, {MCH_DLL_CLEANUP, "CUDA_DLL_CLEANUP"},
-        N(SETDEVICE), N(GETDEVICE), N(SYNCHRONIZEDEVICE), N(CREATE_MEMORYPOINTER), N(FREE_MEMORYPOINTER), N(ALLOCMEM_HALF), N(ALLOCMEM), N(FREEMEM), N(GETMEM), N(SETMEM), N(CREATE_CUDNN), N(FREE_CUDNN), N(CREATE_TENSORDESC), N(FREE_TENSORDESC), N(SET_TENSORDESC), N(CREATE_EXTENSION), N(FREE_EXTENSION), N(EXTENSION_RUN), N(SOFTMAX_FWD), N(SOFTMAX_BWD), N(ATTN_CREATE), N(ATTN_FREE), N(ATTN_SET), N(ATTN_FWD), N(ATTN_BWD), N(SET), N(COPY), N(GEMM2), N(GEMM), N(GEMV), N(AXPY), N(SCAL), N(SCALE), N(ADD_SCALAR), N(ADD), N(SUB), N(MUL), N(DIV), N(EXP), N(LOG), N(POWX), N(SQRT), N(TRANSPOSE), N(MASK), N(MASK_BATCH), N(TRANSPOSE_HW), N(INVERT), N(CHANNEL_MEAN), N(CHANNEL_MAX), N(CHANNEL_SUB), N(CHANNEL_SUM), N(CHANNEL_DIV), N(CHANNEL_DOT), N(CHANNEL_COPY), N(CHANNEL_FILLFROM), N(CHANNEL_COPYALL), N(CHANNEL_DUP), N(CHANNEL_SUM2), N(EMBED_FWD), N(RELU_FWD), N(RELU_BWD), N(GELU_FWD), N(GELU_BWD), N(SILU_FWD), N(SILU_BWD), N(CREATE_LAYERNORM), N(FREE_LAYERNORM), N(LAYERNORM_FWD), N(LAYERNORM_BWD), N(CREATE_ROPE), N(FREE_ROPE), N(ROPE_FWD), N(ROPE_BWD), N(CREATE_BLOBLOADER), N(FREE_BLOBLOADER), N(BLOBLOADER_LOAD), N(BLOBLOADER_RESETOFFSET), N(BLOBLOADER_ADDTOOFFSET), N(ATTN_DECODE_FWD), N(RMSNORM_FWD), N(SWIGLU_FWD), N(QKV_PROJ_HEADS), N(LINEAR_FWD), N(LINEAR_BWD), N(QKV_HEADS_GRAD), N(RMSNORM_BWD), N(SWIGLU_BWD), N(NORM_ADD_FWD), N(NORM_ADD_BWD)};
+        N(SETDEVICE), N(GETDEVICE), N(SYNCHRONIZEDEVICE), N(CREATE_MEMORYPOINTER), N(FREE_MEMORYPOINTER), N(ALLOCMEM_HALF), N(ALLOCMEM), N(FREEMEM), N(GETMEM), N(SETMEM), N(CREATE_CUDNN), N(FREE_CUDNN), N(CREATE_TENSORDESC), N(FREE_TENSORDESC), N(SET_TENSORDESC), N(CREATE_EXTENSION), N(FREE_EXTENSION), N(EXTENSION_RUN), N(SOFTMAX_FWD), N(SOFTMAX_BWD), N(ATTN_CREATE), N(ATTN_FREE), N(ATTN_SET), N(ATTN_FWD), N(ATTN_BWD), N(SET), N(COPY), N(GEMM2), N(GEMM), N(GEMV), N(AXPY), N(SCAL), N(SCALE), N(ADD_SCALAR), N(ADD), N(SUB), N(MUL), N(DIV), N(EXP), N(LOG), N(POWX), N(SQRT), N(TRANSPOSE), N(MASK), N(MASK_BATCH), N(TRANSPOSE_HW), N(INVERT), N(CHANNEL_MEAN), N(CHANNEL_MAX), N(CHANNEL_SUB), N(CHANNEL_SUM), N(CHANNEL_DIV), N(CHANNEL_DOT), N(CHANNEL_COPY), N(CHANNEL_FILLFROM), N(CHANNEL_COPYALL), N(CHANNEL_DUP), N(CHANNEL_SUM2), N(EMBED_FWD), N(RELU_FWD), N(RELU_BWD), N(GELU_FWD), N(GELU_BWD), N(SILU_FWD), N(SILU_BWD), N(CREATE_LAYERNORM), N(FREE_LAYERNORM), N(LAYERNORM_FWD), N(LAYERNORM_BWD), N(CREATE_ROPE), N(FREE_ROPE), N(ROPE_FWD), N(ROPE_BWD), N(CREATE_BLOBLOADER), N(FREE_BLOBLOADER), N(BLOBLOADER_LOAD), N(BLOBLOADER_RESETOFFSET), N(BLOBLOADER_ADDTOOFFSET), N(ATTN_DECODE_FWD), N(RMSNORM_FWD), N(SWIGLU_FWD), N(QKV_PROJ_HEADS), N(LINEAR_FWD), N(LINEAR_BWD), N(QKV_HEADS_GRAD), N(RMSNORM_BWD), N(SWIGLU_BWD), N(NORM_ADD_FWD), N(NORM_ADD_BWD), N(LINEAR_HEADS_GROUP)};
 #undef N
     for (const auto& t : table)
         if (t.id == fn) return t.name;

@@ -125,6 +125,7 @@ class CUDAFN:
     SWIGLU_BWD = 2009
     NORM_ADD_FWD = 2010
     NORM_ADD_BWD = 2011
+    LINEAR_HEADS_GROUP = 2012
 
 
 class CUDAQRY:
@@ -754,6 +755,10 @@ class CudaDnn:
         if bFp32Sums:
             rgl.append(1)
         self._ex2(CUDAFN.LINEAR_FWD, None, rgl)
+
+    def LinearHeadsGroup(self, nN, nK, nHeads, projections):
+        """Two or three of LinearForward with heads as one call; ``projections``: (nM, nT, hX, hWeight, hBias, hY) of each."""
+        self._ex2(CUDAFN.LINEAR_HEADS_GROUP, None, [len(projections), nN, nK, nHeads] + [v for p in projections for v in p])
 
     def LinearBackward(self, nM, nN, nK, hX, hWeight, hdY, hdWeight, hdBias, hdX, bAccumulate=False):
         """dW += dy^T x, dbias += column sums of dy, dx = (+=) dy W (replaces the three calls of InnerProductLayer.cs:429-494).

@@ -530,10 +530,16 @@ class MultiheadAttentionLayer:
             self.transpose.Forward(b["Q"], b["Qt"])
             self.transposeK.Forward(b["K"], b["Kt"])
         else:
-            # projections written head by head: no transposes behind them
-            self.c_attnQ.ForwardHeads(q, b["Qt"], H)
-            self.c_attnK.ForwardHeads(k, b["Kt"], H)
-            self.c_attnV.ForwardHeads(v, b["Vt"], H)
+            # projections written head by head: no transposes behind them; in 16-bit storage one call
+            projections = ((self.c_attnQ, q, b["Qt"]), (self.c_attnK, k, b["Kt"]), (self.c_attnV, v, b["Vt"]))
+            if self.half:
+                for _, x, y in projections:
+                    y.Reshape(B, H, x.shape_[1], hs)
+                cuda.LinearHeadsGroup(C, C, H, [(x.count(0, 2), x.shape_[1], x.gpu_data, layer.blobs[0].gpu_data,
+                                                 layer.blobs[1].gpu_data if layer.bias_term else 0, y.gpu_data) for layer, x, y in projections])
+            else:
+                for layer, x, y in projections:
+                    layer.ForwardHeads(x, y, H)
         is_qk_mask = (blobMask is not None and blobMask.num_axes == 4 and blobMask.num == 1 and blobMask.channels == 1
                       and blobMask.height == Tq and blobMask.width == Tk)
         full_mask = blobMask is not None and not is_qk_mask and blobMask.count() == B * Tq * Tk and Tq > 1
