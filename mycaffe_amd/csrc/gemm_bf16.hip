@@ -314,7 +314,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Ar
 }
 
 // Up to three products with heads epilogues as one launch: the projections of a multi-head attention layer.  One by one each is less
-// than two rounds of the chip with its own first fetches and last stores (4096 and twice 8192 rows, 512 to 512: @GROUPDOC@).
+// than two rounds of the chip with its own first fetches and last stores (4096 and twice 8192 rows, 512 to 512: 9.4 + 12.3 + 11.9 us, as one launch 21.6).
 struct GemmB16Group { GemmB16Args g[3]; HeadsArg<true> h[3]; int first[4]; };   // first: of the tiles of all, of each; then their number
 template <int WVM, int WVN, int WM, int WN, int OCC>
 __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_group_kernel(GemmB16Group grp)
