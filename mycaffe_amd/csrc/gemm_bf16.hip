@@ -325,6 +325,133 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_group_kernel(Gem
     b16_tile<WVM, WVN, WM, WN, true, true, true>(grp.g[p], grp.h[p], item - grp.first[p]);
 }
 
+// ---------------------------------------------------------------------------
+// Up to 32 rows against the rows of B (a decode step's projections).  Such a product reads B once and does little else.  The lanes of
+// a wavefront take the fragments of 16 rows of B straight to registers, a stage of k at a time with the next one on its way; the
+// rows of A, which every workgroup reads, come through LDS, because as fragments from memory they cost what the same bytes of B do.
+// The k are dealt to NW wavefronts, each with stages of its own (nothing but its own fetches to wait for), whose sums meet in LDS.
+// Microseconds with B not in any cache, before (tiles in parts of the contraction, and a launch that adds them up) and now:
+// 8 x 12288 x 4096 24.2, 20.6 (4.9 TB/s); 8 x 4096 x 4096 15.4, 8.8; 32 x 12288 x 4096 25.2, 23.5; 32 x 4096 x 4096 15.6, 11.7;
+// 8 x 2304 x 768 8.3, 3.7; 8 x 512 x 512 6.2, 3.3.  What is left over the reading of B is the launch's beginning and end.
+template <int MT, int NT, int NW, int S, bool HEADS>
+__global__ __launch_bounds__(64 * NW) void gemm_b16_rows_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
+{
+    constexpr int KW = 128 / MT, KS = KW / 32, P = KW / 8;   // k, products and 16-byte pieces of a row, of a stage
+    constexpr int STAGE = 16 * MT * KW, DA = STAGE / 512;    // elements of A in a stage, fetches
+    constexpr int LDC = 16 * NT + 4;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    bf16_t* ring = reinterpret_cast<bf16_t*>(smem_raw) + wave * S * STAGE;
+    const int r = lane & 15, kq = lane >> 4, n0 = (int)blockIdx.x * 16 * NT;
+    const int row = tid / (2 * NT), c = n0 + (tid % (2 * NT)) * 8;   // of the eight results this thread adds up
+    float bias[8];
+    b16_bias8(g, c, bias);   // on its way before the operands
+    // [row][k] in LDS, piece c of row r at c ^ swap(r): sixteen rows read at one piece fall on sixteen bank groups
+    auto swap = [](int row) { return P == 16 ? row & 15 : (row >> 1) & 7; };
+    constexpr uint32_t OUTSIDE = 0x80000000u;   // fetched from there: zeros
+    const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)g.A, 0, (int)(OUTSIDE - 16), 0x00020000);
+    uint32_t va[DA];
+    int ka[DA];
+#pragma unroll
+    for (int p = 0; p < DA; p++) {
+        const int ra = (p * 64 + lane) / P;
+        ka[p] = ((lane % P) ^ swap(ra)) * 8;
+        va[p] = ra < g.M ? ((uint32_t)ra * (uint32_t)g.lda + ka[p]) * 2 : OUTSIDE;
+    }
+    // lane l holds row l % 16, k = 8 (l / 16) .. + 7 of a product's 32; rows of B past the edge are clamped and never stored
+    const bf16_t* pb[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) pb[j] = g.B + (size_t)min(n0 + j * 16 + r, g.N - 1) * g.ldb + kq * 8;
+    struct Stage { u32x4 b[NT][KS]; };
+    auto fetch = [&](Stage& st, int k, int slot) {
+#pragma unroll
+        for (int p = 0; p < DA; p++) lds_fetch<16>(rsA, ring + slot * STAGE + p * 512, va[p], k * 2);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int i = 0; i < KS; i++) st.b[j][i] = *(const u32x4*)(pb[j] + k + i * 32);
+        asm volatile("" ::: "memory");   // stage after stage
+    };
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Stage& st, int slot) {
+        const bf16_t* pa = ring + slot * STAGE;
+#pragma unroll
+        for (int i = 0; i < KS; i++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                const u32x4 a = *(const u32x4*)(pa + (t * 16 + r) * KW + ((4 * i + kq) ^ swap(t * 16 + r)) * 8);
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)&st.b[j][i], *(const bf16x8*)&a, acc[t][j], 0, 0, 0);
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot has been read: it may be fetched into
+    };
+    // all but the latest S - 1 stages' fetches have landed; and all of them
+    auto waitBefore = [&]() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"((S - 1) * (DA + NT * KS)) : "memory"); };
+    auto waitAll = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+    // stages wave, wave + NW, .. are this wavefront's
+    const int whole = g.K / KW;
+    int left = (whole - wave + NW - 1) / NW, k = wave * KW;
+    Stage st[S];
+#pragma unroll
+    for (int u = 0; u < S - 1; u++)
+        if (left > u) fetch(st[u], k + u * NW * KW, u);
+    for (; left >= 2 * S - 1; left -= S, k += S * NW * KW)
+#pragma unroll
+        for (int u = 0; u < S; u++) {
+            fetch(st[(u + S - 1) % S], k + (u + S - 1) * NW * KW, (u + S - 1) % S);
+            waitBefore();
+            multiply(st[u], u);
+        }
+#pragma unroll
+    for (int u = 0; u < 2 * S - 2; u++)
+        if (left > u) {
+            if (left > u + S - 1) {
+                fetch(st[(u + S - 1) % S], k + (u + S - 1) * NW * KW, (u + S - 1) % S);
+                waitBefore();
+            } else waitAll();
+            multiply(st[u % S], u % S);
+        }
+    if (whole * KW < g.K && whole % NW == wave) {   // the rest, whole 16-byte pieces
+        k = whole * KW;
+#pragma unroll
+        for (int p = 0; p < DA; p++) lds_fetch<16>(rsA, ring + p * 512, k + ka[p] < g.K ? va[p] : OUTSIDE, k * 2);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int i = 0; i < KS; i++) st[0].b[j][i] = k + i * 32 + kq * 8 < g.K ? *(const u32x4*)(pb[j] + k + i * 32) : u32x4{0, 0, 0, 0};
+        waitAll();
+        multiply(st[0], 0);
+    }
+    // the products are the transposed tiles: a lane owns row l % 16, columns 4 (l / 16) .. + 3
+    constexpr int SLICE = S * STAGE / 2;   // floats from one wavefront's stages to the next's
+    float* red = reinterpret_cast<float*>(smem_raw);
+    static_assert(16 * MT * LDC <= SLICE, "the sums fit in place of the stages");
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) *(floatx4*)(red + wave * SLICE + (t * 16 + r) * LDC + j * 16 + kq * 4) = acc[t][j];
+    __syncthreads();
+    if (row >= min(16 * MT, g.M) || c >= g.N) return;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float* p = red + w * SLICE + row * LDC + c - n0;
+        const floatx4 x = *(const floatx4*)p, y = *(const floatx4*)(p + 4);
+#pragma unroll
+        for (int q = 0; q < 4; q++) { v[q] += x[q]; v[4 + q] += y[q]; }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] *= g.alpha;
+    bf16_t* col = nullptr;
+    if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
+    b16_store8<HEADS>(g, hp, row, c, bias, col, v);
+}
+
 // sum over the S partial products in their order, then as b16_store8
 template <bool HEADS>
 __global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<HEADS> hp, int S)
@@ -460,9 +587,55 @@ static GemmB16Args b16_args(const GemmB16& q)
     return a;
 }
 
+// Whether gemm_b16_rows_kernel takes a product (microseconds with B not in any cache, against the tiles and their sum).  Not where a few
+// workgroups would each walk a very long contraction (8 x 64 x 16384: 20.0 against 16.2; 8 x 64 x 8192: 11.3 against 12.1), and not
+// where more than 16 rows meet more columns than one workgroup a CU holds (32 x 14336 x 4096: 36 against 27.6).  Its workgroups read
+// all rows of A while others write, so a result that shares memory with an operand stays with the tiles.
+static bool b16_rows_takes(const GemmB16& q)
+{
+    if (!q.aK || !q.bK || q.m > 32 || (q.k > 8192 && q.n < 4096) || (q.m > 16 && q.n > 768 * 16)) return false;
+    const size_t mk = (size_t)q.m * q.k * 2, nk = (size_t)q.n * q.k * 2, mn = (size_t)q.m * q.n * 2;
+    auto apart = [](const void* p, size_t pb, const void* o, size_t ob) { return (uintptr_t)p + pb <= (uintptr_t)o || (uintptr_t)o + ob <= (uintptr_t)p; };
+    auto free = [&](const void* dst, size_t bytes) {
+        const void* bias = q.heads ? q.heads->bias : (const void*)q.bias;
+        return apart(dst, bytes, q.A, mk) && apart(dst, bytes, q.B, nk) && (!bias || apart(dst, bytes, bias, (size_t)q.n * 2));
+    };
+    if (!q.heads) return free(q.C, mn);
+    const int third = q.heads->H * q.heads->hs;
+    for (int w = 0; w * third < q.n; w++)
+        if (!free(q.heads->dst[w], (size_t)q.m * third * 2)) return false;
+    return true;
+}
+template <int MT, int NT, int NW, int S, bool HEADS>
+static hipError_t launch_b16_rows_shape(hipStream_t s, const GemmB16Args& g, const HeadsArg<HEADS>& ha)
+{
+    constexpr int lds = NW * S * 16 * 128 * 2;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_rows_kernel<MT, NT, NW, S, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((gemm_b16_rows_kernel<MT, NT, NW, S, HEADS>), (unsigned)((g.N + 16 * NT - 1) / (16 * NT)), 64 * NW, lds, s, g, ha);
+    return hipGetLastError();
+}
+// One workgroup a CU of 16, 32 or 48 columns as long as that holds all of them: the wider ones read A as often less, and eight
+// wavefronts with four stages, or more columns and two, keep 100 KB and more of B on their way.  Past that workgroups of four
+// wavefronts, three of them on a CU, so that one's end is another's middle.
+template <int MT, bool HEADS>
+static hipError_t launch_b16_rows(hipStream_t s, const GemmB16Args& g, const HeadsArg<HEADS>& ha)
+{
+    if (g.N <= 256 * 16) return launch_b16_rows_shape<MT, 1, 8, 4, HEADS>(s, g, ha);
+    if (g.N <= 512 * 16) return launch_b16_rows_shape<MT, 2, 8, 2, HEADS>(s, g, ha);
+    if (g.N <= 768 * 16) return launch_b16_rows_shape<MT, 3, 8, 2, HEADS>(s, g, ha);
+    if constexpr (MT == 1) return launch_b16_rows_shape<MT, 1, 4, 3, HEADS>(s, g, ha);
+    return hipErrorInvalidValue;   // b16_rows_takes
+}
+
 hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
 {
     if (!gemm_b16_takes(q) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || !q.aK || !q.bK))) return hipErrorInvalidValue;
+    if (b16_rows_takes(q)) {
+        const GemmB16Args a = b16_args(q);
+        if (q.heads) return q.m > 16 ? launch_b16_rows<2, true>(s, a, heads_arg<true>(q.heads)) : launch_b16_rows<1, true>(s, a, heads_arg<true>(q.heads));
+        return q.m > 16 ? launch_b16_rows<2, false>(s, a, HeadsArg<false>()) : launch_b16_rows<1, false>(s, a, HeadsArg<false>());
+    }
     GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
     if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
     GemmB16Args a = b16_args(q);
