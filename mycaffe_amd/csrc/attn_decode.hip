@@ -163,10 +163,12 @@ __device__ __forceinline__ void decode_consume(const DecodeStage<U>& st, int tb,
     }
 }
 
-template <typename T, int LPR>
+// first: what has to be done to qv, once the first rows are on their way
+struct DecodeNothing { __device__ void operator()() const {} };
+template <typename T, int LPR, typename F = DecodeNothing>
 __device__ __forceinline__ void decode_stream(const T* __restrict__ kc, const T* __restrict__ vc, long long strideT, int t0, int t1,
                                               unsigned rot, int wave, int grp, int d0, bool active,
-                                              const float (&qv)[Vec16<T>::W], float& m, float& l, float (&acc)[Vec16<T>::W])
+                                              const float (&qv)[Vec16<T>::W], float& m, float& l, float (&acc)[Vec16<T>::W], F first = F())
 {
     constexpr int RPW = 64 / LPR;  // rows per wavefront load
     constexpr int U = 4;           // row groups per stage and operand
@@ -175,12 +177,16 @@ __device__ __forceinline__ void decode_stream(const T* __restrict__ kc, const T*
     // The online softmax does not care about row order, so every workgroup starts at its own rotation of the
     // range instead of all of them walking their caches in lockstep.
     const int nIt = (t1 - t0 + STEP - 1) / STEP;
-    if (nIt <= 0) return;
+    if (nIt <= 0) {
+        first();
+        return;
+    }
     int j = (int)(rot % (unsigned)nIt);
     auto next = [&](int x) { return x + 1 == nIt ? 0 : x + 1; };
     const int w0 = t0 + wave * RPW * U;
     DecodeStage<U> A, B;
     decode_issue<T, LPR, U>(A, kc, vc, strideT, w0 + j * STEP, t1, grp, d0, active);
+    first();
     for (int it = 0; it < nIt; it += 2) {
         const int j1 = next(j), j2 = next(j1);
         const bool has1 = it + 1 < nIt, has2 = it + 2 < nIt;
@@ -304,8 +310,8 @@ __device__ __forceinline__ void decode_reduce_wg(float m, float l, float (&acc)[
 // The workgroup that takes the last ticket of a (batch, head) merges all split partials (splits <= 256,
 // 256 threads).  Every wavefront waits for its own partial stores to be acknowledged before the barrier
 // that precedes the ticket, so a workgroup that sees ticket == splits - 1 can read every partial.
-template <typename T>
-__device__ __forceinline__ void decode_merge_last(const float* part, int* counter, int splits, int hs, T* __restrict__ y)
+template <typename T, typename F>
+__device__ __forceinline__ void decode_merge_last(const float* part, int* counter, int splits, int hs, T* __restrict__ y, F last)
 {
     __shared__ int ticket;
     __shared__ float sM[256], sL[256], sA[256];
@@ -314,6 +320,7 @@ __device__ __forceinline__ void decode_merge_last(const float* part, int* counte
     if (threadIdx.x == 0) ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (ticket != splits - 1) return;
+    last();
     // One round trip: thread (g, d) merges splits g, g + G, ... for output dimension d with its own running
     // maximum, four splits' {m, l, value} loads in flight at a time; the G groups then meet in LDS.
     const int tid = threadIdx.x;
@@ -376,8 +383,8 @@ __device__ __forceinline__ void decode_merge_last(const float* part, int* counte
 // d stores dimension d): it waits for its own stores, takes the ticket and, if it is the last one, merges with one lane
 // per dimension and sixteen splits' loads in flight - no workgroup barrier and no LDS on the way.  The other wavefronts
 // are done.
-template <typename T>
-__device__ __forceinline__ void decode_merge_last_wave(const float* part, int* counter, int splits, int hs, T* __restrict__ y)
+template <typename T, typename F>
+__device__ __forceinline__ void decode_merge_last_wave(const float* part, int* counter, int splits, int hs, T* __restrict__ y, F last)
 {
     if (threadIdx.x >= 64) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -385,6 +392,7 @@ __device__ __forceinline__ void decode_merge_last_wave(const float* part, int* c
     if (threadIdx.x == 0) ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     ticket = __builtin_amdgcn_readfirstlane(ticket);
     if (ticket != splits - 1) return;
+    last();
     const int d = threadIdx.x < hs ? threadIdx.x : 0;
     const int stride = hs + 2;
     constexpr int NS = 16;
@@ -420,16 +428,40 @@ __device__ __forceinline__ void decode_merge_last_wave(const float* part, int* c
     if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
 }
 
-template <typename T>
-__device__ __forceinline__ void decode_merge(const float* part, int* counter, int splits, int hs, T* __restrict__ y)
+// last: what the workgroup that merges does besides
+template <typename T, typename F = DecodeNothing>
+__device__ __forceinline__ void decode_merge(const float* part, int* counter, int splits, int hs, T* __restrict__ y, F last = F())
 {
-    if (hs <= 64) decode_merge_last_wave<T>(part, counter, splits, hs, y);
-    else decode_merge_last<T>(part, counter, splits, hs, y);
+    if (hs <= 64) decode_merge_last_wave<T>(part, counter, splits, hs, y, last);
+    else decode_merge_last<T>(part, counter, splits, hs, y, last);
+}
+
+// APPEND: what rope_append_kernel does to q, the new key and the caches at position len - 1, in the attention's own launch (8 x 32
+// heads of 128: 5.0 of 56.5 us, and a launch of the host).  Every head has a key head of its own there.  The workgroup whose rows
+// reach the new position takes it from the new key and value and not from the cache; q, which all splits of a head read, is stored
+// by the workgroup that takes the head's last ticket.
+template <bool APPEND> struct DecodeAppendArg { DecodeAppend p; };
+template <> struct DecodeAppendArg<false> {};
+
+// elements d0 .. of a row, raw as loaded, rotated in their pairs as rope_append_kernel does it and rounded to the storage type
+template <typename T>
+__device__ __forceinline__ u32x4 decode_rotate(u32x4 raw, const float (&c)[Vec16<T>::W / 2], const float (&sn)[Vec16<T>::W / 2])
+{
+    constexpr int W = Vec16<T>::W;
+    float x[W];
+    Vec16<T>::unpack(raw, x);
+#pragma unroll
+    for (int i = 0; i < W / 2; i++) {
+        const float re = x[2 * i], im = x[2 * i + 1];
+        x[2 * i] = re * c[i] - im * sn[i];
+        x[2 * i + 1] = re * sn[i] + im * c[i];
+    }
+    return Vec16<T>::pack(x);
 }
 
 // partial layout: part[((b*H + h)*splits + s) * (hs + 2)] = {m, l, acc[hs]}
-template <typename T, int LPR>
-__global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs a)
+template <typename T, int LPR, bool APPEND>
+__global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs a, DecodeAppendArg<APPEND> app)
 {
     constexpr int W = Vec16<T>::W;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
@@ -443,17 +475,52 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs a)
     const T* kc = (const T*)a.kc + base;
     const T* vc = (const T*)a.vc + base;
 
+    int t0, t1;
+    if constexpr (APPEND) a.dlen = nullptr;   // k_attn_decode
+    decode_range(a, split, &t0, &t1);
     float qv[W];
 #pragma unroll
     for (int i = 0; i < W; i++) qv[i] = 0.f;
-    if (active) {
+    const int pos = a.len - 1;
+    [[maybe_unused]] const bool holder = t0 <= pos && pos < t1 && wave == 0;    // APPEND: of the new row, with its first lane group
+    [[maybe_unused]] u32x4 qNew = {0u, 0u, 0u, 0u}, kNew = {0u, 0u, 0u, 0u}, vNew = {0u, 0u, 0u, 0u};
+    [[maybe_unused]] float rc[W / 2], rs[W / 2];
+    if constexpr (APPEND) {
+        const size_t row = ((size_t)b * a.H + h) * a.hs + d0;
+#pragma unroll
+        for (int i = 0; i < W / 2; i++) { rc[i] = 1.f; rs[i] = 0.f; }
+        if (active) {
+            qNew = *(const u32x4*)(q + d0);
+            if (holder && grp == 0) {
+                kNew = *(const u32x4*)((const T*)app.p.knew + row);
+                vNew = *(const u32x4*)((const T*)app.p.vnew + row);
+            }
+            // without tables anything that is there, so that nothing waits for these loads before the first rows are on their way
+            const size_t at = (size_t)pos * (a.hs / 2) + d0 / 2;
+            const float *fc = app.p.fcos ? app.p.fcos + at : (const float*)a.q, *fs = app.p.fsin ? app.p.fsin + at : (const float*)a.q;
+#pragma unroll
+            for (int i = 0; i < W / 2; i++) { rc[i] = fc[i]; rs[i] = fs[i]; }
+        }
+        t1 = min(t1, pos);
+    } else if (active) {
         Vec16<T>::load(q + d0, qv);
 #pragma unroll
         for (int i = 0; i < W; i++) qv[i] *= a.scale;
     }
+    auto rotateQ = [&]() {
+        if constexpr (APPEND) {
+#pragma unroll
+            for (int i = 0; i < W / 2; i++) {
+                if (!app.p.fcos) rc[i] = 1.f;
+                if (!app.p.fsin) rs[i] = 0.f;
+            }
+            qNew = decode_rotate<T>(qNew, rc, rs);
+            Vec16<T>::unpack(qNew, qv);
+#pragma unroll
+            for (int i = 0; i < W; i++) qv[i] *= a.scale;
+        }
+    };
 
-    int t0, t1;
-    decode_range(a, split, &t0, &t1);
     // splits that hold rows: with a device-side length the launch is sized for the longest cache and the rest idle
     int nAct = a.splits;
     if (a.dlen) {
@@ -467,17 +534,38 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs a)
     float m = -INFINITY, l = 0.f, acc[W];
 #pragma unroll
     for (int i = 0; i < W; i++) acc[i] = 0.f;
-    decode_stream<T, LPR>(kc, vc, a.strideT, t0, t1, (unsigned)((b * a.H + h) * 37 + split * 11), wave, grp, d0, active, qv, m, l, acc);
+    decode_stream<T, LPR>(kc, vc, a.strideT, t0, t1, (unsigned)((b * a.H + h) * 37 + split * 11), wave, grp, d0, active, qv, m, l, acc, rotateQ);
 
     const size_t bh = (size_t)b * a.H + h;
+    if constexpr (APPEND) {
+        if (holder) {
+            kNew = decode_rotate<T>(kNew, rc, rs);   // zeros stay zeros outside the first lane group
+            if (grp == 0 && active) {
+                *(u32x4*)((T*)app.p.knew + bh * a.hs + d0) = kNew;
+                *(u32x4*)((T*)kc + (size_t)pos * a.strideT + d0) = kNew;
+                *(u32x4*)((T*)vc + (size_t)pos * a.strideT + d0) = vNew;
+            }
+            DecodeStage<1> st;
+            st.k[0] = kNew;
+            st.v[0] = vNew;
+            decode_consume<T, LPR, 1>(st, 0, 1, grp, qv, m, l, acc);
+        }
+    }
+    // with every split's wavefronts past their loads of q
+    auto storeQ = [&]() {
+        if constexpr (APPEND) {
+            if (wave == 0 && grp == 0 && active) *(u32x4*)((T*)a.q + bh * a.hs + d0) = qNew;
+        }
+    };
     float* out = a.part + (bh * a.splits + split) * (a.hs + 2);
     if (a.counters && nAct == 1) {
         decode_reduce_wg<T, LPR>(m, l, acc, wave, grp, gl, d0, active, a.hs, out, (T*)a.y + bh * a.hs);
+        storeQ();
         return;
     }
     decode_reduce_wg<T, LPR>(m, l, acc, wave, grp, gl, d0, active, a.hs, out);
     if (a.counters)
-        decode_merge<T>(a.part + bh * a.splits * (a.hs + 2), a.counters + bh, nAct, a.hs, (T*)a.y + bh * a.hs);
+        decode_merge<T>(a.part + bh * a.splits * (a.hs + 2), a.counters + bh, nAct, a.hs, (T*)a.y + bh * a.hs, storeQ);
 }
 
 // Engine form (fp32): one launch per layer does what the reference's decode step does between the QKV
@@ -828,28 +916,38 @@ size_t attn_decode_workspace_bytes(int B, int H, int hs, int len)
     return (size_t)(bh * want) * (size_t)(hs + 2) * sizeof(float);
 }
 
-template <typename T>
-static hipError_t launch_decode(hipStream_t s, DecodeArgs a, int kvH)
+// lanes that cover a row in the vectorised kernel, 0 where it does not take the call
+static int decode_lanes(DType dt, const void* q, const void* kc, const void* vc, int hs, long long strideB, long long strideH, long long strideT)
 {
-    constexpr int W = Vec16<T>::W;
-    (void)kvH;
-    int lpr = (a.hs + W - 1) / W;
+    const int W = dt == F32 ? Vec16<float>::W : Vec16<bf16_t>::W;
     int lprp = 1;
-    while (lprp < lpr) lprp <<= 1;
-    bool fast = (a.hs % W == 0) && lprp <= 64 && (a.strideT % W == 0) && (a.strideH % W == 0) && (a.strideB % W == 0) &&
-                (((uintptr_t)a.q | (uintptr_t)a.kc | (uintptr_t)a.vc) % 16 == 0);
+    while (lprp < (hs + W - 1) / W) lprp <<= 1;
+    const bool fast = hs % W == 0 && lprp <= 64 && strideT % W == 0 && strideH % W == 0 && strideB % W == 0 &&
+                      (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) % 16 == 0);
+    return fast ? lprp : 0;
+}
+
+template <typename T>
+static hipError_t launch_decode(hipStream_t s, DecodeArgs a, const DecodeAppend* app)
+{
+    const int lprp = decode_lanes(std::is_same<T, float>::value ? F32 : BF16, a.q, a.kc, a.vc, a.hs, a.strideB, a.strideH, a.strideT);
+    const bool fast = lprp > 0;
     if (fast) {
         int rpi = 4 * (64 / lprp) * 4;
         a.rowsPerIter = rpi;
         pick_splits(a.B, a.H, a.len, rpi, &a.splits, &a.chunk);
         dim3 grid(a.splits, a.H, a.B);
         switch (lprp) {
-#define CASE(L) case L: hipLaunchKernelGGL((attn_decode_kernel<T, L>), grid, 256, 0, s, a); break;
+#define CASE(L)                                                                                                             \
+    case L:                                                                                                                 \
+        if (app) hipLaunchKernelGGL((attn_decode_kernel<T, L, true>), grid, 256, 0, s, a, DecodeAppendArg<true>{*app});      \
+        else hipLaunchKernelGGL((attn_decode_kernel<T, L, false>), grid, 256, 0, s, a, DecodeAppendArg<false>{});            \
+        break;
             CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32) CASE(64)
 #undef CASE
         }
     } else {
-        if (a.hs > 512) return hipErrorInvalidValue;
+        if (a.hs > 512 || app) return hipErrorInvalidValue;
         a.rowsPerIter = 64;
         pick_splits(a.B, a.H, a.len, 64, &a.splits, &a.chunk);
         dim3 grid(a.splits, a.H, a.B);
@@ -863,21 +961,45 @@ static hipError_t launch_decode(hipStream_t s, DecodeArgs a, int kvH)
     return hipGetLastError();
 }
 
+// Whether k_attn_decode takes the rotation and the append along.  A row of the new position has to be nobody else's: a key head per
+// head, rows of the caches that do not overlap, and tensors that share no memory (as two launches the second sees what the first
+// wrote, whoever else wrote there).
+bool attn_decode_appends(DType dt, const void* q, const void* kc, const void* vc, const void* y, int B, int H, int kvH, int hs, int len,
+                         long long strideB, long long strideH, long long strideT, const DecodeAppend& app)
+{
+    if (kvH != H || !decode_lanes(dt, q, kc, vc, hs, strideB, strideH, strideT) || (((uintptr_t)app.knew | (uintptr_t)app.vnew) & 15) != 0) return false;
+    struct { long long stride, count; } dim[3] = {{strideB, B}, {strideH, H}, {strideT, len}};
+    std::sort(dim, dim + 3, [](const auto& x, const auto& y) { return x.stride < y.stride; });
+    long long span = hs;
+    for (const auto& d : dim) {
+        if (d.count == 1) continue;
+        if (d.stride < span) return false;
+        span += (d.count - 1) * d.stride;
+    }
+    const size_t es = dt == F32 ? 4 : 2, row = (size_t)B * H * hs * es, cache = (size_t)span * es;
+    const struct { const void* p; size_t bytes; } used[6] = {{q, row}, {y, row}, {app.knew, row}, {app.vnew, row}, {kc, cache}, {vc, cache}};
+    for (int i = 0; i < 6; i++)
+        for (int j = 0; j < i; j++)
+            if ((uintptr_t)used[i].p < (uintptr_t)used[j].p + used[j].bytes && (uintptr_t)used[j].p < (uintptr_t)used[i].p + used[i].bytes) return false;
+    return true;
+}
+
 hipError_t k_attn_decode(hipStream_t s, DType dt, const void* q, const void* kc, const void* vc, void* y, int B, int H,
                          int kvH, int hs, int len, long long strideB, long long strideH, long long strideT, float scale,
-                         void* workspace, size_t workspaceBytes, const int* dlen, int* counters)
+                         void* workspace, size_t workspaceBytes, const int* dlen, int* counters, const DecodeAppend* app)
 {
     if (B <= 0 || H <= 0 || hs <= 0 || len <= 0) return hipSuccess;
     if (kvH <= 0 || H % kvH != 0) return hipErrorInvalidValue;
     if (B > 65535 || H > 65535) return hipErrorInvalidValue;
+    if (app && (dlen || !counters)) return hipErrorInvalidValue;
     if (workspaceBytes < attn_decode_workspace_bytes(B, H, hs, len)) return hipErrorInvalidValue;
     DecodeArgs a;
     a.q = q; a.kc = kc; a.vc = vc; a.y = y; a.part = (float*)workspace;
     a.B = B; a.H = H; a.kvMul = H / kvH; a.hs = hs; a.len = len; a.splits = 1; a.chunk = len;
     a.strideB = strideB; a.strideH = strideH; a.strideT = strideT; a.scale = scale;
     a.dlen = dlen; a.rowsPerIter = 64; a.counters = counters;
-    if (dt == F32) return launch_decode<float>(s, a, kvH);
-    return launch_decode<bf16_t>(s, a, kvH);
+    if (dt == F32) return launch_decode<float>(s, a, app);
+    return launch_decode<bf16_t>(s, a, app);
 }
 
 // The splits of a launch that leaves the merge to the next kernel (batch 1, the whole cache in one iteration per split), and

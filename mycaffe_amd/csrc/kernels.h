@@ -221,9 +221,13 @@ size_t attn_decode_workspace_bytes(int B, int H, int hs, int len);
 hipError_t k_attn_decode(hipStream_t s, DType dt, const void* q, const void* kc, const void* vc, void* y, int B, int H,
                          int kvH, int hs, int len, long long strideB, long long strideH, long long strideT,
                          float scale, void* workspace, size_t workspaceBytes, const int* dlen = nullptr,
-                         int* counters = nullptr);
+                         int* counters = nullptr, const struct DecodeAppend* app = nullptr);
 // `counters`: B*H zero-initialised ints that stay zero between launches; when given, the last
 // workgroup of every (batch, head) merges the split partials inside the kernel (no second launch).
+// With `app` (counters set, no dlen, and attn_decode_appends says so) the call does k_rope_append's work at position len - 1 as well.
+struct DecodeAppend { void* knew; const void* vnew; const float *fcos, *fsin; };
+bool attn_decode_appends(DType dt, const void* q, const void* kc, const void* vc, const void* y, int B, int H, int kvH, int hs, int len,
+                         long long strideB, long long strideH, long long strideT, const DecodeAppend& app);
 //
 // Decode step of the llama2 engine in one launch: rotate q / k at position *dlen - 1, append k, v to the caches
 // ([B][seqLen][kvH*hs], stored as cacheType: fp32, or bf16 with hs a multiple of 8), attend over positions

@@ -2608,10 +2608,14 @@ long Kernel::attn_decode_fwd(float* pf, long lf, MCH_LONGLONG* pl, long ll, bool
         wsHave = m_wsBytes;
         ERRCHK(tickets((size_t)(B * H), &tk));
     }
+    DecodeAppend app = {};
+    bool fused = false;
     if (append) {
-        HIPCHK(k_rope_append(s, Q->dt(), Q->ptr, KN->ptr, VN->ptr, KC->ptr, VC->ptr, (int)B, (int)H, (int)KVH, (int)hs,
-                             (int)len - 1, sB, sH, sT, rp ? (const float*)rp->dcos.get() : nullptr,
-                             rp ? (const float*)rp->dsin.get() : nullptr));
+        app = {KN->ptr, VN->ptr, rp ? (const float*)rp->dcos.get() : nullptr, rp ? (const float*)rp->dsin.get() : nullptr};
+        fused = attn_decode_appends(Q->dt(), Q->ptr, KC->ptr, VC->ptr, Y->ptr, (int)B, (int)H, (int)KVH, (int)hs, (int)len, sB, sH, sT, app);
+        if (!fused)
+            HIPCHK(k_rope_append(s, Q->dt(), Q->ptr, KN->ptr, VN->ptr, KC->ptr, VC->ptr, (int)B, (int)H, (int)KVH, (int)hs,
+                                 (int)len - 1, sB, sH, sT, app.fcos, app.fsin));
         m_mem.touch((long)pl[5]);
         m_mem.touch((long)pl[6]);
         m_mem.touch((long)pl[7]);
@@ -2620,7 +2624,7 @@ long Kernel::attn_decode_fwd(float* pf, long lf, MCH_LONGLONG* pl, long ll, bool
     // the static array keeps what the last call left: the tickets must start at zero (a fill kernel, not a memset node)
     if (staticScratch) HIPCHK(k_set(s, F32, tk, (size_t)(B * H), 0.f));
     HIPCHK(k_attn_decode(s, Q->dt(), Q->ptr, KC->ptr, VC->ptr, Y->ptr, (int)B, (int)H, (int)KVH, (int)hs, (int)len, sB, sH,
-                         sT, scale, ws, wsHave, nullptr, tk));
+                         sT, scale, ws, wsHave, nullptr, tk, fused ? &app : nullptr));
     m_mem.touch((long)pl[8]);
     return 0;
 }
