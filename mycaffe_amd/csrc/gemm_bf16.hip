@@ -28,6 +28,8 @@ struct GemmB16Args {
     float* part;              // kChunk < K: partial products, [part][M][N]
     bool vecC;
     const bf16_t* bias;
+    float* rowPart;           // sums of op(A)'s rows over some of the k: [part][tile column][M], to be added to rowSum (M)
+    bf16_t* rowSum;
 };
 
 // the bias of eight columns from c on (past the matrix the last one, never stored); all eight loads are under way at once
@@ -90,8 +92,9 @@ __device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<
     }
 }
 
-// tile `item` of a product
-template <int WVM, int WVN, int WM, int WN, bool AK, bool BKC, bool HEADS>
+// tile `item` of a product.  SUMS: the tiles of a row of tiles also add up the rows of op(A), each the stages that are its turn, from
+// the fragments it multiplies: the bias gradient beside a weight gradient (8000 x 3072, 6.2 to 12.8 us and a launch of 5 on their own).
+template <int WVM, int WVN, int WM, int WN, bool AK, bool BKC, bool HEADS, bool SUMS = false>
 __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HEADS>& hp, int item)
 {
     constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64, KS = 4;
@@ -209,6 +212,14 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
     __syncthreads();
     const uint32_t smemAddr = (uint32_t)(uintptr_t)LDS3(smem);
     TrFragment a[2][WM], b[2][WN];
+    [[maybe_unused]] float sums[WM][8];
+    [[maybe_unused]] int turn = n0 / BN;   // stages until this tile's next
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int t = 0; t < WM; t++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) sums[t][e] = 0.f;
+    }
     for (int kt = 0; kt < nk; kt++) {
         const bf16_t* pa = smem + (kt & 1) * STAGE;
         const bf16_t* pb = pa + BM * BK;
@@ -231,6 +242,17 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
 #pragma unroll
             for (int t = 0; t < WN; t++)
                 if (!BKC) tr_wait(b[cur][t]);
+            if constexpr (SUMS) {
+                if (wn == 0 && turn == 0) {
+#pragma unroll
+                    for (int t = 0; t < WM; t++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            sums[t][2 * e] += __uint_as_float(a[cur][t].w[e] << 16);
+                            sums[t][2 * e + 1] += __uint_as_float(a[cur][t].w[e] & 0xffff0000u);
+                        }
+                }
+            }
             // in issue order: a product, the fragments of the next k-step spread over the products, and from the first
             // product on one fetch of the next stage each
             constexpr int RF = (WM + WN + NMF - 1) / NMF * (AK && BKC ? 1 : 2);
@@ -252,8 +274,20 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (SUMS) turn = turn == 0 ? g.tilesN - 1 : turn - 1;
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
+    }
+    if constexpr (SUMS) {
+        if (wn == 0) {
+#pragma unroll
+            for (int t = 0; t < WM; t++) {
+                float v = ((sums[t][0] + sums[t][1]) + (sums[t][2] + sums[t][3])) + ((sums[t][4] + sums[t][5]) + (sums[t][6] + sums[t][7]));
+                v += __shfl_xor(v, 32);
+                const int r = m0 + wm + t * 32 + fr;
+                if (half == 0 && r < M) g.rowPart[(size_t)(part * g.tilesN + n0 / BN) * M + r] = v;
+            }
+        }
     }
 
     // The products are the transposed tiles: a lane owns row lane % 32, register v is column 8 (v / 4) + 4 (lane / 32) + v % 4.
@@ -306,11 +340,11 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
 // each XCD (workgroup index mod 8) takes a contiguous run of the tiles
 __device__ __forceinline__ int b16_xcd_item(int total) { return (int)(blockIdx.x % 8) * ((total + 7) / 8) + (int)(blockIdx.x / 8); }
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS>
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS, bool SUMS>
 __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
 {
     const int total = g.tilesM * g.tilesN * g.parts, item = b16_xcd_item(total);
-    if (item < total) b16_tile<WVM, WVN, WM, WN, AK, BKC, HEADS>(g, hp, item);
+    if (item < total) b16_tile<WVM, WVN, WM, WN, AK, BKC, HEADS, SUMS>(g, hp, item);
 }
 
 // Up to three products with heads epilogues as one launch: the projections of a multi-head attention layer.  One by one each is less
@@ -452,13 +486,29 @@ __global__ __launch_bounds__(64 * NW) void gemm_b16_rows_kernel(GemmB16Args g, H
     b16_store8<HEADS>(g, hp, row, c, bias, col, v);
 }
 
-// sum over the S partial products in their order, then as b16_store8
+// sum over the S partial products in their order, then as b16_store8; the first rowBlocks workgroups add the partial row sums to rowSum
 template <bool HEADS>
-__global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<HEADS> hp, int S)
+__global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<HEADS> hp, int S, int rowBlocks)
 {
+    const int block = (int)blockIdx.x - rowBlocks;
+    if (block < 0) {
+        const int r = (int)blockIdx.x * 256 + threadIdx.x;
+        if (r >= g.M) return;
+        const int count = g.parts * g.tilesN;
+        float v = 0.f;
+        for (int p0 = 0; p0 < count; p0 += 8) {   // eight loads under way
+            float x[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) x[q] = g.rowPart[(size_t)min(p0 + q, count - 1) * g.M + r];
+#pragma unroll
+            for (int q = 0; q < 8; q++) v += p0 + q < count ? x[q] : 0.f;
+        }
+        g.rowSum[r] = f32_to_bf16(bf16_to_f32(g.rowSum[r]) + v);
+        return;
+    }
     const int oct = (g.N + 7) / 8;
     const size_t mn = (size_t)g.M * g.N;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < (size_t)g.M * oct; e += (size_t)256 * gridDim.x) {
+    for (size_t e = (size_t)block * 256 + threadIdx.x; e < (size_t)g.M * oct; e += (size_t)256 * (gridDim.x - rowBlocks)) {
         const int r = (int)(e / oct), c = (int)(e % oct) * 8;
         const float* p = g.part + (size_t)r * g.N + c;
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -539,33 +589,43 @@ size_t gemm_b16_workspace_bytes(int m, int n, int k)
     const GemmB16Plan p = gemm_b16_plan(m, n, k);
     return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
 }
+static int b16_tile_columns(int shape, int n) { const int bn = g_b16Shapes[shape == B16_128X192_ALONE ? B16_128X192 : shape].bn; return (n + bn - 1) / bn; }
+// With the sums of op(A)'s rows: the partial products (none where the contraction is not cut), then the partial sums.  0: not together.
+// A partial sum is one of sixteen accumulators per row and tile: up to 128 values each they are no longer than the column sums' own.
+size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k)
+{
+    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    const GemmB16Plan p = gemm_b16_plan(m, n, k);
+    const long long columns = b16_tile_columns(p.shape, n);
+    if (p.kChunk / (16 * columns) > 128) return 0;
+    return gemm_b16_workspace_bytes(m, n, k) + (size_t)p.splits * columns * m * sizeof(float);
+}
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS>
-static hipError_t launch_b16(hipStream_t s, const GemmB16Args& a, const HeadsEpilogue* he)
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS, bool SUMS>
+static hipError_t launch_b16(hipStream_t s, GemmB16Args& g, const HeadsEpilogue* he)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN, CH = WN % 2 == 0 ? 2 : WN;
     constexpr int stages = 2 * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
-    GemmB16Args g = a;
     g.tilesM = (g.M + BM - 1) / BM;
     g.tilesN = (g.N + BN - 1) / BN;
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS, SUMS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
     return hipGetLastError();
 }
-template <bool AK, bool BKC, bool HEADS>
-static hipError_t launch_b16_shape(hipStream_t s, const GemmB16Args& a, int shape, const HeadsEpilogue* he = nullptr)
+template <bool AK, bool BKC, bool HEADS, bool SUMS = false>
+static hipError_t launch_b16_shape(hipStream_t s, GemmB16Args& a, int shape, const HeadsEpilogue* he = nullptr)
 {
     switch (shape) {
-    case 0: return launch_b16<4, 2, 2, 4, 2, AK, BKC, HEADS>(s, a, he);
-    case 1: return launch_b16<4, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
-    case B16_128X192: return launch_b16<2, 2, 2, 3, 2, AK, BKC, HEADS>(s, a, he);
-    case B16_128X192_ALONE: return launch_b16<4, 2, 1, 3, 2, AK, BKC, HEADS>(s, a, he);
-    case 3: return launch_b16<2, 2, 2, 2, 2, AK, BKC, HEADS>(s, a, he);
-    case 4: return launch_b16<2, 2, 1, 2, 3, AK, BKC, HEADS>(s, a, he);
-    default: return launch_b16<2, 2, 1, 1, 4, AK, BKC, HEADS>(s, a, he);
+    case 0: return launch_b16<4, 2, 2, 4, 2, AK, BKC, HEADS, SUMS>(s, a, he);
+    case 1: return launch_b16<4, 2, 2, 3, 2, AK, BKC, HEADS, SUMS>(s, a, he);
+    case B16_128X192: return launch_b16<2, 2, 2, 3, 2, AK, BKC, HEADS, SUMS>(s, a, he);
+    case B16_128X192_ALONE: return launch_b16<4, 2, 1, 3, 2, AK, BKC, HEADS, SUMS>(s, a, he);
+    case 3: return launch_b16<2, 2, 2, 2, 2, AK, BKC, HEADS, SUMS>(s, a, he);
+    case 4: return launch_b16<2, 2, 1, 2, 3, AK, BKC, HEADS, SUMS>(s, a, he);
+    default: return launch_b16<2, 2, 1, 1, 4, AK, BKC, HEADS, SUMS>(s, a, he);
     }
 }
 
@@ -637,18 +697,26 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
         return q.m > 16 ? launch_b16_rows<2, false>(s, a, HeadsArg<false>()) : launch_b16_rows<1, false>(s, a, HeadsArg<false>());
     }
     GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
+    if (q.rowSum) {
+        const size_t need = gemm_b16_row_sums_workspace_bytes(q.m, q.n, q.k);
+        if (need == 0 || !ws || wsBytes < need || ((uintptr_t)ws & 15) || q.heads || q.aK || q.bK) return hipErrorInvalidValue;
+    }
     if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
     GemmB16Args a = b16_args(q);
     a.parts = p.splits; a.kChunk = p.kChunk;
     a.part = (float*)ws;
+    a.rowSum = q.rowSum;
+    a.rowPart = a.part + (p.splits > 1 ? (size_t)p.splits * q.m * q.n : 0);
     hipError_t e;
     if (q.heads) e = launch_b16_shape<true, true, true>(s, a, p.shape, q.heads);
+    else if (q.rowSum) e = launch_b16_shape<false, false, false, true>(s, a, p.shape);
     else if (q.aK) e = q.bK ? launch_b16_shape<true, true, false>(s, a, p.shape) : launch_b16_shape<true, false, false>(s, a, p.shape);
     else e = q.bK ? launch_b16_shape<false, true, false>(s, a, p.shape) : launch_b16_shape<false, false, false>(s, a, p.shape);
-    if (e != hipSuccess || p.splits == 1) return e;
-    const int grid = (int)std::min<size_t>(((size_t)q.m * ((q.n + 7) / 8) + 255) / 256, 4096);
-    if (q.heads) hipLaunchKernelGGL(gemm_b16_sum_kernel<true>, grid, 256, 0, s, a, heads_arg<true>(q.heads), p.splits);
-    else hipLaunchKernelGGL(gemm_b16_sum_kernel<false>, grid, 256, 0, s, a, HeadsArg<false>(), p.splits);
+    const int rowBlocks = q.rowSum ? (q.m + 255) / 256 : 0;
+    const int grid = rowBlocks + (p.splits > 1 ? (int)std::min<size_t>(((size_t)q.m * ((q.n + 7) / 8) + 255) / 256, 4096) : 0);
+    if (e != hipSuccess || grid == 0) return e;
+    if (q.heads) hipLaunchKernelGGL(gemm_b16_sum_kernel<true>, grid, 256, 0, s, a, heads_arg<true>(q.heads), p.splits, 0);
+    else hipLaunchKernelGGL(gemm_b16_sum_kernel<false>, grid, 256, 0, s, a, HeadsArg<false>(), p.splits, rowBlocks);
     return hipGetLastError();
 }
 

@@ -233,9 +233,11 @@ struct GemmB16 {
     float alpha, beta;
     const bf16_t* bias;   // as in GemmF32
     const HeadsEpilogue* heads;
+    bf16_t* rowSum = nullptr;   // (m) += the sums of op(A)'s rows; both operands with their rows at unit stride
 };
 bool gemm_b16_takes(const GemmB16& g);   // 16-byte chunks of both operands aligned and whole
 size_t gemm_b16_workspace_bytes(int m, int n, int k);
+size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k);   // with rowSum; 0: not taken together
 hipError_t gemm_b16(hipStream_t s, const GemmB16& g, void* ws, size_t wsBytes);
 bool gemm_b16_group(hipStream_t s, const GemmB16* q, int count, hipError_t* e);   // several with heads, of one n and k, as one launch
 

@@ -171,6 +171,9 @@ hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, 
                   float beta, float* y, void* ws = nullptr, size_t wsBytes = 0);
 hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float* X, const float* W, const float* dY, float* dW, float* db, float* dX, float beta,
                                 bool* done);   // the gradients of an inner product as one launch, where sizes and memory allow (*done)
+// dW (n x k) += dY^T X and db (n) += column sums of dY (m x n) together; workspace 0: not taken together, one after the other
+size_t k_weight_bias_grad_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* dY, const void* dW, const void* db);
+hipError_t k_weight_bias_grad(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* dY, void* dW, void* db, void* ws, size_t wsBytes);
 size_t k_bias_grad_workspace_bytes(int m, int n);
 hipError_t k_bias_grad(hipStream_t s, DType dt, int m, int n, const void* dY, void* db, void* ws, size_t wsBytes);   // db += column sums
 

@@ -2277,13 +2277,19 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             }
         }
         const size_t wsW = k_gemm_workspace_bytes(dt, true, false, (int)N, (int)K, (int)M), wsB = dB ? k_bias_grad_workspace_bytes((int)M, (int)N) : 0;
+        const size_t wsT = dB ? k_weight_bias_grad_workspace_bytes(dt, (int)M, (int)N, (int)K, X->ptr, dY->ptr, dW->ptr, dB->ptr) : 0;   // both together
         const size_t wsX = dX ? k_gemm_workspace_bytes(dt, false, false, (int)M, (int)K, (int)N) : 0, most = std::max(wsW, std::max(wsB, wsX));
         void* ws = nullptr;
-        size_t have = most;
+        size_t have = std::max(most, wsT);
         workspace_or_none(&have, &ws);
+        if (have < most) { have = most; workspace_or_none(&have, &ws); }   // what the calls one after the other need may still be there
         if (have < wsB) { have = wsB; ERRCHK(workspace(wsB, &ws)); }   // the products do without, the column sums do not
-        HIPCHK(k_gemm(s, dt, true, false, (int)N, (int)K, (int)M, 1.f, dY->ptr, X->ptr, 1.f, dW->ptr, ws, have));
-        if (dB) HIPCHK(k_bias_grad(s, dt, (int)M, (int)N, dY->ptr, dB->ptr, ws, have));
+        if (wsT > 0 && have >= wsT) {
+            HIPCHK(k_weight_bias_grad(s, dt, (int)M, (int)N, (int)K, X->ptr, dY->ptr, dW->ptr, dB->ptr, ws, have));
+        } else {
+            HIPCHK(k_gemm(s, dt, true, false, (int)N, (int)K, (int)M, 1.f, dY->ptr, X->ptr, 1.f, dW->ptr, ws, have));
+            if (dB) HIPCHK(k_bias_grad(s, dt, (int)M, (int)N, dY->ptr, dB->ptr, ws, have));
+        }
         if (dX) HIPCHK(k_gemm(s, dt, false, false, (int)M, (int)K, (int)N, 1.f, dY->ptr, W->ptr, accum ? 1.f : 0.f, dX->ptr, ws, have));
         m_mem.touch((long)pl[6]);
         if (dB) m_mem.touch((long)pl[7]);
