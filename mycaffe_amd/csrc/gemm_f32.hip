@@ -34,6 +34,7 @@ struct GemmF32Args {
     const int* flag;
     float* part;              // kChunk < K: partial products, [split][M][N]
     bool vecC;                // C rows can be read and written in 16-byte pieces
+    int kTail;                // of the contraction's end, what the split kernel does not fetch in chunks of four
     const float* bias;
 };
 
@@ -424,8 +425,8 @@ template <int WM, int WN> __device__ __forceinline__ bool split_lost(const float
     return __any(low < TINY - 1u || !(sum < __builtin_inff()));
 }
 
-// a wavefront's sums by the fp32 matrix cores, operands read from memory value by value
-template <int WM, int WN, bool AK, bool BKC>
+// a wavefront's sums by the fp32 matrix cores, operands read from memory value by value; ADD: to what acc holds
+template <int WM, int WN, bool AK, bool BKC, bool ADD>
 __device__ __forceinline__ void f32_sums(const GemmF32Args& g, const float* A, const float* B, int m, int n, int kBegin, int kEnd, int lane, floatx16 (&acc)[WM][WN])
 {
     const int fr = lane & 31, half = lane >> 5;
@@ -440,7 +441,8 @@ __device__ __forceinline__ void f32_sums(const GemmF32Args& g, const float* A, c
 #pragma unroll
         for (int j = 0; j < WN; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+            for (int v = 0; v < 16; v++)
+                if (!ADD) acc[i][j][v] = 0.f;
     for (int k0 = kBegin; k0 < kEnd; k0 += 8) {
         float x[4][WM], y[4][WN];
 #pragma unroll
@@ -466,7 +468,7 @@ __device__ __forceinline__ void f32_sums(const GemmF32Args& g, const float* A, c
 // bytes of one plane of R rows by 16 KS k
 template <int R, int KS, bool KFAST> constexpr int split_plane() { return KFAST ? 2 * KS * (R * 16 + 128 / KS) : 16 * KS * R * 2; }
 
-template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool HEADS>
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
 __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
 {
     constexpr int NT = 64 * WVM * WVN, BK = 16 * KS, BM = 32 * WVM * WM, BN = 32 * WVN * WN;
@@ -481,7 +483,8 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     if (item >= total) return;
     F32Item it;
     f32_item<BM, BN>(g, item, it);
-    const int M = g.M, N = g.N, m0 = it.m0, n0 = it.n0, kBegin = it.kBegin, kEnd = it.kEnd;
+    const int M = g.M, N = g.N, m0 = it.m0, n0 = it.n0, kBegin = it.kBegin;
+    const int kEnd = !VEC && it.kEnd == g.K ? max(kBegin, it.kEnd - g.kTail) : it.kEnd;   // of what is fetched in chunks
     const float* __restrict__ A = g.A + (size_t)it.batch * g.sA;
     const float* __restrict__ B = g.B + (size_t)it.batch * g.sB;
     const int wm = (wave / WVN) * (32 * WM), wn = (wave % WVN) * (32 * WN);
@@ -497,7 +500,10 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     // Chunk e of a stage, k at unit stride: row e / (BK / 4), k = 4 (e % (BK / 4)); row index at unit stride: k = e / (rows / 4),
     // rows 4 (e % (rows / 4)) .. + 3.  Where B's chunks do not divide by the threads, the last threads repeat earlier chunks.
     // Byte offsets from a buffer resource that begins at the tile, and where the row index is at unit stride at the stage, so that
-    // operands of any size are reached with 32 bits; rows past the edge are clamped (valid memory) and never stored.
+    // operands of any size are reached with 32 bits; rows past the edge are clamped (valid memory) and never stored.  Not VEC, operands
+    // that are not whole aligned chunks: a fetch of four values needs the alignment of one, a chunk across the last row goes on in the next
+    // k, and the last k, where there is none, and what is left of four k are the tail (996 rows, 768 to 27230, forward, backward and
+    // softmax: 1850 us on the fp32 matrix cores, value by value; 836).
     constexpr uint32_t OUTSIDE = 0x80000000u;
     constexpr int CK = BK / 4;
     const float* baseA = A + (AK ? (size_t)m0 * g.lda : (size_t)m0);
@@ -512,7 +518,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             wa[p] = (e % CK / 2) * KGA + (e / CK) * 16 + (e & 1) * 8;
         } else {
             const int k = e / (BM / 4), row = 4 * (e % (BM / 4));
-            va[p] = 4 * ((uint32_t)k * (uint32_t)g.lda + min(row, M - 4 - m0));
+            va[p] = 4 * ((uint32_t)k * (uint32_t)g.lda + min(row, VEC ? M - 4 - m0 : (M - 1 - m0) & ~3));
             wa[p] = (k * BM + (row ^ (block_swizzle<BM * 2>(k) * 8))) * 2;
         }
     }
@@ -524,7 +530,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             wb[p] = 3 * PLA + (e % CK / 2) * KGB + (e / CK) * 16 + (e & 1) * 8;
         } else {
             const int k = e / (BN / 4), row = 4 * (e % (BN / 4));
-            vb[p] = 4 * ((uint32_t)k * (uint32_t)g.ldb + min(row, N - 4 - n0));
+            vb[p] = 4 * ((uint32_t)k * (uint32_t)g.ldb + min(row, VEC ? N - 4 - n0 : (N - 1 - n0) & ~3));
             wb[p] = 3 * PLA + (k * BN + (row ^ (block_swizzle<BN * 2>(k) * 8))) * 2;
         }
     }
@@ -552,7 +558,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             if (k0 + (BKC ? 4 * (e % CK) : e / (BN / 4)) >= kEnd) vb[p] = OUTSIDE;
         }
     };
-    const int nk = (kEnd - kBegin + BK - 1) / BK;
+    const int nk = VEC ? (kEnd - kBegin + BK - 1) / BK : max(1, (kEnd - kBegin + BK - 1) / BK);
     int fetched = 0, kFetch = kBegin;   // the stage that is fetched and its first k
     auto nextStage = [&]() {
         if (fetched + 1 < nk) {         // past the end the last stage is fetched again, its products never made
@@ -687,7 +693,8 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
         if (kt + 1 < nk) stage(1);
     }
     __syncthreads();
-    if (split_lost(acc)) f32_sums<WM, WN, AK, BKC>(g, A, B, m0 + wm, n0 + wn, kBegin, kEnd, lane, acc);
+    if (split_lost(acc)) f32_sums<WM, WN, AK, BKC, false>(g, A, B, m0 + wm, n0 + wn, kBegin, it.kEnd, lane, acc);
+    else if (!VEC && kEnd < it.kEnd) f32_sums<WM, WN, AK, BKC, true>(g, A, B, m0 + wm, n0 + wn, kEnd, it.kEnd, lane, acc);
     f32_store<WM, WN, HEADS>(g, hp, acc, reinterpret_cast<float*>(smem_raw) + wave * 32 * (32 * WN + 4), lane, m0 + wm, n0 + wn, it.part, it.batch);
 }
 // ---------------------------------------------------------------------------
@@ -993,13 +1000,13 @@ static double gemm_f32_small_time(long long tiles, int k)
 // 32000 takes 51 against 44 us); 32 x 32 tiles where their estimate is the smallest, which is a tenth of a round of the larger ones.
 enum { F32_TILES, F32_SPLIT, F32_SMALL };
 struct GemmF32Choice { int kernel; GemmF32Plan plan; double time; };
-static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool vec, bool fp32Sums, bool heads = false)
+static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool fp32Sums, bool heads = false)
 {
     GemmF32Choice c;
     c.kernel = F32_TILES;
     c.plan = gemm_f32_plan(m, n, k, batch, causal, wsBytes, &c.time);
     if (fp32Sums) return c;
-    if (vec && k >= 64 && (double)m * n * k * batch >= 268435456.0) {   // faster than the fp32 matrix cores at every size from there on
+    if (k >= 64 && (double)m * n * k * batch >= 268435456.0) {   // faster than the fp32 matrix cores at every size from there on
         c.kernel = F32_SPLIT;
         c.plan = gemm_f32_split_plan(m, n, k, batch, causal, wsBytes, &c.time);
     }
@@ -1014,8 +1021,8 @@ static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal)
 {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
-    // which kernel takes it depends on the operands' alignment and on the caller too: enough for any
-    const int splits = std::max(gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, true, false).plan.splits, gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, false, false).plan.splits);
+    // which kernel takes it depends on the caller too: enough for any
+    const int splits = std::max(gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, false).plan.splits, gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, true).plan.splits);
     return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
 }
 
@@ -1051,13 +1058,13 @@ static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const Gem
 // wavefronts of a SIMD that the registers are to hold
 #define SPLIT_SHAPES(X) X(0, 2, 4, 4, 2, 1, 2) X(1, 4, 2, 2, 3, 1, 2) X(2, 2, 2, 2, 3, 1, 2) X(3, 2, 2, 2, 2, 1, 2) X(4, 2, 2, 1, 2, 2, 2) X(5, 2, 2, 1, 1, 2, 2)
 
-template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool HEADS>
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_split(hipStream_t s, const GemmF32Args& a, int splits, int batch, const HeadsEpilogue* he)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN;
     constexpr int stages = 2 * 3 * (split_plane<BM, KS, AK>() + split_plane<BN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
     constexpr int lds = stages > store ? stages : store;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     GemmF32Args g = a;
     g.tilesM = (g.M + BM - 1) / BM;
@@ -1066,15 +1073,15 @@ static hipError_t launch_split(hipStream_t s, const GemmF32Args& a, int splits, 
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
     const int per = (int)((total + 7) / 8);
-    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, HEADS>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
     return hipGetLastError();
 }
 
-template <bool AK, bool BKC, bool HEADS>
+template <bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_split_shape(hipStream_t s, const GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
 {
     switch (p.shape) {
-#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, HEADS>(s, a, p.splits, batch, he);
+#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
         SPLIT_SHAPES(X)
 #undef X
     }
@@ -1107,8 +1114,7 @@ template <bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_layout(hipStream_t s, const GemmF32Args& a, const GemmF32Choice& c, int batch, const HeadsEpilogue* he)
 {
     if (c.kernel == F32_SMALL) return launch_small<4, 64, AK, BKC, VEC, HEADS>(s, a, batch, he);
-    if constexpr (VEC)
-        if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, HEADS>(s, a, c.plan, batch, he);
+    if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
     return launch_f32_tile<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
 }
 
@@ -1138,9 +1144,12 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     const bool vec = near && (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
                      (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0);
     if (!ws || ((uintptr_t)ws & 15)) wsBytes = 0;
-    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, vec, q.fp32Sums || !near, q.heads != nullptr);
+    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, q.fp32Sums || !near, q.heads != nullptr);
     const GemmF32Plan& p = choice.plan;
     a.kChunk = p.kChunk;
+    // rows shorter than the three values that a chunk may read past one: so many more k
+    auto past = [&](bool kFast, int rows, long long ld) { return kFast ? q.k % 4 : rows % 4 == 0 ? 0 : ld >= 3 ? 1 : 3; };
+    a.kTail = std::max(past(q.aK, q.m, q.lda), past(q.bK, q.n, q.ldb));
     hipError_t e;
     if (q.heads) e = vec ? launch_layout<true, true, true, true>(s, a, choice, 1, q.heads) : launch_layout<true, true, false, true>(s, a, choice, 1, q.heads);
 #define LAYOUT(AKV, BKV) (vec ? launch_layout<AKV, BKV, true, false>(s, a, choice, q.batch, nullptr) : launch_layout<AKV, BKV, false, false>(s, a, choice, q.batch, nullptr))
@@ -1173,7 +1182,7 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     if (tilesW + tilesX > (1ll << 20)) return hipSuccess;
     // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
     // time that one launch waits for the last one's stores
-    const double apart = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, vec, false).time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, vec, false).time + 2.5 +
+    const double apart = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false).time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false).time + 2.5 +
                          (db ? m <= 1024 ? 4.5 : 9.0 : 0.0);
     if (gemm_f32_small_time(tilesW + tilesX, std::max(m, n)) >= apart) return hipSuccess;
     GemmF32Args w = {}, x = {};
