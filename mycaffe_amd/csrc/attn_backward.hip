@@ -339,7 +339,9 @@ template <int KIND> __device__ inline bool bwd_masked(const AttnBwdArgs& a, int 
 }
 
 // KIND: 0 none, 1 causal, 2 key mask (B,Tk), 3 mask (B,Tq,Tk) or, with mb = 0, one (Tq,Tk) mask for all sequences
-template <typename T, int HS, int KIND, int BQ, int OCC>
+// PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 54 us
+// here and 47 for dq; the row kernels 671 and 450)
+template <typename T, int HS, int KIND, int BQ, int OCC, bool PADDED>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs a, int mb)
 {
     typedef BwdTile<T, HS, BQ> TL;
@@ -363,23 +365,25 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     const int ibh = rank % nbh;
     const int b = ibh / a.H, h = ibh % a.H;
     const size_t bh = (size_t)b * a.H + h;
+    const int hs = PADDED ? a.hs : HS;
+    auto chunk = [&](const T* row, int col) { return !PADDED || col < hs ? *(const u32x4*)(row + col) : u32x4{0, 0, 0, 0}; };
     const int kw = kblock * BK + wave * 32;          // first key of this wavefront
     const int key = kw + l32;
     const bool waveActive = kw < a.Tk;
-    const T* qp = (const T*)a.q + bh * a.Tq * HS;
-    const T* gp = (const T*)a.dy + bh * a.Tq * HS;
-    const T* kp = (const T*)a.k + bh * a.Tk * HS;
-    const T* vp = (const T*)a.v + bh * a.Tk * HS;
+    const T* qp = (const T*)a.q + bh * a.Tq * hs;
+    const T* gp = (const T*)a.dy + bh * a.Tq * hs;
+    const T* kp = (const T*)a.k + bh * a.Tk * hs;
+    const T* vp = (const T*)a.v + bh * a.Tk * hs;
     const float* lse = a.lse2 + bh * a.Tq;
     const float* dsm = a.dsum + bh * a.Tq;
 
     u32x4 kf[KF], vf[KF];
     {
-        const size_t r = (size_t)min(key, a.Tk - 1) * HS;
+        const size_t r = (size_t)min(key, a.Tk - 1) * hs;
 #pragma unroll
         for (int f = 0; f < KF; f++) {
-            kf[f] = *(const u32x4*)(kp + r + f * CPF + half * (CPF / 2));
-            vf[f] = *(const u32x4*)(vp + r + f * CPF + half * (CPF / 2));
+            kf[f] = chunk(kp + r, f * CPF + half * (CPF / 2));
+            vf[f] = chunk(vp + r, f * CPF + half * (CPF / 2));
         }
     }
     bool keyMasked = false;
@@ -394,11 +398,11 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     u32x4 qreg[CPT], greg[CPT];
     float lreg = 0.f, dreg = 0.f;
     auto gload = [&](int q0) {
-        const size_t r = (size_t)min(q0 + srow, a.Tq - 1) * HS;
+        const size_t r = (size_t)min(q0 + srow, a.Tq - 1) * hs;
 #pragma unroll
         for (int i = 0; i < CPT; i++) {
-            qreg[i] = *(const u32x4*)(qp + r + (cg + TPR * i) * EPC);
-            greg[i] = *(const u32x4*)(gp + r + (cg + TPR * i) * EPC);
+            qreg[i] = chunk(qp + r, (cg + TPR * i) * EPC);
+            greg[i] = chunk(gp + r, (cg + TPR * i) * EPC);
         }
         if (tid < BQ) {
             const int qq = q0 + tid;
@@ -491,13 +495,14 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     }
     // dk[key, d] = scale * dK^T[d, key]; register v of tile dt is d = 32*dt + 8*(v/4) + 4*half + v%4
     if (waveActive && key < a.Tk) {
-        T* dkr = (T*)a.dk + (bh * a.Tk + key) * HS;
-        T* dvr = (T*)a.dv + (bh * a.Tk + key) * HS;
+        T* dkr = (T*)a.dk + (bh * a.Tk + key) * hs;
+        T* dvr = (T*)a.dv + (bh * a.Tk + key) * hs;
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const int d = 32 * dt + 8 * g + 4 * half;
+                if (PADDED && d >= hs) continue;
                 TR::store4(dkr + d, ak[dt][4 * g] * a.scale, ak[dt][4 * g + 1] * a.scale, ak[dt][4 * g + 2] * a.scale,
                            ak[dt][4 * g + 3] * a.scale);
                 TR::store4(dvr + d, av[dt][4 * g], av[dt][4 * g + 1], av[dt][4 * g + 2], av[dt][4 * g + 3]);
@@ -505,7 +510,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     }
 }
 
-template <typename T, int HS, int KIND, int BKS, int OCC>
+template <typename T, int HS, int KIND, int BKS, int OCC, bool PADDED>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs a, int mb)
 {
     typedef BwdTile<T, HS, BKS> TL;
@@ -528,21 +533,23 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
     const int ibh = rank % nbh;
     const int b = ibh / a.H, h = ibh % a.H;
     const size_t bh = (size_t)b * a.H + h;
+    const int hs = PADDED ? a.hs : HS;
+    auto chunk = [&](const T* row, int col) { return !PADDED || col < hs ? *(const u32x4*)(row + col) : u32x4{0, 0, 0, 0}; };
     const int q0w = qblock * BM + wave * 32;
     const int qrow = q0w + l32;
     const bool waveActive = q0w < a.Tq;
-    const T* qp = (const T*)a.q + bh * a.Tq * HS;
-    const T* gp = (const T*)a.dy + bh * a.Tq * HS;
-    const T* kp = (const T*)a.k + bh * a.Tk * HS;
-    const T* vp = (const T*)a.v + bh * a.Tk * HS;
+    const T* qp = (const T*)a.q + bh * a.Tq * hs;
+    const T* gp = (const T*)a.dy + bh * a.Tq * hs;
+    const T* kp = (const T*)a.k + bh * a.Tk * hs;
+    const T* vp = (const T*)a.v + bh * a.Tk * hs;
 
     u32x4 qf[KF], gf[KF];
     {
-        const size_t r = (size_t)min(qrow, a.Tq - 1) * HS;
+        const size_t r = (size_t)min(qrow, a.Tq - 1) * hs;
 #pragma unroll
         for (int f = 0; f < KF; f++) {
-            qf[f] = *(const u32x4*)(qp + r + f * CPF + half * (CPF / 2));
-            gf[f] = *(const u32x4*)(gp + r + f * CPF + half * (CPF / 2));
+            qf[f] = chunk(qp + r, f * CPF + half * (CPF / 2));
+            gf[f] = chunk(gp + r, f * CPF + half * (CPF / 2));
         }
     }
     const float lrow = qrow < a.Tq ? a.lse2[bh * a.Tq + qrow] : INFINITY;
@@ -550,9 +557,9 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
     // the dY fragments already in registers and stored for the dK/dV kernel, which is launched after this one.
     float drow = 0.f;
     if (a.computeD) {
-        const T* yp = (const T*)a.y + bh * a.Tq * HS + (size_t)min(qrow, a.Tq - 1) * HS;
+        const T* yp = (const T*)a.y + bh * a.Tq * hs + (size_t)min(qrow, a.Tq - 1) * hs;
 #pragma unroll
-        for (int f = 0; f < KF; f++) drow += TR::dot(*(const u32x4*)(yp + f * CPF + half * (CPF / 2)), gf[f]);
+        for (int f = 0; f < KF; f++) drow += TR::dot(chunk(yp, f * CPF + half * (CPF / 2)), gf[f]);
         drow += __shfl_xor(drow, 32, 64);
         if (qrow < a.Tq && half == 0) a.dsum[bh * a.Tq + qrow] = drow;
         if (qrow >= a.Tq) drow = 0.f;
@@ -569,11 +576,11 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
     u32x4 kreg[CPT], vreg[CPT];
     float mreg = 1.f;
     auto gload = [&](int k0) {
-        const size_t r = (size_t)min(k0 + srow, a.Tk - 1) * HS;
+        const size_t r = (size_t)min(k0 + srow, a.Tk - 1) * hs;
 #pragma unroll
         for (int i = 0; i < CPT; i++) {
-            kreg[i] = *(const u32x4*)(kp + r + (cg + TPR * i) * EPC);
-            vreg[i] = *(const u32x4*)(vp + r + (cg + TPR * i) * EPC);
+            kreg[i] = chunk(kp + r, (cg + TPR * i) * EPC);
+            vreg[i] = chunk(vp + r, (cg + TPR * i) * EPC);
         }
         if (KIND == 2 && tid < BKS) mreg = (k0 + tid < a.Tk) ? a.mask[(size_t)b * a.Tk + k0 + tid] : 1.f;
     };
@@ -647,25 +654,26 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
         __syncthreads();
     }
     if (waveActive && qrow < a.Tq) {
-        T* dqr = (T*)a.dq + (bh * a.Tq + qrow) * HS;
+        T* dqr = (T*)a.dq + (bh * a.Tq + qrow) * hs;
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
 #pragma unroll
             for (int g = 0; g < 4; g++)
-                TR::store4(dqr + 32 * dt + 8 * g + 4 * half, aq[dt][4 * g] * a.scale, aq[dt][4 * g + 1] * a.scale,
-                           aq[dt][4 * g + 2] * a.scale, aq[dt][4 * g + 3] * a.scale);
+                if (!PADDED || 32 * dt + 8 * g + 4 * half < hs)
+                    TR::store4(dqr + 32 * dt + 8 * g + 4 * half, aq[dt][4 * g] * a.scale, aq[dt][4 * g + 1] * a.scale,
+                               aq[dt][4 * g + 2] * a.scale, aq[dt][4 * g + 3] * a.scale);
     }
 }
 
-template <typename T, int HS, int BS, int OCC, int KIND>
+template <typename T, int HS, int BS, int OCC, int KIND, bool PADDED>
 static hipError_t bwd_launch_kind(hipStream_t s, const AttnBwdArgs& a, int mb)
 {
     typedef BwdTile<T, HS, BS> TL;
     const size_t nT = TL::TRR ? 0 : 1;   // transposed tiles
     const size_t kvBytes = ((size_t)2 * BS * TL::LDR + nT * 2 * HS * TL::LDT) * sizeof(T) + 2 * BS * sizeof(float);
     const size_t qBytes = ((size_t)2 * BS * TL::LDR + nT * HS * TL::LDT) * sizeof(T) + BS * sizeof(float);
-    auto kkv = attn_bwd_dkv_mfma_kernel<T, HS, KIND, BS, OCC>;
-    auto kq = attn_bwd_dq_mfma_kernel<T, HS, KIND, BS, OCC>;
+    auto kkv = attn_bwd_dkv_mfma_kernel<T, HS, KIND, BS, OCC, PADDED>;
+    auto kq = attn_bwd_dq_mfma_kernel<T, HS, KIND, BS, OCC, PADDED>;
     static bool configured = false;   // per instantiation; the attribute is idempotent, so a race only repeats the call
     if (!configured) {
         hipError_t e = hipFuncSetAttribute((const void*)kkv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kvBytes);
@@ -682,19 +690,19 @@ static hipError_t bwd_launch_kind(hipStream_t s, const AttnBwdArgs& a, int mb)
     return hipGetLastError();
 }
 
-template <typename T, int HS, int BS, int OCC> static hipError_t bwd_launch_cfg(hipStream_t s, const AttnBwdArgs& a, int kind, int mb)
+template <typename T, int HS, int BS, int OCC, bool PADDED = false> static hipError_t bwd_launch_cfg(hipStream_t s, const AttnBwdArgs& a, int kind, int mb)
 {
     switch (kind) {
-    case 0: return bwd_launch_kind<T, HS, BS, OCC, 0>(s, a, mb);
-    case 1: return bwd_launch_kind<T, HS, BS, OCC, 1>(s, a, mb);
-    case 2: return bwd_launch_kind<T, HS, BS, OCC, 2>(s, a, mb);
-    default: return bwd_launch_kind<T, HS, BS, OCC, 3>(s, a, mb);
+    case 0: return bwd_launch_kind<T, HS, BS, OCC, 0, PADDED>(s, a, mb);
+    case 1: return bwd_launch_kind<T, HS, BS, OCC, 1, PADDED>(s, a, mb);
+    case 2: return bwd_launch_kind<T, HS, BS, OCC, 2, PADDED>(s, a, mb);
+    default: return bwd_launch_kind<T, HS, BS, OCC, 3, PADDED>(s, a, mb);
     }
 }
 
-bool attn_bwd_mfma_usable(DType, const AttnBwdArgs& a)
+bool attn_bwd_mfma_usable(DType dt, const AttnBwdArgs& a)
 {
-    if (a.hs != 64 && a.hs != 128) return false;
+    if (a.hs > 128 || a.hs % (dt == F32 ? 4 : 8) != 0) return false;
     return (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.y | (uintptr_t)a.dy | (uintptr_t)a.dq | (uintptr_t)a.dk |
              (uintptr_t)a.dv) & 15) == 0;
 }
@@ -708,6 +716,12 @@ hipError_t attn_bwd_mfma_launch(hipStream_t s, DType dt, const AttnBwdArgs& a)
     case MASK_KEY: kind = 2; break;
     case MASK_BQK: kind = 3; break;
     default: kind = 3; mb = 0; break;          // MASK_QK: one (Tq,Tk) mask for every sequence
+    }
+    if (a.hs != 64 && a.hs != 128) {
+        if (dt == F32) return a.hs <= 32 ? bwd_launch_cfg<float, 32, 32, 2, true>(s, a, kind, mb)
+                            : a.hs < 64  ? bwd_launch_cfg<float, 64, 32, 2, true>(s, a, kind, mb)
+                                         : bwd_launch_cfg<float, 128, 32, 1, true>(s, a, kind, mb);
+        return a.hs < 64 ? bwd_launch_cfg<bf16_t, 64, 64, 2, true>(s, a, kind, mb) : bwd_launch_cfg<bf16_t, 128, 32, 1, true>(s, a, kind, mb);
     }
     if (dt == BF16) {
         if (a.hs == 64) return bwd_launch_cfg<bf16_t, 64, 64, 2>(s, a, kind, mb);

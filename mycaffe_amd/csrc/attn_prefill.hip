@@ -224,7 +224,9 @@ __device__ __forceinline__ void flash_softmax_step(floatx16 (&s)[QT], floatx16 (
 
 // KIND: 0 no mask, 1 causal, 2 per-key mask (B, Tk), 3 per-sequence mask (B, Tq, Tk).  OCC: workgroups per CU the register budget is set for.
 // PREFETCH: hold the next K / V block in registers while computing on the current one.
-template <typename T, int HS, int KIND, int QT, int NW, int OCC, bool PREFETCH>
+// PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 33 us;
+// the kernel with a wavefront per row, which had these, 546).
+template <typename T, int HS, int KIND, int QT, int NW, int OCC, bool PREFETCH, bool PADDED>
 __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
 {
     typedef FlashTraits<T> TR;
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
     // Row stride of the row-major V tile.  The transposing read takes 32 contiguous bytes from each of four rows per
     // 16 lanes, so rows must start 8 banks (32 bytes) apart modulo the bank count: 144 bytes (head size 64) does, 272
     // (head size 128 with the K padding) puts neighbouring rows 4 banks apart and halves the read rate; 288 does not.
-    constexpr int LDVR = (HS * (int)sizeof(T)) % 256 == 0 ? HS + 2 * PAD : HS + PAD;
+    constexpr int LDVR = (HS * (int)sizeof(T)) % 256 == 0 || HS == 32 ? HS + 2 * PAD : HS + PAD;   // 96 bytes at 32
     constexpr int CHR = HS / EPC;             // 16-byte chunks per K / V row
     constexpr int KPT = (BN * CHR) / NT;      // K chunks per thread per block
     // 16-bit storage keeps V row-major in LDS, staged exactly like K, and reads the V^T fragments with the transposing
@@ -271,10 +273,12 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         b = blockIdx.z;
     }
     const size_t bh = (size_t)b * a.H + h;
+    const int hs = PADDED ? a.hs : HS;
+    auto chunk = [&](const T* row, int col) { return !PADDED || col < hs ? *(const u32x4*)(row + col) : u32x4{0, 0, 0, 0}; };
     const int q0 = qblock * BM + wave * 32 * QT;      // first row of this wavefront
-    const T* qp = (const T*)a.q + bh * a.Tq * HS;
-    const T* kp = (const T*)a.k + bh * a.Tk * HS;
-    const T* vp = (const T*)a.v + bh * a.Tk * HS;
+    const T* qp = (const T*)a.q + bh * a.Tq * hs;
+    const T* kp = (const T*)a.k + bh * a.Tk * hs;
+    const T* vp = (const T*)a.v + bh * a.Tk * hs;
 
     // Q fragments: lane (query l32 of tile qt, half) holds elements f*CPF + half*CPF/2 .. of its row
     u32x4 qf[QT][KF];
@@ -282,7 +286,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
     for (int qt = 0; qt < QT; qt++) {
         int row = min(q0 + qt * 32 + l32, a.Tq - 1);
 #pragma unroll
-        for (int f = 0; f < KF; f++) qf[qt][f] = *(const u32x4*)(qp + (size_t)row * HS + f * CPF + half * (CPF / 2));
+        for (int f = 0; f < KF; f++) qf[qt][f] = chunk(qp + (size_t)row * hs, f * CPF + half * (CPF / 2));
     }
     floatx16 o[DT][QT];
 #pragma unroll
@@ -308,18 +312,18 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
 #pragma unroll
         for (int i = 0; i < KPT; i++) {
             const int e = tid + i * NT;
-            kreg[i] = *(const u32x4*)(kp + (size_t)min(kbase + e / CHR, a.Tk - 1) * HS + (e % CHR) * EPC);
+            kreg[i] = chunk(kp + (size_t)min(kbase + e / CHR, a.Tk - 1) * hs, (e % CHR) * EPC);
         }
         if (VROW) {
 #pragma unroll
             for (int i = 0; i < VPW; i++) {
                 const int e = tid + i * NT;
-                vreg[i] = *(const u32x4*)(vp + (size_t)min(kbase + e / CHR, a.Tk - 1) * HS + (e % CHR) * EPC);
+                vreg[i] = chunk(vp + (size_t)min(kbase + e / CHR, a.Tk - 1) * hs, (e % CHR) * EPC);
             }
         } else {
-            const size_t vrow = (size_t)min(kbase + lane, a.Tk - 1) * HS;
+            const size_t vrow = (size_t)min(kbase + lane, a.Tk - 1) * hs;
 #pragma unroll
-            for (int i = 0; i < VPW; i++) vreg[i] = *(const u32x4*)(vp + vrow + (wave + NW * i) * EPC);
+            for (int i = 0; i < VPW; i++) vreg[i] = chunk(vp + vrow, (wave + NW * i) * EPC);
         }
     };
     auto sstore = [&](int kb) {
@@ -467,13 +471,14 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         if (a.lse2 && qrow < a.Tq && half == 0)
             a.lse2[bh * a.Tq + qrow] = (m[qt] == a.maskedRaw) ? -INFINITY : __builtin_fmaf(m[qt], a.c, __log2f(lt));
         if (qrow < a.Tq) {
-            T* yr = (T*)a.y + attn_y_row(a.yMerged, b, h, a.H, a.Tq, qrow, HS);
+            T* yr = (T*)a.y + attn_y_row(a.yMerged, b, h, a.H, a.Tq, qrow, hs);
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
                 for (int g = 0; g < 4; g++)
-                    TR::store4(yr + 32 * dt + 8 * g + 4 * half, o[dt][qt][4 * g] * inv, o[dt][qt][4 * g + 1] * inv,
-                               o[dt][qt][4 * g + 2] * inv, o[dt][qt][4 * g + 3] * inv);
+                    if (!PADDED || 32 * dt + 8 * g + 4 * half < hs)
+                        TR::store4(yr + 32 * dt + 8 * g + 4 * half, o[dt][qt][4 * g] * inv, o[dt][qt][4 * g + 1] * inv,
+                                   o[dt][qt][4 * g + 2] * inv, o[dt][qt][4 * g + 3] * inv);
         }
     }
 }
@@ -862,23 +867,24 @@ __global__ __launch_bounds__(256) void flash_short_causal_f32_kernel(FlashArgs a
     }
 }
 
-template <typename T, int HS, int QT, int NW, int OCC, bool PREFETCH>
+template <typename T, int HS, int QT, int NW, int OCC, bool PREFETCH, bool PADDED = false>
 static hipError_t flash_launch_cfg(hipStream_t s, const FlashArgs& f, int kind)
 {
     constexpr int BM = NW * 32 * QT;
     dim3 grid((f.Tq + BM - 1) / BM, f.H, f.B);
     if (kind == MASK_CAUSAL) grid = dim3(((f.Tq + BM - 1) / BM) * f.H * f.B, 1, 1);
-    if (kind == MASK_NONE) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 0, QT, NW, OCC, PREFETCH>), grid, NW * 64, 0, s, f);
-    else if (kind == MASK_CAUSAL) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 1, QT, NW, OCC, PREFETCH>), grid, NW * 64, 0, s, f);
-    else if (kind == MASK_KEY) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 2, QT, NW, OCC, PREFETCH>), grid, NW * 64, 0, s, f);
-    else hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 3, QT, NW, OCC, PREFETCH>), grid, NW * 64, 0, s, f);   // MASK_BQK, MASK_QK
+    if (kind == MASK_NONE) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 0, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);
+    else if (kind == MASK_CAUSAL) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 1, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);
+    else if (kind == MASK_KEY) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 2, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);
+    else hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 3, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);   // MASK_BQK, MASK_QK
     return hipGetLastError();
 }
 
 hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* handled)
 {
     *handled = false;
-    if (a.hs != 64 && a.hs != 128) return hipSuccess;
+    // rows of whole 16-byte chunks; the kernels with a wavefront per row are left to other head sizes
+    if (a.hs > 128 || a.hs % (dt == F32 ? 4 : 8) != 0) return hipSuccess;
     if ((((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.y) & 15) != 0) return hipSuccess;
     FlashArgs f;
     f.maskBatch = a.kind == MASK_QK ? 0 : 1;   // a shared (Tq,Tk) mask is the per-sequence form with batch stride 0
@@ -890,6 +896,7 @@ hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* h
     f.lse2 = a.lse2;
     f.yMerged = a.yMerged;
     f.causalGroup = 0;
+    f.hs = a.hs;
     if (a.kind == MASK_CAUSAL && a.hs == 128 && dt == BF16) {
         // when K and V of all heads together exceed what the caches hold (128 MB taken as the line), walk the heads in
         // at most four groups of a multiple of 8 heads
@@ -898,6 +905,14 @@ hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* h
         if (kvBytes > 128e6 && nbh % 8 == 0) f.causalGroup = (int)(((nbh + 3) / 4 + 7) / 8 * 8);
     }
     *handled = true;
+    if (a.hs != 64 && a.hs != 128) {
+        if (dt == F32) return a.hs <= 32 ? flash_launch_cfg<float, 32, 1, 4, 2, false, true>(s, f, a.kind)
+                            : a.hs < 64  ? flash_launch_cfg<float, 64, 1, 4, 2, false, true>(s, f, a.kind)
+                                         : flash_launch_cfg<float, 128, 1, 8, 1, false, true>(s, f, a.kind);
+        return a.hs <= 32 ? flash_launch_cfg<bf16_t, 32, 1, 4, 3, true, true>(s, f, a.kind)
+             : a.hs < 64  ? flash_launch_cfg<bf16_t, 64, 1, 4, 3, true, true>(s, f, a.kind)
+                          : flash_launch_cfg<bf16_t, 128, 1, 8, 1, true, true>(s, f, a.kind);
+    }
     // Tile shapes picked by measurement on MI355X.  Head size 64: four wavefronts with one 32-row tile each
     // (128-row workgroups) give enough equal-sized workgroups to balance 256 CUs at T = 1024; head size 128
     // keeps eight wavefronts per workgroup so that each staged K / V block serves more rows.

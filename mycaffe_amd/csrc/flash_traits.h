@@ -144,6 +144,7 @@ struct FlashArgs {
     float* lse2;         // optional [B*H*Tq]: log2 of the softmax denominator of every row, kept for the backward pass
     int yMerged;         // y laid out (B,Tq,H,hs) instead of (B,H,Tq,hs)
     int causalGroup;     // causal launches: heads per group of the workgroup order (0: all heads in one group)
+    int hs;              // head size, of the kernels that take any up to their own
 };
 
 // Rank of a workgroup of a causal launch in the heaviest-first order.  Workgroup i goes to XCD i % 8 and, within it, the
