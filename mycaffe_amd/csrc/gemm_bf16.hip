@@ -28,9 +28,10 @@ struct GemmB16Args {
     float* part;              // kChunk < K: partial products, [part][M][N]
     bool vecC;
     const bf16_t* bias;
-    float* rowPart;           // sums of op(A)'s rows over some of the k: [part][tile column][M], to be added to rowSum (M)
-    bf16_t* rowSum;
 };
+
+// sums of op(A)'s rows over some of the k, [part][tile column][M], behind the partial products
+__device__ __forceinline__ float* b16_row_part(const GemmB16Args& g) { return g.part + (g.kChunk < g.K ? (size_t)g.parts * g.M * g.N : 0); }
 
 // the bias of eight columns from c on (past the matrix the last one, never stored); all eight loads are under way at once
 __device__ __forceinline__ void b16_bias8(const GemmB16Args& g, int c, float (&bias)[8])
@@ -48,15 +49,17 @@ __device__ __forceinline__ void b16_bias8(const GemmB16Args& g, int c, float (&b
 }
 
 // eight values of row r from column c on (inside the matrix up to N), alpha applied, and the bias, to C or through the heads
-// epilogue, whose column c of row 0 is at col
-template <bool HEADS>
-__device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<HEADS>& hp, int r, int c, const float (&bias)[8], bf16_t* col, float (&v)[8])
+// epilogue, whose column c of row 0 is at col and row r rowAt further.  HEADS: 0 none, 1 without a rotation, 2 with (a rotation's code in the ends of a tile
+// costs those that have none 1 us of 31: 3744 x 2880 x 960, 30.0 us, with a rotation 34.3, 42.1 with its tables read value by value and
+// every row's place divided out)
+template <int HEADS>
+__device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<(HEADS > 0)>& hp, int r, int c, const float (&bias)[8], bf16_t* col, size_t rowAt, float (&v)[8])
 {
 #pragma unroll
     for (int q = 0; q < 8; q++) v[q] += bias[q];
     if (g.vecC) {
         bf16_t* cp = g.C + (size_t)r * g.N + c;
-        if constexpr (HEADS) cp = col + heads_row(hp.he, r);
+        if constexpr (HEADS) cp = col + rowAt;
         if (!HEADS && g.beta != 0.f) {
             const u32x4 o = *(const u32x4*)cp;
             const uint32_t w[4] = {o.x, o.y, o.z, o.w};
@@ -68,7 +71,7 @@ __device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<
         }
         u32x4 p;
         p.x = pack2_bf16(v[0], v[1]); p.y = pack2_bf16(v[2], v[3]); p.z = pack2_bf16(v[4], v[5]); p.w = pack2_bf16(v[6], v[7]);
-        if constexpr (HEADS) p = heads_rope_piece<bf16_t>(hp.he, r, c, p);
+        if constexpr (HEADS == 2) p = heads_rope_piece<bf16_t>(hp.he, r, c, p);
         *(u32x4*)cp = p;
         return;
     }
@@ -78,10 +81,11 @@ __device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<
         const bool two = c + q + 1 < g.N;
         if constexpr (HEADS) {
             float o0 = bf16_to_f32(f32_to_bf16(v[q])), o1 = bf16_to_f32(f32_to_bf16(v[q + 1]));   // as the storage type holds them
-            if (hp.he.fcos && c + q < 2 * hp.he.H * hp.he.hs) {
-                const size_t ti = heads_rope_at(hp.he, r, c + q);
-                heads_rope_pair(hp.he.fcos[ti], hp.he.fsin[ti], o0, o1);
-            }
+            if constexpr (HEADS == 2)
+                if (hp.he.fcos && c + q < 2 * hp.he.H * hp.he.hs) {
+                    const size_t ti = heads_rope_at(hp.he, r, c + q);
+                    heads_rope_pair(hp.he.fcos[ti], hp.he.fsin[ti], o0, o1);
+                }
             *heads_dst<bf16_t>(hp.he, r, c + q) = f32_to_bf16(o0);
             if (two) *heads_dst<bf16_t>(hp.he, r, c + q + 1) = f32_to_bf16(o1);
         } else {
@@ -94,8 +98,8 @@ __device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<
 
 // tile `item` of a product.  SUMS: the tiles of a row of tiles also add up the rows of op(A), each the stages that are its turn, from
 // the fragments it multiplies: the bias gradient beside a weight gradient (8000 x 3072, 6.2 to 12.8 us and a launch of 5 on their own).
-template <int WVM, int WVN, int WM, int WN, bool AK, bool BKC, bool HEADS, bool SUMS = false>
-__device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HEADS>& hp, int item)
+template <int WVM, int WVN, int WM, int WN, bool AK, bool BKC, int HEADS, bool SUMS = false>
+__device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(HEADS > 0)>& hp, int item)
 {
     constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64, KS = 4;
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;               // 16-byte chunks per thread and stage
@@ -285,7 +289,7 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
                 float v = ((sums[t][0] + sums[t][1]) + (sums[t][2] + sums[t][3])) + ((sums[t][4] + sums[t][5]) + (sums[t][6] + sums[t][7]));
                 v += __shfl_xor(v, 32);
                 const int r = m0 + wm + t * 32 + fr;
-                if (half == 0 && r < M) g.rowPart[(size_t)(part * g.tilesN + n0 / BN) * M + r] = v;
+                if (half == 0 && r < M) b16_row_part(g)[(size_t)(part * g.tilesN + n0 / BN) * M + r] = v;
             }
         }
     }
@@ -314,9 +318,18 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
                 b16_bias8(g, c, bias);
                 if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
             }
+            // the rows' places: added up, not divided out for each
+            size_t nextAt = 0;
+            int t = 0;
+            if constexpr (HEADS) nextAt = heads_row(hp.he, m0 + wm + i * 32 + rr, t);
 #pragma unroll 2
             for (int it = 0; it < NIT; it++) {
                 const int row = it * RPI + rr, r = m0 + wm + i * 32 + row;
+                const size_t rowAt = nextAt;
+                if constexpr (HEADS) {
+                    nextAt += (size_t)(RPI * hp.he.hs);
+                    for (t += RPI; t >= hp.he.T; t -= hp.he.T) nextAt += hp.he.perBatch - (unsigned long long)(uint32_t)hp.he.T * (uint32_t)hp.he.hs;
+                }
                 if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
                 const float4 t0 = *(const float4*)(cs + row * LDC + cc), t1 = *(const float4*)(cs + row * LDC + cc + 4);
                 float v[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
@@ -331,7 +344,7 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
                             if (c + q < N) cp[q] = v[q];
                     }
                 } else {
-                    b16_store8<HEADS>(g, hp, r, c, bias, col, v);
+                    b16_store8<HEADS>(g, hp, r, c, bias, col, rowAt, v);
                 }
             }
         }
@@ -340,11 +353,12 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<HE
 // each XCD (workgroup index mod 8) takes a contiguous run of the tiles
 __device__ __forceinline__ int b16_xcd_item(int total) { return (int)(blockIdx.x % 8) * ((total + 7) / 8) + (int)(blockIdx.x / 8); }
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS, bool SUMS>
-__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
+__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<(HEADS > 0)> hp)
 {
     const int total = g.tilesM * g.tilesN * g.parts, item = b16_xcd_item(total);
-    if (item < total) b16_tile<WVM, WVN, WM, WN, AK, BKC, HEADS, SUMS>(g, hp, item);
+    if (item >= total) return;
+    b16_tile<WVM, WVN, WM, WN, AK, BKC, HEADS, SUMS>(g, hp, item);
 }
 
 // Up to three products with heads epilogues as one launch: the projections of a multi-head attention layer.  One by one each is less
@@ -356,7 +370,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_group_kernel(Gem
     const int item = b16_xcd_item(grp.first[3]);
     if (item >= grp.first[3]) return;
     const int p = item >= grp.first[2] ? 2 : item >= grp.first[1] ? 1 : 0;
-    b16_tile<WVM, WVN, WM, WN, true, true, true>(grp.g[p], grp.h[p], item - grp.first[p]);
+    b16_tile<WVM, WVN, WM, WN, true, true, 1>(grp.g[p], grp.h[p], item - grp.first[p]);
 }
 
 // ---------------------------------------------------------------------------
@@ -367,8 +381,8 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_group_kernel(Gem
 // Microseconds with B not in any cache, before (tiles in parts of the contraction, and a launch that adds them up) and now:
 // 8 x 12288 x 4096 24.2, 20.6 (4.9 TB/s); 8 x 4096 x 4096 15.4, 8.8; 32 x 12288 x 4096 25.2, 23.5; 32 x 4096 x 4096 15.6, 11.7;
 // 8 x 2304 x 768 8.3, 3.7; 8 x 512 x 512 6.2, 3.3.  What is left over the reading of B is the launch's beginning and end.
-template <int MT, int NT, int NW, int S, bool HEADS>
-__global__ __launch_bounds__(64 * NW) void gemm_b16_rows_kernel(GemmB16Args g, HeadsArg<HEADS> hp)
+template <int MT, int NT, int NW, int S, int HEADS>
+__global__ __launch_bounds__(64 * NW) void gemm_b16_rows_kernel(GemmB16Args g, HeadsArg<(HEADS > 0)> hp)
 {
     constexpr int KW = 128 / MT, KS = KW / 32, P = KW / 8;   // k, products and 16-byte pieces of a row, of a stage
     constexpr int STAGE = 16 * MT * KW, DA = STAGE / 512;    // elements of A in a stage, fetches
@@ -482,28 +496,30 @@ __global__ __launch_bounds__(64 * NW) void gemm_b16_rows_kernel(GemmB16Args g, H
 #pragma unroll
     for (int q = 0; q < 8; q++) v[q] *= g.alpha;
     bf16_t* col = nullptr;
-    if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
-    b16_store8<HEADS>(g, hp, row, c, bias, col, v);
+    size_t rowAt = 0;
+    if constexpr (HEADS) { col = heads_col<bf16_t>(hp.he, c); rowAt = heads_row(hp.he, row); }
+    b16_store8<HEADS>(g, hp, row, c, bias, col, rowAt, v);
 }
 
 // sum over the S partial products in their order, then as b16_store8; the first rowBlocks workgroups add the partial row sums to rowSum
-template <bool HEADS>
-__global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<HEADS> hp, int S, int rowBlocks)
+template <int HEADS>
+__global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsArg<(HEADS > 0)> hp, int S, int rowBlocks, bf16_t* rowSum)
 {
     const int block = (int)blockIdx.x - rowBlocks;
     if (block < 0) {
         const int r = (int)blockIdx.x * 256 + threadIdx.x;
         if (r >= g.M) return;
         const int count = g.parts * g.tilesN;
+        const float* rowPart = b16_row_part(g);
         float v = 0.f;
         for (int p0 = 0; p0 < count; p0 += 8) {   // eight loads under way
             float x[8];
 #pragma unroll
-            for (int q = 0; q < 8; q++) x[q] = g.rowPart[(size_t)min(p0 + q, count - 1) * g.M + r];
+            for (int q = 0; q < 8; q++) x[q] = rowPart[(size_t)min(p0 + q, count - 1) * g.M + r];
 #pragma unroll
             for (int q = 0; q < 8; q++) v += p0 + q < count ? x[q] : 0.f;
         }
-        g.rowSum[r] = f32_to_bf16(bf16_to_f32(g.rowSum[r]) + v);
+        rowSum[r] = f32_to_bf16(bf16_to_f32(rowSum[r]) + v);
         return;
     }
     const int oct = (g.N + 7) / 8;
@@ -525,8 +541,9 @@ __global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsA
         float bias[8];
         b16_bias8(g, c, bias);
         bf16_t* col = nullptr;
-        if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
-        b16_store8<HEADS>(g, hp, r, c, bias, col, v);
+        size_t rowAt = 0;
+        if constexpr (HEADS) { col = heads_col<bf16_t>(hp.he, c); rowAt = heads_row(hp.he, r); }
+        b16_store8<HEADS>(g, hp, r, c, bias, col, rowAt, v);
     }
 }
 
@@ -601,7 +618,7 @@ size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k)
     return gemm_b16_workspace_bytes(m, n, k) + (size_t)p.splits * columns * m * sizeof(float);
 }
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, bool HEADS, bool SUMS>
+template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
 static hipError_t launch_b16(hipStream_t s, GemmB16Args& g, const HeadsEpilogue* he)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN, CH = WN % 2 == 0 ? 2 : WN;
@@ -612,10 +629,10 @@ static hipError_t launch_b16(hipStream_t s, GemmB16Args& g, const HeadsEpilogue*
     g.tilesN = (g.N + BN - 1) / BN;
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS, SUMS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS, SUMS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, heads_arg<(HEADS > 0)>(he));
     return hipGetLastError();
 }
-template <bool AK, bool BKC, bool HEADS, bool SUMS = false>
+template <bool AK, bool BKC, int HEADS, bool SUMS = false>
 static hipError_t launch_b16_shape(hipStream_t s, GemmB16Args& a, int shape, const HeadsEpilogue* he = nullptr)
 {
     switch (shape) {
@@ -666,8 +683,8 @@ static bool b16_rows_takes(const GemmB16& q)
         if (!free(q.heads->dst[w], (size_t)q.m * third * 2)) return false;
     return true;
 }
-template <int MT, int NT, int NW, int S, bool HEADS>
-static hipError_t launch_b16_rows_shape(hipStream_t s, const GemmB16Args& g, const HeadsArg<HEADS>& ha)
+template <int MT, int NT, int NW, int S, int HEADS>
+static hipError_t launch_b16_rows_shape(hipStream_t s, const GemmB16Args& g, const HeadsArg<(HEADS > 0)>& ha)
 {
     constexpr int lds = NW * S * 16 * 128 * 2;
     static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_rows_kernel<MT, NT, NW, S, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -678,8 +695,8 @@ static hipError_t launch_b16_rows_shape(hipStream_t s, const GemmB16Args& g, con
 // One workgroup a CU of 16, 32 or 48 columns as long as that holds all of them: the wider ones read A as often less, and eight
 // wavefronts with four stages, or more columns and two, keep 100 KB and more of B on their way.  Past that workgroups of four
 // wavefronts, three of them on a CU, so that one's end is another's middle.
-template <int MT, bool HEADS>
-static hipError_t launch_b16_rows(hipStream_t s, const GemmB16Args& g, const HeadsArg<HEADS>& ha)
+template <int MT, int HEADS>
+static hipError_t launch_b16_rows(hipStream_t s, const GemmB16Args& g, const HeadsArg<(HEADS > 0)>& ha)
 {
     if (g.N <= 256 * 16) return launch_b16_rows_shape<MT, 1, 8, 4, HEADS>(s, g, ha);
     if (g.N <= 512 * 16) return launch_b16_rows_shape<MT, 2, 8, 2, HEADS>(s, g, ha);
@@ -693,8 +710,9 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
     if (!gemm_b16_takes(q) || (q.heads && (q.alpha != 1.f || q.beta != 0.f || !q.aK || !q.bK))) return hipErrorInvalidValue;
     if (b16_rows_takes(q)) {
         const GemmB16Args a = b16_args(q);
-        if (q.heads) return q.m > 16 ? launch_b16_rows<2, true>(s, a, heads_arg<true>(q.heads)) : launch_b16_rows<1, true>(s, a, heads_arg<true>(q.heads));
-        return q.m > 16 ? launch_b16_rows<2, false>(s, a, HeadsArg<false>()) : launch_b16_rows<1, false>(s, a, HeadsArg<false>());
+        if (q.heads && q.heads->fcos) return q.m > 16 ? launch_b16_rows<2, 2>(s, a, heads_arg<true>(q.heads)) : launch_b16_rows<1, 2>(s, a, heads_arg<true>(q.heads));
+        if (q.heads) return q.m > 16 ? launch_b16_rows<2, 1>(s, a, heads_arg<true>(q.heads)) : launch_b16_rows<1, 1>(s, a, heads_arg<true>(q.heads));
+        return q.m > 16 ? launch_b16_rows<2, 0>(s, a, HeadsArg<false>()) : launch_b16_rows<1, 0>(s, a, HeadsArg<false>());
     }
     GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
     if (q.rowSum) {
@@ -705,18 +723,17 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
     GemmB16Args a = b16_args(q);
     a.parts = p.splits; a.kChunk = p.kChunk;
     a.part = (float*)ws;
-    a.rowSum = q.rowSum;
-    a.rowPart = a.part + (p.splits > 1 ? (size_t)p.splits * q.m * q.n : 0);
     hipError_t e;
-    if (q.heads) e = launch_b16_shape<true, true, true>(s, a, p.shape, q.heads);
-    else if (q.rowSum) e = launch_b16_shape<false, false, false, true>(s, a, p.shape);
-    else if (q.aK) e = q.bK ? launch_b16_shape<true, true, false>(s, a, p.shape) : launch_b16_shape<true, false, false>(s, a, p.shape);
-    else e = q.bK ? launch_b16_shape<false, true, false>(s, a, p.shape) : launch_b16_shape<false, false, false>(s, a, p.shape);
+    if (q.heads && q.heads->fcos) e = launch_b16_shape<true, true, 2>(s, a, p.shape, q.heads);
+    else if (q.heads) e = launch_b16_shape<true, true, 1>(s, a, p.shape, q.heads);
+    else if (q.rowSum) e = launch_b16_shape<false, false, 0, true>(s, a, p.shape);
+    else if (q.aK) e = q.bK ? launch_b16_shape<true, true, 0>(s, a, p.shape) : launch_b16_shape<true, false, 0>(s, a, p.shape);
+    else e = q.bK ? launch_b16_shape<false, true, 0>(s, a, p.shape) : launch_b16_shape<false, false, 0>(s, a, p.shape);
     const int rowBlocks = q.rowSum ? (q.m + 255) / 256 : 0;
     const int grid = rowBlocks + (p.splits > 1 ? (int)std::min<size_t>(((size_t)q.m * ((q.n + 7) / 8) + 255) / 256, 4096) : 0);
     if (e != hipSuccess || grid == 0) return e;
-    if (q.heads) hipLaunchKernelGGL(gemm_b16_sum_kernel<true>, grid, 256, 0, s, a, heads_arg<true>(q.heads), p.splits, 0);
-    else hipLaunchKernelGGL(gemm_b16_sum_kernel<false>, grid, 256, 0, s, a, HeadsArg<false>(), p.splits, rowBlocks);
+    if (q.heads) hipLaunchKernelGGL(gemm_b16_sum_kernel<2>, grid, 256, 0, s, a, heads_arg<true>(q.heads), p.splits, 0, (bf16_t*)nullptr);
+    else hipLaunchKernelGGL(gemm_b16_sum_kernel<0>, grid, 256, 0, s, a, HeadsArg<false>(), p.splits, rowBlocks, q.rowSum);
     return hipGetLastError();
 }
 

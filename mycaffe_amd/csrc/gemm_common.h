@@ -102,6 +102,7 @@ template <> struct BigTraits<float> {
 struct HeadsEpilogue {
     const void* bias; void* dst[3]; int T, H, hs; const float* fcos; const float* fsin; int seq;
     uint32_t mT, mC, mhs, mseq;   // floor(2^32 / T), / (H hs), / hs, / seq
+    unsigned long long perBatch;  // H T hs
 };
 static inline HeadsEpilogue heads_epilogue(const void* bias, void* q, void* k, void* v, int T, int H, int hs, const float* fcos, const float* fsin, int seq)
 {
@@ -109,6 +110,7 @@ static inline HeadsEpilogue heads_epilogue(const void* bias, void* q, void* k, v
     HeadsEpilogue he;
     he.bias = bias; he.dst[0] = q; he.dst[1] = k; he.dst[2] = v; he.T = T; he.H = H; he.hs = hs;
     he.fcos = fcos; he.fsin = fsin; he.seq = seq;
+    he.perBatch = (unsigned long long)H * T * hs;
     he.mT = magic(T); he.mC = magic(H * hs); he.mhs = magic(hs); he.mseq = magic(seq);
     return he;
 }
@@ -138,11 +140,15 @@ __device__ __forceinline__ T* heads_col(const HeadsEpilogue& he, int col)
     const int which = heads_div(col, he.H * he.hs, he.mC, w), h = heads_div(w, he.hs, he.mhs, d);
     return (T*)(which == 0 ? he.dst[0] : which == 1 ? he.dst[1] : he.dst[2]) + (size_t)h * he.T * he.hs + d;
 }
+__device__ __forceinline__ size_t heads_row(const HeadsEpilogue& he, int row, int& t)   // t: the row's position in its sequence
+{
+    const int b = heads_div(row, he.T, he.mT, t);
+    return (size_t)((uint32_t)b * he.perBatch + (unsigned long long)(uint32_t)t * (uint32_t)he.hs);
+}
 __device__ __forceinline__ size_t heads_row(const HeadsEpilogue& he, int row)
 {
     int t;
-    const int b = heads_div(row, he.T, he.mT, t);
-    return ((size_t)b * he.H * he.T + t) * he.hs;
+    return heads_row(he, row, t);
 }
 template <typename T>
 __device__ __forceinline__ T* heads_dst(const HeadsEpilogue& he, int row, int col) { return heads_col<T>(he, col) + heads_row(he, row); }
@@ -171,9 +177,12 @@ __device__ __forceinline__ u32x4 heads_rope_piece(const HeadsEpilogue& he, int r
     constexpr int NP = 8 / (int)sizeof(T);
     const size_t ti = heads_rope_at(he, row, col);
     uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    // a piece's pairs are whole aligned pieces of the tables too (hs is a multiple of the elements of a piece)
+    typedef float Row __attribute__((ext_vector_type(NP)));
+    const Row cs = *(const Row*)(he.fcos + ti), sns = *(const Row*)(he.fsin + ti);
 #pragma unroll
     for (int i = 0; i < NP; i++) {
-        const float c = he.fcos[ti + i], sn = he.fsin[ti + i];
+        const float c = cs[i], sn = sns[i];
         if constexpr (sizeof(T) == 4) {
             float re = __uint_as_float(w[2 * i]), im = __uint_as_float(w[2 * i + 1]);
             heads_rope_pair(c, sn, re, im);
@@ -181,7 +190,7 @@ __device__ __forceinline__ u32x4 heads_rope_piece(const HeadsEpilogue& he, int r
         } else {
             float re = __uint_as_float(w[i] << 16), im = __uint_as_float(w[i] & 0xffff0000u);
             heads_rope_pair(c, sn, re, im);
-            w[i] = (uint32_t)f32_to_bf16(re) | ((uint32_t)f32_to_bf16(im) << 16);
+            w[i] = pack2_bf16(re, im);
         }
     }
     u32x4 o; o.x = w[0]; o.y = w[1]; o.z = w[2]; o.w = w[3];
