@@ -1282,18 +1282,28 @@ template <typename T> static void bias_grad(hipStream_t s, DType dt, int m, int 
     hipLaunchKernelGGL(gemv_t_sum_kernel<T>, (n + 63) / 64, 64, 0, s, n, chunks, 1.f, (const float*)part, 1.f, db);
 }
 // Weight and bias gradient as one pass over dY (16-bit storage, 8000 rows, 768 to 3072: 69.5 us one after the other, 55.9 together;
-// 3072 to 768: 62.5, 56.8; 2048 rows, 512 to 512: 18.0, 11.7).  Up to 1024 rows the column sums are one short launch; a bias that shares memory with
-// another operand is left to the calls one after the other.
+// 3072 to 768: 62.5, 56.8; 2048 rows, 512 to 512: 18.0, 11.7; fp32, 8000 rows,
+// 768 to 3072: 210, 193).  A bias that
+// shares memory with another operand is left to the calls one after the other.
 size_t k_weight_bias_grad_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* dY, const void* dW, const void* db)
 {
-    if (dt != BF16 || m <= 1024 || !gemm_b16_takes(b16_product(true, false, n, k, m, 1.f, dY, X, 1.f, nullptr))) return 0;
-    auto apart = [&](const void* o, size_t elems) { return (uintptr_t)db + 2 * (size_t)n <= (uintptr_t)o || (uintptr_t)o + 2 * elems <= (uintptr_t)db; };
+    const size_t es = dt == F32 ? 4 : 2;
+    auto apart = [&](const void* o, size_t elems) { return (uintptr_t)db + es * n <= (uintptr_t)o || (uintptr_t)o + es * elems <= (uintptr_t)db; };
     if (!apart(X, (size_t)m * k) || !apart(dY, (size_t)m * n) || !apart(dW, (size_t)n * k)) return 0;
-    return gemm_b16_row_sums_workspace_bytes(n, k, m);
+    if (dt == F32) return gemm_f32_row_sums_workspace_bytes(n, k, m, (((uintptr_t)X | (uintptr_t)dY) & 15) == 0 && n % 4 == 0 && k % 4 == 0);
+    return gemm_b16_takes(b16_product(true, false, n, k, m, 1.f, dY, X, 1.f, nullptr)) ? gemm_b16_row_sums_workspace_bytes(n, k, m) : 0;
 }
 hipError_t k_weight_bias_grad(hipStream_t s, DType dt, int m, int n, int k, const void* X, const void* dY, void* dW, void* db, void* ws, size_t wsBytes)
 {
-    if (dt != BF16) return hipErrorInvalidValue;
+    if (dt == F32) {
+        GemmF32 g = {};
+        g.m = n; g.n = k; g.k = m;
+        g.A = (const float*)dY; g.B = (const float*)X; g.C = (float*)dW;
+        g.lda = n; g.ldb = g.ldc = k;
+        g.alpha = g.beta = 1.f; g.batch = 1;
+        g.rowSum = (float*)db;
+        return gemm_f32(s, g, ws, wsBytes);
+    }
     GemmB16 g = b16_product(true, false, n, k, m, 1.f, dY, X, 1.f, dW);
     g.rowSum = (bf16_t*)db;
     return gemm_b16(s, g, ws, wsBytes);

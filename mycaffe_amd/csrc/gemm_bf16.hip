@@ -509,17 +509,7 @@ __global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsA
     if (block < 0) {
         const int r = (int)blockIdx.x * 256 + threadIdx.x;
         if (r >= g.M) return;
-        const int count = g.parts * g.tilesN;
-        const float* rowPart = b16_row_part(g);
-        float v = 0.f;
-        for (int p0 = 0; p0 < count; p0 += 8) {   // eight loads under way
-            float x[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) x[q] = rowPart[(size_t)min(p0 + q, count - 1) * g.M + r];
-#pragma unroll
-            for (int q = 0; q < 8; q++) v += p0 + q < count ? x[q] : 0.f;
-        }
-        rowSum[r] = f32_to_bf16(bf16_to_f32(rowSum[r]) + v);
+        rowSum[r] = f32_to_bf16(bf16_to_f32(rowSum[r]) + sum_partials(b16_row_part(g) + r, g.parts * g.tilesN, g.M));
         return;
     }
     const int oct = (g.N + 7) / 8;
@@ -614,7 +604,7 @@ size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k)
     if (m <= 0 || n <= 0 || k <= 0) return 0;
     const GemmB16Plan p = gemm_b16_plan(m, n, k);
     const long long columns = b16_tile_columns(p.shape, n);
-    if (p.kChunk / (16 * columns) > 128) return 0;
+    if (p.kChunk / (16 * columns) > 128 || (k <= 1024 && p.splits == 1)) return 0;   // one short launch would only be another
     return gemm_b16_workspace_bytes(m, n, k) + (size_t)p.splits * columns * m * sizeof(float);
 }
 

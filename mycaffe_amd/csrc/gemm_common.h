@@ -54,6 +54,20 @@ template <int ROWB> __device__ __forceinline__ int block_swizzle(int k)
     return ROWB % 256 == 0 ? (k & 3) * 4 : ((k >> 1) & 1) * 4;   // in chunks; rows 128 bytes apart modulo 256 alternate already
 }
 
+// the sum of p[0], p[stride], .. : eight loads under way, and eight sums, so that none is long
+__device__ __forceinline__ float sum_partials(const float* p, int count, int stride)
+{
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int p0 = 0; p0 < count; p0 += 8) {
+        float x[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) x[q] = p[(size_t)min(p0 + q, count - 1) * stride];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] += p0 + q < count ? x[q] : 0.f;
+    }
+    return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+}
+
 template <typename T> __device__ inline float ldf(const T* p, size_t i);
 template <> __device__ inline float ldf<float>(const float* p, size_t i) { return p[i]; }
 template <> __device__ inline float ldf<bf16_t>(const bf16_t* p, size_t i) { return bf16_to_f32(p[i]); }
@@ -228,9 +242,11 @@ struct GemmF32 {
     const float* bias;                     // null, or n values added to every row of C (batch 1)
     const HeadsEpilogue* heads;            // written through this epilogue instead of to C (alpha 1, beta 0, batch 1, bias null)
     bool fp32Sums;                         // on the fp32 matrix cores, one value of k after the other, whatever the size
+    float* rowSum;                         // (m) += the sums of op(A)'s rows; dense operands, both with their rows at unit stride
 };
 enum { CAUSAL_NO = 0, CAUSAL_A_LOWER /* A(i,k) zero for k > i */, CAUSAL_A_UPPER /* k < i */, CAUSAL_B_LOWER /* B(k,j) zero for k < j */, CAUSAL_B_UPPER /* k > j */ };
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal);
+size_t gemm_f32_row_sums_workspace_bytes(int m, int n, int k, bool vec);   // with rowSum; vec: operands in whole aligned 16-byte chunks; 0: not taken together
 hipError_t gemm_f32(hipStream_t s, const GemmF32& g, void* ws, size_t wsBytes);
 
 // The same in 16-bit storage, dense row-major operands (gemm_bf16.hip): op(A) stored (m, k) or (k, m), op(B) (n, k) or (k, n)

@@ -468,7 +468,18 @@ __device__ __forceinline__ void f32_sums(const GemmF32Args& g, const float* A, c
 // bytes of one plane of R rows by 16 KS k
 template <int R, int KS, bool KFAST> constexpr int split_plane() { return KFAST ? 2 * KS * (R * 16 + 128 / KS) : 16 * KS * R * 2; }
 
-template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
+// floats that the split kernel's stages, and then its results, take in LDS: behind them the row sums
+template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC> constexpr int split_lds()
+{
+    constexpr int stages = 2 * 3 * (split_plane<32 * WVM * WM, KS, AK>() + split_plane<32 * WVN * WN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
+    return (stages > store ? stages : store) / 4;
+}
+// sums of op(A)'s rows over some of the k, [part][tile column][M], behind the partial products
+__device__ __forceinline__ float* f32_row_part(const GemmF32Args& g) { return g.part + (g.kChunk < g.K ? (size_t)g.parts * g.M * g.N : 0); }
+
+// SUMS: the tiles of a row of tiles also add up the rows of op(A), each the stages that are its turn, from the chunks it fetches: the
+// bias gradient beside a weight gradient (8192 rows, 768 to 2304: 169 us one after the other, 157 together).
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS>
 __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
 {
     constexpr int NT = 64 * WVM * WVN, BK = 16 * KS, BM = 32 * WVM * WM, BN = 32 * WVN * WN;
@@ -578,8 +589,19 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             else raw[c] = __builtin_amdgcn_raw_buffer_load_b128(resource(stageB), vb[c - PA], 0, 0);
         }
     };
+    // SUMS: a thread's chunks of A are of the same four rows; without branches, between reads that are under way
+    static_assert(!SUMS || (!AK && NT % (BM / 4) == 0), "");
+    [[maybe_unused]] float sums[4] = {0.f, 0.f, 0.f, 0.f};
+    [[maybe_unused]] int turn = n0 / BN, putting = 0;   // the stage that is put, and stages until this tile's next
+    [[maybe_unused]] uint32_t mine = turn == 0 ? 0xffffffffu : 0u;
     // part s of chunk c to its plane of a stage
     auto put = [&](int c, int s, unsigned char* stage) {
+        if constexpr (SUMS) {
+            if (s == 0 && c < PA) {
+                sums[0] += __uint_as_float(raw[c].x & mine); sums[1] += __uint_as_float(raw[c].y & mine);
+                sums[2] += __uint_as_float(raw[c].z & mine); sums[3] += __uint_as_float(raw[c].w & mine);
+            }
+        }
         float v[4] = {__uint_as_float(raw[c].x), __uint_as_float(raw[c].y), __uint_as_float(raw[c].z), __uint_as_float(raw[c].w)};
         const uint2 p = split_part(v, s == 2);
         raw[c].x = __float_as_uint(v[0]); raw[c].y = __float_as_uint(v[1]); raw[c].z = __float_as_uint(v[2]); raw[c].w = __float_as_uint(v[3]);
@@ -641,6 +663,11 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
         const int at = u * STAGE;
         unsigned char* next = smem_raw + STAGE - at;
         nextStage();
+        if constexpr (SUMS) {
+            putting++;
+            turn = turn == 0 ? g.tilesN - 1 : turn - 1;
+            mine = turn == 0 && putting < nk ? 0xffffffffu : 0u;   // past the end the last stage is put again
+        }
         // what goes between the products: chunks of the next stage part by part to the other buffer, each then fetched anew
         constexpr int SLOTS = (6 * KS - 2) * NMF, STEPS = 3 * P;
         auto slot = [&](int q) {
@@ -691,6 +718,17 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     for (int kt = 0; kt < nk; kt += 2) {
         stage(0);
         if (kt + 1 < nk) stage(1);
+    }
+    if constexpr (SUMS) {
+        float* all = reinterpret_cast<float*>(smem_raw) + split_lds<WVM, WVN, WM, WN, KS, AK, BKC>();
+        *(float4*)(all + 4 * tid) = make_float4(sums[0], sums[1], sums[2], sums[3]);
+        __syncthreads();
+        if (tid < BM && m0 + tid < M) {
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < NT / (BM / 4); w++) v += all[w * BM + tid];
+            f32_row_part(g)[(size_t)(it.part * g.tilesN + n0 / BN) * M + m0 + tid] = v;
+        }
     }
     __syncthreads();
     if (split_lost(acc)) f32_sums<WM, WN, AK, BKC, false>(g, A, B, m0 + wm, n0 + wn, kBegin, it.kEnd, lane, acc);
@@ -888,14 +926,23 @@ __global__ __launch_bounds__(64 * NW) void linear_bwd_f32_small_kernel(GemmF32Ar
     }
 }
 
+// the row sums that gemm_f32_sum_kernel adds to `sum`: `count` partial ones for each of M rows, by its first `blocks` workgroups
+struct F32RowSums { int blocks, count; const float* part; float* sum; };
 // C = sum over the S partial products, in their order (alpha is in them already), + beta C; or through the heads epilogue
 template <bool HEADS>
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(const float* __restrict__ part, int S, int M, int N, long long ldc, float beta, bool vecC,
-                                                           float* __restrict__ C, const float* __restrict__ bias, HeadsArg<HEADS> hp)
+                                                           float* __restrict__ C, const float* __restrict__ bias, HeadsArg<HEADS> hp, F32RowSums rows)
 {
+    const int block = (int)blockIdx.x - rows.blocks;
+    if (block < 0) {   // the first workgroups: the partial row sums
+        const int r = (int)blockIdx.x * 256 + threadIdx.x;
+        if (r >= M) return;
+        rows.sum[r] += sum_partials(rows.part + r, rows.count, M);
+        return;
+    }
     const int quads = (N + 3) / 4;
     const size_t mn = (size_t)M * N;
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < (size_t)M * quads; e += (size_t)blockDim.x * gridDim.x) {
+    for (size_t e = (size_t)block * blockDim.x + threadIdx.x; e < (size_t)M * quads; e += (size_t)blockDim.x * (gridDim.x - rows.blocks)) {
         const int r = (int)(e / quads), c = (int)(e % quads) * 4;
         const float* p = part + (size_t)r * N + c;
         float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -969,18 +1016,19 @@ static GemmF32Plan gemm_f32_plan(int m, int n, int k, int batch, bool causal, si
     });
 }
 
+static const int g_splitTile[6][2] = {{256, 256}, {256, 192}, {128, 192}, {128, 128}, {64, 128}, {64, 64}};   // of gemm_f32_split_kernel
+
 // gemm_f32_split_kernel.  Microseconds: what the workgroups of the busiest CU take for their stages and ends, and, because the
 // clock follows the load, a share that grows with the workgroups in all.  Fitted by least squares to 700 measurements of 40 sizes
 // in three layouts and up to 16 parts; the tile chosen is within 1 % of the best one on average, 8 % at most.
 static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool causal, size_t wsBytes, double* estimate)
 {
-    static const int tile[6][2] = {{256, 256}, {256, 192}, {128, 192}, {128, 128}, {64, 128}, {64, 64}};
     struct Fit { double stage, ends, loadStage, loadEnds, once; };
     static const struct { int k; Fit alone, shared; } fit[6] = {
         {16, {1.475, 9.5, 0.34, 0, 0}, {1.56, 4.9, 0.64, 0, 0}},      {16, {1.125, 9.55, 0.36, 0, 0}, {1.153, 5.7, 0.55, 0, 0}},
         {16, {0.817, 8.9, 0.156, 0.7, 0}, {0.546, 3.1, 0.39, 0, 0}},  {16, {0.669, 3.64, 0, 5.0, 0}, {0.383, 0.25, 0.286, 0, 2.4}},
         {32, {0.89, 1.3, 0.066, 2.1, 1.1}, {0.457, 0, 0.332, 0, 5.4}}, {32, {0.637, 1.1, 0.056, 1.07, 0}, {0.307, 0, 0.133, 0.38, 3.0}}};
-    return best_plan(m, n, k, batch, causal, wsBytes, 6, tile, estimate, [](int sh, long long items, long long perCu, int chunk) {
+    return best_plan(m, n, k, batch, causal, wsBytes, 6, g_splitTile, estimate, [](int sh, long long items, long long perCu, int chunk) {
         const Fit& f = perCu == 1 ? fit[sh].alone : fit[sh].shared;
         const double nk = (chunk + fit[sh].k - 1) / fit[sh].k, load = items / 256.0;
         return perCu * (nk * f.stage + f.ends) + load * (nk * f.loadStage + f.loadEnds) + f.once;
@@ -1018,12 +1066,29 @@ static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal
     return c;
 }
 
+// 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
+static bool f32_near(bool kFast, int rows, int k, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(k, 128) * ld + 256) < (1ll << 29); }
+
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal)
 {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
     // which kernel takes it depends on the caller too: enough for any
     const int splits = std::max(gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, false).plan.splits, gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, true).plan.splits);
     return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
+}
+
+// With the sums of op(A)'s rows: the partial products (none where the contraction is not cut), then the partial sums.  0: not together,
+// because another kernel takes the product, because a sum would be longer than the column sums' own (128 values in each of eight
+// accumulators and more a row and tile), or because one short launch (up to 1024 k) would only be another.
+static int split_tile_columns(int shape, int n) { return (n + g_splitTile[shape][1] - 1) / g_splitTile[shape][1]; }
+size_t gemm_f32_row_sums_workspace_bytes(int m, int n, int k, bool vec)
+{
+    if (m <= 0 || n <= 0 || k <= 0 || !vec || !f32_near(false, m, k, m) || !f32_near(false, n, k, n)) return 0;
+    const GemmF32Choice c = gemm_f32_choose(m, n, k, 1, false, SIZE_MAX, false);
+    if (c.kernel != F32_SPLIT || (k <= 1024 && c.plan.splits == 1)) return 0;
+    const int columns = split_tile_columns(c.plan.shape, n);
+    if (c.plan.kChunk / (8 * columns) > 128) return 0;
+    return ((c.plan.splits > 1 ? (size_t)c.plan.splits * m * n : 0) + (size_t)c.plan.splits * columns * m) * sizeof(float);
 }
 
 template <int WM, int WN, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
@@ -1058,30 +1123,28 @@ static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const Gem
 // wavefronts of a SIMD that the registers are to hold
 #define SPLIT_SHAPES(X) X(0, 2, 4, 4, 2, 1, 2) X(1, 4, 2, 2, 3, 1, 2) X(2, 2, 2, 2, 3, 1, 2) X(3, 2, 2, 2, 2, 1, 2) X(4, 2, 2, 1, 2, 2, 2) X(5, 2, 2, 1, 1, 2, 2)
 
-template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS>
-static hipError_t launch_split(hipStream_t s, const GemmF32Args& a, int splits, int batch, const HeadsEpilogue* he)
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS>
+static hipError_t launch_split(hipStream_t s, GemmF32Args& g, int splits, int batch, const HeadsEpilogue* he)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN;
-    constexpr int stages = 2 * 3 * (split_plane<BM, KS, AK>() + split_plane<BN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
-    constexpr int lds = stages > store ? stages : store;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    constexpr int lds = 4 * split_lds<WVM, WVN, WM, WN, KS, AK, BKC>() + (SUMS ? 64 * WVM * WVN * 16 : 0);
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
-    GemmF32Args g = a;
     g.tilesM = (g.M + BM - 1) / BM;
     g.tilesN = (g.N + BN - 1) / BN;
     g.parts = splits > 1 ? splits : batch;
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
     const int per = (int)((total + 7) / 8);
-    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
     return hipGetLastError();
 }
 
-template <bool AK, bool BKC, bool VEC, bool HEADS>
-static hipError_t launch_split_shape(hipStream_t s, const GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
+template <bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS = false>
+static hipError_t launch_split_shape(hipStream_t s, GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
 {
     switch (p.shape) {
-#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS>(s, a, p.splits, batch, he);
+#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>(s, a, p.splits, batch, he);
         SPLIT_SHAPES(X)
 #undef X
     }
@@ -1111,15 +1174,12 @@ static hipError_t launch_small(hipStream_t s, const GemmF32Args& a, int batch, c
 
 // VEC: operands in whole aligned 16-byte chunks
 template <bool AK, bool BKC, bool VEC, bool HEADS>
-static hipError_t launch_layout(hipStream_t s, const GemmF32Args& a, const GemmF32Choice& c, int batch, const HeadsEpilogue* he)
+static hipError_t launch_layout(hipStream_t s, GemmF32Args& a, const GemmF32Choice& c, int batch, const HeadsEpilogue* he)
 {
     if (c.kernel == F32_SMALL) return launch_small<4, 64, AK, BKC, VEC, HEADS>(s, a, batch, he);
     if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
     return launch_f32_tile<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
 }
-
-// 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
-static bool f32_near(bool kFast, int rows, int k, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(k, 128) * ld + 256) < (1ll << 29); }
 
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
 {
@@ -1147,20 +1207,27 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, q.fp32Sums || !near, q.heads != nullptr);
     const GemmF32Plan& p = choice.plan;
     a.kChunk = p.kChunk;
+    if (q.rowSum) {
+        const size_t need = gemm_f32_row_sums_workspace_bytes(q.m, q.n, q.k, vec && !q.aK && !q.bK && q.lda == q.m && q.ldb == q.n && q.batch == 1 && !q.fp32Sums);
+        if (need == 0 || wsBytes < need) return hipErrorInvalidValue;
+    }
     // rows shorter than the three values that a chunk may read past one: so many more k
     auto past = [&](bool kFast, int rows, long long ld) { return kFast ? q.k % 4 : rows % 4 == 0 ? 0 : ld >= 3 ? 1 : 3; };
     a.kTail = std::max(past(q.aK, q.m, q.lda), past(q.bK, q.n, q.ldb));
     hipError_t e;
-    if (q.heads) e = vec ? launch_layout<true, true, true, true>(s, a, choice, 1, q.heads) : launch_layout<true, true, false, true>(s, a, choice, 1, q.heads);
+    if (q.rowSum) e = launch_split_shape<false, false, true, false, true>(s, a, p, 1);
+    else if (q.heads) e = vec ? launch_layout<true, true, true, true>(s, a, choice, 1, q.heads) : launch_layout<true, true, false, true>(s, a, choice, 1, q.heads);
 #define LAYOUT(AKV, BKV) (vec ? launch_layout<AKV, BKV, true, false>(s, a, choice, q.batch, nullptr) : launch_layout<AKV, BKV, false, false>(s, a, choice, q.batch, nullptr))
     else if (q.aK) e = q.bK ? LAYOUT(true, true) : LAYOUT(true, false);
     else e = q.bK ? LAYOUT(false, true) : LAYOUT(false, false);
 #undef LAYOUT
-    if (e != hipSuccess || p.splits == 1) return e;
+    F32RowSums rows = {};
+    if (q.rowSum) rows = {(q.m + 255) / 256, p.splits * a.tilesN, a.part + (p.splits > 1 ? (size_t)p.splits * q.m * q.n : 0), q.rowSum};
     const size_t quads = (size_t)q.m * ((q.n + 3) / 4);
-    const int grid = (int)std::min<size_t>((quads + 255) / 256, 4096);
-    if (q.heads) hipLaunchKernelGGL(gemm_f32_sum_kernel<true>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, heads_arg<true>(q.heads));
-    else hipLaunchKernelGGL(gemm_f32_sum_kernel<false>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, HeadsArg<false>());
+    const int grid = rows.blocks + (p.splits > 1 ? (int)std::min<size_t>((quads + 255) / 256, 4096) : 0);
+    if (e != hipSuccess || grid == 0) return e;
+    if (q.heads) hipLaunchKernelGGL(gemm_f32_sum_kernel<true>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, heads_arg<true>(q.heads), rows);
+    else hipLaunchKernelGGL(gemm_f32_sum_kernel<false>, grid, 256, 0, s, (const float*)ws, p.splits, q.m, q.n, q.ldc, q.beta, a.vecC, q.C, a.bias, HeadsArg<false>(), rows);
     return hipGetLastError();
 }
 
@@ -1182,8 +1249,10 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     if (tilesW + tilesX > (1ll << 20)) return hipSuccess;
     // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
     // time that one launch waits for the last one's stores
-    const double apart = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false).time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false).time + 2.5 +
-                         (db ? m <= 1024 ? 4.5 : 9.0 : 0.0);
+    const bool together = db && gemm_f32_row_sums_workspace_bytes(n, k, m, vec) > 0;   // the column sums with the weight gradient
+    const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false);
+    const double apart = dw.time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false).time + 2.5 +
+                         (!db ? 0.0 : together ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
     if (gemm_f32_small_time(tilesW + tilesX, std::max(m, n)) >= apart) return hipSuccess;
     GemmF32Args w = {}, x = {};
     w.M = n; w.N = k; w.K = w.kChunk = m;
