@@ -82,6 +82,11 @@ template <> struct BigTraits<bf16_t> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<bf16x8*>(&a), *reinterpret_cast<bf16x8*>(&b), c, 0, 0, 0);
     }
     __device__ static inline float ld(const bf16_t* p) { return bf16_to_f32(*p); }
+    __device__ static inline float4 ld4(const bf16_t* p)   // aligned
+    {
+        const uint2 w = *(const uint2*)p;
+        return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u));
+    }
     __device__ static inline void st4(bf16_t* p, float a, float b, float c, float d)
     {
         uint2 w;
@@ -101,6 +106,7 @@ template <> struct BigTraits<float> {
         return c;
     }
     __device__ static inline float ld(const float* p) { return *p; }
+    __device__ static inline float4 ld4(const float* p) { return *(const float4*)p; }
     __device__ static inline void st4(float* p, float a, float b, float c, float d) { *(float4*)p = make_float4(a, b, c, d); }
 };
 
