@@ -2,7 +2,6 @@
 //
 //  * gemm_f32.hip, gemm_bf16.hip : the tiled matrix-core kernels behind most products.
 //  * gemm_nt_wide_kernel  : A B^T of sizes that 256 x 288 or (16-bit) 256 x 192 tiles divide, one workgroup per CU.
-//  * gemm_nt_f32out_kernel: fp32 A B^T of 16-bit operands (the Llama engine's prompt pass), with its epilogues.
 //  * gemm_generic         : any transpose / stride combination (column-major strided-batched gemm2, sizes the tiles do not
 //                           take), 64x64x16 LDS tiles, fp32 FMA.
 //  * gemv                 : HBM-bound y = A x, one wavefront per row, 128-bit loads.
@@ -93,312 +92,6 @@ static hipError_t launch_generic(hipStream_t s, int M, int N, int K, float alpha
 static inline bool gemm_is_tiny(int m, int n, int k) { return (long long)m * n <= 1024 && k <= 64; }
 
 // ---------------------------------------------------------------------------
-// MFMA, NT, 16-bit operands with an fp32 result: 2 x 2 wavefronts, each owning WM x WN MFMA 32x32 tiles, so a workgroup
-// covers (64 WM) x (64 WN) of C.  K is walked in stages of 64 through a double-buffered LDS stage (one barrier per stage); a
-// k-step is one 16-byte fragment per lane and operand, one v_mfma_f32_32x32x16_bf16.
-// Tiles are numbered so that each XCD (workgroup index mod 8) works on a contiguous band of tile rows and re-uses its A rows
-// out of its own L2.
-// Epilogues of the prompt pass of the Llama engine (fp32 results of 16-bit operands; llama2_ext.hip), which save the
-// round trip of the product through memory and the kernel that would read it back:
-//   EPI 1, SwiGLU of the stacked W1 | W3 product.  Tile column c multiplies weight row (c & 1) hid + c / 2, so that a
-//     lane's register quad holds (w1 x, w3 x) of two consecutive hidden units j: out[j] = silu(w1 x) (w3 x), stored as
-//     bf16 (rows of hid), or as the bf16 nearest to it followed, hid further on, by the bf16 nearest to the remainder
-//     (rows of 2 hid: the operand form of k_gemm_bf16_f32's split product).
-//   EPI 2, rotation and scatter of the stacked Wq | Wk | Wv product (row = sequence b, position p): q and k rotated at p
-//     (adjacent pairs, the decode kernel's arithmetic), q / k / v written as (B, H, P, hs) head tensors - fp32 or bf16,
-//     every key / value head repeated for the query heads that share it - and the rotated key and the value appended to
-//     the caches [b][p][kvd] (fp32 or bf16; the head tensors then carry the values the cache holds).
-struct PromptEpilogue {
-    void* out; int hid; int split;                                   // EPI 1
-    void* q; void* k; void* v; void* kc; void* vc;                   // EPI 2
-    const float* fcos; const float* fsin;
-    int P, H, kvH, hs, seqLen, heads16, cache16, kvMul;
-    float invP, invHs;
-};
-__device__ __forceinline__ uint32_t pe_pack(float a, float b) { return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16); }
-__device__ __forceinline__ float pe_round(float a) { return bf16_to_f32(f32_to_bf16(a)); }
-// four consecutive values to a tensor of fp32 or bf16
-__device__ __forceinline__ void pe_store4(void* base, size_t idx, int is16, const float (&v)[4])
-{
-    if (is16) *(uint2*)((bf16_t*)base + idx) = make_uint2(pe_pack(v[0], v[1]), pe_pack(v[2], v[3]));
-    else *(float4*)((float*)base + idx) = make_float4(v[0], v[1], v[2], v[3]);
-}
-__device__ __forceinline__ void prompt_epilogue_swiglu(const PromptEpilogue& pe, int r, int c, const float (&a)[4])
-{
-    const int j = c >> 1;   // c is a multiple of 4: hidden units j, j + 1
-    float o[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) o[q] = a[2 * q] * (1.0f / (1.0f + expf(-a[2 * q]))) * a[2 * q + 1];
-    bf16_t* row = (bf16_t*)pe.out + (size_t)r * (pe.split ? 2 : 1) * pe.hid;
-    *(uint32_t*)(row + j) = pe_pack(o[0], o[1]);
-    if (pe.split) *(uint32_t*)(row + pe.hid + j) = pe_pack(o[0] - pe_round(o[0]), o[1] - pe_round(o[1]));
-}
-// x / d for 0 <= x < 2^24, d > 0, through the reciprocal (an integer division is some forty instructions)
-__device__ __forceinline__ int pe_div(int x, int d, float inv)
-{
-    int q = (int)((float)x * inv);
-    if ((q + 1) * d <= x) q++;
-    if (q * d > x) q--;
-    return q;
-}
-__device__ __forceinline__ void prompt_epilogue_rope(const PromptEpilogue& pe, int r, int c, const float (&a)[4])
-{
-    const int dim = pe.H * pe.hs, kvd = pe.kvH * pe.hs, kvMul = pe.kvMul, half = pe.hs >> 1;
-    const int b = pe_div(r, pe.P, pe.invP), p = r - b * pe.P;
-    float o[4] = {a[0], a[1], a[2], a[3]};
-    const int which = c < dim ? 0 : c < dim + kvd ? 1 : 2;
-    const int cc = which == 0 ? c : which == 1 ? c - dim : c - dim - kvd;
-    const int h = pe_div(cc, pe.hs, pe.invHs), d = cc - h * pe.hs;
-    if (which < 2) {
-        const float2 cs = *(const float2*)(pe.fcos + (size_t)p * half + (d >> 1)), sn = *(const float2*)(pe.fsin + (size_t)p * half + (d >> 1));
-        o[0] = a[0] * cs.x - a[1] * sn.x; o[1] = a[0] * sn.x + a[1] * cs.x;
-        o[2] = a[2] * cs.y - a[3] * sn.y; o[3] = a[2] * sn.y + a[3] * cs.y;
-    }
-    if (which == 0) {
-        pe_store4(pe.q, (((size_t)b * pe.H + h) * pe.P + p) * pe.hs + d, pe.heads16, o);
-        return;
-    }
-    if (pe.cache16) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) o[q] = pe_round(o[q]);   // the pass attends over the values the cache holds
-    }
-    pe_store4(which == 1 ? pe.kc : pe.vc, ((size_t)b * pe.seqLen + p) * kvd + cc, pe.cache16, o);
-    for (int g = 0; g < kvMul; g++)
-        pe_store4(which == 1 ? pe.k : pe.v, (((size_t)b * pe.H + h * kvMul + g) * pe.P + p) * pe.hs + d, pe.heads16, o);
-}
-
-// SPLIT: a row of A is 2 K long, the upper halves of K fp32 values followed by what the upper halves leave over (see
-// k_gemm_bf16_split), and B is walked twice: C = alpha (A_hi + A_lo) B^T + beta C.
-template <int WM, int WN, int OCC, bool SPLIT, int EPI>
-__global__ __launch_bounds__(256, OCC) void gemm_nt_f32out_kernel(int M, int N, int K, float alpha, const bf16_t* __restrict__ A,
-                                                                  const bf16_t* __restrict__ B, float beta, float* __restrict__ C, int tilesN,
-                                                                  int tilesTotal, int bandRows, int colBlock, PromptEpilogue pe)
-{
-    typedef bf16_t T;
-    typedef BigTraits<T> TR;
-    constexpr int E = TR::E;
-    constexpr int BK = 8 * E;                                 // elements per stage and row (128 bytes)
-    constexpr int BM = 64 * WM, BN = 64 * WN, LDK = BK + E;   // row stride 16 B past a power of two: conflict-free 128-bit reads
-    constexpr int CPR = 8;                                    // 16-byte chunks per tile row
-    constexpr int RPP = 256 / CPR;                            // rows covered by one pass of the 256 threads
-    constexpr int PA = BM / RPP, PB = BN / RPP;               // passes (16-byte chunks per thread) per operand
-    constexpr int KS = 4;                                     // k-steps (fragments of 2 E elements) per stage
-    constexpr int NMF = WM * WN;                              // tile products per k-step
-    // Memory instructions ride along with the tile products (below): RF fragment reads and SC staging instructions per
-    // product.  One of each where a k-step has at least as many products as fragments (every tile of 128 x 128 and up);
-    // two with the 64-row tiles, whose wavefronts own one or two MFMA tiles.
-    constexpr int RF = (WM + WN + NMF - 1) / NMF;
-    constexpr int SC = ((PA + PB + KS / 2 - 1) / (KS / 2) + NMF - 1) / NMF;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    T* smem = reinterpret_cast<T*>(smem_raw);
-    T* As = smem;                        // [2][BM * LDK]
-    T* Bs = smem + 2 * BM * LDK;         // [2][BN * LDK]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int per = (tilesTotal + 7) / 8;
-    int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-    if (colBlock > 0) {
-        // The XCD's band of bandRows tile rows is walked in blocks of colBlock tile columns, so that the tiles in
-        // flight on the XCD at one time share few enough A and B rows for its L2 to hold them.
-        const int i = (int)(blockIdx.x / 8), nb = (tilesN + colBlock - 1) / colBlock;
-        const int blk = min(i / (bandRows * colBlock), nb - 1);
-        const int rem = i - blk * bandRows * colBlock;
-        const int width = blk == nb - 1 ? tilesN - blk * colBlock : colBlock;
-        tile = ((int)(blockIdx.x % 8) * bandRows + rem / width) * tilesN + blk * colBlock + rem % width;
-    }
-    if (tile >= tilesTotal) return;
-    const int m0 = (tile / tilesN) * BM, n0 = (tile % tilesN) * BN;
-    const int wm = (wave >> 1) * (32 * WM), wn = (wave & 1) * (32 * WN);
-    const int lr = tid / CPR, lc = (tid % CPR) * E;
-
-    floatx16 acc[WM][WN];
-#pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-        for (int j = 0; j < WN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-
-    // rows past the matrix edge are clamped: they are loaded (valid memory) and never stored
-    const T* ga[PA];
-    const T* gb[PB];
-#pragma unroll
-    for (int p = 0; p < PA; p++) ga[p] = A + (size_t)min(m0 + lr + p * RPP, M - 1) * (SPLIT ? 2 * K : K) + lc;
-#pragma unroll
-    for (int p = 0; p < PB; p++) {
-        const int c = min(n0 + lr + p * RPP, N - 1);
-        gb[p] = B + (size_t)(EPI == 1 ? (c & 1) * pe.hid + (c >> 1) : c) * K + lc;
-    }
-    T* sa = As + lr * LDK + lc;
-    T* sb = Bs + lr * LDK + lc;
-    u32x4 ra[PA], rb[PB];
-
-    const int nkB = K / BK, nk = SPLIT ? 2 * nkB : nkB;   // stage kt of A goes with stage kt % nkB of B
-    // stage 0 -> LDS buffer 0, stage 1 -> registers
-#pragma unroll
-    for (int p = 0; p < PA; p++) ra[p] = *(const u32x4*)(ga[p]);
-#pragma unroll
-    for (int p = 0; p < PB; p++) rb[p] = *(const u32x4*)(gb[p]);
-#pragma unroll
-    for (int p = 0; p < PA; p++) *(u32x4*)(sa + p * RPP * LDK) = ra[p];
-#pragma unroll
-    for (int p = 0; p < PB; p++) *(u32x4*)(sb + p * RPP * LDK) = rb[p];
-    {
-        const int s1 = min(1, nk - 1), k1 = s1 * BK, k1b = (SPLIT ? s1 % nkB : s1) * BK;
-#pragma unroll
-        for (int p = 0; p < PA; p++) ra[p] = *(const u32x4*)(ga[p] + k1);
-#pragma unroll
-        for (int p = 0; p < PB; p++) rb[p] = *(const u32x4*)(gb[p] + k1b);
-    }
-    __syncthreads();
-    const int fr = lane & 31, fg = (lane >> 5) * E;
-    const T* fa = As + (wm + fr) * LDK + fg;
-    const T* fb = Bs + (wn + fr) * LDK + fg;
-    u32x4 a[2][WM], b[2][WN];
-    // One stage: KS k-steps of NMF tile products on LDS buffer kt & 1.  Riding along between them (the wavefront
-    // is alone on its SIMD, so whatever it issues between two MFMAs is hidden behind the first one's passes, and
-    // whatever it issues in a block of its own is not):
-    //   first half of the k-steps : the registers holding stage kt + 1 go to the other LDS buffer
-    //   second half               : stage kt + 2 is fetched from global memory into those registers
-    //   every k-step but the last : the fragments of the next k-step are read from LDS
-    // Past the end of K the extra fetches re-read the last stage (valid memory, never consumed).
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        const T* pa = fa + buf * BM * LDK;
-        const T* pb = fb + buf * BN * LDK;
-        T* wa = sa + (buf ^ 1) * BM * LDK;
-        T* wb = sb + (buf ^ 1) * BN * LDK;
-        const int s2 = min(kt + 2, nk - 1), k2 = s2 * BK, k2b = (SPLIT ? (s2 >= nkB ? s2 - nkB : s2) : s2) * BK;
-#pragma unroll
-        for (int t = 0; t < WM; t++) a[0][t] = *(const u32x4*)(pa + t * 32 * LDK);
-#pragma unroll
-        for (int t = 0; t < WN; t++) b[0][t] = *(const u32x4*)(pb + t * 32 * LDK);
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const int cur = ks & 1, nxt = cur ^ 1;
-            // this k-step's share of the staging traffic: chunks [c0, c1) of the PA + PB chunks per thread
-            constexpr int HALF = KS / 2;
-            const int part = ks % HALF;
-            const int c0 = (PA + PB) * part / HALF, c1 = (PA + PB) * (part + 1) / HALF;
-            // written in issue order, one small scheduling region per tile product so that the order stays as
-            // written: product q, then the q-th fragment read of the next k-step, then the q-th staging instruction
-#pragma unroll
-            for (int q = 0; q < NMF; q++) {
-                const int i = q / WN, j = q % WN;
-                acc[i][j] = TR::mma(b[cur][j], a[cur][i], acc[i][j]);
-                if (ks + 1 < KS) {
-#pragma unroll
-                    for (int r = q * RF; r < (q + 1) * RF; r++) {
-                        if (r < WM) a[nxt][r] = *(const u32x4*)(pa + r * 32 * LDK + (ks + 1) * 2 * E);
-                        else if (r < WM + WN) b[nxt][r - WM] = *(const u32x4*)(pb + (r - WM) * 32 * LDK + (ks + 1) * 2 * E);
-                    }
-                }
-#pragma unroll
-                for (int c = c0 + q * SC; c < c0 + (q + 1) * SC; c++) {
-                    if (c >= c1) break;
-                    if (ks < HALF) {
-                        if (c < PA) *(u32x4*)(wa + c * RPP * LDK) = ra[c];
-                        else *(u32x4*)(wb + (c - PA) * RPP * LDK) = rb[c - PA];
-                    } else {
-                        if (c < PA) ra[c] = *(const u32x4*)(ga[c] + k2);
-                        else rb[c - PA] = *(const u32x4*)(gb[c - PA] + k2b);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-    }
-    // The tile products above are the TRANSPOSED 32x32 tiles (B fragment as the row operand), so a lane owns one
-    // row of C (lane%32) and register v is column 8*(v/4) + 4*(lane/32) + v%4: four consecutive columns per
-    // register quad.
-    const int row_l = lane & 31, col_l = (lane >> 5) * 4;
-    // fp32 results of 16-bit operands.  A lane owns a row of the tile, so its own stores would be 16 bytes each in 32
-    // different rows; each wavefront passes its tile, 32 rows at a time, through its own slice of LDS (free after
-    // the last barrier) and the lanes then walk the rows: consecutive lanes take consecutive quads of columns, and
-    // whatever the epilogue stores is contiguous along the row.
-    constexpr int CW = 32 * WN, LDC = CW + 4;
-    constexpr int LPR = CW / 4, RPI = 64 / LPR;             // lanes per row, rows per pass
-    constexpr int NIT = (32 + RPI - 1) / RPI;
-    float* cs = reinterpret_cast<float*>(smem_raw) + wave * 32 * LDC;
-    const int rr = lane / LPR, cc = (lane % LPR) * 4;
-    const bool vec4 = (N & 3) == 0 && (((uintptr_t)C) & 15) == 0;
-#pragma unroll
-    for (int i = 0; i < WM; i++) {
-#pragma unroll
-        for (int j = 0; j < WN; j++)
-#pragma unroll
-            for (int g = 0; g < 4; g++)
-                *(float4*)(cs + row_l * LDC + j * 32 + 8 * g + col_l) =
-                    make_float4(alpha * acc[i][j][4 * g], alpha * acc[i][j][4 * g + 1], alpha * acc[i][j][4 * g + 2], alpha * acc[i][j][4 * g + 3]);
-        // same wavefront wrote and reads: LDS operations of one wavefront complete in order
-#pragma unroll 4
-        for (int it = 0; it < NIT; it++) {
-            const int row = it * RPI + rr, r = m0 + wm + i * 32 + row, c = n0 + wn + cc;
-            if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
-            const float4 v = *(const float4*)(cs + row * LDC + cc);
-            if (EPI != 0) {
-                // N is a multiple of 4 here: a quad is inside the matrix or outside it
-                const float a4[4] = {v.x, v.y, v.z, v.w};
-                if (EPI == 1) prompt_epilogue_swiglu(pe, r, c, a4);
-                else prompt_epilogue_rope(pe, r, c, a4);
-                continue;
-            }
-            float* cp = C + (size_t)r * N + c;
-            if (vec4 && c + 3 < N) {
-                float4 o = v;
-                if (beta != 0.f) {
-                    const float4 old = *(const float4*)cp;
-                    o.x += beta * old.x; o.y += beta * old.y; o.z += beta * old.z; o.w += beta * old.w;
-                }
-                *(float4*)cp = o;
-            } else {
-                const float a4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (c + q < N) cp[q] = a4[q] + (beta != 0.f ? beta * cp[q] : 0.f);
-            }
-        }
-    }
-}
-
-template <int WM, int WN, int OCC, bool SPLIT, int EPI>
-static hipError_t launch_f32out(hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* B, float beta, float* C,
-                                const PromptEpilogue* prompt)
-{
-    typedef bf16_t T;
-    PromptEpilogue pe = {};
-    if (prompt) pe = *prompt;
-    constexpr int E = BigTraits<T>::E;
-    const int tm = (m + 64 * WM - 1) / (64 * WM), tn = (n + 64 * WN - 1) / (64 * WN);
-    const long long total = (long long)tm * tn;
-    if (total > (1ll << 30)) return hipErrorInvalidValue;
-    const int per = (int)((total + 7) / 8);
-    size_t lds = (size_t)2 * (64 * WM + 64 * WN) * (9 * E) * sizeof(T);
-    const size_t ldsEpilogue = (size_t)4 * 32 * (32 * WN + 4) * sizeof(float);
-    if (ldsEpilogue > lds) lds = ldsEpilogue;
-    static bool attr = false;   // per instantiation: allow more than the default 64 KB of dynamic LDS
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_nt_f32out_kernel<WM, WN, OCC, SPLIT, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    // Bands of whole tile rows per XCD (tm divisible by 8): pick the column block so that the rows of A and B behind
-    // one block of tiles stay under 3 MB of the XCD's 4 MB L2; 0 keeps the plain row-major walk of the band.
-    int bandRows = 0, colBlock = 0;
-    if (tm % 8 == 0 && tn > 1) {
-        bandRows = tm / 8;
-        const double rowBytes = 64.0 * WM * k * sizeof(T), colBytes = 64.0 * WN * k * sizeof(T), budget = 3.0 * 1024 * 1024;
-        const int fit = (int)((budget - bandRows * rowBytes) / colBytes);
-        if (fit >= 1 && fit < tn) {
-            const int nb = (tn + fit - 1) / fit;
-            colBlock = (tn + nb - 1) / nb;   // equal-width blocks
-        }
-    }
-    hipLaunchKernelGGL((gemm_nt_f32out_kernel<WM, WN, OCC, SPLIT, EPI>), dim3(per * 8), 256, lds, s, m, n, k, alpha, (const T*)A, (const T*)B, beta,
-                       C, tn, (int)total, bandRows, colBlock, pe);
-    return hipGetLastError();
-}
-
 // ---------------------------------------------------------------------------
 // NT, one 256 x 288 (WN = 9) or 256 x 192 (WN = 6) tile per workgroup and one workgroup per CU: 8192 x 2304 (the fused
 // QKV projection of a 768-wide layer over 8192 tokens) is exactly 256 tiles of 256 x 288, one round of the chip, and a
@@ -788,60 +481,6 @@ hipError_t k_gemm_bias_heads_group(hipStream_t s, int count, int n, int k, int H
     hipError_t e = hipSuccess;
     *done = gemm_b16_group(s, q, count, &e);
     return e;
-}
-
-// C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
-// split = false: A is X rounded to bf16, m rows of k.  split = true keeps the activations' precision: A holds every row of
-// an fp32 X as two bf16 rows back to back, the bf16 nearest to each of its k values and then the bf16 nearest to what
-// those leave over, and the kernel walks W once for each.  The products are exact and accumulate in fp32, so what is lost
-// is the part of X below its leading sixteen bits: 2^-17 relative, against 2^-9 for activations rounded to bf16.
-// k a multiple of 64, 16-byte aligned operands.
-template <bool SPLIT, int EPI>
-static hipError_t gemm_bf16_f32_tiles(hipStream_t s, int m, int n, int k, float alpha, const void* A, const void* W, float beta, float* C,
-                                      const PromptEpilogue* pe)
-{
-    // Tile shapes as k_gemm picks them for bf16: below 200 tiles of 128 x 128, 64 x 128 tiles where they give every CU
-    // one, else 64 x 64 (2048 x 768: 384 tiles of 64 x 64 measure 27.8 us a product, 192 of 64 x 128 30.1 us).
-    const long long t128 = (long long)((m + 127) / 128) * ((n + 127) / 128);
-    if (t128 < 200) {
-        const long long t64x128 = (long long)((m + 63) / 64) * ((n + 127) / 128);
-        if (t64x128 >= 200) return launch_f32out<1, 2, 3, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
-        return launch_f32out<1, 1, 3, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
-    }
-    if (n % 192 == 0 && t128 <= 512) return launch_f32out<2, 3, 2, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
-    return launch_f32out<2, 2, 2, SPLIT, EPI>(s, m, n, k, alpha, A, W, beta, C, pe);
-}
-static bool bf16_f32_operands_ok(int k, const void* A, const void* W) { return k > 0 && k % 64 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0; }
-hipError_t k_gemm_bf16_f32(hipStream_t s, int m, int n, int k, float alpha, const void* A, bool split, const void* W, float beta, float* C)
-{
-    if (m <= 0 || n <= 0) return hipSuccess;
-    if (!bf16_f32_operands_ok(k, A, W)) return hipErrorInvalidValue;
-    return split ? gemm_bf16_f32_tiles<true, 0>(s, m, n, k, alpha, A, W, beta, C, nullptr) : gemm_bf16_f32_tiles<false, 0>(s, m, n, k, alpha, A, W, beta, C, nullptr);
-}
-// out (m x hid) = silu(X W1^T) (X W3^T) for the stacked 16-bit W13 (2 hid x k), as bf16 rows (outSplit: hi | lo rows)
-hipError_t k_gemm_bf16_swiglu(hipStream_t s, int m, int hid, int k, const void* A, bool split, const void* W13, void* out, bool outSplit)
-{
-    if (m <= 0 || hid <= 0) return hipSuccess;
-    if (!bf16_f32_operands_ok(k, A, W13) || (hid & 1) || (((uintptr_t)out) & 3)) return hipErrorInvalidValue;
-    PromptEpilogue pe = {};
-    pe.out = out; pe.hid = hid; pe.split = outSplit ? 1 : 0;
-    return split ? gemm_bf16_f32_tiles<true, 1>(s, m, 2 * hid, k, 1.f, A, W13, 0.f, nullptr, &pe) : gemm_bf16_f32_tiles<false, 1>(s, m, 2 * hid, k, 1.f, A, W13, 0.f, nullptr, &pe);
-}
-// the stacked 16-bit Wqkv ((H + 2 kvH) hs x k) product of B x P rows, rotated and scattered (PromptEpilogue, EPI 2)
-hipError_t k_gemm_bf16_qkv_rope(hipStream_t s, int B, int P, int H, int kvH, int hs, int k, const void* A, bool split, const void* Wqkv,
-                                void* q, void* kh, void* vh, bool heads16, void* kc, void* vc, bool cache16, int seqLen,
-                                const float* fcos, const float* fsin)
-{
-    const int m = B * P, n = (H + 2 * kvH) * hs;
-    if (m <= 0 || n <= 0) return hipSuccess;
-    if (!bf16_f32_operands_ok(k, A, Wqkv) || (hs & 3) || kvH <= 0 || H % kvH != 0) return hipErrorInvalidValue;
-    if ((((uintptr_t)q | (uintptr_t)kh | (uintptr_t)vh | (uintptr_t)kc | (uintptr_t)vc) & 15) != 0) return hipErrorInvalidValue;
-    PromptEpilogue pe = {};
-    pe.q = q; pe.k = kh; pe.v = vh; pe.kc = kc; pe.vc = vc; pe.fcos = fcos; pe.fsin = fsin;
-    pe.P = P; pe.H = H; pe.kvH = kvH; pe.hs = hs; pe.seqLen = seqLen; pe.heads16 = heads16 ? 1 : 0; pe.cache16 = cache16 ? 1 : 0;
-    pe.kvMul = H / kvH; pe.invP = 1.0f / (float)P; pe.invHs = 1.0f / (float)hs;
-    if (m >= (1 << 24) || n >= (1 << 24)) return hipErrorInvalidValue;
-    return split ? gemm_bf16_f32_tiles<true, 2>(s, m, n, k, 1.f, A, Wqkv, 0.f, nullptr, &pe) : gemm_bf16_f32_tiles<false, 2>(s, m, n, k, 1.f, A, Wqkv, 0.f, nullptr, &pe);
 }
 
 size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k)

@@ -1,8 +1,8 @@
 // 16-bit GEMM on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16), any operand layout, fp32 accumulation, gfx950.
 //
 // WVM x WVN wavefronts of WM x WN MFMA tiles each cover (32 WVM WM) x (32 WVN WN) of C and walk K in stages of 64 that go
-// from global memory straight into LDS (buffer loads to LDS: no staging registers, no writes to issue), double-buffered, one
-// barrier per stage.  At this matrix rate a tile is bound by what it moves: 128 x 128 needs 64 bytes per clock and CU from
+// from global memory straight into LDS (buffer loads to LDS: no staging registers, no writes to issue), two to four of them there,
+// one barrier per stage.  At this matrix rate a tile is bound by what it moves: 128 x 128 needs 64 bytes per clock and CU from
 // L2, all that L2 has; 256 x 256 half of that.  Large products therefore take 256 x 256 or 256 x 192 with eight
 // wavefronts, one workgroup per CU, whichever leaves the shorter last round, small ones the tile that fills the chip.
 //
@@ -96,10 +96,104 @@ __device__ __forceinline__ void b16_store8(const GemmB16Args& g, const HeadsArg<
     }
 }
 
+// Epilogues of the prompt pass of the Llama engine (fp32 results of 16-bit operands; llama2_ext.hip), which save the
+// round trip of the product through memory and the kernel that would read it back:
+//   1, SwiGLU of the stacked W1 | W3 product.  Tile column c multiplies weight row (c & 1) hid + c / 2, so that a
+//     lane's register quad holds (w1 x, w3 x) of two consecutive hidden units j: out[j] = silu(w1 x) (w3 x), stored as
+//     bf16 (rows of hid), or as the bf16 nearest to it followed, hid further on, by the bf16 nearest to the remainder
+//     (rows of 2 hid: the operand form of k_gemm_bf16_f32's split product).
+//   2, rotation and scatter of the stacked Wq | Wk | Wv product (row = sequence b, position p): q and k rotated at p
+//     (adjacent pairs, the decode kernel's arithmetic), q / k / v written as (B, H, P, hs) head tensors - fp32 or bf16,
+//     every key / value head repeated for the query heads that share it - and the rotated key and the value appended to
+//     the caches [b][p][kvd] (fp32 or bf16; the head tensors then carry the values the cache holds).
+struct PromptEpilogue {
+    void* out; int hid; int split;                                   // 1
+    void* q; void* k; void* v; void* kc; void* vc;                   // 2
+    const float* fcos; const float* fsin;
+    int P, H, kvH, hs, seqLen, heads16, cache16, kvMul;
+    float invP, invHs;
+    int kB;                                                          // all: of B, which is walked again from there on (K or K / 2)
+};
+// the argument behind a product's: nothing, the heads epilogue's (1, 2), the prompt pass's (3: none of its epilogues, 4, 5: 1, 2)
+struct PromptArg { PromptEpilogue pe; };
+template <int END> using B16Arg = std::conditional_t<(END >= 3), PromptArg, HeadsArg<(END > 0)>>;
+__device__ __forceinline__ uint32_t pe_pack(float a, float b) { return pack2_bf16(a, b); }
+__device__ __forceinline__ float pe_round(float a) { return bf16_to_f32(f32_to_bf16(a)); }
+// four consecutive values to a tensor of fp32 or bf16
+__device__ __forceinline__ void pe_store4(void* base, size_t idx, int is16, const float (&v)[4])
+{
+    if (is16) *(uint2*)((bf16_t*)base + idx) = make_uint2(pe_pack(v[0], v[1]), pe_pack(v[2], v[3]));
+    else *(float4*)((float*)base + idx) = make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void prompt_epilogue_swiglu(const PromptEpilogue& pe, int r, int c, const float (&a)[4])
+{
+    const int j = c >> 1;   // c is a multiple of 4: hidden units j, j + 1
+    float o[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) o[q] = a[2 * q] * (1.0f / (1.0f + expf(-a[2 * q]))) * a[2 * q + 1];
+    bf16_t* row = (bf16_t*)pe.out + (size_t)r * (pe.split ? 2 : 1) * pe.hid;
+    *(uint32_t*)(row + j) = pe_pack(o[0], o[1]);
+    if (pe.split) *(uint32_t*)(row + pe.hid + j) = pe_pack(o[0] - pe_round(o[0]), o[1] - pe_round(o[1]));
+}
+// x / d for 0 <= x < 2^24, d > 0, through the reciprocal (an integer division is some forty instructions)
+__device__ __forceinline__ int pe_div(int x, int d, float inv)
+{
+    int q = (int)((float)x * inv);
+    if ((q + 1) * d <= x) q++;
+    if (q * d > x) q--;
+    return q;
+}
+__device__ __forceinline__ void prompt_epilogue_rope(const PromptEpilogue& pe, int r, int c, const float (&a)[4])
+{
+    const int dim = pe.H * pe.hs, kvd = pe.kvH * pe.hs, kvMul = pe.kvMul, half = pe.hs >> 1;
+    const int b = pe_div(r, pe.P, pe.invP), p = r - b * pe.P;
+    float o[4] = {a[0], a[1], a[2], a[3]};
+    const int which = c < dim ? 0 : c < dim + kvd ? 1 : 2;
+    const int cc = which == 0 ? c : which == 1 ? c - dim : c - dim - kvd;
+    const int h = pe_div(cc, pe.hs, pe.invHs), d = cc - h * pe.hs;
+    if (which < 2) {
+        const float2 cs = *(const float2*)(pe.fcos + (size_t)p * half + (d >> 1)), sn = *(const float2*)(pe.fsin + (size_t)p * half + (d >> 1));
+        o[0] = a[0] * cs.x - a[1] * sn.x; o[1] = a[0] * sn.x + a[1] * cs.x;
+        o[2] = a[2] * cs.y - a[3] * sn.y; o[3] = a[2] * sn.y + a[3] * cs.y;
+    }
+    if (which == 0) {
+        pe_store4(pe.q, (((size_t)b * pe.H + h) * pe.P + p) * pe.hs + d, pe.heads16, o);
+        return;
+    }
+    if (pe.cache16) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) o[q] = pe_round(o[q]);   // the pass attends over the values the cache holds
+    }
+    pe_store4(which == 1 ? pe.kc : pe.vc, ((size_t)b * pe.seqLen + p) * kvd + cc, pe.cache16, o);
+    for (int g = 0; g < kvMul; g++)
+        pe_store4(which == 1 ? pe.k : pe.v, (((size_t)b * pe.H + h * kvMul + g) * pe.P + p) * pe.hs + d, pe.heads16, o);
+}
+
+// eight values of row r from column c on to an fp32 matrix, beta C added
+__device__ __forceinline__ void prompt_store8(const GemmB16Args& g, int r, int c, const float (&v)[8])
+{
+    float* cp = (float*)g.C + (size_t)r * g.N + c;
+#pragma unroll
+    for (int q = 0; q < 8; q += 4) {
+        if (g.vecC && c + q < g.N) {
+            float4 o = make_float4(v[q], v[q + 1], v[q + 2], v[q + 3]);
+            if (g.beta != 0.f) {
+                const float4 old = *(const float4*)(cp + q);
+                o.x += g.beta * old.x; o.y += g.beta * old.y; o.z += g.beta * old.z; o.w += g.beta * old.w;
+            }
+            *(float4*)(cp + q) = o;
+        } else {
+#pragma unroll
+            for (int e = q; e < q + 4; e++)
+                if (c + e < g.N) cp[e] = v[e] + (g.beta != 0.f ? g.beta * cp[e] : 0.f);
+        }
+    }
+}
+
 // tile `item` of a product.  SUMS: the tiles of a row of tiles also add up the rows of op(A), each the stages that are its turn, from
 // the fragments it multiplies: the bias gradient beside a weight gradient (8000 x 3072, 6.2 to 12.8 us and a launch of 5 on their own).
-template <int WVM, int WVN, int WM, int WN, bool AK, bool BKC, int HEADS, bool SUMS = false>
-__device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(HEADS > 0)>& hp, int item)
+template <int WVM, int WVN, int WM, int WN, int S, bool AK, bool BKC, int HEADS, bool SUMS = false>
+__device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEADS>& hp, int item)
 {
     constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64, KS = 4;
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;               // 16-byte chunks per thread and stage
@@ -108,6 +202,7 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
     static_assert(PA * NT == BM * 8 && PB * NT == BN * 8, "whole chunks per thread");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     bf16_t* smem = reinterpret_cast<bf16_t*>(smem_raw);
+    constexpr bool ENDS_IN_HEADS = HEADS == 1 || HEADS == 2, PROMPT = HEADS >= 3;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles = g.tilesM * g.tilesN;
     const int part = item / tiles, tile = item - part * tiles;
@@ -139,6 +234,15 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
         if (BKC) vb[p] = ((uint32_t)min(e / 8, N - 1 - n0) * (uint32_t)g.ldb + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
         else vb[p] = ((uint32_t)(e / (BN / 8)) * (uint32_t)g.ldb + min(((e % (BN / 8)) ^ block_swizzle<BN * 2>(e / (BN / 8))) * 8, N - 8 - n0)) * 2;
     }
+    // a prompt product's B by its addresses: pairs of rows of a stacked matrix lie far apart
+    [[maybe_unused]] const bf16_t* pb64[PB];
+    if constexpr (PROMPT) {
+#pragma unroll
+        for (int p = 0; p < PB; p++) {
+            const int e = p * NT + tid, c = min(n0 + e / 8, N - 1);
+            pb64[p] = g.B + (size_t)(HEADS == 4 ? (c & 1) * hp.pe.hid + (c >> 1) : c) * g.ldb + ((e & 7) ^ ((e >> 4) & 7)) * 8;
+        }
+    }
     auto resource = [](const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(OUTSIDE - 16), 0x00020000); };
     const __amdgpu_buffer_rsrc_t rsA = resource(baseA), rsB = resource(baseB);
     // where resources begin at stages: the stage that is fetched next, and the way to the one after it (0 from the last on).
@@ -149,7 +253,7 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
         if (!AK) stageA += stepA;
         if (!BKC) stageB += stepB;
     };
-    // before the last stage is fetched, once: the chunks past the end of the contraction
+    // before a stage is fetched that ends the contraction or lies past it: the chunks past the end
     auto lastStage = [&](int k0) {
         asm volatile("" ::: "memory");   // a branch, not a select in every stage
         stepA = stepB = 0;
@@ -172,7 +276,8 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
             else lds_fetch<16>(resource(stageA), to, va[p], 0);
         } else {
             bf16_t* to = stage + BM * BK + ((p - PA) * NT + wave * 64) * 8;
-            if (BKC) lds_fetch<16>(rsB, to, vb[p - PA], k0 * 2);
+            if constexpr (PROMPT) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(pb64[p - PA] + (k0 >= hp.pe.kB ? k0 - hp.pe.kB : k0)), LDS3(to), 16, 0, 0);
+            else if (BKC) lds_fetch<16>(rsB, to, vb[p - PA], k0 * 2);
             else lds_fetch<16>(resource(stageB), to, vb[p - PA], 0);
         }
     };
@@ -208,12 +313,26 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
         else tr_read<BN * 2>(stageAddr + tb[t], ks * 16 * (BN * 2), o);
     };
 
+    // S stages in LDS: one is read, the S - 1 after it are fetched
     const int nk = (kEnd - kBegin + BK - 1) / BK;
-    if (nk == 1) lastStage(kBegin);
 #pragma unroll
-    for (int p = 0; p < PA + PB; p++) fetch(p, kBegin, smem);
-    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the fetches have landed in LDS
-    __syncthreads();
+    for (int u = 0; u < S - 1; u++) {
+        if (u > 0) advance();
+        if (u + 1 >= nk) lastStage(kBegin + u * BK);
+#pragma unroll
+        for (int p = 0; p < PA + PB; p++) fetch(p, PROMPT ? kBegin + min(u, nk - 1) * BK : kBegin + u * BK, smem + u * STAGE);
+        asm volatile("" ::: "memory");
+    }
+    // the oldest of S - 1 stages under way has landed, of this wavefront and then of all
+    auto landed = [&]() {
+        if constexpr (S == 2) {
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+            __syncthreads();
+        } else {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S - 2) * (PA + PB)) : "memory");
+        }
+    };
+    landed();
     const uint32_t smemAddr = (uint32_t)(uintptr_t)LDS3(smem);
     TrFragment a[2][WM], b[2][WN];
     [[maybe_unused]] float sums[WM][8];
@@ -224,14 +343,16 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
 #pragma unroll
             for (int e = 0; e < 8; e++) sums[t][e] = 0.f;
     }
+    int slot = 0;
     for (int kt = 0; kt < nk; kt++) {
-        const bf16_t* pa = smem + (kt & 1) * STAGE;
+        const bf16_t* pa = smem + slot * STAGE;
         const bf16_t* pb = pa + BM * BK;
-        bf16_t* next = smem + ((kt & 1) ^ 1) * STAGE;   // read during stage kt - 1; free since the barrier that ended it
-        const int k1 = kBegin + min(kt + 1, nk - 1) * BK;   // past the end the last stage is fetched again, never read
+        bf16_t* next = smem + (slot == 0 ? S - 1 : slot - 1) * STAGE;   // read during stage kt - 1; free since the barrier that ended it
+        // past the end two stages fetch the last one again, never read, and more of them nothing
+        const int k1 = kBegin + (S == 2 || PROMPT ? min(kt + S - 1, nk - 1) : kt + S - 1) * BK;
         advance();
-        if (kt + 2 == nk) lastStage(k1);
-        const uint32_t stageAddr = smemAddr + (kt & 1) * STAGE * 2;
+        if (S == 2 ? kt + 2 == nk : kt + S >= nk) lastStage(k1);
+        const uint32_t stageAddr = smemAddr + slot * STAGE * 2;
 #pragma unroll
         for (int t = 0; t < WM; t++) fragA(pa, stageAddr, t, 0, a[0][t]);
 #pragma unroll
@@ -279,6 +400,10 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
             }
         }
         if constexpr (SUMS) turn = turn == 0 ? g.tilesN - 1 : turn - 1;
+        slot = slot == S - 1 ? 0 : slot + 1;
+        landed();
+    }
+    if constexpr (S > 2) {   // what was fetched past the end
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
     }
@@ -314,26 +439,36 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
             const int c = n0 + wn + c0 * 32 + cc;
             float bias[8];
             bf16_t* col = nullptr;
-            if (!split && c < N) {
+            if (!PROMPT && !split && c < N) {
                 b16_bias8(g, c, bias);
-                if constexpr (HEADS) col = heads_col<bf16_t>(hp.he, c);
+                if constexpr (ENDS_IN_HEADS) col = heads_col<bf16_t>(hp.he, c);
             }
             // the rows' places: added up, not divided out for each
             size_t nextAt = 0;
             int t = 0;
-            if constexpr (HEADS) nextAt = heads_row(hp.he, m0 + wm + i * 32 + rr, t);
+            if constexpr (ENDS_IN_HEADS) nextAt = heads_row(hp.he, m0 + wm + i * 32 + rr, t);
 #pragma unroll 2
             for (int it = 0; it < NIT; it++) {
                 const int row = it * RPI + rr, r = m0 + wm + i * 32 + row;
                 const size_t rowAt = nextAt;
-                if constexpr (HEADS) {
+                if constexpr (ENDS_IN_HEADS) {
                     nextAt += (size_t)(RPI * hp.he.hs);
                     for (t += RPI; t >= hp.he.T; t -= hp.he.T) nextAt += hp.he.perBatch - (unsigned long long)(uint32_t)hp.he.T * (uint32_t)hp.he.hs;
                 }
                 if (rr >= RPI || row >= 32 || r >= M || c >= N) continue;
                 const float4 t0 = *(const float4*)(cs + row * LDC + cc), t1 = *(const float4*)(cs + row * LDC + cc + 4);
                 float v[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
-                if (split) {
+                if constexpr (PROMPT) {
+                    const float lo[4] = {v[0], v[1], v[2], v[3]}, hi[4] = {v[4], v[5], v[6], v[7]};   // of a multiple of four columns
+                    if constexpr (HEADS == 3) prompt_store8(g, r, c, v);
+                    else if constexpr (HEADS == 4) {
+                        prompt_epilogue_swiglu(hp.pe, r, c, lo);
+                        if (c + 4 < N) prompt_epilogue_swiglu(hp.pe, r, c + 4, hi);
+                    } else {
+                        prompt_epilogue_rope(hp.pe, r, c, lo);
+                        if (c + 4 < N) prompt_epilogue_rope(hp.pe, r, c + 4, hi);
+                    }
+                } else if (split) {
                     float* cp = g.part + ((size_t)part * M + r) * N + c;
                     if (g.vecC) {
                         *(float4*)cp = t0;
@@ -344,7 +479,7 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
                             if (c + q < N) cp[q] = v[q];
                     }
                 } else {
-                    b16_store8<HEADS>(g, hp, r, c, bias, col, rowAt, v);
+                    if constexpr (!PROMPT) b16_store8<HEADS>(g, hp, r, c, bias, col, rowAt, v);
                 }
             }
         }
@@ -353,24 +488,24 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const HeadsArg<(H
 // each XCD (workgroup index mod 8) takes a contiguous run of the tiles
 __device__ __forceinline__ int b16_xcd_item(int total) { return (int)(blockIdx.x % 8) * ((total + 7) / 8) + (int)(blockIdx.x / 8); }
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
-__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, HeadsArg<(HEADS > 0)> hp)
+template <int WVM, int WVN, int WM, int WN, int S, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
+__global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_kernel(GemmB16Args g, B16Arg<HEADS> hp)
 {
     const int total = g.tilesM * g.tilesN * g.parts, item = b16_xcd_item(total);
     if (item >= total) return;
-    b16_tile<WVM, WVN, WM, WN, AK, BKC, HEADS, SUMS>(g, hp, item);
+    b16_tile<WVM, WVN, WM, WN, S, AK, BKC, HEADS, SUMS>(g, hp, item);
 }
 
 // Up to three products with heads epilogues as one launch: the projections of a multi-head attention layer.  One by one each is less
 // than two rounds of the chip with its own first fetches and last stores (4096 and twice 8192 rows, 512 to 512: 9.4 + 12.3 + 11.9 us, as one launch 21.6).
 struct GemmB16Group { GemmB16Args g[3]; HeadsArg<true> h[3]; int first[4]; };   // first: of the tiles of all, of each; then their number
-template <int WVM, int WVN, int WM, int WN, int OCC>
+template <int WVM, int WVN, int WM, int WN, int S, int OCC>
 __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_b16_group_kernel(GemmB16Group grp)
 {
     const int item = b16_xcd_item(grp.first[3]);
     if (item >= grp.first[3]) return;
     const int p = item >= grp.first[2] ? 2 : item >= grp.first[1] ? 1 : 0;
-    b16_tile<WVM, WVN, WM, WN, true, true, 1>(grp.g[p], grp.h[p], item - grp.first[p]);
+    b16_tile<WVM, WVN, WM, WN, S, true, true, 1>(grp.g[p], grp.h[p], item - grp.first[p]);
 }
 
 // ---------------------------------------------------------------------------
@@ -540,39 +675,42 @@ __global__ __launch_bounds__(256) void gemm_b16_sum_kernel(GemmB16Args g, HeadsA
 // ---------------------------------------------------------------------------
 // How a product is cut: the tile and the number of parts of the contraction with the smallest estimated time.
 struct GemmB16Plan { int shape, splits, kChunk; };
-// microseconds of one tile per 768 k and for its ends (first fetches, and stores that all CUs issue at once), with two and
-// more workgroups on the CU and alone on it.  Fitted to all six shapes, in 1 to 8 parts, at 32 sizes (M 512 .. 8192, N 384 ..
-// 3072, K 512 .. 8192, the three layouts): over those the shape taken is 0.5 % slower than the fastest on average and 12 % at
-// worst.  A 128 x 192 tile alone on its CU is dealt to eight wavefronts, two per SIMD, because with four nothing covers the wait
-// at the end of a stage (8192 x 768 x 768, 256 tiles: 14.8 us against 15.7 with four and 16.4 in 64 x 128 tiles); with two
-// such tiles on a CU four wavefronts each are better (8192 x 2304 x 768: 36.3 us against 42.9).
-struct GemmB16Shape { int bm, bn; double perK, ends, perKAlone, endsAlone; };
-static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 15.0, 7.5}, {256, 192, 10.0, 10.5, 10.0, 10.5}, {128, 192, 6.8, 4.4, 10.3, 4.5},
-                                           {128, 128, 4.2, 3.5, 7.0, 4.2}, {64, 128, 3.7, 1.3, 6.0, 1.5}, {64, 64, 2.5, 0.9, 4.1, 0.9}};
-enum { B16_128X192 = 2, B16_128X192_ALONE = 6 };
+// The tiles: 256 x 256 and 256 x 192 for large products; the others with as many stages in LDS as leave room for the workgroups that
+// share a CU.  With two stages a small tile waits for every one of them (2048 x 768 x 4096 in 64 x 64 tiles: 33.8 us; 128 x 64 on eight
+// wavefronts with four stages 19.9; 1024^3 10.3, 6.7; 8192 x 768 x 768 in 128 x 192 on eight wavefronts 14.7, with three 13.0).
+// Wavefronts, MFMA tiles of one, stages, workgroups a CU is to hold:
+#define B16_SHAPES(X) X(0, 4, 2, 2, 4, 2, 2) X(1, 4, 2, 2, 3, 2, 2) X(2, 2, 2, 2, 3, 2, 2) X(3, 4, 2, 1, 3, 3, 2) X(4, 2, 2, 2, 2, 2, 2) \
+                      X(5, 2, 2, 2, 2, 3, 1) X(6, 2, 2, 1, 2, 3, 2) X(7, 4, 2, 1, 1, 4, 2) X(8, 2, 2, 1, 1, 4, 2)
+// Microseconds of one tile per 768 k and for its ends, with two and more on the CU (and once besides) and alone on it.  Fitted to 56 sizes
+// (M 64 .. 8192, N 256 .. 4096, K 256 .. 4096) in three layouts, the shared ones of the large tiles to 32 larger sizes: the shape taken
+// is 1 % slower than the fastest on average and 17 % at worst.
+struct GemmB16Shape { int bm, bn; double perK, ends, once, perKAlone, endsAlone; };
+static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 0, 13.1, 6.5},    {256, 192, 10.0, 10.5, 0, 11.3, 5.7},    {128, 192, 6.8, 4.4, 0, 9.0, 4.5},
+                                           {128, 192, 9.1, 4.0, 1.0, 6.37, 4.75}, {128, 128, 4.2, 3.5, 1.0, 7.7, 3.0}, {128, 128, 4.79, 3.38, 2.5, 4.62, 4.75},
+                                           {64, 128, 3.21, 0.89, 2.7, 3.67, 3.31},  {128, 64, 3.30, 2.14, 1.8, 3.21, 3.25}, {64, 64, 2.25, 0.67, 2.6, 2.69, 2.93}};
+static constexpr int B16_NSHAPES = sizeof(g_b16Shapes) / sizeof(g_b16Shapes[0]);
 
 static double b16_time(const GemmB16Shape& s, long long tiles, int k)
 {
     const double len = ((k + 63) / 64 * 64) / 768.0;
     const long long perCu = ((tiles + 7) / 8 + 31) / 32;
-    return perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends);
+    return perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends) + s.once;
 }
 
 static GemmB16Plan gemm_b16_plan(int m, int n, int k)
 {
-    GemmB16Plan best = {5, 1, k};
+    GemmB16Plan best = {0, 1, k};
     double bestT = 1e30;
-    for (int sh = 0; sh < 6; sh++) {
+    for (int sh = 0; sh < B16_NSHAPES; sh++) {
         const GemmB16Shape& s = g_b16Shapes[sh];
         const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn);
         for (int S = 1; S <= 16; S++) {
             if (S > 1 && k / S < 256) break;
             const int chunk = ((k + S - 1) / S + 63) / 64 * 64;
             if ((k + chunk - 1) / chunk != S) continue;
-            const long long perCu = ((tiles * S + 7) / 8 + 31) / 32;
             double t = b16_time(s, tiles * S, chunk);
             if (S > 1) t += 4.0 + (double)(S + 1) * m * n * 4.0 / 4.0e6;
-            if (t < bestT) { bestT = t; best = {sh == B16_128X192 && perCu == 1 ? B16_128X192_ALONE : sh, S, S > 1 ? chunk : k}; }
+            if (t < bestT) { bestT = t; best = {sh, S, S > 1 ? chunk : k}; }
         }
     }
     return best;
@@ -596,7 +734,7 @@ size_t gemm_b16_workspace_bytes(int m, int n, int k)
     const GemmB16Plan p = gemm_b16_plan(m, n, k);
     return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
 }
-static int b16_tile_columns(int shape, int n) { const int bn = g_b16Shapes[shape == B16_128X192_ALONE ? B16_128X192 : shape].bn; return (n + bn - 1) / bn; }
+static int b16_tile_columns(int shape, int n) { return (n + g_b16Shapes[shape].bn - 1) / g_b16Shapes[shape].bn; }
 // With the sums of op(A)'s rows: the partial products (none where the contraction is not cut), then the partial sums.  0: not together.
 // A partial sum is one of sixteen accumulators per row and tile: up to 128 values each they are no longer than the column sums' own.
 size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k)
@@ -608,32 +746,29 @@ size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k)
     return gemm_b16_workspace_bytes(m, n, k) + (size_t)p.splits * columns * m * sizeof(float);
 }
 
-template <int WVM, int WVN, int WM, int WN, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
-static hipError_t launch_b16(hipStream_t s, GemmB16Args& g, const HeadsEpilogue* he)
+template <int WVM, int WVN, int WM, int WN, int S, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
+static hipError_t launch_b16(hipStream_t s, GemmB16Args& g, const B16Arg<HEADS>& end)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN, CH = WN % 2 == 0 ? 2 : WN;
-    constexpr int stages = 2 * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    constexpr int stages = S * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_kernel<WVM, WVN, WM, WN, S, OCC, AK, BKC, HEADS, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     g.tilesM = (g.M + BM - 1) / BM;
     g.tilesN = (g.N + BN - 1) / BN;
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, OCC, AK, BKC, HEADS, SUMS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, heads_arg<(HEADS > 0)>(he));
+    hipLaunchKernelGGL((gemm_b16_kernel<WVM, WVN, WM, WN, S, OCC, AK, BKC, HEADS, SUMS>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, g, end);
     return hipGetLastError();
 }
 template <bool AK, bool BKC, int HEADS, bool SUMS = false>
-static hipError_t launch_b16_shape(hipStream_t s, GemmB16Args& a, int shape, const HeadsEpilogue* he = nullptr)
+static hipError_t launch_b16_shape(hipStream_t s, GemmB16Args& a, int shape, const B16Arg<HEADS>& end = B16Arg<HEADS>{})
 {
     switch (shape) {
-    case 0: return launch_b16<4, 2, 2, 4, 2, AK, BKC, HEADS, SUMS>(s, a, he);
-    case 1: return launch_b16<4, 2, 2, 3, 2, AK, BKC, HEADS, SUMS>(s, a, he);
-    case B16_128X192: return launch_b16<2, 2, 2, 3, 2, AK, BKC, HEADS, SUMS>(s, a, he);
-    case B16_128X192_ALONE: return launch_b16<4, 2, 1, 3, 2, AK, BKC, HEADS, SUMS>(s, a, he);
-    case 3: return launch_b16<2, 2, 2, 2, 2, AK, BKC, HEADS, SUMS>(s, a, he);
-    case 4: return launch_b16<2, 2, 1, 2, 3, AK, BKC, HEADS, SUMS>(s, a, he);
-    default: return launch_b16<2, 2, 1, 1, 4, AK, BKC, HEADS, SUMS>(s, a, he);
+#define X(I, WVM, WVN, WM, WN, S, OCC) case I: return launch_b16<WVM, WVN, WM, WN, S, OCC, AK, BKC, HEADS, SUMS>(s, a, end);
+        B16_SHAPES(X)
+#undef X
     }
+    return hipErrorInvalidValue;
 }
 
 static GemmB16Args b16_args(const GemmB16& q)
@@ -714,8 +849,8 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
     a.parts = p.splits; a.kChunk = p.kChunk;
     a.part = (float*)ws;
     hipError_t e;
-    if (q.heads && q.heads->fcos) e = launch_b16_shape<true, true, 2>(s, a, p.shape, q.heads);
-    else if (q.heads) e = launch_b16_shape<true, true, 1>(s, a, p.shape, q.heads);
+    if (q.heads && q.heads->fcos) e = launch_b16_shape<true, true, 2>(s, a, p.shape, heads_arg<true>(q.heads));
+    else if (q.heads) e = launch_b16_shape<true, true, 1>(s, a, p.shape, heads_arg<true>(q.heads));
     else if (q.rowSum) e = launch_b16_shape<false, false, 0, true>(s, a, p.shape);
     else if (q.aK) e = q.bK ? launch_b16_shape<true, true, 0>(s, a, p.shape) : launch_b16_shape<true, false, 0>(s, a, p.shape);
     else e = q.bK ? launch_b16_shape<false, true, 0>(s, a, p.shape) : launch_b16_shape<false, false, 0>(s, a, p.shape);
@@ -727,12 +862,12 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
     return hipGetLastError();
 }
 
-template <int WVM, int WVN, int WM, int WN, int OCC>
+template <int WVM, int WVN, int WM, int WN, int S, int OCC>
 static hipError_t launch_b16_group(hipStream_t s, GemmB16Group& grp, int count)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN, CH = WN % 2 == 0 ? 2 : WN;
-    constexpr int stages = 2 * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_group_kernel<WVM, WVN, WM, WN, OCC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    constexpr int stages = S * (BM + BN) * 64 * 2, slices = WVM * WVN * 32 * (32 * CH + 4) * 4, lds = stages > slices ? stages : slices;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_b16_group_kernel<WVM, WVN, WM, WN, S, OCC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     long long total = 0;
     for (int p = 0; p < 3; p++) {
@@ -746,42 +881,102 @@ static hipError_t launch_b16_group(hipStream_t s, GemmB16Group& grp, int count)
     }
     grp.first[3] = (int)total;
     for (int p = count; p < 3; p++) grp.first[p] = (int)total;
-    hipLaunchKernelGGL((gemm_b16_group_kernel<WVM, WVN, WM, WN, OCC>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, grp);
+    hipLaunchKernelGGL((gemm_b16_group_kernel<WVM, WVN, WM, WN, S, OCC>), dim3((unsigned)((total + 7) / 8 * 8)), 64 * WVM * WVN, lds, s, grp);
     return hipGetLastError();
 }
 
 // `count` (2 or 3) products A B^T through their heads epilogues, all of one n and k, as one launch.  False: a product is none that
-// gemm_b16 takes, or they are too few rows to fill a CU each (gemm_b16 may cut those in parts).
+// gemm_b16 takes, or one that gemm_b16_rows_kernel may take.
 bool gemm_b16_group(hipStream_t s, const GemmB16* q, int count, hipError_t* e)
 {
     GemmB16Group grp = {};
     for (int p = 0; p < count; p++) {
-        if (!gemm_b16_takes(q[p]) || !q[p].heads || !q[p].aK || !q[p].bK || q[p].n != q[0].n || q[p].k != q[0].k) return false;
+        if (!gemm_b16_takes(q[p]) || !q[p].heads || !q[p].aK || !q[p].bK || q[p].n != q[0].n || q[p].k != q[0].k || q[p].m <= 32) return false;
         grp.g[p] = b16_args(q[p]);
         grp.h[p].he = *q[p].heads;
     }
     int best = 0;
     double bestT = 1e30;
-    long long small = 0;
-    for (int sh = 0; sh < 6; sh++) {
+    for (int sh = 0; sh < B16_NSHAPES; sh++) {
         const GemmB16Shape& c = g_b16Shapes[sh];
         long long tiles = 0;
         for (int p = 0; p < count; p++) tiles += (long long)((q[p].m + c.bm - 1) / c.bm) * ((q[p].n + c.bn - 1) / c.bn);
         const double t = b16_time(c, tiles, q[0].k);
-        if (t < bestT) { bestT = t; best = sh == B16_128X192 && tiles <= 256 ? B16_128X192_ALONE : sh; }
-        small = tiles;
+        if (t < bestT) { bestT = t; best = sh; }
     }
-    if (small < 256) return false;
     switch (best) {
-    case 0: *e = launch_b16_group<4, 2, 2, 4, 2>(s, grp, count); break;
-    case 1: *e = launch_b16_group<4, 2, 2, 3, 2>(s, grp, count); break;
-    case B16_128X192: *e = launch_b16_group<2, 2, 2, 3, 2>(s, grp, count); break;
-    case B16_128X192_ALONE: *e = launch_b16_group<4, 2, 1, 3, 2>(s, grp, count); break;
-    case 3: *e = launch_b16_group<2, 2, 2, 2, 2>(s, grp, count); break;
-    case 4: *e = launch_b16_group<2, 2, 1, 2, 3>(s, grp, count); break;
-    default: *e = launch_b16_group<2, 2, 1, 1, 4>(s, grp, count); break;
+#define X(I, WVM, WVN, WM, WN, S, OCC) case I: *e = launch_b16_group<WVM, WVN, WM, WN, S, OCC>(s, grp, count); break;
+        B16_SHAPES(X)
+#undef X
     }
     return true;
+}
+
+// ---------------------------------------------------------------------------
+// C (m x n, fp32) = alpha X W^T + beta C for a 16-bit weight matrix W (n x k), on the bf16 matrix cores, C in fp32.
+// split = false: A is X rounded to bf16, m rows of k.  split = true keeps the activations' precision: A holds every row of
+// an fp32 X as two bf16 rows back to back, the bf16 nearest to each of its k values and then the bf16 nearest to what
+// those leave over, and the kernel walks W once for each.  The products are exact and accumulate in fp32, so what is lost
+// is the part of X below its leading sixteen bits: 2^-17 relative, against 2^-9 for activations rounded to bf16.
+// k a multiple of 64, 16-byte aligned operands.
+// The tile with the smallest estimate for the whole contraction; a row of A that is split is 2 k long, and B is walked twice.  us at 2048
+// rows of 768, split, before (a kernel that staged through registers) and now: with the rotation, to 2304 columns, 40.6, 30.9; with
+// SwiGLU, to 4096, 40.5, 35.5; to 768, and from 2048 to 768, 26.9, 21.9 on average; to 32000 254, 249.
+template <int END>
+static hipError_t gemm_b16_prompt(hipStream_t s, int m, int n, int k, float alpha, const void* A, bool split, const void* W, float beta, float* C,
+                                  const PromptEpilogue* pe)
+{
+    GemmB16Args a = {};
+    a.M = m; a.N = n; a.K = a.kChunk = split ? 2 * k : k;
+    a.A = (const bf16_t*)A; a.B = (const bf16_t*)W; a.C = (bf16_t*)C;
+    a.lda = a.K; a.ldb = k;
+    a.alpha = alpha; a.beta = beta;
+    a.parts = 1;
+    a.vecC = n % 4 == 0 && ((uintptr_t)C & 15) == 0;
+    PromptArg end = {};
+    if (pe) end.pe = *pe;
+    end.pe.kB = k;
+    int best = 0;
+    double bestT = 1e30;
+    for (int sh = 0; sh < B16_NSHAPES; sh++) {
+        const GemmB16Shape& c = g_b16Shapes[sh];
+        const long long tiles = (long long)((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+        const double t = b16_time(c, tiles, a.K);
+        if (t < bestT) { bestT = t; best = sh; }
+    }
+    return launch_b16_shape<true, true, END>(s, a, best, end);
+}
+static bool bf16_f32_operands_ok(int k, const void* A, const void* W) { return k > 0 && k % 64 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0; }
+hipError_t k_gemm_bf16_f32(hipStream_t s, int m, int n, int k, float alpha, const void* A, bool split, const void* W, float beta, float* C)
+{
+    if (m <= 0 || n <= 0) return hipSuccess;
+    if (!bf16_f32_operands_ok(k, A, W)) return hipErrorInvalidValue;
+    return gemm_b16_prompt<3>(s, m, n, k, alpha, A, split, W, beta, C, nullptr);
+}
+// out (m x hid) = silu(X W1^T) (X W3^T) for the stacked 16-bit W13 (2 hid x k), as bf16 rows (outSplit: hi | lo rows)
+hipError_t k_gemm_bf16_swiglu(hipStream_t s, int m, int hid, int k, const void* A, bool split, const void* W13, void* out, bool outSplit)
+{
+    if (m <= 0 || hid <= 0) return hipSuccess;
+    if (!bf16_f32_operands_ok(k, A, W13) || (hid & 1) || (((uintptr_t)out) & 3)) return hipErrorInvalidValue;
+    PromptEpilogue pe = {};
+    pe.out = out; pe.hid = hid; pe.split = outSplit ? 1 : 0;
+    return gemm_b16_prompt<4>(s, m, 2 * hid, k, 1.f, A, split, W13, 0.f, nullptr, &pe);
+}
+// the stacked 16-bit Wqkv ((H + 2 kvH) hs x k) product of B x P rows, rotated and scattered (PromptEpilogue, 2)
+hipError_t k_gemm_bf16_qkv_rope(hipStream_t s, int B, int P, int H, int kvH, int hs, int k, const void* A, bool split, const void* Wqkv,
+                                void* q, void* kh, void* vh, bool heads16, void* kc, void* vc, bool cache16, int seqLen,
+                                const float* fcos, const float* fsin)
+{
+    const int m = B * P, n = (H + 2 * kvH) * hs;
+    if (m <= 0 || n <= 0) return hipSuccess;
+    if (!bf16_f32_operands_ok(k, A, Wqkv) || (hs & 3) || kvH <= 0 || H % kvH != 0) return hipErrorInvalidValue;
+    if ((((uintptr_t)q | (uintptr_t)kh | (uintptr_t)vh | (uintptr_t)kc | (uintptr_t)vc) & 15) != 0) return hipErrorInvalidValue;
+    PromptEpilogue pe = {};
+    pe.q = q; pe.k = kh; pe.v = vh; pe.kc = kc; pe.vc = vc; pe.fcos = fcos; pe.fsin = fsin;
+    pe.P = P; pe.H = H; pe.kvH = kvH; pe.hs = hs; pe.seqLen = seqLen; pe.heads16 = heads16 ? 1 : 0; pe.cache16 = cache16 ? 1 : 0;
+    pe.kvMul = H / kvH; pe.invP = 1.0f / (float)P; pe.invHs = 1.0f / (float)hs;
+    if (m >= (1 << 24) || n >= (1 << 24)) return hipErrorInvalidValue;
+    return gemm_b16_prompt<5>(s, m, n, k, 1.f, A, split, Wqkv, 0.f, nullptr, &pe);
 }
 
 }  // namespace mch

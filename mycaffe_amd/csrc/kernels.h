@@ -152,7 +152,7 @@ size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, c
 // split, every row of X as two bf16 rows (nearest bf16, then the bf16 nearest to the remainder; m x 2k)
 hipError_t k_gemm_bf16_f32(hipStream_t s, int m, int n, int k, float alpha, const void* A, bool split, const void* W, float beta, float* C);
 // the same product with the epilogues of the Llama prompt pass: SwiGLU of the stacked W1 | W3 (bf16 rows of hid, or hi | lo
-// rows of 2 hid), and rotation + scatter of the stacked Wq | Wk | Wv into head tensors and caches (gemm.hip, PromptEpilogue)
+// rows of 2 hid), and rotation + scatter of the stacked Wq | Wk | Wv into head tensors and caches (gemm_bf16.hip, PromptEpilogue)
 hipError_t k_gemm_bf16_swiglu(hipStream_t s, int m, int hid, int k, const void* A, bool split, const void* W13, void* out, bool outSplit);
 hipError_t k_gemm_bf16_qkv_rope(hipStream_t s, int B, int P, int H, int kvH, int hs, int k, const void* A, bool split, const void* Wqkv,
                                 void* q, void* kh, void* vh, bool heads16, void* kc, void* vc, bool cache16, int seqLen,
