@@ -680,14 +680,17 @@ struct GemmB16Plan { int shape, splits, kChunk; };
 // wavefronts with four stages 19.9; 1024^3 10.3, 6.7; 8192 x 768 x 768 in 128 x 192 on eight wavefronts 14.7, with three 13.0).
 // Wavefronts, MFMA tiles of one, stages, workgroups a CU is to hold:
 #define B16_SHAPES(X) X(0, 4, 2, 2, 4, 2, 2) X(1, 4, 2, 2, 3, 2, 2) X(2, 2, 2, 2, 3, 2, 2) X(3, 4, 2, 1, 3, 3, 2) X(4, 2, 2, 2, 2, 2, 2) \
-                      X(5, 2, 2, 2, 2, 3, 1) X(6, 2, 2, 1, 2, 3, 2) X(7, 4, 2, 1, 1, 4, 2) X(8, 2, 2, 1, 1, 4, 2)
-// Microseconds of one tile per 768 k and for its ends, with two and more on the CU (and once besides) and alone on it.  Fitted to 56 sizes
-// (M 64 .. 8192, N 256 .. 4096, K 256 .. 4096) in three layouts, the shared ones of the large tiles to 32 larger sizes: the shape taken
-// is 1 % slower than the fastest on average and 17 % at worst.
+                      X(5, 2, 2, 2, 2, 3, 1) X(6, 2, 2, 1, 2, 3, 2) X(7, 4, 2, 1, 1, 4, 2) X(8, 2, 2, 1, 1, 4, 2) X(9, 2, 2, 1, 2, 2, 3)
+// Microseconds of one tile per 768 k and for its ends, with two and more on the CU (and once besides) and alone on it.  Fitted to 250
+// sizes (M 64 .. 32000, N 256 .. 32000, K 256 .. 8192) in three layouts with up to eight parts, 60 launches in a row: the choice is
+// 0.4 % slower than the fastest on average and 10 % at worst.  (64 x 128 with two stages has short contractions with two or three tiles
+// on a CU, 8192 x 512 x 512 7.9 us against 8.5 in 128 x 128 with three.)
 struct GemmB16Shape { int bm, bn; double perK, ends, once, perKAlone, endsAlone; };
-static const GemmB16Shape g_b16Shapes[] = {{256, 256, 17.0, 5.0, 0, 13.1, 6.5},    {256, 192, 10.0, 10.5, 0, 11.3, 5.7},    {128, 192, 6.8, 4.4, 0, 9.0, 4.5},
-                                           {128, 192, 9.1, 4.0, 1.0, 6.37, 4.75}, {128, 128, 4.2, 3.5, 1.0, 7.7, 3.0}, {128, 128, 4.79, 3.38, 2.5, 4.62, 4.75},
-                                           {64, 128, 3.21, 0.89, 2.7, 3.67, 3.31},  {128, 64, 3.30, 2.14, 1.8, 3.21, 3.25}, {64, 64, 2.25, 0.67, 2.6, 2.69, 2.93}};
+static const GemmB16Shape g_b16Shapes[] = {{256, 256, 12.56, 9.20, 0, 12.64, 9.12},  {256, 192, 14.34, 5.68, 0.29, 10.62, 8.68},
+                                           {128, 192, 5.33, 4.68, 0.29, 9.01, 5.00}, {128, 192, 6.54, 4.85, 0.12, 6.94, 6.06},
+                                           {128, 128, 4.01, 2.78, 0.77, 7.00, 3.85}, {128, 128, 4.73, 3.27, 1.60, 4.79, 5.71},
+                                           {64, 128, 2.78, 1.05, 2.42, 3.74, 4.62},  {128, 64, 3.24, 1.71, 2.90, 3.50, 3.60},
+                                           {64, 64, 2.03, 0.47, 3.25, 2.21, 3.31},   {64, 128, 2.99, 0.69, 2.72, 6.12, 3.18}};
 static constexpr int B16_NSHAPES = sizeof(g_b16Shapes) / sizeof(g_b16Shapes[0]);
 
 static double b16_time(const GemmB16Shape& s, long long tiles, int k)
@@ -709,7 +712,7 @@ static GemmB16Plan gemm_b16_plan(int m, int n, int k)
             const int chunk = ((k + S - 1) / S + 63) / 64 * 64;
             if ((k + chunk - 1) / chunk != S) continue;
             double t = b16_time(s, tiles * S, chunk);
-            if (S > 1) t += 4.0 + (double)(S + 1) * m * n * 4.0 / 4.0e6;
+            if (S > 1) t += 2.0 + (double)(S + 1) * m * n * 4.0 / 3.4e6;
             if (t < bestT) { bestT = t; best = {sh, S, S > 1 ? chunk : k}; }
         }
     }
