@@ -36,7 +36,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
-MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "f32": 157.3}
+MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "f32": 157.3}   # fp32 products as three bf16 parts per value may pass the latter (bound: 2500 / 6)
 
 C4 = dict(dim=768, hidden_dim=2048, n_layers=12, n_heads=12, n_kv_heads=12, vocab_size=32000, seq_len=1024)
 N_PROMPT = 128
@@ -397,7 +397,7 @@ def bench_decode_attention(cuda, reps, warm=5, cases=None):
     if "bf16_B32_L4096" not in out:
         return out
     best = out["bf16_B32_L4096"]
-    out["roofline"] = {"kernel": "rope_append_kernel + attn_decode_kernel (bf16, batch 32, L 4096, 32 x 128)", "bound": "hbm", "achieved": best["GBps"],
+    out["roofline"] = {"kernel": "attn_decode_kernel with the rotation and the append (bf16, batch 32, L 4096, 32 x 128)", "bound": "hbm", "achieved": best["GBps"],
                        "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": best["frac_hbm"],
                        "traffic": recorded_traffic("attn_decode_bf16_B32_L4096")}
     return out
