@@ -406,14 +406,15 @@ long Kernel::mem(long h, MemItem** it)
     return 0;
 }
 
-// Whether a product's alpha takes a factor of an operand.  A power of two changes no bit; any other spares every element of the operand
-// a rounding, and the result has one for it.  Between 2^-24 and 2^24, so that no sum comes near an end of the range that the
-// scaled operand's would not (the score gradient of 32 heads of 32, 932 positions: a pass of 39 us).
+// Whether a product's alpha takes a factor of an operand: a power of two, of which every sum is the same number times that power, so that
+// no bit changes as long as neither that sum nor a partial one leaves the range.  2^-8 to 2^8 (the scale of head sizes up to 65536): with a
+// larger factor outside of the sums too much of the range is lost to them (1e35 scaled by 2^-20 and multiplied by 1e4).  Any other factor
+// changes the sums themselves and is applied before the product (taking 32^-1/2 into alpha spared 32 heads of 32, 932 positions,
+// a pass of 39 us, and turned finite results above 2^128 times it into infinities).
 static inline bool goes_into_alpha(float f)
 {
     int e;
-    if (!(f > 0.f) || !std::isfinite(f)) return false;
-    return frexpf(f, &e) == 0.5f ? e > -100 && e < 100 : e > -24 && e < 24;
+    return f > 0.f && std::isfinite(f) && frexpf(f, &e) == 0.5f && e >= -7 && e <= 9;
 }
 
 long Kernel::mem_factor(long h, MemItem** it, float* fold)
@@ -877,7 +878,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (m < 0 || n < 0 || k < 0 || batch < 1 || lda < 1 || ldb < 1 || ldc < 1 || sA < 0 || sB < 0 || sC < 0)
             return MCH_ERROR_PARAM_OUT_OF_RANGE;
         MemItem *A, *B, *C;
-        float fold = 1.f;   // deferred scalings of the operands (MatMulGrad scales a gradient, then multiplies by it twice)
+        float fold = 1.f;   // deferred power-of-two scalings of the operands (MatMulGrad scales a gradient, then multiplies by it twice)
         if (timing || (long)pl[9] == (long)pl[6] || (long)pl[9] == (long)pl[7]) {
             ERRCHK(mem((long)pl[6], &A));
             ERRCHK(mem((long)pl[7], &B));

@@ -180,7 +180,8 @@ private:
     long tickets(size_t count, int** p);
     long mem(long h, MemItem** it);                                            // with any deferred scaling applied
     long mem_lazy(long h, MemItem** it);                                       // as it is; the caller deals with `pending`
-    // an operand of a product: a deferred scaling that the product's alpha takes (goes_into_alpha) stays deferred and goes into *fold
+    // an operand of a product: a deferred scaling by a power of two that the product's alpha takes (goes_into_alpha) stays
+    // deferred and goes into *fold
     long mem_factor(long h, MemItem** it, float* fold);
     // the target of a call that writes all `count` elements without reading any: what was held back for it is dropped
     long mem_overwritten(long h, MemItem** it, long long count);
