@@ -370,24 +370,26 @@ static GemmB16 b16_product(bool tA, bool tB, int m, int n, int k, float alpha, c
 {
     return GemmB16{m, n, k, (const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, !tA, tB, alpha, beta, nullptr, nullptr, nullptr};
 }
-// X (m x kk) W^T (n x kk) through the tile kernels' HEADS epilogue `he`; in 16-bit storage, operands the tile kernels do not
+// X (m x kk) W^T (n x kk) through the tile kernels' HEADS epilogue `he`, or to Y; in 16-bit storage, operands the tile kernels do not
 // take go through a scratch matrix (m x n) and a splitting pass
-static size_t gemm_heads_workspace_bytes(DType dt, int m, int n, int kk, const void* X, const void* W)
+static size_t gemm_heads_workspace_bytes(DType dt, int m, int n, int kk, const void* X, const void* W, const HeadsEpilogue& he, const void* Y)
 {
     if (dt == F32) return gemm_f32_workspace_bytes(m, n, kk, 1, false);
-    return gemm_b16_takes(b16_product(false, true, m, n, kk, 1.f, X, W, 0.f, nullptr)) ? gemm_b16_workspace_bytes(m, n, kk) : (size_t)m * n * sizeof(bf16_t);
+    GemmB16 g = b16_product(false, true, m, n, kk, 1.f, X, W, 0.f, (void*)Y);
+    if (!Y) g.heads = &he;
+    return gemm_b16_takes(g) ? gemm_b16_workspace_bytes(g) : (size_t)m * n * sizeof(bf16_t);
 }
 bool k_gemm_bias_needs_workspace(DType dt, int m, int n, int k, const void* X, const void* W)
 {
     return dt != F32 && !gemm_b16_takes(b16_product(false, true, m, n, k, 1.f, X, W, 0.f, nullptr));
 }
-size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W)
+size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W, const void* Y, bool heads)
 {
-    return gemm_heads_workspace_bytes(dt, m, n, k, X, W);
+    return gemm_heads_workspace_bytes(dt, m, n, k, X, W, heads_epilogue(nullptr, (void*)Y, nullptr, nullptr, m, 1, n, nullptr, nullptr, 1), heads ? nullptr : Y);
 }
-size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W)
+size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* q, const void* k, const void* v)
 {
-    return gemm_heads_workspace_bytes(dt, B * T, 3 * H * hs, H * hs, X, W);
+    return gemm_heads_workspace_bytes(dt, B * T, 3 * H * hs, H * hs, X, W, heads_epilogue(nullptr, (void*)q, (void*)k, (void*)v, T, H, hs, nullptr, nullptr, 1), nullptr);
 }
 
 // Y: row-major result, only the bias of `he` is added; null: through `he`
@@ -395,10 +397,6 @@ static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int
                                       void* ws, size_t wsBytes, bool fp32Sums)
 {
     if (dt == F32) {
-        hipError_t fit;
-        if (fp32Sums && (Y ? launch_wide_f32_if_fits<false>(&fit, s, m, n, kk, 1.f, X, W, Y, &he)
-                           : he.hs % 4 == 0 && (((uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0 &&
-                                 launch_wide_f32_if_fits<true>(&fit, s, m, n, kk, 1.f, X, W, he.dst[0], &he))) return fit;
         GemmF32 g = {};
         g.m = m; g.n = n; g.k = kk;
         g.A = (const float*)X; g.B = (const float*)W;
@@ -409,6 +407,10 @@ static hipError_t gemm_heads_dispatch(hipStream_t s, DType dt, int m, int n, int
         if (Y) g.bias = (const float*)he.bias;
         else g.heads = &he;
         g.fp32Sums = fp32Sums;
+        hipError_t fit;
+        if ((fp32Sums || gemm_f32_shares(g)) && (Y ? launch_wide_f32_if_fits<false>(&fit, s, m, n, kk, 1.f, X, W, Y, &he)
+                                                   : he.hs % 4 == 0 && (((uintptr_t)he.dst[1] | (uintptr_t)he.dst[2]) & 15) == 0 &&
+                                                         launch_wide_f32_if_fits<true>(&fit, s, m, n, kk, 1.f, X, W, he.dst[0], &he))) return fit;
         return gemm_f32(s, g, ws, wsBytes);
     }
     hipError_t fit;
@@ -483,11 +485,12 @@ hipError_t k_gemm_bias_heads_group(hipStream_t s, int count, int n, int k, int H
     return e;
 }
 
-size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k)
+size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k, const void* A, const void* B, const void* C)
 {
     if (m <= 0 || n <= 0 || k <= 1) return 0;
     if (dt == F32) return gemm_is_tiny(m, n, k) ? 0 : gemm_f32_workspace_bytes(m, n, k, 1, false);
-    return gemm_b16_takes(b16_product(tA, tB, m, n, k, 1.f, nullptr, nullptr, 0.f, nullptr)) ? gemm_b16_workspace_bytes(m, n, k) : 0;
+    const GemmB16 g = b16_product(tA, tB, m, n, k, 1.f, A, B, 0.f, (void*)C);
+    return gemm_b16_takes(g) ? gemm_b16_workspace_bytes(g) : 0;
 }
 
 hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k, float alpha, const void* A,
@@ -501,6 +504,8 @@ hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k
         g.aK = !tA; g.bK = tB;
         g.lda = tA ? m : k; g.ldb = tB ? k : n; g.ldc = n;
         g.alpha = alpha; g.beta = beta; g.batch = 1;
+        hipError_t e;
+        if (!tA && tB && beta == 0.f && gemm_f32_shares(g) && launch_wide_f32_if_fits<false>(&e, s, m, n, k, alpha, A, B, C)) return e;
         return gemm_f32(s, g, ws, wsBytes);
     }
     if (dt == BF16 && k > 1) {
@@ -953,12 +958,13 @@ template <typename T> static void bias_grad(hipStream_t s, DType dt, int m, int 
 // Weight and bias gradient as one pass over dY (16-bit storage, 8000 rows, 768 to 3072: 69.5 us one after the other, 55.9 together;
 // 3072 to 768: 62.5, 56.8; 2048 rows, 512 to 512: 18.0, 11.7; fp32, 8000 rows,
 // 768 to 3072: 210, 193).  A bias that
-// shares memory with another operand is left to the calls one after the other.
+// shares memory with another operand, or a weight gradient that does, is left to the calls one after the other.
 size_t k_weight_bias_grad_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* dY, const void* dW, const void* db)
 {
     const size_t es = dt == F32 ? 4 : 2;
-    auto apart = [&](const void* o, size_t elems) { return (uintptr_t)db + es * n <= (uintptr_t)o || (uintptr_t)o + es * elems <= (uintptr_t)db; };
-    if (!apart(X, (size_t)m * k) || !apart(dY, (size_t)m * n) || !apart(dW, (size_t)n * k)) return 0;
+    const size_t mk = (size_t)m * k * es, mn = (size_t)m * n * es, nk = (size_t)n * k * es;
+    auto meet = [](const void* a, size_t na, const void* b, size_t nb) { return values_meet((const char*)a, (long long)na, (const char*)b, (long long)nb); };
+    if (meet(db, es * n, X, mk) || meet(db, es * n, dY, mn) || meet(db, es * n, dW, nk) || meet(dW, nk, X, mk) || meet(dW, nk, dY, mn)) return 0;
     if (dt == F32) return gemm_f32_row_sums_workspace_bytes(n, k, m, (((uintptr_t)X | (uintptr_t)dY) & 15) == 0 && n % 4 == 0 && k % 4 == 0);
     return gemm_b16_takes(b16_product(true, false, n, k, m, 1.f, dY, X, 1.f, nullptr)) ? gemm_b16_row_sums_workspace_bytes(n, k, m) : 0;
 }

@@ -700,15 +700,29 @@ static double b16_time(const GemmB16Shape& s, long long tiles, int k)
     return perCu == 1 ? len * s.perKAlone + s.endsAlone : perCu * (len * s.perK + s.ends) + s.once;
 }
 
-static GemmB16Plan gemm_b16_plan(int m, int n, int k)
+// A result in the memory of an operand is right where everything has been read before any of it is written: where the contraction is
+// cut into parts, or where one workgroup reads all that it overwrites - a single tile; with C in the rows of A (B16_ROWS) one tile in
+// width, with C in the columns of B (B16_COLUMNS) one in height.  Such a cut is taken if there is one.
+enum { B16_APART, B16_ROWS, B16_COLUMNS, B16_MEETS };
+static int b16_shares(const GemmB16& q)
 {
-    GemmB16Plan best = {0, 1, k};
+    const bool a = result_meets(q.C, (long long)q.m * q.n, q.heads, q.m, q.n, q.A, (long long)q.m * q.k);
+    const bool b = result_meets(q.C, (long long)q.m * q.n, q.heads, q.m, q.n, q.B, (long long)q.n * q.k);
+    if (!a && !b) return B16_APART;
+    if (!b && q.C == q.A && q.aK && q.n == q.k) return B16_ROWS;
+    if (!a && q.C == q.B && !q.bK && q.m == q.k) return B16_COLUMNS;
+    return B16_MEETS;
+}
+static GemmB16Plan gemm_b16_plan(int m, int n, int k, int shares = B16_APART, int maxParts = 16)
+{
+    GemmB16Plan best = {0, 0, k};
     double bestT = 1e30;
     for (int sh = 0; sh < B16_NSHAPES; sh++) {
         const GemmB16Shape& s = g_b16Shapes[sh];
-        const long long tiles = (long long)((m + s.bm - 1) / s.bm) * ((n + s.bn - 1) / s.bn);
-        for (int S = 1; S <= 16; S++) {
+        const long long high = (m + s.bm - 1) / s.bm, wide = (n + s.bn - 1) / s.bn, tiles = high * wide;
+        for (int S = 1; S <= maxParts; S++) {
             if (S > 1 && k / S < 256) break;
+            if (S == 1 && ((shares != B16_APART && shares != B16_ROWS && high > 1) || (shares != B16_APART && shares != B16_COLUMNS && wide > 1))) continue;
             const int chunk = ((k + S - 1) / S + 63) / 64 * 64;
             if ((k + chunk - 1) / chunk != S) continue;
             double t = b16_time(s, tiles * S, chunk);
@@ -716,7 +730,7 @@ static GemmB16Plan gemm_b16_plan(int m, int n, int k)
             if (t < bestT) { bestT = t; best = {sh, S, S > 1 ? chunk : k}; }
         }
     }
-    return best;
+    return best.splits ? best : gemm_b16_plan(m, n, k, B16_APART, maxParts);
 }
 
 bool gemm_b16_takes(const GemmB16& q)
@@ -731,11 +745,11 @@ bool gemm_b16_takes(const GemmB16& q)
     };
     return near(q.aK, q.m) && near(q.bK, q.n);
 }
-size_t gemm_b16_workspace_bytes(int m, int n, int k)
+size_t gemm_b16_workspace_bytes(const GemmB16& q)
 {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
-    const GemmB16Plan p = gemm_b16_plan(m, n, k);
-    return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
+    if (q.m <= 0 || q.n <= 0 || q.k <= 0) return 0;
+    const GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k, b16_shares(q));
+    return p.splits > 1 ? (size_t)p.splits * q.m * q.n * sizeof(float) : 0;
 }
 static int b16_tile_columns(int shape, int n) { return (n + g_b16Shapes[shape].bn - 1) / g_b16Shapes[shape].bn; }
 // With the sums of op(A)'s rows: the partial products (none where the contraction is not cut), then the partial sums.  0: not together.
@@ -746,7 +760,7 @@ size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k)
     const GemmB16Plan p = gemm_b16_plan(m, n, k);
     const long long columns = b16_tile_columns(p.shape, n);
     if (p.kChunk / (16 * columns) > 128 || (k <= 1024 && p.splits == 1)) return 0;   // one short launch would only be another
-    return gemm_b16_workspace_bytes(m, n, k) + (size_t)p.splits * columns * m * sizeof(float);
+    return ((p.splits > 1 ? (size_t)p.splits * m * n : 0) + (size_t)p.splits * columns * m) * sizeof(float);
 }
 
 template <int WVM, int WVN, int WM, int WN, int S, int OCC, bool AK, bool BKC, int HEADS, bool SUMS>
@@ -799,17 +813,8 @@ static GemmB16Args b16_args(const GemmB16& q)
 static bool b16_rows_takes(const GemmB16& q)
 {
     if (!q.aK || !q.bK || q.m > 32 || (q.k > 8192 && q.n < 4096) || (q.m > 16 && q.n > 768 * 16)) return false;
-    const size_t mk = (size_t)q.m * q.k * 2, nk = (size_t)q.n * q.k * 2, mn = (size_t)q.m * q.n * 2;
-    auto apart = [](const void* p, size_t pb, const void* o, size_t ob) { return (uintptr_t)p + pb <= (uintptr_t)o || (uintptr_t)o + ob <= (uintptr_t)p; };
-    auto free = [&](const void* dst, size_t bytes) {
-        const void* bias = q.heads ? q.heads->bias : (const void*)q.bias;
-        return apart(dst, bytes, q.A, mk) && apart(dst, bytes, q.B, nk) && (!bias || apart(dst, bytes, bias, (size_t)q.n * 2));
-    };
-    if (!q.heads) return free(q.C, mn);
-    const int third = q.heads->H * q.heads->hs;
-    for (int w = 0; w * third < q.n; w++)
-        if (!free(q.heads->dst[w], (size_t)q.m * third * 2)) return false;
-    return true;
+    return b16_shares(q) == B16_APART &&
+           !result_meets(q.C, (long long)q.m * q.n, q.heads, q.m, q.n, q.heads ? (const bf16_t*)q.heads->bias : q.bias, (long long)q.n);
 }
 template <int MT, int NT, int NW, int S, int HEADS>
 static hipError_t launch_b16_rows_shape(hipStream_t s, const GemmB16Args& g, const HeadsArg<(HEADS > 0)>& ha)
@@ -842,12 +847,16 @@ hipError_t gemm_b16(hipStream_t s, const GemmB16& q, void* ws, size_t wsBytes)
         if (q.heads) return q.m > 16 ? launch_b16_rows<2, 1>(s, a, heads_arg<true>(q.heads)) : launch_b16_rows<1, 1>(s, a, heads_arg<true>(q.heads));
         return q.m > 16 ? launch_b16_rows<2, 0>(s, a, HeadsArg<false>()) : launch_b16_rows<1, 0>(s, a, HeadsArg<false>());
     }
-    GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k);
+    const int shares = b16_shares(q);
+    GemmB16Plan p = gemm_b16_plan(q.m, q.n, q.k, shares);
     if (q.rowSum) {
         const size_t need = gemm_b16_row_sums_workspace_bytes(q.m, q.n, q.k);
-        if (need == 0 || !ws || wsBytes < need || ((uintptr_t)ws & 15) || q.heads || q.aK || q.bK) return hipErrorInvalidValue;
+        if (need == 0 || !ws || wsBytes < need || ((uintptr_t)ws & 15) || q.heads || q.aK || q.bK || shares != B16_APART) return hipErrorInvalidValue;
     }
-    if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) { p.splits = 1; p.kChunk = q.k; }
+    if (p.splits > 1 && (!ws || wsBytes < (size_t)p.splits * q.m * q.n * sizeof(float) || ((uintptr_t)ws & 15))) {
+        if (shares == B16_APART) { p.splits = 1; p.kChunk = q.k; }
+        else p = gemm_b16_plan(q.m, q.n, q.k, shares, 1);
+    }
     GemmB16Args a = b16_args(q);
     a.parts = p.splits; a.kChunk = p.kChunk;
     a.part = (float*)ws;

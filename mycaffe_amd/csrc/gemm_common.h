@@ -230,6 +230,21 @@ template <> struct Quad<bf16_t> {
     }
     __device__ static inline void store(bf16_t* p, const float (&v)[4]) { *(uint2*)p = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3])); }
 };
+// whether `n` values at p share memory with `m` values at q
+template <typename T> inline bool values_meet(const T* p, long long n, const T* q, long long m)
+{
+    return p && q && n > 0 && m > 0 && (uintptr_t)p < (uintptr_t)(q + m) && (uintptr_t)q < (uintptr_t)(p + n);
+}
+// whether what a product of m rows and n columns writes, to C (`count` values) or through `heads`, shares memory with `operand`
+template <typename T> inline bool result_meets(const T* C, long long count, const HeadsEpilogue* heads, int m, int n, const T* operand, long long values)
+{
+    if (!heads) return values_meet(C, count, operand, values);
+    const int third = heads->H * heads->hs;
+    for (int w = 0; w * third < n; w++)
+        if (values_meet((const T*)heads->dst[w], (long long)m * third, operand, values)) return true;
+    return false;
+}
+
 // C (m x n) = alpha op(A) op(B) + beta C in fp32, row-major (gemm_f32.hip).  op(A) is m x k: stored with k at unit stride
 // (aK; row i at A + i lda) or with i at unit stride (row k at A + k lda); op(B) is k x n: stored with k at unit stride (bK;
 // column j at B + j ldb) or with j at unit stride (row k at B + k ldb).
@@ -251,6 +266,9 @@ struct GemmF32 {
     float* rowSum;                         // (m) += the sums of op(A)'s rows; dense operands, both with their rows at unit stride
 };
 enum { CAUSAL_NO = 0, CAUSAL_A_LOWER /* A(i,k) zero for k > i */, CAUSAL_A_UPPER /* k < i */, CAUSAL_B_LOWER /* B(k,j) zero for k < j */, CAUSAL_B_UPPER /* k > j */ };
+// a result in the memory of an operand: taken by the kernels that always took such calls, and as before right where one workgroup has all
+// that it overwrites (a single tile, or rows of A in place that one tile is wide enough for) or where the contraction is cut into parts
+bool gemm_f32_shares(const GemmF32& g);
 size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal);
 size_t gemm_f32_row_sums_workspace_bytes(int m, int n, int k, bool vec);   // with rowSum; vec: operands in whole aligned 16-byte chunks; 0: not taken together
 hipError_t gemm_f32(hipStream_t s, const GemmF32& g, void* ws, size_t wsBytes);
@@ -267,7 +285,7 @@ struct GemmB16 {
     bf16_t* rowSum = nullptr;   // (m) += the sums of op(A)'s rows; both operands with their rows at unit stride
 };
 bool gemm_b16_takes(const GemmB16& g);   // 16-byte chunks of both operands aligned and whole
-size_t gemm_b16_workspace_bytes(int m, int n, int k);
+size_t gemm_b16_workspace_bytes(const GemmB16& g);
 size_t gemm_b16_row_sums_workspace_bytes(int m, int n, int k);   // with rowSum; 0: not taken together
 hipError_t gemm_b16(hipStream_t s, const GemmB16& g, void* ws, size_t wsBytes);
 bool gemm_b16_group(hipStream_t s, const GemmB16* q, int count, hipError_t* e);   // several with heads, of one n and k, as one launch

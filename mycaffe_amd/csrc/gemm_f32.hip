@@ -1043,7 +1043,9 @@ static double gemm_f32_small_time(long long tiles, int k)
     return 1.7 + (double)((perCu + 2) / 3) * (0.8 + 0.28 * k / 128) + (double)perCu * (0.3 + 0.46 * k / 128);
 }
 
-// Which kernel takes a product, and its plan.  The bf16 matrix cores from 64 k on (below, the split's error is larger than that of the
+// Which kernel takes a product, and its plan.  (fp32Sums also for a result in an operand's memory: the other two kernels read
+// operands while some of the result is written, the small tiles of one part of the rows and columns each, the split one once more
+// for a wavefront whose parts lost something.)  The bf16 matrix cores from 64 k on (below, the split's error is larger than that of the
 // fp32 matrix cores) and from 2^28 multiplications on (2048 x 512 x 384: 10.2 against 11.0 us; below, the chip is not full, and 16 x 288 x
 // 32000 takes 51 against 44 us); 32 x 32 tiles where their estimate is the smallest, which is a tenth of a round of the larger ones.
 enum { F32_TILES, F32_SPLIT, F32_SMALL };
@@ -1181,6 +1183,13 @@ static hipError_t launch_layout(hipStream_t s, GemmF32Args& a, const GemmF32Choi
     return launch_f32_tile<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
 }
 
+bool gemm_f32_shares(const GemmF32& q)
+{
+    auto values = [&](bool kFast, int rows, long long ld, long long stride) { return (q.batch - 1) * stride + (kFast ? (rows - 1) * ld + q.k : (q.k - 1) * ld + rows); };
+    const long long out = (q.batch - 1) * q.sC + (q.m - 1) * q.ldc + q.n;
+    return result_meets(q.C, out, q.heads, q.m, q.n, q.A, values(q.aK, q.m, q.lda, q.sA)) || result_meets(q.C, out, q.heads, q.m, q.n, q.B, values(q.bK, q.n, q.ldb, q.sB));
+}
+
 hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
 {
     if (q.m <= 0 || q.n <= 0 || q.batch <= 0) return hipSuccess;
@@ -1204,12 +1213,12 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     const bool vec = near && (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
                      (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0);
     if (!ws || ((uintptr_t)ws & 15)) wsBytes = 0;
-    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, q.fp32Sums || !near, q.heads != nullptr);
+    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, q.fp32Sums || !near || gemm_f32_shares(q), q.heads != nullptr);
     const GemmF32Plan& p = choice.plan;
     a.kChunk = p.kChunk;
     if (q.rowSum) {
         const size_t need = gemm_f32_row_sums_workspace_bytes(q.m, q.n, q.k, vec && !q.aK && !q.bK && q.lda == q.m && q.ldb == q.n && q.batch == 1 && !q.fp32Sums);
-        if (need == 0 || wsBytes < need) return hipErrorInvalidValue;
+        if (need == 0 || wsBytes < need || choice.kernel != F32_SPLIT) return hipErrorInvalidValue;
     }
     // rows shorter than the three values that a chunk may read past one: so many more k
     auto past = [&](bool kFast, int rows, long long ld) { return kFast ? q.k % 4 : rows % 4 == 0 ? 0 : ld >= 3 ? 1 : 3; };

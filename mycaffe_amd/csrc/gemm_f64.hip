@@ -339,6 +339,16 @@ template <bool VEC, bool HEADS> static hipError_t d_launch_layout(hipStream_t s,
     return bk ? d_launch_small<4, 64, false, true, VEC, false>(s, g, he, batch) : d_launch_small<4, 64, false, false, VEC, false>(s, g, he, batch);
 }
 
+struct MemRange { const double* p; size_t n; };
+// whether one of the first `out` ranges overlaps another one
+static bool shared_memory(const MemRange* r, int out, int all)
+{
+    for (int i = 0; i < out; i++)
+        for (int j = i + 1; j < all; j++)
+            if (r[i].n && r[j].n && r[i].p < r[j].p + r[j].n && r[j].p < r[i].p + r[i].n) return true;
+    return false;
+}
+
 hipError_t d_gemm(hipStream_t s, int batch, int m, int n, int k, double alpha, const double* A, long long ars, long long acs, const double* B,
                   long long brs, long long bcs, double beta, double* C, long long crs, long long ccs, long long sA, long long sB, long long sC,
                   int zdiv, long long sC2, const double* bias)
@@ -347,7 +357,13 @@ hipError_t d_gemm(hipStream_t s, int batch, int m, int n, int k, double alpha, c
     double time;
     const int kind = d_tiles(m, n, k, batch, &time);
     const long long tiles = (long long)((m + 15) / 16) * ((n + 15) / 16) * batch;
-    if (k > 0 && m > 0 && n > 0 && batch > 0 && tiles < (1ll << 24) && d_small_time(tiles, k) < time && d_near(ars, acs) && d_near(bcs, brs)) {
+    // a result in an operand's memory stays with the larger tiles: right as before where one workgroup reads all that it overwrites
+    auto shares = [&]() {
+        const long long last = batch - 1, out = last / zdiv * sC + (zdiv > 1 ? std::min<long long>(last, zdiv - 1) * sC2 : 0) + (m - 1) * crs + (n - 1) * ccs + 1;
+        const MemRange mem[] = {{C, (size_t)out}, {A, (size_t)(last * sA + (m - 1) * ars + (k - 1) * acs + 1)}, {B, (size_t)(last * sB + (k - 1) * brs + (n - 1) * bcs + 1)}};
+        return shared_memory(mem, 1, 3);
+    };
+    if (k > 0 && m > 0 && n > 0 && batch > 0 && tiles < (1ll << 24) && d_small_time(tiles, k) < time && d_near(ars, acs) && d_near(bcs, brs) && !shares()) {
         if (d_chunks(A, ars, acs, m, k, sA, batch) && d_chunks(B, bcs, brs, n, k, sB, batch)) return d_launch_layout<true, false>(s, g, HeadsD(), batch);
         return d_launch_layout<false, false>(s, g, HeadsD(), batch);
     }
@@ -361,16 +377,6 @@ hipError_t d_gemm(hipStream_t s, int batch, int m, int n, int k, double alpha, c
         hipLaunchKernelGGL((d_gemm_kernel<1, 4>), gridSmall, 1024, lds, s, g);
     } else hipLaunchKernelGGL((d_gemm_kernel<1, 1>), gridSmall, 256, 2 * 2 * 32 * 18 * 8, s, g);
     return hipGetLastError();
-}
-
-struct MemRange { const double* p; size_t n; };
-// whether one of the first `out` ranges overlaps another one
-static bool shared_memory(const MemRange* r, int out, int all)
-{
-    for (int i = 0; i < out; i++)
-        for (int j = i + 1; j < all; j++)
-            if (r[i].n && r[j].n && r[i].p < r[j].p + r[j].n && r[j].p < r[i].p + r[i].n) return true;
-    return false;
 }
 
 // X (m x k) W^T (n x k) + bias through `he`, where 16 x 16 tiles are what the size calls for (*done)

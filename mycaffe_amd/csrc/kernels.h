@@ -128,7 +128,7 @@ hipError_t k_channel_dot(hipStream_t s, DType dt, size_t num, int channels, int 
 // ws: k_gemm_workspace_bytes(...) bytes of scratch for contractions cut into parts (without it they are not)
 hipError_t k_gemm(hipStream_t s, DType dt, bool tA, bool tB, int m, int n, int k, float alpha, const void* A,
                   const void* B, float beta, void* C, void* ws = nullptr, size_t wsBytes = 0);
-size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k);
+size_t k_gemm_workspace_bytes(DType dt, bool tA, bool tB, int m, int n, int k, const void* A, const void* B, const void* C);
 // Fused QKV projection of CausalSelfAttentionLayer: [q|k|v] = X W^T + bias with X (B*T, C), W (3C, C), C = H*hs, written
 // straight into three (B,H,T,hs) tensors.  ws: k_gemm_qkv_heads_workspace_bytes(...) of scratch.
 hipError_t k_gemm_qkv_heads(hipStream_t s, DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* bias,
@@ -143,10 +143,10 @@ hipError_t k_gemm_bias_heads(hipStream_t s, DType dt, int B, int T, int H, int h
 // several of those in 16-bit storage, of one width and contraction, as one launch, if that takes them (*done)
 struct HeadsProjection { int m, T; const void *X, *W, *bias; void* Y; };
 hipError_t k_gemm_bias_heads_group(hipStream_t s, int count, int n, int k, int H, const HeadsProjection* p, bool* done);
-size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W);
+size_t k_gemm_bias_workspace_bytes(DType dt, int m, int n, int k, const void* X, const void* W, const void* Y, bool heads = false);
 // whether the call fails without that scratch (otherwise its contraction stays in one part)
 bool k_gemm_bias_needs_workspace(DType dt, int m, int n, int k, const void* X, const void* W);
-size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W);
+size_t k_gemm_qkv_heads_workspace_bytes(DType dt, int B, int T, int H, int hs, const void* X, const void* W, const void* q, const void* k, const void* v);
 // column-major strided batched gemm with BLAS semantics (fp32)
 // C (fp32) = alpha X W^T + beta C on the bf16 matrix cores: W 16-bit (n x k), k % 64 == 0; A is X as bf16 (m x k) or,
 // split, every row of X as two bf16 rows (nearest bf16, then the bf16 nearest to the remainder; m x 2k)

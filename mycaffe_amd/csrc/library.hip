@@ -340,7 +340,7 @@ long Kernel::flush_pending_product(bool causal)
     if (m_mem.get(p.hA, &A) || m_mem.get(p.hB, &B) || m_mem.get(p.hC, &C)) return 0;   // an operand is gone
     if (p.kind == 1) {
         void* ws = nullptr;
-        size_t wsb = k_gemm_workspace_bytes(C->dt(), false, true, p.m, p.n, p.k);
+        size_t wsb = k_gemm_workspace_bytes(C->dt(), false, true, p.m, p.n, p.k, A->ptr, B->ptr, C->ptr);
         workspace_or_none(&wsb, &ws);
         HIPCHK(k_gemm(m_stream, C->dt(), false, true, p.m, p.n, p.k, p.alpha, A->ptr, B->ptr, 0.f, C->ptr, ws, wsb));
         return 0;
@@ -817,7 +817,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 if (!m_mem.get(p.hA, &X) && !m_mem.get(p.hB, &W) && !m_mem.get(p.hC, &C) && C->half == A->half) {
                     m_pendingProduct = PendingProduct();
                     void* ws = nullptr;
-                    size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr);
+                    size_t wsb = k_gemm_bias_workspace_bytes(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, C->ptr);
                     if (k_gemm_bias_needs_workspace(C->dt(), p.m, p.n, p.k, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
                     else workspace_or_none(&wsb, &ws);
                     HIPCHK(k_gemm_bias(s, C->dt(), p.m, p.n, p.k, X->ptr, W->ptr, B->ptr, C->ptr, ws, wsb));
@@ -856,7 +856,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             RANGE(C, co, (long long)m * n);
             // the transpose combinations of the layers' backward passes turn an operand in scratch memory
             void* ws = nullptr;
-            size_t wsb = k_gemm_workspace_bytes(A->dt(), tA, tB, m, n, k);
+            size_t wsb = k_gemm_workspace_bytes(A->dt(), tA, tB, m, n, k, PTR(A, ao), PTR(B, bo), PTR(C, co));
             workspace_or_none(&wsb, &ws);
             HIPCHK(k_gemm(s, A->dt(), tA, tB, m, n, k, pf[0], PTR(A, ao), PTR(B, bo), pf[1], PTR(C, co), ws, wsb));
         }
@@ -2171,7 +2171,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             }
         }
         void* ws = nullptr;
-        size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr);
+        size_t wsb = k_gemm_qkv_heads_workspace_bytes(X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Q->ptr, K->ptr, V->ptr);
         if (k_gemm_bias_needs_workspace(X->dt(), (int)M, (int)(3 * C), (int)C, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
         else workspace_or_none(&wsb, &ws);
         HIPCHK(k_gemm_qkv_heads(s, X->dt(), (int)B, (int)T, (int)H, (int)hs, X->ptr, W->ptr, Bi ? Bi->ptr : nullptr, Q->ptr, K->ptr,
@@ -2203,7 +2203,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         if (Bi) RANGE(Bi, 0, N);
         RANGE(Y, 0, M * N);
         void* ws = nullptr;
-        size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr);
+        size_t wsb = k_gemm_bias_workspace_bytes(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr, Y->ptr, heads != 0);
         if (k_gemm_bias_needs_workspace(X->dt(), (int)M, (int)N, (int)K, X->ptr, W->ptr)) ERRCHK(workspace(wsb, &ws));
         else workspace_or_none(&wsb, &ws);
         if (heads)
@@ -2281,9 +2281,9 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
                 return 0;
             }
         }
-        const size_t wsW = k_gemm_workspace_bytes(dt, true, false, (int)N, (int)K, (int)M), wsB = dB ? k_bias_grad_workspace_bytes((int)M, (int)N) : 0;
+        const size_t wsW = k_gemm_workspace_bytes(dt, true, false, (int)N, (int)K, (int)M, dY->ptr, X->ptr, dW->ptr), wsB = dB ? k_bias_grad_workspace_bytes((int)M, (int)N) : 0;
         const size_t wsT = dB ? k_weight_bias_grad_workspace_bytes(dt, (int)M, (int)N, (int)K, X->ptr, dY->ptr, dW->ptr, dB->ptr) : 0;   // both together
-        const size_t wsX = dX ? k_gemm_workspace_bytes(dt, false, false, (int)M, (int)K, (int)N) : 0, most = std::max(wsW, std::max(wsB, wsX));
+        const size_t wsX = dX ? k_gemm_workspace_bytes(dt, false, false, (int)M, (int)K, (int)N, dY->ptr, W->ptr, dX->ptr) : 0, most = std::max(wsW, std::max(wsB, wsX));
         void* ws = nullptr;
         size_t have = std::max(most, wsT);
         workspace_or_none(&have, &ws);
