@@ -125,26 +125,20 @@ template <typename T> __global__ __launch_bounds__(256) void attn_bwd_stats_kern
     if (lane == 0) a.lse2[bh * a.Tq + row] = (m == MASKED_SCORE) ? -INFINITY : (m + logf(l)) * LOG2E;
 }
 
-// dQ: one wavefront per query row, lanes over keys
-template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dq_rows_kernel(AttnBwdArgs a)
+// dQ: one query row by one wavefront, lanes over keys; qs, gs: hs floats of LDS each of its own
+template <typename T> __device__ __forceinline__ void attn_bwd_dq_row(const AttnBwdArgs& a, int b, int h, int row, float lse2, float dsum, float* qs, float* gs)
 {
     constexpr int DPL = 4;  // hs <= 256
-    __shared__ float qs[4][256], gs[4][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = blockIdx.x * 4 + wave;
-    const int h = blockIdx.y, b = blockIdx.z;
-    const bool valid = row < a.Tq;
+    const int lane = own_lane();
     const size_t bh = (size_t)b * a.H + h;
-    const size_t ro = (bh * a.Tq + (valid ? row : 0)) * a.hs;
+    const size_t ro = (bh * a.Tq + row) * a.hs;
     for (int d = lane; d < a.hs; d += 64) {
-        qs[wave][d] = ldb((const T*)a.q + ro, d) * a.scale;
-        gs[wave][d] = ldb((const T*)a.dy + ro, d);
+        qs[d] = ldb((const T*)a.q + ro, d) * a.scale;
+        gs[d] = ldb((const T*)a.dy + ro, d);
     }
-    __syncthreads();
-    if (!valid) return;
+    wave_lds_fence();
     const T* k = (const T*)a.k + bh * a.Tk * a.hs;
     const T* v = (const T*)a.v + bh * a.Tk * a.hs;
-    const float lse2 = a.lse2[bh * a.Tq + row], dsum = a.dsum[bh * a.Tq + row];
     const float uniform = 1.0f / a.Tk;
     // causal rows that are not fully masked have zero probability past the diagonal
     const int kend = (a.kind == MASK_CAUSAL && lse2 != -INFINITY) ? min(a.Tk, row + 1) : a.Tk;
@@ -157,8 +151,8 @@ template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dq_rows_ke
             const T* vr = v + (size_t)j * a.hs;
             float s = 0.f, dp = 0.f;
             for (int i = 0; i < a.hs; i++) {
-                s += qs[wave][i] * ldb(kr, i);
-                dp += gs[wave][i] * ldb(vr, i);
+                s += qs[i] * ldb(kr, i);
+                dp += gs[i] * ldb(vr, i);
             }
             const float p = attn_prob(s, attn_masked(a, b, row, j), lse2, uniform);
             float pf, sf;
@@ -179,6 +173,14 @@ template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dq_rows_ke
         const int d = lane + i * 64;
         if (d < a.hs) stb((T*)a.dq + ro, d, acc[i]);
     }
+}
+template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dq_rows_kernel(AttnBwdArgs a)
+{
+    __shared__ float qs[4][256], gs[4][256];
+    const int wave = threadIdx.x >> 6, row = blockIdx.x * 4 + wave;
+    if (row >= a.Tq) return;
+    const size_t at = ((size_t)blockIdx.z * a.H + blockIdx.y) * a.Tq + row;
+    attn_bwd_dq_row<T>(a, blockIdx.z, blockIdx.y, row, a.lse2[at], a.dsum[at], qs[wave], gs[wave]);
 }
 
 // dK, dV: one wavefront per key row, lanes over queries
@@ -340,7 +342,9 @@ template <int KIND> __device__ inline bool bwd_masked(const AttnBwdArgs& a, int 
 
 // KIND: 0 none, 1 causal, 2 key mask (B,Tk), 3 mask (B,Tq,Tk) or, with mb = 0, one (Tq,Tk) mask for all sequences
 // PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 54 us
-// here and 47 for dq; the row kernels 671 and 450)
+// here and 47 for dq; the row kernels 671 and 450).  Infinities and NaN: as in flash_fwd_kernel, a wavefront whose sums for dq are not
+// finite does its queries over row by row.  dK and dV need that not: what a masked query has to add NaN to them, an infinity in its row of
+// Q or dY, makes its D infinite or NaN, by which the row kernel adds NaN too.
 template <typename T, int HS, int KIND, int BQ, int OCC, bool PADDED>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs a, int mb)
 {
@@ -403,6 +407,10 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
         for (int i = 0; i < CPT; i++) {
             qreg[i] = chunk(qp + r, (cg + TPR * i) * EPC);
             greg[i] = chunk(gp + r, (cg + TPR * i) * EPC);
+        }
+        if (PADDED && q0 + BQ > a.Tq && q0 + srow >= a.Tq) {   // rows past the last one: zeros, as their probabilities
+#pragma unroll
+            for (int i = 0; i < CPT; i++) qreg[i] = greg[i] = u32x4{0, 0, 0, 0};
         }
         if (tid < BQ) {
             const int qq = q0 + tid;
@@ -525,6 +533,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
     float* Ms = TL::TRR ? (float*)Kt : (float*)(Kt + HS * LDT);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    [[maybe_unused]] const int waveId = __builtin_amdgcn_readfirstlane(wave);   // the same, in a scalar register
     const int l32 = lane & 31, half = lane >> 5;
     const int nbh = a.B * a.H;
     const int nqb = (a.Tq + BM - 1) / BM;
@@ -652,6 +661,19 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
         __syncthreads();
         if (more) sstore();
         __syncthreads();
+    }
+    if constexpr (PADDED) {
+        float sum = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) sum += fabsf(aq[dt][v]);
+        if (waveActive && __any(!(sum < INFINITY))) {
+            const int first = qblock * BM + waveId * 32;
+            float* own = (float*)bwd_smem + waveId * 2 * HS;
+            for (int r = 0; r < min(32, a.Tq - first); r++) attn_bwd_dq_row<T>(a, b, h, first + r, __shfl(lrow, r), __shfl(drow, r), own, own + HS);
+            return;
+        }
     }
     if (waveActive && qrow < a.Tq) {
         T* dqr = (T*)a.dq + (bh * a.Tq + qrow) * hs;

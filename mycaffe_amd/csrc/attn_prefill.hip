@@ -39,22 +39,17 @@ struct AttnArgs {
 };
 
 
-// 4 wavefronts per workgroup, one query row each
-template <typename T> __global__ __launch_bounds__(256) void attn_rows_kernel(AttnArgs a)
+// one query row by one wavefront; qs: hs floats of LDS of its own
+template <typename T> __device__ __forceinline__ void attn_row(const AttnArgs& a, int b, int h, int row, float* qs)
 {
     constexpr int DPL = 4;  // hs <= 256
-    __shared__ float qs[4][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = blockIdx.x * 4 + wave;
-    const int h = blockIdx.y, b = blockIdx.z;
-    const bool valid = row < a.Tq;
+    const int lane = own_lane();
     const size_t bh = (size_t)b * a.H + h;
-    const T* q = (const T*)a.q + (bh * a.Tq + (valid ? row : 0)) * a.hs;
+    const T* q = (const T*)a.q + (bh * a.Tq + row) * a.hs;
     const T* k = (const T*)a.k + bh * a.Tk * a.hs;
     const T* v = (const T*)a.v + bh * a.Tk * a.hs;
-    for (int d = lane; d < a.hs; d += 64) qs[wave][d] = ldp(q, d) * a.scale;
-    __syncthreads();
-    if (!valid) return;
+    for (int d = lane; d < a.hs; d += 64) qs[d] = ldp(q, d) * a.scale;
+    wave_lds_fence();
     // causal: keys beyond the row contribute exp(-1e29 - max) == 0 exactly, skip them
     const int kend = (a.kind == MASK_CAUSAL) ? min(a.Tk, row + 1) : a.Tk;
     float m = -INFINITY, l = 0.f, acc[DPL] = {0.f, 0.f, 0.f, 0.f};
@@ -64,7 +59,7 @@ template <typename T> __global__ __launch_bounds__(256) void attn_rows_kernel(At
         if (j < kend) {
             const T* kr = k + (size_t)j * a.hs;
             float d = 0.f;
-            for (int i = 0; i < a.hs; i++) d += qs[wave][i] * ldp(kr, i);
+            for (int i = 0; i < a.hs; i++) d += qs[i] * ldp(kr, i);
             s = d;
             float mv = 1.f;
             if (a.kind == MASK_QK) mv = a.mask[(size_t)row * a.Tk + j];
@@ -103,6 +98,14 @@ template <typename T> __global__ __launch_bounds__(256) void attn_rows_kernel(At
     }
     // a causal row's maximum is never the fill value, so the shortened key range above changes nothing here
     if (a.lse2 && lane == 0) a.lse2[bh * a.Tq + row] = (m == MASKED) ? -INFINITY : (m + __logf(l)) * 1.4426950408889634f;
+}
+
+// 4 wavefronts per workgroup, one query row each
+template <typename T> __global__ __launch_bounds__(256) void attn_rows_kernel(AttnArgs a)
+{
+    __shared__ float qs[4][256];
+    const int wave = threadIdx.x >> 6, row = blockIdx.x * 4 + wave;
+    if (row < a.Tq) attn_row<T>(a, blockIdx.z, blockIdx.y, row, qs[wave]);
 }
 
 hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* handled);
@@ -225,7 +228,8 @@ __device__ __forceinline__ void flash_softmax_step(floatx16 (&s)[QT], floatx16 (
 // KIND: 0 no mask, 1 causal, 2 per-key mask (B, Tk), 3 per-sequence mask (B, Tq, Tk).  OCC: workgroups per CU the register budget is set for.
 // PREFETCH: hold the next K / V block in registers while computing on the current one.
 // PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 33 us;
-// the kernel with a wavefront per row, which had these, 546).
+// the kernel with a wavefront per row, which had these, 546).  A key that a row does not see has weight zero here and is not read there, which
+// differs where it holds an infinity or a NaN: a wavefront whose sums are not finite does its rows over as that kernel does.
 template <typename T, int HS, int KIND, int QT, int NW, int OCC, bool PREFETCH, bool PADDED>
 __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
 {
@@ -253,6 +257,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
     __shared__ float Ms[BN];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    [[maybe_unused]] const int waveId = __builtin_amdgcn_readfirstlane(wave);   // the same, in a scalar register
     const int l32 = lane & 31, half = lane >> 5;
     // Causal work grows with the query block, so the launch is one-dimensional and ordered heaviest block
     // first across ALL (batch, head) pairs: workgroups are dispatched in index order as slots free up, which
@@ -462,6 +467,19 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         __syncthreads();
     }
 
+    bool over = false;
+    if constexpr (PADDED) {
+        float sum = 0.f;
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+            sum += l[qt];
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) sum += fabsf(o[dt][qt][v]);
+        }
+        over = __any(!(sum < INFINITY));
+    }
     // epilogue: y[query, dim] = O^T[dim, query] / l; register v of tile dt is dim 32*dt + 8*(v/4) + 4*half + v%4
 #pragma unroll
     for (int qt = 0; qt < QT; qt++) {
@@ -470,7 +488,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         const float inv = 1.0f / lt;
         if (a.lse2 && qrow < a.Tq && half == 0)
             a.lse2[bh * a.Tq + qrow] = (m[qt] == a.maskedRaw) ? -INFINITY : __builtin_fmaf(m[qt], a.c, __log2f(lt));
-        if (qrow < a.Tq) {
+        if (qrow < a.Tq && !over) {
             T* yr = (T*)a.y + attn_y_row(a.yMerged, b, h, a.H, a.Tq, qrow, hs);
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
@@ -479,6 +497,15 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
                     if (!PADDED || 32 * dt + 8 * g + 4 * half < hs)
                         TR::store4(yr + 32 * dt + 8 * g + 4 * half, o[dt][qt][4 * g] * inv, o[dt][qt][4 * g + 1] * inv,
                                    o[dt][qt][4 * g + 2] * inv, o[dt][qt][4 * g + 3] * inv);
+        }
+    }
+    if constexpr (PADDED) {
+        static_assert(NW * HS * sizeof(float) <= sizeof(Ks), "a row of a wavefront each");   // every wavefront is past its last step
+        if (over) {
+            const int kind = KIND == 0 ? MASK_NONE : KIND == 1 ? MASK_CAUSAL : KIND == 2 ? MASK_KEY : a.maskBatch ? MASK_BQK : MASK_QK;
+            const AttnArgs r = {a.q, a.k, a.v, a.y, a.mask, a.B, a.H, a.Tq, a.Tk, hs, kind, a.scale, nullptr, a.yMerged, 0, AttnDropout()};
+            const int first = qblock * BM + waveId * 32 * QT;
+            for (int row = first; row < min(first + 32 * QT, a.Tq); row++) attn_row<T>(r, b, h, row, (float*)Ks + waveId * HS);
         }
     }
 }
@@ -897,6 +924,7 @@ hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* h
     f.yMerged = a.yMerged;
     f.causalGroup = 0;
     f.hs = a.hs;
+    f.scale = a.scale;
     if (a.kind == MASK_CAUSAL && a.hs == 128 && dt == BF16) {
         // when K and V of all heads together exceed what the caches hold (128 MB taken as the line), walk the heads in
         // at most four groups of a multiple of 8 heads

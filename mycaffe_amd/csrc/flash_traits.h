@@ -126,6 +126,17 @@ template <> struct FlashTraits<float> {
     }
 };
 
+// the lane without a register kept for it
+__device__ __forceinline__ int own_lane() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
+// between what lanes of one wavefront write to LDS and what others of it read there (a wavefront's LDS operations complete in order)
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // offset of output row `row` of head (b, h) in y
 __device__ __forceinline__ size_t attn_y_row(int yMerged, int b, int h, int H, int Tq, int row, int hs)
 {
@@ -145,6 +156,7 @@ struct FlashArgs {
     int yMerged;         // y laid out (B,Tq,H,hs) instead of (B,H,Tq,hs)
     int causalGroup;     // causal launches: heads per group of the workgroup order (0: all heads in one group)
     int hs;              // head size, of the kernels that take any up to their own
+    float scale;         // softmax scale
 };
 
 // Rank of a workgroup of a causal launch in the heaviest-first order.  Workgroup i goes to XCD i % 8 and, within it, the

@@ -5,7 +5,7 @@ import pytest
 
 from oracle import attention_ref as R
 from tests.conftest import BF16_RTOL, FP32_RTOL, bf16_round
-from tests.test_gpu_attention_backward import _check, _fwd_bwd
+from tests.test_gpu_attention_backward import _check, _fwd_bwd, _probs
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +42,59 @@ def test_infinite_neighbours(dev):
     assert np.abs(dev.get(hy, q.shape) - want).max() <= 1e-5 * np.abs(want).max()
     dev.cuda.FreeAttn(ha)
     dev.cuda.FreeCuDNN(hc)
+
+
+# A causal row does not read what lies behind it: infinities and NaN in later keys and values leave the rows before them as they are, and the
+# gradients of those rows.  hs 50 and 100: a kernel with a wavefront per row (16 bits), and none of a power of two.
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("hs", [8, 16, 48, 50, 72, 100])
+@pytest.mark.parametrize("T,at", [(100, 20), (64, 63), (37, 33), (200, 130)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_causal_rows_before_infinities(dev, T, at, hs, half, bad):
+    rng = np.random.default_rng(hs + T)
+    q, k, v, dy = (bf16_round(rng.standard_normal((1, 2, T, hs)).astype(np.float32)) for _ in range(4))
+    mask, tol = R.causal_mask(T), BF16_RTOL if half else FP32_RTOL
+    clean = _probs(q, k, mask, 0)
+    want = [clean @ v.astype(np.float64), *R.attn_backward(q, k, v, clean, dy, np.float64)]
+    k2, v2 = k.copy(), v.copy()
+    k2[0, 0, at, 3], v2[0, 1, at, 5], v2[0, 1, at, hs - 1] = bad, bad, bad
+    y, dq, dk, dv = _fwd_bwd(dev, q, k2, v2, dy, mask, 0, half)
+    for got, exp in ((y, want[0]), (dq, want[1])):
+        assert np.abs(got[:, :, :at] - exp[:, :, :at]).max() <= tol * np.abs(exp).max()
+    # a value past its row's weight: that dimension of the rows from it on, no other
+    others = np.setdiff1d(np.arange(hs), [5, hs - 1])
+    assert np.abs(y[0, 1][:, others] - want[0][0, 1][:, others]).max() <= tol * np.abs(want[0]).max()
+    assert np.array_equal(y[0, 1, at:, [5, hs - 1]], np.full((2, T - at), bad, np.float32), equal_nan=True)
+    # the weights do not depend on values
+    assert np.abs(dv[0, 1] - want[3][0, 1]).max() <= tol * np.abs(want[3]).max()
+
+
+# the last key's row stands in for those past it, with weight zero: its own weight times infinity stays an infinity
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("hs", [16, 48, 72])
+def test_infinity_in_the_last_value(dev, hs, half):
+    rng = np.random.default_rng(hs)
+    q, k, v = (bf16_round(rng.standard_normal((2, 2, 45, hs)).astype(np.float32)) for _ in range(3))
+    v[0, 0, 44, 2], v[1, 1, 44, 7] = np.inf, -np.inf
+    y = _fwd_bwd(dev, q, k, v, np.ones_like(q), None, 0, half)[0]
+    with np.errstate(invalid="ignore"):
+        want = _probs(q, k, None, 0) @ v.astype(np.float64)
+    assert np.array_equal(np.isinf(y), np.isinf(want)) and np.array_equal(y[np.isinf(y)], want[np.isinf(want)].astype(np.float32))
+    fine = np.isfinite(want)
+    assert np.isfinite(y[fine]).all() and np.abs(y[fine] - want[fine]).max() <= (BF16_RTOL if half else FP32_RTOL) * np.abs(want[fine]).max()
+
+
+# the same for the last query's row of the gradient
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("hs", [16, 48, 72])
+def test_infinity_in_the_last_gradient(dev, hs, half):
+    rng = np.random.default_rng(hs)
+    q, k, v, dy = (bf16_round(rng.standard_normal((1, 2, 45, hs)).astype(np.float32)) for _ in range(4))
+    mask, dy2 = R.causal_mask(45), dy.copy()
+    dy2[0, 1, 44, 2] = np.inf
+    p = _probs(q, k, mask, 0)
+    dv = _fwd_bwd(dev, q, k, v, dy2, mask, 0, half)[3]
+    want = np.swapaxes(p, -1, -2) @ dy.astype(np.float64)
+    want[0, 1, :, 2] = np.inf
+    fine = np.isfinite(want)
+    assert np.array_equal(dv[~fine], want[~fine].astype(np.float32)) and np.abs(dv[fine] - want[fine]).max() <= (BF16_RTOL if half else FP32_RTOL) * np.abs(want[fine]).max()
