@@ -401,6 +401,11 @@ MCH_LONG MCH_TimeInvokeFloatEx2Sets(MCH_LONG lKernelIdx, MCH_LONG lFunctionIdx, 
                                     MCH_LONGLONG* plInput, MCH_LONG llInput, MCH_LONG nSets, MCH_LONG nWarmup,
                                     MCH_LONG nReps, float* pfMs, MCH_TCHAR* szErr, MCH_LONG lszErrMax);
 
+/* Which kernel a float product of these sizes goes to, for tests that mean a certain one; runs on the host alone.
+ * flags: 1 causal operand, 2 fp32Sums, 4 written head by head.  Returns 0 for gemm_f32_kernel, 1 for gemm_f32_split_kernel, 2 for
+ * gemm_f32_small_kernel, + 4 times the tile's number there + 64 times the parts of the contraction, given the scratch memory. */
+MCH_LONG MCH_GemmFloatRoute(MCH_LONG m, MCH_LONG n, MCH_LONG k, MCH_LONG nBatch, MCH_LONG flags);
+
 /* ---- entry point that allocates nothing (no counterpart in the reference) ----
  * For callers that cannot allocate device memory: code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  (What the entry point guarantees is that nothing is allocated and that its scratch is cleared

@@ -373,12 +373,18 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, Heads
 // where the fp32 one adds two, so the sums are rounded less often, and the error against 64 bits is below that of the fp32
 // matrix cores from 64 k on (N(0, 1), 2-norm of the error over that of the result: 1.35e-7 against 1.45e-7 at 64 k, 4.3e-7 against
 // 5.0e-7 at 768, 7.0e-7 against 8.0e-7 at 2048; the other way round at 16: 8.2e-8 against 7.4e-8); shorter contractions stay
-// there (SPLIT_MIN_K).
+// there (gemm_f32_choose).
 //
-// Exact results where parts do not hold a value: an infinity or a value above the largest bf16 number leaves a NaN or an
-// infinity among the parts and so in the result, and below 2^-109 the last part loses bits (bf16 ends at 2^-133), 2^-134 of the
-// other factor at most.  A wavefront whose sums hold a NaN, an infinity or anything nonzero below 2^-90 therefore does its tile
-// again on the fp32 matrix cores, straight from memory.
+// Exact results where parts do not hold a value.  An infinity or a value above the largest bf16 number leaves a NaN or an infinity
+// among the parts and so in the sums.  Below 2^-109 the last part, or all of them, lose bits (bf16 ends at 2^-133): up to 2^-134 of
+// the value, and of the sum that times the other factor, which may be any number.  It shows in what the last part is made of, eight
+// bits of an fp32 number that end above its low half wherever bf16 holds them: the low halves of all of them are or-ed together
+// (one v_or3 for two values).  A wavefront does its tile again on the fp32 matrix cores, straight from memory, if its sums hold a NaN, an
+// infinity or anything nonzero below 2^-90, or if a value of the workgroup's operands lost bits and either some value is 2^16 or more (for which
+// they are then read once more) or a sum, zeros among them, is so small that k products with up to 2^16 times those bits may be 2^-25 of
+// it.  So an ordinary tile beside a stray tiny value (GELU of -10) is not made over: 8192 x 3072 x 768 with one in every tile takes 280 us, 218
+// without, 570 with a row of zeros beside one.  (Looking for lost bits takes 1 % of an ordinary product; keeping the largest value
+// along too, for the second reading, 2 - 3 %.)
 //
 // What bounds it is power: at 8192 x 3072 x 768 operands of zeros take 136 us in 128 x 192 tiles, random ones 197 (same instructions), so what
 // helps is fewer instructions and bytes per product.  Values are split once, on their way from registers to LDS (splitting whole
@@ -407,10 +413,47 @@ __device__ __forceinline__ uint2 split_part(float (&v)[4], bool last)
     return p;
 }
 
-// whether the parts may have lost something of these sums (the same for the whole wavefront)
-template <int WM, int WN> __device__ __forceinline__ bool split_lost(const floatx16 (&acc)[WM][WN])
+// written as an instruction, in its place: the compiler would gather those of a stage at its end, and keep the values until then (14
+// registers; 256 x 256 tiles spill)
+__device__ __forceinline__ void or3(uint32_t& m, uint32_t a, uint32_t b) { asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(m) : "v"(a), "v"(b)); }
+
+// what the workgroup's wavefronts leave in LDS for each other: whether a value lost bits, and whether one is LARGE or more
+struct SplitFlags { uint32_t lost, large; };
+constexpr float SPLIT_LARGE = 65536.f;
+
+// whether this thread finds a value of SPLIT_LARGE or more in its share of an operand's R rows (`rows` of them there) from kBegin to kEnd
+template <int R, int NT, bool KFAST> __device__ __forceinline__ bool split_large(const float* base, long long ld, int rows, int kBegin, int kEnd, int tid)
+{
+    constexpr int U = 16, W = KFAST ? 64 : 32;   // loads under way; lanes along the memory
+    const int fast = tid % W, fastEnd = KFAST ? kEnd : min(R, rows), slowEnd = KFAST ? min(R, rows) : kEnd;
+    bool found = false;
+    for (int f = (KFAST ? kBegin : 0) + fast; f < fastEnd; f += W)
+        for (int s0 = (KFAST ? 0 : kBegin) + tid / W; s0 < slowEnd; s0 += U * (NT / W)) {
+            float x[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) x[u] = base[(size_t)min(s0 + u * (NT / W), slowEnd - 1) * ld + f];
+#pragma unroll
+            for (int u = 0; u < U; u++) found |= fabsf(x[u]) >= SPLIT_LARGE;
+        }
+    return found;
+}
+
+// whether the parts may have lost something of these sums of k products (the same for the whole wavefront)
+template <int WM, int WN> __device__ __forceinline__ bool split_lost(const floatx16 (&acc)[WM][WN], const SplitFlags& flags, int k)
 {
     constexpr uint32_t TINY = (127u - 90u) << 24;   // 2^-90 without its sign
+    if (flags.lost) {
+        if (flags.large) return true;
+        const float limit = (float)k * 0x1p-92f;   // 2 k values' 2^-134 times SPLIT_LARGE, 2^25 times that
+        float least = limit;
+#pragma unroll
+        for (int i = 0; i < WM; i++)
+#pragma unroll
+            for (int j = 0; j < WN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) least = fminf(least, fabsf(acc[i][j][v]));
+        if (__any(least < limit)) return true;
+    }
     uint32_t low = 0xffffffffu;
     float sum = 0.f;
 #pragma unroll
@@ -473,6 +516,11 @@ template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC> constexpr
 {
     constexpr int stages = 2 * 3 * (split_plane<32 * WVM * WM, KS, AK>() + split_plane<32 * WVN * WN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
     return (stages > store ? stages : store) / 4;
+}
+// where in bytes the flags lie, behind the row sums
+template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC, bool SUMS> constexpr int split_flags_at()
+{
+    return 4 * split_lds<WVM, WVN, WM, WN, KS, AK, BKC>() + (SUMS ? 64 * WVM * WVN * 16 : 0);
 }
 // sums of op(A)'s rows over some of the k, [part][tile column][M], behind the partial products
 __device__ __forceinline__ float* f32_row_part(const GemmF32Args& g) { return g.part + (g.kChunk < g.K ? (size_t)g.parts * g.M * g.N : 0); }
@@ -594,6 +642,9 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     [[maybe_unused]] float sums[4] = {0.f, 0.f, 0.f, 0.f};
     [[maybe_unused]] int turn = n0 / BN, putting = 0;   // the stage that is put, and stages until this tile's next
     [[maybe_unused]] uint32_t mine = turn == 0 ? 0xffffffffu : 0u;
+    uint32_t rest = 0;      // of all values, or-ed: what the last part is made of
+    SplitFlags* flags = reinterpret_cast<SplitFlags*>(smem_raw + split_flags_at<WVM, WVN, WM, WN, KS, AK, BKC, SUMS>());
+    if (tid == 0) *flags = SplitFlags{0, 0};
     // part s of chunk c to its plane of a stage
     auto put = [&](int c, int s, unsigned char* stage) {
         if constexpr (SUMS) {
@@ -603,6 +654,10 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             }
         }
         float v[4] = {__uint_as_float(raw[c].x), __uint_as_float(raw[c].y), __uint_as_float(raw[c].z), __uint_as_float(raw[c].w)};
+        if (s == 2) {
+            or3(rest, raw[c].x, raw[c].y);
+            or3(rest, raw[c].z, raw[c].w);
+        }
         const uint2 p = split_part(v, s == 2);
         raw[c].x = __float_as_uint(v[0]); raw[c].y = __float_as_uint(v[1]); raw[c].z = __float_as_uint(v[2]); raw[c].w = __float_as_uint(v[3]);
         *(uint2*)(stage + (c < PA ? wa[c] + s * PLA : wb[c - PA] + s * PLB)) = p;
@@ -730,8 +785,14 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             f32_row_part(g)[(size_t)(it.part * g.tilesN + n0 / BN) * M + m0 + tid] = v;
         }
     }
+    if (rest & 0xffffu) flags->lost = 1;
     __syncthreads();
-    if (split_lost(acc)) f32_sums<WM, WN, AK, BKC, false>(g, A, B, m0 + wm, n0 + wn, kBegin, it.kEnd, lane, acc);
+    if (flags->lost) {   // the same for the whole workgroup
+        if (split_large<BM, 64 * WVM * WVN, AK>(baseA, g.lda, M - m0, kBegin, it.kEnd, tid) || split_large<BN, 64 * WVM * WVN, BKC>(baseB, g.ldb, N - n0, kBegin, it.kEnd, tid))
+            flags->large = 1;
+        __syncthreads();
+    }
+    if (split_lost(acc, *flags, it.kEnd - kBegin)) f32_sums<WM, WN, AK, BKC, false>(g, A, B, m0 + wm, n0 + wn, kBegin, it.kEnd, lane, acc);
     else if (!VEC && kEnd < it.kEnd) f32_sums<WM, WN, AK, BKC, true>(g, A, B, m0 + wm, n0 + wn, kEnd, it.kEnd, lane, acc);
     f32_store<WM, WN, HEADS>(g, hp, acc, reinterpret_cast<float*>(smem_raw) + wave * 32 * (32 * WN + 4), lane, m0 + wm, n0 + wn, it.part, it.batch);
 }
@@ -1068,6 +1129,12 @@ static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal
     return c;
 }
 
+int gemm_f32_route(int m, int n, int k, int batch, bool causal, bool fp32Sums, bool heads)
+{
+    const GemmF32Choice c = gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, fp32Sums, heads);
+    return c.kernel + 4 * c.plan.shape + 64 * c.plan.splits;
+}
+
 // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
 static bool f32_near(bool kFast, int rows, int k, long long ld) { return (kFast ? (std::min(rows, 256) + 1) * ld : std::min(k, 128) * ld + 256) < (1ll << 29); }
 
@@ -1129,7 +1196,7 @@ template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, 
 static hipError_t launch_split(hipStream_t s, GemmF32Args& g, int splits, int batch, const HeadsEpilogue* he)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN;
-    constexpr int lds = 4 * split_lds<WVM, WVN, WM, WN, KS, AK, BKC>() + (SUMS ? 64 * WVM * WVN * 16 : 0);
+    constexpr int lds = split_flags_at<WVM, WVN, WM, WN, KS, AK, BKC, SUMS>() + (int)sizeof(SplitFlags);
     static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     g.tilesM = (g.M + BM - 1) / BM;

@@ -189,6 +189,7 @@ EXPORTS = (
     "DLL_InvokeFloatEx2", "DLL_InvokeDoubleEx2", "Internal_GetPointerFloat", "Internal_GetPointerDouble",
     "Internal_AllocHostFloat", "Internal_AllocHostDouble", "DLL_QueryStringFloatEx", "DLL_QueryStringDoubleEx",
     "MCH_TimeInvokeFloatEx2", "MCH_AttnDecodeForwardNoAlloc", "MCH_TimeInvokeFloatEx2Sets",
+    "MCH_GemmFloatRoute",
 )
 EXTENSION_EXPORTS = (
     "DLL_InitFloatCustomExtension", "DLL_InvokeFloatCustomExtension", "DLL_InvokeFloatCustomExtensionEx",
@@ -264,6 +265,8 @@ def load_library(path=None):
     lib.MCH_TimeInvokeFloatEx2Sets.restype = _c_long
     lib.MCH_AttnDecodeForwardNoAlloc.argtypes = [_c_long, _c_float_p, _c_long, _c_longlong_p, _c_long, _c_tchar_p, _c_long]
     lib.MCH_AttnDecodeForwardNoAlloc.restype = _c_long
+    lib.MCH_GemmFloatRoute.argtypes = [_c_long] * 5
+    lib.MCH_GemmFloatRoute.restype = _c_long
     return lib
 
 

@@ -17,6 +17,14 @@ SHAPES = [(2052, 4100, 68),      # two stages of two k-steps, the second short
           (16004, 388, 100), (580, 7000, 132), (1028, 1028, 612), (2056, 1544, 292), (8196, 2308, 76), (1000, 4, 140004)]
 
 
+def tile(m, n, k, batch=1, causal=False, heads=False):
+    """The number of the tile that the split kernel takes a product with; a test of that kernel means a size that goes there."""
+    from mycaffe_amd.cudadnn import load_library
+    route = load_library().MCH_GemmFloatRoute(m, n, k, batch, 1 * causal + 4 * heads)
+    assert route % 4 == 1, (m, n, k, batch, route)
+    return route // 4 % 16
+
+
 def check(got, a, b, rows, cols, alpha=1.0, add=0.0):
     a, b = a[rows].astype(np.float64), b[:, cols].astype(np.float64)
     k = a.shape[1]
@@ -86,6 +94,48 @@ def test_values_that_three_parts_do_not_hold(dev, tA, tB):
     assert fine[700].all() and fine[:, 100].sum() >= m - 5 and fine[641].sum() > n / 2
     # 2^-148: results that end among the denormals
     assert (np.abs(got[fine] - want[fine]) <= BOUND(k) * scale[fine] + 2.0 ** -148).all()
+
+
+# values below 2^-109, of which the parts lose bits or all, times ordinary and very large ones, in either operand
+@pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k,shape", [(4100, 3076, 292, 0), (3076, 3076, 292, 1), (1028, 4612, 580, 2), (2052, 1540, 612, 3), (2056, 1544, 292, 4),
+                                         (2055, 1029, 303, 5), (516, 260, 4100, 5)])
+def test_tiny_values_times_large_ones(dev, m, n, k, shape, tA, tB):
+    assert tile(m, n, k) == shape
+    rng = np.random.default_rng(m + k)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    p2 = lambda e: np.float32(2.0 ** e)  # noqa: E731
+    for v, w in ((a.T, b), (b, a.T)):      # columns of the one tiny, of the other large
+        v[:, 3] *= p2(-118)
+        v[:, 70] *= p2(-125)
+        v[:, 130] = (v[:, 130] * p2(-100)) * p2(-34)     # a few bits among the denormals
+        v[:, 171] = 0
+        v[min(7, k - 1), 171] = p2(-136)
+        v[:, 202] = (v[:, 202] * p2(-100)) * p2(-40)     # times 1: a result among the denormals
+        w[:, 250], w[:, 251], w[:, 252] = w[:, 250] * p2(60), w[:, 251] * p2(80), w[:, 252] * p2(100)
+    ha, hb, hc = dev.put((a.T if tA else a).copy()), dev.put((b.T if tB else b).copy()), dev.zeros(m * n)
+    dev.cuda.gemm(tA, tB, m, n, k, 1.0, ha, hb, 0.0, hc)
+    got, special = dev.get(hc, (m, n)), [3, 70, 130, 171, 202, 250, 251, 252]
+    for rows, cols in ((special, np.arange(n)), (np.arange(m), special), (sample(rng, m), sample(rng, n))):
+        at, a64, b64 = np.ix_(rows, cols), a[rows].astype(np.float64), b[:, cols].astype(np.float64)
+        want, scale = a64 @ b64, np.abs(a64) @ np.abs(b64)
+        fine = scale < 1e38
+        assert (np.abs(got[at][fine] - want[fine]) <= BOUND(k) * scale[fine] + k * 2.0 ** -149).all()
+
+
+# a tiny value in every tile beside ordinary ones: nothing is made over, and nothing has to be
+def test_a_stray_tiny_value_changes_nothing(dev):
+    m, n, k = 4100, 3076, 292
+    tile(m, n, k)
+    rng = np.random.default_rng(8)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    hb, out = dev.put(b), []
+    for tiny in (0.0, 2.0 ** -120, 2.0 ** -140):
+        a[::32, 5] = tiny
+        hc = dev.zeros(m * n)
+        dev.cuda.gemm(False, False, m, n, k, 1.0, dev.put(a), hb, 0.0, hc)
+        out.append(dev.get(hc, (m, n)))
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
 
 
 @pytest.mark.parametrize("B,T,H,hs,rope", [(3, 700, 12, 64, False), (2, 1024, 12, 64, True), (1, 2044, 6, 48, True)])
