@@ -1,5 +1,5 @@
 """fp32 products of 32 x 32 tiles (csrc/gemm_f32.hip, gemm_f32_small_kernel): edges of the tile, contractions around one, two and more
-stages of 128 k, batches, both ends of the causal ranges, the epilogues."""
+stages of 64 k, batches, both ends of the causal ranges, the epilogues."""
 import numpy as np
 import pytest
 
@@ -34,6 +34,14 @@ def test_batches(dev, outer, m, n, k, tA, tB):
     dev.cuda.matmul(outer, m, n, k, ha, hb, hc, 1.0, tA, tB)
     a, b = a.astype(np.float64), b.astype(np.float64)
     assert (np.abs(dev.get(hc, (outer, m, n)) - a @ b) <= BOUND(k) * (np.abs(a) @ np.abs(b))).all()
+
+
+@pytest.mark.parametrize("outer,T,hs", [(24, 256, 48), (3, 1023, 63), (30, 96, 40), (2, 33, 31)])
+def test_causal_operands(dev, outer, T, hs):
+    from mycaffe_amd.cudadnn import load_library
+    from tests.test_gpu_gemm_f32_split import causal_products
+    assert load_library().MCH_GemmFloatRoute(T, hs, T, outer, 1) % 4 == load_library().MCH_GemmFloatRoute(hs, T, T, outer, 1) % 4 == 2
+    causal_products(dev, outer, T, hs)
 
 
 @pytest.mark.parametrize("B,T,H,hs,rope", [(1, 33, 2, 16, False), (2, 30, 6, 48, True), (4, 256, 6, 48, True)])

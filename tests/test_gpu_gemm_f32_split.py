@@ -1,5 +1,6 @@
 """fp32 products on the bf16 matrix cores (csrc/gemm_f32.hip, gemm_f32_split_kernel) where they can go wrong: edges of every tile,
-contractions of one or two stages or that end inside one, parts of a contraction, values that three bf16 numbers do not hold."""
+contractions of one or two stages or that end inside one, parts of a contraction, batches and causal operands, values that three bf16
+numbers do not hold.  Which tile a size goes to is asked of the library, so that other estimates do not lead a test elsewhere."""
 import numpy as np
 import pytest
 
@@ -9,20 +10,22 @@ pytestmark = pytest.mark.gpu
 # walk, and never more than the running sum), and what the split leaves out (2^-25)
 BOUND = lambda k: 2.0 ** -24 * (2 + np.sqrt(6 * k / 16))  # noqa: E731
 
-# the smallest products taken (2^29 multiplications, 64 k) and what the estimate gives them
-SHAPES = [(2052, 4100, 68),      # two stages of two k-steps, the second short
-          (4100, 3076, 64),      # the shortest contraction, edges in both directions
-          (516, 260, 4100),      # parts
-          (132, 132, 32004),     # 32 parts of 64 x 64 tiles
-          (16004, 388, 100), (580, 7000, 132), (1028, 1028, 612), (2056, 1544, 292), (8196, 2308, 76), (1000, 4, 140004)]
+# from the smallest products taken (2^28 multiplications, 64 k), and the tile that the estimate gives them
+SHAPES = [(2052, 4100, 68, 3),      # five stages of one k-step, the last short
+          (4100, 3076, 64, 3),      # the shortest contraction, edges in both directions
+          (516, 260, 4100, 5),      # parts
+          (132, 132, 32004, 5),     # 28 parts of 64 x 64 tiles
+          (1000, 4, 140004, 5),     # 32
+          (4100, 3076, 292, 0), (3076, 3076, 292, 1), (1028, 4612, 580, 2), (2052, 1544, 612, 3), (2056, 1544, 292, 4), (1028, 1540, 292, 5),
+          (1028, 1028, 612, None),  # (32 x 32 tiles, gemm_f32_small_kernel)
+          (16004, 388, 100, 3), (580, 7000, 132, 3), (8196, 2308, 76, 3)]
 
 
 def tile(m, n, k, batch=1, causal=False, heads=False):
-    """The number of the tile that the split kernel takes a product with; a test of that kernel means a size that goes there."""
+    """The number of the tile that the split kernel takes a product with, None where another kernel does."""
     from mycaffe_amd.cudadnn import load_library
     route = load_library().MCH_GemmFloatRoute(m, n, k, batch, 1 * causal + 4 * heads)
-    assert route % 4 == 1, (m, n, k, batch, route)
-    return route // 4 % 16
+    return route // 4 % 16 if route % 4 == 1 else None
 
 
 def check(got, a, b, rows, cols, alpha=1.0, add=0.0):
@@ -37,8 +40,9 @@ def sample(rng, n):
 
 
 @pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False), (True, True)])
-@pytest.mark.parametrize("m,n,k", SHAPES)
-def test_edges(dev, m, n, k, tA, tB):
+@pytest.mark.parametrize("m,n,k,shape", SHAPES)
+def test_edges(dev, m, n, k, shape, tA, tB):
+    assert tile(m, n, k) == shape
     rng = np.random.default_rng(m + n + k)
     a, b, c = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (k, n), (m, n)))
     ha, hb = dev.put((a.T if tA else a).copy()), dev.put((b.T if tB else b).copy())
@@ -53,7 +57,8 @@ def test_edges(dev, m, n, k, tA, tB):
 def test_error_is_not_above_that_of_fp32_sums(dev):
     # against 64 bits, relative to a plain fp32 product's error at the same size
     rng = np.random.default_rng(3)
-    for m, n, k in ((2048, 4096, 64), (2048, 1024, 288), (1024, 1024, 768), (512, 256, 8192)):
+    for m, n, k, shape in ((2048, 4096, 64, 3), (2048, 1024, 288, 5), (2048, 1536, 768, 5), (1024, 1024, 768, None), (512, 256, 8192, 5)):
+        assert tile(m, n, k) == shape
         a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
         hc = dev.zeros(m * n)
         dev.cuda.gemm(False, True, m, n, k, 1.0, dev.put(a), dev.put(b), 0.0, hc)
@@ -67,14 +72,15 @@ def test_error_is_not_above_that_of_fp32_sums(dev):
 
 
 @pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False)])
-def test_values_that_three_parts_do_not_hold(dev, tA, tB):
+@pytest.mark.parametrize("m,n,k,shape", [(1028, 1540, 612, 5), (2056, 1544, 292, 4), (4100, 3076, 292, 0), (1028, 1028, 612, None)])
+def test_values_that_three_parts_do_not_hold(dev, m, n, k, shape, tA, tB):
+    assert tile(m, n, k) == shape
     rng = np.random.default_rng(9)
-    m, n, k = 1028, 1028, 612
     a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
     b[0] = np.where(rng.random(n) < 0.5, 0, 1).astype(np.float32)     # infinities times zero as well
     b[:, 5] = np.abs(b[:, 5])
     big = np.float32(3.4e38)                            # above the largest bf16 number
-    a[3, 0], a[200, 7], a[1027, 611], a[640, 10] = np.inf, np.nan, -np.inf, big
+    a[3, 0], a[200, 7], a[1027, k - 1], a[640, 10] = np.inf, np.nan, -np.inf, big
     a[641, :] = 0
     a[641, 20] = big
     a[700], a[701] = a[700] * np.float32(2.0 ** -120), 0                  # below what the third part holds; zeros
@@ -126,7 +132,7 @@ def test_tiny_values_times_large_ones(dev, m, n, k, shape, tA, tB):
 # a tiny value in every tile beside ordinary ones: nothing is made over, and nothing has to be
 def test_a_stray_tiny_value_changes_nothing(dev):
     m, n, k = 4100, 3076, 292
-    tile(m, n, k)
+    assert tile(m, n, k) == 0
     rng = np.random.default_rng(8)
     a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
     hb, out = dev.put(b), []
@@ -178,8 +184,12 @@ def test_fp32_sums_on_request(dev):
 
 
 # the strided products of the attention chain: a batch, and neither operand's nor the result's rows next to each other
-@pytest.mark.parametrize("outer,m,n,k,tA,tB", [(48, 256, 64, 1020, False, False), (24, 516, 516, 100, False, True), (40, 260, 68, 1000, True, False)])
-def test_batches(dev, outer, m, n, k, tA, tB):
+# (neither transposed: on the fp32 matrix cores, see k_gemm2)
+@pytest.mark.parametrize("tA,tB", [(False, True), (True, False), (True, True), (False, False)])
+@pytest.mark.parametrize("outer,m,n,k,shape", [(48, 256, 64, 1020, None), (40, 260, 68, 1000, None), (4, 2052, 1540, 612, 0), (5, 2048, 772, 292, 1), (47, 515, 133, 515, 2), (24, 516, 516, 100, 3), (9, 1027, 1029, 301, 3),
+                                               (40, 260, 292, 516, 5)])
+def test_batches(dev, outer, m, n, k, shape, tA, tB):
+    assert tile(m, n, k, outer) == shape
     rng = np.random.default_rng(outer)
     a, b = rng.standard_normal((outer, m, k), dtype=np.float32), rng.standard_normal((outer, k, n), dtype=np.float32)
     ha, hb = dev.put((a.transpose(0, 2, 1) if tA else a).copy()), dev.put((b.transpose(0, 2, 1) if tB else b).copy())
@@ -188,3 +198,30 @@ def test_batches(dev, outer, m, n, k, tA, tB):
     got = dev.get(hc, (outer, m, n))
     for i in (0, outer // 2, outer - 1):
         check(got[i], a[i], b[i], np.arange(m), np.arange(n))
+
+
+def causal_products(dev, outer, T, hs):
+    """P^T dY and V P^T for softmax weights P whose zeros above the diagonal the library knows of, against 64 bits."""
+    cuda, rng = dev.cuda, np.random.default_rng(T)
+    sc, v = rng.standard_normal((outer, T, T), dtype=np.float32), rng.standard_normal((outer, T, hs), dtype=np.float32)
+    hp, hsc, hm = dev.zeros(sc.size), dev.put(sc), dev.put(np.tril(np.ones((T, T), np.float32)))
+    hc, d = cuda.CreateCuDNN(), cuda.CreateTensorDesc()
+    cuda.SetTensorDesc(d, outer * T, T, 1, 1, False)
+    cuda.mask(sc.size, T * T, 0.0, -1e9, hsc, hm, hsc)
+    cuda.SoftmaxForward(hc, 1, 0, 1.0, d, hsc, 0.0, d, hp)
+    hout = dev.zeros(v.size)
+    cuda.matmul(outer, T, hs, T, hp, dev.put(v), hout, 1.0, True, False)
+    left = dev.get(hout, v.shape)
+    cuda.matmul(outer, hs, T, T, dev.put(v.transpose(0, 2, 1).copy()), hp, hout, 1.0, False, True)
+    right = dev.get(hout, (outer, hs, T))
+    p = dev.get(hp, sc.shape)
+    assert (np.triu(p[0], 1) == 0).all()
+    for i in (0, outer // 2, outer - 1):
+        check(left[i], p[i].T, v[i], np.arange(T), np.arange(hs))
+        check(right[i], v[i].T, p[i].T, np.arange(hs), np.arange(T))
+
+
+@pytest.mark.parametrize("outer,T,hs,left,right", [(48, 516, 132, 2, 4), (24, 1028, 64, 5, 5), (24, 1027, 67, 3, 3)])
+def test_causal_operands(dev, outer, T, hs, left, right):
+    assert tile(T, hs, T, outer, causal=True) == left and tile(hs, T, T, outer, causal=True) == right
+    causal_products(dev, outer, T, hs)
