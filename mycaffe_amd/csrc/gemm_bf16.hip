@@ -732,6 +732,11 @@ static GemmB16Plan gemm_b16_plan(int m, int n, int k, int shares = B16_APART, in
     }
     return best.splits ? best : gemm_b16_plan(m, n, k, B16_APART, maxParts);
 }
+int gemm_b16_route(int m, int n, int k)
+{
+    const GemmB16Plan p = gemm_b16_plan(m, n, k);
+    return 4 * p.shape + 64 * p.splits;
+}
 
 bool gemm_b16_takes(const GemmB16& q)
 {

@@ -1,5 +1,6 @@
-"""The 16-bit GEMM kernel (csrc/gemm_bf16.hip) where it can go wrong: edges of each of its tiles, contractions that end inside a
-stage, every operand layout, contractions cut into parts, beta, and the bias and head-layout epilogues."""
+"""The 16-bit GEMM kernel (csrc/gemm_bf16.hip) where it can go wrong: edges of each of its tiles (which of them a size goes to is asked of
+the library), contractions that end inside a stage, every operand layout, contractions cut into parts, beta, and the bias and
+head-layout epilogues."""
 import numpy as np
 import pytest
 
@@ -26,6 +27,24 @@ def test_gemm_edges(dev, m, n, k, tA, tB):
         ref = alpha * want + beta * c
         err = np.abs(dev.get(hc, (m, n)) - ref)
         assert (err <= 2.0 ** -8 * np.abs(ref) + 1e-5 * np.abs(ref).max()).all(), err.max()
+
+
+def tile(m, n, k):
+    """The number of the tile that the library takes for these sizes, and the parts of the contraction."""
+    from mycaffe_amd.cudadnn import load_library
+    route = load_library().MCH_GemmFloatRoute(m, n, k, 1, 8)
+    return route // 4 % 16, route // 64
+
+
+# every tile with edges, and those that parts of a contraction get
+@pytest.mark.parametrize("tA,tB", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k,shape,parts", [(6152, 2312, 72, 0, 1), (3080, 4104, 136, 0, 1), (8008, 1032, 520, 1, 1), (4104, 4104, 520, 2, 1), (8008, 520, 520, 3, 1),
+                                               (8008, 264, 72, 4, 1), (2056, 1032, 1544, 5, 1), (2056, 1032, 776, 6, 1), (8200, 72, 72, 7, 1), (72, 72, 136, 8, 1),
+                                               (264, 6152, 72, 9, 1), (6152, 136, 4104, 3, 5), (8200, 72, 4104, 5, 3), (136, 6152, 4104, 6, 3), (72, 3080, 2056, 7, 5),
+                                               (72, 72, 1032, 8, 4), (136, 3080, 4104, 9, 6)])
+def test_every_tile(dev, m, n, k, shape, parts, tA, tB):
+    assert tile(m, n, k) == (shape, parts)
+    test_gemm_edges(dev, m, n, k, tA, tB)
 
 
 @pytest.mark.parametrize("bias", [False, True])
@@ -57,3 +76,12 @@ def test_projection_into_heads_edges(dev, B, T, H, hs, rope, half):
         assert np.abs(got - want).max() <= (2.0 ** -7 if half else 1e-4 if rope else 4e-6) * np.abs(ref).max()
     if hr:
         dev.cuda.FreeRope(hr)
+
+
+# the ends in heads of every tile, with a rotation and without
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("B,T,H,hs,shape", [(3, 2100, 11, 64, 0), (3, 2100, 11, 40, 1), (3, 2100, 5, 64, 2), (2, 1366, 8, 64, 3), (3, 2100, 3, 40, 4), (3, 171, 20, 64, 5),
+                                            (3, 333, 8, 96, 6), (3, 1366, 3, 24, 7), (2, 65, 3, 40, 8), (3, 2100, 2, 24, 9)])
+def test_projection_into_heads_of_every_tile(dev, B, T, H, hs, shape, rope):
+    assert tile(B * T, 3 * H * hs, H * hs) == (shape, 1)
+    test_projection_into_heads_edges(dev, B, T, H, hs, rope, True)

@@ -35,12 +35,15 @@ def get(dev, h, n, half):
     return dev.get(h)
 
 
-# by the estimate: 64 x 64 tiles, 64 x 128, 128 x 128, 128 x 192 on eight wavefronts, 256 x 192 and larger; sizes without whole tiles;
-# a head size that 16-byte pieces do not divide; too few rows for one launch; fp32
+# by the estimate, in this order: 256 x 192 tiles, 64 x 64, 128 x 128 with two stages, 64 x 128 with two, the same, 256 x 256, 64 x 64 twice, fp32;
+# 128 x 192 on four wavefronts and on eight, 128 x 128 and 64 x 128 with three stages, 128 x 64.  Among them sizes without whole tiles, a
+# head size that 16-byte pieces do not divide and too few rows for one launch
 @pytest.mark.parametrize("N,K,heads,rows,half", [
     (512, 512, 8, [(4096, 128), (8192, 256), (8192, 256)], True), (256, 256, 4, [(2000, 50), (1000, 40)], True), (768, 768, 12, [(1030, 103), (4100, 100), (3000, 30)], True),
     (512, 512, 8, [(2048, 64), (2048, 64), (2048, 64)], True), (384, 64, 32, [(5000, 100), (77, 7), (1, 1)], True), (1024, 1024, 16, [(8192, 512), (8192, 512)], True),
-    (512, 512, 8, [(40, 20), (60, 30)], True), (72, 40, 8, [(130, 13), (65, 5)], True), (96, 96, 6, [(130, 13), (65, 5), (33, 33)], False)])
+    (512, 512, 8, [(40, 20), (60, 30)], True), (72, 40, 8, [(130, 13), (65, 5)], True), (96, 96, 6, [(130, 13), (65, 5), (33, 33)], False),
+    (1536, 264, 24, [(6000, 100), (2056, 8)], True), (512, 520, 8, [(4104, 27), (4104, 108)], True), (96, 2056, 4, [(8200, 41), (8200, 200)], True),
+    (96, 1032, 6, [(8200, 200), (8200, 41)], True), (160, 64, 4, [(4104, 54), (4104, 57)], True)])
 def test_projections(dev, N, K, heads, rows, half):
     for bias in (True, False):
         calls, want = run(dev, N, K, heads, rows, half, bias)

@@ -1,5 +1,5 @@
 """16-bit products whose tiles keep three and four stages in LDS (csrc/gemm_bf16.hip, b16_tile with S > 2): contractions shorter than the
-stages, that end inside one, one stage more than the ring; sizes of every tile with edges; all layouts."""
+stages, that end inside one, one stage more than the ring; sizes with edges for each of these tiles; all layouts."""
 import numpy as np
 import pytest
 

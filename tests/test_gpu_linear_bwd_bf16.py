@@ -3,6 +3,8 @@ contractions cut and not, edges, more stages than turns and fewer; gradients add
 import numpy as np
 import pytest
 
+from tests.test_gpu_gemm_bf16 import tile
+
 pytestmark = pytest.mark.gpu
 
 
@@ -18,10 +20,12 @@ def get(dev, h, shape):
 
 
 # rows, outputs, inputs
-@pytest.mark.parametrize("m,n,k", [
-    (1025, 8, 8), (1032, 64, 72), (2000, 96, 200), (8000, 768, 3072), (8000, 3072, 768), (1100, 4096, 1024), (4104, 1000, 264), (1500, 2304, 768),
-    (1030, 8192, 4096), (20000, 40, 24), (1088, 50, 64)])
-def test_gradients(dev, m, n, k):
+@pytest.mark.parametrize("m,n,k,shape", [
+    (1025, 8, 8, 8), (1032, 64, 72, 8), (2000, 96, 200, 8), (8000, 768, 3072, 4), (8000, 3072, 768, 4), (1100, 4096, 1024, 6), (4104, 1000, 264, 8), (1500, 2304, 768, 7),
+    (1030, 8192, 4096, 0), (20000, 40, 24, 8), (1088, 50, 64, 8), (1032, 8200, 1032, 1), (1032, 4104, 4104, 2), (1032, 1032, 4104, 3), (4104, 6152, 136, 3),
+    (8200, 72, 4104, 5), (2056, 72, 3080, 7), (4104, 136, 3080, 9)])
+def test_gradients(dev, m, n, k, shape):
+    assert tile(n, k, m)[0] == shape
     rng = np.random.default_rng(m + n)
     x, w, dy, dw, db = (round_bf16(rng.standard_normal(s, dtype=np.float32)) for s in ((m, k), (n, k), (m, n), (n, k), (n,)))
     hx, hw, hdy, hdw, hdb = (dev.cuda.AllocMemory(a, bHalfSize=True) for a in (x, w, dy, dw, db))

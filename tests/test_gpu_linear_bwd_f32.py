@@ -3,14 +3,18 @@ contractions cut and not, edges, more stages than turns and fewer, an odd number
 import numpy as np
 import pytest
 
+from tests.test_gpu_gemm_f32_split import tile
+
 pytestmark = pytest.mark.gpu
 
 
 # rows, outputs, inputs
-@pytest.mark.parametrize("m,n,k", [
-    (1032, 640, 640), (1000, 512, 1024), (700, 1024, 1024), (2001, 516, 260), (8000, 768, 3072), (8000, 3072, 768), (4100, 2304, 768), (1500, 4096, 1024),
-    (20000, 132, 132), (1048, 8192, 4096), (5000, 1024, 64), (70, 4096, 4096)])
-def test_gradients(dev, m, n, k):
+@pytest.mark.parametrize("m,n,k,shape", [
+    (1032, 640, 640, None), (1000, 512, 1024, None), (700, 1024, 1024, None), (2001, 516, 260, None), (8000, 768, 3072, 0), (8000, 3072, 768, 0), (4100, 2304, 768, 1),
+    (1500, 4096, 1024, 3), (20000, 132, 132, 5), (1048, 8192, 4096, 0), (5000, 1024, 64, 5), (70, 4096, 4096, 3), (1028, 1028, 4100, 2), (4100, 136, 4100, 4),
+    (4100, 516, 136, 5)])   # None: 32 x 32 tiles
+def test_gradients(dev, m, n, k, shape):
+    assert tile(n, k, m) == shape
     rng = np.random.default_rng(m + n)
     x, w, dy, dw, db = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (n, k), (m, n), (n, k), (n,)))
     hx, hw, hdy, hdw, hdb = (dev.put(a) for a in (x, w, dy, dw, db))
