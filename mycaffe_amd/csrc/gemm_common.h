@@ -262,7 +262,7 @@ struct GemmF32 {
     int epoch;
     const float* bias;                     // null, or n values added to every row of C (batch 1)
     const HeadsEpilogue* heads;            // written through this epilogue instead of to C (alpha 1, beta 0, batch 1, bias null)
-    bool fp32Sums;                         // on the fp32 matrix cores, one value of k after the other, whatever the size
+    bool fp32Sums;                         // on the fp32 matrix cores, the k in order, whatever the size (gemm_f32_kernel)
     float* rowSum;                         // (m) += the sums of op(A)'s rows; dense operands, both with their rows at unit stride
 };
 enum { CAUSAL_NO = 0, CAUSAL_A_LOWER /* A(i,k) zero for k > i */, CAUSAL_A_UPPER /* k < i */, CAUSAL_B_LOWER /* B(k,j) zero for k < j */, CAUSAL_B_UPPER /* k > j */ };

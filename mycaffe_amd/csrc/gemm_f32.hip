@@ -383,8 +383,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_kernel(GemmF32Args g, Heads
 // infinity or anything nonzero below 2^-90, or if a value of the workgroup's operands lost bits and either some value is 2^16 or more (for which
 // they are then read once more) or a sum, zeros among them, is so small that k products with up to 2^16 times those bits may be 2^-25 of
 // it.  So an ordinary tile beside a stray tiny value (GELU of -10) is not made over: 8192 x 3072 x 768 with one in every tile takes 280 us, 218
-// without, 570 with a row of zeros beside one.  (Looking for lost bits takes 1 % of an ordinary product; keeping the largest value
-// along too, for the second reading, 2 - 3 %.)
+// without, 570 with a row of zeros beside one.  (Looking for lost bits takes 1 - 2 % of an ordinary product under lasting load and 4 % in the
+// first launches after a pause, whose clock is not at its limit yet; to keep the largest value along, and read nothing again, took 2 - 3 %.)
 //
 // What bounds it is power: at 8192 x 3072 x 768 operands of zeros take 136 us in 128 x 192 tiles, random ones 197 (same instructions), so what
 // helps is fewer instructions and bytes per product.  Values are split once, on their way from registers to LDS (splitting whole
@@ -413,9 +413,9 @@ __device__ __forceinline__ uint2 split_part(float (&v)[4], bool last)
     return p;
 }
 
-// written as an instruction, in its place: the compiler would gather those of a stage at its end, and keep the values until then (14
-// registers; 256 x 256 tiles spill)
-__device__ __forceinline__ void or3(uint32_t& m, uint32_t a, uint32_t b) { asm volatile("v_or3_b32 %0, %0, %1, %2" : "+v"(m) : "v"(a), "v"(b)); }
+// written as an instruction: the compiler would gather those of a stage at its end, and keep the values until then (14 registers; 256 x 256
+// tiles spill)
+__device__ __forceinline__ void or3(uint32_t& m, uint32_t a, uint32_t b) { asm("v_or3_b32 %0, %0, %1, %2" : "+v"(m) : "v"(a), "v"(b)); }
 
 // what the workgroup's wavefronts leave in LDS for each other: whether a value lost bits, and whether one is LARGE or more
 struct SplitFlags { uint32_t lost, large; };
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
 // an instruction.  Stages of 128 k, two workgroups to a CU: 768 x 768 x 700 15.5 instead of 12.5 us, the same where every CU has
 // one; eight wavefronts, five stages, fragments read a stage ahead: no better.
 // Measured, before and now, us: 1024 x 288 x 288 8.7 -> 5.8, 1024 x 288 x 768 12.6 -> 9.9, 768 x 288 x 1024 (A^T B, beta 1) 13.3 -> 8.7,
-// 768 x 768 x 700 (A^T B) 17.1 -> 12.6, 24 times 256 x 48 x 256 8.0 -> 5.5 (causal 8.1 -> 4.9), 96 x 192 x 48 4.4 -> 2.9.
+// 768 x 768 x 700 (A^T B) 17.1 -> 12.6, 24 times 256 x 48 x 256 with a transposed operand 8.3 -> 5.7, 96 x 192 x 48 4.4 -> 2.9.
 //
 // LDS holds [row][k] for an operand with k at unit stride, the 16-byte piece c of row r at c ^ (r & 15), and [k][row] for the other,
 // k and k + 4 of every eight next to each other: the two halves of a wavefront, four k apart, then read from the two halves of the banks.
