@@ -183,23 +183,18 @@ template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dq_rows_ke
     attn_bwd_dq_row<T>(a, blockIdx.z, blockIdx.y, row, a.lse2[at], a.dsum[at], qs[wave], gs[wave]);
 }
 
-// dK, dV: one wavefront per key row, lanes over queries
-template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dkv_rows_kernel(AttnBwdArgs a)
+// dK, dV: one key row by one wavefront, lanes over queries; ks, vs: hs floats of LDS each of its own
+template <typename T> __device__ __forceinline__ void attn_bwd_dkv_row(const AttnBwdArgs& a, int b, int h, int key, float* ks, float* vs)
 {
     constexpr int DPL = 4;
-    __shared__ float ks[4][256], vs[4][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int key = blockIdx.x * 4 + wave;
-    const int h = blockIdx.y, b = blockIdx.z;
-    const bool valid = key < a.Tk;
+    const int lane = own_lane();
     const size_t bh = (size_t)b * a.H + h;
-    const size_t ko = (bh * a.Tk + (valid ? key : 0)) * a.hs;
+    const size_t ko = (bh * a.Tk + key) * a.hs;
     for (int d = lane; d < a.hs; d += 64) {
-        ks[wave][d] = ldb((const T*)a.k + ko, d) * a.scale;
-        vs[wave][d] = ldb((const T*)a.v + ko, d);
+        ks[d] = ldb((const T*)a.k + ko, d) * a.scale;
+        vs[d] = ldb((const T*)a.v + ko, d);
     }
-    __syncthreads();
-    if (!valid) return;
+    wave_lds_fence();
     const T* q = (const T*)a.q + bh * a.Tq * a.hs;
     const T* g = (const T*)a.dy + bh * a.Tq * a.hs;
     const float* lse = a.lse2 + bh * a.Tq;
@@ -216,8 +211,8 @@ template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dkv_rows_k
             const T* gr = g + (size_t)i * a.hs;
             float s = 0.f, dp = 0.f;
             for (int d = 0; d < a.hs; d++) {
-                s += ks[wave][d] * ldb(qr, d);
-                dp += vs[wave][d] * ldb(gr, d);
+                s += ks[d] * ldb(qr, d);
+                dp += vs[d] * ldb(gr, d);
             }
             p = attn_prob(s, attn_masked(a, b, i, key), lse[i], uniform);
             float pf, sf;
@@ -247,6 +242,12 @@ template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dkv_rows_k
             stb((T*)a.dv + ko, d, accV[t]);
         }
     }
+}
+template <typename T> __global__ __launch_bounds__(256) void attn_bwd_dkv_rows_kernel(AttnBwdArgs a)
+{
+    __shared__ float ks[4][256], vs[4][256];
+    const int wave = threadIdx.x >> 6, key = blockIdx.x * 4 + wave;
+    if (key < a.Tk) attn_bwd_dkv_row<T>(a, blockIdx.z, blockIdx.y, key, ks[wave], vs[wave]);
 }
 
 bool attn_bwd_mfma_usable(DType dt, const AttnBwdArgs& a);
@@ -342,12 +343,14 @@ template <int KIND> __device__ inline bool bwd_masked(const AttnBwdArgs& a, int 
 
 // KIND: 0 none, 1 causal, 2 key mask (B,Tk), 3 mask (B,Tq,Tk) or, with mb = 0, one (Tq,Tk) mask for all sequences
 // PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 54 us
-// here and 47 for dq; the row kernels 671 and 450).  Infinities and NaN: as in flash_fwd_kernel, a wavefront whose sums for dq are not
-// finite does its queries over row by row.  dK and dV need that not: what a masked query has to add NaN to them, an infinity in its row of
-// Q or dY, makes its D infinite or NaN, by which the row kernel adds NaN too.
+// here and 47 for dq; the row kernels 671 and 450).  Infinities and NaN: as in flash_fwd_kernel, a wavefront whose sums are not finite does
+// its queries, or keys, over row by row.
+// PARTS: in 16-bit storage probabilities and their gradients go into the products as two bf16 numbers each, which keeps the precision
+// the row kernels had for these head sizes (error of dq, 48 wide, 300 positions: 1.8e-3 so, 2.5e-3 with one bf16 number each).
 template <typename T, int HS, int KIND, int BQ, int OCC, bool PADDED>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs a, int mb)
 {
+    constexpr bool PARTS = PADDED && sizeof(T) == 2;
     typedef BwdTile<T, HS, BQ> TL;
     typedef FlashTraits<T> TR;
     constexpr int NW = 4, BK = NW * 32;
@@ -485,14 +488,18 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
 #pragma unroll
                 for (int t = 0; t < PF; t++) {
                     const u32x4 pp = TR::pack_p(s, t), dd = TR::pack_p(dp, t);
+                    [[maybe_unused]] u32x4 pr, dr;
+                    if constexpr (PARTS) { pr = TR::pack_rest(s, t, pp); dr = TR::pack_rest(dp, t, dd); }
 #pragma unroll
                     for (int dt = 0; dt < DT; dt++) {
                         const u32x4 gt = TL::TRR ? TR::load_vt_rowmajor(&Gs[32 * sub * LDR + dt * 32], LDR, t, lane)
                                                  : TR::load_vt(&Gt[(dt * 32 + l32) * LDT + 32 * sub], t, half);
                         av[dt] = TR::mma(gt, pp, av[dt]);
+                        if constexpr (PARTS) av[dt] = TR::mma(gt, pr, av[dt]);
                         const u32x4 qt = TL::TRR ? TR::load_vt_rowmajor(&Qs[32 * sub * LDR + dt * 32], LDR, t, lane)
                                                  : TR::load_vt(&Qt[(dt * 32 + l32) * LDT + 32 * sub], t, half);
                         ak[dt] = TR::mma(qt, dd, ak[dt]);
+                        if constexpr (PARTS) ak[dt] = TR::mma(qt, dr, ak[dt]);
                     }
                 }
             }
@@ -500,6 +507,19 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
         __syncthreads();
         if (more) sstore();
         __syncthreads();
+    }
+    if constexpr (PADDED) {
+        float sum = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) sum += fabsf(ak[dt][v]) + fabsf(av[dt][v]);
+        if (waveActive && __any(!(sum < INFINITY))) {
+            const int waveId = __builtin_amdgcn_readfirstlane(wave), first = kblock * BK + waveId * 32;
+            float* own = (float*)bwd_smem + waveId * 2 * HS;
+            for (int r = first; r < min(first + 32, a.Tk); r++) attn_bwd_dkv_row<T>(a, b, h, r, own, own + HS);
+            return;
+        }
     }
     // dk[key, d] = scale * dK^T[d, key]; register v of tile dt is d = 32*dt + 8*(v/4) + 4*half + v%4
     if (waveActive && key < a.Tk) {
@@ -521,6 +541,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
 template <typename T, int HS, int KIND, int BKS, int OCC, bool PADDED>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs a, int mb)
 {
+    constexpr bool PARTS = PADDED && sizeof(T) == 2;
     typedef BwdTile<T, HS, BKS> TL;
     typedef FlashTraits<T> TR;
     constexpr int NW = 4, BM = NW * 32;
@@ -649,11 +670,14 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
 #pragma unroll
                 for (int t = 0; t < PF; t++) {
                     const u32x4 dd = TR::pack_p(dp, t);
+                    [[maybe_unused]] u32x4 dr;
+                    if constexpr (PARTS) dr = TR::pack_rest(dp, t, dd);
 #pragma unroll
                     for (int dt = 0; dt < DT; dt++) {
                         const u32x4 kt = TL::TRR ? TR::load_vt_rowmajor(&Ks[32 * sub * LDR + dt * 32], LDR, t, lane)
                                                  : TR::load_vt(&Kt[(dt * 32 + l32) * LDT + 32 * sub], t, half);
                         aq[dt] = TR::mma(kt, dd, aq[dt]);
+                        if constexpr (PARTS) aq[dt] = TR::mma(kt, dr, aq[dt]);
                     }
                 }
             }

@@ -230,10 +230,13 @@ __device__ __forceinline__ void flash_softmax_step(floatx16 (&s)[QT], floatx16 (
 // PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 33 us;
 // the kernel with a wavefront per row, which had these, 546).  A key that a row does not see has weight zero here and is not read there, which
 // differs where it holds an infinity or a NaN: a wavefront whose sums are not finite does its rows over as that kernel does.
+// PARTS: in 16-bit storage the weights go into the product with V as two bf16 numbers each, which keeps the precision these head sizes
+// had there (48 wide, 300 positions: error of y 1.57e-3, all of it the rounding of y; 1.99e-3 with one bf16 number each).
 template <typename T, int HS, int KIND, int QT, int NW, int OCC, bool PREFETCH, bool PADDED>
 __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
 {
     typedef FlashTraits<T> TR;
+    constexpr bool PARTS = PADDED && sizeof(T) == 2;
     constexpr int NT = NW * 64, BM = NW * 32 * QT, BN = 64;
     constexpr int EPC = TR::EPC, CPF = TR::CPF;
     constexpr int KF = HS / CPF;              // fragments along the head dimension (S^T contraction)
@@ -443,10 +446,14 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
                 }
                 // O^T += V^T P^T
                 u32x4 pf[QT][PF];
+                [[maybe_unused]] u32x4 pr[QT][PF];
 #pragma unroll
                 for (int qt = 0; qt < QT; qt++) {
 #pragma unroll
-                    for (int t = 0; t < PF; t++) pf[qt][t] = TR::pack_p(s[qt], t);
+                    for (int t = 0; t < PF; t++) {
+                        pf[qt][t] = TR::pack_p(s[qt], t);
+                        if constexpr (PARTS) pr[qt][t] = TR::pack_rest(s[qt], t, pf[qt][t]);
+                    }
                 }
 #pragma unroll
                 for (int t = 0; t < PF; t++)
@@ -455,7 +462,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
                         const u32x4 vf = VROW ? TR::load_vt_rowmajor(&Vt[32 * sub * LDVR + dt * 32], LDVR, t, lane)
                                               : TR::load_vt(&Vt[(dt * 32 + l32) * LDV + 32 * sub], t, half);
 #pragma unroll
-                        for (int qt = 0; qt < QT; qt++) o[dt][qt] = TR::mma(vf, pf[qt][t], o[dt][qt]);
+                        for (int qt = 0; qt < QT; qt++) {
+                            o[dt][qt] = TR::mma(vf, pf[qt][t], o[dt][qt]);
+                            if constexpr (PARTS) o[dt][qt] = TR::mma(vf, pr[qt][t], o[dt][qt]);
+                        }
                     }
             }
         }

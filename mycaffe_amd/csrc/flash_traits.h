@@ -66,6 +66,12 @@ template <> struct FlashTraits<bf16_t> {
         return u32x4{pack_bf16x2(p[8 * t], p[8 * t + 1]), pack_bf16x2(p[8 * t + 2], p[8 * t + 3]),
                      pack_bf16x2(p[8 * t + 4], p[8 * t + 5]), pack_bf16x2(p[8 * t + 6], p[8 * t + 7])};
     }
+    // what pack_p's fragment leaves of them: with both, sixteen bits of a weight
+    __device__ static inline u32x4 pack_rest(const floatx16& p, int t, u32x4 w)
+    {
+        auto rest = [&](int i, uint32_t x) { return pack_bf16x2(p[8 * t + 2 * i] - __uint_as_float(x << 16), p[8 * t + 2 * i + 1] - __uint_as_float(x & 0xffff0000u)); };
+        return u32x4{rest(0, w.x), rest(1, w.y), rest(2, w.z), rest(3, w.w)};
+    }
     // sum of the eight products of two fragments
     __device__ static inline float dot(u32x4 a, u32x4 b)
     {
@@ -113,6 +119,7 @@ template <> struct FlashTraits<float> {
         return u32x4{__float_as_uint(p[4 * t]), __float_as_uint(p[4 * t + 1]), __float_as_uint(p[4 * t + 2]),
                      __float_as_uint(p[4 * t + 3])};
     }
+    __device__ static inline u32x4 pack_rest(const floatx16&, int, u32x4) { return u32x4{0u, 0u, 0u, 0u}; }   // 16-bit storage only
     __device__ static inline float dot(u32x4 a, u32x4 b)
     {
         return __uint_as_float(a.x) * __uint_as_float(b.x) + __uint_as_float(a.y) * __uint_as_float(b.y) +

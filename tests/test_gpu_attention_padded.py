@@ -98,3 +98,22 @@ def test_infinity_in_the_last_gradient(dev, hs, half):
     want[0, 1, :, 2] = np.inf
     fine = np.isfinite(want)
     assert np.array_equal(dv[~fine], want[~fine].astype(np.float32)) and np.abs(dv[fine] - want[fine]).max() <= (BF16_RTOL if half else FP32_RTOL) * np.abs(want[fine]).max()
+
+
+# 16-bit storage: weights and their gradients keep more than sixteen bits between the products, so that rounding the result is all that shows
+@pytest.mark.parametrize("hs", [8, 16, 32, 48, 80, 96, 120])
+@pytest.mark.parametrize("T,causal", [(64, True), (300, True), (300, False), (1000, True)])
+def test_weights_keep_their_bits(dev, T, causal, hs):
+    rng = np.random.default_rng(hs + T)
+    q, k, v, dy = (bf16_round(rng.standard_normal((2, 2, T, hs)).astype(np.float32)) for _ in range(4))
+    mask = R.causal_mask(T) if causal else None
+    out = _fwd_bwd(dev, q, k, v, dy, mask, 0, True)
+    q, k, v, dy = (a.astype(np.float64) for a in (q, k, v, dy))
+    p = _probs(q, k, mask, 0)
+    t = lambda a: np.swapaxes(a, -1, -2)  # noqa: E731
+    ds = p * (dy @ t(v) - (out[0].astype(np.float64) * dy).sum(-1, keepdims=True)) / np.sqrt(hs)   # D from the result as it is stored
+    norm = lambda a: np.sqrt((a ** 2).sum())  # noqa: E731
+    for got, want in zip(out, (p @ v, ds @ k, t(ds) @ q, t(p) @ dy)):
+        rounding = norm(bf16_round(want.astype(np.float32)) - want)
+        # two roundings of 2^-17 and fp32 sums beside one of 2^-9: 1.0001; a weight rounded to 16 bits adds its own 2^-9 (1.2 - 1.4)
+        assert norm(got - want) <= 1.002 * rounding
