@@ -1166,7 +1166,7 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
             }
             if (known) {
                 e.args = a;
-                if (m_permuteCache.size() >= 64) m_permuteCache.erase(m_permuteCache.begin());
+                if (m_permuteCache.size() >= KEPT_ANSWERS) m_permuteCache.erase(m_permuteCache.begin());
                 m_permuteCache.push_back(e);
             }
         }

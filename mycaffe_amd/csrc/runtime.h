@@ -143,6 +143,9 @@ struct PendingProduct {
     long long sA = 0, sB = 0, sC = 0;
     float alpha = 1.f;
 };
+// answers that take a read-back from the device, kept per content (a version is given to one content only); the oldest goes first
+constexpr size_t KEPT_ANSWERS = 512;
+struct HeldMaskEntry { long handle; uint64_t version; int T; bool causal; };
 struct OnesCacheEntry { uint64_t version = 0; int n = 0; bool ones = false; };
 struct PermuteCacheEntry { uint64_t key[6]; int axes; PermuteArgs args; };
 struct ExtensionState {
@@ -199,7 +202,7 @@ private:
     // host read-back per content of a handle (a model has one such blob per inner product)
     bool vector_is_ones(long h, MemItem* v, int n);
     std::unordered_map<long, OnesCacheEntry> m_onesCache;
-    long m_heldMaskHandle = 0; uint64_t m_heldMaskVersion = 0; int m_heldMaskT = 0; bool m_heldMaskCausal = false;
+    std::vector<HeldMaskEntry> m_heldMasks;
     // Tensors whose entries above the diagonal of every (len, len) matrix are exact zeros: outputs of a softmax with a causal
     // mask folded in, and their gradients.  m_zeroFlags[slot] (device) holds `epoch` if a masked entry was not exactly zero
     // after all, or what a product would multiply it by not finite.  A slot belongs to one softmax output and what was derived from it.
