@@ -99,7 +99,7 @@ enum {
     MCH_FN_ATTN_SET = 162,                  /* f{dropout} l{hCudnn, hAttn, gpuId, training, batch, blockSize, heads, hs, seed} (device.h:2463-2485);
                                              * dropout in [0, 1) acts in training mode only (attn.cu:578-583): a new mask per forward call from a
                                              * counter-based generator seeded with `seed`, repeated by the backward call that follows */
-    MCH_FN_ATTN_FWD = 163,                  /* l{hCudnn, hAttn, blockSize, hQ, hK, hV, hMask, hY, batchMask[, blockSizeK[, mergedY]]} (device.h:2488-2506, attn.cu:518-602) */
+    MCH_FN_ATTN_FWD = 163,                  /* l{hCudnn, hAttn, blockSize, hQ, hK, hV, hMask, hY, batchMask[, blockSizeK[, mergedY[, oneWave]]]} (device.h:2488-2506, attn.cu:518-602) */
     MCH_FN_ATTN_BWD = 164,                  /* l{hCudnn, hAttn, hQ, hdQ, hK, hdK, hV, hdV, hMask, hY, hdY} (device.h:2509-2529, attn.cu:608-661) */
     MCH_FN_SET = 200,                       /* f{val} l{n, h, 0, idx, xOff} (device.h:6038-6061) */
     MCH_FN_COPY = 202,                      /* l{n, hSrc, hDst, srcOff, dstOff, hStream, srcHalf, dstHalf} (device.h:6063-6095) */
@@ -259,7 +259,7 @@ MCH_LONG DLL_InvokeFloatEx(MCH_LONG lKernelIdx, MCH_LONG lFunctionIdx, float* pI
  * SQRT, INVERT, EXP, LOG, MASK, MASK_BATCH, TRANSPOSE, TRANSPOSE_HW, CHANNEL_COPY / MEAN / MAX / SUB / DIV / DOT / SUM /
  * SUM2 / FILLFROM / COPYALL / DUP, EMBED_FWD, SILU / GELU / RELU forward and backward, SWIGLU_FWD, RMSNORM_FWD, CREATE /
  * FREE_LAYERNORM and LAYERNORM_FWD / BWD, CREATE / FREE_CUDNN, CREATE / FREE / SET_TENSORDESC, SOFTMAX_FWD / BWD,
- * ATTN_CREATE / FREE / SET / FWD / BWD (no dropout; the tenth and eleventh values of ATTN_FWD as on the float side),
+ * ATTN_CREATE / FREE / SET / FWD / BWD (no dropout; the tenth and eleventh values of ATTN_FWD as on the float side, the twelfth ignored),
  * CREATE_ROPE / FREE_ROPE / ROPE_FWD / BWD, and the fused ids ATTN_DECODE_FWD, QKV_PROJ_HEADS, QKV_HEADS_GRAD,
  * LINEAR_FWD / BWD, RMSNORM_BWD, SWIGLU_BWD and NORM_ADD_FWD / BWD - same packing as the float ids above: what the attention, multi-head attention and transformer block layers
  * call, forward and backward.  Products run on the double matrix cores, the rest in one-element-per-thread kernels.  Any other id (blob loaders, extensions), and DLL_InvokeDoubleEx (extensions and blob loaders are float objects),

@@ -341,19 +341,39 @@ template <int KIND> __device__ inline bool bwd_masked(const AttnBwdArgs& a, int 
     return false;
 }
 
+// the odd wavefronts' sums to the even ones before them, a lane's own registers, through LDS that nothing is read from any more
+template <int DT> __device__ __forceinline__ void bwd_meet(float* lds, floatx16 (&acc)[DT], int wave, int lane)
+{
+    float* at = lds + (wave >> 1) * DT * 16 * 64 + lane;
+    if (wave & 1)
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) at[(dt * 16 + v) * 64] = acc[dt][v];
+    __syncthreads();
+    if (!(wave & 1))
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[dt][v] += at[(dt * 16 + v) * 64];
+}
+
 // KIND: 0 none, 1 causal, 2 key mask (B,Tk), 3 mask (B,Tq,Tk) or, with mb = 0, one (Tq,Tk) mask for all sequences
 // PADDED: rows of any head size of whole 16-byte chunks up to HS, zeros up to HS (10 x 8 heads of 16, 592 positions, fp32, causal: 54 us
 // here and 47 for dq; the row kernels 671 and 450).  Infinities and NaN: as in flash_fwd_kernel, a wavefront whose sums are not finite does
 // its queries, or keys, over row by row.
 // PARTS: in 16-bit storage probabilities and their gradients go into the products as two bf16 numbers each, which keeps the precision
 // the row kernels had for these head sizes (error of dq, 48 wide, 300 positions: 1.8e-3 so, 2.5e-3 with one bf16 number each).
-template <typename T, int HS, int KIND, int BQ, int OCC, bool PADDED>
+// SP: wavefronts that share 32 keys, or queries.  Two of them take the 32-row steps of a stage in turn and add up their sums through LDS in
+// the end (flash_split_pays).
+template <typename T, int HS, int KIND, int BQ, int OCC, bool PADDED, int SP>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs a, int mb)
 {
+    static_assert(SP == 1 || (SP == 2 && BQ == 64), "a step of a stage each");
     constexpr bool PARTS = PADDED && sizeof(T) == 2;
     typedef BwdTile<T, HS, BQ> TL;
     typedef FlashTraits<T> TR;
-    constexpr int NW = 4, BK = NW * 32;
+    constexpr int NW = 4, BK = NW * 32 / SP;
     constexpr int EPC = TL::EPC, CPF = TL::CPF, KF = TL::KF, PF = TL::PF, DT = TL::DT, LDR = TL::LDR, LDT = TL::LDT;
     constexpr int TPR = TL::TPR, CPT = TL::CPT;
     extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
@@ -365,6 +385,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     float* Ds = Ls + BQ;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    [[maybe_unused]] const int waveId = __builtin_amdgcn_readfirstlane(wave);   // the same, in a scalar register
     const int l32 = lane & 31, half = lane >> 5;
     const int nbh = a.B * a.H;
     const int rank = KIND == 1 ? flash_causal_rank(OCC) : (int)blockIdx.x;
@@ -374,7 +395,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     const size_t bh = (size_t)b * a.H + h;
     const int hs = PADDED ? a.hs : HS;
     auto chunk = [&](const T* row, int col) { return !PADDED || col < hs ? *(const u32x4*)(row + col) : u32x4{0, 0, 0, 0}; };
-    const int kw = kblock * BK + wave * 32;          // first key of this wavefront
+    const int kw = kblock * BK + wave / SP * 32;     // first key of this wavefront
     const int key = kw + l32;
     const bool waveActive = kw < a.Tk;
     const T* qp = (const T*)a.q + bh * a.Tq * hs;
@@ -451,7 +472,8 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
         if (more) gload(q0 + BQ);
         if (waveActive) {
 #pragma unroll
-            for (int sub = 0; sub < BQ / 32; sub++) {
+            for (int it = 0; it < BQ / 32 / SP; it++) {
+                const int sub = SP == 2 ? waveId & 1 : it;
                 const int qs0 = q0 + 32 * sub;
                 if (qs0 >= a.Tq) continue;
                 if (KIND == 1 && qs0 + 31 < kw) continue;     // every (query, key) pair of the tile is masked
@@ -508,6 +530,11 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
         if (more) sstore();
         __syncthreads();
     }
+    if constexpr (SP == 2) {
+        bwd_meet((float*)bwd_smem, ak, wave, lane);
+        bwd_meet((float*)bwd_smem + 2 * DT * 16 * 64, av, wave, lane);
+        if (wave & 1) return;
+    }
     if constexpr (PADDED) {
         float sum = 0.f;
 #pragma unroll
@@ -515,8 +542,8 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
 #pragma unroll
             for (int v = 0; v < 16; v++) sum += fabsf(ak[dt][v]) + fabsf(av[dt][v]);
         if (waveActive && __any(!(sum < INFINITY))) {
-            const int waveId = __builtin_amdgcn_readfirstlane(wave), first = kblock * BK + waveId * 32;
-            float* own = (float*)bwd_smem + waveId * 2 * HS;
+            const int first = kblock * BK + waveId / SP * 32;
+            float* own = (float*)bwd_smem + (SP == 2 ? waveId / 2 * (DT * 16 * 64) : waveId * 2 * HS);   // (a pair's own part)
             for (int r = first; r < min(first + 32, a.Tk); r++) attn_bwd_dkv_row<T>(a, b, h, r, own, own + HS);
             return;
         }
@@ -538,13 +565,14 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dkv_mfma_kernel(AttnBwdArgs
     }
 }
 
-template <typename T, int HS, int KIND, int BKS, int OCC, bool PADDED>
+template <typename T, int HS, int KIND, int BKS, int OCC, bool PADDED, int SP>
 __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs a, int mb)
 {
+    static_assert(SP == 1 || (SP == 2 && BKS == 64), "a step of a stage each");
     constexpr bool PARTS = PADDED && sizeof(T) == 2;
     typedef BwdTile<T, HS, BKS> TL;
     typedef FlashTraits<T> TR;
-    constexpr int NW = 4, BM = NW * 32;
+    constexpr int NW = 4, BM = NW * 32 / SP;
     constexpr int EPC = TL::EPC, CPF = TL::CPF, KF = TL::KF, PF = TL::PF, DT = TL::DT, LDR = TL::LDR, LDT = TL::LDT;
     constexpr int TPR = TL::TPR, CPT = TL::CPT;
     extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
@@ -565,7 +593,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
     const size_t bh = (size_t)b * a.H + h;
     const int hs = PADDED ? a.hs : HS;
     auto chunk = [&](const T* row, int col) { return !PADDED || col < hs ? *(const u32x4*)(row + col) : u32x4{0, 0, 0, 0}; };
-    const int q0w = qblock * BM + wave * 32;
+    const int q0w = qblock * BM + wave / SP * 32;
     const int qrow = q0w + l32;
     const bool waveActive = q0w < a.Tq;
     const T* qp = (const T*)a.q + bh * a.Tq * hs;
@@ -591,7 +619,7 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
 #pragma unroll
         for (int f = 0; f < KF; f++) drow += TR::dot(chunk(yp, f * CPF + half * (CPF / 2)), gf[f]);
         drow += __shfl_xor(drow, 32, 64);
-        if (qrow < a.Tq && half == 0) a.dsum[bh * a.Tq + qrow] = drow;
+        if (qrow < a.Tq && half == 0 && (SP == 1 || !(wave & 1))) a.dsum[bh * a.Tq + qrow] = drow;
         if (qrow >= a.Tq) drow = 0.f;
     } else if (qrow < a.Tq) {
         drow = a.dsum[bh * a.Tq + qrow];
@@ -639,7 +667,8 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
         if (more) gload(kb + BKS);
         if (waveActive) {
 #pragma unroll
-            for (int sub = 0; sub < BKS / 32; sub++) {
+            for (int it = 0; it < BKS / 32 / SP; it++) {
+                const int sub = SP == 2 ? waveId & 1 : it;
                 const int k0 = kb + 32 * sub;
                 if (k0 >= a.Tk) continue;
                 if (KIND == 1 && k0 > q0w + 31) continue;     // keys past this wavefront's last row
@@ -686,6 +715,10 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
         if (more) sstore();
         __syncthreads();
     }
+    if constexpr (SP == 2) {
+        bwd_meet((float*)bwd_smem, aq, wave, lane);
+        if (wave & 1) return;
+    }
     if constexpr (PADDED) {
         float sum = 0.f;
 #pragma unroll
@@ -693,8 +726,8 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
 #pragma unroll
             for (int v = 0; v < 16; v++) sum += fabsf(aq[dt][v]);
         if (waveActive && __any(!(sum < INFINITY))) {
-            const int first = qblock * BM + waveId * 32;
-            float* own = (float*)bwd_smem + waveId * 2 * HS;
+            const int first = qblock * BM + waveId / SP * 32;
+            float* own = (float*)bwd_smem + (SP == 2 ? waveId / 2 * (DT * 16 * 64) : waveId * 2 * HS);   // (a pair's own part)
             for (int r = 0; r < min(32, a.Tq - first); r++) attn_bwd_dq_row<T>(a, b, h, first + r, __shfl(lrow, r), __shfl(drow, r), own, own + HS);
             return;
         }
@@ -711,38 +744,56 @@ __global__ __launch_bounds__(256, OCC) void attn_bwd_dq_mfma_kernel(AttnBwdArgs 
     }
 }
 
-template <typename T, int HS, int BS, int OCC, int KIND, bool PADDED>
+template <typename T, int HS, int BS, int OCC, int KIND, bool PADDED, int SP, bool DQ>
 static hipError_t bwd_launch_kind(hipStream_t s, const AttnBwdArgs& a, int mb)
 {
     typedef BwdTile<T, HS, BS> TL;
-    const size_t nT = TL::TRR ? 0 : 1;   // transposed tiles
-    const size_t kvBytes = ((size_t)2 * BS * TL::LDR + nT * 2 * HS * TL::LDT) * sizeof(T) + 2 * BS * sizeof(float);
-    const size_t qBytes = ((size_t)2 * BS * TL::LDR + nT * HS * TL::LDT) * sizeof(T) + BS * sizeof(float);
-    auto kkv = attn_bwd_dkv_mfma_kernel<T, HS, KIND, BS, OCC, PADDED>;
-    auto kq = attn_bwd_dq_mfma_kernel<T, HS, KIND, BS, OCC, PADDED>;
+    const size_t nT = TL::TRR ? 0 : DQ ? 1 : 2;   // transposed tiles
+    const size_t bytes = ((size_t)2 * BS * TL::LDR + nT * HS * TL::LDT) * sizeof(T) + (DQ ? 1 : 2) * BS * sizeof(float);
+    void (*kernel)(AttnBwdArgs, int) = nullptr;
+    if constexpr (DQ) kernel = attn_bwd_dq_mfma_kernel<T, HS, KIND, BS, OCC, PADDED, SP>;
+    else kernel = attn_bwd_dkv_mfma_kernel<T, HS, KIND, BS, OCC, PADDED, SP>;
     static bool configured = false;   // per instantiation; the attribute is idempotent, so a race only repeats the call
     if (!configured) {
-        hipError_t e = hipFuncSetAttribute((const void*)kkv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kvBytes);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute((const void*)kq, hipFuncAttributeMaxDynamicSharedMemorySize, (int)qBytes);
+        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) return e;
         configured = true;
     }
-    const int nbh = a.B * a.H;
-    const long long gkv = (long long)((a.Tk + 127) / 128) * nbh, gq = (long long)((a.Tq + 127) / 128) * nbh;
-    if (gkv > 0x7fffffffll || gq > 0x7fffffffll) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kq, dim3((unsigned)gq), 256, qBytes, s, a, mb);      // first: it may produce D for the other kernel
-    hipLaunchKernelGGL(kkv, dim3((unsigned)gkv), 256, kvBytes, s, a, mb);
+    constexpr int ROWS = 128 / SP;
+    const long long grid = (long long)(((DQ ? a.Tq : a.Tk) + ROWS - 1) / ROWS) * a.B * a.H;
+    if (grid > 0x7fffffffll) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), 256, bytes, s, a, mb);
     return hipGetLastError();
+}
+
+template <typename T, int HS, int BS, int OCC, bool PADDED, int SP, bool DQ> static hipError_t bwd_launch_half(hipStream_t s, const AttnBwdArgs& a, int kind, int mb)
+{
+    switch (kind) {
+    case 0: return bwd_launch_kind<T, HS, BS, OCC, 0, PADDED, SP, DQ>(s, a, mb);
+    case 1: return bwd_launch_kind<T, HS, BS, OCC, 1, PADDED, SP, DQ>(s, a, mb);
+    case 2: return bwd_launch_kind<T, HS, BS, OCC, 2, PADDED, SP, DQ>(s, a, mb);
+    default: return bwd_launch_kind<T, HS, BS, OCC, 3, PADDED, SP, DQ>(s, a, mb);
+    }
 }
 
 template <typename T, int HS, int BS, int OCC, bool PADDED = false> static hipError_t bwd_launch_cfg(hipStream_t s, const AttnBwdArgs& a, int kind, int mb)
 {
-    switch (kind) {
-    case 0: return bwd_launch_kind<T, HS, BS, OCC, 0, PADDED>(s, a, mb);
-    case 1: return bwd_launch_kind<T, HS, BS, OCC, 1, PADDED>(s, a, mb);
-    case 2: return bwd_launch_kind<T, HS, BS, OCC, 2, PADDED>(s, a, mb);
-    default: return bwd_launch_kind<T, HS, BS, OCC, 3, PADDED>(s, a, mb);
+    const int nbh = a.B * a.H;
+    // a whole mask's values cost the keys' kernel registers that a pair of wavefronts does not have (heads of 64: 64 of them in memory, 37
+    // alone), so there only launches of one round are split (4 x 12 heads, 700 positions: 431 | 468 us; 2 x 12 of 256: 110 | 68)
+    constexpr bool F = sizeof(T) == 4 && HS <= 64;
+    auto pays = [&](int rows, int others) {
+        return F && flash_split_pays(nbh, rows, others, kind == 1, true) && (kind != 3 || (long long)nbh * ((rows + 63) / 64) <= 256);
+    };
+    hipError_t e;
+    // dq first: it may produce D for the other kernel
+    if constexpr (F) {
+        e = pays(a.Tq, a.Tk) ? bwd_launch_half<T, HS, 64, 2, PADDED, 2, true>(s, a, kind, mb) : bwd_launch_half<T, HS, BS, OCC, PADDED, 1, true>(s, a, kind, mb);
+        if (e != hipSuccess) return e;
+        return pays(a.Tk, a.Tq) ? bwd_launch_half<T, HS, 64, 2, PADDED, 2, false>(s, a, kind, mb) : bwd_launch_half<T, HS, BS, OCC, PADDED, 1, false>(s, a, kind, mb);
+    } else {
+        e = bwd_launch_half<T, HS, BS, OCC, PADDED, 1, true>(s, a, kind, mb);
+        return e != hipSuccess ? e : bwd_launch_half<T, HS, BS, OCC, PADDED, 1, false>(s, a, kind, mb);
     }
 }
 

@@ -34,6 +34,7 @@ struct AttnArgs {
     float scale;
     float* lse2;   // optional [B*H*Tq]: log2 of the row's softmax denominator (-inf marks a fully masked row)
     int yMerged;   // 1: y is written head-merged, (B,Tq,H,hs), the layout the output projection reads; 0: (B,H,Tq,hs)
+    int oneWave;   // fp32: a row's sums by one wavefront, in the order of its keys
     int useDropout;
     AttnDropout drop;
 };
@@ -113,7 +114,7 @@ hipError_t attn_flash2_launch(hipStream_t s, const FlashArgs& f, int hs, bool ca
 
 hipError_t k_attn_prefill(hipStream_t s, DType dt, const void* q, const void* k, const void* v, void* y, int B, int H,
                           int Tq, int Tk, int hs, float scale, const float* mask, MaskKind kind, float* lse2, bool yMerged,
-                          const AttnDropout* dropout)
+                          const AttnDropout* dropout, bool oneWave)
 {
     if (B <= 0 || H <= 0 || Tq <= 0 || Tk <= 0 || hs <= 0) return hipSuccess;
     if (B > 65535 || H > 65535) return hipErrorInvalidValue;
@@ -122,6 +123,7 @@ hipError_t k_attn_prefill(hipStream_t s, DType dt, const void* q, const void* k,
     a.q = q; a.k = k; a.v = v; a.y = y; a.mask = mask;
     a.B = B; a.H = H; a.Tq = Tq; a.Tk = Tk; a.hs = hs; a.kind = (int)kind; a.scale = scale; a.lse2 = lse2;
     a.yMerged = yMerged ? 1 : 0;
+    a.oneWave = oneWave ? 1 : 0;
     a.useDropout = dropout ? 1 : 0;
     if (dropout) a.drop = *dropout;
     bool handled = false;
@@ -176,8 +178,9 @@ __device__ __forceinline__ float flash_half_max(float v)
 // dependency chains interleave.  On return s holds the weights p.  MASKED: scores equal to
 // `sentinel` stand for the reference's -1e29 fill; their weight is decided by comparison (1
 // while the row maximum is still the sentinel, else exactly 0) because exp2 of a difference
-// of two huge products would not cancel exactly.
-template <bool MASKED, int DT, int QT>
+// of two huge products would not cancel exactly.  LATE: the steps need not begin with one that has a score above -inf, whose
+// weights would be NaN: those of a step before the first such one are zero.
+template <bool MASKED, bool LATE, int DT, int QT>
 __device__ __forceinline__ void flash_softmax_step(floatx16 (&s)[QT], floatx16 (&o)[DT][QT], float (&m)[QT], float (&l)[QT],
                                                    float c, float sentinel, float lazy)
 {
@@ -198,8 +201,9 @@ __device__ __forceinline__ void flash_softmax_step(floatx16 (&s)[QT], floatx16 (
         // at most 2^8 (exact in the final normalisation, since l uses the same reference) and the rescale of
         // the output accumulators below is skipped on most steps
         mnew[qt] = (mx[qt] > m[qt] + lazy) ? mx[qt] : m[qt];
-        alpha[qt] = __builtin_amdgcn_exp2f((m[qt] - mnew[qt]) * c);
-        mc[qt] = mnew[qt] * c;
+        const float at = LATE && mnew[qt] == -INFINITY ? 0.f : mnew[qt];
+        alpha[qt] = __builtin_amdgcn_exp2f((m[qt] - at) * c);
+        mc[qt] = at * c;
         m[qt] = mnew[qt];
         same = same && (alpha[qt] == 1.0f);
     }
@@ -232,12 +236,15 @@ __device__ __forceinline__ void flash_softmax_step(floatx16 (&s)[QT], floatx16 (
 // differs where it holds an infinity or a NaN: a wavefront whose sums are not finite does its rows over as that kernel does.
 // PARTS: in 16-bit storage the weights go into the product with V as two bf16 numbers each, which keeps the precision these head sizes
 // had there (48 wide, 300 positions: error of y 1.57e-3, all of it the rounding of y; 1.99e-3 with one bf16 number each).
-template <typename T, int HS, int KIND, int QT, int NW, int OCC, bool PREFETCH, bool PADDED>
+// SP: wavefronts that share 32 QT rows.  Two of them take the 32-key steps of a block in turn, each with its own maximum, sum and output tile,
+// which meet in LDS in the end (flash_split_pays).
+template <typename T, int HS, int KIND, int QT, int NW, int OCC, bool PREFETCH, bool PADDED, int SP>
 __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
 {
     typedef FlashTraits<T> TR;
     constexpr bool PARTS = PADDED && sizeof(T) == 2;
-    constexpr int NT = NW * 64, BM = NW * 32 * QT, BN = 64;
+    constexpr int NT = NW * 64, BM = NW * 32 * QT / SP, BN = 64;
+    static_assert(SP == 1 || (SP == 2 && QT == 1 && NW == 4), "pairs of wavefronts, one step of a block each");
     constexpr int EPC = TR::EPC, CPF = TR::CPF;
     constexpr int KF = HS / CPF;              // fragments along the head dimension (S^T contraction)
     constexpr int PF = 32 / CPF;              // fragments along a 32-key step (P V contraction)
@@ -283,7 +290,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
     const size_t bh = (size_t)b * a.H + h;
     const int hs = PADDED ? a.hs : HS;
     auto chunk = [&](const T* row, int col) { return !PADDED || col < hs ? *(const u32x4*)(row + col) : u32x4{0, 0, 0, 0}; };
-    const int q0 = qblock * BM + wave * 32 * QT;      // first row of this wavefront
+    const int q0 = qblock * BM + wave / SP * 32 * QT;      // first row of this wavefront
     const T* qp = (const T*)a.q + bh * a.Tq * hs;
     const T* kp = (const T*)a.k + bh * a.Tk * hs;
     const T* vp = (const T*)a.v + bh * a.Tk * hs;
@@ -382,7 +389,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         unsigned long long zeros = 0;      // bit = key of this block is masked (KIND 2)
         if (KIND == 2) zeros = __ballot(Ms[lane] == 0.f);
 #pragma unroll
-        for (int sub = 0; sub < 2; sub++) {
+        for (int it = 0; it < 2 / SP; it++) {
+            const int sub = SP == 2 ? waveId & 1 : it;
             const int k0 = kb * BN + 32 * sub;
             // causal: this wavefront's last row is q0 + 32*QT - 1; keys past it contribute nothing
             const bool active = (KIND != 1) || (k0 <= q0 + 32 * QT - 1);
@@ -439,10 +447,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
                             s[qt][v] = sv;
                         }
                     }
-                    if (KIND == 1) flash_softmax_step<false, DT, QT>(s, o, m, l, c, a.maskedRaw, a.lazy);
-                    else flash_softmax_step<true, DT, QT>(s, o, m, l, c, a.maskedRaw, a.lazy);
+                    if (KIND == 1) flash_softmax_step<false, SP == 2, DT, QT>(s, o, m, l, c, a.maskedRaw, a.lazy);
+                    else flash_softmax_step<true, SP == 2, DT, QT>(s, o, m, l, c, a.maskedRaw, a.lazy);
                 } else {
-                    flash_softmax_step<false, DT, QT>(s, o, m, l, c, a.maskedRaw, a.lazy);
+                    flash_softmax_step<false, SP == 2, DT, QT>(s, o, m, l, c, a.maskedRaw, a.lazy);
                 }
                 // O^T += V^T P^T
                 u32x4 pf[QT][PF];
@@ -477,6 +485,38 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         __syncthreads();
     }
 
+    // a wavefront's own LDS from here on, K and V having been read
+    float* own = (float*)Ks + (SP == 1 ? waveId * HS : 0);
+    if (SP == 2 && wave >= 2) own = (float*)Vt;
+    if constexpr (SP == 2) {
+        // the odd wavefront's part to the even one: its maximum and sum and, one after the other, the output tiles of 32 dims, a lane's
+        // own registers
+        float* to = own;
+        static_assert(sizeof(Ks) >= 18 * 64 * sizeof(float) && sizeof(Vt) >= 18 * 64 * sizeof(float), "a tile and the sums");
+        float scale = 0.f, theirs = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) {
+            if (dt > 0) __syncthreads();
+            if (wave & 1) {
+                if (dt == 0) { to[lane] = m[0]; to[64 + lane] = l[0]; }
+#pragma unroll
+                for (int v = 0; v < 16; v++) to[(2 + v) * 64 + lane] = o[dt][0][v];
+            }
+            __syncthreads();
+            if (!(wave & 1)) {
+                if (dt == 0) {
+                    const float mo = to[lane], mn = fmaxf(m[0], mo), at = mn == -INFINITY ? 0.f : mn;
+                    scale = __builtin_amdgcn_exp2f((m[0] - at) * a.c);
+                    theirs = __builtin_amdgcn_exp2f((mo - at) * a.c);
+                    l[0] = l[0] * scale + to[64 + lane] * theirs;
+                    m[0] = mn;
+                }
+#pragma unroll
+                for (int v = 0; v < 16; v++) o[dt][0][v] = o[dt][0][v] * scale + to[(2 + v) * 64 + lane] * theirs;
+            }
+        }
+        if (wave & 1) return;
+    }
     bool over = false;
     if constexpr (PADDED) {
         float sum = 0.f;
@@ -513,9 +553,9 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         static_assert(NW * HS * sizeof(float) <= sizeof(Ks), "a row of a wavefront each");   // every wavefront is past its last step
         if (over) {
             const int kind = KIND == 0 ? MASK_NONE : KIND == 1 ? MASK_CAUSAL : KIND == 2 ? MASK_KEY : a.maskBatch ? MASK_BQK : MASK_QK;
-            const AttnArgs r = {a.q, a.k, a.v, a.y, a.mask, a.B, a.H, a.Tq, a.Tk, hs, kind, a.scale, nullptr, a.yMerged, 0, AttnDropout()};
-            const int first = qblock * BM + waveId * 32 * QT;
-            for (int row = first; row < min(first + 32 * QT, a.Tq); row++) attn_row<T>(r, b, h, row, (float*)Ks + waveId * HS);
+            const AttnArgs r = {a.q, a.k, a.v, a.y, a.mask, a.B, a.H, a.Tq, a.Tk, hs, kind, a.scale, nullptr, a.yMerged, 1, 0, AttnDropout()};
+            const int first = qblock * BM + waveId / SP * 32 * QT;
+            for (int row = first; row < min(first + 32 * QT, a.Tq); row++) attn_row<T>(r, b, h, row, own);
         }
     }
 }
@@ -651,7 +691,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_pipe_bf16_kernel(FlashArgs
                 if ((KIND == 1 && key > qrow) || key >= a.Tk) sc[0][v] = -INFINITY;
             }
         }
-        flash_softmax_step<false, DT, 1>(sc, o, m, l, c, a.maskedRaw, lazy);
+        flash_softmax_step<false, false, DT, 1>(sc, o, m, l, c, a.maskedRaw, lazy);
         pc[0] = TR::pack_p(sc[0], 0);
         pc[1] = TR::pack_p(sc[0], 1);
     };
@@ -863,7 +903,7 @@ __global__ __launch_bounds__(256) void flash_short_causal_f32_kernel(FlashArgs a
                 if (key > qrow || key >= a.Tk) s[0][v] = -INFINITY;
             }
         }
-        flash_softmax_step<false, DT, 1>(s, o, m, l, a.c, a.maskedRaw, a.lazy);
+        flash_softmax_step<false, false, DT, 1>(s, o, m, l, a.c, a.maskedRaw, a.lazy);
 #pragma unroll
         for (int t = 0; t < PF; t++) {
             const u32x4 pf = TR::pack_p(s[0], t);
@@ -904,16 +944,16 @@ __global__ __launch_bounds__(256) void flash_short_causal_f32_kernel(FlashArgs a
     }
 }
 
-template <typename T, int HS, int QT, int NW, int OCC, bool PREFETCH, bool PADDED = false>
+template <typename T, int HS, int QT, int NW, int OCC, bool PREFETCH, bool PADDED = false, int SP = 1>
 static hipError_t flash_launch_cfg(hipStream_t s, const FlashArgs& f, int kind)
 {
-    constexpr int BM = NW * 32 * QT;
+    constexpr int BM = NW * 32 * QT / SP;
     dim3 grid((f.Tq + BM - 1) / BM, f.H, f.B);
     if (kind == MASK_CAUSAL) grid = dim3(((f.Tq + BM - 1) / BM) * f.H * f.B, 1, 1);
-    if (kind == MASK_NONE) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 0, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);
-    else if (kind == MASK_CAUSAL) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 1, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);
-    else if (kind == MASK_KEY) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 2, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);
-    else hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 3, QT, NW, OCC, PREFETCH, PADDED>), grid, NW * 64, 0, s, f);   // MASK_BQK, MASK_QK
+    if (kind == MASK_NONE) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 0, QT, NW, OCC, PREFETCH, PADDED, SP>), grid, NW * 64, 0, s, f);
+    else if (kind == MASK_CAUSAL) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 1, QT, NW, OCC, PREFETCH, PADDED, SP>), grid, NW * 64, 0, s, f);
+    else if (kind == MASK_KEY) hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 2, QT, NW, OCC, PREFETCH, PADDED, SP>), grid, NW * 64, 0, s, f);
+    else hipLaunchKernelGGL((flash_fwd_kernel<T, HS, 3, QT, NW, OCC, PREFETCH, PADDED, SP>), grid, NW * 64, 0, s, f);   // MASK_BQK, MASK_QK
     return hipGetLastError();
 }
 
@@ -943,7 +983,10 @@ hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* h
         if (kvBytes > 128e6 && nbh % 8 == 0) f.causalGroup = (int)(((nbh + 3) / 4 + 7) / 8 * 8);
     }
     *handled = true;
+    const bool split = dt == F32 && a.hs <= 64 && !a.oneWave && flash_split_pays(a.B * a.H, a.Tq, a.Tk, a.kind == MASK_CAUSAL, false);
     if (a.hs != 64 && a.hs != 128) {
+        if (split)
+            return a.hs <= 32 ? flash_launch_cfg<float, 32, 1, 4, 2, false, true, 2>(s, f, a.kind) : flash_launch_cfg<float, 64, 1, 4, 2, false, true, 2>(s, f, a.kind);
         if (dt == F32) return a.hs <= 32 ? flash_launch_cfg<float, 32, 1, 4, 2, false, true>(s, f, a.kind)
                             : a.hs < 64  ? flash_launch_cfg<float, 64, 1, 4, 2, false, true>(s, f, a.kind)
                                          : flash_launch_cfg<float, 128, 1, 8, 1, false, true>(s, f, a.kind);
@@ -1002,12 +1045,16 @@ hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* h
         return flash_launch_cfg<bf16_t, 128, 1, 8, 1, true>(s, f, a.kind);
     }
     if (a.hs == 64) {
-        // causal self attention whose 128-row blocks would not give every CU a workgroup: one workgroup per 32 rows,
-        // the key steps dealt to its wavefronts
-        if (a.kind == MASK_CAUSAL && !a.lse2 && a.Tq == a.Tk && (long long)((a.Tq + 127) / 128) * a.H * a.B < 256) {
+        // causal self attention whose 128-row blocks would not give every other CU a workgroup, or whose heaviest 64-row block would be over
+        // 1.5 times what each CU has to do: one workgroup per 32 rows, the key steps dealt to its wavefronts (12 heads, 2 x 640 positions:
+        // 31 us, pairs of wavefronts 35; 10 x 2048: 92 and 103; 24 x 1024: 71 and 54)
+        const int nbh = a.B * a.H, b128 = (a.Tq + 127) / 128, b64 = (a.Tq + 63) / 64;
+        const long long blocks = (long long)nbh * b128;
+        if (a.kind == MASK_CAUSAL && !a.lse2 && a.Tq == a.Tk && (blocks <= 128 || (blocks < 256 && (a.oneWave || (long long)nbh * (b64 + 1) <= 330)))) {
             hipLaunchKernelGGL(flash_short_causal_f32_kernel, dim3((a.Tq + 31) / 32, a.H, a.B), 256, 0, s, f);
             return hipGetLastError();
         }
+        if (split) return flash_launch_cfg<float, 64, 1, 4, 2, false, false, 2>(s, f, a.kind);
         return flash_launch_cfg<float, 64, 1, 4, 2, false>(s, f, a.kind);
     }
     return flash_launch_cfg<float, 128, 1, 8, 1, false>(s, f, a.kind);

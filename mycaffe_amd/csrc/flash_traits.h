@@ -166,6 +166,25 @@ struct FlashArgs {
     float scale;         // softmax scale
 };
 
+// Whether the fp32 kernels with head sizes up to 64 give 32 rows to two wavefronts (SP = 2, 64 rows to a workgroup) instead of one (128 rows),
+// for `nbh` heads of `rows` rows over `others` keys (or of keys over queries).  A wavefront's own rows are one serial chain - scores, weights,
+// sums - over all steps of 32 `others`, and below two workgroups a CU its matrix unit waits for it; two wavefronts halve that chain and leave
+// fewer rows of a last block empty, at the price of staging twice as often and of one meeting.  Measured (us, one | two; heads of 64):
+//   12 heads, 4 sequences, causal:  128 rows  29 | 23 (24 sequences)   700 rows  64 | 47, backward 180 | 128   1024 rows (3 of 16)  92 | 76, 258 | 228
+//   unmasked, workgroups of 128 rows:  12: 16 | 12, 41 | 28   48: 27 | 19, 70 | 46   180: 59 | 57, 152 | 166   288: 107 | 86, 313 | 268
+//                                      384: 152 | 121, 456 | 385   400: 26 | 31, 59 | 75 (96 rows)   792: 52 | 53, 142 | 157   1056: 363 | 369, 1125 | 1228
+// Those follow the rounds of 256 workgroups each way takes, a round of the smaller ones counting 3/5.  A causal launch is as long as its
+// heaviest block once that is a good part of what every CU has to do: 3/4 in the forward pass (8 x 12 heads, 700 rows, 0.76: 81 | 71; 12 x 20,
+// 256 rows, 0.71: 39 | 36; 8 x 12, 1024 rows, 0.59: 135 | 140), 9/8 in the backward one, whose blocks are dealt out better (10 x 12, 384 rows,
+// 1.07: 107 | 115; 3 x 16, 1024 rows, 1.19: 258 | 228).  One step of others leaves the second wavefront nothing (64 x 6, 20 rows: 19 | 24).
+inline bool flash_split_pays(int nbh, int rows, int others, bool causal, bool backward)
+{
+    const long long blocks = (rows + 127) / 128, one = (nbh * blocks + 255) / 256, two = ((long long)nbh * ((rows + 63) / 64) + 255) / 256;
+    if (others <= 32) return false;
+    if (causal && blocks > 1) return 256 * 2 * (backward ? 8 : 12) >= 9 * nbh * (blocks + 1);
+    return 3 * two < 5 * one;
+}
+
 // Rank of a workgroup of a causal launch in the heaviest-first order.  Workgroup i goes to XCD i % 8 and, within it, the
 // first launches land on its 32 CUs in turn, `occ` rounds of 32 before the XCD is full.  A CU keeps what it was given in
 // those rounds, so every second one of them is walked backwards: the CU that got the heaviest block of one round gets

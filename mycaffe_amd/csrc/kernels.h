@@ -205,7 +205,8 @@ __host__ __device__ inline bool attn_dropout_keep(uint64_t seed, uint64_t index,
 }
 hipError_t k_attn_prefill(hipStream_t s, DType dt, const void* q, const void* k, const void* v, void* y, int B, int H,
                           int Tq, int Tk, int hs, float scale, const float* mask, MaskKind kind, float* lse2 = nullptr,
-                          bool yMerged = false, const AttnDropout* dropout = nullptr);
+                          bool yMerged = false, const AttnDropout* dropout = nullptr, bool oneWave = false);
+// oneWave: in fp32 a row's sums stay with one wavefront, in the order of its keys, at every size (csrc/flash_traits.h, flash_split_pays).
 // yMerged: y is written as (B,Tq,H,hs), the head-merged layout the output projection reads, instead of (B,H,Tq,hs).
 // With lse2 ([B*H*Tq] fp32) the forward pass also stores log2 of every row's softmax denominator (scores scaled, masked
 // ones at -1e29; -inf marks a row whose keys are all masked), which is all the backward pass needs of the probabilities.

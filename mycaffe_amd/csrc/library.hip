@@ -1999,11 +1999,12 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
         return 0;
     }
     case MCH_FN_ATTN_FWD: {
-        // l{hCudnn,hAttn,blockSize,hQ,hK,hV,hMask,hY,batchMask[,blockSizeK[,mergedY]]} (device.h:2488-2506, attn.cu:518-602)
+        // l{hCudnn,hAttn,blockSize,hQ,hK,hV,hMask,hY,batchMask[,blockSizeK[,mergedY[,oneWave]]]} (device.h:2488-2506, attn.cu:518-602)
         // The optional 10th value (key length when it differs from the query length) and 11th (1: Y is written
         // head-merged, (B,T,H,hs), ready for the output projection) have no counterpart in the reference, whose
-        // handle needs T_q == T_k and always writes (B,H,T,hs).
-        NEED_L(9, 11);
+        // handle needs T_q == T_k and always writes (B,H,T,hs).  The 12th (1: a row's sums in one order at every size) is for what a
+        // ReLU follows (TransformerBlockLayer, fp32_sums).
+        NEED_L(9, 12);
         const bool mergedY = ll > 10 && pl[10] != 0;
         AttnState* st = m_attn.get((long)pl[1]);
         if (!st || !st->set) return MCH_ERROR_ATTN_NOT_INITIALIZED;
@@ -2071,7 +2072,7 @@ long Kernel::run(long fn, float* pf, long lf, MCH_LONGLONG* pl, long ll, float**
             st->drop.keepScale = 1.0f / (1.0f - st->dropout);
         }
         HIPCHK(k_attn_prefill(s, Q->dt(), Q->ptr, K->ptr, V->ptr, Y->ptr, st->batch, st->heads, T, Tk, st->hs, st->scale,
-                              M ? (const float*)M->ptr : nullptr, kind, lse, mergedY, drop ? &st->drop : nullptr));
+                              M ? (const float*)M->ptr : nullptr, kind, lse, mergedY, drop ? &st->drop : nullptr, ll > 11 && pl[11] != 0));
         // the backward pass needs this output (dY . Y per row); the C# layer hands ATTN_BWD a Y buffer that holds the
         // head-merged layout by then (CausalSelfAttentionLayer.cs:668-672), so a copy stays with the handle
         if (lse) HIPCHK(k_convert(s, Y->dt(), Y->ptr, Y->dt(), st->ysave, (size_t)qn));

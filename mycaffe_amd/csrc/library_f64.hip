@@ -1844,9 +1844,9 @@ long KernelD::run(long fn, const double* pf, long lf, const MCH_LONGLONG* pl, lo
         return 0;
     }
     case MCH_FN_ATTN_FWD: {
-        // l{hCudnn,hAttn,blockSize,hQ,hK,hV,hMask,hY,batchMask[,blockSizeK[,mergedY]]}; the tenth and eleventh values as in the
-        // fp32 library (key length when it differs, Y written head-merged)
-        NEED_L(9, 11);
+        // l{hCudnn,hAttn,blockSize,hQ,hK,hV,hMask,hY,batchMask[,blockSizeK[,mergedY[,oneWave]]]}; the tenth and eleventh values as in the
+        // fp32 library (key length when it differs, Y written head-merged), the twelfth makes no difference here
+        NEED_L(9, 12);
         AttnD* st = m_attn.get((long)pl[1]);
         if (!st || !st->set) return MCH_ERROR_ATTN_NOT_INITIALIZED;
         const int T = (int)pl[2], Tk = ll > 9 ? (int)pl[9] : T;

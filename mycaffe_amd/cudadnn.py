@@ -724,15 +724,18 @@ class CudaDnn:
         self._ex2(CUDAFN.CUDA_ATTN_SET, [fDropout], [hCuDnn, hAttn, nGpuID, int(bTraining), nBatch, nBlockSize, nHeads, nSize, lSeed])
 
     def AttnScaledDotProductForward(self, hCuDnn, hAttn, nBlockSize, hQdata, hKdata, hVdata, hMaskdata, hYdata,
-                                    bBatchMask=True, nBlockSizeK=None, bMergedY=False):
+                                    bBatchMask=True, nBlockSizeK=None, bMergedY=False, bOneWave=False):
         """CudaDnn.cs:5673-5679.  ``nBlockSizeK`` (key length, when it differs from the
         query length) is an optional tenth value with no counterpart in the reference, and so
         are ``bBatchMask=2`` (a (B,T_q,T_k) mask) and ``bMergedY`` (eleventh value: Y written
-        head-merged, (B,T,H,hs), instead of (B,H,T,hs))."""
+        head-merged, (B,T,H,hs), instead of (B,H,T,hs)) and ``bOneWave`` (twelfth value: a row's fp32 sums in one order
+        at every size)."""
         rgl = [hCuDnn, hAttn, nBlockSize, hQdata, hKdata, hVdata, hMaskdata, hYdata, int(bBatchMask)]
-        if nBlockSizeK is not None or bMergedY:
+        if nBlockSizeK is not None or bMergedY or bOneWave:
             rgl.append(nBlockSizeK if nBlockSizeK is not None else nBlockSize)
-        if bMergedY:
+        if bMergedY or bOneWave:
+            rgl.append(int(bMergedY))
+        if bOneWave:
             rgl.append(1)
         self._ex2(CUDAFN.CUDA_ATTN_FWD, None, rgl)
 

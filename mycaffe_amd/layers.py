@@ -424,7 +424,7 @@ class CausalSelfAttentionLayer:
                 self.c_proj.Forward(out, top)
                 return
             cuda.AttnScaledDotProductForward(self.hCudnn, self.hAttn, T, b["Qt"].gpu_data, b["Kt"].gpu_data, b["Vt"].gpu_data,
-                                             mask.gpu_data, out.gpu_data, False)
+                                             mask.gpu_data, out.gpu_data, False, bOneWave=self.training and self.c_attn.fp32_sums)
         else:
             self.transposeQ.Forward(b["Kt"], b["Kt1"])
             dfScale = 1.0 / math.sqrt(hs)
