@@ -21,6 +21,7 @@
 // which reads as zeros.  (Vector instructions are not free next to the fp32 MFMA: a 64-bit address per fetch and a select per
 // register on the way to LDS cost 6 % of a whole product.)
 #include "gemm_common.h"
+#include "xcd_runs.h"
 
 namespace mch {
 
@@ -1104,7 +1105,10 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
 // VEC: as above; otherwise 4 bytes per lane go into LDS, to the same places.
 // rowSums: null, or a value for every row of C to which the sum of the row of A is added (by the tiles of the first columns).
 constexpr int SMALL_STAGES = 3;
-template <int NW, int BK, bool AK, bool BKC, bool VEC, bool HEADS>
+constexpr int SMALL_TILE_COST = 84;   // what a tile costs beside its contraction, in k (the last term of gemm_f32_small_time)
+// LEVELS: sums of eight stages each, which are added up: the rounding of a long contraction like that of one cut into parts (130 x 768 x
+// 2304: error against float64 4.3e-7 in one run, 2.1e-7 so).
+template <int NW, int BK, bool AK, bool BKC, bool VEC, bool HEADS, bool LEVELS = false>
 __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const HeadsArg<HEADS>& hp, const F32Item& it, float* rowSums, float* smem)
 {
     constexpr int NT = 64 * NW, W = VEC ? 4 : 1, P = 32 * BK / W / NT, STAGE = 2 * 32 * BK, S = SMALL_STAGES;   // values per lane and fetch; fetches per thread, operand and stage
@@ -1166,15 +1170,16 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
         return v;
     };
     floatx16 acc;
+    [[maybe_unused]] floatx16 all;
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    for (int v = 0; v < 16; v++) { acc[v] = 0.f; all[v] = 0.f; }
     const bool sumRows = rowSums && it.n0 == 0;
     float rowSum = 0.f;
 #pragma unroll
     for (int i = 0; i < S - 1; i++)
         if (i < nk) fetch(smem + i * STAGE);
     int buf = 0, free = S - 1;
-    for (int kt = 0; kt < nk; kt++) {
+    auto step = [&](int kt) {
         // the stage has landed, of this wavefront and then of all, while the stages after it are still on their way (__syncthreads
         // would wait for those too)
         if (kt + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(2 * P * (S - 2)) : "memory");
@@ -1200,7 +1205,17 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
 #pragma unroll
             for (int j = 0; j < J; j++)   // zeros past the end
                 rowSum += (__uint_as_float(a[j].x) + __uint_as_float(a[j].y)) + (__uint_as_float(a[j].z) + __uint_as_float(a[j].w));
-    }
+    };
+    if constexpr (LEVELS) {
+        for (int kt = 0; kt < nk;) {
+            const int end = min(nk, kt + 8);
+            for (; kt < end; kt++) step(kt);
+#pragma unroll
+            for (int v = 0; v < 16; v++) { all[v] += acc[v]; acc[v] = 0.f; }
+        }
+        acc = all;
+    } else
+        for (int kt = 0; kt < nk; kt++) step(kt);
     __syncthreads();
     float* slice = smem + wave * 32 * LDC;
 #pragma unroll
@@ -1255,23 +1270,23 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_small_kernel(GemmF32Args g, 
 // The gradients of an inner product whose products do not fill the chip, as one launch: w is dW += dY^T X, its tiles of the first
 // columns add the column sums of dY to db, and x is dX = dY W.  Apart they are three or four launches, each with its own first
 // fetch and end, on half the CUs.  (The ones with the longer contraction come
-// first.)  Kernel trace, us: 1024 rows, 288 to 768 11.5 + 4.0 + 10.9 + 3.9 -> 14.0, 1024 rows, 288 to 864 12.0 + 4.2 + 11.1 + 4.0 -> 19.1, 12
-// rows, 12 to 3 with the column sums 4.1 + 1.9 + 3.2 -> 3.9 (and two launches of the host's 3.6 us each fewer).
-template <int NW, int BK, bool VEC>
-__global__ __launch_bounds__(64 * NW) void linear_bwd_f32_small_kernel(GemmF32Args w, GemmF32Args x, float* db)
+// first, in runs of equal work, xcd_runs.h.)  Calls in a row, us, apart and together: 1024 rows, 288 to 768 23.9 and 15.1, 288 to 864 25.4 and
+// 16.6, 768 to 288 21.2 and 15.5; 200 rows, 384 to 1536 21.6 and 13.4; 1500 rows, 768 to 768 53 and 40; 2800 rows, 768 to 768 65 and 69.
+template <int NW, int BK, bool VEC, bool LEVELS>
+__global__ __launch_bounds__(64 * NW) void linear_bwd_f32_small_kernel(GemmF32Args w, GemmF32Args x, float* db, XcdRuns runs)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     float* smem = reinterpret_cast<float*>(smem_raw);
-    const int tilesW = w.tilesM * w.tilesN, tilesX = x.tilesM * x.tilesN, total = tilesW + tilesX, at = xcd_item(total);
-    if (at >= total) return;
+    const int tilesW = w.tilesM * w.tilesN, tilesX = x.tilesM * x.tilesN, at = runs.first[blockIdx.x % 8] + (int)(blockIdx.x / 8);
+    if (at >= runs.first[blockIdx.x % 8 + 1]) return;
     const int item = w.K >= x.K ? at : at < tilesX ? tilesW + at : at - tilesX;
     F32Item it;
     if (item < tilesW) {
         f32_item<32, 32>(w, item, it);
-        f32_small_tile<NW, BK, false, false, VEC, false>(w, HeadsArg<false>(), it, db, smem);
+        f32_small_tile<NW, BK, false, false, VEC, false, LEVELS>(w, HeadsArg<false>(), it, db, smem);
     } else {
         f32_item<32, 32>(x, item - tilesW, it);
-        f32_small_tile<NW, BK, true, false, VEC, false>(x, HeadsArg<false>(), it, nullptr, smem);
+        f32_small_tile<NW, BK, true, false, VEC, false, LEVELS>(x, HeadsArg<false>(), it, nullptr, smem);
     }
 }
 
@@ -1652,11 +1667,13 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     if (tilesW + tilesX > (1ll << 20)) return hipSuccess;
     // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
     // time that one launch waits for the last one's stores
-    const bool together = db && gemm_f32_row_sums_workspace_bytes(n, k, m, vec) > 0;   // the column sums with the weight gradient
+    const bool sumsToo = db && gemm_f32_row_sums_workspace_bytes(n, k, m, vec) > 0;   // the column sums with the weight gradient
     const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false);
     const double apart = dw.time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false).time + 2.5 +
-                         (!db ? 0.0 : together ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
-    if (gemm_f32_small_time(tilesW + tilesX, std::max(m, n)) >= apart) return hipSuccess;
+                         (!db ? 0.0 : sumsToo ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
+    // the one launch, fitted to 43 sizes (0.8 .. 1.24 of what was measured, 4.4 to 199 us); a tenth on top of it, as both sides are estimates
+    const double together = 2.65 + (0.714 * (double)(tilesW + tilesX) + 0.458 / 128 * ((double)tilesW * m + (double)tilesX * n)) / 256 + 0.64 * std::max(m, n) / 128;
+    if (1.1 * together >= apart) return hipSuccess;
     GemmF32Args w = {}, x = {};
     w.M = n; w.N = k; w.K = w.kChunk = m;
     w.A = dY; w.B = X; w.C = dW;
@@ -1671,15 +1688,24 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     x.vecC = k % 4 == 0 && ((uintptr_t)dX & 15) == 0;
     x.tilesM = (m + 31) / 32; x.tilesN = (int)tilesK;
     constexpr int lds = small_lds<4, 64>();
+    typedef void (*Kernel)(GemmF32Args, GemmF32Args, float*, XcdRuns);
+    static const Kernel kernels[2][2] = {{linear_bwd_f32_small_kernel<4, 64, false, false>, linear_bwd_f32_small_kernel<4, 64, true, false>},
+                                         {linear_bwd_f32_small_kernel<4, 64, false, true>, linear_bwd_f32_small_kernel<4, 64, true, true>}};
     static const hipError_t attr = [] {
-        const hipError_t e = hipFuncSetAttribute((const void*)linear_bwd_f32_small_kernel<4, 64, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        return e != hipSuccess ? e : hipFuncSetAttribute((const void*)linear_bwd_f32_small_kernel<4, 64, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < 4 && e == hipSuccess; i++) e = hipFuncSetAttribute((const void*)kernels[i / 2][i % 2], hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        return e;
     }();
     if (attr != hipSuccess) return attr;
-    const int grid = (int)((tilesW + tilesX + 7) / 8) * 8;
+    // Long contractions of which a CU has more than one: the calls apart cut them or add fewer values in a row, and another workgroup
+    // is there while one adds up (1024 rows, 288 to 768: 14.9 -> 15.5 us; 142 tiles of up to 2000 rows 16.0 -> 17.0, which stay as they are)
+    const bool levels = tilesW + tilesX > 256 && std::max(m, n) > 512;
+    int most;
+    const bool wFirst = w.K >= x.K;
+    const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.K, x.K) + SMALL_TILE_COST, wFirst ? tilesX : tilesW, std::min(w.K, x.K) + SMALL_TILE_COST, &most);
+    const int grid = 8 * most;
     *done = true;
-    if (vec) hipLaunchKernelGGL((linear_bwd_f32_small_kernel<4, 64, true>), grid, 256, lds, s, w, x, db);
-    else hipLaunchKernelGGL((linear_bwd_f32_small_kernel<4, 64, false>), grid, 256, lds, s, w, x, db);
+    hipLaunchKernelGGL(kernels[levels][vec], grid, 256, lds, s, w, x, db, runs);
     return hipGetLastError();
 }
 

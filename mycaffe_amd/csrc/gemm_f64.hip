@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "gemm_f64.h"
+#include "xcd_runs.h"
 
 namespace mch {
 
@@ -128,6 +129,7 @@ template <int W, int G> __global__ __launch_bounds__(256 * G) void d_gemm_kernel
 // then next to each other.  VEC: 16 bytes a lane; otherwise 4, whatever the strides and the alignment.
 // rowSums: null, or a value for every row of C to which the sum of the row of A is added (by the tiles of the first columns).
 constexpr int D_STAGES = 3;
+constexpr int D_TILE_COST = 112;   // what a tile costs beside its contraction, in k (the last term of d_small_time)
 template <int BYTES> __device__ __forceinline__ void d_lds_fetch(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voffset)
 {
     typedef __attribute__((address_space(3))) void* shared_ptr;
@@ -274,14 +276,15 @@ __global__ __launch_bounds__(64 * NW) void d_gemm_small_kernel(GemmD g, HeadsD h
 }
 
 // the gradients of an inner product as one launch: w is dW += dY^T X, whose first tiles add the column sums of dY to db, x is dX = dY W
-// (kernel trace, 256 rows: 256 to 256 8.4 + 3.8 + 7.9 -> 5.5 us, 1024 to 256 9.2 + 3.9 + 8.4 -> 14.0, 256 to 1024 10.2 + 3.8 + 21.0 -> 20.0); the longer contraction first
+// (calls in a row, us, apart and together, 256 rows: 256 to 256 10.6 and 5.1, 1024 to 256 18.4 and 12.0, 256 to 1024 20.6 and 12.1, 256 to 768 14.6 and 9.8; 1024 rows,
+// 288 to 768 40 and 29); the longer contraction first, in runs of equal work (xcd_runs.h)
 template <int NW, int BK, bool VEC>
-__global__ __launch_bounds__(64 * NW) void d_linear_bwd_small_kernel(GemmD w, GemmD x, double* db, int tilesN, int tilesW, int tilesX)
+__global__ __launch_bounds__(64 * NW) void d_linear_bwd_small_kernel(GemmD w, GemmD x, double* db, int tilesN, int tilesW, int tilesX, XcdRuns runs)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char d_smem_raw[];
     double* smem = reinterpret_cast<double*>(d_smem_raw);
-    const int at = d_xcd_item(tilesW + tilesX);
-    if (at >= tilesW + tilesX) return;
+    const int at = runs.first[blockIdx.x % 8] + (int)(blockIdx.x / 8);
+    if (at >= runs.first[blockIdx.x % 8 + 1]) return;
     const int item = w.k >= x.k ? at : at < tilesX ? tilesW + at : at - tilesX;
     if (item < tilesW) d_small_tile<NW, BK, false, false, VEC, false>(w, HeadsD(), item / tilesN * 16, item % tilesN * 16, 0, db, smem);
     else d_small_tile<NW, BK, true, false, VEC, false>(x, HeadsD(), (item - tilesW) / tilesN * 16, (item - tilesW) % tilesN * 16, 0, nullptr, smem);
@@ -414,14 +417,19 @@ hipError_t d_linear_bwd_small(hipStream_t s, int m, int n, int k, const double* 
     d_tiles(m, k, n, 1, &apartX);
     // against the launches apart: the column sums, and 2.5 us for each time that one launch waits for the last one's stores
     const double apart = std::min(apartW, d_small_time(tilesW, m)) + std::min(apartX, d_small_time(tilesX, n)) + 2.5 + (db ? 4.5 : 0.0);
-    if (d_small_time(tilesW + tilesX, std::max(m, n)) >= apart) return hipSuccess;
+    // the one launch, fitted to 23 sizes (0.8 .. 1.18 of what was measured, 4.6 to 93 us); a tenth on top of it, as both sides are estimates
+    const double together = 3.1 + (0.49 * (double)(tilesW + tilesX) + 0.384 / 128 * ((double)tilesW * m + (double)tilesX * n)) / 256 + 0.15 * std::max(m, n) / 128;
+    if (1.1 * together >= apart) return hipSuccess;
     const GemmD w = {n, k, m, 1.0, 1.0, dY, X, dW, 1, n, k, 1, k, 1, 0, 0, 0, 0, 1, nullptr}, x = {m, k, n, 1.0, beta, dY, W, dX, n, 1, k, 1, k, 1, 0, 0, 0, 0, 1, nullptr};
     const bool vec = d_chunks(dY, 1, n, n, m, 0, 1) && d_chunks(dY, n, 1, m, n, 0, 1) && d_chunks(X, 1, k, k, m, 0, 1) && d_chunks(W, 1, k, k, n, 0, 1);
     *done = true;
     constexpr int lds = d_small_lds<4, 64>();
-    const int grid = (int)((tilesW + tilesX + 7) / 8) * 8;
-    if (vec) hipLaunchKernelGGL((d_linear_bwd_small_kernel<4, 64, true>), grid, 256, lds, s, w, x, db, (int)tilesN, (int)tilesW, (int)tilesX);
-    else hipLaunchKernelGGL((d_linear_bwd_small_kernel<4, 64, false>), grid, 256, lds, s, w, x, db, (int)tilesN, (int)tilesW, (int)tilesX);
+    int most;
+    const bool wFirst = w.k >= x.k;
+    const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.k, x.k) + D_TILE_COST, wFirst ? tilesX : tilesW, std::min(w.k, x.k) + D_TILE_COST, &most);
+    const int grid = 8 * most;
+    if (vec) hipLaunchKernelGGL((d_linear_bwd_small_kernel<4, 64, true>), grid, 256, lds, s, w, x, db, (int)tilesN, (int)tilesW, (int)tilesX, runs);
+    else hipLaunchKernelGGL((d_linear_bwd_small_kernel<4, 64, false>), grid, 256, lds, s, w, x, db, (int)tilesN, (int)tilesW, (int)tilesX, runs);
     return hipGetLastError();
 }
 

@@ -1,0 +1,34 @@
+"""The gradients of an inner product in one launch, whose tiles are dealt to the XCDs in runs of equal work (csrc/xcd_runs.h): fewer tiles
+than XCDs, one product much longer than the other, contractions around the eight stages of a level of sums."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_double import devd  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows, outputs, inputs)
+SIZES = [(5, 3, 2), (40, 1536, 384), (256, 1024, 256), (2000, 64, 256), (130, 2304, 768),   # long weight or long data gradient
+         (511, 600, 512), (512, 600, 512), (513, 600, 512), (576, 513, 520), (1025, 400, 384), (1029, 401, 387)]
+
+
+@pytest.mark.parametrize("base", ["float", "double"])
+@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gradients(dev, devd, base, m, n, k, accumulate):  # noqa: F811
+    t, unit = (np.float32, 2.0 ** -24) if base == "float" else (np.float64, 2.0 ** -53)
+    c = dev.cuda if base == "float" else devd.cuda
+    rng = np.random.default_rng(m + n + k)
+    x, w, dy, dw, db, dx = (rng.standard_normal(s).astype(t) for s in ((m, k), (n, k), (m, n), (n, k), (n,), (m, k)))
+    h = [c.AllocMemory(a.ravel()) for a in (x, w, dy, dw, db, dx)]
+    c.LinearBackward(m, n, k, *h, accumulate)
+    x, w, dy, dw, db, dx = (a.astype(np.float64) for a in (x, w, dy, dw, db, dx))
+    # a sum of l products rounds l times at the size of its partial sums, by chance in either direction: sqrt(l) of them in all, and a few at the end
+    bound = lambda l: unit * (4 + np.sqrt(l))  # noqa: E731
+    for handle, want, scale, l in ((h[3], dw + dy.T @ x, np.abs(dw) + np.abs(dy).T @ np.abs(x), m), (h[4], db + dy.sum(0), np.abs(db) + np.abs(dy).sum(0), m),
+                                   (h[5], accumulate * dx + dy @ w, np.abs(dx) + np.abs(dy) @ np.abs(w), n)):
+        got = np.asarray(c.GetMemoryFloat(handle, want.size)).reshape(want.shape)
+        assert (np.abs(got - want) <= bound(l) * scale).all()
+    for a in h:
+        c.FreeMemory(a)
