@@ -1,4 +1,4 @@
-// 16-bit GEMM on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16), any operand layout, fp32 accumulation, gfx950.
+// 16-bit GEMM on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), any operand layout, fp32 accumulation, gfx950.
 //
 // WVM x WVN wavefronts of WM x WN MFMA tiles each cover (32 WVM WM) x (32 WVN WN) of C and walk K in stages of 64 that go
 // from global memory straight into LDS (buffer loads to LDS: no staging registers, no writes to issue), two to four of them there,
@@ -6,10 +6,16 @@
 // L2, all that L2 has; 256 x 256 half of that.  Large products therefore take 256 x 256 or 256 x 192 with eight
 // wavefronts, one workgroup per CU, whichever leaves the shorter last round, small ones the tile that fills the chip.
 //
+// Large products run at the power limit (1.8 GHz at 8192 x 3072 x 6144), where what an instruction costs is time: products of 16 x 16 x 32
+// alone, on normally distributed values, reach 2.0 PFLOP/s, those of 32 x 32 x 16 1.8 (2.4 and 2.5 on zeros), and a wavefront reads the same
+// fragments for either (4096^3, A B^T 124 -> 119 us, A B 125.5 -> 123; 8000 x 3072 x 768 47.7 -> 46.5).  The sums are the same bits.  Where
+// both operands are read transposed and a wavefront has 32 x 32 of C the longer instruction stays: half as much has to arrive before the
+// first product of a stage (768 x 768 x 8192, A^T B: 23.2 us, 24.7 with 16 x 16).
+//
 //   * k at unit stride: LDS holds [row][64 k] without padding, the 16-byte piece c of row r at position c ^ ((r >> 1) & 7)
 //     (sixteen consecutive rows read by a 128-bit access then fall on sixteen bank groups).
 //   * row index at unit stride: LDS holds [k][row] as it is stored, the 32-row blocks of row k exchanged by a function of
-//     k & 3, and the fragments are read with the transposing 64-bit access (ds_read_b64_tr_b16: lane i of a group of
+//     k & 3 and their halves by k & 8, and the fragments are read with the transposing 64-bit access (ds_read_b64_tr_b16: lane i of a group of
 //     sixteen receives column i of the 4 x 16 block whose rows four lanes each address).  Gradients need no operand turned
 //     in memory first (57 of 570 us of an MLP's training step).
 //   * The contraction may end anywhere a 16-byte chunk ends: chunks past the end get an offset outside the buffer, which
@@ -195,14 +201,16 @@ __device__ __forceinline__ void prompt_store8(const GemmB16Args& g, int r, int c
 template <int WVM, int WVN, int WM, int WN, int S, bool AK, bool BKC, int HEADS, bool SUMS = false>
 __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEADS>& hp, int item)
 {
-    constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64, KS = 4;
+    constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64;
+    constexpr bool PROMPT = HEADS >= 3;
+    constexpr int F = !AK && !BKC && WM * WN == 1 ? 32 : 16, KM = 512 / F, KS = BK / KM, TM = 32 * WM / F, TN = 32 * WN / F;   // rows and k of a product; products' tiles of a wavefront
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;               // 16-byte chunks per thread and stage
     constexpr int STAGE = (BM + BN) * BK;                           // elements of one stage: A's part, then B's
-    constexpr int NMF = WM * WN;
+    constexpr int NMF = TM * TN;
     static_assert(PA * NT == BM * 8 && PB * NT == BN * 8, "whole chunks per thread");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     bf16_t* smem = reinterpret_cast<bf16_t*>(smem_raw);
-    constexpr bool ENDS_IN_HEADS = HEADS == 1 || HEADS == 2, PROMPT = HEADS >= 3;
+    constexpr bool ENDS_IN_HEADS = HEADS == 1 || HEADS == 2;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles = g.tilesM * g.tilesN;
     const int part = item / tiles, tile = item - part * tiles;
@@ -221,18 +229,20 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
     constexpr uint32_t OUTSIDE = 0x80000000u;
     const bf16_t* baseA = g.A + (AK ? (size_t)m0 * g.lda : (size_t)m0);
     const bf16_t* baseB = g.B + (BKC ? (size_t)n0 * g.ldb : (size_t)n0);
+    // (16 x 16: groups of lanes eight k apart read the same sixteen rows, from the other half of their 32)
+    auto place = [](auto rowb, int k) { return block_swizzle<decltype(rowb)::value>(k) + (F == 16 ? ((k >> 3) & 1) * 2 : 0); };
     uint32_t va[PA], vb[PB];
 #pragma unroll
     for (int p = 0; p < PA; p++) {
         const int e = p * NT + tid;
         if (AK) va[p] = ((uint32_t)min(e / 8, M - 1 - m0) * (uint32_t)g.lda + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
-        else va[p] = ((uint32_t)(e / (BM / 8)) * (uint32_t)g.lda + min(((e % (BM / 8)) ^ block_swizzle<BM * 2>(e / (BM / 8))) * 8, M - 8 - m0)) * 2;
+        else va[p] = ((uint32_t)(e / (BM / 8)) * (uint32_t)g.lda + min(((e % (BM / 8)) ^ place(std::integral_constant<int, BM * 2>(), e / (BM / 8))) * 8, M - 8 - m0)) * 2;
     }
 #pragma unroll
     for (int p = 0; p < PB; p++) {
         const int e = p * NT + tid;
         if (BKC) vb[p] = ((uint32_t)min(e / 8, N - 1 - n0) * (uint32_t)g.ldb + ((e & 7) ^ ((e >> 4) & 7)) * 8) * 2;
-        else vb[p] = ((uint32_t)(e / (BN / 8)) * (uint32_t)g.ldb + min(((e % (BN / 8)) ^ block_swizzle<BN * 2>(e / (BN / 8))) * 8, N - 8 - n0)) * 2;
+        else vb[p] = ((uint32_t)(e / (BN / 8)) * (uint32_t)g.ldb + min(((e % (BN / 8)) ^ place(std::integral_constant<int, BN * 2>(), e / (BN / 8))) * 8, N - 8 - n0)) * 2;
     }
     // a prompt product's B by its addresses: pairs of rows of a stacked matrix lie far apart
     [[maybe_unused]] const bf16_t* pb64[PB];
@@ -282,35 +292,40 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
         }
     };
 
-    floatx16 acc[WM][WN];
+    typedef std::conditional_t<F == 32, floatx16, floatx4> Sums;
+    Sums acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < WM; i++)
+    for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < WN; j++)
+        for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+            for (int v = 0; v < F * F / 64; v++) acc[i][j][v] = 0.f;
 
-    // fragments: lane l holds row l % 32, k = 8 (l / 32) .. + 7 of a k-step of 16
-    const int fr = lane & 31, half = lane >> 5;
+    // fragments: lane l holds row l % F, k = 8 (l / F) .. + 7 of a k-step of KM
+    const int fr = lane & (F - 1), kp = lane / F;
     int koff[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) koff[ks] = ((2 * ks + half) ^ ((fr >> 1) & 7)) * 8;
-    // transposing reads: lane i of a group of sixteen addresses row k = 8 half + i / 4 (and + 4) of the k-step, columns
-    // 16 (group & 1) + 4 (i % 4) .. + 3; k % 4 is the same for both reads, so the exchange of the 32-row blocks is one
+    for (int ks = 0; ks < KS; ks++) koff[ks] = ((KM / 8 * ks + kp) ^ ((fr >> 1) & 7)) * 8;
+    // transposing reads: lane i of a group of sixteen addresses row k = 8 kp + i / 4 (and + 4) of the k-step, columns
+    // 16 (group & 1) (F = 32) + 4 (i % 4) .. + 3; k % 4 is the same for both reads, so the exchange of the 32-row blocks is one
     // constant per lane.  Byte offsets of this lane's first element of every block of rows:
-    const int tk = 8 * half + ((lane & 15) >> 2), tcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-    uint32_t ta[WM], tb[WN];
+    const int tk = 8 * kp + ((lane & 15) >> 2), tcol = (F == 32 ? ((lane >> 4) & 1) * 16 : 0) + (lane & 3) * 4;
+    uint32_t ta[TM], tb[TN];
 #pragma unroll
-    for (int t = 0; t < WM; t++) ta[t] = (uint32_t)(tk * BM + ((wm + t * 32) ^ (block_swizzle<BM * 2>(tk) * 8)) + tcol) * 2;
+    for (int t = 0; t < TM; t++) ta[t] = (uint32_t)(tk * BM + ((wm + t * F) ^ (place(std::integral_constant<int, BM * 2>(), tk) * 8)) + tcol) * 2;
 #pragma unroll
-    for (int t = 0; t < WN; t++) tb[t] = (uint32_t)(BM * BK + tk * BN + ((wn + t * 32) ^ (block_swizzle<BN * 2>(tk) * 8)) + tcol) * 2;
+    for (int t = 0; t < TN; t++) tb[t] = (uint32_t)(BM * BK + tk * BN + ((wn + t * F) ^ (place(std::integral_constant<int, BN * 2>(), tk) * 8)) + tcol) * 2;
     auto fragA = [&](const bf16_t* pa, uint32_t stageAddr, int t, int ks, TrFragment& o) {
-        if (AK) o.w = *(const u32x4*)(pa + (wm + t * 32 + fr) * BK + koff[ks]);
-        else tr_read<BM * 2>(stageAddr + ta[t], ks * 16 * (BM * 2), o);
+        if (AK) o.w = *(const u32x4*)(pa + (wm + t * F + fr) * BK + koff[ks]);
+        else tr_read<BM * 2>(stageAddr + ta[t], ks * KM * (BM * 2), o);
     };
     auto fragB = [&](const bf16_t* pb, uint32_t stageAddr, int t, int ks, TrFragment& o) {
-        if (BKC) o.w = *(const u32x4*)(pb + (wn + t * 32 + fr) * BK + koff[ks]);
-        else tr_read<BN * 2>(stageAddr + tb[t], ks * 16 * (BN * 2), o);
+        if (BKC) o.w = *(const u32x4*)(pb + (wn + t * F + fr) * BK + koff[ks]);
+        else tr_read<BN * 2>(stageAddr + tb[t], ks * KM * (BN * 2), o);
+    };
+    auto multiply = [&](const TrFragment& x, const TrFragment& y, Sums& o) {
+        if constexpr (F == 32) o = BigTraits<bf16_t>::mma(x.w, y.w, o);
+        else o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)&x.w, *(const bf16x8*)&y.w, o, 0, 0, 0);
     };
 
     // S stages in LDS: one is read, the S - 1 after it are fetched
@@ -334,12 +349,12 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
     };
     landed();
     const uint32_t smemAddr = (uint32_t)(uintptr_t)LDS3(smem);
-    TrFragment a[2][WM], b[2][WN];
-    [[maybe_unused]] float sums[WM][8];
+    TrFragment a[2][TM], b[2][TN];
+    [[maybe_unused]] float sums[TM][8];
     [[maybe_unused]] int turn = n0 / BN;   // stages until this tile's next
     if constexpr (SUMS) {
 #pragma unroll
-        for (int t = 0; t < WM; t++)
+        for (int t = 0; t < TM; t++)
 #pragma unroll
             for (int e = 0; e < 8; e++) sums[t][e] = 0.f;
     }
@@ -354,23 +369,23 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
         if (S == 2 ? kt + 2 == nk : kt + S >= nk) lastStage(k1);
         const uint32_t stageAddr = smemAddr + slot * STAGE * 2;
 #pragma unroll
-        for (int t = 0; t < WM; t++) fragA(pa, stageAddr, t, 0, a[0][t]);
+        for (int t = 0; t < TM; t++) fragA(pa, stageAddr, t, 0, a[0][t]);
 #pragma unroll
-        for (int t = 0; t < WN; t++) fragB(pb, stageAddr, t, 0, b[0][t]);
+        for (int t = 0; t < TN; t++) fragB(pb, stageAddr, t, 0, b[0][t]);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const int cur = ks & 1, nxt = cur ^ 1;
             // what the transposing reads of this k-step's fragments brought, by now long issued
 #pragma unroll
-            for (int t = 0; t < WM; t++)
+            for (int t = 0; t < TM; t++)
                 if (!AK) tr_wait(a[cur][t]);
 #pragma unroll
-            for (int t = 0; t < WN; t++)
+            for (int t = 0; t < TN; t++)
                 if (!BKC) tr_wait(b[cur][t]);
             if constexpr (SUMS) {
                 if (wn == 0 && turn == 0) {
 #pragma unroll
-                    for (int t = 0; t < WM; t++)
+                    for (int t = 0; t < TM; t++)
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             sums[t][2 * e] += __uint_as_float(a[cur][t].w[e] << 16);
@@ -380,17 +395,17 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
             }
             // in issue order: a product, the fragments of the next k-step spread over the products, and from the first
             // product on one fetch of the next stage each
-            constexpr int RF = (WM + WN + NMF - 1) / NMF * (AK && BKC ? 1 : 2);
+            constexpr int RF = (TM + TN + NMF - 1) / NMF * (AK && BKC ? 1 : 2);
             constexpr int FE = (PA + PB + (KS - 1) * NMF - 1) / ((KS - 1) * NMF);   // fetches per product
 #pragma unroll
             for (int q = 0; q < NMF; q++) {
-                const int i = q / WN, j = q % WN;
-                acc[i][j] = BigTraits<bf16_t>::mma(b[cur][j].w, a[cur][i].w, acc[i][j]);
+                const int i = q / TN, j = q % TN;
+                multiply(b[cur][j], a[cur][i], acc[i][j]);
                 if (ks + 1 < KS) {
 #pragma unroll
                     for (int r = q * RF; r < (q + 1) * RF; r++) {
-                        if (r < WM) fragA(pa, stageAddr, r, ks + 1, a[nxt][r]);
-                        else if (r < WM + WN) fragB(pb, stageAddr, r - WM, ks + 1, b[nxt][r - WM]);
+                        if (r < TM) fragA(pa, stageAddr, r, ks + 1, a[nxt][r]);
+                        else if (r < TM + TN) fragB(pb, stageAddr, r - TM, ks + 1, b[nxt][r - TM]);
                     }
                 }
 #pragma unroll
@@ -410,31 +425,37 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
     if constexpr (SUMS) {
         if (wn == 0) {
 #pragma unroll
-            for (int t = 0; t < WM; t++) {
+            for (int t = 0; t < TM; t++) {
                 float v = ((sums[t][0] + sums[t][1]) + (sums[t][2] + sums[t][3])) + ((sums[t][4] + sums[t][5]) + (sums[t][6] + sums[t][7]));
                 v += __shfl_xor(v, 32);
-                const int r = m0 + wm + t * 32 + fr;
-                if (half == 0 && r < M) b16_row_part(g)[(size_t)(part * g.tilesN + n0 / BN) * M + r] = v;
+                if (F == 16) v += __shfl_xor(v, 16);
+                const int r = m0 + wm + t * F + fr;
+                if (kp == 0 && r < M) b16_row_part(g)[(size_t)(part * g.tilesN + n0 / BN) * M + r] = v;
             }
         }
     }
 
-    // The products are the transposed tiles: a lane owns row lane % 32, register v is column 8 (v / 4) + 4 (lane / 32) + v % 4.
+    // The products are the transposed tiles: a lane owns row lane % F, register v is column 4 (lane / F) + v (F = 32:
+    // 8 (v / 4) + 4 (lane / 32) + v % 4).
     // Each wavefront passes 32 rows by CH tiles of columns at a time through its own slice of LDS (free after the last
     // barrier; operations of one wavefront complete in order) and the lanes walk the rows eight columns each.
     constexpr int CH = WN % 2 == 0 ? 2 : WN, CW = 32 * CH, LDC = CW + 4, LPR = CW / 8, RPI = 64 / LPR, NIT = (32 + RPI - 1) / RPI;
     float* cs = reinterpret_cast<float*>(smem_raw) + wave * 32 * LDC;
-    const int rr = lane / LPR, cc = (lane % LPR) * 8, fg = half * 4;
+    const int rr = lane / LPR, cc = (lane % LPR) * 8, fg = kp * 4;
 #pragma unroll
     for (int i = 0; i < WM; i++)
 #pragma unroll
         for (int c0 = 0; c0 < WN; c0 += CH) {
+            // 32 rows of CH tiles of 32 columns: the products' tiles in them, four columns of a row at a time
 #pragma unroll
-            for (int j = 0; j < CH; j++)
+            for (int x = 0; x < 32 / F; x++)
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    *(float4*)(cs + fr * LDC + j * 32 + 8 * q + fg) = make_float4(g.alpha * acc[i][c0 + j][4 * q], g.alpha * acc[i][c0 + j][4 * q + 1],
-                                                                                 g.alpha * acc[i][c0 + j][4 * q + 2], g.alpha * acc[i][c0 + j][4 * q + 3]);
+                for (int j = 0; j < CW / F; j++)
+#pragma unroll
+                    for (int q = 0; q < F * F / 256; q++) {
+                        const Sums& o = acc[32 / F * i + x][32 / F * c0 + j];
+                        *(float4*)(cs + (x * F + fr) * LDC + j * F + 8 * q + fg) = make_float4(g.alpha * o[4 * q], g.alpha * o[4 * q + 1], g.alpha * o[4 * q + 2], g.alpha * o[4 * q + 3]);
+                    }
             // a lane keeps its columns while it walks the rows
             const int c = n0 + wn + c0 * 32 + cc;
             float bias[8];
