@@ -104,8 +104,10 @@ static inline bool gemm_is_tiny(int m, int n, int k) { return (long long)m * n <
 //     lane that fills position s of row r fetches piece s ^ ((r >> 1) & 7)): a 128-bit read serves sixteen lanes per
 //     cycle out of 64 banks, and sixteen consecutive rows (two per 256 bytes of bank space) then fall on sixteen
 //     different bank groups.
-//   * A k-step is one A fragment and WN B fragments for WN tile products; only RB B fragments are held: fragment
+//   * A k-step is 32 rows of A and 32 WN of B; only RB fragments of B are held: fragment
 //     f + RB - 1 of the (k-step, column) sequence is read while fragment f is multiplied.
+//   * In 16 bits the products are 16 x 16 x 32, two for a fragment of B, which cost less power than 32 x 32 x 16 (gemm_bf16.hip): 8192 x
+//     2304 x 768 34.9 -> 32.5 us, 8192 x 3072 x 768 53.5 -> 48.2, 8192 x 3072 x 12288 553 -> 515, the same bits.
 // No edge handling: launched only where the tiles divide the matrix (wide_tile_fits).
 // HEADS: 0 none, 1 without a rotation, 2 with.
 template <typename T, int WN, int HEADS>
@@ -114,7 +116,8 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
                                                                int tilesTotal, HeadsEpilogue he)
 {
     typedef BigTraits<T> TR;
-    constexpr int E = TR::E, BK = 8 * E, BM = 256, BN = 32 * WN, KS = 4;   // a stage is 128 bytes of every row
+    constexpr int E = TR::E, BK = 8 * E, BM = 256, BN = 32 * WN;   // a stage is 128 bytes of every row
+    constexpr int F = sizeof(T) == 2 ? 16 : 32, TM = 32 / F, TN = WN * TM, PS = 64 / F, KS = 8 / PS;   // rows of a product; its tiles; 16-byte pieces of a row in a k-step
     constexpr int ROWS = BM + BN;                 // rows of one stage: A's 256, then B's 32 WN
     constexpr int STAGE = ROWS * BK;              // elements of one stage buffer
     constexpr int NP = (ROWS + 63) / 64;          // fetch instructions per thread and stage (a wavefront fills 8 rows with each)
@@ -128,11 +131,14 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
     const int m0 = (tile / tilesN) * BM, n0 = (tile % tilesN) * BN;
     const int wm = wave * 32;
 
-    floatx16 acc[WN];
+    typedef std::conditional_t<F == 16, floatx4, floatx16> Sums;
+    Sums acc[TM][TN];
 #pragma unroll
-    for (int j = 0; j < WN; j++)
+    for (int t = 0; t < TM; t++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[j][v] = 0.f;
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < F * F / 64; v++) acc[t][j][v] = 0.f;
 
     // fetch p of a stage: rows 64 p + 8 wave .. + 7 of the stage; this lane fills position tid & 7 of row 64 p + tid / 8.
     // The last fetch covers the 32 rows past a multiple of 64 only: wavefronts 0 .. 3.
@@ -153,33 +159,41 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the fetches have landed in LDS
     __syncthreads();
 
-    // fragment of rows base + lane % 32, k-step ks: piece 2 ks + lane / 32, kept at position piece ^ ((row >> 1) & 7)
-    const int fr = lane & 31, half = lane >> 5;
+    // fragment of rows base + lane % F, k-step ks: piece PS ks + lane / F, kept at position piece ^ ((row >> 1) & 7)
+    const int fr = lane & (F - 1), kp = lane / F;
     int koff[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) koff[ks] = ((2 * ks + half) ^ ((fr >> 1) & 7)) * E;
+    for (int ks = 0; ks < KS; ks++) koff[ks] = ((PS * ks + kp) ^ ((fr >> 1) & 7)) * E;
     const T* fa = smem + (wm + fr) * BK;
     const T* fb = smem + (BM + fr) * BK;
-    u32x4 a[2], b[RB];
+    u32x4 a[2][TM], b[RB];
     for (int kt = 0; kt < nk; kt++) {
         const T* pa = fa + (kt & 1) * STAGE;
         const T* pb = fb + (kt & 1) * STAGE;
         T* next = smem + ((kt & 1) ^ 1) * STAGE;   // read during stage kt - 1; free since the barrier that ended it
         const int k1 = min(kt + 1, nk - 1) * BK;   // past the end the last stage is fetched again (valid memory, never read)
-        a[0] = *(const u32x4*)(pa + koff[0]);
 #pragma unroll
-        for (int f = 0; f < RB - 1; f++) b[f] = *(const u32x4*)(pb + (f % WN) * 32 * BK + koff[f / WN]);
+        for (int t = 0; t < TM; t++) a[0][t] = *(const u32x4*)(pa + t * F * BK + koff[0]);
+#pragma unroll
+        for (int f = 0; f < RB - 1; f++) b[f] = *(const u32x4*)(pb + (f % TN) * F * BK + koff[f / TN]);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             // written in issue order, one scheduling region per tile product: the product, a fragment read, and with
             // each of the stage's first products one fetch of the next stage
 #pragma unroll
-            for (int j = 0; j < WN; j++) {
-                acc[j] = TR::mma(b[(ks * WN + j) % RB], a[ks & 1], acc[j]);
-                const int f = ks * WN + j + RB - 1, fks = f / WN, fj = f % WN;
-                if (fks < KS) b[f % RB] = *(const u32x4*)(pb + fj * 32 * BK + koff[fks]);
-                if (j == WN / 2 && ks + 1 < KS) a[(ks + 1) & 1] = *(const u32x4*)(pa + koff[ks + 1]);
-                const int n = ks * WN + j;
+            for (int j = 0; j < TN; j++) {
+#pragma unroll
+                for (int t = 0; t < TM; t++) {
+                    const u32x4 &x = b[(ks * TN + j) % RB], &y = a[ks & 1][t];
+                    if constexpr (F == 16) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)&x, *(const bf16x8*)&y, acc[t][j], 0, 0, 0);
+                    else acc[t][j] = TR::mma(x, y, acc[t][j]);
+                }
+                const int f = ks * TN + j + RB - 1, fks = f / TN, fj = f % TN;
+                if (fks < KS) b[f % RB] = *(const u32x4*)(pb + fj * F * BK + koff[fks]);
+                if (j == TN / 2 && ks + 1 < KS)
+#pragma unroll
+                    for (int t = 0; t < TM; t++) a[(ks + 1) & 1][t] = *(const u32x4*)(pa + t * F * BK + koff[ks + 1]);
+                const int n = ks * TN + j;
                 if (n < NP) fetch(n, k1, next);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -188,8 +202,8 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
         __syncthreads();
     }
 
-    // The products are the transposed 32x32 tiles, a lane owns row lane % 32 and
-    // register v is column 8 (v / 4) + 4 (lane / 32) + v % 4.  Each wavefront passes its 32 rows, CH tiles of columns at
+    // The products are the transposed tiles, a lane owns row lane % F and register v is column 4 (lane / F) + v (F = 32:
+    // 8 (v / 4) + 4 (lane / 32) + v % 4).  Each wavefront passes its 32 rows, CH tiles of columns at
     // a time (in fp32 three: eight slices have to fit the LDS), through its own slice of LDS (free after the last barrier) and
     // stores 16-byte pieces, dealt to the lanes in row-major order.
     constexpr int CH = sizeof(T) == 2 ? WN : 3;
@@ -198,24 +212,26 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_wide_kernel(int M, int N, int 
     // 768 into heads, 16 bits: 38.6 us with the place of every piece divided out and the bias read value by value, 36.8 so).
     constexpr int CW = 32 * CH, LDC = CW + E, LPR = 12, RPI = 5, NIT = (32 + RPI - 1) / RPI, GW = LPR * E;
     static_assert(CW % GW == 0, "whole groups of columns");
-    const int row_l = lane & 31, col_l = (lane >> 5) * 4, rr = lane / LPR, cc = (lane % LPR) * E;
+    const int col_l = kp * 4, rr = lane / LPR, cc = (lane % LPR) * E;
     const bool vecBias = ((uintptr_t)he.bias & (4 * sizeof(T) - 1)) == 0;
     T* cs = smem + wave * 32 * LDC;
 #pragma unroll
     for (int c = 0; c < WN / CH; c++) {
 #pragma unroll
-        for (int jj = 0; jj < CH; jj++)
+        for (int jj = 0; jj < CH * TM; jj++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int j = c * CH + jj;
+            for (int g = 0; g < F * F / 256; g++) {
+                const int j = c * CH * TM + jj;
                 float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (he.bias) {
-                    const T* bp = (const T*)he.bias + n0 + j * 32 + 8 * g + col_l;
+                    const T* bp = (const T*)he.bias + n0 + j * F + 8 * g + col_l;
                     if (vecBias) b = TR::ld4(bp);
                     else b = make_float4(TR::ld(bp), TR::ld(bp + 1), TR::ld(bp + 2), TR::ld(bp + 3));
                 }
-                TR::st4(cs + row_l * LDC + jj * 32 + 8 * g + col_l, alpha * acc[j][4 * g] + b.x, alpha * acc[j][4 * g + 1] + b.y,
-                        alpha * acc[j][4 * g + 2] + b.z, alpha * acc[j][4 * g + 3] + b.w);
+#pragma unroll
+                for (int t = 0; t < TM; t++)
+                    TR::st4(cs + (t * F + fr) * LDC + jj * F + 8 * g + col_l, alpha * acc[t][j][4 * g] + b.x, alpha * acc[t][j][4 * g + 1] + b.y,
+                            alpha * acc[t][j][4 * g + 2] + b.z, alpha * acc[t][j][4 * g + 3] + b.w);
             }
         // same wavefront wrote and reads, and writes the next chunk after it has read this one: LDS operations of one
         // wavefront complete in order
