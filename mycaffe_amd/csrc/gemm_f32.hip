@@ -1277,8 +1277,9 @@ __global__ __launch_bounds__(64 * NW) void linear_bwd_f32_small_kernel(GemmF32Ar
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     float* smem = reinterpret_cast<float*>(smem_raw);
-    const int tilesW = w.tilesM * w.tilesN, tilesX = x.tilesM * x.tilesN, at = runs.first[blockIdx.x % 8] + (int)(blockIdx.x / 8);
-    if (at >= runs.first[blockIdx.x % 8 + 1]) return;
+    const int tilesW = w.tilesM * w.tilesN, tilesX = x.tilesM * x.tilesN, at = runs.first[blockIdx.x % 8] + (int)(blockIdx.x / 8), end = runs.first[blockIdx.x % 8 + 1];
+    asm volatile("" : : "s"(w.K), "s"(x.K), "s"(tilesW), "s"(tilesX), "s"(at), "s"(end));   // one trip for the arguments, not one after the other
+    if (at >= end) return;
     const int item = w.K >= x.K ? at : at < tilesX ? tilesW + at : at - tilesX;
     F32Item it;
     if (item < tilesW) {
@@ -1668,8 +1669,8 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
     // time that one launch waits for the last one's stores
     const bool sumsToo = db && gemm_f32_row_sums_workspace_bytes(n, k, m, vec) > 0;   // the column sums with the weight gradient
-    const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false);
-    const double apart = dw.time + gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false).time + 2.5 +
+    const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false), dx = gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false);
+    const double apart = dw.time + dx.time + 2.5 +
                          (!db ? 0.0 : sumsToo ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
     // the one launch, fitted to 43 sizes (0.8 .. 1.24 of what was measured, 4.4 to 199 us); a tenth on top of it, as both sides are estimates
     const double together = 2.65 + (0.714 * (double)(tilesW + tilesX) + 0.458 / 128 * ((double)tilesW * m + (double)tilesX * n)) / 256 + 0.64 * std::max(m, n) / 128;
@@ -1697,9 +1698,9 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
         return e;
     }();
     if (attr != hipSuccess) return attr;
-    // Long contractions of which a CU has more than one: the calls apart cut them or add fewer values in a row, and another workgroup
-    // is there while one adds up (1024 rows, 288 to 768: 14.9 -> 15.5 us; 142 tiles of up to 2000 rows 16.0 -> 17.0, which stay as they are)
-    const bool levels = tilesW + tilesX > 256 && std::max(m, n) > 512;
+    // Long contractions that the calls apart would not give to 32 x 32 tiles: those cut them, or add fewer values in a row.  (With fewer
+    // tiles than CUs nothing else is there while one adds up: 142 tiles of up to 2000 rows 16.0 -> 17.0 us.)
+    const bool levels = tilesW + tilesX > 256 && ((dw.kernel != F32_SMALL && m > 512) || (dx.kernel != F32_SMALL && n > 512));
     int most;
     const bool wFirst = w.K >= x.K;
     const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.K, x.K) + SMALL_TILE_COST, wFirst ? tilesX : tilesW, std::min(w.K, x.K) + SMALL_TILE_COST, &most);

@@ -283,8 +283,9 @@ __global__ __launch_bounds__(64 * NW) void d_linear_bwd_small_kernel(GemmD w, Ge
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char d_smem_raw[];
     double* smem = reinterpret_cast<double*>(d_smem_raw);
-    const int at = runs.first[blockIdx.x % 8] + (int)(blockIdx.x / 8);
-    if (at >= runs.first[blockIdx.x % 8 + 1]) return;
+    const int at = runs.first[blockIdx.x % 8] + (int)(blockIdx.x / 8), end = runs.first[blockIdx.x % 8 + 1];
+    asm volatile("" : : "s"(w.k), "s"(x.k), "s"(tilesN), "s"(tilesW), "s"(tilesX), "s"(at), "s"(end));   // one trip for the arguments, not one after the other
+    if (at >= end) return;
     const int item = w.k >= x.k ? at : at < tilesX ? tilesW + at : at - tilesX;
     if (item < tilesW) d_small_tile<NW, BK, false, false, VEC, false>(w, HeadsD(), item / tilesN * 16, item % tilesN * 16, 0, db, smem);
     else d_small_tile<NW, BK, true, false, VEC, false>(x, HeadsD(), (item - tilesW) / tilesN * 16, (item - tilesW) % tilesN * 16, 0, nullptr, smem);
