@@ -1,6 +1,6 @@
-// fp32 GEMM, any operand layout, gfx950: on the 16-bit matrix cores with every value as two fp16 or three bf16 numbers
-// (gemm_f32_split_kernel, below), and on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) where that is not taken: gemm_f32_small_kernel for
-// products that do not fill the chip, gemm_f32_kernel.
+// fp32 GEMM, any operand layout, gfx950: on the bf16 matrix cores with every value as three bf16 numbers (gemm_f32_split_kernel,
+// below), and on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) where that is not taken: gemm_f32_small_kernel for products that do not
+// fill the chip, gemm_f32_kernel.
 //
 // gemm_f32_kernel serves the inner products (A B^T), their gradients (A B and A^T B) and the batched products of the explicit
 // attention chain.  2 x 2 wavefronts, each owning WM x WN MFMA tiles of 32 x 32, so a workgroup covers (64 WM) x (64 WN) of
@@ -531,212 +531,32 @@ __device__ __forceinline__ void f32_sums(const GemmF32Args& g, const float* A, c
     }
 }
 
-// PAIR: every value, scaled by a power of two, as two fp16 numbers, x 2^e = h + l / 2048, and of their products hh + (hl + lh) / 2048:
-// half the matrix instructions, and less than half the instructions that make the parts.  Two numbers of eleven bits hold a value to
-// 2^-23 of it (the sign of l is a bit), the product left out is 2^-25 of one of two values on average and 2^-22 at most.  That is more than three
-// bf16 parts leave out, but what an fp32 sum is off by is mostly its roundings, and there are half as many: against 64 bits, N(0, 1),
-// 1.4e-7 at 288 k (three parts 2.7e-7), 1.9e-7 at 768 (4.3e-7), 1.8e-7 at 3072 (3.1e-7), 1.9e-7 at 8192 (3.4e-7).
-//
-// fp16 ends at 2^-24 and 65504, so that a value's place in it matters.  l is held times 2048, in sums of its own, and is then whole
-// wherever h is above 2^-12; a workgroup scales each row by a power of two from a sample of its operands (pair_sample, pair_exponent),
-// and looks at its sums in the end (pair_holds): a wavefront whose sums hold a NaN or an infinity (a value beyond the sample by
-// more than 32 times, or its own), or are smaller than what may have been lost beside them, makes them again on the fp32 matrix cores.
-// The sample costs 2 to 3 %, the look back 2 %, knowing rows of zeros from tiny ones 2 %.
-//
-// What bounds it is power, as with three parts (operands of zeros: 107 us for 145), so every value is kept in as few instructions as there
-// are.  Two sums a result take 128 registers at 2 x 2 tiles a wavefront, which is what two wavefronts a SIMD leave room for (2 x 3 spill,
-// and with the low parts in the same sums 2 x 3 and 4 x 2 are 10 - 15 % faster still, but hold a value only to 2^-18 of the row's largest).
-// Measured, three parts and now, us: 8192 x 3072 x 768 197 -> 150, 8192 x 768 x 3072 196 -> 137, 768 x 3072 x 8192 (A^T B) 200 -> 150, 1000 x 32000 x
-// 768 250 -> 197, 4096 x 4096 x 4096 590 -> 427, 2800 x 2304 x 768 78 -> 47, 2800 x 768 x 768 36 -> 29.
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ floatx16 mma_f16(u32x4 a, u32x4 b, floatx16 c)
-{
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<half8*>(&a), *reinterpret_cast<half8*>(&b), c, 0, 0, 0);
-}
-// four values times their scales: h as two pairs, and what it leaves in v (exact); then that, times PAIR_UP, as two pairs.  Written as
-// instructions: a mixed fma multiplies, subtracts and rounds in one, where the compiler makes two.
-constexpr float PAIR_UP = 2048.f;   // h has eleven bits
-__device__ __forceinline__ uint2 pair_high(u32x4& v, float s0, float s1, float s2, float s3)
-{
-    uint2 p;
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(p.x) : "v"(v.x), "v"(s0));
-    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(p.x) : "v"(v.y), "v"(s1));
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(p.y) : "v"(v.z), "v"(s2));
-    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(p.y) : "v"(v.w), "v"(s3));
-    asm("v_fma_mix_f32 %0, %0, %1, -%2 op_sel_hi:[0,0,1]" : "+v"(v.x) : "v"(s0), "v"(p.x));
-    asm("v_fma_mix_f32 %0, %0, %1, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(v.y) : "v"(s1), "v"(p.x));
-    asm("v_fma_mix_f32 %0, %0, %1, -%2 op_sel_hi:[0,0,1]" : "+v"(v.z) : "v"(s2), "v"(p.y));
-    asm("v_fma_mix_f32 %0, %0, %1, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(v.w) : "v"(s3), "v"(p.y));
-    return p;
-}
-__device__ __forceinline__ uint2 pair_low(const u32x4& v)
-{
-    uint2 p;
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(p.x) : "v"(v.x), "s"(PAIR_UP));
-    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(p.x) : "v"(v.y), "s"(PAIR_UP));
-    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(p.y) : "v"(v.z), "s"(PAIR_UP));
-    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(p.y) : "v"(v.w), "s"(PAIR_UP));
-    return p;
-}
-__device__ __forceinline__ float pair_scale(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }   // 2^e
-
-// What a workgroup's wavefronts leave in LDS for each other, per row: the largest magnitude of its sample, as bits, the exponent of its scale,
-// and whether any value of it is not zero.
-template <int BM, int BN> struct PairState { uint32_t most[BM + BN]; uint32_t any[BM + BN]; int exponent[BM + BN]; };
-
-// Thread tid's share of the sample of an operand's `rows` rows (R in a tile) from kBegin to kEnd: of each row sixteen values, in four
-// pieces or one by one over the whole range, at other k in other rows.  Largest magnitudes to most[row], as bits.
-template <int R, int NT, bool KFAST, bool VEC> __device__ __forceinline__ void pair_sample(const float* base, long long ld, int rows, int kBegin, int kEnd, int tid, uint32_t* most)
-{
-    constexpr int COUNT = (4 * R + NT - 1) / NT, G = KFAST ? 4 : 16;
-    const int len = KFAST ? (kEnd - kBegin) / 4 : kEnd - kBegin, step = max(1, len / G);
-    u32x4 v[COUNT];
-#pragma unroll
-    for (int c = 0; c < COUNT; c++) {
-        const int e = (tid + NT * c) % (4 * R), row = KFAST ? e % R : e % (R / 4) * 4, at = KFAST ? e / R : e / (R / 4);
-        const int k = kBegin + (KFAST ? 4 : 1) * min((int)((long long)len * at / G) + row * 37 % step, max(0, len - 1));
-        if constexpr (KFAST) {
-            const uint32_t* q = (const uint32_t*)(base + (size_t)min(row, rows - 1) * ld);
-            if (VEC) v[c] = *(const u32x4*)(q + k);
-            else { v[c].x = q[k]; v[c].y = q[min(k + 1, kEnd - 1)]; v[c].z = q[min(k + 2, kEnd - 1)]; v[c].w = q[min(k + 3, kEnd - 1)]; }
-        } else {
-            const uint32_t* q = (const uint32_t*)(base + (size_t)k * ld);
-            if (VEC) v[c] = *(const u32x4*)(q + min(row, rows - 4));
-            else { v[c].x = q[min(row, rows - 1)]; v[c].y = q[min(row + 1, rows - 1)]; v[c].z = q[min(row + 2, rows - 1)]; v[c].w = q[min(row + 3, rows - 1)]; }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < COUNT; c++) {
-        const int e = (tid + NT * c) % (4 * R), row = KFAST ? e % R : e % (R / 4) * 4;
-        const uint32_t x = v[c].x & 0x7fffffffu, y = v[c].y & 0x7fffffffu, z = v[c].z & 0x7fffffffu, w = v[c].w & 0x7fffffffu;
-        if constexpr (KFAST) atomicMax(most + row, max(max(x, y), max(z, w)));
-        else { atomicMax(most + row, x); atomicMax(most + row + 1, y); atomicMax(most + row + 2, z); atomicMax(most + row + 3, w); }
-    }
-}
-// The exponent of the power of two that a row is scaled by.  It takes the largest value of the tile's sample to [2^10, 2^11), 32 times below
-// fp16's largest (gradients of a softmax over 32000 have values seven times the sample's largest); a row whose own sample is more than
-// 2^10 below that is taken up to 2^10 below (the first position's query gradient is rounding alone).
-__device__ __forceinline__ int pair_exponent(uint32_t most, uint32_t row)
-{
-    const int tile = (int)(most >> 23), gap = row ? tile - (int)(row >> 23) : 0;
-    return most ? min(max(137 - tile + max(0, gap - 10), -126), 126) : 0;
-}
-
-// Whether a wavefront's sums (scaled, of k products) hold what they should.  A value above 2^-12 after scaling is its two parts to 2^-23
-// of it, one below to 2^-36; the other factor is up to 2^11 (as far as the sample shows), so that what is lost is at most 2 k 2^-36 2^11,
-// which is what fp32 sums of k products are off by, 2^-24 sqrt(k), of a sum of 2 sqrt(k).  A smaller one may be a difference of large ones
-// (one in every thirty wavefronts of N(0, 1)): it is good as well if the magnitudes of some of its products add up to that, sixteen of them
-// where a lane has one such sum, 32 of every sum otherwise.  (32 of every sum at once, and a limit 30 times higher, took a fifth of the
-// product's time.)  Rows of zeros are exact.  False where an operand was beyond fp16, too.
-template <int WM, int WN, bool AK, bool BKC, int BM, int BN>
-__device__ __forceinline__ bool pair_holds(const GemmF32Args& g, const floatx16 (&acc)[WM][WN], const PairState<BM, BN>& st, const float* A, const float* B, int m, int n,
-                                           int wm, int wn, int kBegin, int kEnd, int lane)
-{
-    const int fr = lane & 31, half = lane >> 5;
-    const float limit = 2.f * sqrtf((float)(kEnd - kBegin));
-    float sum = 0.f, least = limit;
-#pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-        for (int j = 0; j < WN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                sum += fabsf(acc[i][j][v]);
-                least = fminf(least, fabsf(acc[i][j][v]));
-            }
-    if (__any(!(sum < __builtin_inff()))) return false;
-    if (!__any(least < limit)) return true;
-    auto column = [&](int j, int v) { return j * 32 + 8 * (v / 4) + 4 * half + v % 4; };
-    auto scaled = [&](float x, int row) { return __builtin_ldexpf(fabsf(x), st.exponent[row]); };   // a row of A, or BM + one of B
-    auto kOf = [&](int u, int of) { return kBegin + (kEnd - kBegin) / of * u + (kEnd - kBegin) % of * u / of; };
-    int at = -1, count = 0;   // a lane's first small sum, and how many it has
-#pragma unroll
-    for (int i = WM - 1; i >= 0; i--)
-#pragma unroll
-        for (int j = WN - 1; j >= 0; j--)
-#pragma unroll
-            for (int v = 15; v >= 0; v--) {
-                const bool under = fabsf(acc[i][j][v]) < limit;
-                at = under ? (i * WN + j) * 16 + v : at;
-                count += under ? 1 : 0;
-            }
-    if (!__any(count > 1)) {
-        float x[16], y[16], mag = limit;
-        if (at >= 0) {
-            const int row = at / (16 * WN) * 32 + fr, col = column(at / 16 % WN, at % 16);
-            const float* a = A + (size_t)min(m + row, g.M - 1) * (AK ? g.lda : 1);
-            const float* b = B + (size_t)min(n + col, g.N - 1) * (BKC ? g.ldb : 1);
-#pragma unroll
-            for (int u = 0; u < 16; u++) {
-                x[u] = a[(size_t)kOf(u, 16) * (AK ? 1 : g.lda)];
-                y[u] = b[(size_t)kOf(u, 16) * (BKC ? 1 : g.ldb)];
-            }
-            mag = 0.f;
-#pragma unroll
-            for (int u = 0; u < 16; u++) mag += fabsf(x[u]) * fabsf(y[u]);
-            mag = __builtin_ldexpf(mag, st.exponent[wm + row] + st.exponent[BM + wn + col]);
-        }
-        if (!__any(!(mag >= limit))) return true;
-    }
-    floatx16 mag[WM][WN];
-#pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-        for (int j = 0; j < WN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) mag[i][j][v] = 0.f;
-#pragma unroll 8
-    for (int u = 0; u < 16; u++) {
-        const int k = kOf(2 * u + half, 32);
-        float x[WM], y[WN];
-#pragma unroll
-        for (int t = 0; t < WM; t++) x[t] = scaled(A[(size_t)min(m + t * 32 + fr, g.M - 1) * (AK ? g.lda : 1) + (size_t)k * (AK ? 1 : g.lda)], wm + t * 32 + fr);
-#pragma unroll
-        for (int t = 0; t < WN; t++) y[t] = scaled(B[(size_t)min(n + t * 32 + fr, g.N - 1) * (BKC ? g.ldb : 1) + (size_t)k * (BKC ? 1 : g.ldb)], BM + wn + t * 32 + fr);
-#pragma unroll
-        for (int i = 0; i < WM; i++)
-#pragma unroll
-            for (int j = 0; j < WN; j++) mag[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[j], x[i], mag[i][j], 0, 0, 0);
-    }
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < WM; i++) {
-        const bool row = st.any[wm + i * 32 + fr] != 0;
-#pragma unroll
-        for (int j = 0; j < WN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) bad |= fabsf(acc[i][j][v]) < limit && !(mag[i][j][v] >= limit) && row && st.any[BM + wn + column(j, v)] != 0;
-    }
-    return !__any(bad);
-}
-
 // bytes of one plane of R rows by 16 KS k
 template <int R, int KS, bool KFAST> constexpr int split_plane() { return KFAST ? 2 * KS * (R * 16 + 128 / KS) : 16 * KS * R * 2; }
 
 // floats that the split kernel's stages, and then its results, take in LDS: behind them the row sums
-template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC, bool PAIR> constexpr int split_lds()
+template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC> constexpr int split_lds()
 {
-    constexpr int stages = 2 * (PAIR ? 2 : 3) * (split_plane<32 * WVM * WM, KS, AK>() + split_plane<32 * WVN * WN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
+    constexpr int stages = 2 * 3 * (split_plane<32 * WVM * WM, KS, AK>() + split_plane<32 * WVN * WN, KS, BKC>()), store = 4 * WVM * WVN * 32 * (32 * WN + 4);
     return (stages > store ? stages : store) / 4;
 }
-// where in bytes the flags lie (of PAIR the state), behind the row sums
-template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC, bool SUMS, bool PAIR> constexpr int split_flags_at()
+// where in bytes the flags lie, behind the row sums
+template <int WVM, int WVN, int WM, int WN, int KS, bool AK, bool BKC, bool SUMS> constexpr int split_flags_at()
 {
-    return 4 * split_lds<WVM, WVN, WM, WN, KS, AK, BKC, PAIR>() + (SUMS ? 64 * WVM * WVN * 16 : 0);
+    return 4 * split_lds<WVM, WVN, WM, WN, KS, AK, BKC>() + (SUMS ? 64 * WVM * WVN * 16 : 0);
 }
 // sums of op(A)'s rows over some of the k, [part][tile column][M], behind the partial products
 __device__ __forceinline__ float* f32_row_part(const GemmF32Args& g) { return g.part + (g.kChunk < g.K ? (size_t)g.parts * g.M * g.N : 0); }
 
 // SUMS: the tiles of a row of tiles also add up the rows of op(A), each the stages that are its turn, from the chunks it fetches: the
 // bias gradient beside a weight gradient (8192 rows, 768 to 2304: 169 us one after the other, 157 together).
-template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS, bool PAIR>
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS>
 __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(GemmF32Args g, HeadsArg<HEADS> hp)
 {
-    constexpr int PARTS = PAIR ? 2 : 3;
     constexpr int NT = 64 * WVM * WVN, BK = 16 * KS, BM = 32 * WVM * WM, BN = 32 * WVN * WN;
     constexpr int PA = (BM * BK / 4 + NT - 1) / NT, PB = (BN * BK / 4 + NT - 1) / NT, P = PA + PB;   // chunks of four values per thread and stage
     constexpr int KGA = BM * 16 + 128 / KS, KGB = BN * 16 + 128 / KS;                                  // bytes between groups of eight k
-    constexpr int PLA = split_plane<BM, KS, AK>(), PLB = split_plane<BN, KS, BKC>(), STAGE = PARTS * (PLA + PLB);
+    constexpr int PLA = split_plane<BM, KS, AK>(), PLB = split_plane<BN, KS, BKC>(), STAGE = 3 * (PLA + PLB);
     constexpr int NMF = WM * WN;
     static_assert(PA * NT == BM * BK / 4 && (KS == 1 || KS % 2 == 0), "whole chunks of A; fragments change registers from k-step to k-step");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -758,15 +578,6 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
         for (int j = 0; j < WN; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-    floatx16 cross[PAIR ? WM : 1][PAIR ? WN : 1];   // h l + l h, times PAIR_UP
-    if constexpr (PAIR) {
-#pragma unroll
-        for (int i = 0; i < WM; i++)
-#pragma unroll
-            for (int j = 0; j < WN; j++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) cross[i][j][v] = 0.f;
-    }
 
     // Chunk e of a stage, k at unit stride: row e / (BK / 4), k = 4 (e % (BK / 4)); row index at unit stride: k = e / (rows / 4),
     // rows 4 (e % (rows / 4)) .. + 3.  Where B's chunks do not divide by the threads, the last threads repeat earlier chunks.
@@ -798,11 +609,11 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
         const int e = chunkB(p);
         if (BKC) {
             vb[p] = 4 * ((uint32_t)min(e / CK, N - 1 - n0) * (uint32_t)g.ldb + 4 * (e % CK));
-            wb[p] = PARTS * PLA + (e % CK / 2) * KGB + (e / CK) * 16 + (e & 1) * 8;
+            wb[p] = 3 * PLA + (e % CK / 2) * KGB + (e / CK) * 16 + (e & 1) * 8;
         } else {
             const int k = e / (BN / 4), row = 4 * (e % (BN / 4));
             vb[p] = 4 * ((uint32_t)k * (uint32_t)g.ldb + min(row, VEC ? N - 4 - n0 : (N - 1 - n0) & ~3));
-            wb[p] = PARTS * PLA + (k * BN + (row ^ (block_swizzle<BN * 2>(k) * 8))) * 2;
+            wb[p] = 3 * PLA + (k * BN + (row ^ (block_swizzle<BN * 2>(k) * 8))) * 2;
         }
     }
     auto resource = [](const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(OUTSIDE - 16), 0x00020000); };
@@ -854,18 +665,9 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
     [[maybe_unused]] float sums[4] = {0.f, 0.f, 0.f, 0.f};
     [[maybe_unused]] int turn = n0 / BN, putting = 0;   // the stage that is put, and stages until this tile's next
     [[maybe_unused]] uint32_t mine = turn == 0 ? 0xffffffffu : 0u;
-    [[maybe_unused]] uint32_t rest = 0;      // of all values, or-ed: what the last part is made of
-    unsigned char* const state = smem_raw + split_flags_at<WVM, WVN, WM, WN, KS, AK, BKC, SUMS, PAIR>();
-    [[maybe_unused]] SplitFlags* flags = reinterpret_cast<SplitFlags*>(state);
-    using State = PairState<BM, BN>;
-    [[maybe_unused]] State* pair = reinterpret_cast<State*>(state);
-    // PAIR: per row, or-ed over its k.  A thread's chunks are of one row each, or all of the same four rows.
-    static_assert(!PAIR || (NT % (BM / 4) == 0 && NT % (BN / 4) == 0 && PB * NT == BN * BK / 4 && PA % 2 == 0 && PB % 2 == 0), "");
-    [[maybe_unused]] uint32_t anyA[AK ? PA : 4] = {}, anyB[BKC ? PB : 4] = {};
-    [[maybe_unused]] float scaleA[AK ? PA : 4], scaleB[BKC ? PB : 4];   // of those rows
-    auto rowA = [&](int p) { return AK ? (tid + NT * p) / CK : 4 * (tid % (BM / 4)) + p; };
-    auto rowB = [&](int p) { return BKC ? (tid + NT * p) / CK : 4 * (tid % (BN / 4)) + p; };
-    if (!PAIR && tid == 0) *flags = SplitFlags{0, 0};
+    uint32_t rest = 0;      // of all values, or-ed: what the last part is made of
+    SplitFlags* flags = reinterpret_cast<SplitFlags*>(smem_raw + split_flags_at<WVM, WVN, WM, WN, KS, AK, BKC, SUMS>());
+    if (tid == 0) *flags = SplitFlags{0, 0};
     // part s of chunk c to its plane of a stage
     auto put = [&](int c, int s, unsigned char* stage) {
         if constexpr (SUMS) {
@@ -873,26 +675,6 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
                 sums[0] += __uint_as_float(raw[c].x & mine); sums[1] += __uint_as_float(raw[c].y & mine);
                 sums[2] += __uint_as_float(raw[c].z & mine); sums[3] += __uint_as_float(raw[c].w & mine);
             }
-        }
-        if constexpr (PAIR) {
-            if (s == 0) {
-                if (c < PA ? AK : BKC) {
-                    uint32_t& a = c < PA ? anyA[AK ? c : 0] : anyB[BKC ? c - PA : 0];
-                    or3(a, raw[c].x, raw[c].y);
-                    or3(a, raw[c].z, raw[c].w);
-                } else {
-                    uint32_t* a = c < PA ? anyA : anyB;
-                    if ((c < PA ? c : c - PA) % 2 == 0) {   // with the next chunk's: half the instructions
-                        or3(a[0], raw[c].x, raw[c + 1].x); or3(a[1], raw[c].y, raw[c + 1].y);
-                        or3(a[2], raw[c].z, raw[c + 1].z); or3(a[3], raw[c].w, raw[c + 1].w);
-                    }
-                }
-            }
-            const bool rows4 = c < PA ? !AK : !BKC;
-            const float* f = c < PA ? scaleA + (AK ? c : 0) : scaleB + (BKC ? c - PA : 0);
-            const uint2 p = s == 0 ? pair_high(raw[c], f[0], f[rows4 ? 1 : 0], f[rows4 ? 2 : 0], f[rows4 ? 3 : 0]) : pair_low(raw[c]);
-            *(uint2*)(stage + (c < PA ? wa[c] + s * PLA : wb[c - PA] + s * PLB)) = p;
-            return;
         }
         float v[4] = {__uint_as_float(raw[c].x), __uint_as_float(raw[c].y), __uint_as_float(raw[c].z), __uint_as_float(raw[c].w)};
         if (s == 2) {
@@ -913,7 +695,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
         ta[t] = AK ? half * KGA + (wm + t * 32 + fr) * 16 : (tk * BM + ((wm + t * 32) ^ (block_swizzle<BM * 2>(tk) * 8)) + tcol) * 2;
 #pragma unroll
     for (int t = 0; t < WN; t++)
-        tb[t] = PARTS * PLA + (BKC ? half * KGB + (wn + t * 32 + fr) * 16 : (tk * BN + ((wn + t * 32) ^ (block_swizzle<BN * 2>(tk) * 8)) + tcol) * 2);
+        tb[t] = 3 * PLA + (BKC ? half * KGB + (wn + t * 32 + fr) * 16 : (tk * BN + ((wn + t * 32) ^ (block_swizzle<BN * 2>(tk) * 8)) + tcol) * 2);
     const uint32_t smemAddr = (uint32_t)(uintptr_t)LDS3(smem_raw);
     // part s of k-step ks of the stage at `at`
     auto readA = [&](TrFragment (&f)[WM], int at, int ks, int s) {
@@ -943,39 +725,14 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
 #pragma unroll
     for (int c = 0; c < P; c++) fetch(c);
     nextStage();
-    if constexpr (PAIR) {
-        for (int i = tid; i < BM + BN; i += NT) pair->most[i] = pair->any[i] = 0;
-        __syncthreads();
-        if (kEnd > kBegin) {
-            pair_sample<BM, NT, AK, VEC>(baseA, g.lda, M - m0, kBegin, kEnd, tid, pair->most);
-            pair_sample<BN, NT, BKC, VEC>(baseB, g.ldb, N - n0, kBegin, kEnd, tid, pair->most + BM);
-        }
-        __syncthreads();
-        uint32_t mostA = 0, mostB = 0;
-#pragma unroll
-        for (int r = 0; r < BM; r += 64) mostA = max(mostA, pair->most[r + lane]);
-#pragma unroll
-        for (int r = 0; r < BN; r += 64) mostB = max(mostB, pair->most[BM + r + lane]);
-#pragma unroll
-        for (int o = 32; o; o >>= 1) {
-            mostA = max(mostA, (uint32_t)__shfl_xor((int)mostA, o));
-            mostB = max(mostB, (uint32_t)__shfl_xor((int)mostB, o));
-        }
-#pragma unroll
-        for (int p = 0; p < (AK ? PA : 4); p++) scaleA[p] = pair_scale(pair_exponent(mostA, pair->most[rowA(p)]));
-#pragma unroll
-        for (int p = 0; p < (BKC ? PB : 4); p++) scaleB[p] = pair_scale(pair_exponent(mostB, pair->most[BM + rowB(p)]));
-        for (int r = tid; r < BM + BN; r += NT) pair->exponent[r] = pair_exponent(r < BM ? mostA : mostB, pair->most[r]);   // for the end
-    }
 #pragma unroll
     for (int c = 0; c < P; c++) {
 #pragma unroll
-        for (int s = 0; s < PARTS; s++) put(c, s, smem_raw);
+        for (int s = 0; s < 3; s++) put(c, s, smem_raw);
         fetch(c);
     }
     __syncthreads();
-    TrFragment ah[2][WM], bh[2][WN], al[WM], bl[WN];
-    [[maybe_unused]] TrFragment am[WM], bm[WN];
+    TrFragment ah[2][WM], bh[2][WN], am[WM], bm[WN], al[WM], bl[WN];
     readA(ah[0], 0, 0, 0);
     readB(bh[0], 0, 0, 0);
     arrived(ah[0], bh[0]);
@@ -990,55 +747,39 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             mine = turn == 0 && putting < nk ? 0xffffffffu : 0u;   // past the end the last stage is put again
         }
         // what goes between the products: chunks of the next stage part by part to the other buffer, each then fetched anew
-        constexpr int SLOTS = (PAIR ? 3 * KS - 1 : 6 * KS - 2) * NMF, STEPS = PARTS * P;
+        constexpr int SLOTS = (6 * KS - 2) * NMF, STEPS = 3 * P;
         auto slot = [&](int q) {
 #pragma unroll
             for (int st = STEPS * q / SLOTS; st < STEPS * (q + 1) / SLOTS; st++) {
-                put(st / PARTS, st % PARTS, next);
-                if (st % PARTS == PARTS - 1) fetch(st / PARTS);
+                put(st / 3, st % 3, next);
+                if (st % 3 == 2) fetch(st / 3);
             }
             __builtin_amdgcn_sched_barrier(0);
         };
-        auto kstep = [&](auto number) {   // (a loop of this length is not unrolled)
-            constexpr int ks = decltype(number)::value;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
             const int cur = (KS * u + ks) & 1, nxt = cur ^ 1;
-            int q = ks * (PAIR ? 3 : 6) * NMF;
+            int q = ks * 6 * NMF;
             auto products = [&](TrFragment (&a)[WM], TrFragment (&b)[WN], bool fill) {
 #pragma unroll
                 for (int t = 0; t < NMF; t++) {
                     // the transposed tile (B as the row operand): a lane owns a row of C
-                    acc[t / WN][t % WN] = PAIR ? mma_f16(b[t % WN].w, a[t / WN].w, acc[t / WN][t % WN]) : BigTraits<bf16_t>::mma(b[t % WN].w, a[t / WN].w, acc[t / WN][t % WN]);
+                    acc[t / WN][t % WN] = BigTraits<bf16_t>::mma(b[t % WN].w, a[t / WN].w, acc[t / WN][t % WN]);
                     if (fill) slot(q + t);
                 }
                 q += NMF;
             };
-            [[maybe_unused]] auto crossed = [&](TrFragment (&a)[WM], TrFragment (&b)[WN], bool fill) {
-#pragma unroll
-                for (int t = 0; t < NMF; t++) {
-                    floatx16& c = cross[PAIR ? t / WN : 0][PAIR ? t % WN : 0];
-                    c = mma_f16(b[t % WN].w, a[t / WN].w, c);
-                    if (fill) slot(q + t);
-                }
-                q += NMF;
-            };
-            if constexpr (!PAIR) {
-                readA(am, at, ks, 1);
-                readB(bm, at, ks, 1);
-                products(ah[cur], bh[cur], true);
-                arrived(am, bm);
-                readA(al, at, ks, 2);
-                readB(bl, at, ks, 2);
-                products(ah[cur], bm, true);
-                products(am, bh[cur], true);
-                products(am, bm, true);
-            } else {
-                readA(al, at, ks, 1);
-                readB(bl, at, ks, 1);
-                products(ah[cur], bh[cur], true);
-            }
+            readA(am, at, ks, 1);
+            readB(bm, at, ks, 1);
+            products(ah[cur], bh[cur], true);
+            arrived(am, bm);
+            readA(al, at, ks, 2);
+            readB(bl, at, ks, 2);
+            products(ah[cur], bm, true);
+            products(am, bh[cur], true);
+            products(am, bm, true);
             arrived(al, bl);
-            if constexpr (PAIR) crossed(ah[cur], bl, true);
-            if constexpr (ks + 1 < KS) {
+            if (ks + 1 < KS) {
                 readA(ah[nxt], at, ks + 1, 0);
                 readB(bh[nxt], at, ks + 1, 0);
             } else {
@@ -1047,23 +788,17 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
                 readB(bh[nxt], STAGE - at, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (PAIR) crossed(al, bh[cur], ks + 1 < KS);
-            else {
-                products(ah[cur], bl, ks + 1 < KS);
-                products(al, bh[cur], ks + 1 < KS);
-            }
+            products(ah[cur], bl, ks + 1 < KS);
+            products(al, bh[cur], ks + 1 < KS);
             arrived(ah[nxt], bh[nxt]);
-        };
-        kstep(std::integral_constant<int, 0>());
-        if constexpr (KS > 1) kstep(std::integral_constant<int, 1>());
-        static_assert(KS <= 2, "");
+        }
     };
     for (int kt = 0; kt < nk; kt += 2) {
         stage(0);
         if (kt + 1 < nk) stage(1);
     }
     if constexpr (SUMS) {
-        float* all = reinterpret_cast<float*>(smem_raw) + split_lds<WVM, WVN, WM, WN, KS, AK, BKC, PAIR>();
+        float* all = reinterpret_cast<float*>(smem_raw) + split_lds<WVM, WVN, WM, WN, KS, AK, BKC>();
         *(float4*)(all + 4 * tid) = make_float4(sums[0], sums[1], sums[2], sums[3]);
         __syncthreads();
         if (tid < BM && m0 + tid < M) {
@@ -1072,29 +807,6 @@ __global__ __launch_bounds__(64 * WVM * WVN, OCC) void gemm_f32_split_kernel(Gem
             for (int w = 0; w < NT / (BM / 4); w++) v += all[w * BM + tid];
             f32_row_part(g)[(size_t)(it.part * g.tilesN + n0 / BN) * M + m0 + tid] = v;
         }
-    }
-    if constexpr (PAIR) {
-#pragma unroll
-        for (int p = 0; p < (AK ? PA : 4); p++) atomicOr(&pair->any[rowA(p)], anyA[p] & 0x7fffffffu);
-#pragma unroll
-        for (int p = 0; p < (BKC ? PB : 4); p++) atomicOr(&pair->any[BM + rowB(p)], anyB[p] & 0x7fffffffu);
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < NMF; t++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[t / WN][t % WN][v] += cross[PAIR ? t / WN : 0][PAIR ? t % WN : 0][v] * (1.f / PAIR_UP);
-        if (pair_holds<WM, WN, AK, BKC, BM, BN>(g, acc, *pair, A, B, m0 + wm, n0 + wn, wm, wn, kBegin, kEnd, lane)) {
-#pragma unroll
-            for (int t = 0; t < NMF; t++) {
-                const int e = pair->exponent[wm + t / WN * 32 + fr];
-#pragma unroll
-                for (int v = 0; v < 16; v++)
-                    acc[t / WN][t % WN][v] = __builtin_ldexpf(acc[t / WN][t % WN][v], -e - pair->exponent[BM + wn + t % WN * 32 + 8 * (v / 4) + 4 * half + v % 4]);
-            }
-            if (!VEC && kEnd < it.kEnd) f32_sums<WM, WN, AK, BKC, true>(g, A, B, m0 + wm, n0 + wn, kEnd, it.kEnd, lane, acc);
-        } else f32_sums<WM, WN, AK, BKC, false>(g, A, B, m0 + wm, n0 + wn, kBegin, it.kEnd, lane, acc);
-        f32_store<WM, WN, HEADS>(g, hp, acc, reinterpret_cast<float*>(smem_raw) + wave * 32 * (32 * WN + 4), lane, m0 + wm, n0 + wn, it.part, it.batch);
-        return;
     }
     if (rest & 0xffffu) flags->lost = 1;
     __syncthreads();
@@ -1422,21 +1134,6 @@ static GemmF32Plan gemm_f32_split_plan(int m, int n, int k, int batch, bool caus
     });
 }
 
-// The same of its form with two fp16 numbers, by 3000 measurements of 37 sizes; 1 % from the best tile and parts on average, 7 % at most.
-static const int g_pairTile[4][2] = {{256, 128}, {128, 128}, {64, 128}, {64, 64}};   // of its form with two fp16 numbers
-static GemmF32Plan gemm_f32_pair_plan(int m, int n, int k, size_t wsBytes, double* estimate)
-{
-    struct Fit { double stage, ends, loadStage, loadEnds, once; };
-    static const struct { Fit alone, shared; } fit[4] = {
-        {{0.863, 0, 0.59, 1.9, 14.1}, {1.006, 8.3, 0.546, 4.5, 1.8}}, {{0.811, 12.2, 0.153, 1.7, 0}, {0.437, 5.0, 0.441, 0, 5.3}},
-        {{0.619, 8.4, 0.056, 1.5, 0}, {0.342, 0.8, 0.188, 1.4, 7.4}}, {{0.426, 0, 0.064, 0.3, 6.9}, {0.253, 0, 0.065, 1.04, 6.8}}};
-    return best_plan(m, n, k, 1, false, wsBytes, 4, g_pairTile, estimate, [](int sh, long long items, long long perCu, int chunk) {
-        const Fit& f = perCu == 1 ? fit[sh].alone : fit[sh].shared;
-        const double nk = (chunk + 31) / 32, load = items / 256.0;
-        return perCu * (nk * f.stage + f.ends) + load * (nk * f.loadStage + f.loadEnds) + f.once;
-    });
-}
-
 // gemm_f32_small_kernel, microseconds: what the workgroups of the busiest CU take for their products, and what each three of them that
 // run at once (by LDS) take for their stages' latencies.  Within 10 % of 34 sizes.
 static double gemm_f32_small_time(long long tiles, int k)
@@ -1449,14 +1146,10 @@ static double gemm_f32_small_time(long long tiles, int k)
 // operands while some of the result is written, the small tiles of one part of the rows and columns each, the split one once more
 // for a wavefront whose parts lost something.)  The bf16 matrix cores from 64 k on (below, the split's error is larger than that of the
 // fp32 matrix cores) and from 2^28 multiplications on (2048 x 512 x 384: 10.2 against 11.0 us; below, the chip is not full, and 16 x 288 x
-// 32000 takes 51 against 44 us); there as two fp16 numbers a value where that is estimated to take less time, from some 300 k on (its start and end
-// cost 5 us a tile more: 7588 x 4340 x 64 takes 50 us against 48, 2544 x 1816 x 1164 60 against 85), and not in the batches of the explicit
-// attention, whose operands are read and written at the memory's rate and hold softmax weights of any magnitude; 32 x 32 tiles where their
-// estimate is the smallest, which is a tenth of a round of the larger ones.
-enum { F32_TILES, F32_SPLIT, F32_SMALL, F32_PAIR };
-enum F32Pairs { NO_PAIRS, PAIRS, PAIRS_FIRST };   // what may go as two fp16 numbers: nothing; what is faster so; whatever three parts take
+// 32000 takes 51 against 44 us); 32 x 32 tiles where their estimate is the smallest, which is a tenth of a round of the larger ones.
+enum { F32_TILES, F32_SPLIT, F32_SMALL };
 struct GemmF32Choice { int kernel; GemmF32Plan plan; double time; };
-static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool fp32Sums, bool heads = false, F32Pairs pairs = PAIRS)
+static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal, size_t wsBytes, bool fp32Sums, bool heads = false)
 {
     GemmF32Choice c;
     c.kernel = F32_TILES;
@@ -1465,11 +1158,6 @@ static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal
     if (k >= 64 && (double)m * n * k * batch >= 268435456.0) {   // faster than the fp32 matrix cores at every size from there on
         c.kernel = F32_SPLIT;
         c.plan = gemm_f32_split_plan(m, n, k, batch, causal, wsBytes, &c.time);
-        if (pairs != NO_PAIRS && batch == 1 && !causal) {
-            double t;
-            const GemmF32Plan p = gemm_f32_pair_plan(m, n, k, wsBytes, &t);
-            if (heads || pairs == PAIRS_FIRST || t < c.time) c = {F32_PAIR, p, t};   // (the epilogues of the larger products exist in that form)
-        }
     }
     c.time += 1.8;   // a launch, which the next estimate holds
     // the heads epilogue of 16 rows and more a lane, one after the other (1024 x 864 x 288: 13.3 us, 9.3 without it)
@@ -1481,8 +1169,8 @@ static GemmF32Choice gemm_f32_choose(int m, int n, int k, int batch, bool causal
 
 int gemm_f32_route(int m, int n, int k, int batch, bool causal, bool fp32Sums, bool heads)
 {
-    const GemmF32Choice c = gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, fp32Sums, heads, NO_PAIRS), p = gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, fp32Sums, heads);
-    return c.kernel + 4 * c.plan.shape + 64 * c.plan.splits + (p.kernel == F32_PAIR ? (1 + p.plan.shape) << 16 | p.plan.splits << 20 : 0);
+    const GemmF32Choice c = gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, fp32Sums, heads);
+    return c.kernel + 4 * c.plan.shape + 64 * c.plan.splits;
 }
 
 // 31-bit byte offsets within a tile's rows of k (256 at most), or within the k rows of a stage (128)
@@ -1492,21 +1180,20 @@ size_t gemm_f32_workspace_bytes(int m, int n, int k, int batch, bool causal)
 {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
     // which kernel takes it depends on the caller too: enough for any
-    int splits = gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, false).plan.splits;
-    for (bool fp32Sums : {true, false}) splits = std::max(splits, gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, fp32Sums, true).plan.splits);
+    const int splits = std::max(gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, false).plan.splits, gemm_f32_choose(m, n, k, batch, causal, SIZE_MAX, true).plan.splits);
     return splits > 1 ? (size_t)splits * m * n * sizeof(float) : 0;
 }
 
 // With the sums of op(A)'s rows: the partial products (none where the contraction is not cut), then the partial sums.  0: not together,
 // because another kernel takes the product, because a sum would be longer than the column sums' own (128 values in each of eight
 // accumulators and more a row and tile), or because one short launch (up to 1024 k) would only be another.
-static int pair_tile_columns(int shape, int n) { return (n + g_pairTile[shape][1] - 1) / g_pairTile[shape][1]; }
+static int split_tile_columns(int shape, int n) { return (n + g_splitTile[shape][1] - 1) / g_splitTile[shape][1]; }
 size_t gemm_f32_row_sums_workspace_bytes(int m, int n, int k, bool vec)
 {
     if (m <= 0 || n <= 0 || k <= 0 || !vec || !f32_near(false, m, k, m) || !f32_near(false, n, k, n)) return 0;
-    const GemmF32Choice c = gemm_f32_choose(m, n, k, 1, false, SIZE_MAX, false, false, PAIRS_FIRST);
-    if (c.kernel != F32_PAIR || (k <= 1024 && c.plan.splits == 1)) return 0;
-    const int columns = pair_tile_columns(c.plan.shape, n);
+    const GemmF32Choice c = gemm_f32_choose(m, n, k, 1, false, SIZE_MAX, false);
+    if (c.kernel != F32_SPLIT || (k <= 1024 && c.plan.splits == 1)) return 0;
+    const int columns = split_tile_columns(c.plan.shape, n);
     if (c.plan.kChunk / (8 * columns) > 128) return 0;
     return ((c.plan.splits > 1 ? (size_t)c.plan.splits * m * n : 0) + (size_t)c.plan.splits * columns * m) * sizeof(float);
 }
@@ -1542,14 +1229,13 @@ static hipError_t launch_f32_tile(hipStream_t s, const GemmF32Args& a, const Gem
 // the shapes of gemm_f32_split_kernel, in the order of gemm_f32_split_plan: wavefronts, tiles of a wavefront, k-steps of a stage,
 // wavefronts of a SIMD that the registers are to hold
 #define SPLIT_SHAPES(X) X(0, 2, 4, 4, 2, 1, 2) X(1, 4, 2, 2, 3, 1, 2) X(2, 2, 2, 2, 3, 1, 2) X(3, 2, 2, 2, 2, 1, 2) X(4, 2, 2, 1, 2, 2, 2) X(5, 2, 2, 1, 1, 2, 2)
-#define PAIR_SHAPES(X) X(0, 4, 2, 2, 2, 2, 2) X(1, 2, 2, 2, 2, 2, 2) X(2, 2, 2, 1, 2, 2, 2) X(3, 2, 2, 1, 1, 2, 2)
 
-template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS, bool PAIR>
+template <int WVM, int WVN, int WM, int WN, int KS, int OCC, bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS>
 static hipError_t launch_split(hipStream_t s, GemmF32Args& g, int splits, int batch, const HeadsEpilogue* he)
 {
     constexpr int BM = 32 * WVM * WM, BN = 32 * WVN * WN;
-    constexpr int lds = split_flags_at<WVM, WVN, WM, WN, KS, AK, BKC, SUMS, PAIR>() + (int)(PAIR ? sizeof(PairState<BM, BN>) : sizeof(SplitFlags));
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    constexpr int lds = split_flags_at<WVM, WVN, WM, WN, KS, AK, BKC, SUMS>() + (int)sizeof(SplitFlags);
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     g.tilesM = (g.M + BM - 1) / BM;
     g.tilesN = (g.N + BN - 1) / BN;
@@ -1557,27 +1243,16 @@ static hipError_t launch_split(hipStream_t s, GemmF32Args& g, int splits, int ba
     const long long total = (long long)g.tilesM * g.tilesN * g.parts;
     if (total > (1ll << 27)) return hipErrorInvalidValue;
     const int per = (int)((total + 7) / 8);
-    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS, PAIR>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
+    hipLaunchKernelGGL((gemm_f32_split_kernel<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>), dim3(per * 8), 64 * WVM * WVN, lds, s, g, heads_arg<HEADS>(he));
     return hipGetLastError();
 }
 
-template <bool AK, bool BKC, bool VEC>
-static hipError_t launch_split_shape(hipStream_t s, GemmF32Args& a, const GemmF32Plan& p, int batch)
-{
-    switch (p.shape) {
-#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, false, false, false>(s, a, p.splits, batch, nullptr);
-        SPLIT_SHAPES(X)
-#undef X
-    }
-    return hipErrorInvalidValue;
-}
-
 template <bool AK, bool BKC, bool VEC, bool HEADS, bool SUMS = false>
-static hipError_t launch_pair_shape(hipStream_t s, GemmF32Args& a, const GemmF32Plan& p, const HeadsEpilogue* he = nullptr)
+static hipError_t launch_split_shape(hipStream_t s, GemmF32Args& a, const GemmF32Plan& p, int batch, const HeadsEpilogue* he = nullptr)
 {
     switch (p.shape) {
-#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS, true>(s, a, p.splits, 1, he);
-        PAIR_SHAPES(X)
+#define X(I, WVM, WVN, WM, WN, KS, OCC) case I: return launch_split<WVM, WVN, WM, WN, KS, OCC, AK, BKC, VEC, HEADS, SUMS>(s, a, p.splits, batch, he);
+        SPLIT_SHAPES(X)
 #undef X
     }
     return hipErrorInvalidValue;
@@ -1609,9 +1284,7 @@ template <bool AK, bool BKC, bool VEC, bool HEADS>
 static hipError_t launch_layout(hipStream_t s, GemmF32Args& a, const GemmF32Choice& c, int batch, const HeadsEpilogue* he)
 {
     if (c.kernel == F32_SMALL) return launch_small<4, 64, AK, BKC, VEC, HEADS>(s, a, batch, he);
-    if (c.kernel == F32_PAIR) return launch_pair_shape<AK, BKC, VEC, HEADS>(s, a, c.plan, he);
-    if constexpr (!HEADS)
-        if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, VEC>(s, a, c.plan, batch);
+    if (c.kernel == F32_SPLIT) return launch_split_shape<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
     return launch_f32_tile<AK, BKC, VEC, HEADS>(s, a, c.plan, batch, he);
 }
 
@@ -1645,18 +1318,18 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     const bool vec = near && (((uintptr_t)q.A | (uintptr_t)q.B) & 15) == 0 && q.lda % 4 == 0 && q.ldb % 4 == 0 && (q.batch == 1 || (q.sA % 4 == 0 && q.sB % 4 == 0)) &&
                      (q.aK ? q.k % 4 == 0 : q.m % 4 == 0) && (q.bK ? q.k % 4 == 0 : q.n % 4 == 0);
     if (!ws || ((uintptr_t)ws & 15)) wsBytes = 0;
-    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, q.fp32Sums || !near || gemm_f32_shares(q), q.heads != nullptr, q.rowSum ? PAIRS_FIRST : PAIRS);
+    const GemmF32Choice choice = gemm_f32_choose(q.m, q.n, q.k, q.batch, q.causal != 0, wsBytes, q.fp32Sums || !near || gemm_f32_shares(q), q.heads != nullptr);
     const GemmF32Plan& p = choice.plan;
     a.kChunk = p.kChunk;
     if (q.rowSum) {
         const size_t need = gemm_f32_row_sums_workspace_bytes(q.m, q.n, q.k, vec && !q.aK && !q.bK && q.lda == q.m && q.ldb == q.n && q.batch == 1 && !q.fp32Sums);
-        if (need == 0 || wsBytes < need || choice.kernel != F32_PAIR) return hipErrorInvalidValue;
+        if (need == 0 || wsBytes < need || choice.kernel != F32_SPLIT) return hipErrorInvalidValue;
     }
     // rows shorter than the three values that a chunk may read past one: so many more k
     auto past = [&](bool kFast, int rows, long long ld) { return kFast ? q.k % 4 : rows % 4 == 0 ? 0 : ld >= 3 ? 1 : 3; };
     a.kTail = std::max(past(q.aK, q.m, q.lda), past(q.bK, q.n, q.ldb));
     hipError_t e;
-    if (q.rowSum) e = launch_pair_shape<false, false, true, false, true>(s, a, p);
+    if (q.rowSum) e = launch_split_shape<false, false, true, false, true>(s, a, p, 1);
     else if (q.heads) e = vec ? launch_layout<true, true, true, true>(s, a, choice, 1, q.heads) : launch_layout<true, true, false, true>(s, a, choice, 1, q.heads);
 #define LAYOUT(AKV, BKV) (vec ? launch_layout<AKV, BKV, true, false>(s, a, choice, q.batch, nullptr) : launch_layout<AKV, BKV, false, false>(s, a, choice, q.batch, nullptr))
     else if (q.aK) e = q.bK ? LAYOUT(true, true) : LAYOUT(true, false);

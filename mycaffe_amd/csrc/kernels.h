@@ -169,8 +169,7 @@ hipError_t k_gemm2(hipStream_t s, bool tA, bool tB, int m, int n, int k, float a
 size_t k_gemv_workspace_bytes(bool tA, int m, int n);   // scratch for the partial sums of a transposed product over many rows
 hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, const void* A, const float* x,
                   float beta, float* y, void* ws = nullptr, size_t wsBytes = 0);
-// which kernel an fp32 product goes to (0 gemm_f32_kernel, 1 gemm_f32_split_kernel, 2 gemm_f32_small_kernel) + 4 its tile + 64 parts of the contraction;
-// where two fp16 numbers a value take it before those, + 2^16 (1 + tile) + 2^20 parts
+// which kernel an fp32 product goes to (0 gemm_f32_kernel, 1 gemm_f32_split_kernel, 2 gemm_f32_small_kernel) + 4 its tile + 64 parts of the contraction
 int gemm_f32_route(int m, int n, int k, int batch, bool causal, bool fp32Sums, bool heads);
 int gemm_b16_route(int m, int n, int k);   // the same of a 16-bit product that goes to gemm_b16_kernel (0)
 hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float* X, const float* W, const float* dY, float* dW, float* db, float* dX, float beta,
