@@ -1050,7 +1050,7 @@ hipError_t attn_flash_launch(hipStream_t s, DType dt, const AttnArgs& a, bool* h
         // 31 us, pairs of wavefronts 35; 10 x 2048: 92 and 103; 24 x 1024: 71 and 54)
         const int nbh = a.B * a.H, b128 = (a.Tq + 127) / 128, b64 = (a.Tq + 63) / 64;
         const long long blocks = (long long)nbh * b128;
-        if (a.kind == MASK_CAUSAL && !a.lse2 && a.Tq == a.Tk && (blocks <= 128 || (blocks < 256 && (a.oneWave || (long long)nbh * (b64 + 1) <= 330)))) {
+        if (a.kind == MASK_CAUSAL && !a.lse2 && !a.oneWave && a.Tq == a.Tk && (blocks <= 128 || (blocks < 256 && (long long)nbh * (b64 + 1) <= 330))) {
             hipLaunchKernelGGL(flash_short_causal_f32_kernel, dim3((a.Tq + 31) / 32, a.H, a.B), 256, 0, s, f);
             return hipGetLastError();
         }

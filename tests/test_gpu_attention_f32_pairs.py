@@ -78,9 +78,10 @@ def test_a_step_of_scores_at_minus_infinity(dev, hs):
     c.FreeAttn(ha)
 
 
+@pytest.mark.parametrize("training", [True, False])
 @pytest.mark.parametrize("hs", [32, 64])
-def test_one_order_of_a_rows_sums(dev, hs):
-    """bOneWave: a sequence's outputs are the same bits alone, where pairs of wavefronts would take it, and among many"""
+def test_one_order_of_a_rows_sums(dev, hs, training):
+    """bOneWave: a sequence's outputs are the same bits alone, where several wavefronts would share its rows, and among many"""
     c, H, T, many = dev.cuda, 4, 130, 200
     rng = np.random.default_rng(hs)
     x = [rng.standard_normal((many, H, T, hs)).astype(np.float32) for _ in range(3)]
@@ -89,7 +90,7 @@ def test_one_order_of_a_rows_sums(dev, hs):
         h = [c.AllocMemory(a[:B].ravel()) for a in x]
         hm, y = c.AllocMemory(R.causal_mask(T).ravel()), c.AllocMemory(B * H * T * hs)
         hc, ha = c.CreateCuDNN(), c.CreateAttn()
-        c.SetAttn(hc, ha, 0, True, B, T, H, hs, 0.0)
+        c.SetAttn(hc, ha, 0, training, B, T, H, hs, 0.0)
         c.AttnScaledDotProductForward(hc, ha, T, *h, hm, y, 0, bOneWave=True)
         outs.append(np.asarray(c.GetMemoryFloat(y, H * T * hs)))
         for m in (*h, hm, y):
