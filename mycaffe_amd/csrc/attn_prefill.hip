@@ -537,7 +537,9 @@ __global__ __launch_bounds__(NW * 64, OCC) void flash_fwd_kernel(FlashArgs a)
         const float lt = l[qt] + __shfl_xor(l[qt], 32, 64);
         const float inv = 1.0f / lt;
         if (a.lse2 && qrow < a.Tq && half == 0)
-            a.lse2[bh * a.Tq + qrow] = (m[qt] == a.maskedRaw) ? -INFINITY : __builtin_fmaf(m[qt], a.c, __log2f(lt));
+            a.lse2[bh * a.Tq + qrow] = (m[qt] == a.maskedRaw) ? -INFINITY
+                                     : SP == 2 && m[qt] == -INFINITY ? __builtin_nanf("")   // no score above -inf: no weights, where -inf would say equal ones
+                                     : __builtin_fmaf(m[qt], a.c, __log2f(lt));
         if (qrow < a.Tq && !over) {
             T* yr = (T*)a.y + attn_y_row(a.yMerged, b, h, a.H, a.Tq, qrow, hs);
 #pragma unroll

@@ -78,6 +78,34 @@ def test_a_step_of_scores_at_minus_infinity(dev, hs):
     c.FreeAttn(ha)
 
 
+@pytest.mark.parametrize("kind", ["none", "causal", "key", "qk"])
+@pytest.mark.parametrize("hs", [48, 64])
+def test_every_score_at_minus_infinity(dev, hs, kind):
+    """a softmax over scores of -inf alone has no weights: outputs and all gradients of that head are NaN, those of its neighbours are not"""
+    c, B, H, T = dev.cuda, 1, 2, 130
+    rng = np.random.default_rng(hs)
+    q, k, v, dy = (rng.standard_normal((B, H, T, hs)).astype(np.float32) for _ in range(4))
+    q[..., 0] = 1.0
+    k[:, 0, :, 0] = -np.inf
+    mask = {"none": None, "causal": R.causal_mask(T), "key": np.ones((B, T), np.float32), "qk": np.ones((T, T), np.float32)}[kind]
+    masked = np.zeros((B, 1, T, T), bool) | (np.asarray(R.causal_mask(T)).reshape(1, 1, T, T) == 0) if kind == "causal" else np.zeros((B, 1, T, T), bool)
+    want = exact(q[:, 1:], k[:, 1:], v[:, 1:], dy[:, 1:], masked, 1 / np.sqrt(hs))
+    h = [c.AllocMemory(x.ravel()) for x in (q, k, v, dy)]
+    out = [c.AllocMemory(q.size) for _ in range(4)]
+    hm = c.AllocMemory(np.asarray(mask, np.float32).ravel()) if mask is not None else 0
+    hc, ha = c.CreateCuDNN(), c.CreateAttn()
+    c.SetAttn(hc, ha, 0, True, B, T, H, hs, 0.0)
+    c.AttnScaledDotProductForward(hc, ha, T, *h[:3], hm, out[0], 1 if kind == "key" else 0, None)
+    c.AttnScaledDotProductBackward(hc, ha, h[0], out[1], h[1], out[2], h[2], out[3], hm, out[0], h[3])
+    for name, o, w in zip(("y", "dq", "dk", "dv"), out, want):
+        got = np.asarray(c.GetMemoryFloat(o, q.size)).reshape(q.shape)
+        assert np.isnan(got[:, 0]).all(), name
+        assert np.abs(got[:, 1:] - w).max() <= 3e-5 * max(np.abs(w).max(), 1.0), name
+    for x in (*h, *out, *([hm] if hm else [])):
+        c.FreeMemory(x)
+    c.FreeAttn(ha)
+
+
 @pytest.mark.parametrize("training", [True, False])
 @pytest.mark.parametrize("hs", [32, 64])
 def test_one_order_of_a_rows_sums(dev, hs, training):
