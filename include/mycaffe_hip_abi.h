@@ -404,7 +404,8 @@ MCH_LONG MCH_TimeInvokeFloatEx2Sets(MCH_LONG lKernelIdx, MCH_LONG lFunctionIdx, 
 /* Which kernel a float product of these sizes goes to, for tests that mean a certain one; runs on the host alone.
  * flags: 1 causal operand, 2 fp32Sums, 4 written head by head.  Returns 0 for gemm_f32_kernel, 1 for gemm_f32_split_kernel, 2 for
  * gemm_f32_small_kernel, + 4 times the tile's number there + 64 times the parts of the contraction, given the scratch memory.
- * With flag 8, 16-bit storage: the tile and the parts of a product that gemm_b16_kernel takes. */
+ * With flag 8, 16-bit storage: the tile and the parts of a product that gemm_b16_kernel takes.  With flag 16, the gradients of an inner
+ * product of m rows, n outputs and k inputs, bias included: 1 where they are one launch, 3 where that adds in levels, 0 elsewhere. */
 MCH_LONG MCH_GemmFloatRoute(MCH_LONG m, MCH_LONG n, MCH_LONG k, MCH_LONG nBatch, MCH_LONG flags);
 
 /* ---- entry point that allocates nothing (no counterpart in the reference) ----

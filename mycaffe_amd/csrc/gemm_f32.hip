@@ -1345,6 +1345,33 @@ hipError_t gemm_f32(hipStream_t s, const GemmF32& q, void* ws, size_t wsBytes)
     return hipGetLastError();
 }
 
+// Whether the gradients of an inner product (m rows, n outputs, k inputs) are one launch, and whether that adds in levels.
+struct LinearBwdF32Plan { bool together, levels; };
+static LinearBwdF32Plan linear_bwd_f32_plan(int m, int n, int k, bool bias, bool vec)
+{
+    if (!f32_near(false, n, m, n) || !f32_near(false, k, m, k) || !f32_near(true, m, n, n) || !f32_near(false, k, n, k)) return {false, false};
+    const long long tilesK = (k + 31) / 32, tilesW = (n + 31) / 32 * tilesK, tilesX = (m + 31) / 32 * tilesK;
+    if (tilesW + tilesX > (1ll << 20)) return {false, false};
+    // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
+    // time that one launch waits for the last one's stores
+    const bool sumsToo = bias && gemm_f32_row_sums_workspace_bytes(n, k, m, vec) > 0;   // the column sums with the weight gradient
+    const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false), dx = gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false);
+    const double apart = dw.time + dx.time + 2.5 +
+                         (!bias ? 0.0 : sumsToo ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
+    // the one launch, fitted to 43 sizes (0.8 .. 1.24 of what was measured, 4.4 to 199 us); a tenth on top of it, as both sides are estimates
+    const double together = 2.65 + (0.714 * (double)(tilesW + tilesX) + 0.458 / 128 * ((double)tilesW * m + (double)tilesX * n)) / 256 + 0.64 * std::max(m, n) / 128;
+    if (1.1 * together >= apart) return {false, false};
+    // Long contractions that the calls apart would not give to 32 x 32 tiles: those cut them, or add fewer values in a row.  (With fewer
+    // tiles than CUs nothing else is there while one adds up: 142 tiles of up to 2000 rows 16.0 -> 17.0 us.)
+    return {true, tilesW + tilesX > 256 && ((dw.kernel != F32_SMALL && m > 512) || (dx.kernel != F32_SMALL && n > 512))};
+}
+
+int linear_bwd_f32_route(int m, int n, int k)
+{
+    const LinearBwdF32Plan p = linear_bwd_f32_plan(m, n, k, true, n % 4 == 0 && k % 4 == 0);
+    return (p.together ? 1 : 0) + (p.levels ? 2 : 0);
+}
+
 // The gradients of an inner product as one launch, if that is what the sizes call for (*done): dW (n x k) += dY^T (n x m) X (m x k),
 // db (n, or null) += column sums of dY, dX (m x k) = dY W (n x k) + beta dX.
 hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float* X, const float* W, const float* dY, float* dW, float* db, float* dX, float beta,
@@ -1357,32 +1384,23 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     for (int i = 0; i < 3; i++)
         for (int j = i + 1; j < 6; j++)
             if (mem[i].n && mem[j].n && mem[i].p < mem[j].p + mem[j].n && mem[j].p < mem[i].p + mem[i].n) return hipSuccess;
-    if (!f32_near(false, n, m, n) || !f32_near(false, k, m, k) || !f32_near(true, m, n, n) || !f32_near(false, k, n, k)) return hipSuccess;
     const bool vec = ((((uintptr_t)X | (uintptr_t)W | (uintptr_t)dY) & 15) == 0) && n % 4 == 0 && k % 4 == 0;
-    const long long tilesK = (k + 31) / 32, tilesW = (n + 31) / 32 * tilesK, tilesX = (m + 31) / 32 * tilesK;
-    if (tilesW + tilesX > (1ll << 20)) return hipSuccess;
-    // against the launches apart: their estimates, that of the column sums (one launch, two from 1025 rows on), and 2.5 us for each
-    // time that one launch waits for the last one's stores
-    const bool sumsToo = db && gemm_f32_row_sums_workspace_bytes(n, k, m, vec) > 0;   // the column sums with the weight gradient
-    const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false), dx = gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false);
-    const double apart = dw.time + dx.time + 2.5 +
-                         (!db ? 0.0 : sumsToo ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
-    // the one launch, fitted to 43 sizes (0.8 .. 1.24 of what was measured, 4.4 to 199 us); a tenth on top of it, as both sides are estimates
-    const double together = 2.65 + (0.714 * (double)(tilesW + tilesX) + 0.458 / 128 * ((double)tilesW * m + (double)tilesX * n)) / 256 + 0.64 * std::max(m, n) / 128;
-    if (1.1 * together >= apart) return hipSuccess;
+    const LinearBwdF32Plan plan = linear_bwd_f32_plan(m, n, k, db != nullptr, vec);
+    if (!plan.together) return hipSuccess;
+    const int tilesN = (k + 31) / 32, tilesW = (n + 31) / 32 * tilesN, tilesX = (m + 31) / 32 * tilesN;
     GemmF32Args w = {}, x = {};
     w.M = n; w.N = k; w.K = w.kChunk = m;
     w.A = dY; w.B = X; w.C = dW;
     w.lda = n; w.ldb = k; w.ldc = k;
     w.alpha = 1.f; w.beta = 1.f; w.parts = 1;
     w.vecC = k % 4 == 0 && ((uintptr_t)dW & 15) == 0;
-    w.tilesM = (n + 31) / 32; w.tilesN = (int)tilesK;
+    w.tilesM = (n + 31) / 32; w.tilesN = tilesN;
     x.M = m; x.N = k; x.K = x.kChunk = n;
     x.A = dY; x.B = W; x.C = dX;
     x.lda = n; x.ldb = k; x.ldc = k;
     x.alpha = 1.f; x.beta = beta; x.parts = 1;
     x.vecC = k % 4 == 0 && ((uintptr_t)dX & 15) == 0;
-    x.tilesM = (m + 31) / 32; x.tilesN = (int)tilesK;
+    x.tilesM = (m + 31) / 32; x.tilesN = tilesN;
     constexpr int lds = small_lds<4, 64>();
     typedef void (*Kernel)(GemmF32Args, GemmF32Args, float*, XcdRuns);
     static const Kernel kernels[2][2] = {{linear_bwd_f32_small_kernel<4, 64, false, false>, linear_bwd_f32_small_kernel<4, 64, true, false>},
@@ -1393,15 +1411,12 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
         return e;
     }();
     if (attr != hipSuccess) return attr;
-    // Long contractions that the calls apart would not give to 32 x 32 tiles: those cut them, or add fewer values in a row.  (With fewer
-    // tiles than CUs nothing else is there while one adds up: 142 tiles of up to 2000 rows 16.0 -> 17.0 us.)
-    const bool levels = tilesW + tilesX > 256 && ((dw.kernel != F32_SMALL && m > 512) || (dx.kernel != F32_SMALL && n > 512));
     int most;
     const bool wFirst = w.K >= x.K;
     const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.K, x.K) + SMALL_TILE_COST, wFirst ? tilesX : tilesW, std::min(w.K, x.K) + SMALL_TILE_COST, &most);
     const int grid = 8 * most;
     *done = true;
-    hipLaunchKernelGGL(kernels[levels][vec], grid, 256, lds, s, w, x, db, runs);
+    hipLaunchKernelGGL(kernels[plan.levels][vec], grid, 256, lds, s, w, x, db, runs);
     return hipGetLastError();
 }
 

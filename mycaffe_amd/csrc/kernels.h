@@ -172,6 +172,7 @@ hipError_t k_gemv(hipStream_t s, DType adt, bool tA, int m, int n, float alpha, 
 // which kernel an fp32 product goes to (0 gemm_f32_kernel, 1 gemm_f32_split_kernel, 2 gemm_f32_small_kernel) + 4 its tile + 64 parts of the contraction
 int gemm_f32_route(int m, int n, int k, int batch, bool causal, bool fp32Sums, bool heads);
 int gemm_b16_route(int m, int n, int k);   // the same of a 16-bit product that goes to gemm_b16_kernel (0)
+int linear_bwd_f32_route(int m, int n, int k);   // gradients and bias gradient of an fp32 inner product of m rows, n outputs: 1 one launch, 3 one that adds in levels, 0 neither
 hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float* X, const float* W, const float* dY, float* dW, float* db, float* dX, float beta,
                                 bool* done);   // the gradients of an inner product as one launch, where sizes and memory allow (*done)
 // dW (n x k) += dY^T X and db (n) += column sums of dY (m x n) together; workspace 0: not taken together, one after the other

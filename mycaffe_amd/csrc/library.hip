@@ -3003,6 +3003,7 @@ MCH_LONG MCH_GemmFloatRoute(MCH_LONG m, MCH_LONG n, MCH_LONG k, MCH_LONG batch, 
 {
     if (m < 1 || n < 1 || k < 1 || batch < 1) return 0;
     if (flags & 8) return (MCH_LONG)gemm_b16_route(m, n, k);
+    if (flags & 16) return (MCH_LONG)linear_bwd_f32_route(m, n, k);
     return (MCH_LONG)gemm_f32_route(m, n, k, batch, (flags & 1) != 0, (flags & 2) != 0, (flags & 4) != 0);
 }
 

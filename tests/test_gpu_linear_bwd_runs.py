@@ -3,20 +3,25 @@ than XCDs, one product much longer than the other, contractions around the eight
 import numpy as np
 import pytest
 
+from mycaffe_amd.cudadnn import load_library
 from tests.test_gpu_double import devd  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
 
-# (rows, outputs, inputs)
-SIZES = [(5, 3, 2), (40, 1536, 384), (256, 1024, 256), (2000, 64, 256), (130, 2304, 768),   # long weight or long data gradient
-         (511, 600, 512), (512, 600, 512), (513, 600, 512), (576, 513, 520), (1025, 400, 384), (1029, 401, 387)]
+# rows, outputs, inputs, and how float takes them: 1 one launch, 3 one whose sums are added in levels of eight stages (512 k)
+SIZES = [(5, 3, 2, 1), (40, 1536, 384, 3), (256, 1024, 256, 1), (2000, 64, 256, 3), (130, 2304, 768, 3),   # long weight or long data gradient
+         (511, 600, 512, 1), (512, 600, 512, 1), (513, 600, 512, 1), (576, 513, 520, 1), (1025, 400, 384, 1), (1029, 401, 387, 1),
+         # a level and one more, two whole ones, two and one more, beside contractions below one; in 16-byte pieces and in single values
+         (513, 1025, 1536, 3), (1024, 768, 1536, 3), (1025, 513, 1536, 3), (1536, 33, 257, 3), (2049, 64, 256, 3), (33, 2049, 515, 3)]
 
 
 @pytest.mark.parametrize("base", ["float", "double"])
-@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("m,n,k,route", SIZES)
 @pytest.mark.parametrize("accumulate", [False, True])
-def test_gradients(dev, devd, base, m, n, k, accumulate):  # noqa: F811
+def test_gradients(dev, devd, base, m, n, k, route, accumulate):  # noqa: F811
+    if base == "float":
+        assert load_library().MCH_GemmFloatRoute(m, n, k, 1, 16) == route
     t, unit = (np.float32, 2.0 ** -24) if base == "float" else (np.float64, 2.0 ** -53)
     c = dev.cuda if base == "float" else devd.cuda
     rng = np.random.default_rng(m + n + k)
