@@ -37,3 +37,26 @@ def test_gradients(dev, devd, base, m, n, k, route, accumulate):  # noqa: F811
         assert (np.abs(got - want) <= bound(l) * scale).all()
     for a in h:
         c.FreeMemory(a)
+
+
+@pytest.mark.parametrize("base,m,n,k", [("float", 3667, 280, 188), ("float", 2049, 96, 600), ("float", 2705, 100, 227), ("double", 1367, 77, 160), ("double", 1900, 96, 60),
+                                        ("double", 4000, 48, 21)])
+def test_error_of_the_bias_gradient(dev, devd, base, m, n, k):  # noqa: F811
+    """A bias gradient of many rows is as close to the sum as additions in levels of eight stages leave it."""
+    t, unit, quad, lanes = (np.float32, 2.0 ** -24, 4, 8) if base == "float" else (np.float64, 2.0 ** -53, 2, 16)
+    c, wide = (dev.cuda, np.float64) if base == "float" else (devd.cuda, np.longdouble)
+    if base == "float":
+        assert load_library().MCH_GemmFloatRoute(m, n, k, 1, 16) & 1
+    rng = np.random.default_rng(m)
+    x, w, dy = (rng.standard_normal(s).astype(t) for s in ((m, k), (n, k), (m, n)))
+    h = [c.AllocMemory(a.ravel()) for a in (x, w, dy, np.zeros((n, k), t), np.zeros(n, t), np.zeros((m, k), t))]
+    c.LinearBackward(m, n, k, *h)
+    err = np.asarray(c.GetMemoryFloat(h[4], n)).astype(wide) - dy.astype(wide).sum(0)
+    # an addition is off by at most unit / sqrt(3) of its result in the mean square, and sums of N(0, 1) values have their number as mean square:
+    # the values of a lane's fragment, 16 of those in a level, its levels, the lanes of a row, the gradient that is added to
+    levels = -(-m // 512)
+    squares = m / quad * sum(range(2, quad + 1)) + lanes * levels * sum(quad * i for i in range(1, 17)) + lanes * sum(16 * quad * i for i in range(1, levels + 1)) \
+        + sum(m / lanes * i for i in range(1, lanes + 1)) + m
+    assert np.sqrt((err ** 2).mean()) <= unit * np.sqrt(squares / 3)
+    for a in h:
+        c.FreeMemory(a)
