@@ -135,10 +135,11 @@ __device__ __forceinline__ void f32_store(const GemmF32Args& g, const HeadsArg<H
         bias = f32_bias4(g.bias, c, N);
         if constexpr (HEADS) col = heads_col<float>(hp.he, c);
     }
-    // what the result is added to comes for eight rows at once; in the loop below each row would wait for memory (A^T B, added: 8000 x 512 x
-    // 1000 56.2 us, 51.0 so, 10000 x 288 x 700 40.2, 37.1, 32000 x 768 x 1000 225, 217).  Rows 16 KB apart lie on the same channels of
-    // memory, and there one after the other is the better way (4096 x 4096 x 1024 183 us, 189 at once).
-    const bool add = vec && beta != 0.f && ldc % 4096 != 0;
+    // What the result is added to comes for eight rows at once; in the loop below each row would wait for memory (A^T B, added: 8000 x 512 x
+    // 1000 65 us, 63 so, 32000 x 768 x 1000 255, 244, 5000 x 1000 x 1000 89, 82; A B: 8192 x 3072 x 768 214, 199, 1000 x 4096 x 512 41, 37).
+    // Tiles with eight sums of 16 a lane have no registers for that (46 of them in memory, 9 without: 4096 x 4096 x 1024, A^T B, 172 us, 174
+    // with it), and what goes head by head is not added.
+    const bool add = !HEADS && WM * WN < 8 && vec && beta != 0.f;
     constexpr int AHEAD = NIT < 8 ? NIT : 8;
 #pragma unroll
     for (int i = 0; i < WM; i++) {
