@@ -908,9 +908,10 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
     [[maybe_unused]] floatx16 all;
 #pragma unroll
     for (int v = 0; v < 16; v++) { acc[v] = 0.f; all[v] = 0.f; }
-    // a row's sum in levels of eight stages (the bias gradient of 3667 rows: error against float64 2.1e-7 in one run, 1.2e-7 so)
+    // a row's sum as two, with LEVELS also in levels (the bias gradient of 3667 rows: error against float64 2.1e-7 as one in one run, 1.2e-7 so)
     const bool sumRows = rowSums && it.n0 == 0;
-    float rowSum = 0.f, rowAll = 0.f;
+    constexpr int J = BK / 8 / NW;
+    float rowSum[J] = {}, rowAll = 0.f;
 #pragma unroll
     for (int i = 0; i < S - 1; i++)
         if (i < nk) fetch(smem + i * STAGE);
@@ -923,7 +924,6 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
         const float* stage = smem + buf * STAGE;
         buf = buf == S - 1 ? 0 : buf + 1;
         const int units = (min(BK, kEnd - kBegin - kt * BK) + 7) / 8;
-        constexpr int J = BK / 8 / NW;
         u32x4 a[J], b[J];
 #pragma unroll
         for (int j = 0; j < J; j++) {
@@ -937,12 +937,10 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
 #pragma unroll
         for (int j = 0; j < J; j++)
             if (NW * j < units) acc = BigTraits<float>::mma(b[j], a[j], acc);   // the transposed tile (B as the row operand): a lane owns a row of C
-        if (sumRows) {
+        if (sumRows)
 #pragma unroll
             for (int j = 0; j < J; j++)   // zeros past the end
-                rowSum += (__uint_as_float(a[j].x) + __uint_as_float(a[j].y)) + (__uint_as_float(a[j].z) + __uint_as_float(a[j].w));
-            if (kt % 8 == 7) { rowAll += rowSum; rowSum = 0.f; }
-        }
+                rowSum[j] += (__uint_as_float(a[j].x) + __uint_as_float(a[j].y)) + (__uint_as_float(a[j].z) + __uint_as_float(a[j].w));
     };
     if constexpr (LEVELS) {
         for (int kt = 0; kt < nk;) {
@@ -950,6 +948,8 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
             for (; kt < end; kt++) step(kt);
 #pragma unroll
             for (int v = 0; v < 16; v++) { all[v] += acc[v]; acc[v] = 0.f; }
+#pragma unroll
+            for (int j = 0; j < J; j++) { rowAll += rowSum[j]; rowSum[j] = 0.f; }
         }
         acc = all;
     } else
@@ -958,7 +958,11 @@ __device__ __forceinline__ void f32_small_tile(const GemmF32Args& g, const Heads
     float* slice = smem + wave * 32 * LDC;
 #pragma unroll
     for (int q = 0; q < 4; q++) *(float4*)(slice + fr * LDC + 8 * q + 4 * half) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-    if (sumRows) smem[NW * 32 * LDC + tid] = rowAll + rowSum;
+    if (sumRows) {
+#pragma unroll
+        for (int j = 0; j < J; j++) rowAll += rowSum[j];
+        smem[NW * 32 * LDC + tid] = rowAll;
+    }
     __syncthreads();
     if (sumRows && tid < 32 && it.m0 + tid < g.M) {
         float t = 0.f;

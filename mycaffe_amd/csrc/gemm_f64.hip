@@ -191,9 +191,10 @@ __device__ __forceinline__ void d_small_tile(const GemmD& g, const HeadsD& he, i
         }
     };
     d_vec4 acc = {0.0, 0.0, 0.0, 0.0};
-    // a row's sum in levels of eight stages, as in gemm_f32.hip
+    // a row's sum as two, as in gemm_f32.hip
     const bool sumRows = rowSums && n0 == 0;
-    double rowSum = 0.0, rowAll = 0.0;
+    constexpr int J = BK / 8 / NW;
+    double rowSum[J] = {};
 #pragma unroll
     for (int i = 0; i < S - 1; i++)
         if (i < nk) fetch(smem + i * STAGE);
@@ -205,7 +206,6 @@ __device__ __forceinline__ void d_small_tile(const GemmD& g, const HeadsD& he, i
         const double* stage = smem + buf * STAGE;
         buf = buf == S - 1 ? 0 : buf + 1;
         const int units = (min(BK, g.k - kt * BK) + 7) / 8;
-        constexpr int J = BK / 8 / NW;
         double a[J][2], b[J][2];
 #pragma unroll
         for (int j = 0; j < J; j++) {
@@ -222,17 +222,20 @@ __device__ __forceinline__ void d_small_tile(const GemmD& g, const HeadsD& he, i
                 acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j][0], b[j][0], acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j][1], b[j][1], acc, 0, 0, 0);
             }
-        if (sumRows) {
+        if (sumRows)
 #pragma unroll
-            for (int j = 0; j < J; j++) rowSum += a[j][0] + a[j][1];   // zeros past the end
-            if (kt % 8 == 7) { rowAll += rowSum; rowSum = 0.0; }
-        }
+            for (int j = 0; j < J; j++) rowSum[j] += a[j][0] + a[j][1];   // zeros past the end
     }
     __syncthreads();
     constexpr int LD = 17;
 #pragma unroll
     for (int v = 0; v < 4; v++) smem[(wave * 16 + 4 * v + fq) * LD + fr] = acc[v];
-    if (sumRows) smem[NW * 16 * LD + tid] = rowAll + rowSum;
+    if (sumRows) {
+        double t = 0.0;
+#pragma unroll
+        for (int j = 0; j < J; j++) t += rowSum[j];
+        smem[NW * 16 * LD + tid] = t;
+    }
     __syncthreads();
     if (sumRows && tid < 16 && m0 + tid < g.m) {
         double t = 0.0;
