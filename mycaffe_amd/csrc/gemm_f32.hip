@@ -1421,7 +1421,7 @@ hipError_t linear_bwd_f32_small(hipStream_t s, int m, int n, int k, const float*
     if (attr != hipSuccess) return attr;
     int most;
     const bool wFirst = w.K >= x.K;
-    const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.K, x.K) + SMALL_TILE_COST, wFirst ? tilesX : tilesW, std::min(w.K, x.K) + SMALL_TILE_COST, &most);
+    const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.K, x.K), wFirst ? tilesX : tilesW, std::min(w.K, x.K), SMALL_TILE_COST, &most);
     const int grid = 8 * most;
     *done = true;
     hipLaunchKernelGGL(kernels[plan.levels][vec], grid, 256, lds, s, w, x, db, runs);

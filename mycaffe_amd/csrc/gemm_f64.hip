@@ -433,7 +433,7 @@ hipError_t d_linear_bwd_small(hipStream_t s, int m, int n, int k, const double* 
     constexpr int lds = d_small_lds<4, 64>();
     int most;
     const bool wFirst = w.k >= x.k;
-    const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.k, x.k) + D_TILE_COST, wFirst ? tilesX : tilesW, std::min(w.k, x.k) + D_TILE_COST, &most);
+    const XcdRuns runs = xcd_runs(wFirst ? tilesW : tilesX, std::max(w.k, x.k), wFirst ? tilesX : tilesW, std::min(w.k, x.k), D_TILE_COST, &most);
     const int grid = 8 * most;
     if (vec) hipLaunchKernelGGL((d_linear_bwd_small_kernel<4, 64, true>), grid, 256, lds, s, w, x, db, (int)tilesN, (int)tilesW, (int)tilesX, runs);
     else hipLaunchKernelGGL((d_linear_bwd_small_kernel<4, 64, false>), grid, 256, lds, s, w, x, db, (int)tilesN, (int)tilesW, (int)tilesX, runs);

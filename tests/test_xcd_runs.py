@@ -1,5 +1,5 @@
-"""Tiles of two products dealt to the XCDs (csrc/xcd_runs.h), on the host: every tile once, runs of equal work, and none longer than an XCD holds
-where all tiles are there at once."""
+"""Tiles of two products dealt to the XCDs (csrc/xcd_runs.h), on the host: every tile once, by count where that is the rule, in runs of equal
+work else, and none longer than an XCD holds where that matters."""
 import os
 import subprocess
 
@@ -13,9 +13,9 @@ PROGRAM = """
 int main()
 {
     long long a, b;
-    int ca, cb, most;
-    while (scanf("%lld %d %lld %d", &a, &ca, &b, &cb) == 4) {
-        const mch::XcdRuns r = mch::xcd_runs(a, ca, b, cb, &most);
+    int ka, kb, most;
+    while (scanf("%lld %d %lld %d", &a, &ka, &b, &kb) == 4) {
+        const mch::XcdRuns r = mch::xcd_runs(a, ka, b, kb, 84, &most);
         for (int x = 0; x < 9; x++) printf("%d ", r.first[x]);
         printf("%d\\n", most);
     }
@@ -38,17 +38,18 @@ def runs(tmp_path_factory):
 
 def test_runs(runs):
     rng = np.random.default_rng(1)
-    cases = [(188, 263, 564, 118), (315, 736, 441, 535), (314, 3230, 390, 2619), (9, 811, 69, 168), (1, 100, 0, 90), (0, 100, 1, 90), (256, 1136, 1024, 368), (1 << 19, 70000, 1 << 19, 90)]
-    for _ in range(2000):
-        short = int(2 ** rng.uniform(6.5, 14))
+    cases = [(188, 179, 564, 34), (315, 652, 441, 451), (314, 3118, 390, 2507), (9, 727, 69, 84), (1, 100, 0, 90), (0, 100, 1, 90), (256, 1024, 1024, 256), (56, 3181, 700, 256),
+             (1 << 19, 70000, 1 << 19, 90)]
+    for _ in range(3000):
+        short = int(2 ** rng.uniform(0, 14))
         cases.append((int(2 ** rng.uniform(0, 11)), short + int(2 ** rng.uniform(0, 14)), int(2 ** rng.uniform(0, 11)), short))
-    for (a, ca, b, cb), (*first, most) in zip(cases, runs(cases)):
-        case = (a, ca, b, cb, first)
+    for (a, ka, b, kb), (*first, most) in zip(cases, runs(cases)):
+        case, ca, cb = (a, ka, b, kb, first), ka + 84, kb + 84
         count = np.diff(first)
         assert first[0] == 0 and first[8] == a + b and (count >= 0).all() and most == count.max(), case
-        if a + b <= 8 * 32 or (a + b <= 8 * 96 and ca < 2 * cb):
+        if a + b <= 8 * 32 or (a + b <= 8 * 96 and 5 * ca < 7 * cb):
             assert most <= -(-(a + b) // 8), case            # by count
-        elif a + b <= 8 * 96:
+        elif a + b <= 8 * 96 and kb <= 64:
             assert most <= 96, case                           # what an XCD holds
         else:
             cost = np.minimum(first, a) * ca + np.maximum(np.array(first) - a, 0) * cb
