@@ -1366,8 +1366,12 @@ static LinearBwdF32Plan linear_bwd_f32_plan(int m, int n, int k, bool bias, bool
     const GemmF32Choice dw = gemm_f32_choose(n, k, m, 1, false, SIZE_MAX, false), dx = gemm_f32_choose(m, k, n, 1, false, SIZE_MAX, false);
     const double apart = dw.time + dx.time + 2.5 +
                          (!bias ? 0.0 : sumsToo ? dw.plan.splits > 1 ? 0.5 : 4.5 : m <= 1024 ? 4.5 : 9.0);
-    // the one launch, fitted to 43 sizes (0.8 .. 1.24 of what was measured, 4.4 to 199 us); a tenth on top of it, as both sides are estimates
-    const double together = 2.65 + (0.714 * (double)(tilesW + tilesX) + 0.458 / 128 * ((double)tilesW * m + (double)tilesX * n)) / 256 + 0.64 * std::max(m, n) / 128;
+    // the one launch, fitted to 43 sizes (0.8 .. 1.24 of what was measured, 4.4 to 199 us); a tenth on top of it, as both sides are estimates.  In
+    // 4-byte pieces it takes a quarter longer, and so do the products apart, except in the split kernel: beside two of those an estimate of
+    // its own, fitted to 179 sizes (971 rows, 1996 to 1045: 96 us together, 87 apart; 2385 rows, 2252 to 770 210 and 142)
+    const double tiles = (double)(tilesW + tilesX), work = (double)tilesW * m + (double)tilesX * n, longer = std::max(m, n);
+    const bool pieces = !vec && dw.kernel == F32_SPLIT && dx.kernel == F32_SPLIT;
+    const double together = pieces ? 3.4 + (0.382 * tiles + 0.638 / 128 * work) / 256 + 0.83 * longer / 128 : 2.65 + (0.714 * tiles + 0.458 / 128 * work) / 256 + 0.64 * longer / 128;
     if (1.1 * together >= apart) return {false, false};
     // Long contractions that the calls apart would not give to 32 x 32 tiles: those cut them, or add fewer values in a row.  (With fewer
     // tiles than CUs nothing else is there while one adds up: 142 tiles of up to 2000 rows 16.0 -> 17.0 us.)
