@@ -9,10 +9,11 @@
 // Large products run at the power limit (1.8 GHz at 8192 x 3072 x 6144), where what an instruction costs is time: products of 16 x 16 x 32
 // alone, on normally distributed values, reach 2.0 PFLOP/s, those of 32 x 32 x 16 1.8 (2.4 and 2.5 on zeros), and a wavefront reads the same
 // fragments for either (4096^3, A B^T 124 -> 119 us, A B 125.5 -> 123; 8000 x 3072 x 768 47.7 -> 46.5).  The sums are the same bits.  Where
-// it is not power but the first product of a stage that is waited for, the longer instruction stays, for which half as much has to
-// arrive (time with the shorter one over time with the longer, means of ten sizes of 10^9 multiplications and more): four wavefronts alone on
-// their CU (128 x 128 in three stages: A B 1.03, A^T B 1.09, A^T B^T 1.03, A B^T 1.00), eight with 32 x 32 of C each (1.01, 1.03 in A^T B^T) and
-// both operands read transposed by wavefronts with at most 32 x 64 (1.02).  All others are 0.95 - 1.01.
+// it is not power but the first product of a stage that is waited for, and operands are read transposed, the longer instruction stays, for
+// which half as much has to arrive (time with the shorter one over time with the longer, means of ten sizes of 10^9 multiplications and
+// more): four wavefronts alone on their CU (128 x 128 in three stages: A B 1.03, A^T B 1.09, A^T B^T 1.03), eight with 32 x 32 of C each (A^T B^T
+// 1.03) and both operands read transposed by wavefronts with at most 32 x 64 (1.02).  All others are 0.95 - 1.01, and better where the
+// contraction is short (4096 x 512 x 512 behind an attention launch: 0.8 us less).
 //
 //   * k at unit stride: LDS holds [row][64 k] without padding, the 16-byte piece c of row r at position c ^ ((r >> 1) & 7)
 //     (sixteen consecutive rows read by a 128-bit access then fall on sixteen bank groups).
@@ -205,7 +206,7 @@ __device__ __forceinline__ void b16_tile(const GemmB16Args& g, const B16Arg<HEAD
 {
     constexpr int NT = 64 * WVM * WVN, BM = 32 * WVM * WM, BN = 32 * WVN * WN, BK = 64;
     constexpr bool PROMPT = HEADS >= 3;
-    constexpr bool WAITS = (WVM * WVN == 4 && WM * WN == 4 && S == 3) || (WVM * WVN == 8 && WM * WN == 1) || (!AK && !BKC && WM * WN <= 2);
+    constexpr bool WAITS = (WVM * WVN == 4 && WM * WN == 4 && S == 3 && !(AK && BKC)) || (WVM * WVN == 8 && WM * WN == 1 && !AK) || (!AK && !BKC && WM * WN <= 2);
     constexpr int F = WAITS ? 32 : 16, KM = 512 / F, KS = BK / KM, TM = 32 * WM / F, TN = 32 * WN / F;   // rows and k of a product; products' tiles of a wavefront
     constexpr int PA = BM * 8 / NT, PB = BN * 8 / NT;               // 16-byte chunks per thread and stage
     constexpr int STAGE = (BM + BN) * BK;                           // elements of one stage: A's part, then B's
